@@ -106,10 +106,30 @@ __device__ __forceinline__ void load8_as_float(const float* p, float* v) {
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
+// eight consecutive values of a product: as they are, or the sum of float32 partial sums in the order of the splits, with the
+// loads of up to four splits on their way together
+__device__ __forceinline__ void load8_sum(const bf16_t* p, int, size_t, float* v) { load8_as_float(p, v); }
+__device__ __forceinline__ void load8_sum(const float* p, int n_splits, size_t split_stride, float* v) {
+    load8_as_float(p, v);
+    for (int s0 = 1; s0 < n_splits; s0 += 3) {
+        float t[3][8];
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            if (s0 + u < n_splits) load8_as_float(p + (s0 + u) * split_stride, t[u]);
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            if (s0 + u < n_splits) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] += t[u][i];
+            }
+    }
+}
+
 // The same for bfloat16 activations with eight features per thread and load (16-byte loads of the
 // activations, 32 bytes of the residual stream): the form that prompt portions of many tokens take.
-template <typename DT>   // delta as bfloat16, or as float32 (a product that was written out in float32)
+template <typename DT>   // delta as bfloat16, or as float32 partial sums (one: a product that was written out in float32)
 __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict__ h, const DT* __restrict__ delta,
+                                                               int n_splits, size_t split_stride,
                                                                const int32_t* __restrict__ rows,
                                                                const bf16_t* __restrict__ weight, float w_off, float eps,
                                                                bf16_t* __restrict__ out, int hidden) {
@@ -129,7 +149,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict
         if (one_pass) load8_as_float(weight + j, kept_w);     // with the row's loads, not behind the workgroup's sum
         if (drow) {
             float d[8];
-            load8_as_float(drow + j, d);
+            load8_sum(drow + j, n_splits, split_stride, d);
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] += d[i];
             if (write_back) {
@@ -158,7 +178,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict
             load8_as_float(hrow + j, v);
             if (drow && !write_back) {
                 float d[8];
-                load8_as_float(drow + j, d);
+                load8_sum(drow + j, n_splits, split_stride, d);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] += d[i];
             }
@@ -439,16 +459,16 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
     // enough threads for a row to stay in registers (four values a thread, eight for the widest rows)
     const int threads = (delta_splits > 1 || hidden > 2048) ? 1024 : (hidden > 1024 ? 512 : 256);
     const size_t stride = static_cast<size_t>(delta_rows) * hidden;
-    if (dtype == 1 && delta_splits <= 1 && hidden % 8 == 0 && n_rows >= 32 && !fixed) {
+    if (dtype == 1 && hidden % 8 == 0 && !fixed && (delta_splits <= 1 ? n_rows >= 32 : n_rows > 64)) {
         const int threads = hidden >= 2048 ? 256 : 128;
         float* hf = static_cast<float*>(h);
         if (delta_splits == 0)
             add_rmsnorm_vec8_kernel<bf16_t><<<n_rows, threads, 0, s>>>(
-                hf, static_cast<const bf16_t*>(delta), rows, static_cast<const bf16_t*>(weight), weight_offset,
+                hf, static_cast<const bf16_t*>(delta), 1, stride, rows, static_cast<const bf16_t*>(weight), weight_offset,
                 eps, static_cast<bf16_t*>(out), hidden);
-        else   // one float32 "partial sum": a product written out in float32
+        else   // float32 partial sums; one of them: a product written out in float32
             add_rmsnorm_vec8_kernel<float><<<n_rows, threads, 0, s>>>(
-                hf, static_cast<const float*>(delta), rows, static_cast<const bf16_t*>(weight), weight_offset,
+                hf, static_cast<const float*>(delta), delta_splits, stride, rows, static_cast<const bf16_t*>(weight), weight_offset,
                 eps, static_cast<bf16_t*>(out), hidden);
         EGPT_CHECK_LAUNCH();
         return EGPT_OK;
@@ -603,4 +623,4 @@ extern "C" const char* egpt_error_string(int code) {
     }
 }
 
-extern "C" int egpt_abi_version(void) { return 26; }
+extern "C" int egpt_abi_version(void) { return 27; }

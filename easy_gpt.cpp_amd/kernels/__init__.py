@@ -229,6 +229,10 @@ class KernelBackend:
         """silu(x Wgate^T) * (x Wup^T) as act [T, I] in one kernel, or None."""
         return None
 
+    def gate_up_rows(self, x, w, activation="silu"):
+        """The same for many rows, or None."""
+        return None
+
     def constant_decay_heads(self, *args, **kwargs):
         """act [T, heads * dv]: a linear attention with one constant decay per head from the input product to the gated heads,
         in place of decayed_state_scan and head_norm_gate (operands: `kernels.hip.HipKernels.constant_decay_heads`); None if

@@ -30,7 +30,7 @@ def _load_library() -> ctypes.CDLL:
         lib = ctypes.CDLL(path)
     except (build.BuildError, OSError) as e:
         raise KernelsUnavailable(f"the HIP kernel library could not be built or loaded: {e}") from e
-    if lib.egpt_abi_version() != 26:
+    if lib.egpt_abi_version() != 27:
         raise KernelsUnavailable(f"{path} has an unexpected ABI version")
     return lib
 
@@ -95,6 +95,7 @@ class HipKernels(KernelBackend):
             "egpt_linear": [vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_f32": [vp, vp, vp, vp, i, i, i, i, vp],
             "egpt_gemm_skinny": [vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp],
+            "egpt_gemm_rows": [vp, vp, vp, i, i, i, i, i, i, i, vp],
             "egpt_paged_attention": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp],
             "egpt_paged_attention_mfma": [vp, vp, vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, i, i, vp],
             "egpt_attention_any_tiled": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp],
@@ -281,6 +282,60 @@ class HipKernels(KernelBackend):
         # 1,536 x 1,536 7.7 against 9.2, 2,560 x 2,048 8.9 against 12.0, 2,048 x 2,048 8.1 against 11.8; 4,608 x 3,584 18.9
         # either way, 3,584 x 3,584 14.2 against 13.7, 7,168 x 5,120 25.8 against 22.7)
         return n * k >= (6 << 20 if m > 32 else 16 << 20)
+
+    # The tiles of the product for many rows (gemm_rows.hip): rows of x, rows of w, workgroups that a CU holds, and a fit of
+    # what was measured (some 250 sizes of 72 to 8,191 rows, 12 matrices; a tenth off on average): microseconds of a launch, of
+    # a round of workgroups, and of a step of 64 values of k with one workgroup on a CU and with as many as it holds.
+    _rows_shapes = ((256, 256, 1, -4.4, 16.7, 1.14, 1.14), (192, 256, 1, -2.4, 12.7, 0.94, 0.94), (128, 256, 1, -0.8, 9.0, 0.83, 0.83),
+                    (128, 128, 2, 4.8, 1.8, 0.50, 1.33), (64, 64, 4, 6.3, -2.7, 0.36, 1.06))
+
+    @classmethod
+    def _rows_plan(cls, m: int, n: int, k: int, most_splits: int) -> tuple[int, int]:
+        """(shape, splits of the k range) of the product for many rows: the cheapest by the fit, a split paying for what
+        its reader reads more (4.5 TB/s).  `n`: the rows of w.  (Against the best of everything that was measured, the
+        choice is 8 % slower on average and a third at worst.)"""
+        steps = k // 64
+        best = None
+        for shape, (bm, bn, held, launch, per_round, alone, full) in enumerate(cls._rows_shapes):
+            tiles = -(-m // bm) * -(-n // bn)
+            for s in range(1, most_splits + 1):
+                per = -(-steps // s)
+                if s > 1 and (per < 4 or (s - 1) * per >= steps or s * tiles > 700):
+                    continue
+                rounds, rest = divmod(s * tiles, 256 * held)
+                us = launch + rounds * (per_round + per * full)
+                if rest:
+                    load = max(rest / 256, 1.0)
+                    us += per_round + per * (alone + (full - alone) * (load - 1) / max(held - 1, 1))
+                us = max(us, 3 + n * k * 2 / 4.4e6)                 # the weights alone
+                if s > 1:
+                    us += m * n * (4 * s - 2) / 4.5e6
+                if best is None or us < best[0]:
+                    best = us, shape, s
+        return best[1], best[2]
+
+    @staticmethod
+    def _rows_fit(x, w, k: int) -> bool:
+        """Whether gemm_rows.hip takes these operands."""
+        return (x.dtype == _BF16 and w.dtype == _BF16 and k % 64 == 0 and w.shape[0] % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+                and w.shape[0] * k < 1 << 30)
+
+    @staticmethod
+    def _own_rows(m: int, n: int, k: int, unrounded: bool) -> bool:
+        """Whether a bfloat16 product of more than 64 rows is the framework's own (gemm_rows.hip) instead of the
+        library's first choice, whose times are the second ones here (us, weights from memory)."""
+        if unrounded:
+            # one float32 result, no split: 1,152 x 896 at 96 / 552 / 1,500 rows 6.5 / 6.8 / 8.9 against 7.7 / 8.6 / 10.1, at
+            # 2,048 11.5 against 11.6; 2,048 x 1,536 at 200 rows 10.0 against 9.2, 4,608 x 3,584 at 552 35 against 34
+            return k <= 1024 and m <= 1536
+        if k >= 2 * n:
+            # a long k range, which the library does not split: 896 x 4,864 at 96 / 552 / 2,048 rows 9 / 16 / 31 against 13 / 18
+            # / 34 (with the reader's share), 3,584 x 18,944 48 / 83 / 218 against 88 / 137 / 362; at 4,100 rows even, at
+            # 8,191 a fifth slower
+            return m <= 3584
+        # 896 x 896 at 96 / 552 / 2,048 rows 4.9 / 6.7 / 9.1 against 7.7 / 8.3 / 9.9, 3,584 x 3,584 at 96 / 432 15 / 24 against 20 /
+        # 27; but 1,536 x 1,536 at 1,500 rows 21 against 15, 3,584 x 3,584 at 552 33 against 27
+        return m <= (2048 if k <= 1024 else 448)
 
     def linear(self, x, w, bias, out):
         m, k = x.shape
@@ -528,6 +583,22 @@ class HipKernels(KernelBackend):
                   _GATES[activation], self._stream())
         return out
 
+    def gate_up_rows(self, x, w, activation="silu"):
+        """The same for more than 64 rows.  Returns None where the case is not covered."""
+        t, k = x.shape
+        if t <= 64 or w.shape[0] % 2 or not self._rows_fit(x, w, k):
+            return None
+        # (against the library's product and an activation kernel, us: 9,728 x 896 at 96 / 552 / 2,048 / 8,191 rows 12 / 21 /
+        # 50 / 170 against 17 / 25 / 69 / 202; 17,920 x 1,536 22 / 37 / 122 / 455 against 25 / 44 / 140 / 443; 37,888 x 3,584 59 /
+        # 142 / 456 against 62 / 149 / 561)
+        inter = w.shape[0] // 2
+        self._need(x, "x", _BF16)
+        self._need(w, "w", _BF16, (2 * inter, k))
+        out = torch.empty((t, inter), dtype=_BF16, device=x.device)
+        self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), t, inter, k, 1, 2, _GATES[activation],
+                  self._rows_plan(t, 2 * inter, k, 1)[0], self._stream())
+        return out
+
     def combine_attention(self, part_o, part_ml, out):
         """out act [T, nq*hd] from the parts of a split attention (what paged_attention does with combine=True)."""
         a_splits, t, nq, hd = part_o.shape
@@ -560,6 +631,15 @@ class HipKernels(KernelBackend):
             self._run("egpt_gemm_skinny", x.data_ptr(), w.data_ptr(), None, self._ptr(out), None, self._ptr(target),
                       m, n, k, s, 4, self._stream())
             return out if target is None else target
+        if m > 64 and self._rows_fit(x, w, k) and self._own_rows(m, n, k, unrounded):
+            # many rows on the framework's own kernel: rounded, or float32 partial sums where the k range is split
+            self._need(x, "x")
+            self._need(w, "w", x.dtype, (n, k))
+            shape, s = self._rows_plan(m, n, k, 1 if unrounded else 10)
+            kind = 1 if unrounded or s > 1 else 0
+            out = torch.empty((s, m, n) if kind else (m, n), dtype=_F32 if kind else _BF16, device=x.device)
+            self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, kind, 0, shape, self._stream())
+            return out
         if unrounded and x.dtype == _BF16 and m > 0 and k % 8 == 0:
             # many rows: the library's product (the reference uses cuBLAS for every linear layer), written out in
             # float32; it goes on as a single "partial sum" [1, m, n]

@@ -78,6 +78,8 @@ class SwiGLU(FeedForward):
             residual = pending.residual()
         t = x.shape[0]
         act = k.gate_up_swiglu(x, self.w_gate_up, activation=self.activation)        # a few dozen tokens: product and activation in one kernel
+        if act is None:
+            act = k.gate_up_rows(x, self.w_gate_up, activation=self.activation)      # and more of them
         if act is not None:
             return down(act)
         gate_up = k.product(x, self.w_gate_up)           # act [T, 2I] or float32 partial sums [S, T, 2I]
