@@ -315,6 +315,11 @@ int egpt_moe_group(const int32_t* chosen, int32_t* row_token, int32_t* place, in
 // (an expert's gate rows, then its up rows).  act [n_tokens * top][ff] of the activation type.
 int egpt_moe_gate_up(const void* x, const void* w_gate_up, const int32_t* row_token, const int32_t* tiles, void* act,
                      int n_rows, int hidden, int ff, int experts, int tile_rows, int dtype, void* stream);
+// The same products in bfloat16 with operands staged through LDS (gemm_rows.hip), w [experts][rows of w][k]: kind 2 writes out
+// [n_rows][n] = act(gate) * up (w: n gate rows, then n up rows; act as in egpt_swiglu), 3 relu(.)^2, 1 the product in float32.
+// row_token null: grouped row r reads row r of x.  tile_rows: 64 or 128.  n % 4 == 0, k % 64 == 0, operands on 16 bytes.
+int egpt_moe_rows(const void* x, const void* w, const int32_t* row_token, const int32_t* tiles, void* out, int n_rows, int x_rows,
+                  int n, int k, int experts, int tile_rows, int kind, int act, void* stream);
 // act[row] = relu(x[row_token[row]] Wu_e^T)^2 for every grouped row; w_up [experts][ff][hidden].
 int egpt_moe_up(const void* x, const void* w_up, const int32_t* row_token, const int32_t* tiles, void* act, int n_rows,
                 int hidden, int ff, int experts, int tile_rows, int dtype, void* stream);

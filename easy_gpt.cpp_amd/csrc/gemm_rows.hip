@@ -56,12 +56,20 @@ __device__ __forceinline__ r_i32x4 buffer_of(const void* p, size_t bytes) {
                    __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000};
 }
 
-enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsGated = 2 };
+enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsGated = 2, kRowsRelu2 = 3 };
 
-template <int BM, int BN, int WM, int WN, int WB, int OUT>
+// Products of rows grouped by expert (moe.hip makes the table of tiles): tile i has rows tiles[3 i + 2 ..] of one expert, the
+// numbers of tiles[1 + 3 i ..] being the expert, the tile's first grouped row and its rows; w is [experts][rows of w][k].
+struct Groups {
+    const int32_t* tiles;          // null: one matrix for all rows
+    const int32_t* row_token;      // the row of x that a grouped row reads (null: the grouped row itself)
+    int x_rows;                    // rows of x
+};
+
+template <int BM, int BN, int WM, int WN, int WB, int OUT, bool GROUPED>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k, int splits,
-    int steps_per_split, int act) {
+    int steps_per_split, int act, Groups groups) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int NW = WM * WN;
     constexpr int TM = BM / WM / 16, TN = BN / WN / 16;        // 16 x 16 tiles of a wavefront
@@ -76,29 +84,41 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
 
     // workgroups are handed to the eight dies in turn: a die gets a contiguous range of tiles, rows of x fastest, so that
     // its L2 holds the few rows of w and x that its tiles share
-    const int mt = (m + BM - 1) / BM, nt = OUT == kRowsGated ? (n + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
+    constexpr int BC = OUT == kRowsGated ? BN / 2 : BN;         // columns of the result in a tile
+    const int mt = GROUPED ? groups.tiles[0] : (m + BM - 1) / BM, nt = (n + BC - 1) / BC;
     const int tiles = mt * nt, items = tiles * splits;
     int item = blockIdx.x;
+    if (GROUPED && item >= items) return;                      // (the grid is sized for the most tiles that the rows can make)
     {
         const int q = items / 8, r = items % 8, d = item % 8, i = item / 8;
         item = d * q + (d < r ? d : r) + i;
     }
     const int tile = item % tiles, split = item / tiles;
-    const int m0 = tile % mt * BM, nb = tile / mt;
-    const int n0 = nb * (OUT == kRowsGated ? BN / 2 : BN);
+    int m0 = tile % mt * BM, n0 = tile / mt * BC, rows = min(m - m0, BM);
+    if (GROUPED) {
+        // all columns of a tile of rows after each other: an expert's matrix stays in the die's L2 for its tiles
+        const int32_t* entry = groups.tiles + 1 + 3 * (item / nt);
+        m0 = entry[1];
+        n0 = item % nt * BC;
+        rows = entry[2];
+        w += static_cast<size_t>(entry[0]) * (OUT == kRowsGated ? 2 * n : n) * k;
+    }
     const int total = k / kRowsStep;
     const int s_begin = split * steps_per_split, s_end = min(total, s_begin + steps_per_split);
 
     // ---- loads: a lane's byte offsets from the tile's first rows (rows beyond the last repeat the last)
     const int piece = (lane % 8) ^ (lane / 8);
     const size_t row_bytes = static_cast<size_t>(k) * 2;
-    const r_i32x4 xr = buffer_of(x + static_cast<size_t>(m0) * k, min(m - m0, BM) * row_bytes);
+    const bool gather = GROUPED && groups.row_token != nullptr;
+    const r_i32x4 xr = gather ? buffer_of(x, groups.x_rows * row_bytes) : buffer_of(x + static_cast<size_t>(m0) * k, rows * row_bytes);
     const r_i32x4 wr = buffer_of(w + static_cast<size_t>(n0) * k, (OUT == kRowsGated ? 2 * n - n0 : min(n - n0, BN)) * row_bytes);
     int xo[XL], wo[WL];
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
         const int r = (wave * XL + i) * 8 + lane / 8;
-        xo[i] = min(r, m - m0 - 1) * static_cast<int>(row_bytes) + piece * 16;
+        int g = min(r, rows - 1);
+        if (gather) g = groups.row_token[m0 + g];
+        xo[i] = g * static_cast<int>(row_bytes) + piece * 16;
     }
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
@@ -180,8 +200,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
     // ---- a lane holds columns 4 lg .. 4 lg + 3 of row li of every 16 x 16 tile (n is a multiple of four)
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const int row = m0 + wm * (BM / WM) + i * 16 + li;
-        if (row >= m) continue;
+        const int at = wm * (BM / WM) + i * 16 + li, row = m0 + at;
+        if (at >= rows) continue;
         if constexpr (OUT == kRowsGated) {
 #pragma unroll
             for (int j = 0; j < TN / 2; ++j) {
@@ -202,9 +222,12 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
                     if (col < n) *reinterpret_cast<r_f32x4*>(o) = acc[i][j];
                 } else {
                     bf16_t* o = static_cast<bf16_t*>(out) + static_cast<size_t>(row) * n + col;
+                    r_f32x4 v = acc[i][j];
+                    if constexpr (OUT == kRowsRelu2)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
                     if (col < n)
-                        *reinterpret_cast<r_u16x4*>(o) = r_u16x4{f32_to_bf16_bits(acc[i][j][0]), f32_to_bf16_bits(acc[i][j][1]),
-                                                                 f32_to_bf16_bits(acc[i][j][2]), f32_to_bf16_bits(acc[i][j][3])};
+                        *reinterpret_cast<r_u16x4*>(o) = r_u16x4{f32_to_bf16_bits(v[0]), f32_to_bf16_bits(v[1]), f32_to_bf16_bits(v[2]), f32_to_bf16_bits(v[3])};
                 }
             }
         }
@@ -219,9 +242,25 @@ int launch_rows(const void* x, const void* w, void* out, int m, int n, int k, in
     const dim3 grid(static_cast<unsigned>(mt * nt * splits));
     const auto* xp = static_cast<const bf16_t*>(x);
     const auto* wp = static_cast<const bf16_t*>(w);
-    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsGated><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act);
-    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsF32><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act);
-    else gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsBf16><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act);
+    const Groups none{nullptr, nullptr, 0};
+    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsGated, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsF32, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    else gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsBf16, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    EGPT_CHECK_LAUNCH();
+    return EGPT_OK;
+}
+
+template <int BM, int BN, int WM, int WN, int WB>
+int launch_groups(const void* x, const void* w, void* out, const Groups& g, long tiles, int n, int k, int kind, int act, hipStream_t s) {
+    const long nt = kind == kRowsGated ? (n + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
+    if (tiles * nt > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
+    const unsigned grid = static_cast<unsigned>(tiles * nt);
+    const auto* xp = static_cast<const bf16_t*>(x);
+    const auto* wp = static_cast<const bf16_t*>(w);
+    const int per = k / kRowsStep;
+    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsGated, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
+    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsF32, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
+    else gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsRelu2, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
@@ -232,7 +271,7 @@ using namespace egpt;
 
 extern "C" int egpt_gemm_rows(const void* x, const void* w, void* out, int m, int n, int k, int splits, int kind, int act,
                               int shape, void* stream) {
-    if (!x || !w || !out || m < 0 || n <= 0 || k <= 0 || splits < 1 || kind < 0 || kind > 2 || act < 0 || act > 1) return EGPT_BAD_ARGUMENT;
+    if (!x || !w || !out || m < 0 || n <= 0 || k <= 0 || splits < 1 || kind < 0 || kind > kRowsGated || act < 0 || act > 1) return EGPT_BAD_ARGUMENT;
     if (k % kRowsStep != 0 || n % 4 != 0 || (splits != 1 && kind != kRowsF32)) return EGPT_UNSUPPORTED_SIZE;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16) return EGPT_UNSUPPORTED_SIZE;
     // a lane's byte offsets from its tile's first row are 32-bit numbers
@@ -248,6 +287,26 @@ extern "C" int egpt_gemm_rows(const void* x, const void* w, void* out, int m, in
         case 2: return launch_rows<128, 256, 2, 4, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
         case 3: return launch_rows<128, 128, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
         case 4: return launch_rows<64, 64, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        default: return EGPT_BAD_ARGUMENT;
+    }
+}
+
+extern "C" int egpt_moe_rows(const void* x, const void* w, const int32_t* row_token, const int32_t* tiles, void* out, int n_rows,
+                             int x_rows, int n, int k, int experts, int tile_rows, int kind, int act, void* stream) {
+    if (!x || !w || !tiles || !out || n_rows < 0 || x_rows < 0 || n <= 0 || k <= 0 || experts <= 0 || (!row_token && x_rows != n_rows) ||
+        kind < kRowsF32 || kind > kRowsRelu2 || act < 0 || act > 1)
+        return EGPT_BAD_ARGUMENT;
+    if (k % kRowsStep != 0 || n % 4 != 0) return EGPT_UNSUPPORTED_SIZE;
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16) return EGPT_UNSUPPORTED_SIZE;
+    // byte offsets within x (gathered rows) and within an expert's matrix are 32-bit numbers
+    if (static_cast<long long>(k) * 2 * x_rows > 0x7fffffffLL || static_cast<long long>(k) * 2 * 2 * n > 0x7fffffffLL) return EGPT_UNSUPPORTED_SIZE;
+    if (n_rows == 0) return EGPT_OK;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const Groups g{tiles, row_token, x_rows};
+    const long most = tile_rows > 0 ? n_rows / tile_rows + experts + 1 : 0;
+    switch (tile_rows) {
+        case 64: return launch_groups<64, 64, 2, 2, 3>(x, w, out, g, most, n, k, kind, act, s);
+        case 128: return launch_groups<128, 128, 2, 2, 3>(x, w, out, g, most, n, k, kind, act, s);
         default: return EGPT_BAD_ARGUMENT;
     }
 }

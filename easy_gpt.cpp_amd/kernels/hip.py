@@ -133,6 +133,7 @@ class HipKernels(KernelBackend):
             "egpt_moe_group": [vp, vp, vp, vp, vp, i, i, i, i, vp],
             "egpt_moe_gate_up": [vp, vp, vp, vp, vp, i, i, i, i, i, i, vp],
             "egpt_moe_down": [vp, vp, vp, vp, i, i, i, i, i, i, vp],
+            "egpt_moe_rows": [vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, vp],
             "egpt_moe_combine": [vp, vp, vp, vp, vp, vp, i, i, i, i, vp],
         }
         lib.egpt_scan_key_splits.restype = i
@@ -1571,7 +1572,8 @@ class HipKernels(KernelBackend):
     # ------------------------------------------------------------------ a mixture of experts
     @staticmethod
     def _moe_tile_rows(n_rows: int, experts: int) -> int:
-        """Rows to a tile of the grouped products: 16 while an expert gets few rows, 64 when it gets hundreds."""
+        """Rows to a tile of the grouped products straight from memory: 16 while an expert gets few rows, 64 when it gets
+        hundreds."""
         per_expert = n_rows / max(experts, 1)
         return 16 if per_expert <= 24 else (32 if per_expert <= 96 else 64)
 
@@ -1611,7 +1613,14 @@ class HipKernels(KernelBackend):
             self._need(residual, "residual", _I64, (t, hidden))
         dev = x.device
         n_rows = t * top
-        tile_rows = self._moe_tile_rows(n_rows, experts)
+        # bfloat16 in sizes that gemm_rows.hip takes: its tiles, from the fewest rows on.  Measured against the products straight
+        # from memory (us, gate and up + down product): 16 experts of 896 x 1,024, 32 / 512 / 10,140 rows 12.3 + 8.4 / 17.2 +
+        # 12.2 / 57.8 + 33.1 against 15.0 + 12.3 / 45.3 + 29.2 / 218 + 187; 32 experts of 2,048 x 1,536 75 + 28 / 99 + 43 (1,024
+        # rows) / 200 + 112 against 79 + 40 / 166 + 111 / 734 + 601.  Tiles of 128 rows from 64 rows an expert on (122 + 61 against
+        # 113 + 45 there on the larger experts, 17.2 + 12.2 against 18.0 + 13.4 on the smaller ones).
+        staged = (x.dtype == _BF16 and hidden % 64 == 0 and ff % 64 == 0 and max(t, n_rows) * max(hidden, ff) < 1 << 30
+                  and 2 * ff * hidden < 1 << 29 and (x.data_ptr() | w_gate_up.data_ptr() | w_down.data_ptr()) % 16 == 0)
+        tile_rows = (64 if n_rows < 64 * experts else 128) if staged else self._moe_tile_rows(n_rows, experts)
         chosen = torch.empty((t, top), dtype=_I32, device=dev)
         weight = torch.empty((t, top), dtype=_F32, device=dev)
         row_token = torch.empty((n_rows,), dtype=_I32, device=dev)
@@ -1627,10 +1636,16 @@ class HipKernels(KernelBackend):
                   int(groups), int(keep_groups), int(bool(normalized)), dt, st)
         self._run("egpt_moe_group", chosen.data_ptr(), row_token.data_ptr(), place.data_ptr(), tiles.data_ptr(),
                   counts.data_ptr(), t, top, experts, tile_rows, st)
-        self._run("egpt_moe_gate_up" if gated else "egpt_moe_up", x.data_ptr(), w_gate_up.data_ptr(), row_token.data_ptr(),
-                  tiles.data_ptr(), act.data_ptr(), n_rows, hidden, ff, experts, tile_rows, dt, st)
-        self._run("egpt_moe_down", act.data_ptr(), w_down.data_ptr(), tiles.data_ptr(), y.data_ptr(), n_rows, hidden, ff,
-                  experts, tile_rows, dt, st)
+        if staged:
+            self._run("egpt_moe_rows", x.data_ptr(), w_gate_up.data_ptr(), row_token.data_ptr(), tiles.data_ptr(), act.data_ptr(),
+                      n_rows, t, ff, hidden, experts, tile_rows, 2 if gated else 3, 0, st)
+            self._run("egpt_moe_rows", act.data_ptr(), w_down.data_ptr(), None, tiles.data_ptr(), y.data_ptr(), n_rows, n_rows,
+                      hidden, ff, experts, tile_rows, 1, 0, st)
+        else:
+            self._run("egpt_moe_gate_up" if gated else "egpt_moe_up", x.data_ptr(), w_gate_up.data_ptr(), row_token.data_ptr(),
+                      tiles.data_ptr(), act.data_ptr(), n_rows, hidden, ff, experts, tile_rows, dt, st)
+            self._run("egpt_moe_down", act.data_ptr(), w_down.data_ptr(), tiles.data_ptr(), y.data_ptr(), n_rows, hidden, ff,
+                      experts, tile_rows, dt, st)
         self._run("egpt_moe_combine", y.data_ptr(), x.data_ptr(), place.data_ptr(), weight.data_ptr(), self._ptr(out),
                   self._ptr(residual), t, top, hidden, dt, st)
         return out if residual is None else residual

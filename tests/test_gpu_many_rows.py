@@ -78,3 +78,43 @@ def test_the_norm_adds_partial_sums_of_many_rows(k):
         some = torch.empty((t + 1, hidden), dtype=torch.bfloat16, device="cuda")
         k.rows_add_rmsnorm(h, delta, rows, weight, 1e-6, some)
         assert torch.equal(some, out[rows.long()])
+
+
+@pytest.mark.parametrize("tile_rows", [64, 128])
+@pytest.mark.parametrize("t,top,experts,outputs,hidden,ff", [(1, 1, 1, 1, 64, 64), (5, 3, 4, 6, 128, 64), (150, 2, 5, 7, 64, 192),
+                                                             (130, 1, 3, 3, 192, 128), (40, 4, 700, 1000, 64, 64)])
+def test_rows_grouped_by_expert(k, tile_rows, t, top, experts, outputs, hidden, ff):
+    """Choices from `experts` on have no row; with few choices most experts have none, with one expert in use whole tiles."""
+    g = torch.Generator().manual_seed(t)
+    chosen = torch.stack([torch.randperm(outputs, generator=g)[:top] for _ in range(t)]).int().cuda()
+    if experts == 3:
+        chosen[:] = 1
+    x, w, down = rnd(t, hidden, seed=1), rnd(experts, 2 * ff, hidden, seed=2, scale=0.2), rnd(experts, hidden, ff, seed=3, scale=0.2)
+    n = t * top
+    new = lambda *shape, dtype=torch.int32: torch.full(shape, -7, dtype=dtype, device="cuda")  # noqa: E731
+    row_token, place, counts, tiles = new(n), new(t, top), new(experts), new(1 + 3 * (n // tile_rows + experts + 1))
+    k._run("egpt_moe_group", chosen.data_ptr(), row_token.data_ptr(), place.data_ptr(), tiles.data_ptr(), counts.data_ptr(), t, top,
+           experts, tile_rows, k._stream())
+    flat = chosen.view(-1).long().cpu()
+    kept = flat < experts
+    assert torch.equal(counts.cpu().long(), torch.bincount(flat[kept], minlength=experts))
+    rows = place.view(-1).cpu().long()
+    assert (rows[~kept] == -1).all() and torch.equal(rows[kept].sort().values, torch.arange(int(kept.sum())))
+    assert torch.equal(row_token.cpu().long()[rows[kept]], torch.arange(n)[kept] // top)
+    table = tiles[1 : 1 + 3 * int(tiles[0])].view(-1, 3).cpu()
+    assert int(table[:, 2].sum()) == int(kept.sum()) and int(tiles[0]) == int(((counts.cpu() + tile_rows - 1) // tile_rows).sum())
+    x64, w64, d64 = x.double().cpu(), w.double().cpu(), down.double().cpu()
+    for kind in (2, 3):
+        act, y = new(n, ff, dtype=torch.bfloat16), new(n, hidden, dtype=torch.float32)
+        wk = w if kind == 2 else w[:, :ff].contiguous()
+        k._run("egpt_moe_rows", x.data_ptr(), wk.data_ptr(), row_token.data_ptr(), tiles.data_ptr(), act.data_ptr(), n, t, ff, hidden,
+               experts, tile_rows, kind, 0, k._stream())
+        k._run("egpt_moe_rows", act.data_ptr(), down.data_ptr(), None, tiles.data_ptr(), y.data_ptr(), n, n, hidden, ff, experts,
+               tile_rows, 1, 0, k._stream())
+        for i in kept.nonzero().view(-1).tolist():
+            e, r = int(flat[i]), int(rows[i])
+            z = w64[e] @ x64[i // top]
+            want = z[:ff] * torch.sigmoid(z[:ff]) * z[ff:] if kind == 2 else z[:ff].clamp(min=0) ** 2
+            assert ((act[r].double().cpu() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-4).all()
+            full = d64[e] @ act[r].double().cpu()
+            assert ((y[r].double().cpu() - full).abs() <= 1e-5 * (d64[e].abs() @ act[r].double().cpu().abs()) + 1e-6).all()
