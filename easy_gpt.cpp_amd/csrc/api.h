@@ -48,10 +48,15 @@ int egpt_gemm_skinny(const void* x, const void* w, const void* bias, float* out_
 // egpt_swiglu).  shape: the tile (0 to 4).  k % 64 == 0, n % 4 == 0, operands on 16 bytes.
 int egpt_gemm_rows(const void* x, const void* w, void* out, int m, int n, int k, int n_splits, int kind, int act, int shape,
                    void* stream);
-// float32 product on the matrix cores (float32 operands and accumulation): out [n_splits][m][n] are partial sums over
-// n_splits ranges of k (bias only with one).  k % 4 == 0.  A row's values do not depend on m or on the other rows.
+// float32 product on the matrix cores (float32 operands as three bfloat16 numbers each, float32 accumulation, see gemm.hip):
+// out [n_splits][m][n] are partial sums over n_splits ranges of k (bias only with one).  k % 4 == 0.  A row's values do not
+// depend on m or on the other rows.
 int egpt_gemm_f32(const float* x, const float* w, const float* bias, float* out, int m, int n, int k, int n_splits,
                   void* stream);
+// The same values for many rows, in tiles of tile_rows (64 or 128) rows; fold != 0: out [m][n] is the sum of the partial sums in
+// their order.
+int egpt_gemm_f32_rows(const float* x, const float* w, const float* bias, float* out, int m, int n, int k, int n_splits, int fold,
+                       int tile_rows, void* stream);
 // out = x w^T + bias; x [m,k], w [n,k], out [m,n]; out_f32 != 0 writes float32 whatever dtype is.
 int egpt_linear(const void* x, const void* w, const void* bias, void* out, int m, int n, int k, int dtype,
                 int out_f32, void* stream);

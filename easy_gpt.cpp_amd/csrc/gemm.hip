@@ -1,9 +1,8 @@
 // out[m, n] = sum_k x[m, k] * w[n, k] + bias[n]: the linear layer y = x W^T + b with W stored [out, in]
 // (/root/reference/src/ops.cpp:101-118).
 //
-// gemm_tiled: plain FMA tiles in float32 arithmetic for every element type.  It is the product
-// path for float32 (true 32-bit: no reduced-precision matrix mode) and the fallback for sizes the
-// MFMA kernels refuse.
+// gemm_tiled: plain FMA tiles in float32 arithmetic for every element type, the fallback for sizes the MFMA kernels refuse.
+// gemm_f32_mfma, gemm_f32_rows: the float32 product on the matrix cores, for few rows and for many.
 #include "api.h"
 #include "common.h"
 
@@ -71,109 +70,384 @@ int launch_tiled(const void* x, const void* w, const void* bias, void* out, int 
 }
 
 // ----------------------------------------------------------------------------- float32 on the matrix cores
-// The float32 product: v_mfma_f32_16x16x4_f32 takes float32 operands and accumulates in float32 (no reduced-precision
-// matrix mode).  A wavefront owns 16 rows of w (16 columns of the result) and streams them once for up to 64 rows of
-// x, which the workgroup's four wavefronts share through LDS; more rows are further groups of 64 (blockIdx.z), the k
-// range may be split over workgroups (blockIdx.y) into partial sums out[split][m][n].  Every element of the result is
-// the same sequence of operations whatever m is and wherever its row lies in x: a step of 64 after the other, within
-// a step one instruction after the other, each adding the products of four values of k.  So a token's values do not
+// The float32 product on the bfloat16 matrix instructions, with no less than float32's precision: every operand is the sum of three
+// bfloat16 numbers, x = h + m + l, each the nearest to what the ones before leave (8 + 8 + 8 bits: nothing is left), and of
+// the nine products the six largest are added up; the three others are below 2^-25 of the product and of either sign.  The
+// six products of a block of 32 values of k are one chain of v_mfma_f32_16x16x32_bf16 that begins at zero, and the block's sum
+// is added to the element's in float32.  Error against 64 bits (2-norm, normal operands, k = 896 / 4,864): 1.1e-7 / 2.4e-7,
+// with v_mfma_f32_16x16x4_f32, which took its operands as they are and rounded after every fourth product, 5.4e-7 / 1.25e-6; with
+// one chain over all blocks 4.5e-7 / 1.1e-6.
+// Values that have no such three parts (infinities, NaN, beyond the largest bfloat16) and overflows on the way leave an
+// element that is no finite number: it is then added up again in plain float32, so it comes out as it did.
+//
+// Every element of the result is the same sequence of operations whatever m is and wherever its row lies in x, in all
+// kernels here: block after block of 32 values within a range of k, ranges of k one after the other.  So a token's values do not
 // depend on what else is in the batch, to the bit.
-constexpr int kStepF = 64;            // values of k per step
-constexpr int kLdsRowF = kStepF + 4;  // floats per staged row of x (16 bytes of padding)
+constexpr int kBlockF = 32;                   // values of k per block
+constexpr int kStepF = 64;                    // ranges of k are multiples of this
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 f_bf16x8;
 
-template <int MT>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
+struct Parts {                                // eight values of k as three bfloat16 numbers each
+    f_bf16x8 h, m, l;
+};
+typedef __attribute__((ext_vector_type(2))) __bf16 f_bf16x2;
+// What is left of two values when a pair of bfloat16 numbers is taken away: one instruction each (a dot product with -1 and
+// 0, exact here) instead of a conversion and a subtraction.  The constants stand in registers: as an inline constant
+// -1.0 would be float32's, whose bfloat16 pair is (0, -1).
+__device__ __forceinline__ void take_away(f_bf16x2 pair, float& a, float& b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    unsigned low = 0x0000bf80u, high = 0xbf800000u;
+    asm("" : "+s"(low), "+s"(high));
+    a = __builtin_amdgcn_fdot2_f32_bf16(pair, __builtin_bit_cast(f_bf16x2, low), a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(pair, __builtin_bit_cast(f_bf16x2, high), b, false);
+#endif
+}
+__device__ __forceinline__ Parts split_parts(const f32x4& a, const f32x4& b) {
+    Parts p;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        float x = i < 4 ? a[i] : b[i - 4], y = i < 4 ? a[i + 1] : b[i - 3];
+        f_bf16x2 h{static_cast<__bf16>(x), static_cast<__bf16>(y)};
+        take_away(h, x, y);
+        f_bf16x2 m{static_cast<__bf16>(x), static_cast<__bf16>(y)};
+        take_away(m, x, y);
+        p.h[i] = h[0], p.h[i + 1] = h[1];
+        p.m[i] = m[0], p.m[i + 1] = m[1];
+        p.l[i] = static_cast<__bf16>(x), p.l[i + 1] = static_cast<__bf16>(y);
+    }
+    return p;
+}
+// The sums of N blocks, w[j] with x[j] (or with x[0], X = 1), as chains that go forward side by side: a product waits for the
+// one before it in its chain, not for its neighbours.
+template <int N, int X>
+__device__ __forceinline__ void block_sums(const Parts* w, const Parts* x, f32x4* t) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].l, x[j % X].h, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].h, x[j % X].l, t[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].m, x[j % X].m, t[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].m, x[j % X].h, t[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].h, x[j % X].m, t[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].h, x[j % X].h, t[j], 0, 0, 0);
+}
+// An element over values [k0, k1) of k in plain float32, where the parts' sum is no finite number.
+__device__ __noinline__ float plain_sum(const float* x, const float* w, int k0, int k1) {
+    float v = 0.f;
+    for (int i = k0; i < k1; ++i) v = fmaf(w[i], x[i], v);
+    return v;
+}
+__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+
+// Up to 64 rows of x to a workgroup (further groups of rows: blockIdx.z).  A wavefront owns 16 rows of w (16 columns of the
+// result) and streams them once, as they are (four steps of 64 values ahead: with few rows the kernel is a stream of w, and a
+// stream one step deep was a chain of round trips, 1.1 TB/s on a 17 MB matrix), and splits them in registers; the rows of x
+// are split on their way to LDS, CH steps at a time, and shared by the wavefronts: four steps for up to 16 rows, where a barrier
+// a step was a quarter of the time of a short range, one for more rows, whose LDS would keep workgroups off a CU.  A lane's four
+// values of a row of the result are one store (as four they cost 64 rows of 9,728 columns 2.6 us of 25.7).  The k range may be
+// split over workgroups (blockIdx.y) into partial sums out[split][m][n].
+// us for 8 / 64 rows, each with the ranges that the callers take: 1,152 x 896 4.8 / 8.3, 9,728 x 896 11.3 / 23.1, 896 x 4,864 10.1 /
+// 17.7, 151,936 x 896 109 / 184; with v_mfma_f32_16x16x4_f32 4.8 / 8.5, 12.9 / 23.6, 10.6 / 18.5 and 114 / 210.
+
+template <int MT, int CH, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const float* __restrict__ bias, float* __restrict__ out,
                                                             int m, int n, int k, int steps_per_split) {
-    __shared__ __attribute__((aligned(16))) float xs[2][MT * 16][kLdsRowF];
+    __shared__ __attribute__((aligned(16))) __bf16 xs[2][3][MT * 16][CH * kStepF + 8];   // (16 bytes of padding to a row)
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int li = lane % 16, lg = lane / 16;
     const int split = blockIdx.y;
     const int m0 = blockIdx.z * 64;                       // first row of this group
-    const int n0 = (blockIdx.x * 4 + wave) * 16;
+    const int n0 = (blockIdx.x * NW + wave) * 16;
     const int total_steps = (k + kStepF - 1) / kStepF;
     const int step_begin = split * steps_per_split;
     const int step_end = min(total_steps, step_begin + steps_per_split);
-    // lane (li, lg) of a load takes the lg-th 16 bytes of each 64 of row li: an instruction reads 64 contiguous bytes
-    // of each of its 16 rows; the j-th of its four values goes into the j-th product instruction, x likewise
-    const float* wp = w + static_cast<size_t>(min(n0 + li, n - 1)) * k + lg * 4;
+    // lane (li, lg) takes eight values of row li per block of 32: 128 contiguous bytes of each row an instruction pair
+    const float* wp = w + static_cast<size_t>(min(n0 + li, n - 1)) * k + lg * 8;
     auto load_w = [&](f32x4* av, int step) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int k0 = step * kStepF + q * 16 + lg * 4;
-            av[q] = k0 < k ? *reinterpret_cast<const f32x4*>(wp + static_cast<size_t>(step) * kStepF + q * 16)
-                           : f32x4{0.f, 0.f, 0.f, 0.f};
+            const int at = step * kStepF + q / 2 * kBlockF + q % 2 * 4;
+            av[q] = at + lg * 8 < k ? *reinterpret_cast<const f32x4*>(wp + at) : f32x4{0.f, 0.f, 0.f, 0.f};
         }
     };
-    float4 xr[MT];
-    auto x_load = [&](int step) {
+    // eight values of a row of x per thread and load: MT * 16 rows x 8 * CH pieces
+    constexpr int PC = CH * 8, XP = MT * 16 * PC, XN = (XP + NW * 64 - 1) / (NW * 64);
+    constexpr int XS = CH == 1 ? 2 : 1;                   // stagings on their way
+    f32x4 xr[XS][XN][2];
+    auto x_load = [&](int set, int step) {
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const int c = tid + j * 256, r = m0 + c / 16, kc = step * kStepF + (c % 16) * 4;
-            xr[j] = (r < m && kc < k) ? *reinterpret_cast<const float4*>(x + static_cast<size_t>(r) * k + kc)
-                                      : float4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < XN; ++j) {
+            const int c = tid + j * NW * 64, r = m0 + c / PC, kc = step * kStepF + c % PC * 8;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                xr[set][j][u] = (c < XP && r < m && kc + u * 4 < k)
+                                    ? *reinterpret_cast<const f32x4*>(x + static_cast<size_t>(r) * k + kc + u * 4)
+                                    : f32x4{0.f, 0.f, 0.f, 0.f};
         }
     };
-    auto x_store = [&](int buf) {
+    auto x_store = [&](int set, int buf) {
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const int c = tid + j * 256;
-            *reinterpret_cast<float4*>(&xs[buf][c / 16][(c % 16) * 4]) = xr[j];
+        for (int j = 0; j < XN; ++j) {
+            const int c = tid + j * NW * 64;
+            if (c >= XP) break;
+            const Parts p = split_parts(xr[set][j][0], xr[set][j][1]);
+            *reinterpret_cast<f_bf16x8*>(&xs[buf][0][c / PC][c % PC * 8]) = p.h;
+            *reinterpret_cast<f_bf16x8*>(&xs[buf][1][c / PC][c % PC * 8]) = p.m;
+            *reinterpret_cast<f_bf16x8*>(&xs[buf][2][c / PC][c % PC * 8]) = p.l;
         }
     };
     f32x4 acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // w runs kAhead steps ahead of the products (16 KB per wavefront on their way: with few rows the kernel is a
-    // stream of w, and a stream one step deep was a chain of round trips, 1.1 TB/s on a 17 MB matrix); the order of
-    // the products, and so every bit of the result, is that of the steps
     constexpr int kAhead = 4;
     f32x4 a[kAhead][4];     // (a native vector type: arrays of it stay in registers across the loop's back edge)
+    x_load(0, step_begin);
+    if (XS > 1 && step_begin + CH < step_end) x_load(XS - 1, step_begin + CH);
 #pragma unroll
     for (int u = 0; u < kAhead; ++u)
         if (step_begin + u < step_end) load_w(a[u], step_begin + u);
-    if (step_begin < step_end) {
-        x_load(step_begin);
-        x_store(0);
-        if (step_begin + 1 < step_end) x_load(step_begin + 1);
-    }
+    x_store(0, 0);
+    if (step_begin + XS * CH < step_end) x_load(0, step_begin + XS * CH);
     __syncthreads();
     for (int step0 = step_begin; step0 < step_end; step0 += kAhead) {
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {
             const int step = step0 + u;
             if (step >= step_end) break;
-            const int buf = u & 1;                  // (step - step_begin) & 1: kAhead is even
+            // (kAhead is a multiple of CH; of 2 * CH it is not where a staging is four steps: the count of stagings then)
+            const int buf = CH * 2 <= kAhead ? u / CH & 1 : (step0 - step_begin) / CH & 1;
+            const int in = u % CH * kStepF;
+            const Parts wv[2] = {split_parts(a[u][0], a[u][1]), split_parts(a[u][2], a[u][3])};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float av[4] = {a[u][q][0], a[u][q][1], a[u][q][2], a[u][q][3]};
+            for (int t = 0; t < MT; ++t) {
+                Parts xv[2];
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const float4 b4 = *reinterpret_cast<const float4*>(&xs[buf][t * 16 + li][q * 16 + lg * 4]);
-                    const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], acc[t], 0, 0, 0);
+                for (int q = 0; q < 2; ++q) {
+                    xv[q].h = *reinterpret_cast<const f_bf16x8*>(&xs[buf][0][t * 16 + li][in + q * kBlockF + lg * 8]);
+                    xv[q].m = *reinterpret_cast<const f_bf16x8*>(&xs[buf][1][t * 16 + li][in + q * kBlockF + lg * 8]);
+                    xv[q].l = *reinterpret_cast<const f_bf16x8*>(&xs[buf][2][t * 16 + li][in + q * kBlockF + lg * 8]);
                 }
+                f32x4 sums[2];
+                block_sums<2, 2>(wv, xv, sums);
+                acc[t] += sums[0];
+                acc[t] += sums[1];
             }
             if (step + kAhead < step_end) load_w(a[u], step + kAhead);
-            if (step + 1 < step_end) x_store(buf ^ 1);
-            if (step + 2 < step_end) x_load(step + 2);
-            __syncthreads();
+            if ((u + 1) % CH == 0 && step + 1 < step_end) {
+                const int set = (u + 1) & (XS - 1);
+                x_store(set, buf ^ 1);
+                if (step + 1 + XS * CH < step_end) x_load(set, step + 1 + XS * CH);
+                __syncthreads();
+            }
         }
     }
     // D layout: lane (li, lg) holds rows lg*4 + v of the 16 x 16 tile (an n index) at column li (an m index)
+    const bool whole = n % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;   // four values are one store
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        const int mm = m0 + t * 16 + li;
-        if (mm >= m) continue;
+        const int mm = m0 + t * 16 + li, nn = n0 + lg * 4;
+        if (mm >= m || nn >= n) continue;
+        f32x4 val = acc[t];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int nn = n0 + lg * 4 + v;
-            if (nn >= n) continue;
-            float val = acc[t][v];
-            if (bias) val += bias[nn];
-            out[(static_cast<size_t>(split) * m + mm) * n + nn] = val;
+            if (nn + v >= n) continue;
+            if (!finite(val[v]))
+                val[v] = plain_sum(x + static_cast<size_t>(mm) * k, w + static_cast<size_t>(nn + v) * k, step_begin * kStepF, min(k, step_end * kStepF));
+            if (bias) val[v] += bias[nn + v];
+        }
+        float* to = out + (static_cast<size_t>(split) * m + mm) * n + nn;
+        if (whole) {
+            *reinterpret_cast<f32x4*>(to) = val;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (nn + v < n) to[v] = val[v];
+        }
+    }
+}
+
+// Many rows of x: tiles of 128 rows of x and 128 of w, both split on their way to LDS (a thread eight values of each a block, loaded
+// two blocks ahead), eight wavefronts of 32 x 64.  A block's parts lie in LDS as rows of 64 bytes whose four pieces of 16
+// bytes are exchanged by the row's number (piece p of row r in place p ^ (r / 2 & 3)), so that the lanes that read one
+// piece of many rows hit different banks; two buffers, one barrier a block.
+// FOLD: a workgroup walks all ranges of k and adds their sums up in their order, which is what a reader of partial sums does:
+// the same bits, without the partial sums' traffic.
+// TAIL: k is no multiple of a block (its end is filled with zeros).
+template <int WM, bool FOLD, bool TAIL>
+__global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                            const float* __restrict__ bias, float* __restrict__ out,
+                                                            int m, int n, int k, int blocks_per_split) {
+    constexpr int TM = 2, TN = 4;                          // 16 x 16 tiles of a wavefront
+    constexpr int BM = WM * 32, NT = WM * 128, WL = 512 / NT;   // rows of x; threads; pieces of w that a thread stages
+    constexpr int kPartX = BM * 64, kPartW = 128 * 64;     // bytes of a part of an operand's block
+    __shared__ __attribute__((aligned(128))) char lds[2][3 * (kPartX + kPartW)];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int li = lane % 16, lg = lane / 16;
+    const int wm = wave % WM, wn = wave / WM;
+    // a die gets a contiguous range of tiles, rows of x fastest
+    const int mt = (m + BM - 1) / BM, tiles = mt * ((n + 127) / 128);
+    int tile = blockIdx.x;
+    {
+        const int q = tiles / 8, r = tiles % 8, d = tile % 8, i = tile / 8;
+        tile = d * q + (d < r ? d : r) + i;
+    }
+    const int m0 = tile % mt * BM, n0 = tile / mt * 128;
+    const int total = (k + kBlockF - 1) / kBlockF;
+    const int first = FOLD ? 0 : blockIdx.y * blocks_per_split;
+    const int last = FOLD ? total : min(total, first + blocks_per_split);
+    // ---- staging: a thread's row and its eight values of k
+    const int srow = tid / 4, piece = tid % 4;
+    const float* xp = x + static_cast<size_t>(min(m0 + srow, m - 1)) * k + piece * 8;
+    const float* wp[WL];
+#pragma unroll
+    for (int o = 0; o < WL; ++o) wp[o] = w + static_cast<size_t>(min(n0 + srow + o * (NT / 4), n - 1)) * k + piece * 8;
+    f32x4 raw[2][1 + WL][2];                               // [set][x, w ..][halves]
+    auto load = [&](int set, int block) {                  // (beyond the last block the last one again, which nobody reads)
+        const int at = min(block, last - 1) * kBlockF;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool in = !TAIL || at + piece * 8 + u * 4 < k;
+            const int offset = in ? at + u * 4 : -piece * 8;
+            raw[set][0][u] = *reinterpret_cast<const f32x4*>(xp + offset);
+#pragma unroll
+            for (int o = 0; o < WL; ++o) raw[set][1 + o][u] = *reinterpret_cast<const f32x4*>(wp[o] + offset);
+            if (TAIL && !in)
+#pragma unroll
+                for (int o = 0; o < 1 + WL; ++o) raw[set][o][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    const int place = srow * 64 + (piece ^ (srow / 2 & 3)) * 16;          // (the same for srow + a multiple of 8)
+    auto store = [&](int set, int buf) {
+#pragma unroll
+        for (int o = 0; o < 1 + WL; ++o) {
+            const Parts p = split_parts(raw[set][o][0], raw[set][o][1]);
+            char* to = lds[buf] + (o == 0 ? place : 3 * kPartX + place + (o - 1) * (NT / 4) * 64);
+            constexpr int parts[2] = {kPartX, kPartW};
+            *reinterpret_cast<f_bf16x8*>(to) = p.h;
+            *reinterpret_cast<f_bf16x8*>(to + parts[o > 0]) = p.m;
+            *reinterpret_cast<f_bf16x8*>(to + 2 * parts[o > 0]) = p.l;
+        }
+    };
+    const int read_at = li * 64 + (lg ^ (li / 2 & 3)) * 16;
+    auto piece_of = [&](const char* from) { return *reinterpret_cast<const f_bf16x8*>(from); };
+    f32x4 acc[TM][TN], sum[FOLD ? TM : 1][FOLD ? TN : 1];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (FOLD) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    const int row0 = m0 + wm * 32 + li, col0 = n0 + wn * 64 + lg * 4;
+    // the end of a range [b0, b1) of blocks: elements that are no finite number are added up again
+    auto mend = [&](int b0, int b1) {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) bad |= !finite(acc[i][j][v]);
+        if (!__any(bad)) return;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int row = row0 + i * 16, col = col0 + j * 16 + v;
+                    if (!finite(acc[i][j][v]) && row < m && col < n)
+                        acc[i][j][v] = plain_sum(x + static_cast<size_t>(row) * k, w + static_cast<size_t>(col) * k, b0 * kBlockF, min(k, b1 * kBlockF));
+                }
+    };
+    load(0, first);
+    load(1, first + 1);
+    store(0, 0);
+    load(0, first + 2);
+    int range_begin = first, in_range = 0;
+#pragma unroll 1
+    for (int b0 = first; b0 < last; b0 += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int b = b0 + u;
+            if (b >= last) break;
+            __syncthreads();                               // block b is in buffer u, buffer 1 - u has been read
+            // block b + 1 is split by one of the two wavefronts of a SIMD before its products and by the other behind them:
+            // the vector unit and the matrix cores work at the same time
+            if (wn == 0) {
+                store(1 - u, 1 - u);
+                load(1 - u, b + 3);
+            }
+            const char* xs = lds[u] + wm * 2048 + read_at;
+            const char* ws = lds[u] + 3 * kPartX + wn * 4096 + read_at;
+            Parts wv[TN], xv[TM];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wv[j].h = piece_of(ws + j * 1024);
+            xv[0].h = piece_of(xs);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wv[j].m = piece_of(ws + j * 1024 + kPartW);
+            xv[0].m = piece_of(xs + kPartX);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wv[j].l = piece_of(ws + j * 1024 + 2 * kPartW);
+            xv[0].l = piece_of(xs + 2 * kPartX);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                if (i + 1 < TM) {
+                    xv[i + 1].h = piece_of(xs + (i + 1) * 1024);
+                    xv[i + 1].m = piece_of(xs + (i + 1) * 1024 + kPartX);
+                    xv[i + 1].l = piece_of(xs + (i + 1) * 1024 + 2 * kPartX);
+                }
+                f32x4 sums[TN];
+                block_sums<TN, 1>(wv, &xv[i], sums);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] += sums[j];
+            }
+            if (wn == 1) {
+                store(1 - u, 1 - u);
+                load(1 - u, b + 3);
+            }
+            if (FOLD && (++in_range == blocks_per_split || b + 1 == last)) {
+                mend(range_begin, b + 1);
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        sum[i][j] += acc[i][j];
+                        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                range_begin = b + 1;
+                in_range = 0;
+            }
+        }
+    }
+    if (!FOLD) mend(first, last);
+    float* to = out + (FOLD ? 0 : static_cast<size_t>(blockIdx.y) * m * n);
+    const bool whole = n % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;   // four values are one store
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int row = row0 + i * 16;
+        if (row >= m) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = col0 + j * 16;
+            if (col >= n) continue;
+            f32x4 val = FOLD ? sum[FOLD ? i : 0][FOLD ? j : 0] : acc[i][j];
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (bias && col + v < n) val[v] += bias[col + v];
+            float* at = to + static_cast<size_t>(row) * n + col;
+            if (whole) {
+                *reinterpret_cast<f32x4*>(at) = val;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (col + v < n) at[v] = val[v];
+            }
         }
     }
 }
@@ -192,14 +466,57 @@ extern "C" int egpt_gemm_f32(const float* x, const float* w, const float* bias, 
     if (n_splits > total_steps || (n_splits - 1) * steps_per_split >= total_steps) return EGPT_BAD_ARGUMENT;   // an empty split
     const long groups = (static_cast<long>(m) + 63) / 64;
     if (groups > 65535 || n_splits > 65535) return EGPT_UNSUPPORTED_SIZE;
-    const dim3 grid(static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>(n_splits), static_cast<unsigned>(groups));
+    // Two wavefronts to a workgroup instead of four while twice the workgroups still are about one to a CU: the stream of w then
+    // comes through more CUs (8 rows, us with two / four: 4.8 / 5.0 for 1,152 x 896 in 7 ranges, 126 workgroups of four; 11.7 / 10.1
+    // for 896 x 4,864 in 11, 154).
+    const bool two = (n + 63) / 64 * static_cast<long>(n_splits) * groups < 130;
+    const unsigned cols = two ? 32 : 64;
+    const dim3 grid((n + cols - 1) / cols, static_cast<unsigned>(n_splits), static_cast<unsigned>(groups));
     hipStream_t s = static_cast<hipStream_t>(stream);
+#define EGPT_F32(MT_, CH_)                                                                                             \
+    do {                                                                                                               \
+        if (two) gemm_f32_mfma_kernel<MT_, CH_, 2><<<grid, 128, 0, s>>>(x, w, bias, out, m, n, k, steps_per_split);    \
+        else gemm_f32_mfma_kernel<MT_, CH_, 4><<<grid, 256, 0, s>>>(x, w, bias, out, m, n, k, steps_per_split);        \
+    } while (0)
     switch (m > 64 ? 4 : (m + 15) / 16) {
-        case 1: gemm_f32_mfma_kernel<1><<<grid, 256, 0, s>>>(x, w, bias, out, m, n, k, steps_per_split); break;
-        case 2: gemm_f32_mfma_kernel<2><<<grid, 256, 0, s>>>(x, w, bias, out, m, n, k, steps_per_split); break;
-        case 3: gemm_f32_mfma_kernel<3><<<grid, 256, 0, s>>>(x, w, bias, out, m, n, k, steps_per_split); break;
-        default: gemm_f32_mfma_kernel<4><<<grid, 256, 0, s>>>(x, w, bias, out, m, n, k, steps_per_split); break;
+        case 1:                                           // (a range of two steps has no use for registers and LDS of four)
+            if (steps_per_split <= 2) EGPT_F32(1, 2);
+            else EGPT_F32(1, 4);
+            break;
+        case 2: EGPT_F32(2, 1); break;
+        case 3: EGPT_F32(3, 1); break;
+        default: EGPT_F32(4, 1); break;
     }
+#undef EGPT_F32
+    EGPT_CHECK_LAUNCH();
+    return EGPT_OK;
+}
+
+extern "C" int egpt_gemm_f32_rows(const float* x, const float* w, const float* bias, float* out, int m, int n, int k,
+                                  int n_splits, int fold, int tile_rows, void* stream) {
+    if (!x || !w || !out || m < 0 || n <= 0 || k <= 0 || n_splits < 1) return EGPT_BAD_ARGUMENT;
+    if (k % 4 != 0 || (bias && n_splits != 1)) return EGPT_UNSUPPORTED_SIZE;
+    if (m == 0) return EGPT_OK;
+    const int total_steps = (k + kStepF - 1) / kStepF;
+    const int steps_per_split = (total_steps + n_splits - 1) / n_splits;
+    if (n_splits > total_steps || (n_splits - 1) * steps_per_split >= total_steps) return EGPT_BAD_ARGUMENT;   // an empty split
+    if (tile_rows != 64 && tile_rows != 128) return EGPT_BAD_ARGUMENT;
+    const long tiles = ((static_cast<long>(m) + tile_rows - 1) / tile_rows) * ((n + 127) / 128);
+    if (tiles > 0x7fffffffL || n_splits > 65535) return EGPT_UNSUPPORTED_SIZE;
+    const int per = steps_per_split * (kStepF / kBlockF);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool folded = fold && n_splits > 1, tail = k % kBlockF != 0;
+    const dim3 grid(static_cast<unsigned>(tiles), folded ? 1u : static_cast<unsigned>(n_splits));
+#define EGPT_F32_ROWS(WM_)                                                                                                  \
+    do {                                                                                                                    \
+        if (folded && tail) gemm_f32_rows_kernel<WM_, true, true><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);       \
+        else if (folded) gemm_f32_rows_kernel<WM_, true, false><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);         \
+        else if (tail) gemm_f32_rows_kernel<WM_, false, true><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);           \
+        else gemm_f32_rows_kernel<WM_, false, false><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);                    \
+    } while (0)
+    if (tile_rows == 128) EGPT_F32_ROWS(4);
+    else EGPT_F32_ROWS(2);
+#undef EGPT_F32_ROWS
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }

@@ -94,6 +94,7 @@ class HipKernels(KernelBackend):
                                             i, i, f, i, i, i, i, i, vp],
             "egpt_linear": [vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_f32": [vp, vp, vp, vp, i, i, i, i, vp],
+            "egpt_gemm_f32_rows": [vp, vp, vp, vp, i, i, i, i, i, i, vp],
             "egpt_gemm_skinny": [vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_rows": [vp, vp, vp, i, i, i, i, i, i, i, vp],
             "egpt_paged_attention": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp],
@@ -382,8 +383,7 @@ class HipKernels(KernelBackend):
             return out
         if x.dtype == _F32 and k % 4 == 0:
             # the float32 product on the matrix cores, the whole k range in one piece
-            self._run("egpt_gemm_f32", x.data_ptr(), w.data_ptr(), self._ptr(bias), out.data_ptr(), m, n, k, 1,
-                      self._stream())
+            self._f32_product(x, w, bias, out, 1, self._f32_rows_plan(m, n, k, 1))
             return out
         self._run("egpt_linear", x.data_ptr(), w.data_ptr(), self._ptr(bias), out.data_ptr(), m, n, k, dt,
                   1 if out.dtype == _F32 else 0, self._stream())
@@ -395,12 +395,41 @@ class HipKernels(KernelBackend):
         The count depends on the matrix alone, never on the rows, so that a row's partial sums, and with them
         every value of the 32-bit path, are the same bits in whatever batch the row is computed."""
         steps = -(-k // 64)
-        # at most 12 ranges: a step of few rows wants many workgroups, a prompt pays for every range with a float32
-        # copy of its output (measured at the 0.5B sizes, decode step at batch 8 / 2,048-token prefill: 1.73 / 24.4 ms
-        # with at most 8 ranges, 1.65 / 24.6 with 12, 1.58 / 26.5 with 16)
-        s = min(steps, max(1, 512 // -(-n // 64)), 12)
+        # (9,728 x 896 in 3 / 4 / 5 ranges, us: 12.8 / 11.6 / 11.3 for 8 rows, 21.1 / 24.1 / 23.1 for 64; prompts of many rows have
+        # their ranges added up inside the kernel)
+        s = min(steps, max(1, 768 // -(-n // 64)), 12)
         per = -(-steps // s)
         return -(-steps // per)
+
+    @staticmethod
+    def _f32_rows_plan(m: int, n: int, k: int, s: int) -> tuple[int, bool]:
+        """(rows of a tile, ranges of k added up inside) of the float32 product; 0 rows: the kernel for few rows.  All of them
+        give the same bits.  Costs in us, fitted to 64 to 1,811 rows of 1,152 x 896, 9,728 x 896 and 896 x 4,864 (in 7, 5 and 11
+        ranges): a CU holds one workgroup, which takes 5 us and 0.9 per block of 32 values of k for 64 x 128, 7 and 1.25 for
+        128 x 128; the kernel for few rows takes 1.85 per group of 64 rows and million elements of w and writes at 2.75
+        TB/s; partial sums are written and read at 4.5 TB/s.  (24 layers of these for 1,811 rows, all else included: 13.8 ms, 21.1
+        with the float32 matrix instructions, whose partial sums the readers added up.)"""
+        if m <= 64:
+            return 0, False
+        blocks, cols = -(-k // 32), -(-n // 128)
+        read = m * n * 4 / 4.5e6
+        plans = [(-(-m // 64) * (n * k * 1.85e-6 + s * n * 256 / 2.75e6) + 2 + s * read, 0, False)]
+        for rows, fixed, per_block in ((64, 5.0, 0.9), (128, 7.0, 1.25)):
+            tiles = -(-m // rows) * cols
+            if s > 1:
+                plans.append((5 + -(-tiles // 256) * (fixed + blocks * per_block) + read, rows, True))
+            plans.append((5 + -(-tiles * s // 256) * (fixed + -(-blocks // s) * per_block) + 2 * s * read, rows, False))
+        return min(plans)[1:]
+
+    def _f32_product(self, x, w, bias, out, s: int, plan: tuple[int, bool]) -> None:
+        rows, fold = plan
+        m, k = x.shape
+        n = w.shape[0]
+        if rows:
+            self._run("egpt_gemm_f32_rows", x.data_ptr(), w.data_ptr(), self._ptr(bias), out.data_ptr(), m, n, k, s, int(fold),
+                      rows, self._stream())
+        else:
+            self._run("egpt_gemm_f32", x.data_ptr(), w.data_ptr(), self._ptr(bias), out.data_ptr(), m, n, k, s, self._stream())
 
     @staticmethod
     def _n_splits(m: int, n: int, k: int) -> int:
@@ -654,8 +683,9 @@ class HipKernels(KernelBackend):
             self._need(x, "x")
             self._need(w, "w", _F32, (n, k))
             s = self._f32_splits(n, k)
-            out = torch.empty((s, m, n), dtype=_F32, device=x.device)
-            self._run("egpt_gemm_f32", x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, s, self._stream())
+            plan = self._f32_rows_plan(m, n, k, s)
+            out = torch.empty((1 if plan[1] else s, m, n), dtype=_F32, device=x.device)
+            self._f32_product(x, w, None, out, s, plan)
             return out
         out = torch.empty((m, n), dtype=x.dtype, device=x.device)
         return self.linear(x, w, None, out)
