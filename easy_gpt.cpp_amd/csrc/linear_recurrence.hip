@@ -14,6 +14,8 @@
 // every token (S^T k), so its scan keeps a head's whole key range in one workgroup: egpt_delta_rule_scan.  Its operands
 // come from egpt_short_conv, which runs the short causal convolutions over time with their carried inputs, SiLU, and the
 // unit norms of queries and keys.
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -76,15 +78,39 @@ constexpr int kScanCols = 64;       // value channels per workgroup: a lane is a
 constexpr int kScanKeys = 16;       // key channels per workgroup
 constexpr int kScanWaves = 4;       // wavefronts per workgroup, kScanKeys / kScanWaves key channels each
 
+// The value of lane N of each row of 16 lanes.
+template <int N>
+__device__ __forceinline__ float row_value(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + N, 0xf, 0xf, true));
+#else
+    return v;
+#endif
+}
+// One token for four key channels of a column: their decays, keys and queries are the values of lanes N .. N + 3 of a row.
+template <int N>
+__device__ __forceinline__ void scan_token(float a, float k, float q, float v, float* s, float* part) {
+    s[0] = fmaf(row_value<N>(a), s[0], row_value<N>(k) * v);
+    s[1] = fmaf(row_value<N + 1>(a), s[1], row_value<N + 1>(k) * v);
+    s[2] = fmaf(row_value<N + 2>(a), s[2], row_value<N + 2>(k) * v);
+    s[3] = fmaf(row_value<N + 3>(a), s[3], row_value<N + 3>(k) * v);
+    *part = fmaf(row_value<N + 1>(q), s[1], row_value<N>(q) * s[0]) + fmaf(row_value<N + 3>(q), s[3], row_value<N + 2>(q) * s[2]);
+}
+
 // The recurrence has no term that mixes two key channels but the sum o_t = sum_r S[r][:] q[r], so the key channels are
 // dealt over workgroups: one workgroup of four wavefronts per (request, head, 64 value channels, 16 key channels), whose
 // part of o_t goes to out[split] (float32 [splits][tokens][heads * dv]) for the consumer to add in the order of the
 // splits.  A lane is one column of the state; wavefront w keeps four of the workgroup's key channels of that column in
-// registers.  The queries, keys and decays that a wavefront needs are the same for all its lanes (one address in LDS);
-// what bounds a token is what LDS returns for them (every lane gets its copy), which is why a workgroup takes few key
-// channels.  The wavefronts' parts go through LDS and are added in the order of the wavefronts, a batch of kScanTokens
-// tokens at a time; the batch's operands are staged in LDS, the next batch's loads in flight in registers meanwhile.
-template <typename T, bool ROTATED>
+// registers.  The queries, keys and decays that a wavefront needs are the same for all its lanes: one LDS read brings those of
+// four tokens, 16 values that every row of 16 lanes has, and an instruction takes its one of them out of the row (row_newbcast).
+// The wavefronts' parts go through LDS and are added in the order of the wavefronts, a batch of kScanTokens tokens at a time;
+// the batch's operands are staged in LDS, the next batch's loads in flight in registers meanwhile.
+// FORM says what the product is: 0 whole, in T; 1 one float32 array; 2 partial sums to be added up.  In the first two a batch's
+// loads are plain ones without a branch around them (places beyond the tokens or channels load a neighbour and count as zero),
+// so all of them are on their way together while the batch before is worked on; with one body for all forms a load waited for
+// the one before.  7 heads of 64 x 128, 2,535 tokens in three requests, the longest of 1,357: 172 us with that body, 118 now, of
+// which half are the instructions of the recurrence, 20 a token on a wavefront that has its SIMD to itself.
+template <typename T, bool ROTATED, int FORM>
 __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
     ProductView<T> proj, int proj_width, int q_off, int k_off, int v_off, float q_scale, const float* __restrict__ decay,
     float* __restrict__ states, const int32_t* __restrict__ slots, const unsigned char* __restrict__ fresh,
@@ -118,7 +144,17 @@ __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
         s[i] = (!start_anew && has_col && r < dk) ? state[static_cast<size_t>(r) * dv + j] : 0.f;
     }
     const int channels = heads * dk;
-    float rq[QKA], rk[QKA], ra[QKA], rv[VL];
+    std::conditional_t<FORM == 0, T, float> rq[QKA], rk[QKA], rv[VL];
+    float ra[QKA];
+    auto load = [&](size_t at) {
+        if constexpr (FORM == 0) return proj.whole[at];
+        else if constexpr (FORM == 1) return proj.partial[at];
+        else return proj.at(at);
+    };
+    auto value = [](auto v) {
+        if constexpr (FORM == 0) return to_float(v);
+        else return v;
+    };
     // the value at place r of a head whose columns begin at `at`, turned with its partner
     auto turned = [&](size_t row, size_t at, int r) {
         const float own = proj.at(at + r);
@@ -130,67 +166,100 @@ __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
         const float c = cos_sin[row * rot_dims + 2 * i] * mag, s = cos_sin[row * rot_dims + 2 * i + 1] * mag;
         return first ? __fmaf_rn(own, c, -__fmul_rn(other, s)) : __fmaf_rn(other, s, __fmul_rn(own, c));
     };
+    const float* decays = head_decay ? head_decay : decay;
     auto fetch = [&](int base) {
-        const int count = min(kScanTokens, n - base);
+        const int last = min(kScanTokens, n - base) - 1;
 #pragma unroll
         for (int u = 0; u < QKA; ++u) {
-            const int idx = tid + u * THREADS;
-            const int tt = idx / DKP, r = key0 + idx % DKP;
-            rq[u] = rk[u] = ra[u] = 0.f;
-            if (tt < count && r < dk) {
-                const size_t row = static_cast<size_t>(t0 + base + tt);
-                rq[u] = turned(row, row * proj_width + q_off + h * dk, r);      // (scaled when it is staged: nothing here waits for a load)
-                ra[u] = head_decay ? head_decay[h] : decay[row * channels + h * dk + r];
-                if (!tied_keys) rk[u] = turned(row, row * proj_width + k_off + h * dk, r);
+            const int idx = tid + u * THREADS, r = min(key0 + idx % DKP, dk - 1);
+            const size_t row = static_cast<size_t>(t0 + base + min(idx / DKP, last)), q_at = row * proj_width + q_off + h * dk;
+            const size_t k_at = tied_keys ? q_at : row * proj_width + k_off + h * dk;       // (a tied key is not read)
+            if constexpr (ROTATED) {
+                rq[u] = turned(row, q_at, r);
+                rk[u] = turned(row, k_at, r);
+            } else {
+                rq[u] = load(q_at + r);
+                rk[u] = load(k_at + r);
             }
+            ra[u] = decays[head_decay ? static_cast<size_t>(h) : row * channels + h * dk + r];
         }
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
             const int idx = tid + u * THREADS;
-            const int tt = idx / kScanCols, c = idx % kScanCols;
-            rv[u] = 0.f;
-            if (tt < count && col0 + c < dv)
-                rv[u] = proj.at(static_cast<size_t>(t0 + base + tt) * proj_width + v_off + h * dv + col0 + c);
+            rv[u] = load(static_cast<size_t>(t0 + base + min(idx / kScanCols, last)) * proj_width + v_off + h * dv + min(col0 + idx % kScanCols, dv - 1));
+        }
+    };
+    const int place = lane % 16 / 4 * DKP + wave * DKR + lane % 4;       // this lane's value of a group: token lane % 16 / 4, key lane % 4
+    auto group = [&](int tt, int tokens) __attribute__((always_inline)) {
+        const float a = a_s[tt * DKP + place], k = k_s[tt * DKP + place], q = q_s[tt * DKP + place];
+        float vj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vj[u] = v_s[(tt + u) * kScanCols + lane];
+        float* part = part_s + (tt * NS + wave) * kScanCols + lane;
+        scan_token<0>(a, k, q, vj[0], s, part);
+        if (tokens > 1) scan_token<4>(a, k, q, vj[1], s, part + NS * kScanCols);
+        if (tokens > 2) scan_token<8>(a, k, q, vj[2], s, part + 2 * NS * kScanCols);
+        if (tokens > 3) scan_token<12>(a, k, q, vj[3], s, part + 3 * NS * kScanCols);
+    };
+    // what goes to LDS: made of the loads before a batch's outputs are stored, because a wait for a load behind a store that a
+    // branch may skip waits for the store as well
+    float sq[QKA], sk[QKA], sa[QKA], sv[VL];
+    auto prepare = [&]() {
+#pragma unroll
+        for (int u = 0; u < QKA; ++u) {
+            // (a tied key is 1 - a; a place that holds no channel has a = 0 and would get k = 1, which meets a query of zero
+            // and a state row that is never stored; places behind the last token are not read)
+            const bool in = key0 + (tid + u * THREADS) % DKP < dk;
+            const float q = in ? value(rq[u]) : 0.f, k = in ? value(rk[u]) : 0.f, a = in ? ra[u] : 0.f;
+            sq[u] = (q_silu ? q / (1.0f + expf(-q)) : q) * q_scale;
+            sk[u] = tied_keys ? 1.0f - a : (k_silu ? k / (1.0f + expf(-k)) : k) * k_scale;
+            sa[u] = a;
+        }
+#pragma unroll
+        for (int u = 0; u < VL; ++u) {
+            const float v = value(rv[u]);
+            sv[u] = v_silu ? v / (1.0f + expf(-v)) : v;
         }
     };
     fetch(0);
+    prepare();
     for (int base = 0; base < n; base += kScanTokens) {
         const int count = min(kScanTokens, n - base);
         __syncthreads();                          // the batch before is read, its parts are added
 #pragma unroll
         for (int u = 0; u < QKA; ++u) {
-            // (a tied key is 1 - a; a place that holds no token or no channel has a = 0 and would get k = 1, which meets a
-            // query of zero and a state row that is never stored)
-            q_s[tid + u * THREADS] = (q_silu ? rq[u] / (1.0f + expf(-rq[u])) : rq[u]) * q_scale;
-            k_s[tid + u * THREADS] = tied_keys ? 1.0f - ra[u] : (k_silu ? rk[u] / (1.0f + expf(-rk[u])) : rk[u]) * k_scale;
-            a_s[tid + u * THREADS] = ra[u];
+            q_s[tid + u * THREADS] = sq[u];
+            k_s[tid + u * THREADS] = sk[u];
+            a_s[tid + u * THREADS] = sa[u];
         }
 #pragma unroll
-        for (int u = 0; u < VL; ++u) v_s[tid + u * THREADS] = v_silu ? rv[u] / (1.0f + expf(-rv[u])) : rv[u];
+        for (int u = 0; u < VL; ++u) v_s[tid + u * THREADS] = sv[u];
         __syncthreads();
         if (base + kScanTokens < n) fetch(base + kScanTokens);
-        for (int tt = 0; tt < count; ++tt) {
-            const float vj = v_s[tt * kScanCols + lane];
-            const float4 a = *reinterpret_cast<const float4*>(a_s + tt * DKP + wave * DKR);
-            const float4 k = *reinterpret_cast<const float4*>(k_s + tt * DKP + wave * DKR);
-            const float4 q = *reinterpret_cast<const float4*>(q_s + tt * DKP + wave * DKR);
-            s[0] = fmaf(a.x, s[0], k.x * vj);
-            s[1] = fmaf(a.y, s[1], k.y * vj);
-            s[2] = fmaf(a.z, s[2], k.z * vj);
-            s[3] = fmaf(a.w, s[3], k.w * vj);
-            part_s[(tt * NS + wave) * kScanCols + lane] = (s[0] * q.x + s[1] * q.y) + (s[2] * q.z + s[3] * q.w);
+        // four tokens at a time; the last tokens of a portion, fewer than four, by the same operations
+        if (count == kScanTokens) {
+#pragma unroll
+            for (int tt = 0; tt < kScanTokens; tt += 4) group(tt, 4);
+        } else {
+            int tt = 0;
+            for (; tt + 4 <= count; tt += 4) group(tt, 4);
+            if (tt < count) group(tt, count - tt);
         }
+        if (base + kScanTokens < n) prepare();
         __syncthreads();
+        float o[VL];
+#pragma unroll
+        for (int u = 0; u < VL; ++u) {
+            const int idx = tid + u * THREADS;
+            o[u] = 0.f;
+#pragma unroll
+            for (int w = 0; w < NS; ++w) o[u] += part_s[(idx / kScanCols * NS + w) * kScanCols + idx % kScanCols];
+        }
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
             const int idx = tid + u * THREADS;
             const int tt = idx / kScanCols, c = idx % kScanCols;
-            if (tt < count && col0 + c < dv) {
-                float o = 0.f;
-#pragma unroll
-                for (int w = 0; w < NS; ++w) o += part_s[(tt * NS + w) * kScanCols + c];
-                o_split[(static_cast<size_t>(t0 + base + tt) * heads + h) * dv + col0 + c] = o;
-            }
+            if (tt < count && col0 + c < dv) o_split[(static_cast<size_t>(t0 + base + tt) * heads + h) * dv + col0 + c] = o[u];
         }
     }
     if (has_col) {
@@ -258,7 +327,10 @@ static int launch_scan(const void* proj, int n_splits, int proj_width, int q_off
     const ProductView<T> view = scan_view<T>(proj, n_splits, static_cast<size_t>(n_tokens) * proj_width);
     const int key_splits = (dk + kScanKeys - 1) / kScanKeys;
     dim3 grid(n_seqs, heads, (dv + kScanCols - 1) / kScanCols * key_splits);
-    auto kernel = rot_dims > 0 ? decayed_state_scan_kernel<T, true> : decayed_state_scan_kernel<T, false>;
+    auto kernel = rot_dims > 0 ? decayed_state_scan_kernel<T, true, 2>
+                  : n_splits == 0 ? decayed_state_scan_kernel<T, false, 0>
+                  : n_splits == 1 ? decayed_state_scan_kernel<T, false, 1>
+                                  : decayed_state_scan_kernel<T, false, 2>;
     kernel<<<grid, 64 * kScanWaves, 0, s>>>(view, proj_width, q_off, k_off, v_off, q_scale, decay, states, slots, fresh, q_start, q_len,
                                             out, n_tokens, heads, dk, dv, key_splits, q_silu, tied_keys, k_silu, v_silu, head_decay,
                                             cos_sin, rot_dims, mag, interleaved, k_scale);

@@ -358,6 +358,33 @@ def test_the_state_scan_takes_a_rounded_product_and_a_batch_of_unequal_requests(
     assert torch.equal(states[2].cpu(), before[2]) and torch.equal(states[5].cpu(), before[5])
 
 
+@pytest.mark.parametrize("heads, dk, dv", [(2, 6, 100), (1, 36, 70), (3, 64, 128), (1, 300, 9)])
+@pytest.mark.parametrize("option", ["plain", "q_silu", "tied_keys", "kv_silu", "head_decay"])
+def test_the_state_scan_reads_every_form_of_a_product_alike(k, heads, dk, dv, option):
+    """One float32 array, the same values whole, and the same values with partial sums of zero behind them: the same bits, in
+    portions around the four tokens of a group and the 32 of a batch."""
+    proj, whole, decay, offs = scan_inputs(101, heads, dk, dv, 11, torch.float32)
+    asked = {"plain": {}, "q_silu": dict(q_silu=True), "tied_keys": dict(tied_keys=True), "kv_silu": dict(k_silu=True, v_silu=True),
+             "head_decay": dict(head_decay=torch.linspace(0.5, 0.9, heads, device=DEV))}[option]
+    forms = [proj, whole, torch.cat([proj, torch.zeros_like(proj)])]
+    results = []
+    for form in forms:
+        states, outs, pos = torch.full((1, heads, dk, dv), float("nan"), device=DEV), [], 0
+        for n in (64, 32, 3, 1, 1):
+            part = form[..., pos : pos + n, :].contiguous().to(DEV)
+            d = None if option == "head_decay" else decay[pos : pos + n].contiguous().to(DEV)
+            outs.append(k.decayed_state_scan(part, torch.float32, *offs, 0.5, d, states, i32(0), torch.tensor([pos == 0], device=DEV),
+                                             i32(0), i32(n), heads, dk, dv, **asked))
+            pos += n
+        results.append((torch.cat(outs, dim=-2), states))
+    for out, states in results[1:]:
+        assert torch.equal(out, results[0][0]) and torch.equal(states, results[0][1])
+    if option == "plain":
+        want, last = plain_scan(whole, decay, offs, heads, dk, dv, 0.5)
+        close(added(results[0][0]).view(101, heads, dv), want, torch.float32, "outputs")
+        close(results[0][1][0], last, torch.float32, "the state it leaves")
+
+
 def test_a_token_far_back_stays_in_a_state_that_does_not_decay(k):
     """Decays of one: after 900 tokens the query that matches token 17's key still finds its value."""
     heads, dk, dv, t = 1, 32, 64, 900
