@@ -325,13 +325,20 @@ __global__ __launch_bounds__(256) void whole_norm_store_kernel(
     float val[kKeep];
     float ssq = 0.f, ssk = 0.f;
     if (kept) {
+        constexpr int N = 4;
 #pragma unroll
-        for (int i = 0; i < kKeep; ++i) {
-            const int j = threadIdx.x + i * blockDim.x;
-            val[i] = 0.f;
-            if (j < qw + kw + vw) {
-                val[i] = proj.at(row + j);
-                if (bias) val[i] += to_float(bias[j]);
+        for (int i0 = 0; i0 < kKeep; i0 += N) {
+            if (i0 * static_cast<int>(blockDim.x) >= qw + kw + vw) break;
+            size_t at[N];
+            float v[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) at[i] = row + min(static_cast<int>(threadIdx.x + (i0 + i) * blockDim.x), qw + kw + vw - 1);
+            read_values(proj, at, v);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const int j = threadIdx.x + (i0 + i) * blockDim.x;
+                val[i0 + i] = v[i];
+                if (bias && j < qw + kw + vw) val[i0 + i] += to_float(bias[j]);
             }
         }
 #pragma unroll
@@ -402,6 +409,35 @@ __global__ __launch_bounds__(kWave) void head_norm_gate_kernel(ProductView<float
     const size_t xr = static_cast<size_t>(t) * x_width + static_cast<size_t>(h) * dv;
     const bool act_typed = xa.present();
     float ss = 0.f;
+    if (dv <= 2 * kWave) {                                // a head of up to two values per lane: everything is loaded at once
+        size_t xat[2], gat[2];
+        float v[2], gate[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int d = min(lane + i * kWave, dv - 1);
+            xat[i] = xr + d;
+            gat[i] = static_cast<size_t>(t) * gate_width + gate_off + h * dv + d;
+        }
+        if (act_typed) read_values(xa, xat, v);
+        else read_values(x, xat, v);
+        if (g.present()) read_values(g, gat, gate);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (lane + i * kWave < dv) ss = fmaf(v[i], v[i], ss);
+        const float inv = inv_rms(wave_sum(ss), 1.0f / static_cast<float>(dv), eps);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int d = lane + i * kWave;
+            if (d >= dv) break;
+            float y = v[i] * inv * (weight ? to_float(weight[d]) : 1.0f);
+            if (g.present()) {
+                const float sig = 1.0f / (1.0f + expf(-gate[i]));
+                y *= gate_act == 0 ? gate[i] * sig : (gate_act == 1 ? sig : gate[i]);
+            }
+            out[(static_cast<size_t>(t) * heads + h) * dv + d] = from_float<T>(y);
+        }
+        return;
+    }
     for (int d = lane; d < dv; d += kWave) {
         const float v = act_typed ? xa.at(xr + d) : x.at(xr + d);
         ss = fmaf(v, v, ss);

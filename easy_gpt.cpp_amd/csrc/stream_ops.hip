@@ -32,6 +32,13 @@ __global__ __launch_bounds__(256) void embed_scaled_kernel(const int32_t* __rest
     for (int j = threadIdx.x; j < hidden; j += blockDim.x) o[j] = to_float(row[j]) * factor;
 }
 
+// v * w, and b added to the rounded product: two roundings, whatever the compiler could make of it.
+__device__ __forceinline__ float scaled_then_added(float v, float w, float b, bool add) {
+#pragma clang fp contract(off)
+    const float y = v * w;
+    return add ? y + b : y;
+}
+
 // h += delta (float32, written back unless rows are selected), then out = (h - mean) / sqrt(var + eps) * w + b with
 // var the mean of the squared deviations.  Two passes over a row that lies in LDS: the mean first, then the
 // deviations, so that a row with a large mean loses nothing to cancellation.
@@ -48,12 +55,29 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
     const bool has_delta = delta.present();
     const bool write_back = rows == nullptr && has_delta;
     float sum = 0.f;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
-        float v = hrow[j];
-        if (has_delta) v += delta.at(src * hidden + j);
-        if (write_back) hrow[j] = v;
-        row_s[j] = v;
-        sum += v;
+    constexpr int N = 4;                                   // values of a thread whose loads are on their way together
+    for (int j0 = threadIdx.x; j0 < hidden; j0 += N * 256) {
+        size_t at[N];
+        float v[N], d[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int j = min(j0 + i * 256, hidden - 1);
+            v[i] = hrow[j];
+            at[i] = src * hidden + j;
+        }
+        if (has_delta) {
+            read_values(delta, at, d);
+#pragma unroll
+            for (int i = 0; i < N; ++i) v[i] += d[i];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int j = j0 + i * 256;
+            if (j >= hidden) break;
+            if (write_back) hrow[j] = v[i];
+            row_s[j] = v[i];
+            sum += v[i];
+        }
     }
     const float mean = block_sum(sum, scratch) / static_cast<float>(hidden);
     float dev = 0.f;
@@ -63,10 +87,20 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
     }
     const float inv = 1.0f / sqrtf(block_sum(dev, scratch) / static_cast<float>(hidden) + eps);
     T* orow = out + static_cast<size_t>(r) * hidden;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
-        float y = (row_s[j] - mean) * inv * to_float(weight[j]);
-        if (bias) y += to_float(bias[j]);
-        orow[j] = from_float<T>(y);
+    for (int j0 = threadIdx.x; j0 < hidden; j0 += N * 256) {
+        T w[N], b[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) w[i] = weight[min(j0 + i * 256, hidden - 1)];
+        if (bias) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) b[i] = bias[min(j0 + i * 256, hidden - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int j = j0 + i * 256;
+            if (j >= hidden) break;
+            orow[j] = from_float<T>(scaled_then_added((row_s[j] - mean) * inv, to_float(w[i]), bias ? to_float(b[i]) : 0.f, bias != nullptr));
+        }
     }
 }
 
@@ -84,14 +118,25 @@ __global__ __launch_bounds__(256) void normed_pair_mean_kernel(ProductView<T> a,
     float* b_s = pair_s + hidden;
     const size_t base = static_cast<size_t>(blockIdx.x) * hidden;
     float ssa = 0.f, ssb = 0.f;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
-        float x = a.at(base + j), y = b.at(base + j);
-        if (bias_a) x += to_float(bias_a[j]);
-        if (bias_b) y += to_float(bias_b[j]);
-        a_s[j] = x;
-        b_s[j] = y;
-        ssa = fmaf(x, x, ssa);
-        ssb = fmaf(y, y, ssb);
+    constexpr int N = 4;                                   // values of a thread whose loads are on their way together
+    for (int j0 = threadIdx.x; j0 < hidden; j0 += N * 256) {
+        size_t at[N];
+        float x[N], y[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) at[i] = base + min(j0 + i * 256, hidden - 1);
+        read_values(a, at, x);
+        read_values(b, at, y);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int j = j0 + i * 256;
+            if (j >= hidden) break;
+            if (bias_a) x[i] += to_float(bias_a[j]);
+            if (bias_b) y[i] += to_float(bias_b[j]);
+            a_s[j] = x[i];
+            b_s[j] = y[i];
+            ssa = fmaf(x[i], x[i], ssa);
+            ssb = fmaf(y[i], y[i], ssb);
+        }
     }
     if (wa == nullptr) {
         for (int j = threadIdx.x; j < hidden; j += blockDim.x) out[base + j] = factor_a * a_s[j] + factor_b * b_s[j];
@@ -99,9 +144,21 @@ __global__ __launch_bounds__(256) void normed_pair_mean_kernel(ProductView<T> a,
     }
     const float inv_a = inv_rms(block_sum(ssa, scratch), 1.0f / static_cast<float>(hidden), eps);
     const float inv_b = inv_rms(block_sum(ssb, scratch), 1.0f / static_cast<float>(hidden), eps);
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x)
-        out[base + j] = factor_a == factor_b ? factor_a * (a_s[j] * inv_a * to_float(wa[j]) + b_s[j] * inv_b * to_float(wb[j]))
-                                             : factor_a * (a_s[j] * inv_a * to_float(wa[j])) + factor_b * (b_s[j] * inv_b * to_float(wb[j]));
+    for (int j0 = threadIdx.x; j0 < hidden; j0 += N * 256) {
+        T u[N], w[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            u[i] = wa[min(j0 + i * 256, hidden - 1)];
+            w[i] = wb[min(j0 + i * 256, hidden - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int j = j0 + i * 256;
+            if (j >= hidden) break;
+            out[base + j] = factor_a == factor_b ? factor_a * (a_s[j] * inv_a * to_float(u[i]) + b_s[j] * inv_b * to_float(w[i]))
+                                                 : factor_a * (a_s[j] * inv_a * to_float(u[i])) + factor_b * (b_s[j] * inv_b * to_float(w[i]));
+        }
+    }
 }
 
 // x[t, :] = factor * E[id_t, :] + P[position_t, :]: a token's vector plus a learned vector of its position, added in float32

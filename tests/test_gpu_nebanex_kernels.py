@@ -285,6 +285,34 @@ def test_per_head_norm_with_the_silu_gate(k, dtype, heads, dv, splits):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("splits", [0, 1, 2, 6, 17])
+@pytest.mark.parametrize("width", [1, 63, 65, 128, 129, 255, 257, 1024, 1027, 2050])
+def test_rows_around_the_loads_of_a_thread_in_every_form(k, dtype, splits, width):
+    """Widths at which a thread or a lane has its last value, and partial sums around the loads that are on their way together."""
+    t, s = 3, max(1, splits)
+    parts = rnd(s, t, 2 * width, seed=1, scale=1.0 / math.sqrt(s))
+    if splits == 0:
+        parts = parts.to(dtype).float()
+    x, y = parts[..., :width].contiguous(), parts[..., width:].contiguous()
+    given = lambda p: (p[0].to(dtype) if splits == 0 else p).to(DEV)
+    h, w, b = rnd(t, width, seed=2), (rnd(width, seed=3) + 1).to(dtype), rnd(width, seed=4).to(dtype)
+    hd, out = h.clone().to(DEV), torch.empty((t, width), dtype=dtype, device=DEV)
+    if width > 1:                                            # (a single value has no spread)
+        k.add_layernorm(hd, given(x), None, w.to(DEV), b.to(DEV), 1e-5, out)
+        want = h.to(F64) + x.to(F64).sum(0)
+        close(hd, want, torch.float32, "the stream", 1e-6)
+        close(out, P.layer_norm(want, w.to(F64), b.to(F64), 1e-5), dtype, "layer norm")
+    got = k.normed_pair_mean(given(x), given(y), b.to(DEV), None, w.to(DEV), w.to(DEV), 1e-6, 0.5)
+    want = 0.5 * (P.rms_norm(x.to(F64).sum(0) + b.to(F64), w.to(F64), 1e-6) + P.rms_norm(y.to(F64).sum(0), w.to(F64), 1e-6))
+    close(got[0], want, torch.float32, "two branches", 1e-5)
+    if width <= 257:
+        xf = x[0].to(DEV) if splits == 0 else x.to(DEV)      # (the heads are float32 in either form)
+        k.head_norm_gate(xf, w.to(DEV), 1e-6, given(parts), width, out, 1, width)
+        g = y.to(F64).sum(0)
+        close(out, P.rms_norm(x.to(F64).sum(0), w.to(F64), 1e-6) * g * torch.sigmoid(g), dtype, "head norm and gate")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rank, channels, tau", [(5, 30, 1.0), (16, 96, 8.0), (1, 7, 4.0)])
 def test_decays_from_the_low_rank_projection(k, dtype, rank, channels, tau):
     t, off = 9, 11
