@@ -109,7 +109,10 @@ __device__ __forceinline__ void scan_token(float a, float k, float q, float v, f
 // loads are plain ones without a branch around them (places beyond the tokens or channels load a neighbour and count as zero),
 // so all of them are on their way together while the batch before is worked on; with one body for all forms a load waited for
 // the one before.  7 heads of 64 x 128, 2,535 tokens in three requests, the longest of 1,357: 172 us with that body, 118 now, of
-// which half are the instructions of the recurrence, 20 a token on a wavefront that has its SIMD to itself.
+// which half are the instructions of the recurrence, 20 a token on a wavefront that has its SIMD to itself.  Partial sums and
+// rotated operands take several loads each, which do wait for one another, so there a thread whose place holds no token or
+// channel loads nothing.  (64 decoded tokens of 7 heads out of four partial sums: 22.8 us, 42.9 with loads for every place;
+// rotated 29.4 and 60.1.)
 template <typename T, bool ROTATED, int FORM>
 __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
     ProductView<T> proj, int proj_width, int q_off, int k_off, int v_off, float q_scale, const float* __restrict__ decay,
@@ -144,6 +147,7 @@ __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
         s[i] = (!start_anew && has_col && r < dk) ? state[static_cast<size_t>(r) * dv + j] : 0.f;
     }
     const int channels = heads * dk;
+    constexpr bool kPlain = !ROTATED && FORM != 2;            // every load is one plain load
     std::conditional_t<FORM == 0, T, float> rq[QKA], rk[QKA], rv[VL];
     float ra[QKA];
     auto load = [&](size_t at) {
@@ -171,22 +175,32 @@ __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
         const int last = min(kScanTokens, n - base) - 1;
 #pragma unroll
         for (int u = 0; u < QKA; ++u) {
-            const int idx = tid + u * THREADS, r = min(key0 + idx % DKP, dk - 1);
-            const size_t row = static_cast<size_t>(t0 + base + min(idx / DKP, last)), q_at = row * proj_width + q_off + h * dk;
-            const size_t k_at = tied_keys ? q_at : row * proj_width + k_off + h * dk;       // (a tied key is not read)
-            if constexpr (ROTATED) {
-                rq[u] = turned(row, q_at, r);
-                rk[u] = turned(row, k_at, r);
-            } else {
+            const int idx = tid + u * THREADS, in_head = key0 + idx % DKP, r = kPlain ? min(in_head, dk - 1) : in_head;
+            const int tt = kPlain ? min(idx / DKP, last) : idx / DKP;
+            if constexpr (!kPlain) {
+                rq[u] = rk[u] = ra[u] = 0.f;
+                if (tt > last || r >= dk) continue;
+            }
+            const size_t row = static_cast<size_t>(t0 + base + tt), q_at = row * proj_width + q_off + h * dk;
+            const size_t k_at = tied_keys ? q_at : row * proj_width + k_off + h * dk;
+            if constexpr (kPlain) {
                 rq[u] = load(q_at + r);
-                rk[u] = load(k_at + r);
+                rk[u] = load(k_at + r);                            // (of a tied key nothing is used)
+            } else {
+                rq[u] = turned(row, q_at, r);
+                if (!tied_keys) rk[u] = turned(row, k_at, r);
             }
             ra[u] = decays[head_decay ? static_cast<size_t>(h) : row * channels + h * dk + r];
         }
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
-            const int idx = tid + u * THREADS;
-            rv[u] = load(static_cast<size_t>(t0 + base + min(idx / kScanCols, last)) * proj_width + v_off + h * dv + min(col0 + idx % kScanCols, dv - 1));
+            const int idx = tid + u * THREADS, in_head = col0 + idx % kScanCols, c = kPlain ? min(in_head, dv - 1) : in_head;
+            const int tt = kPlain ? min(idx / kScanCols, last) : idx / kScanCols;
+            if constexpr (!kPlain) {
+                rv[u] = 0.f;
+                if (tt > last || c >= dv) continue;
+            }
+            rv[u] = load(static_cast<size_t>(t0 + base + tt) * proj_width + v_off + h * dv + c);
         }
     };
     const int place = lane % 16 / 4 * DKP + wave * DKR + lane % 4;       // this lane's value of a group: token lane % 16 / 4, key lane % 4
