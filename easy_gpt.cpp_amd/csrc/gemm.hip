@@ -78,7 +78,9 @@ int launch_tiled(const void* x, const void* w, const void* bias, void* out, int 
 // with v_mfma_f32_16x16x4_f32, which took its operands as they are and rounded after every fourth product, 5.4e-7 / 1.25e-6; with
 // one chain over all blocks 4.5e-7 / 1.1e-6.
 // Values that have no such three parts (infinities, NaN, beyond the largest bfloat16) and overflows on the way leave an
-// element that is no finite number: it is then added up again in plain float32, so it comes out as it did.
+// element that is no finite number.  A wavefront that holds one adds its tile up again with v_mfma_f32_16x16x4_f32, which takes
+// float32 operands whole, and takes those elements from there.  (1,811 rows and 9,728 x 896, us: 256, 299 with one row of NaN,
+// 842 with nothing else; 8 rows 8.6 and 14.8.)
 //
 // Every element of the result is the same sequence of operations whatever m is and wherever its row lies in x, in all
 // kernels here: block after block of 32 values within a range of k, ranges of k one after the other.  So a token's values do not
@@ -135,13 +137,50 @@ __device__ __forceinline__ void block_sums(const Parts* w, const Parts* x, f32x4
 #pragma unroll
     for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j].h, x[j % X].h, t[j], 0, 0, 0);
 }
-// An element over values [k0, k1) of k in plain float32, where the parts' sum is no finite number.
-__device__ __noinline__ float plain_sum(const float* x, const float* w, int k0, int k1) {
-    float v = 0.f;
-    for (int i = k0; i < k1; ++i) v = fmaf(w[i], x[i], v);
-    return v;
+// The sums of N tiles of 16 x 16 elements over values [k0, k1) of k (multiples of four) without parts, straight from memory: x and
+// w[j] are the lane's rows li of the operands; v_mfma_f32_16x16x4_f32, sixteen values of k after the other, the i-th instruction of
+// each sixteen the i-th values of the four lanes' quadruples.
+template <int N>
+__device__ __forceinline__ void whole_sums(const float* x, const float* const (&w)[N], int lg, int k0, int k1, f32x4 (&t)[N]) {
+    const f32x4 none{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < N; ++j) t[j] = none;
+#pragma unroll 1
+    for (int b = k0; b < k1; b += 16) {
+        const int at = b + lg * 4;
+        const f32x4 xv = at < k1 ? *reinterpret_cast<const f32x4*>(x + at) : none;
+        f32x4 wv[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) wv[j] = at < k1 ? *reinterpret_cast<const f32x4*>(w[j] + at) : none;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < N; ++j) t[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][i], xv[i], t[j], 0, 0, 0);
+    }
 }
 __device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+// Whether all of a wavefront's elements of N tiles are finite numbers.
+template <int N>
+__device__ __forceinline__ bool all_finite(const f32x4 (&t)[N]) {
+    bool good = true;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) good &= finite(t[j][v]);
+    return __all(good);
+}
+// In place of the elements that are no finite number those of whole_sums.
+template <int N>
+__device__ __forceinline__ void mend(const float* x, const float* const (&w)[N], int lg, int k0, int k1, f32x4 (&t)[N]) {
+    if (all_finite(t)) return;
+    f32x4 whole[N];
+    whole_sums(x, w, lg, k0, k1, whole);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (!finite(t[j][v])) t[j][v] = whole[j][v];
+}
 
 // Up to 64 rows of x to a workgroup (further groups of rows: blockIdx.z).  A wavefront owns 16 rows of w (16 columns of the
 // result) and streams them once, as they are (four steps of 64 values ahead: with few rows the kernel is a stream of w, and a
@@ -248,18 +287,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_mfma_kernel(const float* __r
     }
     // D layout: lane (li, lg) holds rows lg*4 + v of the 16 x 16 tile (an n index) at column li (an m index)
     const bool whole = n % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;   // four values are one store
+    const float* const wrow[1] = {w + static_cast<size_t>(min(n0 + li, n - 1)) * k};
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
         const int mm = m0 + t * 16 + li, nn = n0 + lg * 4;
+        f32x4 sums[1] = {acc[t]};
+        mend(x + static_cast<size_t>(min(mm, m - 1)) * k, wrow, lg, step_begin * kStepF, min(k, step_end * kStepF), sums);
         if (mm >= m || nn >= n) continue;
-        f32x4 val = acc[t];
+        f32x4 val = sums[0];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            if (nn + v >= n) continue;
-            if (!finite(val[v]))
-                val[v] = plain_sum(x + static_cast<size_t>(mm) * k, w + static_cast<size_t>(nn + v) * k, step_begin * kStepF, min(k, step_end * kStepF));
-            if (bias) val[v] += bias[nn + v];
-        }
+        for (int v = 0; v < 4; ++v)
+            if (bias && nn + v < n) val[v] += bias[nn + v];
         float* to = out + (static_cast<size_t>(split) * m + mm) * n + nn;
         if (whole) {
             *reinterpret_cast<f32x4*>(to) = val;
@@ -344,26 +382,13 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
             if (FOLD) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     const int row0 = m0 + wm * 32 + li, col0 = n0 + wn * 64 + lg * 4;
-    // the end of a range [b0, b1) of blocks: elements that are no finite number are added up again
-    auto mend = [&](int b0, int b1) {
-        bool bad = false;
+    // the end of a range [b0, b1) of blocks: elements that are no finite number
+    auto mend_range = [&](int b0, int b1) {
+        const float* wrow[TN];
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int j = 0; j < TN; ++j) wrow[j] = w + static_cast<size_t>(min(n0 + wn * 64 + j * 16 + li, n - 1)) * k;
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) bad |= !finite(acc[i][j][v]);
-        if (!__any(bad)) return;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int row = row0 + i * 16, col = col0 + j * 16 + v;
-                    if (!finite(acc[i][j][v]) && row < m && col < n)
-                        acc[i][j][v] = plain_sum(x + static_cast<size_t>(row) * k, w + static_cast<size_t>(col) * k, b0 * kBlockF, min(k, b1 * kBlockF));
-                }
+        for (int i = 0; i < TM; ++i) mend(x + static_cast<size_t>(min(row0 + i * 16, m - 1)) * k, wrow, lg, b0 * kBlockF, min(k, b1 * kBlockF), acc[i]);
     };
     load(0, first);
     load(1, first + 1);
@@ -412,7 +437,7 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
                 load(1 - u, b + 3);
             }
             if (FOLD && (++in_range == blocks_per_split || b + 1 == last)) {
-                mend(range_begin, b + 1);
+                mend_range(range_begin, b + 1);
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -425,7 +450,7 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
             }
         }
     }
-    if (!FOLD) mend(first, last);
+    if (!FOLD) mend_range(first, last);
     float* to = out + (FOLD ? 0 : static_cast<size_t>(blockIdx.y) * m * n);
     const bool whole = n % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;   // four values are one store
 #pragma unroll
