@@ -71,16 +71,19 @@ int launch_tiled(const void* x, const void* w, const void* bias, void* out, int 
 
 // ----------------------------------------------------------------------------- float32 on the matrix cores
 // The float32 product on the bfloat16 matrix instructions, with no less than float32's precision: every operand is the sum of three
-// bfloat16 numbers, x = h + m + l, each the nearest to what the ones before leave (8 + 8 + 8 bits: nothing is left), and of
+// bfloat16 numbers, 2^24 x = h + m + l, each the nearest to what the ones before leave (8 + 8 + 8 bits: nothing is left), and of
 // the nine products the six largest are added up; the three others are below 2^-25 of the product and of either sign.  The
+// power of two keeps the parts of the smallest numbers in bfloat16's range: the last bit of any float32 number, 2^-149, becomes
+// 2^-125, while without it the parts of 2^-116 lose bits (an error of 2.3e-6 instead of 1.1e-7, and 2.3e-3 at 2^-126).  The
 // six products of a block of 32 values of k are one chain of v_mfma_f32_16x16x32_bf16 that begins at zero, and the block's sum
-// is added to the element's in float32.  Error against 64 bits (2-norm, normal operands, k = 896 / 4,864): 1.1e-7 / 2.4e-7,
+// is taken back by 2^48 and added to the element's in float32.  Error against 64 bits (2-norm, k = 896 / 4,864): 1.1e-7 / 2.4e-7,
 // with v_mfma_f32_16x16x4_f32, which took its operands as they are and rounded after every fourth product, 5.4e-7 / 1.25e-6; with
-// one chain over all blocks 4.5e-7 / 1.1e-6.
-// Values that have no such three parts (infinities, NaN, beyond the largest bfloat16) and overflows on the way leave an
-// element that is no finite number.  A wavefront that holds one adds its tile up again with v_mfma_f32_16x16x4_f32, which takes
-// float32 operands whole, and takes those elements from there.  (1,811 rows and 9,728 x 896, us: 256, 299 with one row of NaN,
-// 842 with nothing else; 8 rows 8.6 and 14.8.)
+// one chain over all blocks 4.5e-7 / 1.1e-6.  (The power of two is a product per operand: nothing with up to 64 rows, 5 to 8 % of
+// the tiles of many rows: 1,811 and 4,096 rows of 9,728 x 896 in 235 and 480 us, 219 and 452 without it.)
+// Values that have no such three parts (infinities, NaN, from 2^104 on) and block sums beyond 2^80 leave an element that is no
+// finite number.  A wavefront that holds one adds its tile up again with v_mfma_f32_16x16x4_f32, which takes
+// float32 operands whole, and takes those elements from there.  (1,811 rows of 9,728 x 896, us: 277, 321 with one row of NaN,
+// 868 with nothing else; 8 rows 8.7 and 15.0.)
 //
 // Every element of the result is the same sequence of operations whatever m is and wherever its row lies in x, in all
 // kernels here: block after block of 32 values within a range of k, ranges of k one after the other.  So a token's values do not
@@ -90,7 +93,10 @@ constexpr int kStepF = 64;                    // ranges of k are multiples of th
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(8))) __bf16 f_bf16x8;
 
-struct Parts {                                // eight values of k as three bfloat16 numbers each
+constexpr float kUp = 0x1p24f;                // what operands are multiplied by
+constexpr float kDown = 0x1p-48f;             // and block sums
+
+struct Parts {                                // eight values of k, times kUp, as three bfloat16 numbers each
     f_bf16x8 h, m, l;
 };
 typedef __attribute__((ext_vector_type(2))) __bf16 f_bf16x2;
@@ -109,7 +115,7 @@ __device__ __forceinline__ Parts split_parts(const f32x4& a, const f32x4& b) {
     Parts p;
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
-        float x = i < 4 ? a[i] : b[i - 4], y = i < 4 ? a[i + 1] : b[i - 3];
+        float x = kUp * (i < 4 ? a[i] : b[i - 4]), y = kUp * (i < 4 ? a[i + 1] : b[i - 3]);
         f_bf16x2 h{static_cast<__bf16>(x), static_cast<__bf16>(y)};
         take_away(h, x, y);
         f_bf16x2 m{static_cast<__bf16>(x), static_cast<__bf16>(y)};
@@ -273,8 +279,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_mfma_kernel(const float* __r
                 }
                 f32x4 sums[2];
                 block_sums<2, 2>(wv, xv, sums);
-                acc[t] += sums[0];
-                acc[t] += sums[1];
+                acc[t] += kDown * sums[0];
+                acc[t] += kDown * sums[1];
             }
             if (step + kAhead < step_end) load_w(a[u], step + kAhead);
             if ((u + 1) % CH == 0 && step + 1 < step_end) {
@@ -430,7 +436,7 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
                 f32x4 sums[TN];
                 block_sums<TN, 1>(wv, &xv[i], sums);
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] += sums[j];
+                for (int j = 0; j < TN; ++j) acc[i][j] += kDown * sums[j];
             }
             if (wn == 1) {
                 store(1 - u, 1 - u);

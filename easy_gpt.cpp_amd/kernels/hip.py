@@ -405,7 +405,7 @@ class HipKernels(KernelBackend):
     def _f32_rows_plan(m: int, n: int, k: int, s: int) -> tuple[int, bool]:
         """(rows of a tile, ranges of k added up inside) of the float32 product; 0 rows: the kernel for few rows.  All of them
         give the same bits.  Costs in us, fitted to 64 to 1,811 rows of 1,152 x 896, 9,728 x 896 and 896 x 4,864 (in 7, 5 and 11
-        ranges): a CU holds one workgroup, which takes 5 us and 0.9 per block of 32 values of k for 64 x 128, 7 and 1.25 for
+        ranges): a CU holds one workgroup, which takes 5 us and 0.96 per block of 32 values of k for 64 x 128, 7 and 1.33 for
         128 x 128; the kernel for few rows takes 1.85 per group of 64 rows and million elements of w and writes at 2.75
         TB/s; partial sums are written and read at 4.5 TB/s.  (24 layers of these for 1,811 rows, all else included: 13.8 ms, 21.1
         with the float32 matrix instructions, whose partial sums the readers added up.)"""
@@ -414,7 +414,7 @@ class HipKernels(KernelBackend):
         blocks, cols = -(-k // 32), -(-n // 128)
         read = m * n * 4 / 4.5e6
         plans = [(-(-m // 64) * (n * k * 1.85e-6 + s * n * 256 / 2.75e6) + 2 + s * read, 0, False)]
-        for rows, fixed, per_block in ((64, 5.0, 0.9), (128, 7.0, 1.25)):
+        for rows, fixed, per_block in ((64, 5.0, 0.96), (128, 7.0, 1.33)):
             tiles = -(-m // rows) * cols
             if s > 1:
                 plans.append((5 + -(-tiles // 256) * (fixed + blocks * per_block) + read, rows, True))

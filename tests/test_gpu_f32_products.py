@@ -158,3 +158,38 @@ def test_every_place_of_a_value_without_parts(k, m, n, kk, splits, kernel):
                 got, want = in_order(run(x, bad)), clean.clone()
                 want[:, col] = value * x[:, where]
                 assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0))
+
+
+@pytest.mark.parametrize("kernel", ["few", 64, 128])
+@pytest.mark.parametrize("small_w", [False, True])
+@pytest.mark.parametrize("power", [-100, -112, -120, -124, -126, -128, -132, -140, -146])
+def test_small_operands_keep_their_bits(k, kernel, small_w, power):
+    """A whole operand of values around 2^power against large partners: float32's error of the product, down into the subnormals
+    (whose own bits are the float32 numbers that both sides are given).  A block of 32 values is rounded once and the blocks'
+    sum 28 times: 2^-24 sqrt(28 + 1) = 3.2e-7 in the 2-norm, were all roundings of the largest size and of random sign."""
+    small, large = rnd(70, 896, seed=15), rnd(130, 896, seed=16) * 2.0 ** 60
+    small = (small.double() * 2.0 ** power).float()
+    assert small.abs().max() < 2.0 ** (power + 3) and small.abs().max() > 0
+    x, w = (large, small) if small_w else (small, large)
+    got = few(k, x, w, 1)[0] if kernel == "few" else many(k, x, w, 1, False, kernel)[0]
+    exact = x.double() @ w.double().t()
+    assert (got.double() - exact).norm() <= 3.2e-7 * exact.norm()
+
+
+def test_small_operands_beside_others(k):
+    """The result's own range: ordinary rows, rows below 2^-126 whose products are subnormal, and rows whose one value below 2^-126
+    meets the only value of its column."""
+    x, w = rnd(40, 192, seed=17), rnd(48, 192, seed=18)
+    clean = few(k, x, w, 1)[0]
+    x[3] = (x[3].double() * 2.0 ** -130).float()
+    x[7], x[7, 5], w2 = 0.0, 1.2345e-39, w.clone()
+    w2[9], w2[9, 5] = 0.0, 3.0
+    for run in (lambda a, b: few(k, a, b, 1)[0], lambda a, b: many(k, a, b, 1, False, 64)[0], lambda a, b: many(k, a, b, 1, False, 128)[0]):
+        got = run(x, w2)
+        exact = x.double() @ w2.double().t()
+        # six blocks are rounded, each result to a multiple of 2^-149 at best
+        bound = 2.0 ** -24 * 8 * (x.double().abs() @ w2.double().abs().t()) + 7 * 2.0 ** -150
+        assert ((got.double() - exact).abs() <= bound).all()
+        same = [r for r in range(40) if r not in (3, 7)]
+        columns = [c for c in range(48) if c != 9]
+        assert torch.equal(got[same][:, columns], clean[same][:, columns])
