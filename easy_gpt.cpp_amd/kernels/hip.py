@@ -325,19 +325,32 @@ class HipKernels(KernelBackend):
     @staticmethod
     def _own_rows(m: int, n: int, k: int, unrounded: bool) -> bool:
         """Whether a bfloat16 product of more than 64 rows is the framework's own (gemm_rows.hip) instead of the
-        library's first choice, whose times are the second ones here (us, weights from memory)."""
+        library's first choice, whose times are the second ones here (us, weights from memory; without `unrounded` together
+        with the norm that reads the result)."""
         if unrounded:
-            # one float32 result, no split: 1,152 x 896 at 96 / 552 / 1,500 rows 6.5 / 6.8 / 8.9 against 7.7 / 8.6 / 10.1, at
-            # 2,048 11.5 against 11.6; 2,048 x 1,536 at 200 rows 10.0 against 9.2, 4,608 x 3,584 at 552 35 against 34
-            return k <= 1024 and m <= 1536
+            # One float32 result, no split: 1,152 x 896 at 96 / 552 / 1,000 / 1,500 rows 6.6 / 7.0 / 8.8 / 9.4 against 7.9 / 8.7 / 10.0 /
+            # 10.1, at 2,048 12.0 against 11.4; 2,752 x 896 at 128 / 640 / 1,024 rows 0.77 / 0.85 / 1.00 of the library's, at
+            # 1,536 1.14.  A longer k: 1,152 x 1,152 at 96 / 300 / 1,500 rows 7.5 / 7.7 / 11.4 against 6.6 / 7.5 / 11.4, 2,048 x 1,536 9.0 /
+            # 9.3 / 17.9 against 7.7 / 9.6 / 16.3, 4,608 x 3,584 24.7 / 32.9 / 57.5 against 20.5 / 24.4 / 53.3.  A narrow w with few
+            # rows: 768 x 768 and 512 x 1,024 at 65 and 128 rows 1.09 to 1.13 of the library's, at 200 0.80 and 0.72.
+            return k <= 1024 and m <= (1536 if n < 2 * k else 1024) and (n >= 896 or k <= 512 or m > 128)
+        if k <= 1024:
+            # 896 x 896 at 96 / 300 / 1,500 / 2,048 rows 8.1 / 10.5 / 14.9 / 17.3 against 11.2 / 11.9 / 15.8 / 16.8, 1,152 x 896 9.6 / 12.2 /
+            # 17.2 / 20.7 against 12.4 / 13.1 / 17.5 / 19.5, 512 x 1,024 at 2,048 1.08 of the library's; 3,072 x 1,024 at 128 / 640 / 1,024
+            # / 1,536 rows 0.93 / 0.97 / 1.02 / 1.19
+            return m <= (1536 if n < 2 * k else 1024)
         if k >= 2 * n:
-            # a long k range, which the library does not split: 896 x 4,864 at 96 / 552 / 2,048 rows 9 / 16 / 31 against 13 / 18
-            # / 34 (with the reader's share), 3,584 x 18,944 48 / 83 / 218 against 88 / 137 / 362; at 4,100 rows even, at
-            # 8,191 a fifth slower
-            return m <= 3584
-        # 896 x 896 at 96 / 552 / 2,048 rows 4.9 / 6.7 / 9.1 against 7.7 / 8.3 / 9.9, 3,584 x 3,584 at 96 / 432 15 / 24 against 20 /
-        # 27; but 1,536 x 1,536 at 1,500 rows 21 against 15, 3,584 x 3,584 at 552 33 against 27
-        return m <= (2048 if k <= 1024 else 448)
+            # A long k range, which the library does not split, so it falls behind the longer the range is.  1,024 x 2,048 at 300 /
+            # 448 / 1,000 rows 12.8 / 14.7 / 22.6 against 13.5 / 14.0 / 16.7, 1,024 x 3,072 at 320 / 640 0.89 and 1.10 of the library's;
+            # 1,024 x 4,096 at 1,000 / 1,500 23.0 / 33.2 against 24.5 / 27.8, 2,048 x 4,096 at 1,024 / 1,536 0.93 / 1.08; 896 x 4,864 at
+            # 1,500 / 2,048 / 3,584 27.7 / 33.4 / 51.3 against 30.7 / 34.6 / 47.6, 4,096 x 14,336 at 2,048 / 3,584 0.95 / 1.11;
+            # 1,536 x 8,960 at 2,048 / 3,584 / 8,191 70 / 106 / 222 against 83 / 113 / 194, 3,584 x 18,944 238 / 452 / 965 against
+            # 382 / 618 / 927 and 484 against 414 at 4,100
+            return m <= (320 if k < 4096 else 1024 if k < 4608 else 3584 if k >= 8192 and n < 4096 else 2048)
+        # 1,280 x 1,280 at 96 / 300 / 1,500 rows 10.8 / 13.8 / 22.4 against 11.5 / 12.7 / 19.8, 1,536 x 1,536 12.5 / 14.9 / 28.1 against 12.1 /
+        # 13.7 / 23.2; 3,584 x 3,584 at 96 / 200 / 552 / 1,500 20 / 23 / 39 / 59 against 26 / 26 / 34 / 56, 4,608 x 3,584 at 300 / 448 31 /
+        # 45 against 31 / 36, 4,096 x 4,096 at 200 / 320 0.85 / 1.11; 4,096 x 2,048 at 200 1.12 (wider ones have not been measured)
+        return n < 2 * k and m <= (256 if k >= 2048 else 128)
 
     def linear(self, x, w, bias, out):
         m, k = x.shape
