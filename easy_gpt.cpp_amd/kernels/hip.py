@@ -329,16 +329,18 @@ class HipKernels(KernelBackend):
         with the norm that reads the result)."""
         if unrounded:
             # One float32 result, no split: 1,152 x 896 at 96 / 552 / 1,000 / 1,500 rows 6.6 / 7.0 / 8.8 / 9.4 against 7.9 / 8.7 / 10.0 /
-            # 10.1, at 2,048 12.0 against 11.4; 2,752 x 896 at 128 / 640 / 1,024 rows 0.77 / 0.85 / 1.00 of the library's, at
-            # 1,536 1.14.  A longer k: 1,152 x 1,152 at 96 / 300 / 1,500 rows 7.5 / 7.7 / 11.4 against 6.6 / 7.5 / 11.4, 2,048 x 1,536 9.0 /
-            # 9.3 / 17.9 against 7.7 / 9.6 / 16.3, 4,608 x 3,584 24.7 / 32.9 / 57.5 against 20.5 / 24.4 / 53.3.  A narrow w with few
-            # rows: 768 x 768 and 512 x 1,024 at 65 and 128 rows 1.09 to 1.13 of the library's, at 200 0.80 and 0.72.
-            return k <= 1024 and m <= (1536 if n < 2 * k else 1024) and (n >= 896 or k <= 512 or m > 128)
+            # 10.1, at 2,048 12.0 against 11.4.  Wide or narrow ones are slower by themselves here and there (2,752 x 896 at 1,024
+            # and 1,536 rows 1.00 and 1.14 of the library's, 768 x 768 at 65 1.12), but the library fills the result with zeros first
+            # and takes the host longer: a design with states, whose steps run kernel by kernel, took 1,487 us for three prompts of
+            # 1,293 tokens with the library for these and 1,279 so, 1,166 and 1,098 for one of 85 (a width of 896).  A longer k: 1,152 x
+            # 1,152 at 96 / 300 / 1,500 rows 7.5 / 7.7 / 11.4 against 6.6 / 7.5 / 11.4, 2,048 x 1,536 9.0 / 9.3 / 17.9 against 7.7 / 9.6 /
+            # 16.3, 4,608 x 3,584 24.7 / 32.9 / 57.5 against 20.5 / 24.4 / 53.3.
+            return k <= 1024 and m <= 1536
         if k <= 1024:
-            # 896 x 896 at 96 / 300 / 1,500 / 2,048 rows 8.1 / 10.5 / 14.9 / 17.3 against 11.2 / 11.9 / 15.8 / 16.8, 1,152 x 896 9.6 / 12.2 /
-            # 17.2 / 20.7 against 12.4 / 13.1 / 17.5 / 19.5, 512 x 1,024 at 2,048 1.08 of the library's; 3,072 x 1,024 at 128 / 640 / 1,024
-            # / 1,536 rows 0.93 / 0.97 / 1.02 / 1.19
-            return m <= (1536 if n < 2 * k else 1024)
+            # 896 x 896 at 96 / 300 / 1,500 / 2,048 rows 8.1 / 10.5 / 14.9 / 17.3 against 11.2 / 11.9 / 15.8 / 16.8 (within a prompt of 2,048
+            # tokens at the 0.5B sizes 1.9 us faster than the library: 3,801 us a step and 3,847), 512 x 1,024 at 1,536 / 2,800 0.94 / 1.09
+            # of the library's; 3,072 x 1,024 at 128 / 640 / 1,024 / 1,536 rows 0.93 / 0.97 / 1.02 / 1.19
+            return m <= (2048 if n < 2 * k else 1024)
         if k >= 2 * n:
             # A long k range, which the library does not split, so it falls behind the longer the range is.  1,024 x 2,048 at 300 /
             # 448 / 1,000 rows 12.8 / 14.7 / 22.6 against 13.5 / 14.0 / 16.7, 1,024 x 3,072 at 320 / 640 0.89 and 1.10 of the library's;

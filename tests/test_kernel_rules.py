@@ -46,18 +46,18 @@ def test_which_rows_go_to_the_library_is_monotonic_in_the_rows():
 
 def test_products_of_many_rows_leave_their_kernel_where_the_library_is_faster():
     # (rows, n, k) with both sides measured more than the runs differ
-    own = [(96, 896, 896), (300, 1152, 896), (1500, 896, 896), (200, 512, 1024), (1000, 1024, 1024), (96, 1280, 1280), (96, 2048, 2048),
+    own = [(96, 896, 896), (300, 1152, 896), (2048, 896, 896), (200, 512, 1024), (1000, 1024, 1024), (96, 1280, 1280), (96, 2048, 2048),
            (200, 3584, 3584), (65, 5120, 5120), (300, 1024, 2048), (1000, 1024, 4096), (2048, 896, 4864), (640, 2048, 5632), (1536, 4096, 14336),
            (3584, 1536, 8960), (3584, 3584, 18944)]
-    library = [(2048, 1152, 896), (2048, 512, 1024), (1536, 3072, 1024), (300, 1280, 1280), (448, 1536, 1536), (448, 2048, 1536),
+    library = [(2800, 1152, 896), (2800, 512, 1024), (1536, 3072, 1024), (300, 1280, 1280), (448, 1536, 1536), (448, 2048, 1536),
                (552, 3584, 3584), (448, 4608, 3584), (320, 4096, 4096), (320, 4096, 2048), (552, 1024, 2048), (1000, 1024, 2048),
                (640, 1536, 3072), (1500, 1024, 4096), (1536, 2048, 4096), (3584, 896, 4864), (3584, 4096, 14336), (4100, 3584, 18944)]
     for sizes in own:
         assert K._own_rows(*sizes, False), sizes
     for sizes in library:
         assert not K._own_rows(*sizes, False), sizes
-    unrounded = [(96, 896, 896), (1500, 1152, 896), (640, 2752, 896), (200, 768, 768), (65, 256, 256)]
-    rounded_only = [(2048, 1152, 896), (1536, 2752, 896), (65, 768, 768), (128, 512, 1024), (96, 1152, 1152), (200, 2048, 2048), (552, 3584, 18944)]
+    unrounded = [(96, 896, 896), (1500, 1152, 896), (1293, 2752, 896), (85, 768, 768), (65, 256, 256)]
+    rounded_only = [(2048, 1152, 896), (96, 1152, 1152), (200, 2048, 2048), (552, 3584, 18944)]
     for sizes in unrounded:
         assert K._own_rows(*sizes, True), sizes
     for sizes in rounded_only:
