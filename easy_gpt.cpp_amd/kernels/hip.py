@@ -341,18 +341,23 @@ class HipKernels(KernelBackend):
             # tokens at the 0.5B sizes 1.9 us faster than the library: 3,801 us a step and 3,847), 512 x 1,024 at 1,536 / 2,800 0.94 / 1.09
             # of the library's; 3,072 x 1,024 at 128 / 640 / 1,024 / 1,536 rows 0.93 / 0.97 / 1.02 / 1.19
             return m <= (2048 if n < 2 * k else 1024)
+        # Below: whole prompts, us a layer that the library would take longer; within a step a product by itself is not the
+        # measure, since what surrounds it changes with the form of its result.
         if k >= 2 * n:
-            # A long k range, which the library does not split, so it falls behind the longer the range is.  1,024 x 2,048 at 300 /
-            # 448 / 1,000 rows 12.8 / 14.7 / 22.6 against 13.5 / 14.0 / 16.7, 1,024 x 3,072 at 320 / 640 0.89 and 1.10 of the library's;
-            # 1,024 x 4,096 at 1,000 / 1,500 23.0 / 33.2 against 24.5 / 27.8, 2,048 x 4,096 at 1,024 / 1,536 0.93 / 1.08; 896 x 4,864 at
-            # 1,500 / 2,048 / 3,584 27.7 / 33.4 / 51.3 against 30.7 / 34.6 / 47.6, 4,096 x 14,336 at 2,048 / 3,584 0.95 / 1.11;
-            # 1,536 x 8,960 at 2,048 / 3,584 / 8,191 70 / 106 / 222 against 83 / 113 / 194, 3,584 x 18,944 238 / 452 / 965 against
-            # 382 / 618 / 927 and 484 against 414 at 4,100
-            return m <= (320 if k < 4096 else 1024 if k < 4608 else 3584 if k >= 8192 and n < 4096 else 2048)
-        # 1,280 x 1,280 at 96 / 300 / 1,500 rows 10.8 / 13.8 / 22.4 against 11.5 / 12.7 / 19.8, 1,536 x 1,536 12.5 / 14.9 / 28.1 against 12.1 /
-        # 13.7 / 23.2; 3,584 x 3,584 at 96 / 200 / 552 / 1,500 20 / 23 / 39 / 59 against 26 / 26 / 34 / 56, 4,608 x 3,584 at 300 / 448 31 /
-        # 45 against 31 / 36, 4,096 x 4,096 at 200 / 320 0.85 / 1.11; 4,096 x 2,048 at 200 1.12 (wider ones have not been measured)
-        return n < 2 * k and m <= (256 if k >= 2048 else 128)
+            # A long k range, which the library does not split, so that it falls behind the longer the range is.  896 x 4,864 at 70 / 300 /
+            # 1,000 / 2,048 / 3,500 / 5,000 tokens 4 / 6 / 5 / 2 / 4 / -24, 1,536 x 8,960 7 / 11 / 10 / 8 / 2 / -1, 2,048 x 11,008 12 / 18 / 23 / 12 /
+            # 20 / -39, 3,584 x 18,944 90 / 44 / 74 / 142 / 159 / 283; 1,024 x 3,072 3 / 5 / 1 / 0 / -2 / -5 (-3 at 1,500), 4,096 x 14,336 6 / 23 /
+            # 24 / 20 / -30 / -95, 5,120 x 13,824 5 / 31 / 31 / -26 / 271 / 228 (16 at 1,500).  Shorter ones by themselves, times over the
+            # library's: 1,024 x 2,048 at 300 / 448 / 1,000 rows 0.95 / 1.05 / 1.35, 1,024 x 4,096 at 1,000 / 1,500 0.94 / 1.19, 2,048 x
+            # 4,096 at 1,024 / 1,536 0.93 / 1.08.
+            if k >= 8192 and k >= 5 * n:
+                return m <= 3584
+            return m <= (320 if k < 3072 else 1024 if k < 4608 else 1536 if k < 3 * n else 2048)
+        # 1,536 x 1,536 at 70 / 200 / 450 / 1,500 tokens 2 / 1 / 0 / -3, 2,048 x 2,048 at 70 / 200 / 450 / 650 6 / 2 / 0 / -3, 3,072 x 3,072 at 70 /
+        # 300 / 450 / 2,048 4 / 1 / -6 / -10, 3,584 x 3,584 at 70 / 450 / 1,000 9 / 3 / -2, 5,120 x 5,120 3 / 11 / 4.  Wider than long ones by
+        # themselves, times over the library's: 4,608 x 3,584 at 200 / 300 / 448 rows 0.79 / 0.98 / 1.24, 4,096 x 2,048 at 128 / 200 / 320 0.88 /
+        # 1.12 / 1.24.
+        return m <= 448 if n <= k else n < 2 * k and m <= 256
 
     def linear(self, x, w, bias, out):
         m, k = x.shape

@@ -46,12 +46,13 @@ def test_which_rows_go_to_the_library_is_monotonic_in_the_rows():
 
 def test_products_of_many_rows_leave_their_kernel_where_the_library_is_faster():
     # (rows, n, k) with both sides measured more than the runs differ
-    own = [(96, 896, 896), (300, 1152, 896), (2048, 896, 896), (200, 512, 1024), (1000, 1024, 1024), (96, 1280, 1280), (96, 2048, 2048),
-           (200, 3584, 3584), (65, 5120, 5120), (300, 1024, 2048), (1000, 1024, 4096), (2048, 896, 4864), (640, 2048, 5632), (1536, 4096, 14336),
-           (3584, 1536, 8960), (3584, 3584, 18944)]
-    library = [(2800, 1152, 896), (2800, 512, 1024), (1536, 3072, 1024), (300, 1280, 1280), (448, 1536, 1536), (448, 2048, 1536),
-               (552, 3584, 3584), (448, 4608, 3584), (320, 4096, 4096), (320, 4096, 2048), (552, 1024, 2048), (1000, 1024, 2048),
-               (640, 1536, 3072), (1500, 1024, 4096), (1536, 2048, 4096), (3584, 896, 4864), (3584, 4096, 14336), (4100, 3584, 18944)]
+    own = [(96, 896, 896), (300, 1152, 896), (2048, 896, 896), (200, 512, 1024), (1000, 1024, 1024), (128, 1536, 1536), (200, 2048, 2048),
+           (200, 3584, 3584), (200, 4608, 3584), (450 - 2, 5120, 5120), (300, 1024, 2048), (1000, 1024, 4096), (650, 1024, 3072), (1500, 896, 4864),
+           (640, 2048, 5632), (1500, 5120, 13824), (2048, 4096, 14336), (3500, 2048, 11008), (3584, 3584, 18944)]
+    library = [(2800, 1152, 896), (2800, 512, 1024), (1536, 3072, 1024), (1500, 1536, 1536), (650, 2048, 2048), (1500, 2048, 1536),
+               (552, 3584, 3584), (448, 4608, 3584), (1500, 4096, 4096), (320, 4096, 2048), (552, 1024, 2048), (1000, 1024, 2048),
+               (1500, 1024, 3072), (1500, 1024, 4096), (1536, 2048, 4096), (5000, 896, 4864), (2048, 5120, 13824), (2500, 4096, 14336),
+               (5000, 2048, 11008)]
     for sizes in own:
         assert K._own_rows(*sizes, False), sizes
     for sizes in library:
