@@ -16,9 +16,10 @@
 // 486 us; with two of w and one of x (160 KB of LDS) 461, and on zeros 470 against 393.  Deeper rings in steps of 32 values
 // (64-byte pieces of rows) gained nothing: 509.  32x32x16 products: the same on zeros, 7 % slower on random numbers.  The
 // order of tiles: a die gets neighbouring tiles of one range of k (2,048 x 3,584 x 18,944 in two ranges: 247 -> 238 us).
-// Against the library's first choice (us): 2,048 rows x 18,944 gated x 3,584 456 against 505 + 43 for the activation;
-// 2,048 x 3,584 x 18,944 211 against 362; 552 x 1,536 x 8,960 26 against 37; 552 x 896 x 896 5.4 against 8.2; but 8,191 x
-// 8,960 gated x 1,536 455 against 342 + 90, and 4,100 x 2,048 x 1,536 41 against 33.
+// Against the library's first choice (us, weights from memory; gated ones with its activation kernel, others with the norm that
+// reads the result): 2,048 rows x 18,944 gated x 3,584 456 against 547, 8,191 x 8,960 gated x 1,536 436 against 446; 2,048 x 3,584 x
+// 18,944 238 against 382, 552 x 1,536 x 8,960 33 against 43, 552 x 896 x 896 11.0 against 12.6; but 8,191 x 18,944 gated x 3,584
+// 1,871 against 1,818 and 2,048 x 2,048 x 1,536 30 against 28.  `_own_rows` and `_own_gate` in kernels/hip.py draw the lines.
 #include "api.h"
 #include "common.h"
 

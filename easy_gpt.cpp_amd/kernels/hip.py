@@ -359,6 +359,27 @@ class HipKernels(KernelBackend):
         # 1.12 / 1.24.
         return m <= 448 if n <= k else n < 2 * k and m <= 256
 
+    @staticmethod
+    def _own_gate(m: int, k: int) -> bool:
+        """Whether gate, up and activation of more than 64 rows are one kernel (gemm_rows.hip) instead of the library's first
+        choice and an activation kernel, whose times are the second ones here (us, weights from memory)."""
+        if k <= 1536:
+            # 9,728 x 896 at 65 / 300 / 1,000 / 2,048 / 8,191 rows 12 / 15 / 27 / 53 / 181 against 15 / 20 / 39 / 66 / 198, 17,920 x
+            # 1,536 24 / 32 / 73 / 132 / 436 against 28 / 35 / 82 / 138 / 446 (at 16,384 rows 878 against 852), 8,192 x 1,024 10 / 16 /
+            # 24 / 39 / 154 against 16 / 20 / 30 / 44 / 156
+            return True
+        if k < 3072:
+            # 4,096 x 2,048 at 65 / 300 / 1,000 / 2,048 / 5,500 rows 15 / 20 / 25 / 36 / 90 against 16 / 20 / 30 / 40 / 94.  Whole prompts,
+            # us a layer that the library would take longer: 22,016 x 2,048 at 70 / 300 / 1,200 / 2,048 / 5,000 tokens 0 / 2 / 7 / 31 /
+            # 10, 19,456 x 2,560 1 / 5 / -1 / 22 / 63.  But at 8,191 rows 12,288 x 2,048 370 against 341, 28,672 x 2,048 857 against 791.
+            return m <= 6144
+        # Large matrices.  With few rows they are a stream of w, which the library reads faster, and with very many rows its larger
+        # tiles lose less at their edges.  Whole prompts, us a layer that the library would take longer: 37,888 x 3,584 at 70 / 128 / 200 /
+        # 500 / 1,200 / 2,500 / 3,500 tokens -6 / -1 / 9 / 8 / 106 / 35 / -36, 16,384 x 3,072 -8 / -7 / 3 / 3 / 2 / 90 / -6, 27,648 x 5,120 at
+        # 128 / 500 / 2,048 / 3,500 0 / 24 / 30 / -23.  Where all rows of w begin at the same place of 8 KB the library is as good or
+        # better: 12,288 x 4,096 at 128 / 300 / 1,200 / 2,048 -5 / -8 / 0 / -16, 28,672 x 4,096 1 / 1 / -31 / -34.
+        return 128 < m <= 3072 and k % 4096 != 0
+
     def linear(self, x, w, bias, out):
         m, k = x.shape
         n = w.shape[0]
@@ -634,13 +655,10 @@ class HipKernels(KernelBackend):
         return out
 
     def gate_up_rows(self, x, w, activation="silu"):
-        """The same for more than 64 rows.  Returns None where the case is not covered."""
+        """The same for more than 64 rows.  Returns None where another way is faster or the case is not covered."""
         t, k = x.shape
-        if t <= 64 or w.shape[0] % 2 or not self._rows_fit(x, w, k):
+        if t <= 64 or w.shape[0] % 2 or not self._rows_fit(x, w, k) or not self._own_gate(t, k):
             return None
-        # (against the library's product and an activation kernel, us: 9,728 x 896 at 96 / 552 / 2,048 / 8,191 rows 12 / 21 /
-        # 50 / 170 against 17 / 25 / 69 / 202; 17,920 x 1,536 22 / 37 / 122 / 455 against 25 / 44 / 140 / 443; 37,888 x 3,584 59 /
-        # 142 / 456 against 62 / 149 / 561)
         inter = w.shape[0] // 2
         self._need(x, "x", _BF16)
         self._need(w, "w", _BF16, (2 * inter, k))

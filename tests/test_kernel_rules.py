@@ -63,3 +63,12 @@ def test_products_of_many_rows_leave_their_kernel_where_the_library_is_faster():
         assert K._own_rows(*sizes, True), sizes
     for sizes in rounded_only:
         assert not K._own_rows(*sizes, True), sizes
+
+
+def test_gate_and_up_leave_their_kernel_where_the_library_is_faster():
+    # (rows, k) with both sides measured more than the runs differ, over matrices of 4,096 to 37,888 rows
+    for m, k in [(65, 896), (2048, 896), (8191, 896), (1000, 1024), (96, 1536), (2500, 1536), (500, 2048), (2048, 2048), (2500, 2560), (200, 3584),
+                 (1200, 3584), (2048, 3584), (2500, 3072), (500, 5120)]:
+        assert K._own_gate(m, k), (m, k)
+    for m, k in [(70, 3072), (128, 3072), (70, 3584), (300, 4096), (2048, 4096), (4096, 8192), (3500, 3584), (5000, 5120), (8191, 2048), (8191, 3072)]:
+        assert not K._own_gate(m, k), (m, k)
