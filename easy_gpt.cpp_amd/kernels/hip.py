@@ -7,6 +7,7 @@ current stream, so they order with torch's own work and can be captured into a g
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -292,10 +293,12 @@ class HipKernels(KernelBackend):
                     (128, 128, 2, 4.8, 1.8, 0.50, 1.33), (64, 64, 4, 6.3, -2.7, 0.36, 1.06))
 
     @classmethod
+    @functools.lru_cache(maxsize=4096)
     def _rows_plan(cls, m: int, n: int, k: int, most_splits: int) -> tuple[int, int]:
         """(shape, splits of the k range) of the product for many rows: the cheapest by the fit, a split paying for what
         its reader reads more (4.5 TB/s).  `n`: the rows of w.  (Against the best of everything that was measured, the
-        choice is 8 % slower on average and a third at worst.)"""
+        choice is 8 % slower on average and a third at worst.)  Found once per sizes, so once for a step's layers: it takes the
+        host 20 to 50 us with ten splits to choose from, as long as several of the products it is for."""
         steps = k // 64
         best = None
         for shape, (bm, bn, held, launch, per_round, alone, full) in enumerate(cls._rows_shapes):
@@ -443,6 +446,7 @@ class HipKernels(KernelBackend):
         return -(-steps // per)
 
     @staticmethod
+    @functools.lru_cache(maxsize=4096)
     def _f32_rows_plan(m: int, n: int, k: int, s: int) -> tuple[int, bool]:
         """(rows of a tile, ranges of k added up inside) of the float32 product; 0 rows: the kernel for few rows.  All of them
         give the same bits.  Costs in us, fitted to 64 to 1,811 rows of 1,152 x 896, 9,728 x 896 and 896 x 4,864 (in 7, 5 and 11

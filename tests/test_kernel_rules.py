@@ -72,3 +72,11 @@ def test_gate_and_up_leave_their_kernel_where_the_library_is_faster():
         assert K._own_gate(m, k), (m, k)
     for m, k in [(70, 3072), (128, 3072), (70, 3584), (300, 4096), (2048, 4096), (4096, 8192), (3500, 3584), (5000, 5120), (8191, 2048), (8191, 3072)]:
         assert not K._own_gate(m, k), (m, k)
+
+
+def test_a_plan_is_found_once_for_its_sizes():
+    for plan, sizes in ((K._rows_plan, (101, 896, 4864, 10)), (K._f32_rows_plan, (101, 896, 4864, 11))):
+        first, before = plan(*sizes), plan.cache_info()
+        assert all(plan(*sizes) == first for _ in range(24))         # a step's layers
+        after = plan.cache_info()
+        assert after.hits == before.hits + 24 and after.misses == before.misses and after.maxsize is not None
