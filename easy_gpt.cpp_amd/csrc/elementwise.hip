@@ -459,7 +459,10 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
     // enough threads for a row to stay in registers (four values a thread, eight for the widest rows)
     const int threads = (delta_splits > 1 || hidden > 2048) ? 1024 : (hidden > 1024 ? 512 : 256);
     const size_t stride = static_cast<size_t>(delta_rows) * hidden;
-    if (dtype == 1 && hidden % 8 == 0 && !fixed && (delta_splits <= 1 ? n_rows >= 32 : n_rows > 64)) {
+    // (loads and stores of 16 bytes: operands that begin elsewhere take the kernel of single values)
+    const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(weight) |
+                           reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    if (dtype == 1 && hidden % 8 == 0 && aligned && !fixed && (delta_splits <= 1 ? n_rows >= 32 : n_rows > 64)) {
         const int threads = hidden >= 2048 ? 256 : 128;
         float* hf = static_cast<float*>(h);
         if (delta_splits == 0)

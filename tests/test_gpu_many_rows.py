@@ -80,6 +80,30 @@ def test_the_norm_adds_partial_sums_of_many_rows(k):
         assert torch.equal(some, out[rows.long()])
 
 
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("which", ["h", "delta", "weight", "out"])
+def test_the_norm_of_many_rows_takes_operands_that_begin_anywhere(k, splits, which):
+    """One operand a value behind 16 bytes: the values of the aligned call, up to the order of a row's sum of 104 squares."""
+    t, hidden = 70, 104
+
+    def place(v, name):
+        if name != which:
+            return v
+        whole = torch.empty(v.numel() + 16, dtype=v.dtype, device="cuda")
+        moved = whole[1 : 1 + v.numel()].view(v.shape)
+        moved.copy_(v)
+        return moved
+
+    h, weight = rnd(t, hidden, seed=7).float(), rnd(hidden, seed=8)
+    delta = rnd(t, hidden, seed=9) if splits == 0 else torch.randn(splits, t, hidden, generator=torch.Generator().manual_seed(9)).cuda()
+    want_h, want = h.clone(), torch.empty((t, hidden), dtype=torch.bfloat16, device="cuda")
+    k.add_rmsnorm(want_h, delta, weight, 1e-6, want)
+    got_h, got = place(h.clone(), "h"), place(torch.zeros_like(want), "out")
+    k.add_rmsnorm(got_h, place(delta, "delta"), place(weight, "weight"), 1e-6, got)
+    assert torch.equal(got_h, want_h)
+    assert ((got.double() - want.double()).abs() <= want.double().abs() * 2.0 ** -7).all()
+
+
 @pytest.mark.parametrize("tile_rows", [64, 128])
 @pytest.mark.parametrize("t,top,experts,outputs,hidden,ff", [(1, 1, 1, 1, 64, 64), (5, 3, 4, 6, 128, 64), (150, 2, 5, 7, 64, 192),
                                                              (130, 1, 3, 3, 192, 128), (40, 4, 700, 1000, 64, 64)])
