@@ -80,3 +80,45 @@ def test_a_plan_is_found_once_for_its_sizes():
         assert all(plan(*sizes) == first for _ in range(24))         # a step's layers
         after = plan.cache_info()
         assert after.hits == before.hits + 24 and after.misses == before.misses and after.maxsize is not None
+
+
+WIDTHS = [64, 128, 320, 896, 1024, 1152, 1536, 2048, 2752, 3584, 4608, 4864, 8960, 9728, 18944, 37888, 151936]
+ROWS = [65, 66, 96, 127, 128, 129, 192, 256, 257, 448, 552, 1000, 1537, 2048, 3584, 4097, 8191, 32768, 100003]
+
+
+def test_plans_of_many_rows_are_launchable():
+    # what egpt_gemm_rows refuses: shapes that do not exist, empty ranges of k, more workgroups than a grid holds
+    for m, n, k, most in itertools.product(ROWS, WIDTHS, [w for w in WIDTHS if w % 64 == 0], (1, 10)):
+        shape, s = K._rows_plan(m, n, k, most)
+        bm, bn = K._rows_shapes[shape][:2]
+        steps = k // 64
+        per = -(-steps // s)
+        what = (m, n, k, most, shape, s)
+        assert 1 <= s <= min(most, steps) and (s - 1) * per < steps, what
+        assert -(-m // bm) * -(-n // bn) * s <= 0x7FFFFFFF, what
+
+
+def test_plans_of_the_float32_product_are_launchable():
+    # what egpt_gemm_f32 and egpt_gemm_f32_rows refuse; up to 64 rows always the kernel for few, nothing is folded there
+    for m, n, k in itertools.product([1, 17, 64] + ROWS, WIDTHS + [5, 36], WIDTHS + [4, 100]):
+        for s in {1, K._f32_splits(n, k)}:
+            rows, fold = K._f32_rows_plan(m, n, k, s)
+            what = (m, n, k, s, rows, fold)
+            assert rows in ((0,) if m <= 64 else (0, 64, 128)), what
+            assert not fold or (s > 1 and rows), what
+            if rows:
+                assert -(-m // rows) * -(-n // 128) <= 0x7FFFFFFF, what
+            else:
+                assert -(-m // 64) <= 65535 and s <= 65535, what
+
+
+def test_the_rules_for_many_rows_change_sides_once():
+    # more rows than a product that goes to the library go there too; a gate product leaves its kernel for good as rows grow,
+    # and on large matrices begins with the library
+    rows = list(range(65, 9000, 61))
+    for n, k, unrounded in itertools.product(WIDTHS, WIDTHS, (False, True)):
+        own = [K._own_rows(m, n, k, unrounded) for m in rows]
+        assert own == sorted(own, reverse=True), (n, k, unrounded)
+    for k in WIDTHS + [3072, 4096, 5120, 8192]:
+        own = [K._own_gate(m, k) for m in rows]
+        assert sum(a != b for a, b in zip(own, own[1:])) <= 2, k
