@@ -452,7 +452,7 @@ class HipKernels(KernelBackend):
         give the same bits.  Costs in us, fitted to 64 to 1,811 rows of 1,152 x 896, 9,728 x 896 and 896 x 4,864 (in 7, 5 and 11
         ranges): a CU holds one workgroup, which takes 5 us and 0.96 per block of 32 values of k for 64 x 128, 7 and 1.33 for
         128 x 128; the kernel for few rows takes 1.85 per group of 64 rows and million elements of w and writes at 2.75
-        TB/s; partial sums are written and read at 4.5 TB/s.  (24 layers of these for 1,811 rows, all else included: 13.8 ms, 21.1
+        TB/s; partial sums are written and read at 4.5 TB/s.  (24 layers of these for 1,811 rows, all else included: 14.3 ms, 21.1
         with the float32 matrix instructions, whose partial sums the readers added up.)"""
         if m <= 64:
             return 0, False
