@@ -79,11 +79,11 @@ int launch_tiled(const void* x, const void* w, const void* bias, void* out, int 
 // is taken back by 2^48 and added to the element's in float32.  Error against 64 bits (2-norm, k = 896 / 4,864): 1.1e-7 / 2.4e-7,
 // with v_mfma_f32_16x16x4_f32, which took its operands as they are and rounded after every fourth product, 5.4e-7 / 1.25e-6; with
 // one chain over all blocks 4.5e-7 / 1.1e-6.  (The power of two is a product per operand: nothing with up to 64 rows, 5 to 8 % of
-// the tiles of many rows: 1,811 and 4,096 rows of 9,728 x 896 in 235 and 480 us, 219 and 452 without it.)
+// a tile of 128 rows: 1,811 and 4,096 rows of 9,728 x 896 in 235 and 480 us, 219 and 452 without it.)
 // Values that have no such three parts (infinities, NaN, from 2^104 on) and block sums beyond 2^80 leave an element that is no
 // finite number.  A wavefront that holds one adds its tile up again with v_mfma_f32_16x16x4_f32, which takes
-// float32 operands whole, and takes those elements from there.  (1,811 rows of 9,728 x 896, us: 277, 321 with one row of NaN,
-// 868 with nothing else; 8 rows 8.7 and 15.0.)
+// float32 operands whole, and takes those elements from there.  (1,811 rows of 9,728 x 896, us: 251, 280 with one row of NaN,
+// 737 with nothing else; 8 rows 8.7 and 15.0.)
 //
 // Every element of the result is the same sequence of operations whatever m is and wherever its row lies in x, in all
 // kernels here: block after block of 32 values within a range of k, ranges of k one after the other.  So a token's values do not
@@ -319,6 +319,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_mfma_kernel(const float* __r
 // two blocks ahead), eight wavefronts of 32 x 64.  A block's parts lie in LDS as rows of 64 bytes whose four pieces of 16
 // bytes are exchanged by the row's number (piece p of row r in place p ^ (r / 2 & 3)), so that the lanes that read one
 // piece of many rows hit different banks; two buffers, one barrier a block.
+// With 64 rows of x the workgroup is half as large and a CU holds two (LDS, and up to 256 registers): 1,811 and 4,096 rows of 9,728 x
+// 896 in 224 and 489 us, one to a CU 271 and 593 (each lane had more than 256 registers); with 128 rows 235 and 480.
 // FOLD: a workgroup walks all ranges of k and adds their sums up in their order, which is what a reader of partial sums does:
 // the same bits, without the partial sums' traffic.
 // TAIL: k is no multiple of a block (its end is filled with zeros).

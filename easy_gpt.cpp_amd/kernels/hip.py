@@ -449,21 +449,25 @@ class HipKernels(KernelBackend):
     @functools.lru_cache(maxsize=4096)
     def _f32_rows_plan(m: int, n: int, k: int, s: int) -> tuple[int, bool]:
         """(rows of a tile, ranges of k added up inside) of the float32 product; 0 rows: the kernel for few rows.  All of them
-        give the same bits.  Costs in us, fitted to 64 to 1,811 rows of 1,152 x 896, 9,728 x 896 and 896 x 4,864 (in 7, 5 and 11
-        ranges): a CU holds one workgroup, which takes 5 us and 0.96 per block of 32 values of k for 64 x 128, 7 and 1.33 for
-        128 x 128; the kernel for few rows takes 1.85 per group of 64 rows and million elements of w and writes at 2.75
-        TB/s; partial sums are written and read at 4.5 TB/s.  (24 layers of these for 1,811 rows, all else included: 14.3 ms, 21.1
-        with the float32 matrix instructions, whose partial sums the readers added up.)"""
+        give the same bits.  Costs in us, fitted to 65 to 8,191 rows of twelve matrices from 256 x 256 to 17,920 x 1,536 with the
+        norm that reads the result (the choice is 0.4 % slower than the best of everything measured on average, 7 % at worst): a
+        workgroup takes 1.07 per block of 32 values of k for 64 x 128, or 1.59 with the second one that a CU holds, 1.5 for 128 x 128,
+        which has a CU to itself; the kernel for few rows takes 1.73 per group of 64 rows and million elements of w; partial sums
+        cost what is written and read beyond one sum, and their reader 7 ns a row.  (24 layers of the 0.5B sizes for 1,811 rows, all
+        else included: 13.3 ms, 21.1 with the float32 matrix instructions, whose partial sums the readers added up.)"""
         if m <= 64:
             return 0, False
         blocks, cols = -(-k // 32), -(-n // 128)
-        read = m * n * 4 / 4.5e6
-        plans = [(-(-m // 64) * (n * k * 1.85e-6 + s * n * 256 / 2.75e6) + 2 + s * read, 0, False)]
-        for rows, fixed, per_block in ((64, 5.0, 0.96), (128, 7.0, 1.33)):
-            tiles = -(-m // rows) * cols
-            if s > 1:
-                plans.append((5 + -(-tiles // 256) * (fixed + blocks * per_block) + read, rows, True))
-            plans.append((5 + -(-tiles * s // 256) * (fixed + -(-blocks // s) * per_block) + 2 * s * read, rows, False))
+        many = 0.22 * (s - 1) * m * n * 4e-6 + 0.007 * m if s > 1 else 0.0
+        plans = [(3.7 + -(-m // 64) * n * k * 1.73e-6 + many, 0, False)]
+        for rows, held, fixed, alone, full in ((64, 2, 2.6, 1.07, 1.59), (128, 1, 3.8, 1.5, 1.5)):
+            for fold in ((True, False) if s > 1 else (False,)):
+                rounds, rest = divmod(-(-m // rows) * cols * (1 if fold else s), 256 * held)
+                per = blocks if fold else -(-blocks // s)
+                us = 2.4 + rounds * (fixed + per * full)
+                if rest:
+                    us += fixed + per * (alone if rest <= 256 else full)
+                plans.append((us + (0.0 if fold else many), rows, fold))
         return min(plans)[1:]
 
     def _f32_product(self, x, w, bias, out, s: int, plan: tuple[int, bool]) -> None:
