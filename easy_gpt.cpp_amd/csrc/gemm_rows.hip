@@ -10,16 +10,24 @@
 // half's operands in registers already; behind it the next loads go out and the next step's first half is read under the
 // second half's products.
 //
-// What bounds it: alone, the loop runs at 1.9 PFLOP/s on zeros and 1.6 on random numbers (the card then lowers its clock).
+// A workgroup stays for several tiles: as many are launched as the CUs hold, and the loads of a workgroup's next tile go out under
+// the last steps of the one before, so that a tile's first products do not wait for memory and the result leaves meanwhile.
+//
+// What bounds it: alone, the loop runs at 1.9 PFLOP/s on zeros and 1.6 on random numbers (the card then lowers its clock): 2,640
+// cycles a step of 256 x 256, where the products take 2,048, and so do the LDS's reads and writes together.  Beside its steps
+// a tile of 256 x 256 takes 10,000 cycles when it is activated (47,000 in all at 14 steps of k): 128 exponentials and
+// reciprocals a lane, each of four issues, and the instructions around them, two wavefronts to a SIMD.  What it was before: a
+// workgroup per tile, expf and the division in full, all rows of x before the next columns (us, weights from memory): 2,048 rows
+// x 9,728 x 896 gated 53.3 -> 41.2, 8,191 x 9,728 x 896 172 -> 127, 8,191 x 17,920 x 1,536 444 -> 351, 2,048 x 37,888 x 3,584 461 -> 416;
+// 8,191 x 896 x 896 23.1 -> 18.2.  Of that the strips of eight tiles of rows (`item_of`) are the 8,191 x 17,920 x 1,536's 442 -> 361: an
+// XCD's 32 workgroups otherwise read 32 tiles of x for one of w.  Four wavefronts of 128 x 128 (fewer LDS reads): the registers do
+// not suffice, 3,300 cycles a step.
 // The weights come from memory, and all workgroups that share a tile of w ask for it at the same time, so nobody finds it in
-// the L2 and everybody waits for memory's latency: with one step of both operands on its way, 2,048 x 37,888 x 3,584 took
-// 486 us; with two of w and one of x (160 KB of LDS) 461, and on zeros 470 against 393.  Deeper rings in steps of 32 values
-// (64-byte pieces of rows) gained nothing: 509.  32x32x16 products: the same on zeros, 7 % slower on random numbers.  The
-// order of tiles: a die gets neighbouring tiles of one range of k (2,048 x 3,584 x 18,944 in two ranges: 247 -> 238 us).
-// Against the library's first choice (us, weights from memory; gated ones with its activation kernel, others with the norm that
-// reads the result): 2,048 rows x 18,944 gated x 3,584 456 against 547, 8,191 x 8,960 gated x 1,536 436 against 446; 2,048 x 3,584 x
-// 18,944 238 against 382, 552 x 1,536 x 8,960 33 against 43, 552 x 896 x 896 11.0 against 12.6; but 8,191 x 18,944 gated x 3,584
-// 1,871 against 1,818 and 2,048 x 2,048 x 1,536 30 against 28.  `_own_rows` and `_own_gate` in kernels/hip.py draw the lines.
+// the L2 and everybody waits for memory's latency: two steps of w and one of x are on their way (160 KB of LDS).  Deeper rings in
+// steps of 32 values (64-byte pieces of rows) gained nothing, 32x32x16 products are 7 % slower on random numbers.
+// `_own_rows`, `_own_short` and `_own_gate` in kernels/hip.py draw the lines to the library, with both sides' times.
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -27,18 +35,19 @@ namespace egpt {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 r_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float r_f32x4;
-typedef __attribute__((ext_vector_type(4))) unsigned short r_u16x4;
+typedef __attribute__((ext_vector_type(4))) __bf16 r_bf16x4;
+typedef __attribute__((ext_vector_type(2))) unsigned r_u32x2;
+typedef __attribute__((ext_vector_type(4))) unsigned r_u32x4;
 typedef __attribute__((address_space(3))) void lds_void;
 
+constexpr int kLdsOfCu = 160 * 1024;
+constexpr int kStrip = 8;                      // tiles of rows that are walked together, column by column
 constexpr int kRowsStep = 64;                  // values of k per step: 128 bytes a row
 
-// At most N of this wavefront's loads into LDS are still on their way, and its LDS reads are done; then all wavefronts meet.
-// (The loads are written in assembly and have no result in registers; __syncthreads() alone does not wait for them.)
+// At most N of this wavefront's memory operations are still on their way (they end in the order in which they were made).
+// The loads into LDS are written in assembly and have no result in registers; __syncthreads() alone does not wait for them.
 template <int N>
-__device__ __forceinline__ void landed() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | 0x0f70 | (N >> 4) << 14);
-    __syncthreads();
-}
+__device__ __forceinline__ void arrived() { __builtin_amdgcn_s_waitcnt((N & 15) | 0x0f70 | (N >> 4) << 14); }
 
 typedef __attribute__((ext_vector_type(4))) int r_i32x4;
 
@@ -57,6 +66,31 @@ __device__ __forceinline__ r_i32x4 buffer_of(const void* p, size_t bytes) {
                    __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000};
 }
 
+// gate_activation of four values.  A wavefront issues a vector instruction in four cycles and holds 64 gates a lane, so what an
+// activation takes is seen in the kernel: expf and the division with their cases spelled out are some 45 instructions a value
+// (5 us of a tile of 256 x 256), these 13.  exp2 of a product whose rounding error is put back, a reciprocal made good by the
+// division's remainder: no case of either arises while |exponent| < 87; beyond it the general form.
+template <int ACT>
+__device__ __forceinline__ r_f32x4 gate4(r_f32x4 z) {
+    r_f32x4 v;
+    float most = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float y = gate_exponent(z[e], ACT);
+        most = fmaxf(most, fabsf(y));
+        const float t = y * -1.442695041f;
+        float p = __builtin_amdgcn_exp2f(t);
+        p = fmaf(p, fmaf(t, -0.6931471806f, -y), p);
+        const float d = 1.0f + p, r = __builtin_amdgcn_rcpf(d), q = z[e] * r;
+        v[e] = fmaf(fmaf(-q, d, z[e]), r, q);
+    }
+    if (!(most < 87.f)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = gate_activation(z[e], ACT);
+    }
+    return v;
+}
+
 enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsGated = 2, kRowsRelu2 = 3 };
 
 // Products of rows grouped by expert (moe.hip makes the table of tiles): tile i has rows tiles[3 i + 2 ..] of one expert, the
@@ -68,7 +102,7 @@ struct Groups {
 };
 
 template <int BM, int BN, int WM, int WN, int WB, int OUT, bool GROUPED>
-__global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
+__global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) void gemm_rows_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k, int splits,
     int steps_per_split, int act, Groups groups) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -83,66 +117,97 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
     const int li = lane % 16, lg = lane / 16;
     const int wm = wave / WN, wn = wave % WN;
 
-    // workgroups are handed to the eight dies in turn: a die gets a contiguous range of tiles, rows of x fastest, so that
-    // its L2 holds the few rows of w and x that its tiles share
+    // Workgroups are handed to the eight dies in turn: a die gets a contiguous range of items, rows of x fastest, so that
+    // its L2 holds the few rows of w and x that its tiles share.  A workgroup takes items blockIdx.x, blockIdx.x +
+    // gridDim.x ... (a grid of several items to a workgroup is a multiple of eight).
     constexpr int BC = OUT == kRowsGated ? BN / 2 : BN;         // columns of the result in a tile
     const int mt = GROUPED ? groups.tiles[0] : (m + BM - 1) / BM, nt = (n + BC - 1) / BC;
     const int tiles = mt * nt, items = tiles * splits;
-    int item = blockIdx.x;
-    if (GROUPED && item >= items) return;                      // (the grid is sized for the most tiles that the rows can make)
-    {
-        const int q = items / 8, r = items % 8, d = item % 8, i = item / 8;
-        item = d * q + (d < r ? d : r) + i;
-    }
-    const int tile = item % tiles, split = item / tiles;
-    int m0 = tile % mt * BM, n0 = tile / mt * BC, rows = min(m - m0, BM);
-    if (GROUPED) {
-        // all columns of a tile of rows after each other: an expert's matrix stays in the die's L2 for its tiles
-        const int32_t* entry = groups.tiles + 1 + 3 * (item / nt);
-        m0 = entry[1];
-        n0 = item % nt * BC;
-        rows = entry[2];
-        w += static_cast<size_t>(entry[0]) * (OUT == kRowsGated ? 2 * n : n) * k;
-    }
+    const int strips = (mt + kStrip - 1) / kStrip, per_strip = (mt + strips - 1) / strips;
+    if (GROUPED && static_cast<int>(blockIdx.x) >= items) return;      // (the grid is sized for the most tiles that the rows can make)
     const int total = k / kRowsStep;
-    const int s_begin = split * steps_per_split, s_end = min(total, s_begin + steps_per_split);
-
-    // ---- loads: a lane's byte offsets from the tile's first rows (rows beyond the last repeat the last)
-    const int piece = (lane % 8) ^ (lane / 8);
     const size_t row_bytes = static_cast<size_t>(k) * 2;
     const bool gather = GROUPED && groups.row_token != nullptr;
-    const r_i32x4 xr = gather ? buffer_of(x, groups.x_rows * row_bytes) : buffer_of(x + static_cast<size_t>(m0) * k, rows * row_bytes);
-    const r_i32x4 wr = buffer_of(w + static_cast<size_t>(n0) * k, (OUT == kRowsGated ? 2 * n - n0 : min(n - n0, BN)) * row_bytes);
+    struct Item {
+        int m0, n0, rows, split, begin, end;               // first row, first column, rows, range of k: its number, its steps
+        r_i32x4 x, w;                                      // operands from the tile's first row on (nothing beyond its last)
+    };
+    auto item_of = [&](int index) {
+        Item it;
+        if (index >= items) {                              // none: loads from it touch no memory
+            it.m0 = it.n0 = it.rows = it.split = it.begin = it.end = 0;
+            it.x = buffer_of(x, 0);
+            it.w = buffer_of(w, 0);
+            return it;
+        }
+        const int q = items / 8, r = items % 8, d = index % 8;
+        const int item = d * q + (d < r ? d : r) + index / 8;
+        const bf16_t* from = w;
+        if (GROUPED) {
+            // all columns of a tile of rows after each other: an expert's matrix stays in the die's L2 for its tiles
+            const int32_t* entry = groups.tiles + 1 + 3 * (item / nt);
+            it.m0 = entry[1];
+            it.n0 = item % nt * BC;
+            it.rows = entry[2];
+            it.split = 0;
+            from += static_cast<size_t>(entry[0]) * (OUT == kRowsGated ? 2 * n : n) * k;
+        } else {
+            it.split = item / tiles;
+            const int tile = item - it.split * tiles, strip = tile / (per_strip * nt), top = strip * per_strip;
+            const int high = min(per_strip, mt - top), at = tile - top * nt, column = at / high;
+            it.m0 = (top + at - column * high) * BM;
+            it.n0 = column * BC;
+            it.rows = min(m - it.m0, BM);
+        }
+        it.begin = it.split * steps_per_split;
+        it.end = min(total, it.begin + steps_per_split);
+        it.x = gather ? buffer_of(x, groups.x_rows * row_bytes) : buffer_of(x + static_cast<size_t>(it.m0) * k, it.rows * row_bytes);
+        it.w = buffer_of(from + static_cast<size_t>(it.n0) * k, (OUT == kRowsGated ? 2 * n - it.n0 : min(n - it.n0, BN)) * row_bytes);
+        return it;
+    };
+    int index = blockIdx.x;
+    Item now = item_of(index);
+
+    // ---- loads: a lane's byte offsets from the tile's first rows, the same for every tile (what lies beyond an operand's
+    // last row reads as zero; gate columns beyond the last are up columns, and nobody stores them)
+    const int piece = (lane % 8) ^ (lane / 8);
     int xo[XL], wo[WL];
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
-        const int r = (wave * XL + i) * 8 + lane / 8;
-        int g = min(r, rows - 1);
-        if (gather) g = groups.row_token[m0 + g];
+        int g = (wave * XL + i) * 8 + lane / 8;
+        if (gather) g = groups.row_token[now.m0 + min(g, now.rows - 1)];
         xo[i] = g * static_cast<int>(row_bytes) + piece * 16;
     }
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
         const int r = (wave * WL + i) * 8 + lane / 8;
-        int g = min(r, n - n0 - 1);
+        int g = r;
         if (OUT == kRowsGated) {
             // a wavefront's columns: the first half of them gates, the second half the up columns of the same numbers
             constexpr int C = BN / WN;
-            const int col = r / C * (C / 2) + r % (C / 2);
-            g = min(col, n - n0 - 1) + (r % C >= C / 2 ? n : 0);
+            g = r / C * (C / 2) + r % (C / 2) + (r % C >= C / 2 ? n : 0);
         }
         wo[i] = g * static_cast<int>(row_bytes) + piece * 16;
     }
-    const int last = s_end - 1;                              // (beyond the last step the last one again, which nobody reads)
-    auto load_x = [&](int buffer, int step) {
-        const int at = min(step, last) * (kRowsStep * 2);
-#pragma unroll
-        for (int i = 0; i < XL; ++i) load_to_lds(xr, xo[i], at, xs + buffer * kXBytes + (wave * XL + i) * 1024);
+    // where the next step's loads of an operand come from: `left` steps of an item from byte `at` of its rows on, `by` further
+    // each (an item that is none stays where it is)
+    struct Source {
+        r_i32x4 rows;
+        int at, by, left;
     };
-    auto load_w = [&](int buffer, int step) {
-        const int at = min(step, last) * (kRowsStep * 2);
+    auto source_x = [&](const Item& it) { return Source{it.x, it.begin * (kRowsStep * 2), it.rows > 0 ? kRowsStep * 2 : 0, it.rows > 0 ? it.end - it.begin : 1 << 30}; };
+    auto source_w = [&](const Item& it) { return Source{it.w, it.begin * (kRowsStep * 2), it.rows > 0 ? kRowsStep * 2 : 0, it.rows > 0 ? it.end - it.begin : 1 << 30}; };
+    auto load_x = [&](int buffer, Source& from) {
 #pragma unroll
-        for (int i = 0; i < WL; ++i) load_to_lds(wr, wo[i], at, ws + buffer * kWBytes + (wave * WL + i) * 1024);
+        for (int i = 0; i < XL; ++i) load_to_lds(from.rows, xo[i], from.at, xs + buffer * kXBytes + (wave * XL + i) * 1024);
+        from.at += from.by;
+        --from.left;
+    };
+    auto load_w = [&](int buffer, Source& from) {
+#pragma unroll
+        for (int i = 0; i < WL; ++i) load_to_lds(from.rows, wo[i], from.at, ws + buffer * kWBytes + (wave * WL + i) * 1024);
+        from.at += from.by;
+        --from.left;
     };
     // ---- operands of a half step
     const int xa = (wm * (BM / WM) + li) * 128, wa = (wn * (BN / WN) + li) * 128;
@@ -157,10 +222,12 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
         for (int i = 0; i < TM; ++i) xf[h][i] = *reinterpret_cast<const r_bf16x8*>(xfrom + i * 2048);
     };
     r_f32x4 acc[TM][TN];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = r_f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < TN; ++j) acc[i][j] = r_f32x4{0.f, 0.f, 0.f, 0.f};
+    };
     auto multiply = [&](int h) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -175,64 +242,121 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_rows_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    load_x(0, s_begin);
-    load_w(0, s_begin);
-    load_x(1, s_begin + 1);
+    // ---- the result: a lane holds columns 4 lg .. 4 lg + 3 of row li of every 16 x 16 tile (n is a multiple of four).  Rounded
+    // results of two neighbouring tiles change places between lanes, so that a lane stores 16 bytes and four of them 64 bytes
+    // of a row (8,191 x 896 x 896: 21.0 us with 8 bytes a lane, 18.2 so).  Every
+    // wavefront makes at least kStores stores whatever the tile's edges are (those beyond an edge go nowhere), so that the
+    // first wait of the next item can count them.
+    constexpr int TC = OUT == kRowsGated ? TN / 2 : TN;
+    constexpr bool kPairs = OUT != kRowsF32 && TC % 2 == 0;
+    constexpr int kStores = kPairs ? TM * TC / 2 : TM * TC;
+    constexpr int kOutBytes = OUT == kRowsF32 ? 4 : 2;
+    auto store_as = [&](auto activation) {
+        constexpr int ACT = decltype(activation)::value;
+        char* from = static_cast<char*>(out) + (static_cast<size_t>(now.split) * m + now.m0) * n * kOutBytes;
+        const auto to = __builtin_amdgcn_make_buffer_rsrc(from, 0, now.rows * n * kOutBytes, 0x00020000);
+        const int col0 = now.n0 + wn * (BC / WN);
+        auto value = [&](int i, int j) {
+            r_f32x4 v = acc[i][j];
+            if constexpr (OUT == kRowsGated) v = gate4<ACT>(v) * acc[i][j + TN / 2];
+            if constexpr (OUT == kRowsRelu2) {
 #pragma unroll
-    for (int i = 1; i < WB; ++i) load_w(i, s_begin + i);
-    landed<0>();
-    read(0, 0, 0);
-    int xb = 0, wb = 0;
-#pragma unroll 1
-    for (int s = s_begin; s < s_end; ++s) {
-        const int xn = xb ^ 1, wnext = wb + 1 == WB ? 0 : wb + 1;
-        read(xb, wb, 1);
-        multiply(0);
-        landed<(WB - 2) * WL>();
-        __builtin_amdgcn_sched_barrier(0);
-        load_x(xb, s + 2);
-        load_w(wb, s + WB);
-        read(xn, wnext, 0);
-        multiply(1);
-        xb = xn;
-        wb = wnext;
-    }
-    __builtin_amdgcn_s_waitcnt(0x0f70);                      // (nothing is on its way to LDS when the workgroup ends)
-    // ---- a lane holds columns 4 lg .. 4 lg + 3 of row li of every 16 x 16 tile (n is a multiple of four)
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int at = wm * (BM / WM) + i * 16 + li, row = m0 + at;
-        if (at >= rows) continue;
-        if constexpr (OUT == kRowsGated) {
-#pragma unroll
-            for (int j = 0; j < TN / 2; ++j) {
-                const int col = n0 + wn * (BN / WN / 2) + j * 16 + lg * 4;
-                bf16_t* o = static_cast<bf16_t*>(out) + static_cast<size_t>(row) * n + col;
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = gate_activation(acc[i][j][e], act) * acc[i][j + TN / 2][e];
-                if (col < n)
-                    *reinterpret_cast<r_u16x4*>(o) = r_u16x4{f32_to_bf16_bits(v[0]), f32_to_bf16_bits(v[1]), f32_to_bf16_bits(v[2]), f32_to_bf16_bits(v[3])};
+                for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
             }
-        } else {
+            return v;
+        };
+        auto rounded = [&](int i, int j) { return __builtin_bit_cast(r_u32x2, __builtin_convertvector(value(i, j), r_bf16x4)); };
+        if (kPairs && n % 8 == 0) {
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int col = n0 + wn * (BN / WN) + j * 16 + lg * 4;
-                if constexpr (OUT == kRowsF32) {
-                    float* o = static_cast<float*>(out) + (static_cast<size_t>(split) * m + row) * n + col;
-                    if (col < n) *reinterpret_cast<r_f32x4*>(o) = acc[i][j];
-                } else {
-                    bf16_t* o = static_cast<bf16_t*>(out) + static_cast<size_t>(row) * n + col;
-                    r_f32x4 v = acc[i][j];
-                    if constexpr (OUT == kRowsRelu2)
+            for (int i = 0; i < TM; ++i) {
+                const int at = (wm * (BM / WM) + i * 16 + li) * n;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
-                    if (col < n)
-                        *reinterpret_cast<r_u16x4*>(o) = r_u16x4{f32_to_bf16_bits(v[0]), f32_to_bf16_bits(v[1]), f32_to_bf16_bits(v[2]), f32_to_bf16_bits(v[3])};
+                for (int j = 0; j < TC / 2 * 2; j += 2) {
+                    const r_u32x2 a = rounded(i, j), b = rounded(i, j + 1);
+                    const r_u32x2 p = __builtin_bit_cast(r_u32x2, __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false));
+                    const r_u32x2 q = __builtin_bit_cast(r_u32x2, __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false));
+                    const int col = col0 + (j + lg % 2) * 16 + lg / 2 * 8;
+                    __builtin_amdgcn_raw_buffer_store_b128(r_u32x4{p[0], q[0], p[1], q[1]}, to, col < n ? (at + col) * 2 : 0x7ffffff0, 0, 0);
                 }
             }
+            return;
         }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int at = (wm * (BM / WM) + i * 16 + li) * n;
+#pragma unroll
+            for (int j = 0; j < TC; ++j) {
+                const int col = col0 + j * 16 + lg * 4, offset = col < n ? (at + col) * kOutBytes : 0x7ffffff0;
+                if constexpr (OUT == kRowsF32) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(r_u32x4, value(i, j)), to, offset, 0, 0);
+                else __builtin_amdgcn_raw_buffer_store_b64(rounded(i, j), to, offset, 0, 0);
+            }
+        }
+    };
+    auto store = [&]() {
+        if (OUT == kRowsGated && act != kGateSilu) store_as(std::integral_constant<int, kGateGeluTanh>());
+        else store_as(std::integral_constant<int, kGateSilu>());
+    };
+    Source fx = source_x(now), fw = source_w(now);
+    const Item none = item_of(items);
+    load_x(0, fx);
+    load_w(0, fw);
+    if (fx.left == 0) fx = source_x(none);
+    if (fw.left == 0) fw = source_w(none);
+    load_x(1, fx);
+#pragma unroll
+    for (int i = 1; i < WB; ++i) {
+        load_w(i, fw);
+        if (fw.left == 0 && i + 1 < WB) fw = source_w(none);
     }
+    // (where there is a next item, this one has WB steps at least)
+    Item next = item_of(index + gridDim.x);
+    clear();
+    arrived<0>();
+    __syncthreads();
+    read(0, 0, 0);
+    int xb = 0, wb = 0, left = now.end - now.begin;
+    auto step = [&]() {
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        load_x(xb, fx);
+        load_w(wb, fw);
+        xb ^= 1;
+        wb = wb + 1 == WB ? 0 : wb + 1;
+        read(xb, wb, 0);
+        multiply(1);
+        --left;
+    };
+    bool stored = false;
+#pragma unroll 1
+    for (;;) {
+        // an item's first step and its last WB ones, under which the loads of the workgroup's next item begin
+        read(xb, wb, 1);
+        multiply(0);
+        if (stored) arrived<((WB - 2) * WL + kStores < 63 ? (WB - 2) * WL + kStores : 63)>();
+        else arrived<(WB - 2) * WL>();
+        stored = false;
+        if (fx.left == 0) fx = source_x(next);
+        if (fw.left == 0) fw = source_w(next);
+        step();
+        // those between, a line of their own without branches (a branch in every step: 1.4 us a step of 256 x 256 against 1.2)
+#pragma unroll 1
+        while (left > WB) {
+            read(xb, wb, 1);
+            multiply(0);
+            arrived<(WB - 2) * WL>();
+            step();
+        }
+        if (left > 0) continue;
+        store();
+        if (next.rows == 0) break;
+        clear();
+        stored = true;
+        index += gridDim.x;
+        now = next;
+        next = item_of(index + gridDim.x);
+        left = now.end - now.begin;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);                      // (nothing is on its way to LDS when the workgroup ends)
 #endif
 }
 
@@ -240,7 +364,12 @@ template <int BM, int BN, int WM, int WN, int WB>
 int launch_rows(const void* x, const void* w, void* out, int m, int n, int k, int splits, int per, int kind, int act, hipStream_t s) {
     const long mt = (m + BM - 1) / BM, nt = kind == kRowsGated ? (n + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
     if (mt * nt * splits > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
-    const dim3 grid(static_cast<unsigned>(mt * nt * splits));
+    // as many workgroups as the CUs hold, each taking its items in turn, where every item has the three steps that are on
+    // their way when it begins; else a workgroup per item
+    constexpr int kHeld = kLdsOfCu / ((2 * BM + WB * BN) * 128);
+    const int last_steps = k / kRowsStep - (splits - 1) * per;
+    const long held = per >= WB && last_steps >= WB ? 256L * kHeld : mt * nt * splits;
+    const dim3 grid(static_cast<unsigned>(mt * nt * splits < held ? mt * nt * splits : held));
     const auto* xp = static_cast<const bf16_t*>(x);
     const auto* wp = static_cast<const bf16_t*>(w);
     const Groups none{nullptr, nullptr, 0};
@@ -275,8 +404,8 @@ extern "C" int egpt_gemm_rows(const void* x, const void* w, void* out, int m, in
     if (!x || !w || !out || m < 0 || n <= 0 || k <= 0 || splits < 1 || kind < 0 || kind > kRowsGated || act < 0 || act > 1) return EGPT_BAD_ARGUMENT;
     if (k % kRowsStep != 0 || n % 4 != 0 || (splits != 1 && kind != kRowsF32)) return EGPT_UNSUPPORTED_SIZE;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16) return EGPT_UNSUPPORTED_SIZE;
-    // a lane's byte offsets from its tile's first row are 32-bit numbers
-    if (static_cast<long long>(k) * 2 * (kind == kRowsGated ? 2LL * n : 256) > 0x7fffffffLL) return EGPT_UNSUPPORTED_SIZE;
+    // a lane's byte offsets from its tile's first row are 32-bit numbers, in the operands and in the result
+    if (static_cast<long long>(k) * 2 * (kind != kRowsGated ? 256 : n > 256 ? 2LL * n : n + 256LL) > 0x7fffffffLL || n > 0x1fffff) return EGPT_UNSUPPORTED_SIZE;
     if (m == 0) return EGPT_OK;
     const int total = k / kRowsStep, per = (total + splits - 1) / splits;
     if (splits > total || (splits - 1) * per >= total) return EGPT_BAD_ARGUMENT;      // an empty range
@@ -300,7 +429,7 @@ extern "C" int egpt_moe_rows(const void* x, const void* w, const int32_t* row_to
     if (k % kRowsStep != 0 || n % 4 != 0) return EGPT_UNSUPPORTED_SIZE;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16) return EGPT_UNSUPPORTED_SIZE;
     // byte offsets within x (gathered rows) and within an expert's matrix are 32-bit numbers
-    if (static_cast<long long>(k) * 2 * x_rows > 0x7fffffffLL || static_cast<long long>(k) * 2 * 2 * n > 0x7fffffffLL) return EGPT_UNSUPPORTED_SIZE;
+    if (static_cast<long long>(k) * 2 * (x_rows > 128 ? x_rows : 128) > 0x7fffffffLL || static_cast<long long>(k) * 2 * (n > 128 ? 2LL * n : n + 128LL) > 0x7fffffffLL || n > 0x3fffff) return EGPT_UNSUPPORTED_SIZE;
     if (n_rows == 0) return EGPT_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const Groups g{tiles, row_token, x_rows};

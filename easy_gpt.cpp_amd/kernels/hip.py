@@ -323,7 +323,7 @@ class HipKernels(KernelBackend):
     def _rows_fit(x, w, k: int) -> bool:
         """Whether gemm_rows.hip takes these operands."""
         return (x.dtype == _BF16 and w.dtype == _BF16 and k % 64 == 0 and w.shape[0] % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
-                and w.shape[0] * k < 1 << 30)
+                and w.shape[0] * k < 1 << 30 and max(w.shape[0], k) < 1 << 21)
 
     @staticmethod
     def _own_rows(m: int, n: int, k: int, unrounded: bool) -> bool:
@@ -361,6 +361,16 @@ class HipKernels(KernelBackend):
         # themselves, times over the library's: 4,608 x 3,584 at 200 / 300 / 448 rows 0.79 / 0.98 / 1.24, 4,096 x 2,048 at 128 / 200 / 320 0.88 /
         # 1.12 / 1.24.
         return m <= 448 if n <= k else n < 2 * k and m <= 256
+
+    @staticmethod
+    def _own_short(n: int, k: int) -> bool:
+        """Whether the product is the framework's own with every number of rows above 64, also beyond the lines of `_own_rows`: a short k
+        range makes a tile of its beginning and its end for the most part, and a workgroup's next tile begins under the
+        end of the one before.  us, weights from memory, rounded: 896 x 896 at 2,535 / 6,000 / 8,191 rows 10.5 / 16.4 / 17.5 against 19.5 /
+        19.0 / 23.8, 2,752 x 896 at 3,584 / 8,191 22.0 / 40.8 against 29.6 / 62.6; unrounded: 1,152 x 896 at 2,048 / 6,000 / 8,191 11.8 / 20.0 /
+        25.1 against 13.0 / 26.6 / 27.4.  Three times as wide as long there is nothing left: 3,072 x 1,024 unrounded at 2,048 / 8,191 rows 20.7 /
+        61.6 against 19.4 / 55.4."""
+        return k <= 1024 and n <= 2 * k or k <= 896 and n < 4 * k
 
     @staticmethod
     def _own_gate(m: int, k: int) -> bool:
@@ -707,7 +717,7 @@ class HipKernels(KernelBackend):
             self._run("egpt_gemm_skinny", x.data_ptr(), w.data_ptr(), None, self._ptr(out), None, self._ptr(target),
                       m, n, k, s, 4, self._stream())
             return out if target is None else target
-        if m > 64 and self._rows_fit(x, w, k) and self._own_rows(m, n, k, unrounded):
+        if m > 64 and self._rows_fit(x, w, k) and (self._own_rows(m, n, k, unrounded) or self._own_short(n, k)):
             # many rows on the framework's own kernel: rounded, or float32 partial sums where the k range is split
             self._need(x, "x")
             self._need(w, "w", x.dtype, (n, k))

@@ -142,3 +142,47 @@ def test_rows_grouped_by_expert(k, tile_rows, t, top, experts, outputs, hidden, 
             assert ((act[r].double().cpu() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-4).all()
             full = d64[e] @ act[r].double().cpu()
             assert ((y[r].double().cpu() - full).abs() <= 1e-5 * (d64[e].abs() @ act[r].double().cpu().abs()) + 1e-6).all()
+
+
+@pytest.mark.parametrize("shape", range(5))
+@pytest.mark.parametrize("kk,splits", [(128, 1), (192, 1), (256, 1), (384, 2), (448, 2)])
+def test_a_workgroup_takes_several_tiles_in_turn(k, shape, kk, splits):
+    # more tiles than the CUs hold workgroups, with edges in both directions; two steps (a workgroup per tile), three (all of a
+    # tile's loads under the tile before), four, and split ranges of three and of four and three steps
+    m, n = ((2049, 9004), (2049, 9004), (2049, 9004), (2300, 4100), (2300, 2052))[shape]
+    x, w = rnd(m, kk, seed=9), rnd(n, kk, seed=10)
+    want = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * kk * 2.0 ** -24
+    parts = run(k, x, w, shape, splits, 1)
+    assert ((parts.double().sum(0) - want).abs() <= bound).all()
+    if splits > 1:
+        return
+    rounded = run(k, x, w, shape, 1, 0)
+    assert ((rounded.double() - want).abs() <= bound + want.abs() * 2.0 ** -8).all()
+    some = (n // 2) // 8 * 8 + (0 if kk == 192 else 4)             # rounded results leave in eights of columns, or in fours
+    w = torch.cat([w[:some] * 0.2, w[:some] * 0.2])
+    both = x.double() @ w.double().t()
+    z, u = both[:, :some], both[:, some:]
+    out = run(k, x, w, shape, 1, 2).double()
+    gate = z * torch.sigmoid(z) * u
+    assert ((out - gate).abs() <= gate.abs() * 2.0 ** -8 + 1e-4 * (1 + z.abs()) * (1 + u.abs())).all()
+
+
+@pytest.mark.parametrize("act", [0, 1])
+def test_the_activation_over_its_range(k, act):
+    # gates from the smallest to the largest, up values of one: the result is the activation itself, off by a few float32
+    # roundings (4 units of 2^-23, and as much again of the exponent, whose error is one of the factor) and rounded to
+    # bfloat16.  Beyond 87 the exponential leaves float32's normal numbers.
+    z = torch.cat([torch.linspace(-12, 12, 385), torch.tensor([1e-30, -1e-30, 1e-6, -40.0, 40.0, -86.5, 86.5, -87.5, 87.5, -95.0, -300.0, 300.0, 1e30,
+                                                               -1e30])]).to(torch.bfloat16)
+    m = z.numel()
+    x = torch.zeros(m, 64, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = z, 1.0
+    w = torch.zeros(16, 64, dtype=torch.bfloat16)
+    w[:8, 0], w[8:, 1] = 1.0, 1.0
+    out = run(k, x.cuda(), w.cuda(), 4, 1, 2, act).cpu().double()
+    zd = z.double()
+    y = zd if act == 0 else 1.5957691216057308 * (zd + 0.044715 * zd ** 3)
+    want = zd * torch.sigmoid(y)
+    off = want.abs() * (2.0 ** -8 + (1 + y.abs().clamp(max=100.0)) * 2.0 ** -21) + 1e-37
+    assert ((out - want[:, None]).abs() <= off[:, None]).all()
