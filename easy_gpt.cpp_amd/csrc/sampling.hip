@@ -102,9 +102,14 @@ __global__ __launch_bounds__(kSampleThreads) void argmax_kernel(const float* __r
 // workgroup per row picks among the pieces (lowest index among equal maxima in both stages).
 constexpr int kArgmaxPieces = 32;
 
+// For sampling each wavefront leaves the maximum of its share as well (sub_val [rows][kSubPieces], -infinity where it had no
+// token).
+constexpr int kSubPieces = kArgmaxPieces * 4;
+
 __global__ __launch_bounds__(256) void argmax_pieces_kernel(const float* __restrict__ logits,
                                                             float* __restrict__ piece_val,
-                                                            int32_t* __restrict__ piece_idx, int vocab) {
+                                                            int32_t* __restrict__ piece_idx, float* __restrict__ sub_val,
+                                                            int vocab) {
     __shared__ float s_val[16];
     __shared__ int s_idx[16];
     const int r = blockIdx.x, c = blockIdx.y;
@@ -121,12 +126,15 @@ __global__ __launch_bounds__(256) void argmax_pieces_kernel(const float* __restr
         piece_val[r * kArgmaxPieces + c] = val;
         piece_idx[r * kArgmaxPieces + c] = begin + best;
     }
+    if (sub_val && threadIdx.x < 4) sub_val[r * kSubPieces + c * 4 + threadIdx.x] = n > 0 ? s_val[threadIdx.x] : -INFINITY;
 }
 
-__global__ __launch_bounds__(64) void argmax_pick_kernel(const float* __restrict__ piece_val,
-                                                         const int32_t* __restrict__ piece_idx,
-                                                         int32_t* __restrict__ out) {
-    const int r = blockIdx.x, lane = threadIdx.x;
+// The row's best token out of its pieces' (lowest index among equal maxima) and its value, by a whole wavefront.
+struct BestToken {
+    int index;
+    float value;
+};
+__device__ __forceinline__ BestToken best_of_pieces(const float* __restrict__ piece_val, const int32_t* __restrict__ piece_idx, int r, int lane) {
     float v = lane < kArgmaxPieces ? piece_val[r * kArgmaxPieces + lane] : -INFINITY;
     int i = lane < kArgmaxPieces ? piece_idx[r * kArgmaxPieces + lane] : 0x7fffffff;
 #pragma unroll
@@ -135,7 +143,13 @@ __global__ __launch_bounds__(64) void argmax_pick_kernel(const float* __restrict
         const int oi = __shfl_xor(i, o, kWave);
         argmax_combine(v, i, ov, oi);
     }
-    if (lane == 0) out[r] = i;
+    return {__builtin_amdgcn_readfirstlane(i), __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)))};
+}
+__global__ __launch_bounds__(64) void argmax_pick_kernel(const float* __restrict__ piece_val,
+                                                         const int32_t* __restrict__ piece_idx,
+                                                         int32_t* __restrict__ out) {
+    const int best = best_of_pieces(piece_val, piece_idx, blockIdx.x, threadIdx.x).index;
+    if (threadIdx.x == 0) out[blockIdx.x] = best;
 }
 
 // weight of token j: exp((x_j - max) / T), in [0, 1]
@@ -236,28 +250,24 @@ __device__ uint32_t select_by_count(const float* __restrict__ w, int vocab, unsi
     return prefix;
 }
 
-// Among the weights >= floor_bits, the largest bit pattern tau with mass(w >= tau) >= need: the smallest set of
-// most likely tokens whose mass reaches need, ties at tau included whole.  Sixteen-way search on the bit
-// pattern: each pass sums, per thread and then over the workgroup in a fixed order, the fixed-point mass at or
-// above fifteen pivots; about eight passes.
-__device__ uint32_t select_by_mass(const float* __restrict__ w, int vocab, uint32_t floor_bits, unsigned long long need,
-                                   unsigned long long* wave_sums /* [16][15] */, uint32_t* shared_lo,
+// Among the weights >= lo, the largest bit pattern tau with mass(w >= tau) >= need: the smallest set of most likely tokens whose
+// mass reaches need, ties at tau included whole.  In between, mass(w >= lo) >= need and mass(w >= hi) = above < need.  Each pass
+// divides [lo, hi): weights that crowd into a few exponents by fifteen pivots, whose masses every thread sums in registers;
+// after that by 64 bins in LDS (152,000 weights of a row that top-p alone cuts, four such passes: 540 -> 170 us a row, where
+// seven passes of pivots walked it).  Masses are fixed-point integers, whose sums depend on no order.
+__device__ uint32_t select_by_mass(const float* __restrict__ w, int vocab, uint32_t lo, uint32_t hi, unsigned long long above,
+                                   unsigned long long need, unsigned long long* sums /* [16][15] */, uint32_t* shared_lo,
                                    uint32_t* shared_hi, unsigned long long* shared_above) {
-    uint32_t lo = floor_bits, hi = 0x3f800001u;      // mass(w >= lo) >= need, mass(w >= hi) < need
-    unsigned long long above = 0ull;                 // mass(w >= hi), known from the pass that set hi
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, n_waves = blockDim.x / kWave;
-    while (hi - lo > 1u) {
-        // the first pass puts its pivots on exponent boundaries near 1.0, where the mass is; later passes
-        // divide [lo, hi) evenly
-        const bool first = hi == 0x3f800001u && lo < 0x38000000u;
-        const uint32_t step = first ? 0x01000000u : (hi - lo + 15u) / 16u;
-        const uint32_t base = first ? 0x37000000u : lo;               // pivot i = base + (i + 1) * step
+    if (lo + 1u < hi && hi == 0x3f800001u && lo < 0x38000000u) {
+        // pivots on exponent boundaries near 1.0, where the mass is
+        const uint32_t base = 0x37000000u, step = 0x01000000u;       // pivot i = base + (i + 1) * step
         unsigned long long acc[15];
 #pragma unroll
         for (int i = 0; i < 15; ++i) acc[i] = 0ull;
         for_each_in_row(w, vocab, threadIdx.x, blockDim.x, [&](int, float wj) {
             const uint32_t bits = __float_as_uint(wj);
-            if (bits > base && bits < hi && bits >= floor_bits) {     // only these can lie at or above a pivot
+            if (bits > base && bits < hi && bits >= lo) {             // only these can lie at or above a pivot
                 const unsigned long long f = fixed_of(wj);
 #pragma unroll
                 for (int i = 0; i < 15; ++i) acc[i] += bits >= base + (i + 1) * step ? f : 0ull;
@@ -268,7 +278,7 @@ __device__ uint32_t select_by_mass(const float* __restrict__ w, int vocab, uint3
             unsigned long long v = acc[i];
 #pragma unroll
             for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-            if (lane == 0) wave_sums[wave * 15 + i] = v;
+            if (lane == 0) sums[wave * 15 + i] = v;
         }
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -279,7 +289,7 @@ __device__ uint32_t select_by_mass(const float* __restrict__ w, int vocab, uint3
                 if (pivot >= hi) break;
                 if (pivot <= lo) continue;
                 unsigned long long mass = above;
-                for (int wv = 0; wv < n_waves; ++wv) mass += wave_sums[wv * 15 + i];
+                for (int wv = 0; wv < n_waves; ++wv) mass += sums[wv * 15 + i];
                 if (mass >= need) {
                     new_lo = pivot;
                 } else {
@@ -298,244 +308,437 @@ __device__ uint32_t select_by_mass(const float* __restrict__ w, int vocab, uint3
         above = *shared_above;
         __syncthreads();
     }
+    while (lo + 1u < hi) {                           // (every pass leaves at most 1 / 32 of the range, and one pattern in the end)
+        const int width = 32 - __clz(static_cast<int>(hi - lo - 1u));
+        const int shift = width > 6 ? width - 6 : 0;
+        if (threadIdx.x < kWave) sums[threadIdx.x] = 0ull;
+        __syncthreads();
+        for_each_in_row(w, vocab, threadIdx.x, blockDim.x, [&](int, float wj) {
+            const uint32_t bits = __float_as_uint(wj);
+            if (bits >= lo && bits < hi) atomicAdd(&sums[(bits - lo) >> shift], fixed_of(wj));
+        });
+        __syncthreads();
+        if (threadIdx.x < kWave) {
+            const int bin = kWave - 1 - lane;        // from the greatest weights down
+            const unsigned long long mine = sums[bin];
+            unsigned long long incl = mine;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const unsigned long long up = __shfl_up(incl, o, kWave);
+                if (lane >= o) incl += up;
+            }
+            const unsigned long long reached = __ballot(above + incl >= need);
+            const int holder = reached ? __ffsll(static_cast<long long>(reached)) - 1 : kWave - 1;
+            if (lane == holder) {
+                *shared_lo = lo + (static_cast<uint32_t>(bin) << shift);
+                *shared_hi = min(hi, lo + (static_cast<uint32_t>(bin + 1) << shift));
+                *shared_above = above + incl - mine;
+            }
+        }
+        __syncthreads();
+        lo = *shared_lo;
+        hi = *shared_hi;
+        above = *shared_above;
+        __syncthreads();
+    }
     return lo;
 }
 
 // ---- wide vocabularies: the row-wide work spread over many workgroups, the selection on what is left of the row
 //
 // The selection below walks its row a dozen times with one workgroup, which for 150,000 tokens is 300 us whatever the
-// number of rows.  For a wide vocabulary three small kernels with kSamplePieces workgroups per row come first: they
-// count the weights by exponent (those within 2^-16 of the largest, which hold the top-k tokens and the top-p mass of
-// any distribution that is not nearly flat), decide below which exponent no token can be kept, and write the tokens at
-// or above it, in index order, into a list of candidates.  The selection then runs on that list: one thread per
-// candidate when they are at most kSampleThreads (the usual case), the row-walking selection otherwise.  A row for
-// which neither cut is asked gets no list: the pieces' masses say in which piece the drawn point lies, and that
-// piece alone is walked.
+// number of rows.  For a wide vocabulary kernels with kSamplePieces workgroups per row come first and leave it a list of
+// candidates.
+//
+// Top-k of at most kSubPieces tokens: the search for the row's maximum leaves the maxima of 128 shares of the row, and the k-th
+// largest of those is no larger than the k-th largest token.  One pass lists the tokens that weigh as much (some 30 for a k of
+// 20, ties among them), in any order; the last kernel puts them in index order.
+//
+// All other rows: the weights are counted by exponent, then the tokens at or above the exponent below which none can be kept are
+// listed, in index order.  The selection runs on that list: one thread per candidate when they are at most kSampleThreads,
+// the row-walking selection otherwise.  A row for which neither cut is asked gets no list: the pieces' masses say in which
+// piece the drawn point lies, and that piece alone is walked.  Counted are the weights within 2^-16 of the largest, an exponent
+// a bin, which hold the top-p mass of any distribution that is not nearly flat.
+//
+// 64 rows of 151,936, us: top-k 20, top-p 0.95 at 0.8 52 to 455 (rows whose k-th weight lay below 2^-16 of the largest had all
+// their vocabulary for candidates) -> 33; top-k 50 at 0.6 490 to 505 -> 38; one row of the former 31 -> 23; top-p alone 590 -> 230.
 constexpr int kSamplePieces = 32;
 constexpr int kTopBins = 16;            // exponents 127 (weight 1.0) down to 112, one bin each; bin kTopBins: the rest
 
-__device__ __forceinline__ int top_bin_of(uint32_t bits) {           // bits of a weight in [0, 1]
+__device__ __forceinline__ int top_bin_of(uint32_t bits) {           // bits of a weight in [0, 1]; kTopBins: below the bins (and NaN)
     const int e = static_cast<int>(bits >> 23);
-    return e >= 128 - kTopBins ? 127 - e : kTopBins;
+    return e >= 128 - kTopBins && e <= 127 ? 127 - e : kTopBins;
+}
+// The exponential's argument; below kNoTopBin (ln 2^-15 is -10.40) the weight lies in none of the top bins.
+__device__ __forceinline__ float exponent_of(float x, float mx, float inv_t) { return (x - mx) * inv_t; }
+constexpr float kNoTopBin = -10.5f;
+// A row with top-k whose candidates follow from the shares' maxima: nothing of it underflows, and there are k maxima.
+constexpr float kLeastExponent = -80.0f;
+
+// The k-th largest of a row's kSubPieces maxima (k <= kSubPieces; 256 threads, `mine` the maximum of thread t < kSubPieces).
+__device__ float bound_of_row(float mine, int k, float* s_sub /* [kSubPieces] */, unsigned int* s_bound) {
+    const int t = threadIdx.x;
+    if (t < kSubPieces) s_sub[t] = mine;
+    if (t == 0) *s_bound = 0xffffffffu;
+    __syncthreads();
+    if (t < kSubPieces) {
+        int greater = 0;
+#pragma unroll
+        for (int i = 0; i < kSubPieces / 4; ++i) {
+            const float4 v = reinterpret_cast<const float4*>(s_sub)[i];
+            greater += (v.x > mine) + (v.y > mine) + (v.z > mine) + (v.w > mine);
+        }
+        // the least of those that fewer than k exceed; bits in the order of the numbers
+        const unsigned int bits = __float_as_uint(mine), order = bits & 0x80000000u ? ~bits : bits | 0x80000000u;
+        if (greater < k) atomicMin(s_bound, order);
+    }
+    __syncthreads();
+    const unsigned int order = *s_bound;
+    return __uint_as_float(order & 0x80000000u ? order & 0x7fffffffu : ~order);
 }
 
-// piece_count / piece_mass [rows][kSamplePieces][kTopBins + 1]: per piece of the row, how many weights each bin holds
-// and their mass in fixed point
-__global__ __launch_bounds__(256) void sample_hist_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
-                                                          const int32_t* __restrict__ best, unsigned int* __restrict__ piece_count,
+// The candidates of a piece by the bound of its row, in no order: tight ones (they weigh as much as the bound) from the front of the
+// piece's part of the row's list, loose ones (down to the exponent's beginning, if it is one of the top bins': with them the
+// list is the one that counting by exponent would leave, and the draw adds up the same numbers in the same places) from its
+// back.  `first`: the thread's tokens begin + t, begin + t + 256 ..., kCollectAhead of them, on their way since the kernel began.
+constexpr int kCollectAhead = 20;
+__device__ void collect_candidates(const float* __restrict__ row, int begin, int n, const float (&first)[kCollectAhead], float mx, float inv_t,
+                                   float bound_t, float* __restrict__ ow, int32_t* __restrict__ oi, int* s_n /* [2], zeros */) {
+    // (expf may be off by a unit either way: 2^-18 below the bound is below every token that is not)
+    const float tight = expf(bound_t) * (1.0f - 3.8147e-6f);
+    const uint32_t bits = __float_as_uint(tight);
+    const float loose = top_bin_of(bits) < kTopBins ? __uint_as_float(bits & 0x7f800000u) : tight;
+    const float far = bound_t - 0.75f;                       // e^-0.75 < 1/2
+    auto look = [&](float x, int j) {
+        const float t = exponent_of(x, mx, inv_t);
+        if (!(t >= far)) return;
+        const float w = expf(t);
+        if (w < loose) return;
+        const int to = w >= tight ? begin + atomicAdd(&s_n[0], 1) : begin + n - 1 - atomicAdd(&s_n[1], 1);
+        ow[to] = w;
+        oi[to] = begin + j;
+    };
+#pragma unroll
+    for (int i = 0; i < kCollectAhead; ++i)
+        if (static_cast<int>(threadIdx.x) + 256 * i < n) look(first[i], threadIdx.x + 256 * i);
+    for (int j0 = 256 * kCollectAhead; j0 < n; j0 += 256 * kCollectAhead) {
+        float v[kCollectAhead];
+#pragma unroll
+        for (int i = 0; i < kCollectAhead; ++i) {
+            const int j = j0 + threadIdx.x + 256 * i;
+            v[i] = j < n ? row[begin + j] : -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < kCollectAhead; ++i)
+            if (j0 + static_cast<int>(threadIdx.x) + 256 * i < n) look(v[i], j0 + threadIdx.x + 256 * i);
+    }
+}
+
+// Rows whose candidates follow from the maxima: their lists.  Others:
+// piece_count, piece_mass [rows][kSamplePieces][kTopBins + 1]: per piece of the row, how many weights each bin holds, and, where the
+// row's draw asks for it (no top-k), their mass in fixed point
+__global__ __launch_bounds__(256, 8) void sample_count_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
+                                                          const int32_t* __restrict__ top_k, const float* __restrict__ piece_val,
+                                                          const int32_t* __restrict__ piece_idx, const float* __restrict__ sub_val,
+                                                          int32_t* __restrict__ best_out, int32_t* __restrict__ listed,
+                                                          int32_t* __restrict__ list_count,
+                                                          float* __restrict__ cand_w, int32_t* __restrict__ cand_idx,
+                                                          unsigned int* __restrict__ piece_count,
                                                           unsigned long long* __restrict__ piece_mass, int vocab) {
+    __shared__ __attribute__((aligned(16))) float s_sub[kSubPieces];
+    __shared__ unsigned int s_bound;
+    __shared__ int s_n[2];
     __shared__ unsigned int s_count[kTopBins + 1];
     __shared__ unsigned long long s_mass[kTopBins + 1];
     const int r = blockIdx.x, c = blockIdx.y;
     const float temp = temperature[r];
-    if (!(temp > 0.f)) return;
+    const int k = top_k[r];
+    const bool by_count = k > 0 && k < vocab;
     const float* row = logits + static_cast<size_t>(r) * vocab;
-    const float mx = row[best[r]];
-    const float inv_t = 1.0f / fmaxf(temp, 1e-6f);
     const int piece = (vocab + kSamplePieces - 1) / kSamplePieces;
     const int begin = min(vocab, c * piece), n = min(vocab, begin + piece) - begin;
-    for (int i = threadIdx.x; i <= kTopBins; i += blockDim.x) {
-        s_count[i] = 0u;
-        s_mass[i] = 0ull;
-    }
-    __syncthreads();
-    // Nearly every weight lies below the top bins and is summed in registers; the few above go to the bins in LDS
-    // (integer additions: the order does not matter).
-    unsigned int rest_count = 0u;
-    unsigned long long rest_mass = 0ull;
-    for_each_in_row(row + begin, n, threadIdx.x, blockDim.x, [&](int, float x) {
-        const float w = weight_of(x, mx, inv_t);
-        const int bin = top_bin_of(__float_as_uint(w));
-        const unsigned long long f = fixed_of(w);
-        if (bin == kTopBins) {
-            rest_count += 1u;
-            rest_mass += f;
-        } else {
-            atomicAdd(&s_count[bin], 1u);
-            atomicAdd(&s_mass[bin], f);
+    // everything that can be asked for is asked for at once: what follows is a chain of waits otherwise
+    const bool may_list = temp > 0.f && by_count && k <= kSubPieces;
+    float first[kCollectAhead], sub = 0.f;
+    if (may_list) {
+#pragma unroll
+        for (int i = 0; i < kCollectAhead; ++i) {
+            const int j = threadIdx.x + 256 * i;
+            first[i] = j < n ? row[begin + j] : -INFINITY;
         }
-    });
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        rest_count += __shfl_xor(rest_count, o, kWave);
-        rest_mass += __shfl_xor(rest_mass, o, kWave);
+        if (threadIdx.x < kSubPieces) sub = sub_val[r * kSubPieces + threadIdx.x];
     }
-    if (threadIdx.x % kWave == 0 && rest_count) {
-        atomicAdd(&s_count[kTopBins], rest_count);
-        atomicAdd(&s_mass[kTopBins], rest_mass);
-    }
-    __syncthreads();
-    const size_t base = (static_cast<size_t>(r) * kSamplePieces + c) * (kTopBins + 1);
-    for (int i = threadIdx.x; i <= kTopBins; i += blockDim.x) {
-        piece_count[base + i] = s_count[i];
-        piece_mass[base + i] = s_mass[i];
-    }
-}
-
-// cutoff[r]: bit pattern below which no weight of row r can be kept; offsets[r][0..kSamplePieces]: where each piece's
-// candidates start in the row's list (the last entry is their number)
-__global__ __launch_bounds__(64) void sample_plan_kernel(const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-                                                         const float* __restrict__ top_p,
-                                                         const unsigned int* __restrict__ piece_count,
-                                                         const unsigned long long* __restrict__ piece_mass,
-                                                         uint32_t* __restrict__ cutoff, int32_t* __restrict__ offsets,
-                                                         unsigned long long* __restrict__ row_mass,
-                                                         const float* __restrict__ uniform, int32_t* __restrict__ direct_piece,
-                                                         unsigned long long* __restrict__ direct_target, int vocab) {
-    __shared__ unsigned int s_count[kTopBins + 1];
-    __shared__ unsigned long long s_mass[kTopBins + 1];
-    __shared__ int s_bin;
-    const int r = blockIdx.x, t = threadIdx.x;
-    if (!(temperature[r] > 0.f)) {
-        if (t == 0) direct_piece[r] = -1;
-        return;
-    }
-    const size_t base = static_cast<size_t>(r) * kSamplePieces * (kTopBins + 1);
-    {
-        // Neither cut is asked for: the draw needs no selection.  The pieces' masses are known, so the drawn point
-        // (in fixed point, of the whole row's mass) names its piece and what is left of it inside that piece; the
-        // last kernel walks that piece alone.  No list of candidates is made for such a row.
-        const int k = top_k[r];
-        const float p = top_p[r];
-        if (!(k > 0 && k < vocab) && !(p > 0.f && p < 1.f)) {
-            unsigned long long mine = 0ull;
-            if (t < kSamplePieces)
-                for (int i = 0; i <= kTopBins; ++i) mine += piece_mass[base + t * (kTopBins + 1) + i];
-            unsigned long long incl = mine;
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const unsigned long long up = __shfl_up(incl, o, kWave);
-                if (t >= o) incl += up;
-            }
-            const unsigned long long total = __shfl(incl, kSamplePieces - 1, kWave);
-            const float u = fminf(fmaxf(uniform[r], 0.f), 0.99999994f);
-            unsigned long long target = static_cast<unsigned long long>(static_cast<double>(u) * static_cast<double>(total));
-            if (total > 0ull && target >= total) target = total - 1ull;
-            const bool here = t < kSamplePieces && incl > target && incl - mine <= target;   // at most one piece
-            const unsigned long long holders = __ballot(here);
-            const int piece = holders ? __ffsll(static_cast<long long>(holders)) - 1 : 0;      // (an empty row: piece 0)
-            const unsigned long long inside = __shfl(target - (incl - mine), piece, kWave);
-            if (t < kSamplePieces) offsets[r * (kSamplePieces + 1) + t] = 0;
-            if (t == 0) {
-                direct_piece[r] = piece;
-                direct_target[r] = holders ? inside : 0ull;
-                offsets[r * (kSamplePieces + 1) + kSamplePieces] = 0;
-                cutoff[r] = 0xffffffffu;
-                row_mass[r] = total;
-            }
+    const BestToken best = best_of_pieces(piece_val, piece_idx, r, threadIdx.x % kWave);
+    if (c == 0 && threadIdx.x == 0) best_out[r] = best.index;
+    if (!(temp > 0.f)) return;
+    const float mx = best.value;
+    const float inv_t = 1.0f / fmaxf(temp, 1e-6f);
+    if (may_list) {
+        if (threadIdx.x < 2) s_n[threadIdx.x] = 0;
+        const float bound_t = exponent_of(bound_of_row(sub, k, s_sub, &s_bound), mx, inv_t);
+        if (bound_t >= kLeastExponent && fabsf(mx) < INFINITY) {
+            collect_candidates(row, begin, n, first, mx, inv_t, bound_t, cand_w + static_cast<size_t>(r) * vocab,
+                               cand_idx + static_cast<size_t>(r) * vocab, s_n);
+            if (c == 0 && threadIdx.x == 0) listed[r] = 1;
+            __syncthreads();
+            if (threadIdx.x < 2) list_count[(r * kSamplePieces + c) * 2 + threadIdx.x] = s_n[threadIdx.x];
             return;
         }
     }
-    if (t <= kTopBins) {
-        unsigned int cv = 0u;
-        unsigned long long mv = 0ull;
-        for (int c = 0; c < kSamplePieces; ++c) {
-            cv += piece_count[base + c * (kTopBins + 1) + t];
-            mv += piece_mass[base + c * (kTopBins + 1) + t];
+    if (c == 0 && threadIdx.x == 0) listed[r] = 0;
+    if (threadIdx.x <= kTopBins) {
+        s_count[threadIdx.x] = 0u;
+        s_mass[threadIdx.x] = 0ull;
+    }
+    __syncthreads();
+    // Nearly every weight lies below the top bins and is summed in registers; the few above go to the bins in LDS
+    // (integer additions: the order does not matter).  With top-k a weight that lies below them is not even computed.
+    unsigned int low = 0u;
+    unsigned long long low_mass = 0ull;
+    for_each_in_row(row + begin, n, threadIdx.x, blockDim.x, [&](int, float x) {
+        const float t = exponent_of(x, mx, inv_t);
+        if (!by_count || !(t < kNoTopBin)) {
+            const float w = expf(t);
+            const int bin = top_bin_of(__float_as_uint(w));
+            if (bin < kTopBins) {
+                atomicAdd(&s_count[bin], 1u);
+                if (!by_count) atomicAdd(&s_mass[bin], fixed_of(w));
+                return;
+            }
+            low_mass += static_cast<unsigned int>(w * 1099511627776.0f);          // fixed_of: below 2^-15, and 2^40 is exact
         }
-        s_count[t] = cv;
-        s_mass[t] = mv;
+        low += t <= 0.f ? 1u : 0u;                           // (a NaN is no candidate)
+    });
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        low += __shfl_xor(low, o, kWave);
+        low_mass += __shfl_xor(low_mass, o, kWave);
+    }
+    if (threadIdx.x % kWave == 0 && low) {
+        atomicAdd(&s_count[kTopBins], low);
+        if (!by_count) atomicAdd(&s_mass[kTopBins], low_mass);
+    }
+    __syncthreads();
+    const size_t base = (static_cast<size_t>(r) * kSamplePieces + c) * (kTopBins + 1);
+    if (threadIdx.x <= kTopBins) {
+        piece_count[base + threadIdx.x] = s_count[threadIdx.x];
+        piece_mass[base + threadIdx.x] = s_mass[threadIdx.x];
+    }
+}
+
+// What a row's counts say, found by a workgroup of 256 for itself: the last bin whose tokens can be kept (kTopBins: every token can; -1:
+// neither cut is asked for, and the draw needs no list), and where each piece's candidates start in the row's list.
+struct SamplePlan {
+    int last;
+    int start, end, total;              // of the workgroup's piece; of the row
+    unsigned long long row_mass;        // the mass of the whole row: what top-p without top-k refers to
+    int direct_piece;                   // without cuts: the piece that holds the drawn point, and what is left of it there
+    unsigned long long direct_target;   // (top-p without top-k: the mass of the bins above `last`, from which its search goes on)
+};
+struct SamplePlanSpace {
+    unsigned int count[kSamplePieces][kTopBins + 1];
+    unsigned long long mass[kSamplePieces][kTopBins + 1], bin_mass[kTopBins + 1];
+    unsigned int bin_count[kTopBins + 1];
+    int last, start[kSamplePieces + 1];
+};
+__device__ __forceinline__ SamplePlan plan_of_row(int r, int c, int k, float p, float u, const unsigned int* __restrict__ piece_count,
+                                                  const unsigned long long* __restrict__ piece_mass, int vocab, SamplePlanSpace& space) {
+    SamplePlan plan{kTopBins, 0, 0, 0, 0ull, -1, 0ull};
+    const int t = threadIdx.x;
+    const bool by_count = k > 0 && k < vocab, by_mass = p > 0.f && p < 1.f;
+    const unsigned int* counts = piece_count + static_cast<size_t>(r) * kSamplePieces * (kTopBins + 1);
+    const unsigned long long* masses = piece_mass + static_cast<size_t>(r) * kSamplePieces * (kTopBins + 1);
+    if (!by_count && !by_mass) {
+        // The pieces' masses are known, so the drawn point (in fixed point, of the whole row's mass) names its piece and what is
+        // left of it inside that piece; the last kernel walks that piece alone.  (Every wavefront finds the same.)
+        const int lane = t % kWave;
+        unsigned long long mine = 0ull;
+        if (lane < kSamplePieces) {
+#pragma unroll
+            for (int i = 0; i <= kTopBins; ++i) mine += masses[lane * (kTopBins + 1) + i];
+        }
+        unsigned long long incl = mine;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const unsigned long long up = __shfl_up(incl, o, kWave);
+            if (lane >= o) incl += up;
+        }
+        const unsigned long long total = __shfl(incl, kSamplePieces - 1, kWave);
+        u = fminf(fmaxf(u, 0.f), 0.99999994f);
+        unsigned long long target = static_cast<unsigned long long>(static_cast<double>(u) * static_cast<double>(total));
+        if (total > 0ull && target >= total) target = total - 1ull;
+        const bool here = lane < kSamplePieces && incl > target && incl - mine <= target;   // at most one piece
+        const unsigned long long holders = __ballot(here);
+        const int piece = holders ? __ffsll(static_cast<long long>(holders)) - 1 : 0;      // (an empty row: piece 0)
+        const unsigned long long inside = __shfl(target - (incl - mine), piece, kWave);
+        plan.last = -1;
+        plan.row_mass = total;
+        plan.direct_piece = piece;
+        plan.direct_target = holders ? inside : 0ull;
+        return plan;
+    }
+    for (int i = t; i < kSamplePieces * (kTopBins + 1); i += 256) (&space.count[0][0])[i] = counts[i];
+    if (!by_count)
+        for (int i = t; i < kSamplePieces * (kTopBins + 1); i += 256) (&space.mass[0][0])[i] = masses[i];
+    __syncthreads();
+    if (t <= kTopBins) {
+        unsigned int v = 0u;
+#pragma unroll
+        for (int i = 0; i < kSamplePieces; ++i) v += space.count[i][t];
+        space.bin_count[t] = v;
+    } else if (!by_count && t >= kWave && t < kWave + (kTopBins + 1)) {
+        unsigned long long v = 0ull;
+#pragma unroll
+        for (int i = 0; i < kSamplePieces; ++i) v += space.mass[i][t - kWave];
+        space.bin_mass[t - kWave] = v;
     }
     __syncthreads();
     if (t == 0) {
-        // the last bin whose tokens can be kept (kTopBins: every token can)
-        const int k = top_k[r];
-        const float p = top_p[r];
         int last = kTopBins;
-        if (k > 0 && k < vocab) {                    // the k-th largest weight lies in this bin; top-p only removes more
+        if (by_count) {                                      // the k-th largest weight lies in this bin; top-p only removes more
             unsigned int cum = 0u;
             for (int i = 0; i <= kTopBins; ++i) {
-                cum += s_count[i];
-                if (cum >= static_cast<unsigned int>(k)) {
-                    last = i;
-                    break;
-                }
+                if (cum < static_cast<unsigned int>(k)) last = i;
+                cum += space.bin_count[i];
             }
-        } else if (p > 0.f && p < 1.f) {             // the mass p of the whole row is reached within this bin
-            unsigned long long total = 0ull;
-            for (int i = 0; i <= kTopBins; ++i) total += s_mass[i];
+        } else {                                             // the mass p of the whole row is reached within this bin
+            unsigned long long total = 0ull, cum = 0ull;
+            for (int i = 0; i <= kTopBins; ++i) total += space.bin_mass[i];
             unsigned long long need = static_cast<unsigned long long>(static_cast<double>(p) * static_cast<double>(total));
             if (need == 0ull) need = 1ull;
-            unsigned long long cum = 0ull;
+            unsigned long long over = 0ull;
             for (int i = 0; i <= kTopBins; ++i) {
-                cum += s_mass[i];
-                if (cum >= need) {
+                if (cum < need) {
                     last = i;
-                    break;
+                    over = cum;
                 }
+                cum += space.bin_mass[i];
             }
+            space.bin_mass[0] = total;
+            space.bin_mass[1] = over;
         }
-        s_bin = last;
-        direct_piece[r] = -1;
-        cutoff[r] = last >= kTopBins ? 0u : static_cast<uint32_t>(127 - last) << 23;
-        unsigned long long all = 0ull;
-        for (int i = 0; i <= kTopBins; ++i) all += s_mass[i];
-        row_mass[r] = all;                           // the mass of the whole row: what top-p without top-k refers to
+        space.last = last;
     }
     __syncthreads();
-    // where each piece's candidates start: thread c counts piece c, a prefix sum over the wavefront does the rest
-    const int last = s_bin;
-    int mine = 0;
-    if (t < kSamplePieces) {
-        unsigned int v[kTopBins + 1];
+    plan.last = space.last;
+    plan.row_mass = by_count ? 0ull : space.bin_mass[0];
+    plan.direct_target = by_count ? 0ull : space.bin_mass[1];
+    if (t < kWave) {
+        int mine = 0;
+        if (t < kSamplePieces) {
 #pragma unroll
-        for (int i = 0; i <= kTopBins; ++i) v[i] = piece_count[base + t * (kTopBins + 1) + i];
+            for (int i = 0; i <= kTopBins; ++i) mine += i <= plan.last ? static_cast<int>(space.count[t][i]) : 0;
+        }
+        int incl = mine;
 #pragma unroll
-        for (int i = 0; i <= kTopBins; ++i) mine += i <= last ? static_cast<int>(v[i]) : 0;
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int up = __shfl_up(incl, o, kWave);
+            if (t >= o) incl += up;
+        }
+        if (t <= kSamplePieces) space.start[t] = incl - mine;
     }
-    int incl = mine;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int up = __shfl_up(incl, o, kWave);
-        if (t >= o) incl += up;
-    }
-    if (t < kSamplePieces) offsets[r * (kSamplePieces + 1) + t] = incl - mine;
-    if (t == kSamplePieces - 1) offsets[r * (kSamplePieces + 1) + kSamplePieces] = incl;
+    __syncthreads();
+    plan.start = space.start[c];
+    plan.end = space.start[c + 1];
+    plan.total = space.start[kSamplePieces];
+    return plan;
 }
 
-// the candidates of a piece, in index order: cand_w / cand_idx [rows][vocab]
-__global__ __launch_bounds__(256) void sample_compact_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
-                                                             const int32_t* __restrict__ best, const uint32_t* __restrict__ cutoff,
-                                                             const int32_t* __restrict__ offsets, float* __restrict__ cand_w,
-                                                             int32_t* __restrict__ cand_idx,
-                                                             const int32_t* __restrict__ direct_piece, int vocab) {
+// the candidates of a piece, in index order: cand_w / cand_idx [rows][vocab]; their number and the plan's other findings per row
+__global__ __launch_bounds__(256, 8) void sample_compact_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
+                                                             const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
+                                                             const float* __restrict__ uniform, const int32_t* __restrict__ best,
+                                                             const unsigned int* __restrict__ piece_count,
+                                                             const unsigned long long* __restrict__ piece_mass,
+                                                             const int32_t* __restrict__ listed, float* __restrict__ cand_w,
+                                                             int32_t* __restrict__ cand_idx, int32_t* __restrict__ cand_count,
+                                                             unsigned long long* __restrict__ row_mass,
+                                                             int32_t* __restrict__ direct_piece,
+                                                             unsigned long long* __restrict__ direct_target,
+                                                             int32_t* __restrict__ last_bin, int vocab) {
     __shared__ int s_wave[4];
+    __shared__ SamplePlanSpace s_plan;
     const int r = blockIdx.x, c = blockIdx.y;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const float temp = temperature[r];
-    if (!(temp > 0.f) || direct_piece[r] >= 0) return;
+    if (!(temp > 0.f) || listed[r] != 0) {
+        if (c == 0 && threadIdx.x == 0) direct_piece[r] = -1;
+        return;
+    }
     const float* row = logits + static_cast<size_t>(r) * vocab;
     const float mx = row[best[r]];
     const float inv_t = 1.0f / fmaxf(temp, 1e-6f);
-    const uint32_t cut = cutoff[r];
+    {
+        const int k = top_k[r];
+        const float p = top_p[r];
+        if (c > 0 && !(k > 0 && k < vocab) && !(p > 0.f && p < 1.f)) return;      // no list is made without cuts
+    }
+    SamplePlan plan = plan_of_row(r, c, top_k[r], top_p[r], uniform[r], piece_count, piece_mass, vocab, s_plan);
+    if (!(fabsf(mx) < INFINITY)) {                           // an infinity or nothing but NaN: the row's best token and no draw
+        plan.total = 0;
+        plan.last = plan.direct_piece = -1;
+    }
+    if (c == 0 && threadIdx.x == 0) {
+        cand_count[r] = plan.total;
+        last_bin[r] = plan.last;
+        row_mass[r] = plan.row_mass;
+        direct_piece[r] = plan.direct_piece;
+        direct_target[r] = plan.direct_target;
+    }
+    if (plan.last < 0) return;
     const int piece = (vocab + kSamplePieces - 1) / kSamplePieces;
     const int begin = min(vocab, c * piece), end = min(vocab, begin + piece);
     float* ow = cand_w + static_cast<size_t>(r) * vocab;
     int32_t* oi = cand_idx + static_cast<size_t>(r) * vocab;
-    int at = offsets[r * (kSamplePieces + 1) + c];
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    // 256 tokens at a time, token j by thread j: the order of the list is the order of the tokens
-    for (int j0 = begin; j0 < end; j0 += 256) {
-        const int j = j0 + threadIdx.x;
-        float w = 0.f;
-        bool keep = false;
-        if (j < end) {
-            w = weight_of(row[j], mx, inv_t);
-            keep = __float_as_uint(w) >= cut;
+    int at = plan.start;
+    if (plan.end == at) return;
+    // a token's weight if it is a candidate.  The top bins go by the weight's bits, its argument only tells most others apart
+    const uint32_t cut = static_cast<uint32_t>(127 - min(plan.last, kTopBins - 1)) << 23;
+    const float far = plan.last < kTopBins ? -0.6931472f * static_cast<float>(plan.last) - 0.01f : -INFINITY;
+    auto weight_of_candidate = [&](float x, float& w) {
+        const float t = exponent_of(x, mx, inv_t);
+        if (plan.last >= kTopBins) {
+            if (t <= 0.f) w = expf(t);
+            return t <= 0.f;
         }
-        const unsigned long long mask = __ballot(keep);
-        const int before = __popcll(mask & ((1ull << lane) - 1ull));
-        if (lane == 0) s_wave[wave] = __popcll(mask);
+        if (t < far) return false;
+        w = expf(t);
+        return top_bin_of(__float_as_uint(w)) < kTopBins && __float_as_uint(w) >= cut;
+    };
+    // Every wavefront takes a run of kRun groups of 64 tokens, all loads of a run on their way together; the order of the list is the
+    // order of the tokens.
+    constexpr int kRun = 20;
+    for (int j0 = begin; j0 < end; j0 += 4 * kRun * kWave) {
+        float v[kRun];
+        const int j = j0 + wave * kRun * kWave + lane;
+#pragma unroll
+        for (int i = 0; i < kRun; ++i) v[i] = j + i * kWave < end ? row[j + i * kWave] : 0.f;
+        unsigned long long masks[kRun];
+        int mine = 0;
+#pragma unroll
+        for (int i = 0; i < kRun; ++i) {
+            float w = 0.f;
+            const bool keep = j + i * kWave < end && weight_of_candidate(v[i], w);
+            v[i] = w;
+            masks[i] = __ballot(keep);
+            mine += __popcll(masks[i]);
+        }
+        if (lane == 0) s_wave[wave] = mine;
         __syncthreads();
-        int wave_base = 0, total = 0;
+        int to = at;
         for (int i = 0; i < 4; ++i) {
-            wave_base += i < wave ? s_wave[i] : 0;
-            total += s_wave[i];
+            to += i < wave ? s_wave[i] : 0;
+            at += s_wave[i];
         }
-        if (keep) {
-            ow[at + wave_base + before] = w;
-            oi[at + wave_base + before] = j;
+#pragma unroll
+        for (int i = 0; i < kRun; ++i) {
+            if (masks[i] >> lane & 1ull) {
+                const int place = to + __popcll(masks[i] & ((1ull << lane) - 1ull));
+                ow[place] = v[i];
+                oi[place] = j + i * kWave;
+            }
+            to += __popcll(masks[i]);
         }
-        at += total;
         __syncthreads();
     }
 }
@@ -546,11 +749,13 @@ __global__ __launch_bounds__(256) void sample_compact_kernel(const float* __rest
 // iff the mass of the greater weights is below it: the same sets as the thresholds of select_by_count and
 // select_by_mass (ties whole).  Counts and fixed-point masses are integers, so nothing depends on an order; the
 // draw walks the kept weights in index order.  Returns the picked position in the list or -1 (every thread).
-__device__ int pick_from_short_list(const float* __restrict__ w, int n, bool cut_by_count, unsigned int k, float p,
+__device__ int pick_from_short_list(float wj /* of thread j < n */, int n, bool cut_by_count, unsigned int k, float p,
                                     bool mass_of_row, unsigned long long row_mass, float u, float* s_list /* [kSampleThreads] */,
                                     unsigned long long* s_wave /* [16] */, float* s_piece /* [16] */, int* s_pick /* [2] */) {
+    __shared__ __attribute__((aligned(16))) unsigned long long s_fixed[kSampleThreads];
     const int j = threadIdx.x, lane = j % kWave, wave = j / kWave, n_waves = blockDim.x / kWave;
-    const float wj = j < n ? w[j] : 0.f;
+    if (j >= n) wj = 0.f;
+    s_fixed[j] = fixed_of(wj);
     s_list[j] = wj;                                   // slots past n hold 0: never greater than a weight
     if (j < 2) s_pick[j] = j == 0 ? 0x7fffffff : -1;
     __syncthreads();
@@ -560,8 +765,8 @@ __device__ int pick_from_short_list(const float* __restrict__ w, int n, bool cut
     for (int i = 0; i < n4; ++i) {                    // every thread reads the same address: a broadcast
         const float4 v = reinterpret_cast<const float4*>(s_list)[i];
         above += (v.x > wj) + (v.y > wj) + (v.z > wj) + (v.w > wj);
-        mass_above += (v.x > wj ? fixed_of(v.x) : 0ull) + (v.y > wj ? fixed_of(v.y) : 0ull) +
-                      (v.z > wj ? fixed_of(v.z) : 0ull) + (v.w > wj ? fixed_of(v.w) : 0ull);
+        const ulonglong2 a = reinterpret_cast<const ulonglong2*>(s_fixed)[2 * i], b = reinterpret_cast<const ulonglong2*>(s_fixed)[2 * i + 1];
+        mass_above += (v.x > wj ? a.x : 0ull) + (v.y > wj ? a.y : 0ull) + (v.z > wj ? b.x : 0ull) + (v.w > wj ? b.y : 0ull);
     }
     bool keep = j < n && (!cut_by_count || above < k);
     if (p > 0.f && p < 1.f) {
@@ -637,15 +842,51 @@ __device__ int pick_in_piece(const float* __restrict__ row, int begin, int n, fl
     return s_pick[0];
 }
 
+// The unordered candidates of a row whose list follows from the maxima (n of them, a weight and an index to a thread): those at
+// or above the beginning of the k-th weight's exponent, in index order, are
+// left in s_list and s_order.  Returns their number (every thread).
+__device__ int order_candidates(float wj, int ij, int n, unsigned int k, float* s_list, int* s_order, unsigned int* s_cell /* [2] */) {
+    const int j = threadIdx.x;
+    if (j < 2) s_cell[j] = j == 0 ? 0xffffffffu : 0u;
+    s_list[j] = j < n ? wj : 0.f;
+    __syncthreads();
+    unsigned int above = 0u;
+    const int n4 = (n + 3) / 4;
+    for (int i = 0; i < n4; ++i) {
+        const float4 v = reinterpret_cast<const float4*>(s_list)[i];
+        above += (v.x > wj) + (v.y > wj) + (v.z > wj) + (v.w > wj);
+    }
+    if (j < n && above < k) atomicMin(&s_cell[0], __float_as_uint(wj));        // the k-th weight is the least of these
+    __syncthreads();
+    const uint32_t kth = s_cell[0];
+    const uint32_t cut = top_bin_of(kth) < kTopBins ? kth & 0x7f800000u : 0u;
+    const bool in = j < n && __float_as_uint(wj) >= cut;
+    s_order[j] = in ? ij : 0x7fffffff;
+    if (in) atomicAdd(&s_cell[1], 1u);
+    __syncthreads();
+    int rank = 0;
+    for (int i = 0; i < n4; ++i) {
+        const int4 v = reinterpret_cast<const int4*>(s_order)[i];
+        rank += (v.x < ij) + (v.y < ij) + (v.z < ij) + (v.w < ij);
+    }
+    __syncthreads();
+    if (in) {
+        s_list[rank] = wj;
+        s_order[rank] = ij;
+    }
+    __syncthreads();
+    return static_cast<int>(s_cell[1]);
+}
+
 // One workgroup per row.  `weights` is scratch [rows][vocab] float32: the weights are computed once and the
 // selection passes read them back (from cache).  With a list of candidates (cand_idx != null) `weights` holds the
-// candidates' weights, cand_count[r * cand_stride] their number, and `best` the row's argmax.
+// candidates' weights, cand_count[r] their number, and `best` the row's argmax.
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     const float* __restrict__ logits, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
     const float* __restrict__ top_p, const float* __restrict__ uniform, int32_t* __restrict__ out,
     float* __restrict__ weights, int vocab, const int32_t* __restrict__ cand_idx, const int32_t* __restrict__ cand_count,
-    int cand_stride, const int32_t* __restrict__ best_in, const unsigned long long* __restrict__ row_mass,
-    const int32_t* __restrict__ direct_piece, const unsigned long long* __restrict__ direct_target) {
+    const int32_t* __restrict__ listed, const int32_t* __restrict__ list_count, const int32_t* __restrict__ best_in, const unsigned long long* __restrict__ row_mass,
+    const int32_t* __restrict__ direct_piece, const unsigned long long* __restrict__ direct_target, const int32_t* __restrict__ last_bin) {
     __shared__ float s_val[16];
     __shared__ int s_idx[16];
     __shared__ unsigned int hist[256];
@@ -658,47 +899,111 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     __shared__ float s_before;
     __shared__ __attribute__((aligned(16))) float s_list[kSampleThreads];
     __shared__ int s_pick[2];
+    __shared__ __attribute__((aligned(16))) int s_order[kSampleThreads];
     const int r = blockIdx.x;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, n_waves = blockDim.x / kWave;
     const float* row = logits + static_cast<size_t>(r) * vocab;
     float* w = weights + static_cast<size_t>(r) * vocab;
     const int32_t* idx_of = cand_idx ? cand_idx + static_cast<size_t>(r) * vocab : nullptr;
-    const float temp = temperature[r];
-    const int best = cand_idx ? best_in[r] : block_argmax(row, vocab, s_val, s_idx);
+    // (a row's few numbers at once: behind the branches that ask for them each would be a wait of its own)
+    const float temp = temperature[r], p = top_p[r], u = uniform[r];
+    const int k = top_k[r];
+    int known_best = 0, is_listed = 0, direct = -1, count = 0, more = 0;
+    if (cand_idx) {
+        known_best = best_in[r];
+        is_listed = listed[r];
+        direct = direct_piece[r];
+        if (lane < kSamplePieces) {
+            count = list_count[(r * kSamplePieces + lane) * 2];
+            more = list_count[(r * kSamplePieces + lane) * 2 + 1];
+        }
+    }
+    const int best = cand_idx ? known_best : block_argmax(row, vocab, s_val, s_idx);
     if (!(temp > 0.f)) {  // greedy, as the reference for temperature <= 0 (sampler.cpp:46-49)
         if (threadIdx.x == 0) out[r] = best;
         return;
     }
     const int full_vocab = vocab;
-    if (cand_idx && direct_piece[r] >= 0) {          // no cuts: the drawn point's piece is known, walk it
+    if (direct >= 0) {                               // no cuts: the drawn point's piece is known, walk it
         const int piece = (vocab + kSamplePieces - 1) / kSamplePieces;
-        const int begin = min(vocab, direct_piece[r] * piece), n = min(vocab, begin + piece) - begin;
+        const int begin = min(vocab, direct * piece), n = min(vocab, begin + piece) - begin;
         const int at = pick_in_piece(row, begin, n, row[best], 1.0f / fmaxf(temp, 1e-6f), direct_target[r], s_wave, s_pick);
         if (threadIdx.x == 0) out[r] = at < 0 ? best : at;
         return;
     }
-    if (cand_idx) {
-        vocab = cand_count[r * cand_stride];         // from here on the row is the list of candidates
+    const float mx = row[best];
+    const float inv_t = 1.0f / fmaxf(temp, 1e-6f);
+    const bool unordered = is_listed != 0;
+    const int row_piece = (full_vocab + kSamplePieces - 1) / kSamplePieces;
+    if (unordered) {
+        // the pieces' lists: every wavefront adds up what lies before its two pieces, and brings those together
+        static_assert(kSamplePieces == 2 * kSampleThreads / kWave, "two pieces to a wavefront");
+        int before = count, before_more = more;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int a = __shfl_up(before, o, kWave), b = __shfl_up(before_more, o, kWave);
+            if (lane >= o) {
+                before += a;
+                before_more += b;
+            }
+        }
+        const int tight = __shfl(before, kWave - 1, kWave), loose = __shfl(before_more, kWave - 1, kWave);
+        const bool with_loose = tight + loose <= kSampleThreads;
+        if (tight <= kSampleThreads) {
+            const int n = with_loose ? tight + loose : tight;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int c = 2 * wave + h, mine = __shfl(count, c, kWave), also = with_loose ? __shfl(more, c, kWave) : 0;
+                const int to = __shfl(before, c, kWave) - mine, to_more = tight + __shfl(before_more, c, kWave) - __shfl(more, c, kWave);
+                const int begin = min(full_vocab, c * row_piece), end = min(full_vocab, begin + row_piece);
+                for (int i = lane; i < mine + also; i += kWave) {
+                    const int from = i < mine ? begin + i : end - 1 - (i - mine), at = i < mine ? to + i : to_more + i - mine;
+                    s_list[at] = w[from];
+                    s_order[at] = idx_of[from];
+                }
+            }
+            __syncthreads();
+            const int j = threadIdx.x;
+            const float wj = j < n ? s_list[j] : 0.f;
+            const int ij = j < n ? s_order[j] : 0x7fffffff;
+            __syncthreads();
+            vocab = order_candidates(wj, ij, n, static_cast<unsigned int>(k), s_list, s_order, hist);
+        } else {
+            // more than a thousand equals: the thresholds from the list, brought together in the first piece's place and behind it
+            // (every piece's part moves towards the front, one piece after the other), the draw from the row
+            int to = 0;
+            for (int c = 0; c < kSamplePieces; ++c) {
+                const int mine = __shfl(count, c, kWave), begin = min(full_vocab, c * row_piece);
+                for (int i0 = 0; i0 < mine; i0 += kSampleThreads) {
+                    const int i = i0 + threadIdx.x;
+                    const float v = i < mine ? w[begin + i] : 0.f;
+                    __syncthreads();
+                    if (i < mine) w[to + i] = v;
+                    __syncthreads();
+                }
+                to += mine;
+            }
+            vocab = tight;
+        }
+    } else if (cand_idx) {
+        vocab = cand_count[r];                       // from here on the row is the list of candidates
     } else {
-        const float mx = row[best];
-        const float inv_t = 1.0f / fmaxf(temp, 1e-6f);
         for_each_in_row(row, vocab, threadIdx.x, blockDim.x, [&](int j, float x) { w[j] = weight_of(x, mx, inv_t); });
         __syncthreads();   // each thread reads back what others wrote: same workgroup, so a barrier suffices
     }
-    const int k = top_k[r];
     const bool k_active = k > 0 && k < full_vocab;
+    const unsigned long long mass = cand_idx && !k_active ? row_mass[r] : 0ull;
     if (vocab <= kSampleThreads) {                   // a short row or list: one thread per token
-        const int at = pick_from_short_list(w, vocab, k_active && k < vocab, static_cast<unsigned int>(k), top_p[r],
-                                            cand_idx && !k_active, cand_idx ? row_mass[r] : 0ull, uniform[r], s_list,
-                                            s_wave, s_piece, s_pick);
-        if (threadIdx.x == 0) out[r] = at < 0 ? best : (idx_of ? idx_of[at] : at);
+        const float wj = unordered ? s_list[threadIdx.x] : static_cast<int>(threadIdx.x) < vocab ? w[threadIdx.x] : 0.f;
+        const int at = pick_from_short_list(wj, vocab, k_active && k < vocab, static_cast<unsigned int>(k), p,
+                                            cand_idx && !k_active, mass, u, s_list, s_wave, s_piece, s_pick);
+        if (threadIdx.x == 0) out[r] = at < 0 ? best : unordered ? s_order[at] : idx_of ? idx_of[at] : at;
         return;
     }
     // kept set = { j : w_j >= threshold }; the threshold starts at 0 (everything)
     uint32_t threshold = 0u;
     if (k_active && k < vocab)        // (a list of exactly k candidates is the top k)
         threshold = select_by_count(w, vocab, static_cast<unsigned int>(k), hist, &s_a, &s_need);
-    const float p = top_p[r];
     if (p > 0.f && p < 1.f) {
         // mass of what top-k kept, in fixed point: per-thread sums, then over the wavefronts in order
         unsigned long long mine = 0ull;
@@ -713,17 +1018,28 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
         for (int i = 0; i < n_waves; ++i) kept += s_wave[i];
         __syncthreads();
         // (a list of candidates without top-k holds only the upper part of the row: the mass p refers to the whole row)
-        if (cand_idx && !k_active) kept = row_mass[r];
+        if (cand_idx && !k_active) kept = mass;
         unsigned long long need = static_cast<unsigned long long>(static_cast<double>(p) * static_cast<double>(kept));
         if (need == 0ull) need = 1ull;
-        threshold = select_by_mass(w, vocab, threshold, need, s_wave, &s_a, &s_b, &s_above);
+        uint32_t top = 0x3f800001u;
+        unsigned long long above = 0ull;
+        if (cand_idx && !k_active) {                 // the bin that holds it is known
+            const int bin = last_bin[r];
+            threshold = bin < kTopBins ? static_cast<uint32_t>(127 - bin) << 23 : 0u;
+            top = bin == 0 ? 0x3f800001u : static_cast<uint32_t>(128 - min(bin, kTopBins)) << 23;
+            above = direct_target[r];
+        }
+        threshold = select_by_mass(w, vocab, threshold, top, above, need, s_wave, &s_a, &s_b, &s_above);
     }
     // inverse CDF in index order.  Every wavefront owns a contiguous piece of the row; the piece that holds the
     // drawn point is then walked 64 tokens at a time with a prefix sum over the lanes.
+    if (unordered) vocab = full_vocab;
+    auto weight_or_none = [&](float x) { return x <= mx ? weight_of(x, mx, inv_t) : 0.f; };      // (a NaN is no candidate)
     const int piece = ((vocab + n_waves - 1) / n_waves + kWave - 1) / kWave * kWave;
     const int p_begin = min(vocab, wave * piece), p_end = min(vocab, p_begin + piece);
     float mine = 0.f;
-    for_each_in_row(w + p_begin, p_end - p_begin, lane, kWave, [&](int, float wj) {
+    for_each_in_row((unordered ? row : w) + p_begin, p_end - p_begin, lane, kWave, [&](int, float wj) {
+        if (unordered) wj = weight_or_none(wj);
         mine += __float_as_uint(wj) >= threshold ? wj : 0.f;
     });
     mine = wave_sum(mine);
@@ -732,8 +1048,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     if (threadIdx.x == 0) {
         float total = 0.f;
         for (int i = 0; i < n_waves; ++i) total += s_piece[i];
-        const float u = fminf(fmaxf(uniform[r], 0.f), 0.99999994f);
-        const float target = u * total;
+        const float target = fminf(fmaxf(u, 0.f), 0.99999994f) * total;
         float cum = 0.f;
         int owner = -1;
         float before = 0.f;
@@ -758,7 +1073,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
             const int j = base + lane;
             float wj = 0.f;
             if (j < p_end) {
-                const float v = w[j];
+                const float v = unordered ? weight_or_none(row[j]) : w[j];
                 wj = __float_as_uint(v) >= threshold ? v : 0.f;
             }
             float incl = wj;                     // inclusive prefix sum over the lanes
@@ -775,7 +1090,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
         }
         if (lane == 0) {
             const int at = pick >= 0 ? pick : last_kept;
-            out[r] = at < 0 ? best : (idx_of ? idx_of[at] : at);
+            out[r] = at < 0 ? best : (idx_of && !unordered ? idx_of[at] : at);
         }
     }
 }
@@ -792,7 +1107,7 @@ extern "C" int egpt_argmax(const float* logits, int32_t* out, void* scratch, int
     if (scratch && vocab >= 8192) {
         float* pv = static_cast<float*>(scratch);
         int32_t* pi = reinterpret_cast<int32_t*>(pv + static_cast<size_t>(n_rows) * kArgmaxPieces);
-        argmax_pieces_kernel<<<dim3(n_rows, kArgmaxPieces), 256, 0, s>>>(logits, pv, pi, vocab);
+        argmax_pieces_kernel<<<dim3(n_rows, kArgmaxPieces), 256, 0, s>>>(logits, pv, pi, nullptr, vocab);
         EGPT_CHECK_LAUNCH();
         argmax_pick_kernel<<<n_rows, kWave, 0, s>>>(pv, pi, out);
     } else {
@@ -846,13 +1161,13 @@ extern "C" int egpt_sample(const float* logits, const float* temperature, const 
         return EGPT_BAD_ARGUMENT;
     if (n_rows == 0) return EGPT_OK;
     sample_kernel<<<n_rows, kSampleThreads, 0, static_cast<hipStream_t>(stream)>>>(
-        logits, temperature, top_k, top_p, uniform, out, weights, vocab, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr);
+        logits, temperature, top_k, top_p, uniform, out, weights, vocab, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
 
-// The same for wide vocabularies, in stages (argmax, counts by exponent, the plan, the list of candidates, the
-// selection on the list).  workspace: egpt_sample_workspace(n_rows, vocab) bytes of device memory.
+// The same for wide vocabularies, in stages (maxima of pieces, counts by exponent, the list of candidates, the selection
+// on the list).  workspace: egpt_sample_workspace(n_rows, vocab) bytes of device memory.
 static size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 extern "C" size_t egpt_sample_workspace(int n_rows, int vocab) {
@@ -860,8 +1175,9 @@ extern "C" size_t egpt_sample_workspace(int n_rows, int vocab) {
     return align256(r * v * 4) * 2                                         // candidates: weights, indices
            + align256(r * kSamplePieces * (kTopBins + 1) * 8)            // masses
            + align256(r * kSamplePieces * (kTopBins + 1) * 4)            // counts
-           + align256(r * (kSamplePieces + 1) * 4) + align256(r * 4) * 2   // offsets, cutoff, best
+           + align256(r * 4) * 2                                           // number of candidates, best
            + align256(r * 8) * 2 + align256(r * 4)                         // mass of the row; the direct draw's point, piece
+           + align256(r * 4) * 2 + align256(r * kSamplePieces * 8) + align256(r * kSubPieces * 4)  // lists by the maxima, the shares' maxima
            + align256(r * kArgmaxPieces * 8);                              // argmax pieces
 }
 
@@ -878,29 +1194,28 @@ extern "C" int egpt_sample_wide(const float* logits, const float* temperature, c
     int32_t* cand_idx = reinterpret_cast<int32_t*>(p);                         p += align256(r * v * 4);
     unsigned long long* piece_mass = reinterpret_cast<unsigned long long*>(p); p += align256(r * kSamplePieces * (kTopBins + 1) * 8);
     unsigned int* piece_count = reinterpret_cast<unsigned int*>(p);            p += align256(r * kSamplePieces * (kTopBins + 1) * 4);
-    int32_t* offsets = reinterpret_cast<int32_t*>(p);                          p += align256(r * (kSamplePieces + 1) * 4);
-    uint32_t* cutoff = reinterpret_cast<uint32_t*>(p);                         p += align256(r * 4);
+    int32_t* cand_count = reinterpret_cast<int32_t*>(p);                       p += align256(r * 4);
     int32_t* best = reinterpret_cast<int32_t*>(p);                             p += align256(r * 4);
     unsigned long long* row_mass = reinterpret_cast<unsigned long long*>(p);   p += align256(r * 8);
     unsigned long long* direct_target = reinterpret_cast<unsigned long long*>(p); p += align256(r * 8);
     int32_t* direct_piece = reinterpret_cast<int32_t*>(p);                     p += align256(r * 4);
+    int32_t* last_bin = reinterpret_cast<int32_t*>(p);                         p += align256(r * 4);
+    int32_t* listed = reinterpret_cast<int32_t*>(p);                           p += align256(r * 4);
+    int32_t* list_count = reinterpret_cast<int32_t*>(p);                       p += align256(r * kSamplePieces * 8);
+    float* sub = reinterpret_cast<float*>(p);                                  p += align256(r * kSubPieces * 4);
     float* pv = reinterpret_cast<float*>(p);
     int32_t* pi = reinterpret_cast<int32_t*>(pv + r * kArgmaxPieces);
-    argmax_pieces_kernel<<<dim3(n_rows, kArgmaxPieces), 256, 0, s>>>(logits, pv, pi, vocab);
+    argmax_pieces_kernel<<<dim3(n_rows, kArgmaxPieces), 256, 0, s>>>(logits, pv, pi, sub, vocab);
     EGPT_CHECK_LAUNCH();
-    argmax_pick_kernel<<<n_rows, kWave, 0, s>>>(pv, pi, best);
+    sample_count_kernel<<<dim3(n_rows, kSamplePieces), 256, 0, s>>>(logits, temperature, top_k, pv, pi, sub, best, listed, list_count, cand_w, cand_idx,
+                                                                    piece_count, piece_mass, vocab);
     EGPT_CHECK_LAUNCH();
-    sample_hist_kernel<<<dim3(n_rows, kSamplePieces), 256, 0, s>>>(logits, temperature, best, piece_count, piece_mass, vocab);
-    EGPT_CHECK_LAUNCH();
-    sample_plan_kernel<<<n_rows, 64, 0, s>>>(temperature, top_k, top_p, piece_count, piece_mass, cutoff, offsets, row_mass,
-                                             uniform, direct_piece, direct_target, vocab);
-    EGPT_CHECK_LAUNCH();
-    sample_compact_kernel<<<dim3(n_rows, kSamplePieces), 256, 0, s>>>(logits, temperature, best, cutoff, offsets, cand_w,
-                                                                      cand_idx, direct_piece, vocab);
+    sample_compact_kernel<<<dim3(n_rows, kSamplePieces), 256, 0, s>>>(logits, temperature, top_k, top_p, uniform, best, piece_count,
+                                                                      piece_mass, listed, cand_w, cand_idx, cand_count, row_mass,
+                                                                      direct_piece, direct_target, last_bin, vocab);
     EGPT_CHECK_LAUNCH();
     sample_kernel<<<n_rows, kSampleThreads, 0, s>>>(logits, temperature, top_k, top_p, uniform, out, cand_w, vocab, cand_idx,
-                                                    offsets + kSamplePieces, kSamplePieces + 1, best, row_mass,
-                                                    direct_piece, direct_target);
+                                                    cand_count, listed, list_count, best, row_mass, direct_piece, direct_target, last_bin);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
