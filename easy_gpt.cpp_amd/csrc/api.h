@@ -89,6 +89,24 @@ int egpt_paged_attention_tiled(const void* qkv, void* out, const void* k_cache, 
                                int hd, int page_size, float scale, int window, int shape, int key_splits,
                                float* part_o, float* part_ml, int single_splits, int single_waves, int single_lean,
                                void* stream);
+// Decoded tokens with their keys dealt out by the contexts' lengths: the table [slots * 8 + n_seqs * 2] int32 is made once per step
+// (q_len null: every request brings one token; else those that do not are left out), slots <= 256, n_seqs <= slots.
+// egpt_paged_attention_mixed is egpt_paged_attention_tiled with the requests of one token taken that way;
+// egpt_attention_decode_ranged is egpt_attention_decode_fused so.  Parts: [slots][nq][hd] and [slots][nq][2] float32.
+int egpt_decode_ranges(const int32_t* kv_len, const int32_t* q_start, const int32_t* q_len, int n_seqs, int slots, int window,
+                       int32_t* table, void* stream);
+int egpt_paged_attention_mixed(const void* qkv, void* out, const void* k_cache, const void* v_cache,
+                               const int32_t* block_table, int table_width, const int32_t* q_start,
+                               const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv,
+                               int hd, int page_size, float scale, int window, int shape, int key_splits,
+                               float* part_o, float* part_ml, const int32_t* ranges, int slots, float* range_o,
+                               float* range_ml, void* stream);
+int egpt_attention_decode_ranged(const float* qkv_prod, int in_splits, const float* row_ss, int ss_splits, int hidden,
+                                 float eps, const void* bias, const float* cos_sin, const int32_t* slots, void* out,
+                                 float* part_o, float* part_ml, void* k_cache, void* v_cache, const int32_t* block_table,
+                                 int table_width, const int32_t* q_start, const int32_t* kv_len, int n_seqs, int nq, int nkv,
+                                 int hd, int page_size, float scale, int window, const int32_t* ranges, int range_slots,
+                                 void* stream);
 // One decoded token per request: workgroups of n_waves wavefronts per (request, kv head, key split); lean != 0: the
 // variant with half the loads in flight per round and fewer registers.
 int egpt_paged_attention_decode(const void* qkv, void* out, float* part_o, float* part_ml, const void* k_cache,

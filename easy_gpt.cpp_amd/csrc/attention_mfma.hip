@@ -1003,6 +1003,76 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     }
 }
 
+// Deals the keys of a step's decoded tokens out over `slots` workgroups (per kv head): a request's blocks of 32 keys go to as few
+// of them as leave none with more than `per` blocks, `per` being the least for which they all suffice (kLeastPer at least).  One
+// launch a step, for all layers.  With the same number of key ranges for every request the longest one sets a layer's
+// time: 12 heads of 128 on 2, 40 requests of 128 to 2,048 tokens, a layer 23.5 us -> 18.2; 14 heads of 64 on 2, one request of 8,000
+// tokens beside 31 of 500 21.8 -> 15.0.  This kernel takes 4 to 5 us, once a step.
+// table [slots][kRangeInts]: request (-1: none), first block, end, tokens in the cache, the token's row, number of parts;
+// then [n_seqs][2]: a request's first slot, its number of parts.  n_seqs <= slots <= 256; q_len null: all of one token.
+constexpr int kRangeInts = 8, kRangeSlots = 256, kLeastPer = 8, kMostParts = 64;
+__global__ __launch_bounds__(kRangeSlots) void decode_ranges_kernel(const int32_t* __restrict__ kv_len, const int32_t* __restrict__ q_start,
+                                                                    const int32_t* __restrict__ q_len, int n_seqs, int slots, int window,
+                                                                    int32_t* __restrict__ table) {
+    __shared__ int s_part[4];
+    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+    auto block_total = [&](int v) {
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+        __syncthreads();
+        if (lane == 0) s_part[wave] = v;
+        __syncthreads();
+        return s_part[0] + s_part[1] + s_part[2] + s_part[3];
+    };
+    const bool here = t < n_seqs && (q_len == nullptr || q_len[t] == 1);
+    const int kv = here ? kv_len[t] : 0, p = kv - 1;
+    const int begin = (window > 0 ? max(0, p - window + 1) : 0) / 32, end = here ? p / 32 + 1 : begin;
+    const int blocks = max(end - begin, here ? 1 : 0);
+    int most = blocks;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, kWave));
+    if (lane == 0) s_part[wave] = most;
+    __syncthreads();
+    most = max(max(s_part[0], s_part[1]), max(s_part[2], s_part[3]));
+    __syncthreads();
+    int low = max(kLeastPer, (most + kMostParts - 1) / kMostParts), high = max(low, most);
+    while (low < high) {
+        const int per = (low + high) / 2;
+        if (block_total((blocks + per - 1) / per) <= slots) high = per;
+        else low = per + 1;
+    }
+    const int parts = (blocks + low - 1) / low;
+    int incl = parts;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int up = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += up;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) s_part[wave] = incl;
+    __syncthreads();
+    int first = incl - parts, total = 0;
+    for (int w = 0; w < 4; ++w) {
+        first += w < wave ? s_part[w] : 0;
+        total += s_part[w];
+    }
+    if (t < n_seqs) {
+        table[slots * kRangeInts + 2 * t] = first;
+        table[slots * kRangeInts + 2 * t + 1] = parts;
+    }
+    const int per = parts > 0 ? (blocks + parts - 1) / parts : 0;
+    for (int i = 0; i < parts; ++i) {
+        int32_t* e = table + (first + i) * kRangeInts;
+        e[0] = t;
+        e[1] = min(end, begin + i * per);
+        e[2] = min(end, begin + (i + 1) * per);
+        e[3] = kv;
+        e[4] = q_start[t];
+        e[5] = parts;
+    }
+    if (t >= total && t < slots) table[t * kRangeInts] = -1;
+}
+
 // What the fused variant of the decode kernel computes its queries (and the new token's key and value) from:
 // the QKV product as it comes out of the skinny product kernel, before bias, rotation and rounding.
 struct FusedQkv {
@@ -1030,42 +1100,50 @@ struct FusedQkv {
 // qkv_rope_store_kernel, so the same bits) and keeps the queries in LDS.  The workgroup whose key range ends
 // with the new token does the same for that token's key and value, writes them to the cache and, because
 // its own loads of that cache line may have been issued before, puts them into its operands itself.
-template <int HD, int PF, bool FUSED, bool MIXED = false>
+//
+// RANGED: the keys are dealt out by `decode_ranges_kernel`, every request getting as many workgroups as its context is long;
+// grid (slots, kv heads), and a part is kept by its slot.
+template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false>
 __global__ __launch_bounds__(512) void attention_decode_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ q_start,
     const int32_t* __restrict__ kv_len, int n_tokens, int nq, int nkv, int page_size, float scale, int window,
-    int n_splits, FusedQkv f, const int32_t* __restrict__ q_len) {
+    int n_splits, FusedQkv f, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ranges) {
     constexpr int KD = HD / 32, DT = HD / 16;
     constexpr int kRow = HD + 2;
     // MIXED: a step that also holds portions of prompts; this kernel takes its requests of one token, parts are kept
     // by request (n_tokens is the number of requests then) and the rest is another kernel's.  (A parameter of the
     // template, so that the kernel of the decode step is compiled as if this were not here.)
-    if constexpr (MIXED) {
+    if constexpr (MIXED && !RANGED) {
         if (q_len[blockIdx.x] != 1) return;
+    }
+    const int32_t* range = ranges + (RANGED ? blockIdx.x * kRangeInts : 0);
+    if constexpr (RANGED) {
+        if (range[0] < 0) return;
     }
     extern __shared__ float wave_state[];          // [n_waves][16][HD + 2]: O, then maximum, then sum
     const int lane = threadIdx.x % kWave, n_waves = blockDim.x / kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // known to be the same for the wavefront
     const int lj = lane % 16, lg = lane / 16;
-    const int b = blockIdx.x, kh = blockIdx.y, split = blockIdx.z;
+    const int b = RANGED ? range[0] : blockIdx.x, kh = blockIdx.y, split = blockIdx.z;
     const int group_size = nq / nkv;
-    const int kv = kv_len[b], tok = q_start[b];
+    const int kv = RANGED ? range[3] : kv_len[b], tok = RANGED ? range[4] : q_start[b];
     const int p = kv - 1;
     const int lo = window > 0 ? max(0, p - window + 1) : 0;
     const bool valid = lj < group_size;
     const int head = kh * group_size + (valid ? lj : 0);
+    if constexpr (RANGED) n_splits = range[5];
     const int width = (nq + 2 * nkv) * HD;
     const int32_t* table = block_table + static_cast<size_t>(b) * table_width;
 
     const int kb_begin = lo / 32, kb_end = p / 32 + 1;
     const int per_split = (kb_end - kb_begin + n_splits - 1) / n_splits;
-    const int s_begin = kb_begin + split * per_split, s_end = min(kb_end, s_begin + per_split);
+    const int s_begin = RANGED ? range[1] : kb_begin + split * per_split, s_end = RANGED ? range[2] : min(kb_end, s_begin + per_split);
     const int per_wave = (max(s_end - s_begin, 0) + n_waves - 1) / n_waves;
     const int w_begin = s_begin + wave * per_wave, w_end = min(s_end, w_begin + per_wave);
     // FUSED: does this workgroup's key range end with the new token?
-    const bool writer = FUSED && split == (kb_end - 1 - kb_begin) / per_split;
+    const bool writer = FUSED && (RANGED ? s_end == kb_end : split == (kb_end - 1 - kb_begin) / per_split);
     bf16_t* q_lds = reinterpret_cast<bf16_t*>(wave_state + n_waves * 16 * kRow);   // FUSED: [16][HD], then k, v [HD]
     bf16_t* k_lds = q_lds + 16 * HD;
     bf16_t* v_lds = k_lds + HD;
@@ -1348,8 +1426,9 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
         if (n_splits == 1) {
             out[(row0 + r) * HD + d] = from_float<bf16_t>(num / den);
         } else {
-            const size_t prow = static_cast<size_t>(split) * n_tokens * nq +
-                                (MIXED ? static_cast<size_t>(b) * nq + kh * group_size : row0) + r;
+            const size_t prow = RANGED ? static_cast<size_t>(blockIdx.x) * nq + kh * group_size + r
+                                       : static_cast<size_t>(split) * n_tokens * nq +
+                                             (MIXED ? static_cast<size_t>(b) * nq + kh * group_size : row0) + r;
             part_o[prow * HD + d] = num;
             if (d == 0) {
                 part_ml[prow * 2] = mx;
@@ -1366,22 +1445,32 @@ __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __res
                                                               const float* __restrict__ part_ml,
                                                               bf16_t* __restrict__ out, int n_rows, int hd, int n_splits,
                                                               const int32_t* __restrict__ q_start = nullptr,
-                                                              const int32_t* __restrict__ q_len = nullptr, int nq = 1) {
+                                                              const int32_t* __restrict__ q_len = nullptr, int nq = 1,
+                                                              const int32_t* __restrict__ dealt = nullptr) {
     const int row = blockIdx.x, lane = threadIdx.x;
     // q_start given: the parts are kept by request, of which only those of one token have any, and the result goes
     // to that token's row
     int out_row = row;
     if (q_start != nullptr) {
         const int seq = row / nq;
-        if (q_len[seq] != 1) return;
+        if (dealt == nullptr && q_len[seq] != 1) return;
         out_row = q_start[seq] * nq + row % nq;
+    }
+    // dealt given: the parts lie by slot, and a request with a single one has its result already
+    int first_part = row, between = n_rows;
+    if (dealt != nullptr) {
+        const int seq = row / nq;
+        n_splits = dealt[2 * seq + 1];
+        if (n_splits <= 1) return;
+        first_part = dealt[2 * seq] * nq + row % nq;
+        between = nq;
     }
     // the first eight splits' parts are asked for together with their weights' inputs, not behind them (a part of a
     // split without visible keys may hold anything: it is read and then dropped)
     float first[8][4];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const size_t pr = static_cast<size_t>(min(i, n_splits - 1)) * n_rows + row;
+        const size_t pr = static_cast<size_t>(min(i, n_splits - 1)) * between + first_part;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int d = lane + r * kWave;
@@ -1390,7 +1479,7 @@ __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __res
     }
     float m = -INFINITY, l = 0.f;
     if (lane < n_splits) {
-        const size_t pr = static_cast<size_t>(lane) * n_rows + row;
+        const size_t pr = static_cast<size_t>(lane) * between + first_part;
         m = part_ml[pr * 2];
         l = part_ml[pr * 2 + 1];
     }
@@ -1405,7 +1494,7 @@ __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __res
             const int s = s0 + i;
             w8[i] = __shfl(wgt, s < n_splits ? s : 0, kWave);
             if (s >= n_splits) w8[i] = 0.f;
-            const size_t pr = static_cast<size_t>(s < n_splits ? s : 0) * n_rows + row;
+            const size_t pr = static_cast<size_t>(s < n_splits ? s : 0) * between + first_part;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int d = lane + r * kWave;
@@ -1455,17 +1544,20 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
                          const void* v_cache, const int32_t* block_table, int table_width, const int32_t* q_start,
                          const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv, int page_size, float scale,
                          int window, int n_splits, int n_waves, int combine, const FusedQkv* fused,
-                         const int32_t* q_len, hipStream_t s) {
+                         const int32_t* q_len, const int32_t* ranges, int slots, hipStream_t s) {
     dim3 grid(n_seqs, nkv, n_splits);
+    if (ranges) grid = dim3(slots, nkv);
     size_t lds = static_cast<size_t>(n_waves) * 16 * (HD + 2) * sizeof(float);
     if (fused) lds += 18 * HD * sizeof(bf16_t);          // 16 query heads, the new key and value
     if (lds > kDecodeLdsMost) return EGPT_UNSUPPORTED_SIZE;
     if (lds > 64 * 1024) {
         // (eight wavefronts at head size 128: more than a kernel may take without being asked; once per instance)
-        static bool raised_fused = false, raised_plain = false, raised_mixed = false;
-        bool& raised = fused ? raised_fused : q_len ? raised_mixed : raised_plain;
+        static bool raised_fused = false, raised_plain = false, raised_mixed = false, raised_ranged_fused = false, raised_ranged = false;
+        bool& raised = ranges ? (fused ? raised_ranged_fused : raised_ranged) : fused ? raised_fused : q_len ? raised_mixed : raised_plain;
         if (!raised) {
-            const void* fn = fused   ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, true>)
+            const void* fn = ranges && fused ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, 2, true, false, true>)
+                             : ranges        ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, 2, false, true, true>)
+                             : fused   ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, true>)
                              : q_len ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, false, true>)
                                      : reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, false>);
             if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kDecodeLdsMost) != hipSuccess)
@@ -1474,23 +1566,37 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
         }
     }
     FusedQkv fq = fused ? *fused : FusedQkv{};
-    if (fused)
+    if (ranges && fused)
+        attention_decode_kernel<HD, 2, true, false, true><<<grid, n_waves * kWave, lds, s>>>(
+            nullptr, static_cast<bf16_t*>(out), part_o, part_ml, static_cast<const bf16_t*>(k_cache),
+            static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start, kv_len, n_tokens, nq, nkv,
+            page_size, scale, window, 1, fq, nullptr, ranges);
+    else if (ranges)
+        attention_decode_kernel<HD, 2, false, true, true><<<grid, n_waves * kWave, lds, s>>>(
+            static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), part_o, part_ml,
+            static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start,
+            kv_len, n_tokens, nq, nkv, page_size, scale, window, 1, fq, q_len, ranges);
+    else if (fused)
         attention_decode_kernel<HD, PF, true><<<grid, n_waves * kWave, lds, s>>>(
             nullptr, static_cast<bf16_t*>(out), part_o, part_ml, static_cast<const bf16_t*>(k_cache),
             static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start, kv_len, n_tokens, nq, nkv,
-            page_size, scale, window, n_splits, fq, nullptr);
+            page_size, scale, window, n_splits, fq, nullptr, nullptr);
     else if (q_len)
         attention_decode_kernel<HD, PF, false, true><<<grid, n_waves * kWave, lds, s>>>(
             static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), part_o, part_ml,
             static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start,
-            kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, fq, q_len);
+            kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, fq, q_len, nullptr);
     else
         attention_decode_kernel<HD, PF, false><<<grid, n_waves * kWave, lds, s>>>(
             static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), part_o, part_ml,
             static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start,
-            kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, fq, nullptr);
+            kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, fq, nullptr, nullptr);
     EGPT_CHECK_LAUNCH();
-    if (n_splits > 1 && combine) {
+    if (ranges) {
+        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), n_tokens * nq,
+                                                             HD, 1, q_start, q_len, nq, ranges + slots * kRangeInts);
+        EGPT_CHECK_LAUNCH();
+    } else if (n_splits > 1 && combine) {
         attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), n_tokens * nq,
                                                              HD, n_splits, q_len ? q_start : nullptr, q_len, nq);
         EGPT_CHECK_LAUNCH();
@@ -1502,12 +1608,13 @@ static int dispatch_decode(const void* qkv, void* out, float* part_o, float* par
                            const void* v_cache, const int32_t* block_table, int table_width, const int32_t* q_start,
                            const int32_t* kv_len, int n_seqs, int nq, int nkv, int hd, int page_size, float scale,
                            int window, int n_splits, int n_waves, int combine, bool lean, const FusedQkv* fused,
-                           const int32_t* q_len, hipStream_t s) {
+                           const int32_t* q_len, const int32_t* ranges, int slots, hipStream_t s) {
     // lean: the variant with half the loads in flight and fewer registers (the caller's choice, see the wrapper)
 #define EGPT_LAUNCH_DECODE(HD_, PF_)                                                                                \
     launch_decode<HD_, PF_>(qkv, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len, \
                             n_seqs, n_seqs, nq, nkv, page_size, scale, window, n_splits, n_waves, combine, fused,   \
-                            q_len, s)
+                            q_len, ranges, slots, s)
+    if (ranges && (slots < n_seqs || slots > kRangeSlots || !part_o || !part_ml)) return EGPT_BAD_ARGUMENT;
     if (hd == 64) return lean ? EGPT_LAUNCH_DECODE(64, 2) : EGPT_LAUNCH_DECODE(64, 4);
     return lean ? EGPT_LAUNCH_DECODE(128, 1) : EGPT_LAUNCH_DECODE(128, 2);
 #undef EGPT_LAUNCH_DECODE
@@ -1555,12 +1662,13 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
                                                              HD, n_splits);
 }
 
-extern "C" int egpt_paged_attention_tiled(const void* qkv, void* out, const void* k_cache, const void* v_cache,
+static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache, const void* v_cache,
                                           const int32_t* block_table, int table_width, const int32_t* q_start,
                                           const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens,
                                           int nq, int nkv, int hd, int page_size, float scale, int window,
                                           int shape, int key_splits, float* part_o, float* part_ml,
-                                          int single_splits, int single_waves, int single_lean, void* stream) {
+                                          int single_splits, int single_waves, int single_lean, const int32_t* ranges, int slots,
+                                          float* range_o, float* range_ml, void* stream) {
     if (!qkv || !out || !k_cache || !v_cache || !block_table || !q_start || !q_len || !kv_len)
         return EGPT_BAD_ARGUMENT;
     if (n_seqs <= 0 || n_tokens < 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || table_width <= 0 || window < 0)
@@ -1618,10 +1726,36 @@ extern "C" int egpt_paged_attention_tiled(const void* qkv, void* out, const void
 #undef EGPT_ROWS32
     EGPT_CHECK_LAUNCH();
     if (skip_single)
-        return dispatch_decode(qkv, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                               n_seqs, nq, nkv, hd, page_size, scale, window, single_splits, single_waves, 1,
-                               single_lean != 0, nullptr, q_len, s);
+        return dispatch_decode(qkv, out, ranges ? range_o : part_o, ranges ? range_ml : part_ml, k_cache, v_cache, block_table, table_width,
+                               q_start, kv_len, n_seqs, nq, nkv, hd, page_size, scale, window, single_splits, single_waves, 1,
+                               single_lean != 0, nullptr, q_len, ranges, slots, s);
     return EGPT_OK;
+}
+
+extern "C" int egpt_paged_attention_tiled(const void* qkv, void* out, const void* k_cache, const void* v_cache,
+                                          const int32_t* block_table, int table_width, const int32_t* q_start,
+                                          const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens,
+                                          int nq, int nkv, int hd, int page_size, float scale, int window,
+                                          int shape, int key_splits, float* part_o, float* part_ml,
+                                          int single_splits, int single_waves, int single_lean, void* stream) {
+    return paged_attention_tiled(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, n_tokens, nq, nkv,
+                                 hd, page_size, scale, window, shape, key_splits, part_o, part_ml, single_splits, single_waves,
+                                 single_lean, nullptr, 0, nullptr, nullptr, stream);
+}
+
+// The same with the requests of one token dealt out by `ranges` (egpt_decode_ranges) over `slots` workgroups of eight wavefronts
+// per kv head; range_o [slots][nq][hd] and range_ml [slots][nq][2] take their parts.
+extern "C" int egpt_paged_attention_mixed(const void* qkv, void* out, const void* k_cache, const void* v_cache,
+                                          const int32_t* block_table, int table_width, const int32_t* q_start,
+                                          const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens,
+                                          int nq, int nkv, int hd, int page_size, float scale, int window,
+                                          int shape, int key_splits, float* part_o, float* part_ml,
+                                          const int32_t* ranges, int slots, float* range_o, float* range_ml, void* stream) {
+    if (!ranges || !range_o || !range_ml || slots < n_seqs) return EGPT_BAD_ARGUMENT;
+    if (slots > kRangeSlots) return EGPT_UNSUPPORTED_SIZE;
+    return paged_attention_tiled(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, n_tokens, nq, nkv,
+                                 hd, page_size, scale, window, shape, key_splits, part_o, part_ml, 1, 8, 1, ranges, slots, range_o,
+                                 range_ml, stream);
 }
 
 // One decoded token per request (n_tokens == n_seqs, q_len all 1), nq / nkv <= 16: workgroups of n_waves
@@ -1640,7 +1774,7 @@ extern "C" int egpt_paged_attention_decode(const void* qkv, void* out, float* pa
         return EGPT_UNSUPPORTED_SIZE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     return dispatch_decode(qkv, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean != 0, nullptr, nullptr, s);
+                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean != 0, nullptr, nullptr, nullptr, 0, s);
 }
 
 // The same with the QKV epilogue folded in: the queries, and the new token's key and value, are computed from
@@ -1648,13 +1782,14 @@ extern "C" int egpt_paged_attention_decode(const void* qkv, void* out, float* pa
 // squares row_ss [ss_splits][n_seqs] or null, bias or null), rotated over the whole head by the angles whose
 // cosines and sines are in cos_sin [n_seqs][hd / 2][2] (egpt_rope_table), and the key and value are stored at
 // slots[t] of the caches.  Token t belongs to request t.
-extern "C" int egpt_attention_decode_fused(const float* qkv_prod, int in_splits, const float* row_ss, int ss_splits,
+static int attention_decode_fused(const float* qkv_prod, int in_splits, const float* row_ss, int ss_splits,
                                            int hidden, float eps, const void* bias, const float* cos_sin,
                                            const int32_t* slots, void* out, float* part_o,
                                            float* part_ml, void* k_cache, void* v_cache, const int32_t* block_table,
                                            int table_width, const int32_t* q_start, const int32_t* kv_len, int n_seqs,
                                            int nq, int nkv, int hd, int page_size, float scale, int window,
-                                           int n_splits, int n_waves, int combine, int lean, void* stream) {
+                                           int n_splits, int n_waves, int combine, int lean, const int32_t* ranges,
+                                           int range_slots, void* stream) {
     if (!qkv_prod || in_splits < 1 || !cos_sin || !slots || !out || !k_cache || !v_cache ||
         !block_table || !q_start || !kv_len || (row_ss && (ss_splits < 1 || hidden < 1)))
         return EGPT_BAD_ARGUMENT;
@@ -1674,7 +1809,35 @@ extern "C" int egpt_attention_decode_fused(const float* qkv_prod, int in_splits,
     f.k_cache_w = static_cast<bf16_t*>(k_cache); f.v_cache_w = static_cast<bf16_t*>(v_cache);
     hipStream_t s = static_cast<hipStream_t>(stream);
     return dispatch_decode(nullptr, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean != 0, &f, nullptr, s);
+                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean != 0, &f, nullptr, ranges, range_slots, s);
+}
+
+extern "C" int egpt_attention_decode_fused(const float* qkv_prod, int in_splits, const float* row_ss, int ss_splits,
+                                           int hidden, float eps, const void* bias, const float* cos_sin,
+                                           const int32_t* slots, void* out, float* part_o,
+                                           float* part_ml, void* k_cache, void* v_cache, const int32_t* block_table,
+                                           int table_width, const int32_t* q_start, const int32_t* kv_len, int n_seqs,
+                                           int nq, int nkv, int hd, int page_size, float scale, int window,
+                                           int n_splits, int n_waves, int combine, int lean, void* stream) {
+    return attention_decode_fused(qkv_prod, in_splits, row_ss, ss_splits, hidden, eps, bias, cos_sin, slots, out, part_o, part_ml, k_cache,
+                                  v_cache, block_table, table_width, q_start, kv_len, n_seqs, nq, nkv, hd, page_size, scale, window,
+                                  n_splits, n_waves, combine, lean, nullptr, 0, stream);
+}
+
+// The same with the keys dealt out by `ranges` (egpt_decode_ranges) over range_slots workgroups of eight wavefronts per kv head;
+// part_o [range_slots][nq][hd] and part_ml [range_slots][nq][2] take their parts, which are combined into out.
+extern "C" int egpt_attention_decode_ranged(const float* qkv_prod, int in_splits, const float* row_ss, int ss_splits,
+                                            int hidden, float eps, const void* bias, const float* cos_sin,
+                                            const int32_t* slots, void* out, float* part_o,
+                                            float* part_ml, void* k_cache, void* v_cache, const int32_t* block_table,
+                                            int table_width, const int32_t* q_start, const int32_t* kv_len, int n_seqs,
+                                            int nq, int nkv, int hd, int page_size, float scale, int window,
+                                            const int32_t* ranges, int range_slots, void* stream) {
+    if (!ranges || !part_o || !part_ml || range_slots < n_seqs) return EGPT_BAD_ARGUMENT;
+    if (range_slots > kRangeSlots) return EGPT_UNSUPPORTED_SIZE;
+    return attention_decode_fused(qkv_prod, in_splits, row_ss, ss_splits, hidden, eps, bias, cos_sin, slots, out, part_o, part_ml, k_cache,
+                                  v_cache, block_table, table_width, q_start, kv_len, n_seqs, nq, nkv, hd, page_size, scale, window,
+                                  1, 8, 1, 1, ranges, range_slots, stream);
 }
 
 // bfloat16 only; head size 64 or 128; page size a multiple of 16.  rows_per_wave: 16 (decoded tokens) or 32.
@@ -1701,6 +1864,16 @@ extern "C" int egpt_paged_attention_mfma(const void* qkv, void* out, float* part
     if (hd == 64) return rows_per_wave == 16 ? launch_mfma<64, 1>(EGPT_ATTN_ARGS) : launch_mfma<64, 2>(EGPT_ATTN_ARGS);
     return rows_per_wave == 16 ? launch_mfma<128, 1>(EGPT_ATTN_ARGS) : launch_mfma<128, 2>(EGPT_ATTN_ARGS);
 #undef EGPT_ATTN_ARGS
+}
+
+// The table by which the decode kernels above deal out the keys (see decode_ranges_kernel): slots * 8 + n_seqs * 2 numbers.
+extern "C" int egpt_decode_ranges(const int32_t* kv_len, const int32_t* q_start, const int32_t* q_len, int n_seqs, int slots, int window,
+                                  int32_t* table, void* stream) {
+    if (!kv_len || !q_start || !table || n_seqs <= 0 || slots < n_seqs || window < 0) return EGPT_BAD_ARGUMENT;
+    if (slots > kRangeSlots) return EGPT_UNSUPPORTED_SIZE;
+    decode_ranges_kernel<<<1, kRangeSlots, 0, static_cast<hipStream_t>(stream)>>>(kv_len, q_start, q_len, n_seqs, slots, window, table);
+    EGPT_CHECK_LAUNCH();
+    return EGPT_OK;
 }
 
 // Combines the parts that egpt_paged_attention_mfma left with combine == 0: out [n_rows][hd] bfloat16.

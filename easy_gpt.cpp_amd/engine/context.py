@@ -28,6 +28,8 @@ class StepContext:
                            cache before any row's attention reads it
     single_token_requests  False when no request of the step brings exactly one token: a kernel that takes those apart
                            from the portions of prompts need not run
+    spread                 of a step of decoded tokens: 0 where the longest context is within 1.4 of the mean, 1 within 2.5, 2 beyond
+    portion_kv             a bound on kv_len over the requests that bring more than one token (None: max_kv_len)
     """
 
     num_tokens: int
@@ -54,6 +56,8 @@ class StepContext:
     shared: dict = field(default_factory=dict)     # what parts of several layers compute once per step and share
     rows_independent: bool = True
     single_token_requests: bool = True     # False when the step is known to hold no request of exactly one token
+    spread: int = 0
+    portion_kv: int | None = None
 
     def cache_view(self, cache_id: int, writes: bool) -> CacheView:
         g, j = self.cache_location[cache_id]

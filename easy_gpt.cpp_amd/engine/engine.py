@@ -253,7 +253,8 @@ class Engine:
         return StepContext(
             num_tokens=t, num_seqs=b, token_ids=d_tok, positions=d_pos, q_start=d_qs, q_len=d_ql, kv_len=d_kv,
             want_rows=d_want if want_rows else None, max_q_len=max(q_len), max_kv_len=max(kv_len),
-            single_token_requests=1 in q_len,
+            single_token_requests=1 in q_len, portion_kv=max((kv for kv, n in zip(kv_len, q_len) if n > 1), default=None),
+            spread=_spread(kv_len) if max(q_len) == 1 else 0,
             q_start_host=q_start, q_len_host=q_len, kv_len_host=kv_len,
             state_slots=d_slot, state_slots_host=[rc.slot for rc in rcs],
             groups=groups, page_size=ps, kv_storage=self.kv, state_storage=self.states,
@@ -325,9 +326,12 @@ class Engine:
         widths = self._table_widths(rcs)
         # The kernels choose their shape (key splits of the attention) by the longest context, and a graph holds
         # one choice: contexts are bucketed in steps of 512 tokens beside the table widths.
-        kv_bound = -(-(max(rc.num_tokens for rc in rcs) + 1) // 512) * 512
-        key = (rows, tuple(widths), kv_bound)
-        plan = self._plan(self._decode_plans, key, lambda: _DecodePlan(self, rows, widths, kv_bound))
+        longest = max(rc.num_tokens for rc in rcs) + 1
+        kv_bound = -(-longest // 512) * 512
+        # ... and how they deal out the keys by how uneven the contexts are (of little consequence up to 16 requests)
+        spread = _spread([rc.num_tokens + 1 for rc in rcs])
+        key = (rows, tuple(widths), (kv_bound, spread))
+        plan = self._plan(self._decode_plans, key, lambda: _DecodePlan(self, rows, widths, kv_bound, spread=spread))
         plan.fill(rcs, tokens)
         if device_tokens is not None:
             plan.ctx.token_ids[:b].copy_(device_tokens, non_blocking=True)      # (behind the upload of the metadata)
@@ -436,11 +440,26 @@ class Engine:
         # (steps with and without requests of one token have graphs of their own: the attention takes those requests
         # apart, in a kernel that the others need not launch; the padding's tokens go either way)
         singles = 1 in counts
-        key = (t_pad, b_pad, r_pad, tuple(widths), singles)
-        plan = self._plan(self._padded_plans, key, lambda: _PaddedPlan(self, t_pad, b_pad, r_pad, widths, singles))
+        # (the attention's shape for the portions goes by their longest context, in powers of two: a new prompt's portion beside
+        # long conversations is not one behind a prefix)
+        portion_kv = t_pad
+        longest = max((rc.num_tokens + n for rc, n in zip(rcs, counts) if n > 1), default=0)
+        while portion_kv < longest:
+            portion_kv *= 2
+        portion_kv = min([portion_kv] + [w * self.page_size for w in widths])
+        key = (t_pad, b_pad, r_pad, tuple(widths), singles, portion_kv)
+        plan = self._plan(self._padded_plans, key, lambda: _PaddedPlan(self, t_pad, b_pad, r_pad, widths, singles, portion_kv))
         n_want = plan.fill(rcs, entries, counts)
         logits = self._run(plan)
         return logits[:n_want] if n_want else None
+
+
+def _spread(contexts: list[int]) -> int:
+    """`StepContext.spread` of a step of decoded tokens; up to 16 of them nothing goes by it."""
+    if len(contexts) <= 16:
+        return 0
+    longest, total = max(contexts) * len(contexts), sum(contexts)
+    return 2 if longest > 2.5 * total else 1 if longest > 1.4 * total else 0
 
 
 def _capture(graph, pool, run):
@@ -461,7 +480,8 @@ def _capture(graph, pool, run):
 class _PaddedPlan:
     """Static buffers, a pinned host mirror and the captured graph of one padded step size."""
 
-    def __init__(self, engine: Engine, t_pad: int, b_pad: int, r_pad: int, widths: list[int], singles: bool = True):
+    def __init__(self, engine: Engine, t_pad: int, b_pad: int, r_pad: int, widths: list[int], singles: bool = True,
+                 portion_kv: int | None = None):
         self.t_pad, self.b_pad, self.widths = t_pad, b_pad, list(widths)
         # (no reference back to the engine: engine and plan would keep each other alive until the collector of
         # reference cycles runs, which may be in the middle of another engine's graph capture, where memory of
@@ -489,7 +509,7 @@ class _PaddedPlan:
             q_start_host=[0] * b_pad, q_len_host=[0] * b_pad, kv_len_host=[0] * b_pad,
             state_slots=view(5), state_slots_host=[0] * b_pad, groups=groups, page_size=ps, kv_storage=engine.kv,
             state_storage=engine.states, cache_location=engine.model.cache_location,
-            group_windows=[n.window for n in engine.cache.groups], single_token_requests=singles,
+            group_windows=[n.window for n in engine.cache.groups], single_token_requests=singles, portion_kv=portion_kv,
         )
         self.c_widths = _ints(self.widths)
         self.copied = None
@@ -561,7 +581,7 @@ class _PaddedPlan:
 class _DecodePlan:
     """Static device buffers, a host mirror and the captured graph of one decode batch shape."""
 
-    def __init__(self, engine: Engine, batch: int, widths: list[int], kv_bound: int, rows_independent: bool = True):
+    def __init__(self, engine: Engine, batch: int, widths: list[int], kv_bound: int, rows_independent: bool = True, spread: int = 0):
         self.batch, self.widths = batch, list(widths)
         dev = engine.device
         n_groups = len(widths)
@@ -585,7 +605,7 @@ class _DecodePlan:
             q_start_host=list(range(b)), q_len_host=[1] * b, kv_len_host=[0] * b,
             state_slots=v(5), state_slots_host=[0] * b, groups=groups, page_size=ps, kv_storage=engine.kv,
             state_storage=engine.states, cache_location=engine.model.cache_location,
-            group_windows=[n.window for n in engine.cache.groups], rows_independent=rows_independent,
+            group_windows=[n.window for n in engine.cache.groups], rows_independent=rows_independent, spread=spread,
         )
         self.row_state = np.full(2 * b, -1, dtype=np.int64)     # per row: (handle, table version) last written
         self.c_widths = _ints(self.widths)

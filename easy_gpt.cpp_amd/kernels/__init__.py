@@ -244,6 +244,16 @@ class KernelBackend:
         sums; False if not covered (nothing was done), else what paged_attention returns."""
         return False
 
+    def decode_ranges(self, kv_len, q_start, q_len, nkv, hd, window, max_kv_len, spread=0):
+        """What the attention of decoded tokens needs to deal out their keys by the contexts' lengths (the `ranges` of
+        attention_decode_fused and paged_attention_mixed; the same for all layers of a kind), or None."""
+        return None
+
+    def paged_attention_mixed(self, *args, ranges=None, portion_kv=None, **kwargs):
+        """paged_attention with two hints: the table of `decode_ranges`, and the longest context of a request that brings
+        more than one token."""
+        return self.paged_attention(*args, **kwargs)
+
     def combine_attention(self, part_o, part_ml, out):
         """out act [T, nq*hd] from the parts of a split attention."""
         raise NotImplementedError

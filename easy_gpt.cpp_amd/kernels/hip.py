@@ -93,6 +93,10 @@ class HipKernels(KernelBackend):
             "egpt_paged_attention_decode": [vp, vp, vp, vp, vp, vp, vp, i, vp, vp, i, i, i, i, i, f, i, i, i, i, i, vp],
             "egpt_attention_decode_fused": [vp, i, vp, i, i, f, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, vp, vp, i, i, i,
                                             i, i, f, i, i, i, i, i, vp],
+            "egpt_decode_ranges": [vp, vp, vp, i, i, i, vp, vp],
+            "egpt_paged_attention_mixed": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, i, vp, vp, vp, i, vp, vp, vp],
+            "egpt_attention_decode_ranged": [vp, i, vp, i, i, f, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, vp, vp, i, i, i, i, i, f, i, vp, i,
+                                             vp],
             "egpt_linear": [vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_f32": [vp, vp, vp, vp, i, i, i, i, vp],
             "egpt_gemm_f32_rows": [vp, vp, vp, vp, i, i, i, i, i, i, vp],
@@ -793,11 +797,41 @@ class HipKernels(KernelBackend):
                   self._ptr(k_cache), self._ptr(v_cache), t, nq, nkv, hd, page_size, dt, self._stream())
         return out
 
+    def decode_ranges(self, kv_len, q_start, q_len, nkv, hd, window, max_kv_len, spread=0):
+        """The table by which the attention of decoded tokens deals out their keys by the contexts' lengths, int32
+        [slots * 8 + B * 2], or None where every request gets the same number of key ranges (`_decode_shape`).  q_len given: a step
+        that also holds portions of prompts.  spread: how uneven the contexts are (`StepContext.spread`)."""
+        (b,) = kv_len.shape
+        if hd not in (64, 128):
+            return None
+        if q_len is None:
+            # A step of decoded tokens, whose parts a kernel combines.  Where the contexts are as long as each other the ranges are
+            # the same and the table is one more trip to memory (0.2 to 0.9 us a layer), so it is taken where they are not: us a layer,
+            # combination included, equal ranges and dealt out: 12 heads of 128 on 2, 40 requests of 128 to 2,048 tokens 23.5 and 18.2, 28
+            # heads of 128 on 4, 24 of 200 to 1,400 19.1 and 17.7 (64 of them, more pairs than half the CUs: 32.3 and 34.5), 14 heads of 64
+            # on 2, 64 of 130 to 2,048 17.0 and 16.5, which the table's own 5 us a step use up, one of 8,000 beside 31 of 500 21.8 and 15.0
+            if b <= self.fused_rows or b * nkv > 128 or max_kv_len > 9216 or spread < (2 if hd == 64 else 1):
+                return None
+        elif b * nkv > 256 or max_kv_len <= (self.singles_apart_beyond if hd == 64 else self.singles_dealt_beyond):
+            return None
+        for name, v in (("kv_len", kv_len), ("q_start", q_start)) + ((("q_len", q_len),) if q_len is not None else ()):
+            self._need(v, name, _I32, (b,))
+        slots = 256 // nkv
+        table = torch.empty(slots * 8 + b * 2, dtype=_I32, device=kv_len.device)
+        self._run("egpt_decode_ranges", kv_len.data_ptr(), q_start.data_ptr(), self._ptr(q_len), b, slots, int(window), table.data_ptr(),
+                  self._stream())
+        return table
+
+    def paged_attention_mixed(self, *args, ranges=None, portion_kv=None, **kwargs):
+        return self.paged_attention(*args, ranges=ranges, portion_kv=portion_kv, **kwargs)
+
     def paged_attention(self, qkv, out, k_cache, v_cache, block_table, q_start, q_len, kv_len, nq, nkv, hd, page_size,
-                        scale, window, max_q_len, max_kv_len, combine=True, singles=True):
+                        scale, window, max_q_len, max_kv_len, combine=True, singles=True, ranges=None, portion_kv=None):
         """combine=False: when the kernel splits the key range, leave the parts to the caller and return
         (part_o [S, T, nq, hd], part_ml [S, T, nq, 2]); `out` is then not written.  Returns None otherwise.
-        singles=False: no request brings exactly one token (a hint: the kernel that takes those apart is not launched)."""
+        singles=False: no request brings exactly one token (a hint: the kernel that takes those apart is not launched).
+        ranges: the table of `decode_ranges` for these requests.  portion_kv: the longest context of a request that brings
+        more than one token (None: the longest of all)."""
         t = qkv.shape[0]
         b, width = block_table.shape
         dt = self._act(qkv, "qkv")
@@ -857,18 +891,34 @@ class HipKernels(KernelBackend):
                 # 643, 141x1: 59 / 665, 141x4: 30 / 185; 28 heads on 4: 141x1: 61 / 671, 141x2: 48 / 378; 40 heads on 8
                 # (160 workgroups): 141x1: 103 / 679.
                 key_splits = 1
-                # (behind a prefix: the longest context is a few thousand tokens and at least twice the step's own)
-                if (blocks_of_32 and max_kv_len >= 2 * t
-                        and max_kv_len >= (self.prefix_keys if hd == 64 else self.prefix_keys // 2)):
+                # (behind a prefix: the portions' longest context is a few thousand tokens and at least twice the step's own.  Not the
+                # longest of all: one portion of 512 tokens of a new prompt beside 40 decoded tokens behind 128 to 2,048, 12 heads of
+                # 128 on 2: 51.8 us a layer in four key ranges, 48.0 in one; 8 behind 1,400 and 28 heads on 4 46.6 and 31.1)
+                longest = max_kv_len if portion_kv is None else min(portion_kv, max_kv_len)
+                if (blocks_of_32 and longest >= 2 * t
+                        and longest >= (self.prefix_keys if hd == 64 else self.prefix_keys // 2)):
                     shape = 142 if hd == 64 else 141
                     workgroups = -(-row_tiles // 8)
-                    tiles = -(-max_kv_len // (64 * (shape % 10)))
+                    tiles = -(-longest // (64 * (shape % 10)))
                     key_splits = max(1, min(256 // workgroups, tiles // 4, 16))
                 # Requests that bring one token (decoded tokens beside the portions) go to the decode kernel in a second
                 # launch: here one workgroup would walk all of such a request's keys, 128 or 256 per iteration of some
                 # 1.7 us, and the longest of them sets the launch's time
                 part_o = part_ml = None
                 n_splits = n_waves = lean = 0
+                if ranges is not None and singles and nq // nkv <= 16:
+                    slots = self._need_ranges(ranges, b, nkv)
+                    range_o = torch.empty((slots, nq, hd), dtype=_F32, device=qkv.device)
+                    range_ml = torch.empty((slots, nq, 2), dtype=_F32, device=qkv.device)
+                    if key_splits > 1:
+                        part_o = torch.empty((key_splits * t, nq, hd), dtype=_F32, device=qkv.device)
+                        part_ml = torch.empty((key_splits * t, nq, 2), dtype=_F32, device=qkv.device)
+                    self._run("egpt_paged_attention_mixed", qkv.data_ptr(), out.data_ptr(), k_cache.data_ptr(),
+                              v_cache.data_ptr(), block_table.data_ptr(), width, q_start.data_ptr(), q_len.data_ptr(),
+                              kv_len.data_ptr(), b, t, nq, nkv, hd, page_size, float(scale), int(window), shape, key_splits,
+                              self._ptr(part_o), self._ptr(part_ml), ranges.data_ptr(), slots, range_o.data_ptr(), range_ml.data_ptr(),
+                              self._stream())
+                    return None
                 if singles and b > 1 and nq // nkv <= 16 and max_kv_len > self.singles_apart_beyond:
                     n_splits, n_waves, lean = self._decode_shape(b, nkv, hd, max_kv_len, True)
                 parts_rows = max(n_splits * b if n_splits > 1 else 0, key_splits * t if key_splits > 1 else 0)
@@ -918,8 +968,19 @@ class HipKernels(KernelBackend):
     # 16.2 against 18.6, behind 4,000 33.2 against 20.5, behind 16,000 122 against 32; four portions beside 24 decoded
     # tokens behind 1,300 keys 36.7 against 38.1, behind 4,000 61.6 against 43.5, behind 16,000 152 against 66
     singles_apart_beyond = 2048
+    # Dealt out by the contexts' lengths (`decode_ranges`) they go there, at head size 128, beyond this.  The tiled kernel alone against it, one
+    # portion of 512 tokens of a new prompt beside decoded ones: 12 heads of 128 on 2, 40 behind 128 to 2,048 48.3 and 36.7 (in equal
+    # ranges 42.3); 28 heads of 128 on 4, 8 behind 1,400 31.3 and 29.9, behind 700 23.4 and 28.6; 14 heads of 64 on 2, 40 behind 128 to
+    # 2,048 24.0 and 29.7, 8 behind 4,000 35.6 and 21.2 (in equal ranges 21.0)
+    singles_dealt_beyond = 1024
     prefix_keys = 4096           # a step's longest context from which its portions are taken to lie behind a prefix
     attention_segment = 64       # keys per segment of the decode kernel for any head size (kSegment in attention_any.hip)
+
+    def _need_ranges(self, ranges, b: int, nkv: int) -> int:
+        """The slots of a table that `decode_ranges` made for b requests."""
+        slots = 256 // nkv
+        self._need(ranges, "ranges", _I32, (slots * 8 + b * 2,))
+        return slots
 
     @staticmethod
     def _decode_shape(b, nkv, hd, max_kv_len, combine):
@@ -1007,7 +1068,7 @@ class HipKernels(KernelBackend):
 
     def attention_decode_fused(self, prod, row_ss, hidden, eps, bias, positions, inv_freq, rotary_dim, slots, out,
                                k_cache, v_cache, block_table, q_start, kv_len, nq, nkv, hd, page_size, scale, window,
-                               max_kv_len, combine=True, cos_sin=None):
+                               max_kv_len, combine=True, cos_sin=None, ranges=None):
         """Attention for a batch of single decoded tokens (token t belongs to request t) straight from the QKV
         product's float32 partial sums prod [S, T, W]: what qkv_rope_store and paged_attention do together, in
         one kernel.  Returns False if the case is not covered (nothing was done), else what paged_attention
@@ -1038,6 +1099,16 @@ class HipKernels(KernelBackend):
             self._need(row_ss, "row_ss", _F32, (ss_splits, t))
         if max_kv_len > table_width * page_size:
             raise ValueError(f"block table of width {table_width} cannot hold {max_kv_len} tokens at page size {page_size}")
+        if ranges is not None and combine:
+            n_slots = self._need_ranges(ranges, b, nkv)
+            part_o = torch.empty((n_slots, nq, hd), dtype=_F32, device=prod.device)
+            part_ml = torch.empty((n_slots, nq, 2), dtype=_F32, device=prod.device)
+            self._run("egpt_attention_decode_ranged", prod.data_ptr(), int(in_splits), self._ptr(row_ss), ss_splits, int(hidden),
+                      float(eps), self._ptr(bias), cos_sin.data_ptr(), slots.data_ptr(), out.data_ptr(),
+                      part_o.data_ptr(), part_ml.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(),
+                      table_width, q_start.data_ptr(), kv_len.data_ptr(), b, nq, nkv, hd, page_size, float(scale),
+                      int(window), ranges.data_ptr(), n_slots, self._stream())
+            return None
         n_splits, n_waves, lean = self._decode_shape(b, nkv, hd, max_kv_len, combine)
         part_o = part_ml = None
         if n_splits > 1:

@@ -130,18 +130,19 @@ class GQAttention(Mixer):
         # the cache in one kernel, straight from the product's partial sums
         parts = False
         cos_sin = self.position.table(ctx) if rot is not None else None
+        ranges = None if want_parts else self._ranges(k, ctx)
         if (prod.dim() == 3 and rot is not None and slots is not None and ctx.max_q_len == 1
                 and ctx.rows_independent):
             parts = k.attention_decode_fused(
                 prod, scale_args.get("row_ss"), scale_args.get("hidden", 0), scale_args.get("eps", 0.0), self.b_qkv,
                 ctx.positions, rot[0], rot[1], slots, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.kv_len,
                 self.n_heads, self.n_kv_heads, self.head_dim, cache.page_size, self.scale, self.window or 0,
-                ctx.max_kv_len, combine=not want_parts, cos_sin=cos_sin)
+                ctx.max_kv_len, combine=not want_parts, cos_sin=cos_sin, ranges=ranges)
         if parts is False:
             if cos_sin is not None:
                 scale_args = dict(scale_args, cos_sin=cos_sin)
             parts = self._epilogue_and_attention(k, prod, t, width, dtype, device, rot, slots, common, scale_args, ctx,
-                                                 cache, attn, want_parts)
+                                                 cache, attn, want_parts, ranges)
         # the output projection: into the residual stream itself where that takes additions (then nothing is returned)
         residual = pending.residual() if pending is not None else None
         if parts is not None:
@@ -156,8 +157,18 @@ class GQAttention(Mixer):
         k.linear(attn, self.w_o, self.b_o, out)
         return out
 
+    def _ranges(self, k, ctx):
+        """How the keys of the step's decoded tokens are dealt out, the same for all layers with these heads and this window."""
+        if not ctx.rows_independent or (ctx.max_q_len > 1 and not getattr(ctx, "single_token_requests", True)):
+            return None
+        key = ("decode_ranges", self.n_kv_heads, self.head_dim, self.window)
+        if key not in ctx.shared:
+            ctx.shared[key] = k.decode_ranges(ctx.kv_len, ctx.q_start, None if ctx.max_q_len == 1 else ctx.q_len, self.n_kv_heads,
+                                              self.head_dim, self.window or 0, ctx.max_kv_len, getattr(ctx, "spread", 0))
+        return ctx.shared[key]
+
     def _epilogue_and_attention(self, k, prod, t, width, dtype, device, rot, slots, common, scale_args, ctx, cache, attn,
-                                want_parts):
+                                want_parts, ranges):
         """Bias, position encoding and the store into the cache, then attention over the cache; returns what
         paged_attention returns (the parts of a split key range, or None when `attn` is written)."""
         qkv = prod if prod.dim() == 2 else torch.empty((t, width), dtype=dtype, device=device)
@@ -181,8 +192,8 @@ class GQAttention(Mixer):
         )
         if want_parts:
             args["combine"] = False
-        return k.paged_attention(qkv, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len,
-                                 **args)
+        return k.paged_attention_mixed(qkv, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len,
+                                       ranges=ranges, portion_kv=getattr(ctx, "portion_kv", None), **args)
 
 
 register_part("mixer", "gq_attention", GQAttention)
