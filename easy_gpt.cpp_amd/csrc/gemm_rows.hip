@@ -10,6 +10,8 @@
 // half's operands in registers already; behind it the next loads go out and the next step's first half is read under the
 // second half's products.
 //
+// Tiles of few rows and columns keep five or six steps of both operands on their way where there are few of them: a step of 64 x 64
+// takes 0.17 us so and 0.32 with two and three, which is the L2's latency (600 x 896 x 4,864 in one range 30.4 us -> 19.1).
 // A workgroup stays for several tiles: as many are launched as the CUs hold, and the loads of a workgroup's next tile go out under
 // the last steps of the one before, so that a tile's first products do not wait for memory and the result leaves meanwhile.
 //
@@ -101,7 +103,7 @@ struct Groups {
     int x_rows;                    // rows of x
 };
 
-template <int BM, int BN, int WM, int WN, int WB, int OUT, bool GROUPED>
+template <int BM, int BN, int WM, int WN, int XB, int WB, int OUT, bool GROUPED>
 __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) void gemm_rows_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k, int splits,
     int steps_per_split, int act, Groups groups) {
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
     constexpr int XL = BM / 8 / NW, WL = BN / 8 / NW;          // loads of a wavefront per step: eight rows each
     static_assert(XL * 8 * NW == BM && WL * 8 * NW == BN, "a step is whole loads");
     constexpr int kXBytes = BM * 128, kWBytes = BN * 128;
-    __shared__ __attribute__((aligned(128))) char xs[2 * kXBytes];
+    __shared__ __attribute__((aligned(128))) char xs[XB * kXBytes];
     __shared__ __attribute__((aligned(128))) char ws[WB * kWBytes];
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int li = lane % 16, lg = lane / 16;
@@ -203,6 +205,9 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
         from.at += from.by;
         --from.left;
     };
+    // at most this many loads behind those of the step that is waited for: step s asks for x of step s + XB, then for w of s + WB
+    constexpr int kBehind = XB < WB ? WL + (XB - 2) * (XL + WL) : (WB - 2) * (XL + WL);
+    static_assert(XB >= 2 && XB <= WB, "the order of a step's loads");
     auto load_w = [&](int buffer, Source& from) {
 #pragma unroll
         for (int i = 0; i < WL; ++i) load_to_lds(from.rows, wo[i], from.at, ws + buffer * kWBytes + (wave * WL + i) * 1024);
@@ -298,29 +303,30 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
     };
     Source fx = source_x(now), fw = source_w(now);
     const Item none = item_of(items);
-    load_x(0, fx);
-    load_w(0, fw);
-    if (fx.left == 0) fx = source_x(none);
-    if (fw.left == 0) fw = source_w(none);
-    load_x(1, fx);
+    // (the order in which the loop would have asked)
 #pragma unroll
-    for (int i = 1; i < WB; ++i) {
-        load_w(i, fw);
-        if (fw.left == 0 && i + 1 < WB) fw = source_w(none);
+    for (int i = -WB; i < 0; ++i) {
+        if (i + XB >= 0) {
+            if (fx.left == 0) fx = source_x(none);
+            load_x(i + XB, fx);
+        }
+        if (fw.left == 0) fw = source_w(none);
+        load_w(i + WB, fw);
     }
     // (where there is a next item, this one has WB steps at least)
     Item next = item_of(index + gridDim.x);
     clear();
-    arrived<0>();
+    arrived<kBehind + XL + WL>();
     __syncthreads();
     read(0, 0, 0);
+    // xb, wb: the buffers of the step
     int xb = 0, wb = 0, left = now.end - now.begin;
     auto step = [&]() {
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
         load_x(xb, fx);
         load_w(wb, fw);
-        xb ^= 1;
+        xb = XB == 2 ? xb ^ 1 : xb + 1 == XB ? 0 : xb + 1;
         wb = wb + 1 == WB ? 0 : wb + 1;
         read(xb, wb, 0);
         multiply(1);
@@ -332,8 +338,8 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
         // an item's first step and its last WB ones, under which the loads of the workgroup's next item begin
         read(xb, wb, 1);
         multiply(0);
-        if (stored) arrived<((WB - 2) * WL + kStores < 63 ? (WB - 2) * WL + kStores : 63)>();
-        else arrived<(WB - 2) * WL>();
+        if (stored) arrived<(kBehind + kStores < 63 ? kBehind + kStores : 63)>();
+        else arrived<kBehind>();
         stored = false;
         if (fx.left == 0) fx = source_x(next);
         if (fw.left == 0) fw = source_w(next);
@@ -343,7 +349,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
         while (left > WB) {
             read(xb, wb, 1);
             multiply(0);
-            arrived<(WB - 2) * WL>();
+            arrived<kBehind>();
             step();
         }
         if (left > 0) continue;
@@ -360,27 +366,27 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
 #endif
 }
 
-template <int BM, int BN, int WM, int WN, int WB>
+template <int BM, int BN, int WM, int WN, int XB, int WB>
 int launch_rows(const void* x, const void* w, void* out, int m, int n, int k, int splits, int per, int kind, int act, hipStream_t s) {
     const long mt = (m + BM - 1) / BM, nt = kind == kRowsGated ? (n + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
     if (mt * nt * splits > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
     // as many workgroups as the CUs hold, each taking its items in turn, where every item has the three steps that are on
     // their way when it begins; else a workgroup per item
-    constexpr int kHeld = kLdsOfCu / ((2 * BM + WB * BN) * 128);
+    constexpr int kHeld = kLdsOfCu / ((XB * BM + WB * BN) * 128);
     const int last_steps = k / kRowsStep - (splits - 1) * per;
     const long held = per >= WB && last_steps >= WB ? 256L * kHeld : mt * nt * splits;
     const dim3 grid(static_cast<unsigned>(mt * nt * splits < held ? mt * nt * splits : held));
     const auto* xp = static_cast<const bf16_t*>(x);
     const auto* wp = static_cast<const bf16_t*>(w);
     const Groups none{nullptr, nullptr, 0};
-    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsGated, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
-    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsF32, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
-    else gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsBf16, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsGated, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsF32, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    else gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsBf16, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
 
-template <int BM, int BN, int WM, int WN, int WB>
+template <int BM, int BN, int WM, int WN, int XB, int WB>
 int launch_groups(const void* x, const void* w, void* out, const Groups& g, long tiles, int n, int k, int kind, int act, hipStream_t s) {
     const long nt = kind == kRowsGated ? (n + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
     if (tiles * nt > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
@@ -388,9 +394,9 @@ int launch_groups(const void* x, const void* w, void* out, const Groups& g, long
     const auto* xp = static_cast<const bf16_t*>(x);
     const auto* wp = static_cast<const bf16_t*>(w);
     const int per = k / kRowsStep;
-    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsGated, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
-    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsF32, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
-    else gemm_rows_kernel<BM, BN, WM, WN, WB, kRowsRelu2, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
+    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsGated, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
+    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsF32, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
+    else gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsRelu2, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
@@ -412,11 +418,13 @@ extern "C" int egpt_gemm_rows(const void* x, const void* w, void* out, int m, in
     hipStream_t s = static_cast<hipStream_t>(stream);
     // the tiles that `_rows_shapes` in kernels/hip.py chooses from
     switch (shape) {
-        case 0: return launch_rows<256, 256, 2, 4, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
-        case 1: return launch_rows<192, 256, 2, 4, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
-        case 2: return launch_rows<128, 256, 2, 4, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
-        case 3: return launch_rows<128, 128, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
-        case 4: return launch_rows<64, 64, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 0: return launch_rows<256, 256, 2, 4, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 1: return launch_rows<192, 256, 2, 4, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 2: return launch_rows<128, 256, 2, 4, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 3: return launch_rows<128, 128, 2, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 4: return launch_rows<64, 64, 2, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 5: return launch_rows<64, 64, 2, 2, 5, 5>(x, w, out, m, n, k, splits, per, kind, act, s);
+        case 6: return launch_rows<64, 128, 2, 2, 6, 6>(x, w, out, m, n, k, splits, per, kind, act, s);
         default: return EGPT_BAD_ARGUMENT;
     }
 }
@@ -435,8 +443,8 @@ extern "C" int egpt_moe_rows(const void* x, const void* w, const int32_t* row_to
     const Groups g{tiles, row_token, x_rows};
     const long most = tile_rows > 0 ? n_rows / tile_rows + experts + 1 : 0;
     switch (tile_rows) {
-        case 64: return launch_groups<64, 64, 2, 2, 3>(x, w, out, g, most, n, k, kind, act, s);
-        case 128: return launch_groups<128, 128, 2, 2, 3>(x, w, out, g, most, n, k, kind, act, s);
+        case 64: return launch_groups<64, 64, 2, 2, 2, 3>(x, w, out, g, most, n, k, kind, act, s);
+        case 128: return launch_groups<128, 128, 2, 2, 2, 3>(x, w, out, g, most, n, k, kind, act, s);
         default: return EGPT_BAD_ARGUMENT;
     }
 }

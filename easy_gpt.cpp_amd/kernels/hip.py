@@ -291,32 +291,36 @@ class HipKernels(KernelBackend):
         return n * k >= (6 << 20 if m > 32 else 16 << 20)
 
     # The tiles of the product for many rows (gemm_rows.hip): rows of x, rows of w, workgroups that a CU holds, and a fit of
-    # what was measured (some 250 sizes of 72 to 8,191 rows, 12 matrices; a tenth off on average): microseconds of a launch, of
-    # a round of workgroups, and of a step of 64 values of k with one workgroup on a CU and with as many as it holds.
-    _rows_shapes = ((256, 256, 1, -4.4, 16.7, 1.14, 1.14), (192, 256, 1, -2.4, 12.7, 0.94, 0.94), (128, 256, 1, -0.8, 9.0, 0.83, 0.83),
-                    (128, 128, 2, 4.8, 1.8, 0.50, 1.33), (64, 64, 4, 6.3, -2.7, 0.36, 1.06))
+    # what was measured (some 460 sizes of 70 to 8,191 rows, 25 matrices): microseconds of a launch, of a round of workgroups, of a
+    # step of 64 values of k with one workgroup on a CU and with as many as it holds, what the form of the result (rounded,
+    # float32, activated) adds to a round, and the rate in TB/s at which the tiles take the weights from memory.
+    _rows_shapes = ((256, 256, 1, 4.01, 4.34, 1.21, 1.39, (0.0, 5.72, 0.74), 5.76), (192, 256, 1, 3.62, 3.21, 0.98, 1.1, (0.0, 4.65, 0.28), 4.18),
+                    (128, 256, 1, 3.95, 0.28, 0.85, 0.9, (0.0, 4.18, 1.13), 4.24), (128, 128, 2, 3.8, -0.03, 0.52, 0.97, (0.0, 1.93, 0.2), 3.61),
+                    (64, 64, 4, 3.93, -0.62, 0.22, 0.81, (0.0, 0.57, 0.29), 2.78), (64, 64, 2, 4.43, -0.67, 0.21, 0.43, (0.0, 0.55, 0.49), 3.15),
+                    (64, 128, 1, 3.76, 1.1, 0.35, 0.37, (0.0, 0.8, 0.63), 3.16))
 
     @classmethod
     @functools.lru_cache(maxsize=4096)
-    def _rows_plan(cls, m: int, n: int, k: int, most_splits: int) -> tuple[int, int]:
+    def _rows_plan(cls, m: int, n: int, k: int, most_splits: int, form: int = 0) -> tuple[int, int]:
         """(shape, splits of the k range) of the product for many rows: the cheapest by the fit, a split paying for what
-        its reader reads more (4.5 TB/s).  `n`: the rows of w.  (Against the best of everything that was measured, the
-        choice is 8 % slower on average and a third at worst.)  Found once per sizes, so once for a step's layers: it takes the
-        host 20 to 50 us with ten splits to choose from, as long as several of the products it is for."""
+        its reader reads more (4.5 TB/s).  `n`: the rows of w; `form`: 0 rounded, 1 float32, 2 activated.  (Against the best of
+        everything that was measured the choice is 1 % slower activated, 0.5 % in float32, 1.7 % where k may be split.)  Found once
+        per sizes, so once for a step's layers: it takes the host 20 to 50 us with ten splits to choose from, as long as several of the
+        products it is for."""
         steps = k // 64
         best = None
-        for shape, (bm, bn, held, launch, per_round, alone, full) in enumerate(cls._rows_shapes):
+        for shape, (bm, bn, held, launch, per_round, alone, full, more, rate) in enumerate(cls._rows_shapes):
             tiles = -(-m // bm) * -(-n // bn)
             for s in range(1, most_splits + 1):
                 per = -(-steps // s)
                 if s > 1 and (per < 4 or (s - 1) * per >= steps or s * tiles > 700):
                     continue
+                round_us = per_round + more[form if s == 1 else 1]
                 rounds, rest = divmod(s * tiles, 256 * held)
-                us = launch + rounds * (per_round + per * full)
+                us = launch + rounds * (round_us + per * full)
                 if rest:
-                    load = max(rest / 256, 1.0)
-                    us += per_round + per * (alone + (full - alone) * (load - 1) / max(held - 1, 1))
-                us = max(us, 3 + n * k * 2 / 4.4e6)                 # the weights alone
+                    us += round_us + per * (alone + (full - alone) * (-(-rest // 256) - 1) / max(held - 1, 1))
+                us = max(us, 3 + n * k * 2 / (rate * 1e6))          # the weights alone
                 if s > 1:
                     us += m * n * (4 * s - 2) / 4.5e6
                 if best is None or us < best[0]:
@@ -367,14 +371,13 @@ class HipKernels(KernelBackend):
         return m <= 448 if n <= k else n < 2 * k and m <= 256
 
     @staticmethod
-    def _own_short(n: int, k: int) -> bool:
-        """Whether the product is the framework's own with every number of rows above 64, also beyond the lines of `_own_rows`: a short k
-        range makes a tile of its beginning and its end for the most part, and a workgroup's next tile begins under the
-        end of the one before.  us, weights from memory, rounded: 896 x 896 at 2,535 / 6,000 / 8,191 rows 10.5 / 16.4 / 17.5 against 19.5 /
-        19.0 / 23.8, 2,752 x 896 at 3,584 / 8,191 22.0 / 40.8 against 29.6 / 62.6; unrounded: 1,152 x 896 at 2,048 / 6,000 / 8,191 11.8 / 20.0 /
-        25.1 against 13.0 / 26.6 / 27.4.  Three times as wide as long there is nothing left: 3,072 x 1,024 unrounded at 2,048 / 8,191 rows 20.7 /
-        61.6 against 19.4 / 55.4."""
-        return k <= 1024 and n <= 2 * k or k <= 896 and n < 4 * k
+    def _own_short(m: int, n: int, k: int) -> bool:
+        """Whether the product is the framework's own beyond the lines of `_own_rows`: with a short k range a tile is its beginning and its
+        end for the most part, and a workgroup's next tile begins under the end of the one before.  us, weights from memory, replayed from
+        a graph: 896 x 896 rounded, with its norm, at 2,535 / 3,500 / 5,000 / 8,191 rows 18.5 / 21.1 / 29.1 / 34.6 against the library's 19.8 / 21.0 /
+        25.2 / 39.7; unrounded 2,752 x 896 at 2,048 / 2,535 / 3,500 / 5,000 / 8,191 19.5 / 20.1 / 25.0 / 31.0 / 50.3 against 18.7 / 28.4 / 27.1 / 49.5 /
+        77.8, 1,152 x 896 at 2,535 / 5,000 / 8,191 13.6 / 19.8 / 25.4 against 11.9 / 15.9 / 27.3.  3,072 x 1,024 at 8,191 67.6 against 53.2."""
+        return k <= 896 and (m >= 6000 or (m >= 2304 and n >= 2 * k) or (m <= 2600 and n <= k))
 
     @staticmethod
     def _own_gate(m: int, k: int) -> bool:
@@ -686,7 +689,7 @@ class HipKernels(KernelBackend):
         self._need(w, "w", _BF16, (2 * inter, k))
         out = torch.empty((t, inter), dtype=_BF16, device=x.device)
         self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), t, inter, k, 1, 2, _GATES[activation],
-                  self._rows_plan(t, 2 * inter, k, 1)[0], self._stream())
+                  self._rows_plan(t, 2 * inter, k, 1, 2)[0], self._stream())
         return out
 
     def combine_attention(self, part_o, part_ml, out):
@@ -721,11 +724,11 @@ class HipKernels(KernelBackend):
             self._run("egpt_gemm_skinny", x.data_ptr(), w.data_ptr(), None, self._ptr(out), None, self._ptr(target),
                       m, n, k, s, 4, self._stream())
             return out if target is None else target
-        if m > 64 and self._rows_fit(x, w, k) and (self._own_rows(m, n, k, unrounded) or self._own_short(n, k)):
+        if m > 64 and self._rows_fit(x, w, k) and (self._own_rows(m, n, k, unrounded) or self._own_short(m, n, k)):
             # many rows on the framework's own kernel: rounded, or float32 partial sums where the k range is split
             self._need(x, "x")
             self._need(w, "w", x.dtype, (n, k))
-            shape, s = self._rows_plan(m, n, k, 1 if unrounded else 10)
+            shape, s = self._rows_plan(m, n, k, 1 if unrounded else 10, 1 if unrounded else 0)
             kind = 1 if unrounded or s > 1 else 0
             out = torch.empty((s, m, n) if kind else (m, n), dtype=_F32 if kind else _BF16, device=x.device)
             self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, kind, 0, shape, self._stream())

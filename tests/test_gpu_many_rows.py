@@ -26,7 +26,7 @@ def run(k, x, w, shape, splits, kind, act=0):
     return out
 
 
-@pytest.mark.parametrize("shape", range(5))
+@pytest.mark.parametrize("shape", range(7))
 @pytest.mark.parametrize("m,n,kk,splits", [(1, 4, 64, 1), (63, 60, 64, 1), (65, 68, 128, 2), (127, 260, 192, 3), (193, 132, 320, 2),
                                            (257, 516, 448, 4), (300, 1152, 896, 1)])
 def test_every_tile_at_its_edges(k, shape, m, n, kk, splits):
@@ -40,7 +40,7 @@ def test_every_tile_at_its_edges(k, shape, m, n, kk, splits):
     assert ((rounded - want).abs() <= bound + want.abs() * 2.0 ** -8).all()
 
 
-@pytest.mark.parametrize("shape", range(5))
+@pytest.mark.parametrize("shape", range(7))
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("m,n,kk", [(2, 4, 64), (65, 36, 128), (130, 260, 192)])
 def test_the_activated_form(k, shape, act, m, n, kk):
@@ -144,12 +144,12 @@ def test_rows_grouped_by_expert(k, tile_rows, t, top, experts, outputs, hidden, 
             assert ((y[r].double().cpu() - full).abs() <= 1e-5 * (d64[e].abs() @ act[r].double().cpu().abs()) + 1e-6).all()
 
 
-@pytest.mark.parametrize("shape", range(5))
+@pytest.mark.parametrize("shape", range(7))
 @pytest.mark.parametrize("kk,splits", [(128, 1), (192, 1), (256, 1), (384, 2), (448, 2)])
 def test_a_workgroup_takes_several_tiles_in_turn(k, shape, kk, splits):
     # more tiles than the CUs hold workgroups, with edges in both directions; two steps (a workgroup per tile), three (all of a
     # tile's loads under the tile before), four, and split ranges of three and of four and three steps
-    m, n = ((2049, 9004), (2049, 9004), (2049, 9004), (2300, 4100), (2300, 2052))[shape]
+    m, n = ((2049, 9004), (2049, 9004), (2049, 9004), (2300, 4100), (2300, 2052), (2300, 2052), (2300, 4100))[shape]
     x, w = rnd(m, kk, seed=9), rnd(n, kk, seed=10)
     want = x.double() @ w.double().t()
     bound = (x.double().abs() @ w.double().abs().t()) * kk * 2.0 ** -24
