@@ -54,7 +54,7 @@ def _library():
         from ..csrc import build
 
         lib = ctypes.CDLL(build.ensure_host_built())
-        if lib.egh_abi_version() != 4:
+        if lib.egh_abi_version() != 5:
             raise RuntimeError("the host library has an unexpected ABI version")
         vp, i = ctypes.c_void_p, ctypes.c_int
         sigs = {
@@ -67,6 +67,7 @@ def _library():
             "egh_slot_index": ([vp, i, i, i], i), "egh_check": ([vp, vp, i], i),
             "egh_fill_decode": ([vp, i, vp, vp, vp, vp, vp], i),
             "egh_fill_decode_rows": ([vp, i, i, vp, vp, vp, vp, vp], i),
+            "egh_uniforms": ([i, vp, vp, vp, vp], None),
             "egh_fill_step": ([vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp], i),
         }
         for name, (args, res) in sigs.items():

@@ -27,8 +27,8 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-ta
          "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-Wno-pass-failed"]
 
 
-HOST_SOURCES = ["host/cache_core.cpp"]
-HOST_HEADERS = ["host/cache_core.h"]
+HOST_SOURCES = ["host/cache_core.cpp", "host/draws.cpp"]
+HOST_HEADERS = ["host/cache_core.h", "host/draws.h"]
 HOST_LIB_NAME = "libeasygpt_host.so"
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra"]
 

@@ -626,4 +626,4 @@ extern "C" const char* egpt_error_string(int code) {
     }
 }
 
-extern "C" int egpt_abi_version(void) { return 27; }
+extern "C" int egpt_abi_version(void) { return 28; }

@@ -67,7 +67,7 @@ struct EghCore {
 
 extern "C" {
 
-int egh_abi_version(void) { return 4; }
+int egh_abi_version(void) { return 5; }
 
 EghCore* egh_create(int n_groups, const int32_t* windows, const int32_t* num_pages, int page_size, int max_requests) {
     if (n_groups < 0 || page_size < 1 || max_requests < 0 || (n_groups > 0 && (!windows || !num_pages))) return nullptr;

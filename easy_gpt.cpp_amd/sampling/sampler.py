@@ -12,6 +12,7 @@ function of (seed, request serial, n) alone, so batching changes nothing.
 """
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass
 
 import torch
@@ -53,6 +54,16 @@ def uniform_for(seed: int, serial: int, n: int) -> float:
     """A number in [0, 1) for the n-th token of request `serial` under `seed`."""
     z = _mix(_mix(_mix(seed) ^ serial) ^ n)
     return (z >> 40) / float(1 << 24)
+
+
+def fill_uniforms(params, serials, counts, out) -> None:
+    """`uniform_for` of every row into the float32 array `out`, by the host library (64 rows: 79 us in Python, 15 so)."""
+    from ..cache.manager import _library
+
+    # (what is beyond 64 bits does not matter: the mixing is modulo 2^64)
+    seeds, serials, counts = (array("Q", v) for v in ([p.seed & _MASK for p in params], [s & _MASK for s in serials],
+                                                      [n & _MASK for n in counts]))
+    _library().egh_uniforms(len(params), *(a.buffer_info()[0] for a in (seeds, serials, counts)), out.ctypes.data)
 
 
 class PendingTokens:
@@ -107,7 +118,7 @@ class Sampler:
             rows = host.numpy()
             rows[0] = [0.0 if p.greedy else p.temperature for p in params]
             rows[1] = [p.top_p for p in params]
-            rows[2] = [uniform_for(p.seed, s, n) for p, s, n in zip(params, serials, counts)]
+            fill_uniforms(params, serials, counts, rows[2])
             rows[3].view("int32")[:] = [p.top_k for p in params]
             dev = host.to(logits.device, non_blocking=pinned)
             k.sample(logits, dev[0], dev[3].view(torch.int32), dev[1], dev[2], out)

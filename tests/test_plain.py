@@ -240,3 +240,17 @@ def test_sampling_distribution():
     kept = (d > 0)
     assert float(p[kept].sum()) >= 0.6 and float(p[kept].sum() - p[kept].min()) < 0.6      # smallest such set
     assert plain.greedy(torch.tensor([1.0, 3.0, 3.0, 2.0])) == 1                             # first maximum wins
+
+
+def test_uniform_numbers_of_a_batch_are_those_of_its_rows():
+    import numpy as np
+
+    from easy_gpt.cpp_amd.sampling.sampler import SamplingParams, fill_uniforms, uniform_for
+
+    seeds = [0, 1, 42, (1 << 63) + 5, (1 << 64) - 1, (1 << 64) + 7, 10**30]
+    serials, counts = [0, 5, (1 << 40) + 1, 3, (1 << 64) - 1, -2, 8], [0, 1, 2, 1 << 33, 70, 5, 9]
+    rows = np.full((4, len(seeds)), -1.0, dtype=np.float32)
+    fill_uniforms([SamplingParams(seed=s) for s in seeds], serials, counts, rows[2])
+    assert rows[2].tolist() == [uniform_for(*r) for r in zip(seeds, serials, counts)]
+    assert (rows[[0, 1, 3]] == -1.0).all()
+    fill_uniforms([], [], [], rows[0][:0])
