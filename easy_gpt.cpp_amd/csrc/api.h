@@ -43,9 +43,9 @@ int egpt_rope_table(const int32_t* positions, const float* inv_freq, float* cos_
 // part of the product into acc_fixed [m][n], a residual stream in fixed point, with integer atomics.
 int egpt_gemm_skinny(const void* x, const void* w, const void* bias, float* out_f32, void* out_bf16, void* acc_fixed,
                      int m, int n, int k, int n_splits, int waves, void* stream);
-// bfloat16 product for more than 64 rows on the matrix cores (see gemm_rows.hip): kind 0 writes out bfloat16 [m][n], 1 float32
+// bfloat16 product for more than 16 rows on the matrix cores (see gemm_rows.hip): kind 0 writes out bfloat16 [m][n], 1 float32
 // partial sums [n_splits][m][n], 2 bfloat16 [m][n] = act(x gate^T) * (x up^T) for w = [gate; up] ([2 n][k]; act as in
-// egpt_swiglu).  shape: the tile (0 to 4).  k % 64 == 0, n % 4 == 0, operands on 16 bytes.
+// egpt_swiglu).  shape: the tile (0 to 6).  k % 64 == 0, n % 4 == 0, operands on 16 bytes.
 int egpt_gemm_rows(const void* x, const void* w, void* out, int m, int n, int k, int n_splits, int kind, int act, int shape,
                    void* stream);
 // float32 product on the matrix cores (float32 operands as three bfloat16 numbers each, float32 accumulation, see gemm.hip):

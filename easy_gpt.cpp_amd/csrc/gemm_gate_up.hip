@@ -9,7 +9,8 @@
 // all rows of x straight into matrix-core operands (x comes from L2, where every workgroup finds it), with all
 // loads of up to KC chunks of 32 in flight before the first product.  The four partial results meet in LDS, are
 // added in wavefront order, and leave as activated bfloat16: neither the float32 product nor a SwiGLU kernel
-// of its own stands between the norm and the down product.
+// of its own stands between the norm and the down product.  gemm_rows.hip is faster for more than 32 rows and for more
+// than 2,048 columns; this one stays for what is smaller and for operands that that one does not take.
 #include "api.h"
 #include "common.h"
 

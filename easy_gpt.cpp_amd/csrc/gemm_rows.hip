@@ -1,4 +1,4 @@
-// out[m, n] = sum_k x[m, k] * w[n, k] in bfloat16 for many rows of x (more than 64): tiles staged through LDS by loads that
+// out[m, n] = sum_k x[m, k] * w[n, k] in bfloat16 for many rows of x (more than 16): tiles staged through LDS by loads that
 // go there directly, v_mfma_f32_16x16x32_bf16, float32 accumulation.  The result leaves as bfloat16, as float32 partial
 // sums of a split k range, or activated: w = [gate; up] and out = act(x gate^T) * (x up^T), both factors still in float32.
 //
@@ -12,6 +12,9 @@
 //
 // Tiles of few rows and columns keep five or six steps of both operands on their way where there are few of them: a step of 64 x 64
 // takes 0.17 us so and 0.32 with two and three, which is the L2's latency (600 x 896 x 4,864 in one range 30.4 us -> 19.1).
+// With 17 to 64 rows the deep rings are what streams the weights: one workgroup to a CU, at 64 rows 1,536 x 8,960 and the norm behind it in
+// 14.7 us (20.4 by the weight-streaming kernel of gemm_skinny.hip, which holds one step of w in registers), 152,064 x 3,584 in 217,
+// 5.0 TB/s; `_few_plan` in kernels/hip.py chooses the shape.
 // A workgroup stays for several tiles: as many are launched as the CUs hold, and the loads of a workgroup's next tile go out under
 // the last steps of the one before, so that a tile's first products do not wait for memory and the result leaves meanwhile.
 //

@@ -272,7 +272,8 @@ class HipKernels(KernelBackend):
         """Whether a bfloat16 product of m rows goes to the library (the reference uses cuBLAS for every linear
         layer).  Up to 16 rows never, beyond 64 always.  Between them the own kernels win where the k range
         has to be split over workgroups (an output narrower than k) and on small matrices, where a step is a
-        chain of round trips to memory; the library wins on large ones, which it streams at 4 to 5 TB/s."""
+        chain of round trips to memory; the library wins on large ones, which it streams at 4 to 5 TB/s.  (`product` and an
+        output matrix take gemm_rows.hip before either, at 17 to 64 rows, where it takes the operands; what is measured here is for the others.)"""
         if m <= 16:
             return False
         if m > 64:
@@ -326,6 +327,22 @@ class HipKernels(KernelBackend):
                 if best is None or us < best[0]:
                     best = us, shape, s
         return best[1], best[2]
+
+    @staticmethod
+    def _few_plan(n: int, k: int, most_splits: int) -> tuple[int, int]:
+        """(shape, splits of the k range) of gemm_rows.hip for 17 to 64 rows, one tile of rows: the weights' way from memory is what
+        counts, so every CU gets one workgroup.  An output of fewer than 256 tiles of 64 columns has its k range split until there are as
+        many, in ranges of two steps or more; ranges of up to 8 steps are on their way at once and a workgroup with the smaller ring begins
+        sooner, longer ones keep five steps in flight.  An output of more tiles goes by 128 columns with six steps in flight, one of more
+        than 512 by 64 again, four workgroups to a CU.  Over 27 matrices of 512 x 512 to 3,584 x 18,944 at 17, 32, 48 and 64 rows this is 0.3 % off the
+        best of all shapes and splits (at most 5 %); 192 workgroups in the place of 256 are 4 % off, 320 10 %, 512 8 %."""
+        tiles = -(-n // 64)
+        steps = k // 64
+        per = -(-steps // max(1, min(256 // tiles, steps // 2, most_splits)))
+        splits = -(-steps // per)
+        if splits * tiles <= 256:
+            return (4 if per <= 8 else 5), splits
+        return (6 if tiles <= 512 else 4), splits
 
     @staticmethod
     def _rows_fit(x, w, k: int) -> bool:
@@ -415,6 +432,15 @@ class HipKernels(KernelBackend):
             return out
         if x.dtype == _BF16 and k % 8 == 0:
             to_f32 = out.dtype == _F32
+            if to_f32 and bias is None and 16 < m <= 64 and n >= 65536 and self._rows_fit(x, w, k):
+                # An output matrix over a whole vocabulary: tiles of 64 x 128 with six steps on their way (us, weights from memory, at
+                # 17 / 32 / 48 / 64 rows, against the weight-streaming kernel up to 32 and the library beyond): 151,936 x 896 56 / 58 / 62 / 67
+                # against 62 / 68 / 76 / 74, 151,936 x 1,536 91 / 97 / 105 / 110 against 103 / 107 / 123 / 118, 102,400 x 2,048 101 / 105 / 108 / 114 against
+                # 104 / 108 / 108 / 122, 152,064 x 3,584 200 / 204 / 208 / 217 against 223 / 233 / 209 / 217, 128,256 x 4,096 194 / 200 / 200 / 204 against 231 /
+                # 239 / 219 / 219.  A smaller vocabulary gains nothing (50,304 x 1,024 24.5 to 27.5 against 23.6 to 25.7), nor do more rows
+                # with a long k (152,064 x 3,584 at 96 rows 239 with tiles of 128 x 128 against 231).
+                self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, 1, 1, 0, 6, self._stream())
+                return out
             if not self._library_rows(m, n, k):
                 # weight-streaming MFMA kernel
                 self._run("egpt_gemm_skinny", x.data_ptr(), w.data_ptr(), self._ptr(bias),
@@ -664,14 +690,27 @@ class HipKernels(KernelBackend):
         if x.dtype != _BF16 or w.dtype != _BF16 or not self.fused_rows < t <= 64 or k % 8 or w.shape[0] % 2:
             return None
         inter = w.shape[0] // 2
+        if groups is None and (t > 32 or inter > 2048) and self._rows_fit(x, w, k):
+            # the kernel for many rows, whose loads are six steps ahead (us, weights from memory, at 17 / 32 / 64 rows, against the kernel below
+            # or the library and SwiGLU): 4,864 x 896 8.0 / 7.8 / 8.5 against 10.3 / 10.6 / 12.9, 8,960 x 1,536 16.7 / 17.3 / 18.8 against 18.6 / 18.8 / 21.2,
+            # 11,008 x 2,048 23.6 / 23.9 / 24.6 against 27.6 / 25.9 / 27.4, 18,944 x 3,584 50.9 / 53.2 / 61.3 against 59.5 / 58.1 / 64.7, 3,072 x 1,024 7.5 /
+            # 7.7 / 8.5 against 7.6 / 8.0 / 10.2.  A small matrix and up to 32 rows: 768 x 896 6.8 / 6.9 / 7.0 against 5.7 / 6.3 / 8.2, 2,048 x 1,024 7.3 /
+            # 7.4 / 7.5 against 6.3 / 6.9 / 9.1, 1,024 x 2,048 10.3 / 10.4 / 10.5 against 9.6 / 10.8 / 15.0.
+            self._need(x, "x", _BF16)
+            self._need(w, "w", _BF16, (2 * inter, k))
+            out = torch.empty((t, inter), dtype=_BF16, device=x.device)
+            self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), t, inter, k, 1, 2, _GATES[activation],
+                      self._few_plan(2 * inter, k, 1)[0], self._stream())
+            return out
         if groups is None:
             if 2 * inter * k >= 16 << 20:
                 # every workgroup reads all of x from L2, which on a large matrix costs more than the float32 product
                 # and the SwiGLU kernel that this saves (measured at 64 rows: 12.8 us against 14.5 on 9,728 x 896,
                 # 37 against 21 on 17,920 x 1,536)
                 return None
-            # two column groups per workgroup halve the reads of x; on small matrices one gives more workgroups
-            groups = 2 if inter * k >= 1 << 20 else 1
+            # two column groups per workgroup halve the reads of x; on small matrices one gives more workgroups (2,048 x 1,024 at
+            # 17 and 32 rows 6.3 and 6.9 us against 8.3 and 8.9 with two)
+            groups = 2 if inter > 2048 and inter * k >= 1 << 20 else 1
         self._need(x, "x", _BF16)
         self._need(w, "w", _BF16, (2 * inter, k))
         out = torch.empty((t, inter), dtype=_BF16, device=x.device)
@@ -710,6 +749,21 @@ class HipKernels(KernelBackend):
         in fixed point [m, n], a product of few rows is added into it instead and the stream is returned."""
         m, k = x.shape
         n = w.shape[0]
+        if 16 < m <= 64 and self._rows_fit(x, w, k):
+            # A few dozen rows: the kernel for many, whose workgroups keep more of the weights on their way than the weight-streaming one and
+            # split the k range, which the library does not.  us, weights from memory, at 17 / 32 / 64 rows, with the norm that reads the
+            # result: 896 x 4,864 9.2 / 9.5 / 10.4 against 9.9 / 10.7 / 12.9, 1,536 x 8,960 13.3 / 13.6 / 14.7 against 17.3 / 18.1 / 20.4, 3,584 x 18,944
+            # 32.2 / 33.3 / 37.3 against 43.4 / 43.3 / 50.2, 896 x 896 7.7 / 7.9 / 8.5 against 7.7 / 8.3 / 10.3; by itself 1,152 x 896 3.8 / 4.0 / 4.3
+            # against 3.8 / 4.3 / 5.9, 4,608 x 3,584 9.3 / 9.6 / 10.7 against 13.4 / 15.2 / 18.5.  What rotates queries and keys reads 8 parts at a
+            # time, what adds to the residual stream any number: no more than that of either.
+            self._need(x, "x")
+            self._need(w, "w", x.dtype, (n, k))
+            shape, s = self._few_plan(n, k, 8 if unrounded else 16)
+            # (one piece is rounded where it always was, so that a reader sees what it saw)
+            kind = 0 if s == 1 and not unrounded and self._library_rows(m, n, k) else 1
+            out = torch.empty((s, m, n) if kind else (m, n), dtype=_F32 if kind else _BF16, device=x.device)
+            self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, kind, 0, shape, self._stream())
+            return out
         if x.dtype == _BF16 and m > 0 and k % 8 == 0 and not self._library_rows(m, n, k):
             self._need(x, "x")
             self._need(w, "w", x.dtype, (n, k))

@@ -122,3 +122,12 @@ def test_the_rules_for_many_rows_change_sides_once():
     for k in WIDTHS + [3072, 4096, 5120, 8192]:
         own = [K._own_gate(m, k) for m in rows]
         assert sum(a != b for a, b in zip(own, own[1:])) <= 2, k
+
+
+def test_few_row_plans_are_launchable():
+    # what egpt_gemm_rows refuses: an empty range, or splits of a result that is not float32
+    for n, k, most in itertools.product(WIDTHS + [8, 16384, 16392, 32776], [w for w in WIDTHS if w % 64 == 0], (1, 8, 16)):
+        shape, s = K._few_plan(n, k, most)
+        steps = k // 64
+        assert 4 <= shape <= 6 and 1 <= s <= most and (s - 1) * -(-steps // s) < steps, (n, k, most)
+        assert s == 1 or (s * -(-n // 64) <= 256 and -(-steps // s) >= 2), (n, k, most)
