@@ -73,10 +73,10 @@ __global__ __launch_bounds__(256) void bounded_gate_kernel(ProductView<T> z, int
     gate[idx] = low + (1.0f - low) * (1.0f / (1.0f + expf(-v)));
 }
 
-constexpr int kScanTokens = 32;     // tokens staged in LDS at a time
+constexpr int kScanTokens = 16;     // tokens staged in LDS at a time
 constexpr int kScanCols = 64;       // value channels per workgroup: a lane is a column of the state
 constexpr int kScanKeys = 16;       // key channels per workgroup
-constexpr int kScanWaves = 4;       // wavefronts per workgroup, kScanKeys / kScanWaves key channels each
+constexpr int kScanWaves = 4;       // wavefronts that walk the tokens, kScanKeys / kScanWaves key channels each; as many beside them
 
 // The value of lane N of each row of 16 lanes.
 template <int N>
@@ -97,24 +97,63 @@ __device__ __forceinline__ void scan_token(float a, float k, float q, float v, f
     *part = fmaf(row_value<N + 1>(q), s[1], row_value<N>(q) * s[0]) + fmaf(row_value<N + 3>(q), s[3], row_value<N + 2>(q) * s[2]);
 }
 
+// Four tokens, as scan_token<0>, <4>, <8> and <12> compute them (the same operations, the same bits), 13 instructions a token
+// where the compiler takes 20: it moves a row's value to a register of its own before every addition that uses it.  An
+// instruction reads a row's values two cycles of issue after they were written at the earliest, hence the wait in front (what
+// the block itself writes it reads as plain operands only).
+#define EGPT_SCAN_TOKEN(A, B, C, D, V, P, S0, S1, S2, S3, T0, T1, T2, T3)                  \
+    "v_mul_f32_dpp " T0 ", %[k], " V " row_newbcast:" A " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_mul_f32_dpp " T1 ", %[k], " V " row_newbcast:" B " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_mul_f32_dpp " T2 ", %[k], " V " row_newbcast:" C " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_mul_f32_dpp " T3 ", %[k], " V " row_newbcast:" D " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_fmac_f32_dpp " T0 ", %[a], " S0 " row_newbcast:" A " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_fmac_f32_dpp " T2 ", %[a], " S2 " row_newbcast:" C " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_fmac_f32_dpp " T1 ", %[a], " S1 " row_newbcast:" B " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_fmac_f32_dpp " T3 ", %[a], " S3 " row_newbcast:" D " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_mul_f32_dpp " P ", %[q], " T0 " row_newbcast:" A " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_mul_f32_dpp " S0 ", %[q], " T2 " row_newbcast:" C " row_mask:0xf bank_mask:0xf\n\t"     \
+    "v_fmac_f32_dpp " P ", %[q], " T1 " row_newbcast:" B " row_mask:0xf bank_mask:0xf\n\t"     \
+    "v_fmac_f32_dpp " S0 ", %[q], " T3 " row_newbcast:" D " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_add_f32 " P ", " P ", " S0 "\n\t"
+__device__ __forceinline__ void scan_four_tokens(float a, float k, float q, const float* v, float* s, float* part) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float t0, t1, t2, t3, p0, p1, p2, p3;
+    asm("s_nop 1\n\t"
+        EGPT_SCAN_TOKEN("0", "1", "2", "3", "%[v0]", "%[p0]", "%[s0]", "%[s1]", "%[s2]", "%[s3]", "%[t0]", "%[t1]", "%[t2]", "%[t3]")
+        EGPT_SCAN_TOKEN("4", "5", "6", "7", "%[v1]", "%[p1]", "%[t0]", "%[t1]", "%[t2]", "%[t3]", "%[s0]", "%[s1]", "%[s2]", "%[s3]")
+        EGPT_SCAN_TOKEN("8", "9", "10", "11", "%[v2]", "%[p2]", "%[s0]", "%[s1]", "%[s2]", "%[s3]", "%[t0]", "%[t1]", "%[t2]", "%[t3]")
+        EGPT_SCAN_TOKEN("12", "13", "14", "15", "%[v3]", "%[p3]", "%[t0]", "%[t1]", "%[t2]", "%[t3]", "%[s0]", "%[s1]", "%[s2]", "%[s3]")
+        : [s0] "+&v"(s[0]), [s1] "+&v"(s[1]), [s2] "+&v"(s[2]), [s3] "+&v"(s[3]), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2),
+          [t3] "=&v"(t3), [p0] "=&v"(p0), [p1] "=&v"(p1), [p2] "=&v"(p2), [p3] "=&v"(p3)
+        : [a] "v"(a), [k] "v"(k), [q] "v"(q), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]));
+    part[0] = p0, part[kScanCols] = p1, part[2 * kScanCols] = p2, part[3 * kScanCols] = p3;
+#endif
+}
+#undef EGPT_SCAN_TOKEN
+
 // The recurrence has no term that mixes two key channels but the sum o_t = sum_r S[r][:] q[r], so the key channels are
-// dealt over workgroups: one workgroup of four wavefronts per (request, head, 64 value channels, 16 key channels), whose
+// dealt over workgroups: one workgroup per (request, head, 64 value channels, 16 key channels), whose
 // part of o_t goes to out[split] (float32 [splits][tokens][heads * dv]) for the consumer to add in the order of the
-// splits.  A lane is one column of the state; wavefront w keeps four of the workgroup's key channels of that column in
-// registers.  The queries, keys and decays that a wavefront needs are the same for all its lanes: one LDS read brings those of
+// splits.  A lane is one column of the state; wavefront w of the first four keeps four of the workgroup's key channels of that
+// column in registers.  The queries, keys and decays that a wavefront needs are the same for all its lanes: one LDS read brings those of
 // four tokens, 16 values that every row of 16 lanes has, and an instruction takes its one of them out of the row (row_newbcast).
-// The wavefronts' parts go through LDS and are added in the order of the wavefronts, a batch of kScanTokens tokens at a time;
-// the batch's operands are staged in LDS, the next batch's loads in flight in registers meanwhile.
+// The wavefronts' parts go through LDS and are added in the order of the wavefronts, a batch of kScanTokens tokens at a time.
+//
+// What bounds it is the walk: one request's tokens one after the other.  So the first four wavefronts do nothing else, and four
+// more, one beside each on its SIMD, bring the operands of the batches to come (two batches' loads in flight in registers, the
+// next batch in LDS) and add and store the parts of the batch before, with one barrier per batch.
+// 7 heads of 64 x 128, 2,535 tokens in three requests, the longest of 1,357: 116 us with the same four wavefronts for both, 73 so, 62
+// with the walk's instructions written out (`scan_four_tokens`): 46 ns a token, of which 52 issues of four cycles are 22; the rest is the
+// trip to LDS at the beginning of a batch and the wavefront beside.  (Loads with the batch's first row as a scalar, which take the wavefront
+// beside a third of its instructions, changed nothing: 75 for the 73.)
 // FORM says what the product is: 0 whole, in T; 1 one float32 array; 2 partial sums to be added up.  In the first two a batch's
 // loads are plain ones without a branch around them (places beyond the tokens or channels load a neighbour and count as zero),
-// so all of them are on their way together while the batch before is worked on; with one body for all forms a load waited for
-// the one before.  7 heads of 64 x 128, 2,535 tokens in three requests, the longest of 1,357: 172 us with that body, 118 now, of
-// which half are the instructions of the recurrence, 20 a token on a wavefront that has its SIMD to itself.  Partial sums and
+// so all of them are on their way together; so are its stores (places without a token or column go nowhere), because a wait for a
+// load beside memory operations that a branch may skip waits for those as well.  Partial sums and
 // rotated operands take several loads each, which do wait for one another, so there a thread whose place holds no token or
-// channel loads nothing.  (64 decoded tokens of 7 heads out of four partial sums: 22.8 us, 42.9 with loads for every place;
-// rotated 29.4 and 60.1.)
+// channel loads nothing.
 template <typename T, bool ROTATED, int FORM>
-__global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
+__global__ __launch_bounds__(128 * kScanWaves) void decayed_state_scan_kernel(
     ProductView<T> proj, int proj_width, int q_off, int k_off, int v_off, float q_scale, const float* __restrict__ decay,
     float* __restrict__ states, const int32_t* __restrict__ slots, const unsigned char* __restrict__ fresh,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, float* __restrict__ out, int n_tokens, int heads,
@@ -123,33 +162,85 @@ __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
     constexpr int NS = kScanWaves, DKR = kScanKeys / kScanWaves, THREADS = 64 * NS, DKP = kScanKeys;
     constexpr int QKA = kScanTokens * DKP / THREADS;          // values of q (or k, or decays) of a batch per thread
     constexpr int VL = kScanTokens * kScanCols / THREADS;     // values of v, and outputs, of a batch per thread
-    static_assert(DKR == 4 && QKA * THREADS == kScanTokens * DKP && VL * THREADS == kScanTokens * kScanCols, "a batch divides evenly");
-    __shared__ __attribute__((aligned(16))) float q_s[kScanTokens * DKP];
-    __shared__ __attribute__((aligned(16))) float k_s[kScanTokens * DKP];
-    __shared__ __attribute__((aligned(16))) float a_s[kScanTokens * DKP];
-    __shared__ float v_s[kScanTokens * kScanCols];
-    __shared__ float part_s[kScanTokens * NS * kScanCols];
+    static_assert(DKR == 4 && kScanCols == kWave && QKA * THREADS == kScanTokens * DKP && VL * THREADS == kScanTokens * kScanCols, "a batch divides evenly");
+    constexpr int kPartWave = kScanTokens * kScanCols;
+    __shared__ __attribute__((aligned(16))) float q_s[2][kScanTokens * DKP];
+    __shared__ __attribute__((aligned(16))) float k_s[2][kScanTokens * DKP];
+    __shared__ __attribute__((aligned(16))) float a_s[2][kScanTokens * DKP];
+    __shared__ float v_s[2][kScanTokens * kScanCols];
+    __shared__ float part_s[2][NS * kPartWave];
     const int b = blockIdx.x, h = blockIdx.y;
     const int split = blockIdx.z % key_splits, col0 = (blockIdx.z / key_splits) * kScanCols, key0 = split * kScanKeys;
     const int n = q_len[b];
     if (n <= 0) return;
     const int t0 = q_start[b];
-    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    const int j = col0 + lane;
-    const bool has_col = j < dv;
-    float* state = states + (static_cast<size_t>(slots[b]) * heads + h) * dk * dv;
-    float* o_split = out + static_cast<size_t>(split) * n_tokens * heads * dv;
-    float s[DKR];
-    const bool start_anew = fresh != nullptr && fresh[b] != 0;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int batches = (n + kScanTokens - 1) / kScanTokens, iterations = (batches + 2) / 2 * 2;
+    if (wave < NS) {
+        // ---- the walk
+        const int j = col0 + lane;
+        const bool has_col = j < dv;
+        float* state = states + (static_cast<size_t>(slots[b]) * heads + h) * dk * dv;
+        float s[DKR];
+        const bool start_anew = fresh != nullptr && fresh[b] != 0;
 #pragma unroll
-    for (int i = 0; i < DKR; ++i) {
-        const int r = key0 + wave * DKR + i;
-        s[i] = (!start_anew && has_col && r < dk) ? state[static_cast<size_t>(r) * dv + j] : 0.f;
+        for (int i = 0; i < DKR; ++i) {
+            const int r = key0 + wave * DKR + i;
+            s[i] = (!start_anew && has_col && r < dk) ? state[static_cast<size_t>(r) * dv + j] : 0.f;
+        }
+        const int place = lane % 16 / 4 * DKP + wave * DKR + lane % 4;   // this lane's value of a group: token lane % 16 / 4, key lane % 4
+        auto walk = [&](int batch, int buffer) {
+            auto group = [&](int tt, int tokens) __attribute__((always_inline)) {
+                const float a = a_s[buffer][tt * DKP + place], k = k_s[buffer][tt * DKP + place], q = q_s[buffer][tt * DKP + place];
+                float vj[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) vj[u] = v_s[buffer][(tt + u) * kScanCols + lane];
+                float* part = part_s[buffer] + wave * kPartWave + tt * kScanCols + lane;
+                if (tokens == 4) return scan_four_tokens(a, k, q, vj, s, part);
+                scan_token<0>(a, k, q, vj[0], s, part);
+                if (tokens > 1) scan_token<4>(a, k, q, vj[1], s, part + kScanCols);
+                if (tokens > 2) scan_token<8>(a, k, q, vj[2], s, part + 2 * kScanCols);
+            };
+            // four tokens at a time; the last tokens of a portion, fewer than four, by the same operations
+            const int count = min(kScanTokens, n - batch * kScanTokens);
+            if (count == kScanTokens) {
+#pragma unroll
+                for (int tt = 0; tt < kScanTokens; tt += 4) group(tt, 4);
+            } else {
+                int tt = 0;
+                for (; tt + 4 <= count; tt += 4) group(tt, 4);
+                if (tt < count) group(tt, count - tt);
+            }
+        };
+        __syncthreads();                                   // the first batch is in LDS
+        if (batches == 1) {
+            walk(0, 0);
+            __syncthreads();
+        } else {
+            for (int i = 0; i < iterations; i += 2) {
+                if (i < batches) walk(i, 0);
+                __syncthreads();
+                if (i + 1 < batches) walk(i + 1, 1);
+                __syncthreads();
+            }
+        }
+        if (has_col) {
+#pragma unroll
+            for (int i = 0; i < DKR; ++i) {
+                const int r = key0 + wave * DKR + i;
+                if (r < dk) state[static_cast<size_t>(r) * dv + j] = s[i];
+            }
+        }
+        return;
     }
+    // ---- operands and results
+    const int tid = (wave - NS) * kWave + lane;
     const int channels = heads * dk;
     constexpr bool kPlain = !ROTATED && FORM != 2;            // every load is one plain load
-    std::conditional_t<FORM == 0, T, float> rq[QKA], rk[QKA], rv[VL];
-    float ra[QKA];
+    struct Loaded {
+        std::conditional_t<FORM == 0, T, float> q[QKA], k[QKA], v[VL];
+        float a[QKA];
+    };
     auto load = [&](size_t at) {
         if constexpr (FORM == 0) return proj.whole[at];
         else if constexpr (FORM == 1) return proj.partial[at];
@@ -171,117 +262,94 @@ __global__ __launch_bounds__(64 * kScanWaves) void decayed_state_scan_kernel(
         return first ? __fmaf_rn(own, c, -__fmul_rn(other, s)) : __fmaf_rn(other, s, __fmul_rn(own, c));
     };
     const float* decays = head_decay ? head_decay : decay;
-    auto fetch = [&](int base) {
-        const int last = min(kScanTokens, n - base) - 1;
+    auto fetch = [&](int batch, Loaded& to) {
+        const int base = batch * kScanTokens;
 #pragma unroll
         for (int u = 0; u < QKA; ++u) {
             const int idx = tid + u * THREADS, in_head = key0 + idx % DKP, r = kPlain ? min(in_head, dk - 1) : in_head;
-            const int tt = kPlain ? min(idx / DKP, last) : idx / DKP;
+            const int tt = kPlain ? min(base + idx / DKP, n - 1) : base + idx / DKP;
             if constexpr (!kPlain) {
-                rq[u] = rk[u] = ra[u] = 0.f;
-                if (tt > last || r >= dk) continue;
+                to.q[u] = to.k[u] = to.a[u] = 0.f;
+                if (tt >= n || r >= dk) continue;
             }
-            const size_t row = static_cast<size_t>(t0 + base + tt), q_at = row * proj_width + q_off + h * dk;
+            const size_t row = static_cast<size_t>(t0 + tt), q_at = row * proj_width + q_off + h * dk;
             const size_t k_at = tied_keys ? q_at : row * proj_width + k_off + h * dk;
             if constexpr (kPlain) {
-                rq[u] = load(q_at + r);
-                rk[u] = load(k_at + r);                            // (of a tied key nothing is used)
+                to.q[u] = load(q_at + r);
+                to.k[u] = load(k_at + r);                          // (of a tied key nothing is used)
             } else {
-                rq[u] = turned(row, q_at, r);
-                if (!tied_keys) rk[u] = turned(row, k_at, r);
+                to.q[u] = turned(row, q_at, r);
+                if (!tied_keys) to.k[u] = turned(row, k_at, r);
             }
-            ra[u] = decays[head_decay ? static_cast<size_t>(h) : row * channels + h * dk + r];
+            to.a[u] = decays[head_decay ? static_cast<size_t>(h) : row * channels + h * dk + r];
         }
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
             const int idx = tid + u * THREADS, in_head = col0 + idx % kScanCols, c = kPlain ? min(in_head, dv - 1) : in_head;
-            const int tt = kPlain ? min(idx / kScanCols, last) : idx / kScanCols;
+            const int tt = kPlain ? min(base + idx / kScanCols, n - 1) : base + idx / kScanCols;
             if constexpr (!kPlain) {
-                rv[u] = 0.f;
-                if (tt > last || c >= dv) continue;
+                to.v[u] = 0.f;
+                if (tt >= n || c >= dv) continue;
             }
-            rv[u] = load(static_cast<size_t>(t0 + base + tt) * proj_width + v_off + h * dv + c);
+            to.v[u] = load(static_cast<size_t>(t0 + tt) * proj_width + v_off + h * dv + c);
         }
     };
-    const int place = lane % 16 / 4 * DKP + wave * DKR + lane % 4;       // this lane's value of a group: token lane % 16 / 4, key lane % 4
-    auto group = [&](int tt, int tokens) __attribute__((always_inline)) {
-        const float a = a_s[tt * DKP + place], k = k_s[tt * DKP + place], q = q_s[tt * DKP + place];
-        float vj[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) vj[u] = v_s[(tt + u) * kScanCols + lane];
-        float* part = part_s + (tt * NS + wave) * kScanCols + lane;
-        scan_token<0>(a, k, q, vj[0], s, part);
-        if (tokens > 1) scan_token<4>(a, k, q, vj[1], s, part + NS * kScanCols);
-        if (tokens > 2) scan_token<8>(a, k, q, vj[2], s, part + 2 * NS * kScanCols);
-        if (tokens > 3) scan_token<12>(a, k, q, vj[3], s, part + 3 * NS * kScanCols);
-    };
-    // what goes to LDS: made of the loads before a batch's outputs are stored, because a wait for a load behind a store that a
-    // branch may skip waits for the store as well
-    float sq[QKA], sk[QKA], sa[QKA], sv[VL];
-    auto prepare = [&]() {
+    auto stage = [&](int buffer, const Loaded& from) {
 #pragma unroll
         for (int u = 0; u < QKA; ++u) {
             // (a tied key is 1 - a; a place that holds no channel has a = 0 and would get k = 1, which meets a query of zero
             // and a state row that is never stored; places behind the last token are not read)
             const bool in = key0 + (tid + u * THREADS) % DKP < dk;
-            const float q = in ? value(rq[u]) : 0.f, k = in ? value(rk[u]) : 0.f, a = in ? ra[u] : 0.f;
-            sq[u] = (q_silu ? q / (1.0f + expf(-q)) : q) * q_scale;
-            sk[u] = tied_keys ? 1.0f - a : (k_silu ? k / (1.0f + expf(-k)) : k) * k_scale;
-            sa[u] = a;
+            const float q = in ? value(from.q[u]) : 0.f, k = in ? value(from.k[u]) : 0.f, a = in ? from.a[u] : 0.f;
+            q_s[buffer][tid + u * THREADS] = (q_silu ? q / (1.0f + expf(-q)) : q) * q_scale;
+            k_s[buffer][tid + u * THREADS] = tied_keys ? 1.0f - a : (k_silu ? k / (1.0f + expf(-k)) : k) * k_scale;
+            a_s[buffer][tid + u * THREADS] = a;
         }
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
-            const float v = value(rv[u]);
-            sv[u] = v_silu ? v / (1.0f + expf(-v)) : v;
+            const float v = value(from.v[u]);
+            v_s[buffer][tid + u * THREADS] = v_silu ? v / (1.0f + expf(-v)) : v;
         }
     };
-    fetch(0);
-    prepare();
-    for (int base = 0; base < n; base += kScanTokens) {
-        const int count = min(kScanTokens, n - base);
-        __syncthreads();                          // the batch before is read, its parts are added
-#pragma unroll
-        for (int u = 0; u < QKA; ++u) {
-            q_s[tid + u * THREADS] = sq[u];
-            k_s[tid + u * THREADS] = sk[u];
-            a_s[tid + u * THREADS] = sa[u];
-        }
-#pragma unroll
-        for (int u = 0; u < VL; ++u) v_s[tid + u * THREADS] = sv[u];
-        __syncthreads();
-        if (base + kScanTokens < n) fetch(base + kScanTokens);
-        // four tokens at a time; the last tokens of a portion, fewer than four, by the same operations
-        if (count == kScanTokens) {
-#pragma unroll
-            for (int tt = 0; tt < kScanTokens; tt += 4) group(tt, 4);
-        } else {
-            int tt = 0;
-            for (; tt + 4 <= count; tt += 4) group(tt, 4);
-            if (tt < count) group(tt, count - tt);
-        }
-        if (base + kScanTokens < n) prepare();
-        __syncthreads();
-        float o[VL];
+    const size_t token_width = static_cast<size_t>(heads) * dv;
+    float* o_first = out + static_cast<size_t>(split) * n_tokens * token_width + t0 * token_width + h * dv + col0;
+    auto finish = [&](int batch, int buffer) {
+        const int count = batch < 0 ? 0 : min(kScanTokens, n - batch * kScanTokens);         // (none or fewer: no such batch)
+        const float* parts = part_s[buffer];
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
-            const int idx = tid + u * THREADS;
-            o[u] = 0.f;
+            const int tt = wave - NS + u * NS;                      // (of the whole wavefront; a lane is a column)
+            float sum = 0.f;
 #pragma unroll
-            for (int w = 0; w < NS; ++w) o[u] += part_s[(idx / kScanCols * NS + w) * kScanCols + idx % kScanCols];
+            for (int w = 0; w < NS; ++w) sum += parts[w * kPartWave + tt * kScanCols + lane];
+#if defined(__HIP_DEVICE_COMPILE__)
+            float* o = o_first + (max(batch, 0) * static_cast<size_t>(kScanTokens) + tt) * token_width;
+            const auto to = __builtin_amdgcn_make_buffer_rsrc(o, 0, tt < count ? min(kScanCols, dv - col0) * 4 : 0, 0x00020000);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), to, lane * 4, 0, 0);
+#endif
         }
-#pragma unroll
-        for (int u = 0; u < VL; ++u) {
-            const int idx = tid + u * THREADS;
-            const int tt = idx / kScanCols, c = idx % kScanCols;
-            if (tt < count && col0 + c < dv) o_split[(static_cast<size_t>(t0 + base + tt) * heads + h) * dv + col0 + c] = o[u];
-        }
+    };
+    Loaded even, odd;
+    fetch(0, even);
+    if (batches == 1) {
+        stage(0, even);
+        __syncthreads();
+        __syncthreads();
+        finish(0, 0);
+        return;
     }
-    if (has_col) {
-#pragma unroll
-        for (int i = 0; i < DKR; ++i) {
-            const int r = key0 + wave * DKR + i;
-            if (r < dk) state[static_cast<size_t>(r) * dv + j] = s[i];
-        }
+    fetch(1, odd);
+    stage(0, even);
+    __syncthreads();
+    for (int i = 0; i < iterations; i += 2) {
+        fetch(i + 2, even);
+        finish(i - 1, 1);
+        stage(1, odd);
+        __syncthreads();
+        fetch(i + 3, odd);
+        finish(i, 0);
+        stage(0, even);
+        __syncthreads();
     }
 }
 
@@ -345,7 +413,7 @@ static int launch_scan(const void* proj, int n_splits, int proj_width, int q_off
                   : n_splits == 0 ? decayed_state_scan_kernel<T, false, 0>
                   : n_splits == 1 ? decayed_state_scan_kernel<T, false, 1>
                                   : decayed_state_scan_kernel<T, false, 2>;
-    kernel<<<grid, 64 * kScanWaves, 0, s>>>(view, proj_width, q_off, k_off, v_off, q_scale, decay, states, slots, fresh, q_start, q_len,
+    kernel<<<grid, 128 * kScanWaves, 0, s>>>(view, proj_width, q_off, k_off, v_off, q_scale, decay, states, slots, fresh, q_start, q_len,
                                             out, n_tokens, heads, dk, dv, key_splits, q_silu, tied_keys, k_silu, v_silu, head_decay,
                                             cos_sin, rot_dims, mag, interleaved, k_scale);
     return EGPT_OK;

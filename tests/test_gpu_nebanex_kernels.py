@@ -413,6 +413,32 @@ def test_the_state_scan_reads_every_form_of_a_product_alike(k, heads, dk, dv, op
         close(results[0][1][0], last, torch.float32, "the state it leaves")
 
 
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("n", [15, 16, 17, 31, 32, 33, 48, 49, 64, 65])
+def test_the_state_scan_of_one_batch_two_and_more(k, n, form):
+    """Portions that end beside the 16 tokens of a batch, an even and an odd number of batches, beside a request of one token, one of
+    none and one of 40: the same bits as token by token, and close to the plain recurrence."""
+    heads, dk, dv, lens = 1, 20, 70, [n, 1, 0, 40]
+    t, starts = sum(lens), [0, n, n + 1, n + 1]
+    proj, whole, decay, offs = scan_inputs(t, heads, dk, dv, 17, torch.float32, splits=max(form, 1))
+    given, d = (whole if form == 0 else proj).to(DEV), decay.to(DEV)
+    states = torch.full((4, heads, dk, dv), float("nan"), device=DEV)
+    got = k.decayed_state_scan(given, torch.float32, *offs, 0.5, d, states, i32(0, 1, 2, 3), torch.ones(4, dtype=torch.bool, device=DEV),
+                               i32(*starts), i32(*lens), heads, dk, dv)
+    singly = torch.full_like(states, float("nan"))
+    for r in (0, 3):
+        for i in range(starts[r], starts[r] + lens[r]):
+            out = k.decayed_state_scan(given[..., i : i + 1, :].contiguous(), torch.float32, *offs, 0.5, d[i : i + 1], singly, i32(r),
+                                       torch.tensor([i == starts[r]], device=DEV), i32(0), i32(1), heads, dk, dv)
+            assert torch.equal(out[:, 0], got[:, i]), (r, i)
+        assert torch.equal(singly[r], states[r])
+        rows = slice(starts[r], starts[r] + lens[r])
+        want, last = plain_scan(whole[rows], decay[rows], offs, heads, dk, dv, 0.5)
+        close(added(got)[rows].view(-1, heads, dv), want, torch.float32, "outputs")
+        close(states[r], last, torch.float32, "the state it leaves")
+    assert torch.isnan(states[2]).all()
+
+
 def graph_time(f, n=20):
     """Microseconds of one call: the shortest of several replays of a graph of n of them."""
     f()
