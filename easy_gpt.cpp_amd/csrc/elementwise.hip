@@ -347,15 +347,17 @@ __device__ __forceinline__ void load4_as_float(const bf16_t* p, float* v) {
     v[2] = __uint_as_float(a.y << 16); v[3] = __uint_as_float(a.y & 0xffff0000u);
 }
 
-// The same for many tokens (prompt portions) in bfloat16, full rotation (rotary_dim == hd), one tensor in and
-// out, angles from the step's table: a thread owns four neighbouring pairs (i, i + hd/2) of one (token, head).
-template <typename IN>
+// The same for many tokens (prompt portions) in bfloat16, full rotation (rotary_dim == hd), one tensor or PARTS partial
+// sums `stride` apart in, one tensor out, angles from the step's table: a thread owns four neighbouring pairs (i, i + hd/2) of one
+// (token, head).  It is bound by its bytes; the parts' loads are all on their way together and are added in their order.
+template <typename IN, int PARTS>
 __global__ __launch_bounds__(256) void qkv_rope_store_rows_kernel(const IN* __restrict__ qkv_in, bf16_t* __restrict__ qkv_out,
                                                                   const bf16_t* __restrict__ bias,
                                                                   const float* __restrict__ cos_sin,
                                                                   const int32_t* __restrict__ slots,
                                                                   bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
-                                                                  int n_tokens, int nq, int nkv, int hd, int page_size) {
+                                                                  int n_tokens, int nq, int nkv, int hd, int page_size,
+                                                                  size_t stride) {
     const int half = hd / 2, chunks = half / 4;
     const int n_heads = nq + 2 * nkv;
     const long idx = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -364,9 +366,17 @@ __global__ __launch_bounds__(256) void qkv_rope_store_rows_kernel(const IN* __re
     const int head = static_cast<int>((idx / chunks) % n_heads);
     const int t = static_cast<int>(idx / (static_cast<long>(chunks) * n_heads));
     const size_t lo = static_cast<size_t>(t) * n_heads * hd + head * hd + i, hi = lo + half;
-    float a[4], b[4];
-    load4_as_float(qkv_in + lo, a);
-    load4_as_float(qkv_in + hi, b);
+    float parts[PARTS][8], *a = parts[0], *b = parts[0] + 4;
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+        load4_as_float(qkv_in + p * stride + lo, parts[p]);
+        load4_as_float(qkv_in + p * stride + hi, parts[p] + 4);
+    }
+#pragma unroll
+    for (int p = 1; p < PARTS; ++p) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) parts[0][j] += parts[p][j];
+    }
     if (bias) {
         float ba[4], bb[4];
         load4_as_float(bias + head * hd + i, ba);
@@ -561,22 +571,25 @@ extern "C" int egpt_qkv_rope_store(const void* qkv_in, int n_splits, const float
     hipStream_t s = static_cast<hipStream_t>(stream);
     const float inv_hidden = row_ss ? 1.0f / static_cast<float>(hidden) : 0.f;
     const size_t stride = static_cast<size_t>(n_tokens) * (nq + 2 * nkv) * hd;
-    if (dtype == 1 && n_splits <= 1 && !row_ss && rotary_dim == hd && n_tokens >= 64 && hd % 8 == 0 && cos_sin) {
+    if (dtype == 1 && n_splits <= 4 && !row_ss && rotary_dim == hd && n_tokens >= 64 && hd % 8 == 0 && cos_sin &&
+        (n_splits < 2 || reinterpret_cast<uintptr_t>(qkv_in) % 16 == 0)) {
         // many tokens: one thread per four pairs of a (token, head).  (bfloat16 only: the float32 path keeps
         // one kernel per operation whatever the batch, so that its results do not depend on the batch in any
-        // bit.)  The input is bfloat16, or one float32 "partial sum".
+        // bit.)  The input is bfloat16, or one to four float32 partial sums.
         const long items = static_cast<long>(n_tokens) * (nq + 2 * nkv) * (hd / 8);
         const unsigned blocks = static_cast<unsigned>((items + 255) / 256);
-        if (n_splits == 0)
-            qkv_rope_store_rows_kernel<bf16_t><<<blocks, 256, 0, s>>>(
-                static_cast<const bf16_t*>(qkv_in), static_cast<bf16_t*>(qkv_out), static_cast<const bf16_t*>(bias),
-                cos_sin, slots, static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), n_tokens, nq, nkv, hd,
-                page_size);
-        else
-            qkv_rope_store_rows_kernel<float><<<blocks, 256, 0, s>>>(
-                static_cast<const float*>(qkv_in), static_cast<bf16_t*>(qkv_out), static_cast<const bf16_t*>(bias),
-                cos_sin, slots, static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), n_tokens, nq, nkv, hd,
-                page_size);
+        auto launch = [&](auto kernel, auto* in) {
+            kernel<<<blocks, 256, 0, s>>>(in, static_cast<bf16_t*>(qkv_out), static_cast<const bf16_t*>(bias), cos_sin, slots,
+                                          static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), n_tokens, nq, nkv, hd, page_size, stride);
+        };
+        const float* partial = static_cast<const float*>(qkv_in);
+        switch (n_splits) {
+            case 0: launch(qkv_rope_store_rows_kernel<bf16_t, 1>, static_cast<const bf16_t*>(qkv_in)); break;
+            case 1: launch(qkv_rope_store_rows_kernel<float, 1>, partial); break;
+            case 2: launch(qkv_rope_store_rows_kernel<float, 2>, partial); break;
+            case 3: launch(qkv_rope_store_rows_kernel<float, 3>, partial); break;
+            default: launch(qkv_rope_store_rows_kernel<float, 4>, partial); break;
+        }
         EGPT_CHECK_LAUNCH();
         return EGPT_OK;
     }

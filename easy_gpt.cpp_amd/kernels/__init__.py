@@ -210,6 +210,11 @@ class KernelBackend:
         a residual stream in fixed point that the backend can add the product into, that stream."""
         raise NotImplementedError
 
+    def product_parts(self, x, w):
+        """product(x, w, unrounded=True) for a consumer that adds up a few partial sums at no more than their bytes' cost also where
+        the rows are many (`qkv_rope_store` with a whole rotation)."""
+        return self.product(x, w, unrounded=True)
+
     def product_normed(self, h, delta, norm_weight, w, weight_offset=0.0):
         """((h + delta) * (weight_offset + norm_weight)) w^T without the rows' 1/rms factor: (float32 partial sums [S, T, N], row sums
         of squares [S2, T], h + delta as a new tensor), or None."""

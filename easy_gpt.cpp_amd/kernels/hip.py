@@ -323,7 +323,7 @@ class HipKernels(KernelBackend):
                     us += round_us + per * (alone + (full - alone) * (-(-rest // 256) - 1) / max(held - 1, 1))
                 us = max(us, 3 + n * k * 2 / (rate * 1e6))          # the weights alone
                 if s > 1:
-                    us += m * n * (4 * s - 2) / 4.5e6
+                    us += m * n * (4 * s - (4 if form == 1 else 2)) / 4.5e6
                 if best is None or us < best[0]:
                     best = us, shape, s
         return best[1], best[2]
@@ -386,6 +386,19 @@ class HipKernels(KernelBackend):
         # themselves, times over the library's: 4,608 x 3,584 at 200 / 300 / 448 rows 0.79 / 0.98 / 1.24, 4,096 x 2,048 at 128 / 200 / 320 0.88 /
         # 1.12 / 1.24.
         return m <= 448 if n <= k else n < 2 * k and m <= 256
+
+    @staticmethod
+    def _own_parts(m: int, n: int, k: int) -> bool:
+        """Whether a float32 product of more than 64 rows whose consumer takes partial sums is the framework's own with its k range split
+        (`product_parts`).  us, weights from memory, replayed from a graph, the reading of further parts at 4.5 TB/s included,
+        against the library or, at k = 896, one range: 1,152 x 896 at 72 / 200 / 448 / 700 / 1,024 rows 4.7 / 5.3 / 6.1 / 7.2 / 10.1 against
+        6.6 / 6.8 / 7.0 / 7.2 / 8.8, 1,152 x 1,152 4.9 / 5.6 / 6.6 / 8.2 / 10.8 against 6.1 / 6.4 / 7.0 / 9.4 / 10.6, 2,048 x 1,536 at 72 / 200 / 320 / 552 /
+        700 / 1,024 6.1 / 7.5 / 10.1 / 13.0 / 14.1 / 15.7 against 9.4 / 10.1 / 10.7 / 16.9 / 16.8 / 16.9, 2,560 x 2,048 at 72 / 200 / 320 / 448 / 700 7.4 / 10.8 /
+        12.5 / 14.7 / 16.9 against 11.6 / 12.8 / 13.1 / 14.3 / 16.5, 4,608 x 3,584 at 72 / 128 / 200 / 320 / 448 / 700 14.3 / 16.8 / 18.8 / 22.9 / 30.1 / 35.4 against
+        18.9 / 23.0 / 25.8 / 23.8 / 27.4 / 36.0."""
+        if m <= 320:
+            return n * k <= 1 << 24
+        return n * k <= 3300000 and m <= (768 if n * k < 2 << 20 else 1024)
 
     @staticmethod
     def _own_short(m: int, n: int, k: int) -> bool:
@@ -806,6 +819,20 @@ class HipKernels(KernelBackend):
             return out
         out = torch.empty((m, n), dtype=x.dtype, device=x.device)
         return self.linear(x, w, None, out)
+
+    rope_parts = 4               # partial sums that `qkv_rope_store` reads in one go where the tokens are many
+
+    def product_parts(self, x, w):
+        m, k = x.shape
+        n = w.shape[0]
+        if m <= 64 or not self._rows_fit(x, w, k) or not self._own_parts(m, n, k):
+            return self.product(x, w, unrounded=True)
+        self._need(x, "x")
+        self._need(w, "w", x.dtype, (n, k))
+        shape, s = self._rows_plan(m, n, k, self.rope_parts, 1)
+        out = torch.empty((s, m, n), dtype=_F32, device=x.device)
+        self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, 1, 0, shape, self._stream())
+        return out
 
     def rope_table(self, positions, inv_freq):
         """float32 [T, half, 2]: (cos, sin) of float(positions[t]) * inv_freq[i].  A step's angles are the same in

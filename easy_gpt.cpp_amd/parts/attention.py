@@ -117,7 +117,12 @@ class GQAttention(Mixer):
             else:
                 x = x.materialize()
         if prod is None:
-            prod = k.product(x, self.w_qkv, unrounded=True)      # act [T, W], or float32 partial sums [S, T, W]
+            # act [T, W], or float32 partial sums [S, T, W]: several also of many rows, where all of a head turns, but not for the
+            # attention of decoded tokens, which reads them once for every range of keys
+            if rot is not None and rot[1] == self.head_dim and not (ctx.max_q_len == 1 and ctx.rows_independent):
+                prod = k.product_parts(x, self.w_qkv)
+            else:
+                prod = k.product(x, self.w_qkv, unrounded=True)
             dtype, device, t = x.dtype, x.device, x.shape[0]
         slots = cache.slots if cache.writes else None
         common = dict(

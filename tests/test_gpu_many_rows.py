@@ -224,3 +224,41 @@ def test_a_few_dozen_rows(k, m, n, kk):
     act = k.gate_up_swiglu(x, w)
     if act is not None:
         assert ((act.double() - gate).abs() <= gate.abs() * 2.0 ** -8 + 1e-4 * (1 + z.abs()) * (1 + u.abs())).all()
+
+
+@pytest.mark.parametrize("m", [64, 65, 72, 320, 321, 552, 769, 1025])
+@pytest.mark.parametrize("n,kk", [(1152, 896), (2048, 1536), (104, 64), (4608, 3584), (96, 200)])
+def test_a_product_in_parts(k, n, kk, m):
+    """On both sides of every line of its rule: the parts add up to the product, four at most beyond 64 rows."""
+    x, w = rnd(m, kk, seed=7), rnd(n, kk, seed=8, scale=0.1)
+    parts = k.product_parts(x, w)
+    assert parts.dtype == torch.float32 and parts.shape[1:] == (m, n) and (m <= 64 or parts.shape[0] <= k.rope_parts)
+    bound = (x.double().abs() @ w.double().abs().t()) * kk * 2.0 ** -24
+    assert ((parts.double().sum(0) - x.double() @ w.double().t()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("parts", [2, 3, 4, 5])
+@pytest.mark.parametrize("t", [63, 64, 65, 130])
+@pytest.mark.parametrize("nq,nkv,hd,biased,shift", [(14, 2, 64, True, 0), (5, 1, 24, False, 0), (3, 3, 128, True, 0), (4, 2, 32, True, 1)])
+def test_rotation_of_a_product_in_parts(k, t, nq, nkv, hd, biased, shift, parts):
+    """Rows rotated and stored out of partial sums, in whichever kernel takes them: the bits of their sum, added in their order, as one
+    float32 array, the cache included; `shift`: an operand that does not begin on 16 bytes."""
+    width, ps = (nq + 2 * nkv) * hd, 4
+    g = torch.Generator().manual_seed(9)
+    prod = torch.randn(parts * t * width + shift, generator=g).cuda()[shift:].view(parts, t, width)
+    whole = prod[0].clone()
+    for p in range(1, parts):
+        whole += prod[p]
+    bias = rnd(width, seed=10) if biased else None
+    positions = torch.arange(t, dtype=torch.int32, device="cuda") * 3
+    inv = (1e4 ** (-2.0 * torch.arange(hd // 2) / hd)).float().cuda()
+    slots = torch.randperm(t + 5, generator=g)[:t].to(torch.int32).cuda()
+    results = []
+    for given in (prod, whole[None]):
+        pages = -(-(t + 5) // ps)
+        kc = torch.zeros((pages, nkv, ps, hd), dtype=torch.bfloat16, device="cuda")
+        vc = torch.zeros((pages, nkv, hd, ps), dtype=torch.bfloat16, device="cuda")
+        out = torch.empty((t, width), dtype=torch.bfloat16, device="cuda")
+        k.qkv_rope_store(given, bias, positions, inv, hd, slots, kc, vc, nq, nkv, hd, ps, out=out, cos_sin=k.rope_table(positions, inv))
+        results.append((out, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*results))

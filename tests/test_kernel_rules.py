@@ -131,3 +131,12 @@ def test_few_row_plans_are_launchable():
         steps = k // 64
         assert 4 <= shape <= 6 and 1 <= s <= most and (s - 1) * -(-steps // s) < steps, (n, k, most)
         assert s == 1 or (s * -(-n // 64) <= 256 and -(-steps // s) >= 2), (n, k, most)
+
+
+def test_products_in_parts_take_no_more_than_their_reader():
+    for m, n, k in itertools.product(ROWS, WIDTHS, [w for w in WIDTHS if w % 64 == 0]):
+        shape, s = K._rows_plan(m, n, k, K.rope_parts, 1)
+        assert 1 <= s <= K.rope_parts and (s - 1) * -(-(k // 64) // s) < k // 64, (m, n, k, shape, s)
+    for n, k in itertools.product(WIDTHS, WIDTHS):
+        own = [K._own_parts(m, n, k) for m in ROWS]
+        assert own == sorted(own, reverse=True), (n, k)
