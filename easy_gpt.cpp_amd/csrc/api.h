@@ -57,6 +57,9 @@ int egpt_gemm_f32(const float* x, const float* w, const float* bias, float* out,
 // their order.
 int egpt_gemm_f32_rows(const float* x, const float* w, const float* bias, float* out, int m, int n, int k, int n_splits, int fold,
                        int tile_rows, void* stream);
+// w = [gate; up] [2 n][k]: out [m][n] = act(x gate^T) * (x up^T), act 0 silu, 1 gelu's tanh form, of the products that
+// egpt_gemm_f32_rows folds from n_splits ranges.
+int egpt_gemm_f32_gated(const float* x, const float* w, float* out, int m, int n, int k, int n_splits, int tile_rows, int act, void* stream);
 // out = x w^T + bias; x [m,k], w [n,k], out [m,n]; out_f32 != 0 writes float32 whatever dtype is.
 int egpt_linear(const void* x, const void* w, const void* bias, void* out, int m, int n, int k, int dtype,
                 int out_f32, void* stream);

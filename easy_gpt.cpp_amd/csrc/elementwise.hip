@@ -639,4 +639,4 @@ extern "C" const char* egpt_error_string(int code) {
     }
 }
 
-extern "C" int egpt_abi_version(void) { return 28; }
+extern "C" int egpt_abi_version(void) { return 29; }

@@ -324,10 +324,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_mfma_kernel(const float* __r
 // FOLD: a workgroup walks all ranges of k and adds their sums up in their order, which is what a reader of partial sums does:
 // the same bits, without the partial sums' traffic.
 // TAIL: k is no multiple of a block (its end is filled with zeros).
-template <int WM, bool FOLD, bool TAIL>
+// GATED: w = [gate; up] of n rows each, and what leaves is act(x gate^T) * (x up^T), the bits that an activation kernel makes of the
+// product: a wavefront's columns are 32 gates and the up columns of the same numbers.  1,811 rows of 9,728 x 896: 218 us and 21 for
+// the activation kernel, 215 so (71 MB less written, 71 less read, and the activation under the other workgroup's products).
+template <int WM, bool FOLD, bool TAIL, bool GATED>
 __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const float* __restrict__ bias, float* __restrict__ out,
-                                                            int m, int n, int k, int blocks_per_split) {
+                                                            int m, int n, int k, int blocks_per_split, int act) {
     constexpr int TM = 2, TN = 4;                          // 16 x 16 tiles of a wavefront
     constexpr int BM = WM * 32, NT = WM * 128, WL = 512 / NT;   // rows of x; threads; pieces of w that a thread stages
     constexpr int kPartX = BM * 64, kPartW = 128 * 64;     // bytes of a part of an operand's block
@@ -336,13 +339,18 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
     const int li = lane % 16, lg = lane / 16;
     const int wm = wave % WM, wn = wave / WM;
     // a die gets a contiguous range of tiles, rows of x fastest
-    const int mt = (m + BM - 1) / BM, tiles = mt * ((n + 127) / 128);
+    constexpr int kCols = GATED ? 64 : 128;                // columns of the result
+    const int mt = (m + BM - 1) / BM, tiles = mt * ((n + kCols - 1) / kCols);
     int tile = blockIdx.x;
     {
         const int q = tiles / 8, r = tiles % 8, d = tile % 8, i = tile / 8;
         tile = d * q + (d < r ? d : r) + i;
     }
-    const int m0 = tile % mt * BM, n0 = tile / mt * 128;
+    const int m0 = tile % mt * BM, n0 = tile / mt * kCols;
+    auto w_row = [&](int r) {                              // the row of w that is row r of the tile (beyond the last one any)
+        if (!GATED) return w + static_cast<size_t>(min(n0 + r, n - 1)) * k;
+        return w + static_cast<size_t>(min(n0 + r / 64 * 32 + r % 32, n - 1) + (r % 64 < 32 ? 0 : n)) * k;
+    };
     const int total = (k + kBlockF - 1) / kBlockF;
     const int first = FOLD ? 0 : blockIdx.y * blocks_per_split;
     const int last = FOLD ? total : min(total, first + blocks_per_split);
@@ -351,7 +359,7 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
     const float* xp = x + static_cast<size_t>(min(m0 + srow, m - 1)) * k + piece * 8;
     const float* wp[WL];
 #pragma unroll
-    for (int o = 0; o < WL; ++o) wp[o] = w + static_cast<size_t>(min(n0 + srow + o * (NT / 4), n - 1)) * k + piece * 8;
+    for (int o = 0; o < WL; ++o) wp[o] = w_row(srow + o * (NT / 4)) + piece * 8;
     f32x4 raw[2][1 + WL][2];                               // [set][x, w ..][halves]
     auto load = [&](int set, int block) {                  // (beyond the last block the last one again, which nobody reads)
         const int at = min(block, last - 1) * kBlockF;
@@ -389,12 +397,12 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             if (FOLD) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-    const int row0 = m0 + wm * 32 + li, col0 = n0 + wn * 64 + lg * 4;
+    const int row0 = m0 + wm * 32 + li, col0 = n0 + wn * (kCols / 2) + lg * 4;
     // the end of a range [b0, b1) of blocks: elements that are no finite number
     auto mend_range = [&](int b0, int b1) {
         const float* wrow[TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) wrow[j] = w + static_cast<size_t>(min(n0 + wn * 64 + j * 16 + li, n - 1)) * k;
+        for (int j = 0; j < TN; ++j) wrow[j] = w_row(wn * 64 + j * 16 + li);
 #pragma unroll
         for (int i = 0; i < TM; ++i) mend(x + static_cast<size_t>(min(row0 + i * 16, m - 1)) * k, wrow, lg, b0 * kBlockF, min(k, b1 * kBlockF), acc[i]);
     };
@@ -466,13 +474,19 @@ __global__ __launch_bounds__(WM * 128) void gemm_f32_rows_kernel(const float* __
         const int row = row0 + i * 16;
         if (row >= m) continue;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
+        for (int j = 0; j < (GATED ? TN / 2 : TN); ++j) {
             const int col = col0 + j * 16;
             if (col >= n) continue;
             f32x4 val = FOLD ? sum[FOLD ? i : 0][FOLD ? j : 0] : acc[i][j];
+            if constexpr (GATED) {
+                const f32x4 up = FOLD ? sum[FOLD ? i : 0][FOLD ? j + TN / 2 : 0] : acc[i][j + TN / 2];
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-                if (bias && col + v < n) val[v] += bias[col + v];
+                for (int v = 0; v < 4; ++v) val[v] = up[v] * gate_activation(val[v], act);
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (bias && col + v < n) val[v] += bias[col + v];
+            }
             float* at = to + static_cast<size_t>(row) * n + col;
             if (whole) {
                 *reinterpret_cast<f32x4*>(at) = val;
@@ -525,33 +539,47 @@ extern "C" int egpt_gemm_f32(const float* x, const float* w, const float* bias, 
     return EGPT_OK;
 }
 
-extern "C" int egpt_gemm_f32_rows(const float* x, const float* w, const float* bias, float* out, int m, int n, int k,
-                                  int n_splits, int fold, int tile_rows, void* stream) {
-    if (!x || !w || !out || m < 0 || n <= 0 || k <= 0 || n_splits < 1) return EGPT_BAD_ARGUMENT;
-    if (k % 4 != 0 || (bias && n_splits != 1)) return EGPT_UNSUPPORTED_SIZE;
-    if (m == 0) return EGPT_OK;
+template <bool GATED>
+static int launch_f32_rows(const float* x, const float* w, const float* bias, float* out, int m, int n, int k, int n_splits, int fold,
+                           int tile_rows, int act, hipStream_t s) {
     const int total_steps = (k + kStepF - 1) / kStepF;
     const int steps_per_split = (total_steps + n_splits - 1) / n_splits;
     if (n_splits > total_steps || (n_splits - 1) * steps_per_split >= total_steps) return EGPT_BAD_ARGUMENT;   // an empty split
     if (tile_rows != 64 && tile_rows != 128) return EGPT_BAD_ARGUMENT;
-    const long tiles = ((static_cast<long>(m) + tile_rows - 1) / tile_rows) * ((n + 127) / 128);
+    constexpr int cols = GATED ? 64 : 128;
+    const long tiles = ((static_cast<long>(m) + tile_rows - 1) / tile_rows) * ((static_cast<long>(n) + cols - 1) / cols);
     if (tiles > 0x7fffffffL || n_splits > 65535) return EGPT_UNSUPPORTED_SIZE;
     const int per = steps_per_split * (kStepF / kBlockF);
-    hipStream_t s = static_cast<hipStream_t>(stream);
     const bool folded = fold && n_splits > 1, tail = k % kBlockF != 0;
     const dim3 grid(static_cast<unsigned>(tiles), folded ? 1u : static_cast<unsigned>(n_splits));
 #define EGPT_F32_ROWS(WM_)                                                                                                  \
     do {                                                                                                                    \
-        if (folded && tail) gemm_f32_rows_kernel<WM_, true, true><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);       \
-        else if (folded) gemm_f32_rows_kernel<WM_, true, false><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);         \
-        else if (tail) gemm_f32_rows_kernel<WM_, false, true><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);           \
-        else gemm_f32_rows_kernel<WM_, false, false><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per);                    \
+        if (folded && tail) gemm_f32_rows_kernel<WM_, true, true, GATED><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per, act);   \
+        else if (folded) gemm_f32_rows_kernel<WM_, true, false, GATED><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per, act);     \
+        else if (tail) gemm_f32_rows_kernel<WM_, false, true, GATED><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per, act);       \
+        else gemm_f32_rows_kernel<WM_, false, false, GATED><<<grid, WM_ * 128, 0, s>>>(x, w, bias, out, m, n, k, per, act);                \
     } while (0)
     if (tile_rows == 128) EGPT_F32_ROWS(4);
     else EGPT_F32_ROWS(2);
 #undef EGPT_F32_ROWS
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
+}
+
+extern "C" int egpt_gemm_f32_rows(const float* x, const float* w, const float* bias, float* out, int m, int n, int k,
+                                  int n_splits, int fold, int tile_rows, void* stream) {
+    if (!x || !w || !out || m < 0 || n <= 0 || k <= 0 || n_splits < 1) return EGPT_BAD_ARGUMENT;
+    if (k % 4 != 0 || (bias && n_splits != 1)) return EGPT_UNSUPPORTED_SIZE;
+    if (m == 0) return EGPT_OK;
+    return launch_f32_rows<false>(x, w, bias, out, m, n, k, n_splits, fold, tile_rows, 0, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int egpt_gemm_f32_gated(const float* x, const float* w, float* out, int m, int n, int k, int n_splits, int tile_rows,
+                                   int act, void* stream) {
+    if (!x || !w || !out || m < 0 || n <= 0 || n > 0x3fffffff || k <= 0 || n_splits < 1 || act < 0 || act > 1) return EGPT_BAD_ARGUMENT;
+    if (k % 4 != 0) return EGPT_UNSUPPORTED_SIZE;
+    if (m == 0) return EGPT_OK;
+    return launch_f32_rows<true>(x, w, nullptr, out, m, n, k, n_splits, 1, tile_rows, act, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int egpt_linear(const void* x, const void* w, const void* bias, void* out, int m, int n, int k, int dtype,

@@ -31,7 +31,7 @@ def _load_library() -> ctypes.CDLL:
         lib = ctypes.CDLL(path)
     except (build.BuildError, OSError) as e:
         raise KernelsUnavailable(f"the HIP kernel library could not be built or loaded: {e}") from e
-    if lib.egpt_abi_version() != 28:
+    if lib.egpt_abi_version() != 29:
         raise KernelsUnavailable(f"{path} has an unexpected ABI version")
     return lib
 
@@ -100,6 +100,7 @@ class HipKernels(KernelBackend):
             "egpt_linear": [vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_f32": [vp, vp, vp, vp, i, i, i, i, vp],
             "egpt_gemm_f32_rows": [vp, vp, vp, vp, i, i, i, i, i, i, vp],
+            "egpt_gemm_f32_gated": [vp, vp, vp, i, i, i, i, i, i, vp],
             "egpt_gemm_skinny": [vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_rows": [vp, vp, vp, i, i, i, i, i, i, i, vp],
             "egpt_paged_attention": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp],
@@ -734,6 +735,18 @@ class HipKernels(KernelBackend):
     def gate_up_rows(self, x, w, activation="silu"):
         """The same for more than 64 rows.  Returns None where another way is faster or the case is not covered."""
         t, k = x.shape
+        if x.dtype == _F32 and t > 64 and k % 4 == 0 and w.shape[0] % 2 == 0:
+            # in float32 where the tiles hold the whole sums: the bits of the product and the activation kernel behind it
+            s = self._f32_splits(w.shape[0], k)
+            rows, fold = self._f32_rows_plan(t, w.shape[0], k, s)
+            if not rows or not (fold or s == 1):
+                return None
+            inter = w.shape[0] // 2
+            self._need(x, "x", _F32)
+            self._need(w, "w", _F32, (2 * inter, k))
+            out = torch.empty((t, inter), dtype=_F32, device=x.device)
+            self._run("egpt_gemm_f32_gated", x.data_ptr(), w.data_ptr(), out.data_ptr(), t, inter, k, s, rows, _GATES[activation], self._stream())
+            return out
         if t <= 64 or w.shape[0] % 2 or not self._rows_fit(x, w, k) or not self._own_gate(t, k):
             return None
         inter = w.shape[0] // 2

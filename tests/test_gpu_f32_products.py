@@ -193,3 +193,24 @@ def test_small_operands_beside_others(k):
         same = [r for r in range(40) if r not in (3, 7)]
         columns = [c for c in range(48) if c != 9]
         assert torch.equal(got[same][:, columns], clean[same][:, columns])
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("m,inter,kk", [(65, 4, 4), (66, 31, 36), (127, 33, 100), (128, 64, 64), (129, 65, 896), (193, 130, 580), (300, 96, 2052),
+                                        (700, 4864, 896)])
+def test_the_gated_form_leaves_the_bits_of_product_and_activation(k, m, inter, kk, act):
+    x, w = rnd(m, kk, seed=5), rnd(2 * inter, kk, seed=6, scale=kk ** -0.5)
+    if kk > 500:
+        x[3, 7], w[inter // 2, 11] = float("inf"), float("nan")
+    splits = k._f32_splits(2 * inter, kk)
+    parts = few(k, x, w, splits)
+    want = torch.empty((m, inter), device="cuda")
+    k.swiglu(parts, want, activation=act)
+    for rows in (64, 128):
+        out = torch.full((m, inter), 7.0, device="cuda")
+        k._run("egpt_gemm_f32_gated", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, inter, kk, splits, rows, 0 if act == "silu" else 1,
+               k._stream())
+        assert torch.equal(out.nan_to_num(nan=1e30), want.nan_to_num(nan=1e30)) and torch.equal(out.isnan(), want.isnan())
+    got = k.gate_up_rows(x, w, activation=act)
+    assert got is None or torch.equal(got.nan_to_num(nan=1e30), want.nan_to_num(nan=1e30))
+    assert got is not None or inter < 4864
