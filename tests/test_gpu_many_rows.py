@@ -262,3 +262,34 @@ def test_rotation_of_a_product_in_parts(k, t, nq, nkv, hd, biased, shift, parts)
         k.qkv_rope_store(given, bias, positions, inv, hd, slots, kc, vc, nq, nkv, hd, ps, out=out, cos_sin=k.rope_table(positions, inv))
         results.append((out, kc, vc))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", [0, 1, 3, 5])
+@pytest.mark.parametrize("t", [64, 77])
+@pytest.mark.parametrize("nq,nkv,hd,biased,shift", [(14, 2, 64, True, 0), (5, 1, 24, False, 0), (4, 2, 32, True, 1)])
+def test_rotated_rows_are_the_same_bits_in_a_large_and_in_a_small_step(k, t, nq, nkv, hd, biased, shift, form, dtype):
+    """Rows of a step of 64 tokens and more against the same rows 16 at a time, which another kernel takes: the result and the cache."""
+    width, ps = (nq + 2 * nkv) * hd, 4
+    g = torch.Generator().manual_seed(11)
+    prod = torch.randn(max(form, 1) * t * width + shift, generator=g).cuda()
+    prod[shift::37] = -0.0
+    prod = (prod if form else prod.to(dtype))[shift:].view(*((form,) if form else ()), t, width)
+    bias = rnd(width, seed=12).to(dtype) if biased else None
+    positions = torch.arange(t, dtype=torch.int32, device="cuda") * 5
+    inv = (1e4 ** (-2.0 * torch.arange(hd // 2) / hd)).float().cuda()
+    cs = k.rope_table(positions, inv)
+    slots = torch.randperm(t + 5, generator=g)[:t].to(torch.int32).cuda()
+    results = []
+    for step in (t, 16):
+        pages = -(-(t + 5) // ps)
+        kc = torch.zeros((pages, nkv, ps, hd), dtype=dtype, device="cuda")
+        vc = torch.zeros((pages, nkv, hd, ps), dtype=dtype, device="cuda")
+        out = torch.empty((t, width), dtype=dtype, device="cuda")
+        for a in range(0, t, step):
+            rows = slice(a, min(t, a + step))
+            k.qkv_rope_store(prod if step == t else prod[..., rows, :].contiguous(), bias, positions[rows], inv, hd, slots[rows], kc, vc, nq, nkv, hd, ps, out=out[rows],
+                             cos_sin=cs[rows])
+        results.append((out, kc, vc))
+    whole = torch.int32 if dtype == torch.float32 else torch.int16
+    assert all(torch.equal(a.view(whole), b.view(whole)) for a, b in zip(*results))
