@@ -150,8 +150,9 @@ __device__ __forceinline__ void scan_four_tokens(float a, float k, float q, cons
 // loads are plain ones without a branch around them (places beyond the tokens or channels load a neighbour and count as zero),
 // so all of them are on their way together; so are its stores (places without a token or column go nowhere), because a wait for a
 // load beside memory operations that a branch may skip waits for those as well.  Partial sums and
-// rotated operands take several loads each, which do wait for one another, so there a thread whose place holds no token or
-// channel loads nothing.
+// rotated operands take several loads each, all of a query and its key's on their way together; there a thread whose place holds no
+// token or channel loads nothing.  (64 decoded tokens of 7 heads out of one array and out of four partial sums: 15.8 and
+// 22.8 us with four wavefronts for all and a load at a time, 12.6 and 17.9 so; rotated 21.0 and 29.7, 16.8 and 19.2.)
 template <typename T, bool ROTATED, int FORM>
 __global__ __launch_bounds__(128 * kScanWaves) void decayed_state_scan_kernel(
     ProductView<T> proj, int proj_width, int q_off, int k_off, int v_off, float q_scale, const float* __restrict__ decay,
@@ -250,17 +251,31 @@ __global__ __launch_bounds__(128 * kScanWaves) void decayed_state_scan_kernel(
         if constexpr (FORM == 0) return to_float(v);
         else return v;
     };
-    // the value at place r of a head whose columns begin at `at`, turned with its partner
-    auto turned = [&](size_t row, size_t at, int r) {
-        const float own = proj.at(at + r);
-        if (!ROTATED || r >= rot_dims) return own;
+    // the values at place r of two heads whose columns begin at `q_at` and `k_at`, turned with their partners; all their loads
+    // are on their way together
+    auto turned = [&](size_t row, size_t q_at, size_t k_at, int r, float& q, float& k) {
+        if (!ROTATED) {
+            float v[2];
+            read_values(proj, {q_at + r, k_at + r}, v);
+            q = v[0], k = v[1];
+            return;
+        }
+        const bool turns = r < rot_dims;
         const int half = rot_dims / 2;
-        const int i = interleaved ? r / 2 : (r < half ? r : r - half);
+        const int i = !turns ? 0 : interleaved ? r / 2 : (r < half ? r : r - half);
         const bool first = interleaved ? (r & 1) == 0 : r < half;
-        const float other = proj.at(at + (interleaved ? (r ^ 1) : (first ? r + half : r - half)));
+        const int partner = !turns ? r : interleaved ? (r ^ 1) : (first ? r + half : r - half);
         const float c = cos_sin[row * rot_dims + 2 * i] * mag, s = cos_sin[row * rot_dims + 2 * i + 1] * mag;
-        return first ? __fmaf_rn(own, c, -__fmul_rn(other, s)) : __fmaf_rn(other, s, __fmul_rn(own, c));
+        float v[4];
+        read_values(proj, {q_at + r, q_at + partner, k_at + r, k_at + partner}, v);
+        auto turn = [&](float own, float other) {
+            return !turns ? own : first ? __fmaf_rn(own, c, -__fmul_rn(other, s)) : __fmaf_rn(other, s, __fmul_rn(own, c));
+        };
+        q = turn(v[0], v[1]);
+        k = turn(v[2], v[3]);
     };
+    // (a token's values are brought by another wavefront than its queries and keys: a decoded token has no other to wait beside)
+    const int v_first = (wave - NS + NS - 1) % NS;
     const float* decays = head_decay ? head_decay : decay;
     auto fetch = [&](int batch, Loaded& to) {
         const int base = batch * kScanTokens;
@@ -273,20 +288,19 @@ __global__ __launch_bounds__(128 * kScanWaves) void decayed_state_scan_kernel(
                 if (tt >= n || r >= dk) continue;
             }
             const size_t row = static_cast<size_t>(t0 + tt), q_at = row * proj_width + q_off + h * dk;
-            const size_t k_at = tied_keys ? q_at : row * proj_width + k_off + h * dk;
+            const size_t k_at = tied_keys ? q_at : row * proj_width + k_off + h * dk;      // (of a tied key nothing is used)
+            to.a[u] = decays[head_decay ? static_cast<size_t>(h) : row * channels + h * dk + r];
             if constexpr (kPlain) {
                 to.q[u] = load(q_at + r);
-                to.k[u] = load(k_at + r);                          // (of a tied key nothing is used)
+                to.k[u] = load(k_at + r);
             } else {
-                to.q[u] = turned(row, q_at, r);
-                if (!tied_keys) to.k[u] = turned(row, k_at, r);
+                turned(row, q_at, k_at, r, to.q[u], to.k[u]);
             }
-            to.a[u] = decays[head_decay ? static_cast<size_t>(h) : row * channels + h * dk + r];
         }
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
-            const int idx = tid + u * THREADS, in_head = col0 + idx % kScanCols, c = kPlain ? min(in_head, dv - 1) : in_head;
-            const int tt = kPlain ? min(base + idx / kScanCols, n - 1) : base + idx / kScanCols;
+            const int in_head = col0 + lane, c = kPlain ? min(in_head, dv - 1) : in_head, own = base + v_first + u * NS;
+            const int tt = kPlain ? min(own, n - 1) : own;
             if constexpr (!kPlain) {
                 to.v[u] = 0.f;
                 if (tt >= n || c >= dv) continue;
@@ -308,7 +322,7 @@ __global__ __launch_bounds__(128 * kScanWaves) void decayed_state_scan_kernel(
 #pragma unroll
         for (int u = 0; u < VL; ++u) {
             const float v = value(from.v[u]);
-            v_s[buffer][tid + u * THREADS] = v_silu ? v / (1.0f + expf(-v)) : v;
+            v_s[buffer][(v_first + u * NS) * kScanCols + lane] = v_silu ? v / (1.0f + expf(-v)) : v;
         }
     };
     const size_t token_width = static_cast<size_t>(heads) * dv;
