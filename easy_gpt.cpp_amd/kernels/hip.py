@@ -330,6 +330,14 @@ class HipKernels(KernelBackend):
         return best[1], best[2]
 
     @staticmethod
+    def _sums_kept(m: int, n: int, k: int) -> bool:
+        """Whether a product of more than 64 rows for a reader that takes float32 sums leaves unrounded also where its k range is one
+        piece (a split one always does).  Rounded halves what is written and read again, m * n * 4 bytes at 4.5 TB/s: up to
+        1 us for a million values, 2 for twice as many out of a short k, and beyond k = 4,096 a few hundredths of the product.  There the
+        float32 sum goes on; elsewhere a rounded one is what the library's product would be as well."""
+        return k > 4096 or m * n <= 1 << 20 or (n >= 4 * k and m * n <= 1 << 21)
+
+    @staticmethod
     def _few_plan(n: int, k: int, most_splits: int) -> tuple[int, int]:
         """(shape, splits of the k range) of gemm_rows.hip for 17 to 64 rows, one tile of rows: the weights' way from memory is what
         counts, so every CU gets one workgroup.  An output of fewer than 256 tiles of 64 columns has its k range split until there are as
@@ -808,8 +816,9 @@ class HipKernels(KernelBackend):
             # many rows on the framework's own kernel: rounded, or float32 partial sums where the k range is split
             self._need(x, "x")
             self._need(w, "w", x.dtype, (n, k))
-            shape, s = self._rows_plan(m, n, k, 1 if unrounded else 10, 1 if unrounded else 0)
-            kind = 1 if unrounded or s > 1 else 0
+            form = 1 if unrounded or self._sums_kept(m, n, k) else 0
+            shape, s = self._rows_plan(m, n, k, 1 if unrounded else 10, form)
+            kind = 1 if form or s > 1 else 0
             out = torch.empty((s, m, n) if kind else (m, n), dtype=_F32 if kind else _BF16, device=x.device)
             self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, kind, 0, shape, self._stream())
             return out

@@ -293,3 +293,16 @@ def test_rotated_rows_are_the_same_bits_in_a_large_and_in_a_small_step(k, t, nq,
         results.append((out, kc, vc))
     whole = torch.int32 if dtype == torch.float32 else torch.int16
     assert all(torch.equal(a.view(whole), b.view(whole)) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("m,n,kk", [(577, 896, 896), (1024, 896, 896), (960, 896, 768), (913, 1024, 1024), (448, 1536, 1536), (256, 3584, 3584),
+                                    (192, 5120, 5120), (2305, 1024, 8192), (65, 18944, 896)])
+def test_sums_that_a_norm_adds_are_not_rounded(k, m, n, kk):
+    # also where k is one range: each element within the float32 sum's own error, which a rounding to bfloat16 would exceed
+    x, w = rnd(m, kk, seed=31), rnd(n, kk, seed=32, scale=kk ** -0.5)
+    got = k.product(x, w)
+    assert got.dtype == torch.float32 and got.dim() == 3
+    got = got.double().sum(0)
+    for a in range(0, m, 256):
+        want = x[a : a + 256].double() @ w.double().t()
+        assert ((got[a : a + 256] - want).abs() <= (x[a : a + 256].double().abs() @ w.double().abs().t()) * kk * 2.0 ** -24).all()

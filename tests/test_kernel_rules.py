@@ -88,12 +88,12 @@ ROWS = [65, 66, 96, 127, 128, 129, 192, 256, 257, 448, 552, 1000, 1537, 2048, 35
 
 def test_plans_of_many_rows_are_launchable():
     # what egpt_gemm_rows refuses: shapes that do not exist, empty ranges of k, more workgroups than a grid holds
-    for m, n, k, most in itertools.product(ROWS, WIDTHS, [w for w in WIDTHS if w % 64 == 0], (1, 10)):
-        shape, s = K._rows_plan(m, n, k, most)
+    for m, n, k, (most, form) in itertools.product(ROWS, WIDTHS, [w for w in WIDTHS if w % 64 == 0], ((1, 0), (10, 0), (10, 1), (1, 2))):
+        shape, s = K._rows_plan(m, n, k, most, form)
         bm, bn = K._rows_shapes[shape][:2]
         steps = k // 64
         per = -(-steps // s)
-        what = (m, n, k, most, shape, s)
+        what = (m, n, k, most, form, shape, s)
         assert 1 <= s <= min(most, steps) and (s - 1) * per < steps, what
         assert -(-m // bm) * -(-n // bn) * s <= 0x7FFFFFFF, what
 
