@@ -412,11 +412,26 @@ class HipKernels(KernelBackend):
     @staticmethod
     def _own_short(m: int, n: int, k: int) -> bool:
         """Whether the product is the framework's own beyond the lines of `_own_rows`: with a short k range a tile is its beginning and its
-        end for the most part, and a workgroup's next tile begins under the end of the one before.  us, weights from memory, replayed from
-        a graph: 896 x 896 rounded, with its norm, at 2,535 / 3,500 / 5,000 / 8,191 rows 18.5 / 21.1 / 29.1 / 34.6 against the library's 19.8 / 21.0 /
-        25.2 / 39.7; unrounded 2,752 x 896 at 2,048 / 2,535 / 3,500 / 5,000 / 8,191 19.5 / 20.1 / 25.0 / 31.0 / 50.3 against 18.7 / 28.4 / 27.1 / 49.5 /
-        77.8, 1,152 x 896 at 2,535 / 5,000 / 8,191 13.6 / 19.8 / 25.4 against 11.9 / 15.9 / 27.3.  3,072 x 1,024 at 8,191 67.6 against 53.2."""
-        return k <= 896 and (m >= 6000 or (m >= 2304 and n >= 2 * k) or (m <= 2600 and n <= k))
+        end for the most part, and a workgroup's next tile begins under the end of the one before.  Drawn through 1,030 points (1,200 to
+        16,384 rows, k of 320 to 896, n from k / 2 to 9,728, rounded with its norm and unrounded; weights from memory, replayed from a graph):
+        the faster side within 1.5 % on average, where `_own_rows` alone loses 7 %.  The library goes in steps of its own, so beside a
+        line either side is ahead in places, by a third at worst.  us, own against the library's:
+        k = 320 to 640: 512 x 512 rounded at 2,304 / 4,096 / 8,191 rows 11.8 / 13.9 / 21.5 against 14.6 / 15.9 / 23.0, 1,920 x 640 at 2,600 / 4,000 / 8,191 /
+        16,384 26.4 / 34.0 / 58.5 / 117 against 27.7 / 39.3 / 76.4 / 146, unrounded 640 x 640 at 3,300 / 6,000 / 7,000 10.4 / 12.3 / 15.7 against 9.7 / 13.4 / 12.5.
+        n up to k: 896 x 896 rounded at 2,048 / 2,600 / 4,000 / 5,000 / 6,000 / 7,000 / 8,191 / 12,000 / 16,384 15.6 / 18.9 / 21.9 / 28.4 / 31.0 / 33.2 / 35.4 / 46.5 /
+        58.2 against 16.4 / 19.9 / 21.9 / 25.4 / 28.8 / 32.8 / 41.0 / 55.9 / 71.8, unrounded 768 x 768 at 2,600 / 3,300 / 5,000 / 7,000 / 12,000 9.3 / 11.7 / 13.3 /
+        18.8 / 24.5 against 9.5 / 10.8 / 12.6 / 15.9 / 27.1.
+        Wider: 2,688 x 896 rounded at 2,048 / 2,600 / 3,300 / 4,000 / 5,000 / 8,191 31.1 / 36.0 / 42.1 / 47.2 / 56.2 / 86.5 against 29.5 / 35.7 / 47.6 / 56.2 / 72.3 /
+        93.3, unrounded 20.2 / 21.4 / 26.3 / 27.0 / 32.6 / 50.2 against 17.0 / 19.3 / 27.9 / 36.8 / 44.6 / 49.7; 9,728 x 896 unrounded at 2,048 / 3,300 / 5,000 / 6,000 /
+        10,000 55.0 / 65.5 / 97.0 / 136 / 190 against 49.3 / 69.5 / 112 / 125 / 200.  A longer k is a tie at best: 1,024 x 1,024 at 4,096 / 5,000 / 8,191 23.8 / 30.8 /
+        38.5 against 23.6 / 28.1 / 38.3; one to three steps of k leave nothing to begin under: 1,024 x 128 at 2,600 / 8,191 16.5 / 34.6 against 15.7 / 29.2,
+        4,096 x 256 at the ends of what is measured 25.7 at 1,600 and 214 at 16,384 against 30.7 and 214."""
+        return 256 <= k <= 640 or (640 < k <= 896 and ((n <= k and m <= 2600) or m >= (3300 if 2 * n >= 3 * k else 7000)))
+
+    @classmethod
+    def _own_many(cls, m: int, n: int, k: int, unrounded: bool) -> bool:
+        """Whether a bfloat16 product of more than 64 rows is the framework's own."""
+        return cls._own_rows(m, n, k, unrounded) or cls._own_short(m, n, k)
 
     @staticmethod
     def _own_gate(m: int, k: int) -> bool:
@@ -812,7 +827,7 @@ class HipKernels(KernelBackend):
             self._run("egpt_gemm_skinny", x.data_ptr(), w.data_ptr(), None, self._ptr(out), None, self._ptr(target),
                       m, n, k, s, 4, self._stream())
             return out if target is None else target
-        if m > 64 and self._rows_fit(x, w, k) and (self._own_rows(m, n, k, unrounded) or self._own_short(m, n, k)):
+        if m > 64 and self._rows_fit(x, w, k) and self._own_many(m, n, k, unrounded):
             # many rows on the framework's own kernel: rounded, or float32 partial sums where the k range is split
             self._need(x, "x")
             self._need(w, "w", x.dtype, (n, k))

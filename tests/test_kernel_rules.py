@@ -124,6 +124,22 @@ def test_the_rules_for_many_rows_change_sides_once():
         assert sum(a != b for a, b in zip(own, own[1:])) <= 2, k
 
 
+def test_a_product_comes_back_from_the_library_once_at_most():
+    # both rules together: own, then perhaps the library, then perhaps own for good; with a long k no way back
+    rows = list(range(65, 20000, 61))
+    for n, k, unrounded in itertools.product(WIDTHS + [448, 2688], WIDTHS + [640, 768], (False, True)):
+        own = [K._own_many(m, n, k, unrounded) for m in rows]
+        assert own[0] or k > 896, (n, k, unrounded)
+        assert sum(a != b for a, b in zip(own, own[1:])) <= (2 if 640 < k <= 896 else 0 if 256 <= k <= 640 else 1), (n, k, unrounded)
+    # (rows, n, k, unrounded) with both sides measured more than the runs differ
+    for sizes in [(2304, 512, 512, False), (8191, 1920, 640, False), (2600, 896, 896, False), (8191, 896, 896, False), (16384, 896, 896, True),
+                  (4000, 2688, 896, False), (5000, 2688, 896, True), (5000, 9728, 896, True)]:
+        assert K._own_many(*sizes), sizes
+    for sizes in [(5000, 896, 896, False), (6000, 896, 896, False), (3300, 768, 768, True), (2048, 2688, 896, True), (2048, 9728, 896, True),
+                  (5000, 1024, 1024, False), (8191, 1024, 128, False), (4000, 4096, 64, False)]:
+        assert not K._own_many(*sizes), sizes
+
+
 def test_few_row_plans_are_launchable():
     # what egpt_gemm_rows refuses: an empty range, or splits of a result that is not float32
     for n, k, most in itertools.product(WIDTHS + [8, 16384, 16392, 32776], [w for w in WIDTHS if w % 64 == 0], (1, 8, 16)):
