@@ -469,7 +469,7 @@ class HipKernels(KernelBackend):
             return out
         if x.dtype == _BF16 and k % 8 == 0:
             to_f32 = out.dtype == _F32
-            if to_f32 and bias is None and 16 < m <= 64 and n >= 65536 and self._rows_fit(x, w, k):
+            if to_f32 and bias is None and 16 < m <= 64 and n >= 65536 and self._rows_fit(x, w, k) and out.data_ptr() % 16 == 0:
                 # An output matrix over a whole vocabulary: tiles of 64 x 128 with six steps on their way (us, weights from memory, at
                 # 17 / 32 / 48 / 64 rows, against the weight-streaming kernel up to 32 and the library beyond): 151,936 x 896 56 / 58 / 62 / 67
                 # against 62 / 68 / 76 / 74, 151,936 x 1,536 91 / 97 / 105 / 110 against 103 / 107 / 123 / 118, 102,400 x 2,048 101 / 105 / 108 / 114 against

@@ -328,3 +328,16 @@ def test_an_activation_is_as_good_as_the_general_one(k, act, low, high):
     unit = torch.exp2(torch.floor(torch.log2(want.abs())) - 7)
     want = torch.round(want / unit) * unit
     assert float((out != want).double().mean()) <= (8e-6 if act == 0 else 1.1e-5)
+
+
+@pytest.mark.parametrize("m", [17, 33, 64])
+def test_an_output_matrix_writes_where_it_is_told(k, m):
+    # logits that do not begin on 16 bytes; what lies before and behind them stays
+    n, kk = 65544, 64
+    x, w = rnd(m, kk, seed=61), rnd(n, kk, seed=62)
+    store = torch.full((m * n + 8,), -7.0, device="cuda")
+    out = store[3 : 3 + m * n].view(m, n)
+    assert k.linear(x, w, None, out) is out
+    bound = (x.double().abs() @ w.double().abs().t()) * kk * 2.0 ** -24
+    assert ((out.double() - x.double() @ w.double().t()).abs() <= bound).all()
+    assert (store[:3] == -7).all() and (store[3 + m * n :] == -7).all()
