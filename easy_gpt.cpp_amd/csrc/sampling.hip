@@ -60,9 +60,15 @@ __device__ __forceinline__ void argmax_combine(float& v, int& i, float ov, int o
     }
 }
 
-__device__ int block_argmax(const float* __restrict__ row, int vocab, float* s_val, int* s_idx) {
+// The row's best token and its value (every thread); kNoToken and -infinity where there is nothing but NaN.
+struct BestToken {
+    int index;
+    float value;
+};
+constexpr int kNoToken = 0x7fffffff;
+__device__ BestToken block_argmax(const float* __restrict__ row, int vocab, float* s_val, int* s_idx) {
     float best = -INFINITY;
-    int best_i = 0x7fffffff;
+    int best_i = kNoToken;
     for_each_in_row(row, vocab, threadIdx.x, blockDim.x, [&](int j, float v) {
         if (v > best || (v == best && j < best_i)) {
             best = v;
@@ -86,7 +92,7 @@ __device__ int block_argmax(const float* __restrict__ row, int vocab, float* s_v
     best = s_val[0];
     best_i = s_idx[0];
     for (int w = 1; w < n_waves; ++w) argmax_combine(best, best_i, s_val[w], s_idx[w]);
-    return best_i == 0x7fffffff ? 0 : best_i;
+    return {best_i, best};
 }
 
 __global__ __launch_bounds__(kSampleThreads) void argmax_kernel(const float* __restrict__ logits,
@@ -94,8 +100,8 @@ __global__ __launch_bounds__(kSampleThreads) void argmax_kernel(const float* __r
     __shared__ float s_val[16];
     __shared__ int s_idx[16];
     const int r = blockIdx.x;
-    const int best = block_argmax(logits + static_cast<size_t>(r) * vocab, vocab, s_val, s_idx);
-    if (threadIdx.x == 0) out[r] = best;
+    const int best = block_argmax(logits + static_cast<size_t>(r) * vocab, vocab, s_val, s_idx).index;
+    if (threadIdx.x == 0) out[r] = best == kNoToken ? 0 : best;
 }
 
 // Two stages for wide vocabularies: workgroup (row, c) finds the maximum of its piece of the row, then one
@@ -115,35 +121,27 @@ __global__ __launch_bounds__(256) void argmax_pieces_kernel(const float* __restr
     const int r = blockIdx.x, c = blockIdx.y;
     const int piece = (vocab + kArgmaxPieces - 1) / kArgmaxPieces;
     const int begin = min(vocab, c * piece), n = min(vocab, begin + piece) - begin;
-    int best = 0;
-    float val = -INFINITY;
-    if (n > 0) {
-        const float* row = logits + static_cast<size_t>(r) * vocab + begin;
-        best = block_argmax(row, n, s_val, s_idx);
-        val = row[best];
-    }
+    BestToken best{kNoToken, -INFINITY};
+    if (n > 0) best = block_argmax(logits + static_cast<size_t>(r) * vocab + begin, n, s_val, s_idx);
     if (threadIdx.x == 0) {
-        piece_val[r * kArgmaxPieces + c] = val;
-        piece_idx[r * kArgmaxPieces + c] = begin + best;
+        piece_val[r * kArgmaxPieces + c] = best.value;
+        piece_idx[r * kArgmaxPieces + c] = best.index == kNoToken ? kNoToken : begin + best.index;
     }
     if (sub_val && threadIdx.x < 4) sub_val[r * kSubPieces + c * 4 + threadIdx.x] = n > 0 ? s_val[threadIdx.x] : -INFINITY;
 }
 
-// The row's best token out of its pieces' (lowest index among equal maxima) and its value, by a whole wavefront.
-struct BestToken {
-    int index;
-    float value;
-};
+// The row's best token out of its pieces' (lowest index among equal maxima; the first of nothing but NaN) and its value, by a whole
+// wavefront.
 __device__ __forceinline__ BestToken best_of_pieces(const float* __restrict__ piece_val, const int32_t* __restrict__ piece_idx, int r, int lane) {
     float v = lane < kArgmaxPieces ? piece_val[r * kArgmaxPieces + lane] : -INFINITY;
-    int i = lane < kArgmaxPieces ? piece_idx[r * kArgmaxPieces + lane] : 0x7fffffff;
+    int i = lane < kArgmaxPieces ? piece_idx[r * kArgmaxPieces + lane] : kNoToken;
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
         const float ov = __shfl_xor(v, o, kWave);
         const int oi = __shfl_xor(i, o, kWave);
         argmax_combine(v, i, ov, oi);
     }
-    return {__builtin_amdgcn_readfirstlane(i), __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)))};
+    return {__builtin_amdgcn_readfirstlane(i == kNoToken ? 0 : i), __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)))};
 }
 __global__ __launch_bounds__(64) void argmax_pick_kernel(const float* __restrict__ piece_val,
                                                          const int32_t* __restrict__ piece_idx,
@@ -918,7 +916,11 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
             more = list_count[(r * kSamplePieces + lane) * 2 + 1];
         }
     }
-    const int best = cand_idx ? known_best : block_argmax(row, vocab, s_val, s_idx);
+    int best = known_best;
+    if (!cand_idx) {
+        best = block_argmax(row, vocab, s_val, s_idx).index;
+        if (best == kNoToken) best = 0;
+    }
     if (!(temp > 0.f)) {  // greedy, as the reference for temperature <= 0 (sampler.cpp:46-49)
         if (threadIdx.x == 0) out[r] = best;
         return;

@@ -82,6 +82,29 @@ def test_rows_of_each_kind_beside_each_other(k):
         assert alone[0] == together[r], r
 
 
+@pytest.mark.parametrize("first", [0, 7, 31])
+def test_a_share_of_nothing_but_nan(k, first):
+    # the row's maximum is that of the other shares, wherever the one without a number lies and wherever the maximum does
+    vocab = 20000
+    piece = -(-vocab // 32)
+    for at in (3, 9000, vocab - 1):
+        if at // piece == first:
+            continue
+        logits = torch.randn(3, vocab, generator=torch.Generator().manual_seed(at))
+        logits[:, at] = 40.0
+        logits[1, :] = float("-inf")
+        logits[1, at] = -3.0
+        logits[2, :] = float("-inf")
+        logits[:, first * piece : (first + 1) * piece] = float("nan")
+        least = 0 if first else piece                               # of the last row: its first token that is a number
+        for top_k, top_p in ((20, 0.9), (200, 0.9), (0, 0.9), (0, 1.0)):
+            for temperature in (0.0, 1.0):
+                assert draw(k, logits.cuda(), temperature, top_k, top_p, torch.tensor([0.5] * 3)).tolist() == [at, at, least], (at, top_k, top_p)
+        out = torch.full((3,), -7, dtype=torch.int32, device="cuda")
+        k.argmax(logits.cuda(), out)
+        assert out.tolist() == [at, at, least]
+
+
 @pytest.mark.parametrize("top_k,top_p", [(20, 0.9), (200, 0.9), (0, 0.9), (0, 1.0)])
 def test_numbers_that_are_none(k, top_k, top_p):
     # a NaN is never drawn; an infinity is; a row of nothing but NaN or minus infinity gives its first token
