@@ -249,10 +249,16 @@ class KernelBackend:
         sums; False if not covered (nothing was done), else what paged_attention returns."""
         return False
 
-    def decode_ranges(self, kv_len, q_start, q_len, nkv, hd, window, max_kv_len, spread=0):
-        """What the attention of decoded tokens needs to deal out their keys by the contexts' lengths (the `ranges` of
-        attention_decode_fused and paged_attention_mixed; the same for all layers of a kind), or None."""
-        return None
+    def deals_out(self, dtype, nq, nkv, hd, page_size, requests, max_kv_len, spread=None) -> bool:
+        """Whether the attention of a step's decoded tokens deals out their keys by the contexts' lengths, and so reads a table of
+        `decode_ranges`: that of a step of decoded tokens alone by attention_decode_fused, whose contexts are as uneven as `spread` says
+        (`StepContext.spread`), or, spread None, that of a step with portions of prompts by paged_attention_mixed."""
+        return False
+
+    def decode_ranges(self, kv_len, q_start, q_len, nkv, window):
+        """The `ranges` of attention_decode_fused (q_len None) and paged_attention_mixed, where `deals_out` says so; the same for all
+        layers with as many kv heads and the same window."""
+        raise NotImplementedError
 
     def paged_attention_mixed(self, *args, ranges=None, portion_kv=None, **kwargs):
         """paged_attention with two hints: the table of `decode_ranges`, and the longest context of a request that brings

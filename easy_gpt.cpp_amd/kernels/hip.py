@@ -918,23 +918,26 @@ class HipKernels(KernelBackend):
                   self._ptr(k_cache), self._ptr(v_cache), t, nq, nkv, hd, page_size, dt, self._stream())
         return out
 
-    def decode_ranges(self, kv_len, q_start, q_len, nkv, hd, window, max_kv_len, spread=0):
-        """The table by which the attention of decoded tokens deals out their keys by the contexts' lengths, int32
-        [slots * 8 + B * 2], or None where every request gets the same number of key ranges (`_decode_shape`).  q_len given: a step
-        that also holds portions of prompts.  spread: how uneven the contexts are (`StepContext.spread`)."""
+    @classmethod
+    def deals_out(cls, dtype, nq, nkv, hd, page_size, requests, max_kv_len, spread=None):
+        if dtype != _BF16 or hd not in (64, 128) or page_size % 16 or nq // nkv > 16:
+            return False
+        if spread is None:
+            return (page_size & (page_size - 1) == 0 and requests * nkv <= 256
+                    and max_kv_len > (cls.singles_apart_beyond if hd == 64 else cls.singles_dealt_beyond))
+        # A step of decoded tokens, whose parts a kernel combines.  Where the contexts are as long as each other the ranges are
+        # the same and the table is one more trip to memory (0.2 to 0.9 us a layer), so it is taken where they are not: us a layer,
+        # combination included, equal ranges and dealt out: 12 heads of 128 on 2, 40 requests of 128 to 2,048 tokens 23.5 and 18.2, 28
+        # heads of 128 on 4, 24 of 200 to 1,400 19.1 and 17.7 (64 of them, more pairs than half the CUs: 32.3 and 34.5), 14 heads of 64
+        # on 2, 64 of 130 to 2,048 17.0 and 16.5, which the table's own 5 us a step use up, one of 8,000 beside 31 of 500 21.8 and 15.0.
+        # The longer the contexts the more: one of 12,000 beside 23 of 500 26.2 and 17.5, 43.4 and 21.0, 93.1 and 23.1 (heads in the order 14 of
+        # 64, 12 of 128, 28 of 128), one of 32,000 beside them 55.5 and 22.7, 96.9 and 27.9, 216 and 33.6, 24 of 100 to 16,000 at head size
+        # 128 65.9 and 50.7, 136 and 92.1.
+        return cls.fused_rows < requests and requests * nkv <= 128 and spread >= (2 if hd == 64 else 1)
+
+    def decode_ranges(self, kv_len, q_start, q_len, nkv, window):
+        """int32 [slots * 8 + B * 2], see decode_ranges_kernel."""
         (b,) = kv_len.shape
-        if hd not in (64, 128):
-            return None
-        if q_len is None:
-            # A step of decoded tokens, whose parts a kernel combines.  Where the contexts are as long as each other the ranges are
-            # the same and the table is one more trip to memory (0.2 to 0.9 us a layer), so it is taken where they are not: us a layer,
-            # combination included, equal ranges and dealt out: 12 heads of 128 on 2, 40 requests of 128 to 2,048 tokens 23.5 and 18.2, 28
-            # heads of 128 on 4, 24 of 200 to 1,400 19.1 and 17.7 (64 of them, more pairs than half the CUs: 32.3 and 34.5), 14 heads of 64
-            # on 2, 64 of 130 to 2,048 17.0 and 16.5, which the table's own 5 us a step use up, one of 8,000 beside 31 of 500 21.8 and 15.0
-            if b <= self.fused_rows or b * nkv > 128 or max_kv_len > 9216 or spread < (2 if hd == 64 else 1):
-                return None
-        elif b * nkv > 256 or max_kv_len <= (self.singles_apart_beyond if hd == 64 else self.singles_dealt_beyond):
-            return None
         for name, v in (("kv_len", kv_len), ("q_start", q_start)) + ((("q_len", q_len),) if q_len is not None else ()):
             self._need(v, name, _I32, (b,))
         slots = 256 // nkv

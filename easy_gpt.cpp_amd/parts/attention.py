@@ -135,9 +135,10 @@ class GQAttention(Mixer):
         # the cache in one kernel, straight from the product's partial sums
         parts = False
         cos_sin = self.position.table(ctx) if rot is not None else None
-        ranges = None if want_parts else self._ranges(k, ctx)
-        if (prod.dim() == 3 and rot is not None and slots is not None and ctx.max_q_len == 1
-                and ctx.rows_independent):
+        fused = (prod.dim() == 3 and rot is not None and slots is not None and ctx.max_q_len == 1
+                 and ctx.rows_independent)
+        ranges = None if want_parts else self._ranges(k, ctx, dtype, cache.page_size, fused and rot[1] == self.head_dim)
+        if fused:
             parts = k.attention_decode_fused(
                 prod, scale_args.get("row_ss"), scale_args.get("hidden", 0), scale_args.get("eps", 0.0), self.b_qkv,
                 ctx.positions, rot[0], rot[1], slots, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.kv_len,
@@ -162,14 +163,18 @@ class GQAttention(Mixer):
         k.linear(attn, self.w_o, self.b_o, out)
         return out
 
-    def _ranges(self, k, ctx):
-        """How the keys of the step's decoded tokens are dealt out, the same for all layers with these heads and this window."""
-        if not ctx.rows_independent or (ctx.max_q_len > 1 and not getattr(ctx, "single_token_requests", True)):
+    def _ranges(self, k, ctx, dtype, page_size, fused):
+        """How the keys of the step's decoded tokens are dealt out, the same for all layers with these kv heads and this window; None
+        where nothing goes by it (`fused`: in a step of decoded tokens alone, attention_decode_fused does)."""
+        decoded = ctx.max_q_len == 1
+        if not ctx.rows_independent or not (fused if decoded else getattr(ctx, "single_token_requests", True)):
             return None
-        key = ("decode_ranges", self.n_kv_heads, self.head_dim, self.window)
+        if not k.deals_out(dtype, self.n_heads, self.n_kv_heads, self.head_dim, page_size, ctx.kv_len.shape[0], ctx.max_kv_len,
+                           getattr(ctx, "spread", 0) if decoded else None):
+            return None
+        key = ("decode_ranges", self.n_kv_heads, self.window)
         if key not in ctx.shared:
-            ctx.shared[key] = k.decode_ranges(ctx.kv_len, ctx.q_start, None if ctx.max_q_len == 1 else ctx.q_len, self.n_kv_heads,
-                                              self.head_dim, self.window or 0, ctx.max_kv_len, getattr(ctx, "spread", 0))
+            ctx.shared[key] = k.decode_ranges(ctx.kv_len, ctx.q_start, None if decoded else ctx.q_len, self.n_kv_heads, self.window or 0)
         return ctx.shared[key]
 
     def _epilogue_and_attention(self, k, prod, t, width, dtype, device, rot, slots, common, scale_args, ctx, cache, attn,

@@ -3,6 +3,9 @@ sizes; between and beyond those they choose speed, not results, but what they re
 kernels take.  Checked here over a grid of sizes, on the CPU (the rules are plain functions of the sizes)."""
 import itertools
 
+import torch
+
+from easy_gpt.cpp_amd.engine.engine import _spread
 from easy_gpt.cpp_amd.kernels.hip import HipKernels as K
 
 BATCHES = [1, 2, 3, 7, 8, 16, 17, 31, 32, 33, 48, 63, 64, 65, 100, 128, 200, 256, 257, 512, 1000, 4096]
@@ -156,3 +159,31 @@ def test_products_in_parts_take_no_more_than_their_reader():
     for n, k in itertools.product(WIDTHS, WIDTHS):
         own = [K._own_parts(m, n, k) for m in ROWS]
         assert own == sorted(own, reverse=True), (n, k)
+
+
+def test_keys_are_dealt_out_where_a_kernel_reads_the_table():
+    f32, bf16 = torch.float32, torch.bfloat16
+    # (nq, nkv, hd, page size, requests, longest context, spread)
+    assert K.deals_out(bf16, 12, 2, 128, 16, 40, 2048, 1) and K.deals_out(bf16, 14, 2, 64, 16, 32, 8192, 2)
+    assert K.deals_out(bf16, 12, 2, 128, 16, 24, 32768, 2)                          # the longer the better
+    assert not K.deals_out(f32, 12, 2, 128, 16, 40, 2048, 2)                        # other kernels' dtype, head size, heads, pages
+    assert not K.deals_out(bf16, 12, 2, 96, 16, 40, 2048, 2) and not K.deals_out(bf16, 34, 2, 64, 16, 40, 2048, 2)
+    assert not K.deals_out(bf16, 12, 2, 128, 8, 40, 2048, 2)
+    assert not K.deals_out(bf16, 14, 2, 64, 16, 64, 2048, 1) and not K.deals_out(bf16, 12, 2, 128, 16, 40, 2048, 0)      # even contexts
+    assert not K.deals_out(bf16, 12, 2, 128, 16, 16, 2048, 2) and not K.deals_out(bf16, 12, 2, 128, 16, 72, 2048, 2)     # few, many
+    # beside portions of prompts
+    assert K.deals_out(bf16, 12, 2, 128, 16, 41, 2048) and K.deals_out(bf16, 14, 2, 64, 16, 64, 4096)
+    assert not K.deals_out(bf16, 12, 2, 128, 16, 41, 1024) and not K.deals_out(bf16, 14, 2, 64, 16, 64, 2048)
+    assert not K.deals_out(f32, 12, 2, 128, 16, 41, 2048) and not K.deals_out(bf16, 12, 2, 128, 48, 41, 2048)
+    assert not K.deals_out(bf16, 12, 2, 128, 16, 129, 2048)
+    # the kernels' limits: a slot for every request, at most 256 of them
+    for nkv, b, spread in itertools.product((1, 2, 3, 4, 8, 40), range(1, 300), (None, 0, 1, 2)):
+        if K.deals_out(bf16, nkv, nkv, 128, 16, b, 1 << 15, spread):
+            assert b <= 256 // nkv <= 256
+
+
+def test_how_uneven_contexts_are():
+    assert _spread([5000] + [10] * 15) == 0                                         # up to 16 nothing goes by it
+    assert _spread([700] * 17) == 0 and _spread([13] * 17 + [18]) == 0
+    assert _spread([100] * 19 + [150]) == 1 and _spread([100] * 19 + [268]) == 1
+    assert _spread([100] * 19 + [280]) == 2 and _spread([1] * 40 + [4000]) == 2
