@@ -11,6 +11,7 @@ the true positions and nothing is padded.
 """
 from __future__ import annotations
 
+import functools
 import sys
 from dataclasses import dataclass, field
 from typing import Sequence
@@ -136,6 +137,8 @@ class Engine:
         self.graph_rows = 64        # steps of at most this many tokens in all run as rows of one token each,
         self.graph_row_reads = 1 << 18      # if the tokens of their portions read at most this many keys in all
         self._graph_pool = None
+        # (of the model alone: an engine that is let go must not wait for the collector of reference cycles)
+        self._step_choices = functools.lru_cache(maxsize=4096)(model.step_choices)
         self._has_windows = any(g.window is not None for g in groups)
 
     @classmethod
@@ -330,6 +333,9 @@ class Engine:
         kv_bound = -(-longest // 512) * 512
         # ... and how they deal out the keys by how uneven the contexts are (of little consequence up to 16 requests)
         spread = _spread([rc.num_tokens + 1 for rc in rcs])
+        if spread:
+            most = min([kv_bound] + [w * self.page_size for w in widths])
+            spread = _same_spread(lambda s: self._step_choices(self.page_size, rows, rows, most, s, None), spread)
         key = (rows, tuple(widths), (kv_bound, spread))
         plan = self._plan(self._decode_plans, key, lambda: _DecodePlan(self, rows, widths, kv_bound, spread=spread))
         plan.fill(rcs, tokens)
@@ -440,13 +446,11 @@ class Engine:
         # (steps with and without requests of one token have graphs of their own: the attention takes those requests
         # apart, in a kernel that the others need not launch; the padding's tokens go either way)
         singles = 1 in counts
-        # (the attention's shape for the portions goes by their longest context, in powers of two: a new prompt's portion beside
-        # long conversations is not one behind a prefix)
-        portion_kv = t_pad
+        # (the attention's shape for the portions goes by their longest context: a new prompt's portion beside long conversations is not
+        # one behind a prefix)
         longest = max((rc.num_tokens + n for rc, n in zip(rcs, counts) if n > 1), default=0)
-        while portion_kv < longest:
-            portion_kv *= 2
-        portion_kv = min([portion_kv] + [w * self.page_size for w in widths])
+        most = min(w * self.page_size for w in widths) if widths else 0
+        portion_kv = _same_portion(lambda n: self._step_choices(self.page_size, t_pad, b_pad, most, None, n), t_pad, longest, most)
         key = (t_pad, b_pad, r_pad, tuple(widths), singles, portion_kv)
         plan = self._plan(self._padded_plans, key, lambda: _PaddedPlan(self, t_pad, b_pad, r_pad, widths, singles, portion_kv))
         n_want = plan.fill(rcs, entries, counts)
@@ -460,6 +464,24 @@ def _spread(contexts: list[int]) -> int:
         return 0
     longest, total = max(contexts) * len(contexts), sum(contexts)
     return 2 if longest > 2.5 * total else 1 if longest > 1.4 * total else 0
+
+
+def _same_spread(choices, spread: int) -> int:
+    """The least `spread` for which the model's layers choose as for this one (`choices`: of a spread): what a step's graph is kept by."""
+    return next(s for s in range(spread + 1) if s == spread or choices(s) == choices(spread))
+
+
+def _same_portion(choices, tokens: int, longest: int, most: int) -> int:
+    """The greatest bound on the portions' contexts, from the step's tokens on in powers of two up to `most` (what the block tables hold),
+    for which the layers choose as for the least that holds `longest`."""
+    bound = tokens
+    while bound < longest:
+        bound *= 2
+    bound = min(bound, most)
+    chosen = choices(bound)
+    while bound < most and choices(min(2 * bound, most)) == chosen:
+        bound = min(2 * bound, most)
+    return bound
 
 
 def _capture(graph, pool, run):

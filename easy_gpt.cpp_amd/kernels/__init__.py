@@ -260,6 +260,10 @@ class KernelBackend:
         layers with as many kv heads and the same window."""
         raise NotImplementedError
 
+    def portion_choice(self, dtype, nq, nkv, hd, page_size, tokens, portion_kv):
+        """What paged_attention_mixed does otherwise for another `portion_kv` in a step of so many tokens, as a value to compare."""
+        return None
+
     def paged_attention_mixed(self, *args, ranges=None, portion_kv=None, **kwargs):
         """paged_attention with two hints: the table of `decode_ranges`, and the longest context of a request that brings
         more than one token."""

@@ -988,43 +988,8 @@ class HipKernels(KernelBackend):
                 # prompt portions (and mixed batches): key/value tiles shared through LDS by the wavefronts of
                 # a workgroup.  Few rows: small workgroups whose wavefronts split the keys, so that the GPU
                 # has enough of them; many rows: 64 rows per workgroup, which read the keys fewer times.
-                row_tiles = -(-t * (nq // nkv) // 16) * nkv
-                # Measured (us for one layer's prompt on a GPU that is warm; row tiles of 16 rows; shape = row tiles x key
-                # splits of a workgroup, 1xx the kernel of 32-row blocks, whose tiles of 64 keys must be whole pages):
-                #   head size 64, 14 heads on 2:   448 tiles 24: 9.4, 44: 10.4 |  896 tiles 24: 16.9, 44: 14.7, 142: 16.4
-                #     1,344 tiles 44: 20.0, 142: 21.3 | 1,792 tiles 44: 29.7, 142: 26.2 | 3,584 tiles 42: 76, 142: 53
-                #     7,168 tiles (8,192 tokens) 42: 292, 142: 175 | 28,560 tiles (32,640 tokens) 42: 3,840, 142: 2,400
-                #   head size 128, 12 heads on 2:  768 tiles 22: 31.0, 42: 26.1, 141: 27.8 | 1,536 tiles 42: 47.1, 141: 47.3
-                #     3,072 tiles 42: 158, 141: 87;  28 heads on 4: 896 tiles 22: 28.8, 42: 16.3, 141: 19.3 | 1,792 tiles
-                #     42: 40.7, 141: 30.0 | 7,168 tiles 42: 341, 141: 190;  40 heads on 8: 1,280 tiles 42: 23.2, 141: 19.6
-                blocks_of_32 = page_size <= 64
-                if hd == 64:
-                    shape = 24 if row_tiles <= 512 else 44 if row_tiles <= 1536 or not blocks_of_32 else 142
-                    if shape == 44 and row_tiles > 2048:
-                        shape = 42
-                else:
-                    shape = 22 if row_tiles <= 192 else 42 if row_tiles <= 1024 or not blocks_of_32 else 141
-                # Portions behind a prefix walk many keys per row and are few blocks of rows: the kernel of 32-row blocks
-                # with 128 rows to a workgroup, and the tiles of keys of a block of rows dealt over as many workgroups
-                # as give every CU one.  Measured (us, a layer; shape x workgroups that share the keys): head size 64,
-                # 14 heads on 2, 512 tokens behind 4,096 / 8,192 / 32,768 keys 24x1: 35 / 70 / 257, 124x1: 32 / 59 / 196,
-                # 142x1: 45 / 84 / 300, 142x4: 27 / 38 / 98; 256 tokens behind 32,768 124x1: 195, 124x4: 66, 142x8: 57; 64
-                # tokens 124x1: 201, 142x16: 40; behind 2,048 keys nothing is gained (24x1: 24, 142x4: 23) and a prompt
-                # without a prefix loses (2,048 tokens 142x1: 28, 142x2: 47); three portions of 512 behind 30,000 keys
-                # 142x1: 283, 124x1: 397.  Head size 128, 12 heads on 2, 512 tokens behind 2,048 / 32,768 keys 42x1: 59 /
-                # 643, 141x1: 59 / 665, 141x4: 30 / 185; 28 heads on 4: 141x1: 61 / 671, 141x2: 48 / 378; 40 heads on 8
-                # (160 workgroups): 141x1: 103 / 679.
-                key_splits = 1
-                # (behind a prefix: the portions' longest context is a few thousand tokens and at least twice the step's own.  Not the
-                # longest of all: one portion of 512 tokens of a new prompt beside 40 decoded tokens behind 128 to 2,048, 12 heads of
-                # 128 on 2: 51.8 us a layer in four key ranges, 48.0 in one; 8 behind 1,400 and 28 heads on 4 46.6 and 31.1)
                 longest = max_kv_len if portion_kv is None else min(portion_kv, max_kv_len)
-                if (blocks_of_32 and longest >= 2 * t
-                        and longest >= (self.prefix_keys if hd == 64 else self.prefix_keys // 2)):
-                    shape = 142 if hd == 64 else 141
-                    workgroups = -(-row_tiles // 8)
-                    tiles = -(-longest // (64 * (shape % 10)))
-                    key_splits = max(1, min(256 // workgroups, tiles // 4, 16))
+                shape, key_splits = self._portion_shape(t, nq, nkv, hd, page_size, longest)
                 # Requests that bring one token (decoded tokens beside the portions) go to the decode kernel in a second
                 # launch: here one workgroup would walk all of such a request's keys, 128 or 256 per iteration of some
                 # 1.7 us, and the longest of them sets the launch's time
@@ -1084,6 +1049,54 @@ class HipKernels(KernelBackend):
         self._run("egpt_paged_attention", qkv.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                   block_table.data_ptr(), width, q_start.data_ptr(), q_len.data_ptr(), kv_len.data_ptr(), b, t,
                   nq, nkv, hd, page_size, float(scale), int(window), dt, self._stream())
+
+    @classmethod
+    def _portion_shape(cls, t, nq, nkv, hd, page_size, longest) -> tuple[int, int]:
+        """(shape, workgroups that share the keys) of the attention of a step of t tokens with portions of prompts; `longest`: their
+        longest context."""
+        row_tiles = -(-t * (nq // nkv) // 16) * nkv
+        # Measured (us for one layer's prompt on a GPU that is warm; row tiles of 16 rows; shape = row tiles x key
+        # splits of a workgroup, 1xx the kernel of 32-row blocks, whose tiles of 64 keys must be whole pages):
+        #   head size 64, 14 heads on 2:   448 tiles 24: 9.4, 44: 10.4 |  896 tiles 24: 16.9, 44: 14.7, 142: 16.4
+        #     1,344 tiles 44: 20.0, 142: 21.3 | 1,792 tiles 44: 29.7, 142: 26.2 | 3,584 tiles 42: 76, 142: 53
+        #     7,168 tiles (8,192 tokens) 42: 292, 142: 175 | 28,560 tiles (32,640 tokens) 42: 3,840, 142: 2,400
+        #   head size 128, 12 heads on 2:  768 tiles 22: 31.0, 42: 26.1, 141: 27.8 | 1,536 tiles 42: 47.1, 141: 47.3
+        #     3,072 tiles 42: 158, 141: 87;  28 heads on 4: 896 tiles 22: 28.8, 42: 16.3, 141: 19.3 | 1,792 tiles
+        #     42: 40.7, 141: 30.0 | 7,168 tiles 42: 341, 141: 190;  40 heads on 8: 1,280 tiles 42: 23.2, 141: 19.6
+        blocks_of_32 = page_size <= 64
+        if hd == 64:
+            shape = 24 if row_tiles <= 512 else 44 if row_tiles <= 1536 or not blocks_of_32 else 142
+            if shape == 44 and row_tiles > 2048:
+                shape = 42
+        else:
+            shape = 22 if row_tiles <= 192 else 42 if row_tiles <= 1024 or not blocks_of_32 else 141
+        # Portions behind a prefix walk many keys per row and are few blocks of rows: the kernel of 32-row blocks
+        # with 128 rows to a workgroup, and the tiles of keys of a block of rows dealt over as many workgroups
+        # as give every CU one.  Measured (us, a layer; shape x workgroups that share the keys): head size 64,
+        # 14 heads on 2, 512 tokens behind 4,096 / 8,192 / 32,768 keys 24x1: 35 / 70 / 257, 124x1: 32 / 59 / 196,
+        # 142x1: 45 / 84 / 300, 142x4: 27 / 38 / 98; 256 tokens behind 32,768 124x1: 195, 124x4: 66, 142x8: 57; 64
+        # tokens 124x1: 201, 142x16: 40; behind 2,048 keys nothing is gained (24x1: 24, 142x4: 23) and a prompt
+        # without a prefix loses (2,048 tokens 142x1: 28, 142x2: 47); three portions of 512 behind 30,000 keys
+        # 142x1: 283, 124x1: 397.  Head size 128, 12 heads on 2, 512 tokens behind 2,048 / 32,768 keys 42x1: 59 /
+        # 643, 141x1: 59 / 665, 141x4: 30 / 185; 28 heads on 4: 141x1: 61 / 671, 141x2: 48 / 378; 40 heads on 8
+        # (160 workgroups): 141x1: 103 / 679.
+        key_splits = 1
+        # (behind a prefix: the portions' longest context is a few thousand tokens and at least twice the step's own.  Not the
+        # longest of all: one portion of 512 tokens of a new prompt beside 40 decoded tokens behind 128 to 2,048, 12 heads of
+        # 128 on 2: 51.8 us a layer in four key ranges, 48.0 in one; 8 behind 1,400 and 28 heads on 4 46.6 and 31.1)
+        if (blocks_of_32 and longest >= 2 * t
+                and longest >= (cls.prefix_keys if hd == 64 else cls.prefix_keys // 2)):
+            shape = 142 if hd == 64 else 141
+            workgroups = -(-row_tiles // 8)
+            tiles = -(-longest // (64 * (shape % 10)))
+            key_splits = max(1, min(256 // workgroups, tiles // 4, 16))
+        return shape, key_splits
+
+    @classmethod
+    def portion_choice(cls, dtype, nq, nkv, hd, page_size, tokens, portion_kv):
+        if dtype != _BF16 or hd not in (64, 128) or page_size & (page_size - 1) or page_size < 16:
+            return None
+        return cls._portion_shape(tokens, nq, nkv, hd, page_size, portion_kv)
 
     # A mixed step's requests of one token go to the decode kernel when the step's longest context is beyond this: the
     # second launch (and a third that combines key ranges) costs some 8 us, a workgroup of the tiled kernel that walks

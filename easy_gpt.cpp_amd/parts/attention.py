@@ -163,6 +163,14 @@ class GQAttention(Mixer):
         k.linear(attn, self.w_o, self.b_o, out)
         return out
 
+    def step_choices(self, page_size, tokens, requests, max_kv_len, spread, portion_kv):
+        k = kernels.backend()
+        heads = (self.w_qkv.dtype, self.n_heads, self.n_kv_heads, self.head_dim, page_size)
+        if spread is None:
+            return k.portion_choice(*heads, tokens, min(portion_kv, max_kv_len))
+        rot = self.position.rotary(self.w_qkv.device)
+        return rot is not None and rot[1] == self.head_dim and k.deals_out(*heads, requests, max_kv_len, spread)
+
     def _ranges(self, k, ctx, dtype, page_size, fused):
         """How the keys of the step's decoded tokens are dealt out, the same for all layers with these kv heads and this window; None
         where nothing goes by it (`fused`: in a step of decoded tokens alone, attention_decode_fused does)."""

@@ -238,6 +238,12 @@ class Mixer(Part):
     def state_need(self) -> StateNeed | None:
         return None
 
+    def step_choices(self, page_size: int, tokens: int, requests: int, max_kv_len: int, spread: int | None, portion_kv: int | None):
+        """What a step's hints decide in this part (`StepContext.spread` of decoded tokens alone, else None; `portion_kv` of a step with
+        portions of prompts), as a value to compare: steps of one size for which it is equal run the same kernels and can share a
+        captured graph.  None: the hints decide nothing."""
+        return None
+
     def forward(self, x: torch.Tensor, ctx: Any, cache: CacheView | None, state: StateView | None) -> torch.Tensor:
         raise NotImplementedError
 

@@ -229,6 +229,10 @@ class SideBySide(Mixer):
     def state_need(self):
         return next((b.state_need() for b in self.branches if b.state_need() is not None), None)
 
+    def step_choices(self, *step):
+        choices = tuple(b.step_choices(*step) for b in self.branches)
+        return choices if any(c is not None for c in choices) else None
+
     def param_specs(self):
         h = self.hidden_size
         specs = [s for b in self.branches for s in b.param_specs()]

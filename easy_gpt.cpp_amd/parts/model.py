@@ -103,6 +103,10 @@ class Model:
             for j, cid in enumerate(grp.cache_ids):
                 self.cache_location[cid] = (g, j)
 
+    def step_choices(self, *step) -> tuple:
+        """`Mixer.step_choices` of the layers."""
+        return tuple(block.mixer.step_choices(*step) for block in self.layers if block.mixer is not None)
+
     # ------------------------------------------------------------------ weights
     def parts(self):
         yield self.embedding

@@ -3,9 +3,12 @@ sizes; between and beyond those they choose speed, not results, but what they re
 kernels take.  Checked here over a grid of sizes, on the CPU (the rules are plain functions of the sizes)."""
 import itertools
 
+import pytest
 import torch
 
-from easy_gpt.cpp_amd.engine.engine import _spread
+from emulated_kernels import EmulatedKernels
+from easy_gpt.cpp_amd import kernels
+from easy_gpt.cpp_amd.engine.engine import _same_portion, _same_spread, _spread
 from easy_gpt.cpp_amd.kernels.hip import HipKernels as K
 
 BATCHES = [1, 2, 3, 7, 8, 16, 17, 31, 32, 33, 48, 63, 64, 65, 100, 128, 200, 256, 257, 512, 1000, 4096]
@@ -187,3 +190,56 @@ def test_how_uneven_contexts_are():
     assert _spread([700] * 17) == 0 and _spread([13] * 17 + [18]) == 0
     assert _spread([100] * 19 + [150]) == 1 and _spread([100] * 19 + [268]) == 1
     assert _spread([100] * 19 + [280]) == 2 and _spread([1] * 40 + [4000]) == 2
+
+
+def attention_of(dtype, heads, kv_heads, head_dim, window=None):
+    from easy_gpt.cpp_amd.parts import PartSpec, make_part
+
+    part = make_part("mixer", PartSpec("gq_attention", dict(n_heads=heads, n_kv_heads=kv_heads, head_dim=head_dim, qkv_bias=False, out_bias=False,
+                                                            window=window, position=PartSpec("rope_half_split", dict(theta=1e4))), "a."), hidden_size=64)
+    width = (heads + 2 * kv_heads) * head_dim
+    part.load(lambda name: torch.zeros((heads * head_dim if "q_proj" in name else kv_heads * head_dim, 64) if "o_proj" not in name
+                                       else (64, heads * head_dim)), dtype, "cpu")
+    assert part.w_qkv.shape == (width, 64)
+    return part
+
+
+class RulesOnly(EmulatedKernels):
+    deals_out, portion_choice = K.deals_out, K.portion_choice
+
+
+@pytest.fixture()
+def rules_only():
+    kernels.use_backend(RulesOnly())
+    yield
+    kernels.use_backend(None)
+
+
+def test_steps_with_the_same_kernels_are_kept_by_the_same_hints(rules_only):
+    bf16, f32 = torch.bfloat16, torch.float32
+    spread = lambda part, rows, most, s: _same_spread(lambda v: part.step_choices(16, rows, rows, most, v, None), s)  # noqa: E731
+    wide, narrow = attention_of(bf16, 12, 2, 128), attention_of(bf16, 14, 2, 64)
+    assert [spread(wide, 40, 2048, s) for s in (0, 1, 2)] == [0, 1, 1] and [spread(narrow, 40, 2048, s) for s in (0, 1, 2)] == [0, 0, 2]
+    for part, rows in ((attention_of(f32, 12, 2, 128), 40), (attention_of(bf16, 12, 2, 96), 40), (wide, 72), (attention_of(bf16, 40, 2, 64), 40)):
+        assert [spread(part, rows, 2048, s) for s in (0, 1, 2)] == [0, 0, 0]
+
+    def portion(part, tokens, longest, most):
+        return _same_portion(lambda n: part.step_choices(16, tokens, 8, most, None, n), tokens, longest, most)
+
+    # below the prefixes' line one bound for all, so a prompt of 2,048 tokens in portions of 512 has one graph
+    assert {portion(narrow, 512, n, 4096) for n in (512, 600, 1024, 1536, 2048)} == {2048}
+    assert {portion(wide, 512, n, 1024) for n in (512, 600, 1024)} == {1024}
+    # behind a prefix as many workgroups share the keys as there are CUs for, however far it goes
+    assert portion(wide, 512, 600, 4096) == 1024 and portion(wide, 512, 1536, 4096) == 4096 and portion(narrow, 512, 4000, 32768) == 32768
+    assert portion(narrow, 64, 2500, 32768) == 4096
+    assert {portion(attention_of(f32, 14, 2, 64), 512, n, 32768) for n in (512, 5000, 30000)} == {32768}
+    # always a bound, and the choice is that of the context's own bound
+    for part, tokens, most in itertools.product((wide, narrow), (64, 192, 512, 2048), (256, 1024, 4096, 32768)):
+        for longest in (1, 65, 500, 1025, 2048, 4097, 9000, 32768):
+            if longest <= most:
+                bound = portion(part, tokens, longest, most)
+                own = tokens
+                while own < longest:
+                    own *= 2
+                assert longest <= bound <= most
+                assert part.step_choices(16, tokens, 8, most, None, bound) == part.step_choices(16, tokens, 8, most, None, min(own, most))
