@@ -30,6 +30,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 
+from ..csrc.host_library import host_library
 from ..parts.base import CacheNeed
 
 
@@ -45,36 +46,6 @@ __all__ = ["CacheManager", "RequestCache", "OutOfPages", "NoFreeSlot"]
 
 EGH_NO_SLOT, EGH_BAD_HANDLE, EGH_OUT_OF_PAGES, EGH_BAD_ARGUMENT, EGH_NO_PAGE, EGH_INVARIANT = -1, -2, -3, -4, -5, -6
 _I32P = ctypes.POINTER(ctypes.c_int32)
-_lib = None
-
-
-def _library():
-    global _lib
-    if _lib is None:
-        from ..csrc import build
-
-        lib = ctypes.CDLL(build.ensure_host_built())
-        if lib.egh_abi_version() != 5:
-            raise RuntimeError("the host library has an unexpected ABI version")
-        vp, i = ctypes.c_void_p, ctypes.c_int
-        sigs = {
-            "egh_create": ([i, vp, vp, i, i], vp), "egh_destroy": ([vp], None), "egh_set_keep_first": ([vp, i, i], i), "egh_admit": ([vp], i),
-            "egh_release": ([vp, i], i), "egh_slot": ([vp, i], i), "egh_num_tokens": ([vp, i], i),
-            "egh_version": ([vp, i], i), "egh_table_len": ([vp, i, i], i), "egh_table": ([vp, i, i, vp, i], i),
-            "egh_pages_needed": ([vp, i, i, vp], i), "egh_free_pages": ([vp, i], i), "egh_used_pages": ([vp, i], i),
-            "egh_num_pages": ([vp, i], i), "egh_high_water": ([vp, i], i), "egh_free_slots": ([vp], i),
-            "egh_reserve": ([vp, i, vp, vp, vp], i), "egh_commit": ([vp, i, vp, vp], i), "egh_unreserve": ([vp, i, vp], i),
-            "egh_slot_index": ([vp, i, i, i], i), "egh_check": ([vp, vp, i], i),
-            "egh_fill_decode": ([vp, i, vp, vp, vp, vp, vp], i),
-            "egh_fill_decode_rows": ([vp, i, i, vp, vp, vp, vp, vp], i),
-            "egh_uniforms": ([i, vp, vp, vp, vp], None),
-            "egh_fill_step": ([vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp], i),
-        }
-        for name, (args, res) in sigs.items():
-            fn = getattr(lib, name)
-            fn.argtypes, fn.restype = args, res
-        _lib = lib
-    return _lib
 
 
 def _ints(values):
@@ -99,7 +70,7 @@ class RequestCache:
         """Per group: page ids in token order, -1 = given back."""
         if not self.live:
             return [[] for _ in self.table_lens]
-        lib, core = _library(), self._manager._core
+        lib, core = host_library(), self._manager._core
         out = []
         for g in range(len(self.table_lens)):
             n = lib.egh_table_len(core, self.handle, g)
@@ -111,7 +82,7 @@ class RequestCache:
     @property
     def version(self) -> int:
         """Changes whenever a table of the request changes."""
-        return _library().egh_version(self._manager._core, self.handle) if self.live else -1
+        return host_library().egh_version(self._manager._core, self.handle) if self.live else -1
 
 
 class PoolView:
@@ -150,7 +121,7 @@ class CacheManager:
             raise ValueError("one page count per group is needed")
         if any(n < 0 for n in counts):
             raise ValueError("num_pages must be >= 0")
-        self._lib = _library()
+        self._lib = host_library()
         windows = [int(g.window) if g.window is not None else 0 for g in self.groups]
         self._core = self._lib.egh_create(len(self.groups), _ints(windows), _ints(counts), self.page_size, int(max_requests))
         if not self._core:

@@ -173,7 +173,8 @@ class GQAttention(Mixer):
 
     def _ranges(self, k, ctx, dtype, page_size, fused):
         """How the keys of the step's decoded tokens are dealt out, the same for all layers with these kv heads and this window; None
-        where nothing goes by it (`fused`: in a step of decoded tokens alone, attention_decode_fused does)."""
+        where nothing goes by it (`fused`: in a step of decoded tokens alone, attention_decode_fused does).  (A context without the
+        hints, as a program that calls this part by itself may make, is taken here and below.)"""
         decoded = ctx.max_q_len == 1
         if not ctx.rows_independent or not (fused if decoded else getattr(ctx, "single_token_requests", True)):
             return None
