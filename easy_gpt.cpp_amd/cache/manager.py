@@ -136,8 +136,8 @@ class CacheManager:
 
     def __del__(self):
         core, self._core = getattr(self, "_core", None), None
-        if core and _lib is not None:
-            _lib.egh_destroy(core)
+        if core:
+            self._lib.egh_destroy(core)
 
     def _refresh(self) -> None:
         lib, core = self._lib, self._core
