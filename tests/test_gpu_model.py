@@ -380,21 +380,27 @@ def test_portions_behind_a_long_context_are_not_laid_out_as_rows(tiny_models):
     assert len(eng._row_plans) == 1
 
 
-def test_wide_layers_with_many_requests_replay_the_library_products_in_the_graph(tmp_path):
-    # 40 requests decoded side by side in a model whose gate/up and output matrices are wide enough for the library's
-    # product at this many rows: the captured graph then holds library nodes, is replayed step after step with the
-    # program's own work in between, and every replay is compared with the plain implementation
+def test_wide_layers_with_many_requests_replay_the_library_products_in_the_graph(tmp_path, monkeypatch):
+    # 40 requests decoded side by side in a model whose gate/up and output matrices are wide enough for the library's product at this
+    # many rows, and whose width of 520 the own kernel for so many rows does not take: the captured graph then holds library nodes, is
+    # replayed step after step with the program's own work in between, and every replay is compared with the plain implementation
     from easy_gpt.cpp_amd import kernels
     from easy_gpt.cpp_amd.weights import write_random_model
 
     cfg = {
-        "architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": 2, "hidden_size": 512,
-        "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "intermediate_size": 6160, "vocab_size": 12400,
+        "architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": 1, "hidden_size": 520,
+        "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "intermediate_size": 16144, "vocab_size": 12400,
         "rope_theta": 10000.0, "rms_norm_eps": 1e-6, "tie_word_embeddings": True, "max_position_embeddings": 64,
     }
     kernels.use_backend(None)
-    k = kernels.backend()
-    assert k._library_rows(40, 2 * 6160, 512) and k._library_rows(40, 12400, 512) and not k._library_rows(40, 512, 6160)
+    captured, mm = set(), torch.mm
+
+    def counted(x, w, **kw):
+        if torch.cuda.is_current_stream_capturing():
+            captured.add((x.shape[0], w.shape[1]))
+        return mm(x, w, **kw)
+
+    monkeypatch.setattr(torch, "mm", counted)
     sharp = str(tmp_path)              # plain random weights: this test is about the replays, not about far keys
     write_random_model(sharp, cfg, seed=9)
     n_req, prompt, steps = 40, 9, 7
@@ -411,6 +417,7 @@ def test_wide_layers_with_many_requests_replay_the_library_products_in_the_graph
     H.assert_rows_match(rows, ref, H.BF16_TOL, "library products in the decode graph")
     plans = list(eng._decode_plans.values())
     assert len(plans) == 1 and plans[0].graph is not None          # an eager visit, then replays
+    assert {n for rows, n in captured if rows == 40} == {2 * 16144, 12400}      # (the prompts' step has others)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
