@@ -378,7 +378,7 @@ template <int BM, int BN, int WM, int WN, int XB, int WB>
 int launch_rows(const void* x, const void* w, void* out, int m, int n, int k, int splits, int per, int kind, int act, hipStream_t s) {
     const long mt = (m + BM - 1) / BM, nt = kind == kRowsGated ? (n + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
     if (mt * nt * splits > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
-    // as many workgroups as the CUs hold, each taking its items in turn, where every item has the three steps that are on
+    // as many workgroups as the CUs hold, each taking its items in turn, where every item has the WB steps that are on
     // their way when it begins; else a workgroup per item
     constexpr int kHeld = kLdsOfCu / ((XB * BM + WB * BN) * 128);
     const int last_steps = k / kRowsStep - (splits - 1) * per;

@@ -169,7 +169,7 @@ __device__ uint32_t select_by_count(const float* __restrict__ w, int vocab, unsi
     int first_level = 3;
     {
         // The highest digit of a weight's pattern is its exponent (two exponents a bin), and the k-th largest
-        // weight is almost always within 2^-16 of the largest (1.0, digit 0x3f): count those eight bins in
+        // weight is almost always within 2^-15 of the largest (1.0, digit 0x3f): count those eight bins in
         // registers.  If the k-th weight is smaller still, the general histogram below takes over.
         unsigned int c[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
         for_each_in_row(w, vocab, threadIdx.x, blockDim.x, [&](int, float wj) {
@@ -355,11 +355,12 @@ __device__ uint32_t select_by_mass(const float* __restrict__ w, int vocab, uint3
 // All other rows: the weights are counted by exponent, then the tokens at or above the exponent below which none can be kept are
 // listed, in index order.  The selection runs on that list: one thread per candidate when they are at most kSampleThreads,
 // the row-walking selection otherwise.  A row for which neither cut is asked gets no list: the pieces' masses say in which
-// piece the drawn point lies, and that piece alone is walked.  Counted are the weights within 2^-16 of the largest, an exponent
+// piece the drawn point lies, and that piece alone is walked.  Counted are the weights within 2^-15 of the largest, an exponent
 // a bin, which hold the top-p mass of any distribution that is not nearly flat.
 //
-// 64 rows of 151,936, us: top-k 20, top-p 0.95 at 0.8 52 to 455 (rows whose k-th weight lay below 2^-16 of the largest had all
-// their vocabulary for candidates) -> 33; top-k 50 at 0.6 490 to 505 -> 38; one row of the former 31 -> 23; top-p alone 590 -> 230.
+// 64 rows of 151,936, us: top-k 20, top-p 0.95 at 0.8 52 to 455 (rows whose k-th weight lay below 2^-15 of the largest had all
+// their vocabulary for candidates) -> 34; top-k 50 at 0.6 500 -> 40; top-k 200 at 1.0 97 -> 62; top-p alone 541 -> 201; one row of the first
+// 30 -> 22.
 constexpr int kSamplePieces = 32;
 constexpr int kTopBins = 16;            // exponents 127 (weight 1.0) down to 112, one bin each; bin kTopBins: the rest
 

@@ -364,36 +364,41 @@ class HipKernels(KernelBackend):
         """Whether a bfloat16 product of more than 64 rows is the framework's own (gemm_rows.hip) instead of the
         library's first choice, whose times are the second ones here (us, weights from memory; without `unrounded` together
         with the norm that reads the result)."""
+        # (All lines were drawn with the kernel that had a workgroup per tile, where whole prompts put them: within a step a product by itself
+        # is not the measure, since what surrounds it changes with the form of its result.  The figures are of the kernel as it is, by
+        # itself, replayed from a graph; beyond a line it is ahead in places.)
         if unrounded:
-            # One float32 result, no split: 1,152 x 896 at 96 / 552 / 1,000 / 1,500 rows 6.6 / 7.0 / 8.8 / 9.4 against 7.9 / 8.7 / 10.0 /
-            # 10.1, at 2,048 12.0 against 11.4.  Wide or narrow ones are slower by themselves here and there (2,752 x 896 at 1,024
-            # and 1,536 rows 1.00 and 1.14 of the library's, 768 x 768 at 65 1.12), but the library fills the result with zeros first
-            # and takes the host longer: a design with states, whose steps run kernel by kernel, took 1,487 us for three prompts of
-            # 1,293 tokens with the library for these and 1,279 so, 1,166 and 1,098 for one of 85 (a width of 896).  A longer k: 1,152 x
-            # 1,152 at 96 / 300 / 1,500 rows 7.5 / 7.7 / 11.4 against 6.6 / 7.5 / 11.4, 2,048 x 1,536 9.0 / 9.3 / 17.9 against 7.7 / 9.6 /
-            # 16.3, 4,608 x 3,584 24.7 / 32.9 / 57.5 against 20.5 / 24.4 / 53.3.
+            # One float32 result, no split: 1,152 x 896 at 96 / 552 / 1,000 / 1,500 rows 6.7 / 7.2 / 8.9 / 9.5 against 7.6 / 8.4 / 9.8 /
+            # 9.8, at 2,048 12.4 against 11.2, 2,752 x 896 at 1,024 and 1,536 12.8 and 18.1 against 13.1 and 16.7, 768 x 768 at 65 6.2 against
+            # 6.5.  Besides, the library fills the result with zeros first and takes the host longer: a design with states, whose steps run
+            # kernel by kernel, took 1,487 us for three prompts of 1,293 tokens with the library for these and 1,279 so, 1,166 and 1,098 for
+            # one of 85 (a width of 896).  A longer k: 1,152 x 1,152 at 96 / 300 / 1,500 rows 7.7 / 7.9 / 11.1 against 6.3 / 7.2 / 11.2, 2,048 x
+            # 1,536 9.0 / 9.4 / 18.3 against 7.3 / 9.3 / 16.6, 4,608 x 3,584 18.0 / 29.3 / 59.4 against 20.5 / 24.1 / 56.7.
             return k <= 1024 and m <= 1536
         if k <= 1024:
-            # 896 x 896 at 96 / 300 / 1,500 / 2,048 rows 8.1 / 10.5 / 14.9 / 17.3 against 11.2 / 11.9 / 15.8 / 16.8 (within a prompt of 2,048
-            # tokens at the 0.5B sizes 1.9 us faster than the library: 3,801 us a step and 3,847), 512 x 1,024 at 1,536 / 2,800 0.94 / 1.09
-            # of the library's; 3,072 x 1,024 at 128 / 640 / 1,024 / 1,536 rows 0.93 / 0.97 / 1.02 / 1.19
+            # 896 x 896 at 96 / 300 / 600 / 1,500 / 2,048 rows 8.4 / 9.9 / 12.8 / 14.4 / 15.5 against 11.0 / 11.6 / 12.5 / 15.6 / 16.5, 1,024 x 1,024 at
+            # 1,200 / 2,048 / 3,000 / 5,000 13.7 / 16.9 / 21.2 / 30.8 against 15.3 / 18.0 / 20.4 / 28.1; 3,072 x 1,024 at 128 / 640 / 1,024 / 1,536 11.9 / 17.7 / 22.0 /
+            # 29.2 against 14.2 / 18.1 / 22.4 / 25.8
             return m <= (2048 if n < 2 * k else 1024)
-        # Below: whole prompts, us a layer that the library would take longer; within a step a product by itself is not the
-        # measure, since what surrounds it changes with the form of its result.
         if k >= 2 * n:
             # A long k range, which the library does not split, so that it falls behind the longer the range is.  896 x 4,864 at 70 / 300 /
-            # 1,000 / 2,048 / 3,500 / 5,000 tokens 4 / 6 / 5 / 2 / 4 / -24, 1,536 x 8,960 7 / 11 / 10 / 8 / 2 / -1, 2,048 x 11,008 12 / 18 / 23 / 12 /
-            # 20 / -39, 3,584 x 18,944 90 / 44 / 74 / 142 / 159 / 283; 1,024 x 3,072 3 / 5 / 1 / 0 / -2 / -5 (-3 at 1,500), 4,096 x 14,336 6 / 23 /
-            # 24 / 20 / -30 / -95, 5,120 x 13,824 5 / 31 / 31 / -26 / 271 / 228 (16 at 1,500).  Shorter ones by themselves, times over the
-            # library's: 1,024 x 2,048 at 300 / 448 / 1,000 rows 0.95 / 1.05 / 1.35, 1,024 x 4,096 at 1,000 / 1,500 0.94 / 1.19, 2,048 x
-            # 4,096 at 1,024 / 1,536 0.93 / 1.08.
+            # 1,000 / 2,048 / 3,500 / 5,000 / 8,191 rows 11.1 / 15.7 / 23.2 / 35.1 / 49.7 / 63.0 / 86.6 against 13.4 / 19.6 / 27.1 / 37.9 / 52.2 / 65.2 / 86.0;
+            # at 70 / 300 / 1,000 / 2,048 / 3,500 / 5,000 1,536 x 8,960 18.5 / 25.5 / 45.6 / 71.1 / 101 / 137 against 26.5 / 34.9 / 55.4 / 80.9 / 112 / 141,
+            # 2,048 x 11,008 23.2 / 32.6 / 65.6 / 95.4 / 151 / 214 against 32.6 / 50.3 / 83.8 / 112 / 170 / 198, 3,584 x 18,944 51.4 / 65.0 / 133 / 246 / 453 /
+            # 737 against 103 / 108 / 195 / 379 / 607 / 993, 4,096 x 14,336 45.4 / 61.1 / 117 / 212 / 377 / 591 against 53.8 / 80.0 / 145 / 231 / 330 / 504;
+            # 5,120 x 13,824 at 70 / 300 / 1,000 / 1,500 / 2,048 / 3,500 53.4 / 69.3 / 138 / 196 / 295 / 552 against 57.5 / 93.1 / 166 / 210 / 259 / 789.  Shorter
+            # ones: 1,024 x 3,072 at 300 / 1,000 / 1,500 / 3,500 13.2 / 20.2 / 25.6 / 37.5 against 15.7 / 20.3 / 24.5 / 37.0, 1,024 x 2,048 at 300 / 448 / 1,000
+            # 11.6 / 13.2 / 19.6 against 13.3 / 13.5 / 15.7, 1,024 x 4,096 at 1,000 / 1,500 22.6 / 29.8 against 23.6 / 27.9, 2,048 x 4,096 at 1,024 / 1,536 33.8 /
+            # 46.3 against 35.3 / 41.6.
             if k >= 8192 and k >= 5 * n:
                 return m <= 3584
             return m <= (320 if k < 3072 else 1024 if k < 4608 else 1536 if k < 3 * n else 2048)
-        # 1,536 x 1,536 at 70 / 200 / 450 / 1,500 tokens 2 / 1 / 0 / -3, 2,048 x 2,048 at 70 / 200 / 450 / 650 6 / 2 / 0 / -3, 3,072 x 3,072 at 70 /
-        # 300 / 450 / 2,048 4 / 1 / -6 / -10, 3,584 x 3,584 at 70 / 450 / 1,000 9 / 3 / -2, 5,120 x 5,120 3 / 11 / 4.  Wider than long ones by
-        # themselves, times over the library's: 4,608 x 3,584 at 200 / 300 / 448 rows 0.79 / 0.98 / 1.24, 4,096 x 2,048 at 128 / 200 / 320 0.88 /
-        # 1.12 / 1.24.
+        # 1,536 x 1,536 at 70 / 200 / 450 / 552 / 1,000 / 1,500 rows 11.2 / 12.0 / 15.2 / 17.6 / 19.7 / 23.9 against 11.8 / 12.7 / 14.9 / 15.0 / 19.8 / 22.9, 2,048 x
+        # 2,048 at 70 / 200 / 450 / 650 / 1,000 10.5 / 12.8 / 19.5 / 22.4 / 23.5 against 12.3 / 13.9 / 16.4 / 19.8 / 22.7, 3,072 x 3,072 at 70 / 300 / 450 / 2,048
+        # 15.3 / 22.9 / 27.1 / 62.9 against 21.0 / 23.8 / 27.2 / 55.9, 3,584 x 3,584 at 70 / 200 / 450 / 552 / 1,000 17.6 / 22.3 / 30.0 / 36.0 / 46.0 against 23.5 /
+        # 25.6 / 32.2 / 34.1 / 45.7, 5,120 x 5,120 at 70 / 300 / 450 / 1,000 28.9 / 37.8 / 46.6 / 70.3 against 28.2 / 43.4 / 52.4 / 75.1.  Wider than long ones:
+        # 4,608 x 3,584 at 200 / 300 / 448 26.1 / 30.3 / 38.2 against 39.4 / 31.4 / 35.6, 4,096 x 2,048 at 128 / 200 / 320 15.5 / 21.6 / 25.0 against
+        # 20.1 / 18.9 / 21.9.
         return m <= 448 if n <= k else n < 2 * k and m <= 256
 
     @staticmethod
@@ -412,21 +417,22 @@ class HipKernels(KernelBackend):
     @staticmethod
     def _own_short(m: int, n: int, k: int) -> bool:
         """Whether the product is the framework's own beyond the lines of `_own_rows`: with a short k range a tile is its beginning and its
-        end for the most part, and a workgroup's next tile begins under the end of the one before.  Drawn through 1,030 points (1,200 to
-        16,384 rows, k of 320 to 896, n from k / 2 to 9,728, rounded with its norm and unrounded; weights from memory, replayed from a graph):
-        the faster side within 1.5 % on average, where `_own_rows` alone loses 7 %.  The library goes in steps of its own, so beside a
-        line either side is ahead in places, by a third at worst.  us, own against the library's:
+        end for the most part, and a workgroup's next tile begins under the end of the one before.  Drawn through 1,260 points (1,200 to
+        16,384 rows, k of 64 to 1,024, n from k / 2 to 9,728, rounded with its norm and unrounded; weights from memory, replayed from a graph):
+        the faster side within 1.9 % on average, where `_own_rows` alone loses 7 %.  The library goes in steps of its own and loses a
+        quarter where n is no multiple of 128, so beside a line either side is ahead in places, by 1.4 at most.  us, own against the library's:
         k = 320 to 640: 512 x 512 rounded at 2,304 / 4,096 / 8,191 rows 11.8 / 13.9 / 21.5 against 14.6 / 15.9 / 23.0, 1,920 x 640 at 2,600 / 4,000 / 8,191 /
         16,384 26.4 / 34.0 / 58.5 / 117 against 27.7 / 39.3 / 76.4 / 146, unrounded 640 x 640 at 3,300 / 6,000 / 7,000 10.4 / 12.3 / 15.7 against 9.7 / 13.4 / 12.5.
         n up to k: 896 x 896 rounded at 2,048 / 2,600 / 4,000 / 5,000 / 6,000 / 7,000 / 8,191 / 12,000 / 16,384 15.6 / 18.9 / 21.9 / 28.4 / 31.0 / 33.2 / 35.4 / 46.5 /
         58.2 against 16.4 / 19.9 / 21.9 / 25.4 / 28.8 / 32.8 / 41.0 / 55.9 / 71.8, unrounded 768 x 768 at 2,600 / 3,300 / 5,000 / 7,000 / 12,000 9.3 / 11.7 / 13.3 /
         18.8 / 24.5 against 9.5 / 10.8 / 12.6 / 15.9 / 27.1.
         Wider: 2,688 x 896 rounded at 2,048 / 2,600 / 3,300 / 4,000 / 5,000 / 8,191 31.1 / 36.0 / 42.1 / 47.2 / 56.2 / 86.5 against 29.5 / 35.7 / 47.6 / 56.2 / 72.3 /
-        93.3, unrounded 20.2 / 21.4 / 26.3 / 27.0 / 32.6 / 50.2 against 17.0 / 19.3 / 27.9 / 36.8 / 44.6 / 49.7; 9,728 x 896 unrounded at 2,048 / 3,300 / 5,000 / 6,000 /
-        10,000 55.0 / 65.5 / 97.0 / 136 / 190 against 49.3 / 69.5 / 112 / 125 / 200.  A longer k is a tie at best: 1,024 x 1,024 at 4,096 / 5,000 / 8,191 23.8 / 30.8 /
+        93.3, unrounded 20.2 / 21.4 / 26.3 / 27.0 / 32.6 / 50.2 against 17.0 / 19.3 / 27.9 / 36.8 / 44.6 / 49.7; at 2,048 / 2,304 / 2,535 / 3,100 / 4,000 2,720 x 896
+        19.7 / 20.5 / 20.8 / 25.6 / 26.5 against 19.2 / 26.7 / 27.4 / 32.4 / 37.5, 2,816 x 896 19.8 / 20.5 / 20.9 / 25.8 / 26.7 against 16.6 / 17.9 / 20.7 / 27.1 / 27.7;
+        9,728 x 896 unrounded at 2,048 / 3,300 / 5,000 / 6,000 / 10,000 55.0 / 65.5 / 97.0 / 136 / 190 against 49.3 / 69.5 / 112 / 125 / 200.  A longer k is a tie at best: 1,024 x 1,024 at 4,096 / 5,000 / 8,191 23.8 / 30.8 /
         38.5 against 23.6 / 28.1 / 38.3; one to three steps of k leave nothing to begin under: 1,024 x 128 at 2,600 / 8,191 16.5 / 34.6 against 15.7 / 29.2,
         4,096 x 256 at the ends of what is measured 25.7 at 1,600 and 214 at 16,384 against 30.7 and 214."""
-        return 256 <= k <= 640 or (640 < k <= 896 and ((n <= k and m <= 2600) or m >= (3300 if 2 * n >= 3 * k else 7000)))
+        return 256 <= k <= 640 or (640 < k <= 896 and ((n <= k and m <= 2600) or m >= (2304 if 2 * n >= 3 * k else 7000)))
 
     @classmethod
     def _own_many(cls, m: int, n: int, k: int, unrounded: bool) -> bool:
@@ -436,22 +442,25 @@ class HipKernels(KernelBackend):
     @staticmethod
     def _own_gate(m: int, k: int) -> bool:
         """Whether gate, up and activation of more than 64 rows are one kernel (gemm_rows.hip) instead of the library's first
-        choice and an activation kernel, whose times are the second ones here (us, weights from memory)."""
+        choice and an activation kernel, whose times are the second ones here (us, weights from memory, replayed from a graph).  The lines
+        were drawn with the kernel that had a workgroup per tile, by whole prompts; beyond those by many rows it is the faster side
+        now."""
         if k <= 1536:
-            # 9,728 x 896 at 65 / 300 / 1,000 / 2,048 / 8,191 rows 12 / 15 / 27 / 53 / 181 against 15 / 20 / 39 / 66 / 198, 17,920 x
-            # 1,536 24 / 32 / 73 / 132 / 436 against 28 / 35 / 82 / 138 / 446 (at 16,384 rows 878 against 852), 8,192 x 1,024 10 / 16 /
-            # 24 / 39 / 154 against 16 / 20 / 30 / 44 / 156
+            # 9,728 x 896 at 65 / 300 / 1,000 / 2,048 / 8,191 rows 10.8 / 12.9 / 24.3 / 43.3 / 136 against 15.0 / 19.9 / 40.1 / 68.9 / 204, 17,920 x
+            # 1,536 21.3 / 30.1 / 65.2 / 123 / 379 against 28.1 / 36.9 / 90.7 / 146 / 470 (at 16,384 rows 746 against 899), 8,192 x 1,024 8.6 / 13.5 /
+            # 22.7 / 34.7 / 124 against 15.7 / 20.1 / 30.7 / 46.5 / 158
             return True
         if k < 3072:
-            # 4,096 x 2,048 at 65 / 300 / 1,000 / 2,048 / 5,500 rows 15 / 20 / 25 / 36 / 90 against 16 / 20 / 30 / 40 / 94.  Whole prompts,
-            # us a layer that the library would take longer: 22,016 x 2,048 at 70 / 300 / 1,200 / 2,048 / 5,000 tokens 0 / 2 / 7 / 31 /
-            # 10, 19,456 x 2,560 1 / 5 / -1 / 22 / 63.  But at 8,191 rows 12,288 x 2,048 370 against 341, 28,672 x 2,048 857 against 791.
+            # 4,096 x 2,048 at 65 / 300 / 1,000 / 2,048 / 5,500 rows 15.1 / 18.2 / 23.3 / 35.7 / 84.7 against 15.4 / 19.5 / 29.8 / 44.2 / 102, 22,016 x 2,048 at
+            # 70 / 300 / 1,200 / 2,048 / 5,000 28.7 / 42.6 / 103 / 161 / 368 against 31.1 / 47.9 / 114 / 202 / 431, 19,456 x 2,560 34.6 / 46.9 / 124 / 193 / 389 against
+            # 37.5 / 54.8 / 135 / 228 / 498.  (At 8,191 rows the kernel as it was lost: 12,288 x 2,048 370 against 341, 28,672 x 2,048 857 against 791;
+            # now 328 and 778 against 371 and 859.)
             return m <= 6144
-        # Large matrices.  With few rows they are a stream of w, which the library reads faster, and with very many rows its larger
-        # tiles lose less at their edges.  Whole prompts, us a layer that the library would take longer: 37,888 x 3,584 at 70 / 128 / 200 /
-        # 500 / 1,200 / 2,500 / 3,500 tokens -6 / -1 / 9 / 8 / 106 / 35 / -36, 16,384 x 3,072 -8 / -7 / 3 / 3 / 2 / 90 / -6, 27,648 x 5,120 at
-        # 128 / 500 / 2,048 / 3,500 0 / 24 / 30 / -23.  Where all rows of w begin at the same place of 8 KB the library is as good or
-        # better: 12,288 x 4,096 at 128 / 300 / 1,200 / 2,048 -5 / -8 / 0 / -16, 28,672 x 4,096 1 / 1 / -31 / -34.
+        # Large matrices.  With few rows they are a stream of w, which the library reads faster: 16,384 x 3,072 at 70 / 128 / 200 / 500 / 1,200 /
+        # 2,500 / 3,500 rows 37.2 / 39.2 / 36.9 / 54.6 / 117 / 224 / 294 against 29.6 / 34.7 / 42.7 / 63.5 / 126 / 321 / 319, 37,888 x 3,584 72.3 / 76.9 / 86.6 / 130 / 274 /
+        # 529 / 758 against 75.4 / 80.1 / 90.4 / 155 / 385 / 596 / 829, 27,648 x 5,120 at 128 / 500 / 2,048 / 3,500 95.0 / 124 / 489 / 743 against 74.2 / 155 / 514 / 788.
+        # Where all rows of w begin at the same place of 8 KB the library is as good or better: 12,288 x 4,096 at 128 / 300 / 1,200 / 2,048 39.1 /
+        # 58.8 / 98.4 / 190 against 37.8 / 58.4 / 106 / 180, 28,672 x 4,096 79.4 / 85.1 / 285 / 402 against 61.1 / 88.3 / 276 / 412.
         return 128 < m <= 3072 and k % 4096 != 0
 
     def linear(self, x, w, bias, out):

@@ -51,7 +51,7 @@ def test_which_rows_go_to_the_library_is_monotonic_in_the_rows():
 
 
 def test_products_of_many_rows_leave_their_kernel_where_the_library_is_faster():
-    # (rows, n, k) with both sides measured more than the runs differ
+    # (rows, n, k) with both sides measured more than the runs differ when the lines were drawn
     own = [(96, 896, 896), (300, 1152, 896), (2048, 896, 896), (200, 512, 1024), (1000, 1024, 1024), (128, 1536, 1536), (200, 2048, 2048),
            (200, 3584, 3584), (200, 4608, 3584), (450 - 2, 5120, 5120), (300, 1024, 2048), (1000, 1024, 4096), (650, 1024, 3072), (1500, 896, 4864),
            (640, 2048, 5632), (1500, 5120, 13824), (2048, 4096, 14336), (3500, 2048, 11008), (3584, 3584, 18944)]
@@ -72,7 +72,7 @@ def test_products_of_many_rows_leave_their_kernel_where_the_library_is_faster():
 
 
 def test_gate_and_up_leave_their_kernel_where_the_library_is_faster():
-    # (rows, k) with both sides measured more than the runs differ, over matrices of 4,096 to 37,888 rows
+    # (rows, k) with both sides measured more than the runs differ when the lines were drawn, over matrices of 4,096 to 37,888 rows
     for m, k in [(65, 896), (2048, 896), (8191, 896), (1000, 1024), (96, 1536), (2500, 1536), (500, 2048), (2048, 2048), (2500, 2560), (200, 3584),
                  (1200, 3584), (2048, 3584), (2500, 3072), (500, 5120)]:
         assert K._own_gate(m, k), (m, k)
