@@ -19,6 +19,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "lds_loads.h"
 
 namespace egpt {
 
@@ -528,17 +529,21 @@ __global__ __launch_bounds__(64 * RT * KS) void attention_tiled_kernel(
 
 // Prompt portions, 32 rows to a wavefront.  The same arithmetic as attention_tiled_kernel with the 32 x 32 x 16 matrix
 // instruction: a wavefront takes a block of 32 rows and 64 keys of each tile, S^T[32 keys, 32 rows] = K Q^T leaves a lane
-// 16 scores of one row (row = lane % 32; the lane's half h = lane / 32 holds keys 8b + 4h + v of a block of 32, b and v
-// in 0..3), and the probabilities are again the second product's operand as they lie: for its step over 16 keys a lane
-// supplies eight of them, the same eight that it holds, so a page's values are staged into LDS in that order (within 16
-// keys: [h][b % 2][v]).  Against the kernel of 16-row tiles, a score costs half the matrix instructions, half the LDS
-// reads and half the staging and loop instructions; what is left per score is its exponential, a multiply-add, a
-// maximum and half a conversion, and the kernel is bound by the issue of these vector instructions (an exponential
-// takes a wavefront's issue slot for about 8.5 cycles, the others for 4.4, a matrix instruction for 8 of its 32: with
-// 32 scores to a lane and tile that is about 1,000 cycles a wavefront and tile, against 640 of the matrix cores), so
-// the loop below is built to keep the vector pipe issuing while the matrix cores work.  A workgroup takes RB blocks
+// 16 scores of one row (row = lane % 32), and the probabilities are again the second product's operand as they lie.  Against
+// the kernel of 16-row tiles, a score costs half the matrix instructions and half the LDS reads; what is left per score is its
+// exponential, a multiply-add, half a maximum and half a conversion.  A workgroup takes RB blocks
 // of rows; KS wavefronts per block split each tile of 64 * KS keys and are combined through LDS at the end.  The tiles
 // of 64 keys must be whole pages (page sizes 16, 32, 64).
+//
+// What bounds it: the vector instructions of the softmax.  A block of 32 rows and 64 keys is 100 of them (an exponential takes a
+// wavefront's issue slot for about 8.5 cycles, the others for 4.4: some 800 cycles with the matrix instructions of the SIMD's other
+// wavefront between them), against 640 cycles of the matrix cores at head size 64 and 1,152 at 128.  With two wavefronts to a SIMD
+// that take matrix and vector instructions in turns a step of both takes 1,000 to 1,300 cycles.  What it was before: one straight line of
+// code that alternated matrix and vector instructions, keys and values through registers into LDS (84 more vector instructions
+// a block, bank conflicts, every load waited for in front of the iteration's barrier), four wavefronts a CU at head size 128, and a
+// block without rows masked in every tile, by which a prompt whose last rows fill their workgroup badly took half as long again.  us a
+// layer: 14 heads of 64 on 2, 2,048 / 6,000 / 8,191 tokens 25.9 / 117 / 171 -> 25.1 / 96 / 146; 12 heads of 128 on 2, 1,024 / 2,048 / 5,000
+// 25.9 / 47.2 / 136 -> 21.0 / 32.8 / 88.6; 28 on 4, 1,024 / 2,048 / 5,000 29.5 / 72.9 / 289 -> 22.6 / 46.0 / 178.
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;      // (native vectors: arrays of them stay in registers)
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
@@ -572,21 +577,23 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     constexpr int FB = HD / 32;                  // blocks of 32 output features
     constexpr int ROWS = 32 * RB;
     constexpr int KT = 64 * KS;                  // keys per LDS tile
-    constexpr int KROW = HD + 8, VROW = KT + 8;  // padded rows (bf16 elements)
-    constexpr int THREADS = 64 * RB * KS;
-    constexpr int CH = HD / (8 * RB);            // 16-byte chunks per thread and tile, of keys and of values
-    constexpr int STAGE = KT * KROW + HD * VROW;
+    constexpr int GROUP = 16 * HD * 2;           // bytes of 16 keys (or of their values)
+    constexpr int SLOT = KT * HD * 2;            // bytes of a tile of keys (or of values)
     constexpr int PER_LANE = FB * 16 + 2;        // floats a lane leaves for the combination
-    constexpr int COMBINE = (KS - 1) * RB * 64 * PER_LANE * 2;    // in bf16 elements
-    static_assert(CH >= 1 && HD % (8 * RB) == 0, "a thread takes whole chunks");
-    __shared__ __attribute__((aligned(16))) bf16_t smem[(2 * STAGE > COMBINE) ? 2 * STAGE : COMBINE];
-    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    constexpr int COMBINE = (KS - 1) * RB * 64 * PER_LANE * 4;
+    constexpr int LOADS = HD / 32, N_LOADS = 4 * LOADS / RB;     // loads of a group; of a tile's keys (and values) by a wavefront
+    constexpr int OWN = N_LOADS > LOADS ? N_LOADS / LOADS : 1;   // groups that they are of
+    static_assert(N_LOADS * RB == 4 * LOADS && (N_LOADS % LOADS == 0 || LOADS % N_LOADS == 0), "a tile is whole loads");
+    // keys, slots 0 and 1, then values, slots 0 to 2
+    __shared__ __attribute__((aligned(128))) char smem[(5 * SLOT > COMBINE) ? 5 * SLOT : COMBINE];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int rb = wave % RB, ksi = wave / RB;
     const int lr = lane % 32, lh = lane / 32;
-    const int kh = blockIdx.y;
+    // (the kv heads of a block of rows after each other, so that all heads' last rows, which have the most keys, begin first)
+    const int kh = blockIdx.x % nkv;
     const int group_size = nq / nkv;
 
-    int b = 0, grp = blockIdx.x;
+    int b = 0, grp = blockIdx.x / nkv;
     for (; b < n_seqs; ++b) {
         // (skip_single: requests of one token are the decode kernel's, which spreads their keys over wavefronts)
         const int groups = (skip_single && q_len[b] == 1) ? 0 : (q_len[b] * group_size + ROWS - 1) / ROWS;
@@ -661,10 +668,13 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     float m_run = -INFINITY;                  // the maximum in units of the raw scores
     // the rows' sums of probabilities come from the matrix cores: a block of "values" whose first feature is all ones
     // (the lanes lane % 32 == 0 hold it) gives them as feature 0 of one more output block, element 0 of the lanes of
-    // half 0 (32 additions per step on the vector pipe, which this kernel waits for, against four matrix instructions)
-    f32x16 o_sum;
+    // half 0 (32 additions per step on the vector pipe against four matrix instructions); in SUMS chains
+    constexpr int SUMS = HD == 64 ? 2 : 1;
+    f32x16 o_sum[SUMS];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o_sum[e] = 0.f;
+    for (int c = 0; c < SUMS; ++c)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o_sum[c][e] = 0.f;
     bf16x8 ones;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ones[e] = static_cast<__bf16>(lr == 0 ? 1.0f : 0.0f);
@@ -672,263 +682,269 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
 #pragma unroll
     for (int e = 0; e < 16; ++e) zero16[e] = 0.f;
 
-    // The loop is a pipeline of three stages over the tiles.  In the iteration of tile i a wavefront issues, as one
-    // straight line of code, the score product of tile i + 1, the exponentials of tile i and the output product of tile
-    // i - 1: the matrix instructions of the two products alternate with the vector instructions of the softmax between
-    // them (in groups whose order scheduling fences keep), so that both pipes work at once.  (With a tile's products on
-    // either side of its softmax, and the wavefronts of a workgroup in step from barrier to barrier, the pipes took
-    // turns: at 8,192 tokens the SIMDs issued vector instructions half of the time and did nothing for much of the
-    // rest.)  What does not fit into a straight
-    // line is kept out of it: masking (tiles on the diagonal or a window's edge) comes before it, and the accumulated
-    // output is rescaled after it, and only when a row's maximum has grown by more than 2^kSlack since the last time:
+    // A tile is two steps of a wavefront: the matrix instructions (the scores of tile i, the output of tile i - 1), then the vector
+    // instructions (the probabilities of tile i).  The two wavefronts of a SIMD take them in turn: wavefronts 4 to 7 are one
+    // step behind, so that one of the two is at its matrix instructions while the other is at its vector instructions, and a
+    // barrier behind every step keeps them so.
+    // The accumulated output is rescaled only when a row's maximum has grown by more than 2^kSlack since the last time:
     // until then the exponentials are taken against the old maximum, so they may reach 2^kSlack instead of 1, which
     // float32 sums and bfloat16 probabilities (the same relative precision at any magnitude) do not mind.
-    // LDS holds the keys of tiles i + 1 and i + 2 and the values of tiles i - 1 and i, two slots each; the keys of tile
-    // i + 3 and the values of tile i + 1 are on their way from memory meanwhile.
+    // Keys and values go from memory straight to LDS, 16 keys (never more than a page's) to a load's base address and a
+    // constant of the lane beside it, so that they cost no vector instructions and no registers.  A wavefront that issues a load waits
+    // until the memory pipe takes it, some 100 cycles when all issue theirs at once, so they are spread over both steps: the
+    // keys of tile i + 1 go out in the first wavefronts' matrix step of tile i (when everybody has read the keys of tile i - 1) and the
+    // values of tile i + 1 in the step behind it, with a third slot so that they have two steps and more to arrive as well.
     constexpr float kSlack = 8.0f;
+    constexpr bool TURNS = RB * KS == 8;
+    const bool second = TURNS && wave >= 4;
     const int page_mask = page_size - 1;             // page sizes here are powers of two
-    const int k_row = tid / RB, k_col = (tid % RB) * CH * 8;                 // key within the tile, first feature
-    const int v_key = (tid % (KT / 8)) * 8, v_row = tid / (KT / 8);          // first of eight keys, feature (+ 8 RB u)
-    // where a run of eight keys goes within its 16 keys of a value row: the first four to half 0, the others to half 1
-    const int v_pos = (v_key / 16) * 16 + ((v_key % 16) / 8) * 4;
-    // Loads without branches, so that they can stand in the straight line: a thread's key row and its run of eight
-    // values lie at the same place of their page in every tile (a tile is whole pages), so a load's address is the
-    // page's number times the pages' stride plus a constant of the thread.  The index into the block table is clamped
-    // to the pages that hold the workgroup's keys, so every load reads memory of this request; what lies outside the
-    // keys that the rows see is replaced by zeros when a tile at either end is put into LDS.
-    u32x4 k_regs[CH], v_regs[CH];
-    int k_page, v_page;
-    const long page_stride = static_cast<long>(nkv) * page_size * HD;
-    const bf16_t* const k_base = k_cache + (static_cast<long>(kh) * page_size + (k_row & page_mask)) * HD + k_col;
-    const bf16_t* const v_base = v_cache + (static_cast<long>(kh) * HD + v_row) * page_size + (v_key & page_mask);
+    // A row of a group of keys lies in LDS as pieces of 16 bytes, exchanged by the row's number (piece p of row r in place
+    // p ^ (r / 2 & 7)), a feature of a group of values as two pieces, exchanged by the feature's (p ^ (f / 8 & 1)): lanes that
+    // read one piece of many rows then hit different banks.  A load puts a lane's 16 bytes at its base + 16 x lane, so the
+    // exchange is made in the addresses that lanes load from.
+    constexpr int PIECES = HD / 8;                   // of a key's row
+    const int load0 = wave * N_LOADS, group0 = load0 / LOADS;    // this wavefront's first load of a tile, and its group
+    int k_off[N_LOADS];
+#pragma unroll
+    for (int i = 0; i < N_LOADS; ++i) {
+        const int row = (load0 + i) % LOADS * (64 / PIECES) + lane / PIECES;
+        k_off[i] = row * HD * 2 + (((lane % PIECES) ^ (row / 2 & 7)) * 16);
+    }
+    const int v_piece = (lane % 2) ^ (lane / 16 & 1);        // (feature lane / 2 of a load's 32)
+    const int v_off = (lane / 2) * page_size * 2 + v_piece * 16;
+    const int v_step = 32 * page_size * 2;
+    const size_t page_bytes = static_cast<size_t>(nkv) * page_size * HD * 2, head_bytes = static_cast<size_t>(page_size) * HD * 2;
+    const char* const k_head = reinterpret_cast<const char*>(k_cache) + kh * head_bytes;
+    const char* const v_head = reinterpret_cast<const char*>(v_cache) + kh * head_bytes;
+    // The page numbers of a wavefront's groups of a tile, by scalar loads (constant address space: no other instruction here writes the
+    // block table).  The index into it is clamped to the pages that hold the workgroup's keys, so every load reads memory of this
+    // request.
     const int idx_lo = blk_lo >> page_shift, idx_hi = blk_p_hi >> page_shift, idx_step = KT >> page_shift;
-    const int k_sub = k_row >> page_shift, v_sub = v_key >> page_shift;
-    auto clamped = [&](int idx) { return min(max(idx, idx_lo), idx_hi); };
-    auto lookup_k = [&](int tile) { k_page = max(table[clamped(tile * idx_step + k_sub)], 0); };
-    auto lookup_v = [&](int tile) { v_page = max(table[clamped(tile * idx_step + v_sub)], 0); };
-    auto fetch_k = [&]() {
-        const bf16_t* src = k_base + k_page * page_stride;
-#pragma unroll
-        for (int u = 0; u < CH; ++u) k_regs[u] = *reinterpret_cast<const u32x4*>(src + u * 8);
+    const auto* const table_c = reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(table));
+    struct Pages {
+        int of[OWN];
     };
-    auto fetch_v = [&]() {
-        const bf16_t* src = v_base + v_page * page_stride;
+    auto lookup = [&](int tile) {
+        Pages p;
 #pragma unroll
-        for (int u = 0; u < CH; ++u)
-            v_regs[u] = *reinterpret_cast<const u32x4*>(src + static_cast<long>(u) * (8 * RB) * page_size);
+        for (int i = 0; i < OWN; ++i) {
+            const int idx = tile * idx_step + ((group0 + i) * 16 >> page_shift);
+            p.of[i] = table_c[min(max(idx, idx_lo), idx_hi)];
+        }
+        return p;
     };
-    auto at_an_end = [&](int tile) { return tile * KT < blk_lo || tile * KT + KT - 1 > blk_p_hi; };
-    auto trim_k = [&](int tile) {            // zeros for the keys of this tile that no row of the workgroup sees
-        if (at_an_end(tile)) {
-            const int kk = tile * KT + k_row;
-            if (!(kk <= blk_p_hi && kk >= blk_lo)) {
+    auto load_k = [&](const Pages& pages, int i, int slot) {
+        const int g = (load0 + i) / LOADS;
+        const unsigned page = max(pages.of[i / LOADS], 0);
+        load_to_lds(buffer_of(k_head + page * page_bytes, head_bytes), k_off[i], (g * 16 & page_mask) * (HD * 2), smem + slot * SLOT + (load0 + i) * 1024);
+    };
+    auto load_v = [&](const Pages& pages, int i, int slot) {
+        const int g = (load0 + i) / LOADS, u = (load0 + i) % LOADS;
+        const unsigned page = max(pages.of[i / LOADS], 0);
+        load_to_lds(buffer_of(v_head + page * page_bytes, head_bytes), v_off, (g * 16 & page_mask) * 2 + u * v_step,
+                    smem + (2 + slot) * SLOT + (load0 + i) * 1024);
+    };
+    // Zeros for the values of this tile that no row of the workgroup sees (their probabilities are zeros, but what lies in the
+    // page may be no number): every lane those that it loaded.
+    auto trim_v = [&](int slot, int tile) {
+        if (tile * KT >= blk_lo && tile * KT + KT - 1 <= blk_p_hi) return;
+#pragma unroll 1
+        for (int i = 0; i < N_LOADS; ++i) {
+            const int key = tile * KT + (load0 + i) / LOADS * 16 + v_piece * 8;
+            u32x4* at = reinterpret_cast<u32x4*>(smem + (2 + slot) * SLOT + (load0 + i) * 1024 + lane * 16);
+            u32x4 v = *at;
 #pragma unroll
-                for (int u = 0; u < CH; ++u) k_regs[u] = u32x4{0u, 0u, 0u, 0u};
-            }
+            for (int e = 0; e < 8; ++e)
+                if (key + e < blk_lo || key + e > blk_p_hi) v[e / 2] &= e % 2 ? 0x0000ffffu : 0xffff0000u;
+            *at = v;
         }
     };
-    auto trim_v = [&](int tile) {
-        if (at_an_end(tile)) {
-            const int vk = tile * KT + v_key;
-            if (!(vk <= blk_p_hi && vk + 7 >= blk_lo)) {
+    Pages pages, next_pages;                         // of the tile whose loads go out next, and of the one behind it
+    int k_slot = 0, v_slot = 0;                      // of the tile that is multiplied
+    auto after = [](int v) { return v == 2 ? 0 : v + 1; };
+    // behind a tile's second step: the next tile's keys and this one's values are there (the next one's values need not be)
+    auto loads_arrived = [&](int tile) {
+        arrived<N_LOADS>();
+        trim_v(v_slot, tile);
+    };
+    // Row lr of a block of 32 keys, as the matrix instruction sees it, is the key whose number has bits 2 and 3 of lr exchanged: a
+    // lane's scores are then those of keys 16 b + 8 h + v (v in 0..7), the run of eight whose values it supplies to the
+    // second product in the order in which a page holds them.
+    const int k_lr = (lr & 0x13) | (lr & 4) << 1 | (lr & 8) >> 1;
+    int k_get[4];                                    // (in the slot of the next keys to be read; the slots are exchanged by a bit)
 #pragma unroll
-                for (int u = 0; u < CH; ++u) v_regs[u] = u32x4{0u, 0u, 0u, 0u};
+    for (int j = 0; j < 4; ++j) k_get[j] = (ksi * 64 + k_lr) * (HD * 2) + (((2 * j + lh) ^ (k_lr / 2 & 7)) * 16);
+    const int v_lane = 2 * SLOT + ksi * 4 * GROUP + lr * 32 + ((lh ^ (lr / 8 & 1)) * 16);
+    int v_get = v_lane + 2 * SLOT;                   // (the slot of the values of the tile before)
+    // The matrix instructions of a step, in order: the rows' sums of tile i - 1, which take nothing from LDS, the scores of tile i,
+    // the output of tile i - 1.  (Consecutive ones go to different accumulators: one that adds to the result of the one before it
+    // would wait for it.)  Operands are read AHEAD instructions ahead.
+    constexpr int N_QK = 2 * NQ, N_PV = 4 * FB, N_LDS = N_QK + N_PV, AHEAD = 6;
+    f32x16 acc[2];
+    bf16x8 pb[4];
+    auto matrix_step = [&](auto&& load) {
+        u32x4 operand[AHEAD];
+        auto read_operand = [&](auto m_c) {
+            constexpr int m = decltype(m_c)::value;
+            if constexpr (m < N_QK)
+                operand[m % AHEAD] = *reinterpret_cast<const u32x4*>(smem + k_get[m / 2 % 4] + m % 2 * 32 * (HD * 2) + m / 8 * 128);
+            else if constexpr (m < N_LDS)
+                operand[m % AHEAD] = *reinterpret_cast<const u32x4*>(smem + v_get + (m - N_QK) / FB * GROUP + (m - N_QK) % FB * 1024);
+        };
+        auto sum = [&](int t) {
+            o_sum[t % SUMS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb[t], o_sum[t % SUMS], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        __builtin_amdgcn_s_setprio(1);
+        static_for<AHEAD>(read_operand);
+        __builtin_amdgcn_sched_barrier(0);
+        sum(0);
+        if constexpr (SUMS == 2) sum(1), sum(2), sum(3);
+        static_for<N_LDS>([&](auto m_c) {
+            constexpr int m = decltype(m_c)::value;
+            const bf16x8 from_lds = __builtin_bit_cast(bf16x8, operand[m % AHEAD]);
+            if constexpr (m < N_QK)
+                acc[m % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(from_lds, q[m / 2], m < 2 ? zero16 : acc[m % 2], 0, 0, 0);
+            else
+                o[(m - N_QK) % FB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(from_lds, pb[(m - N_QK) / FB], o[(m - N_QK) % FB], 0, 0, 0);
+            read_operand(std::integral_constant<int, m + AHEAD>{});
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (SUMS == 1 && m < N_QK && m % 4 == 3 && m / 4 < 3) sum(m / 4 + 1);
+            if constexpr (m % (N_LDS / N_LOADS) == 1) {
+                load(m / (N_LDS / N_LOADS));
+                __builtin_amdgcn_sched_barrier(0);
             }
-        }
-    };
-    // the slots: keys [2][KT][KROW], then values [2][HD][VROW]
-    constexpr int KSLOT = KT * KROW, VSLOT = HD * VROW;
-    static_assert(2 * (KSLOT + VSLOT) == 2 * STAGE, "the slots fill the two stages");
-    bf16_t* const k_put[2] = {smem + k_row * KROW + k_col, smem + KSLOT + k_row * KROW + k_col};
-    bf16_t* const v_put[2] = {smem + 2 * KSLOT + v_row * VROW + v_pos, smem + 2 * KSLOT + VSLOT + v_row * VROW + v_pos};
-    const bf16_t* const k_get[2] = {smem + (ksi * 64 + lr) * KROW + lh * 8, smem + KSLOT + (ksi * 64 + lr) * KROW + lh * 8};
-    const bf16_t* const v_get[2] = {smem + 2 * KSLOT + lr * VROW + ksi * 64 + lh * 8,
-                                    smem + 2 * KSLOT + VSLOT + lr * VROW + ksi * 64 + lh * 8};
-    auto stash_k = [&](auto slot_c) {
-        constexpr int slot = decltype(slot_c)::value;
+        });
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
-        for (int u = 0; u < CH; ++u) *reinterpret_cast<u32x4*>(k_put[slot] + u * 8) = k_regs[u];
-    };
-    auto stash_v = [&](auto slot_c) {
-        constexpr int slot = decltype(slot_c)::value;
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            bf16_t* vp = v_put[slot] + u * 8 * RB * VROW;
-            *reinterpret_cast<u32x2*>(vp) = u32x2{v_regs[u][0], v_regs[u][1]};
-            *reinterpret_cast<u32x2*>(vp + 8) = u32x2{v_regs[u][2], v_regs[u][3]};
-        }
-    };
-    // the scores of a tile from a key slot
-    auto scores = [&](auto slot_c, f32x16 (&acc)[2]) {
-        constexpr int slot = decltype(slot_c)::value;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-            for (int j = 0; j < NQ; ++j) {
-                const u32x4 kk = *reinterpret_cast<const u32x4*>(k_get[slot] + kb * 32 * KROW + j * 16);
-                acc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kk), q[j],
-                                                                  j == 0 ? zero16 : acc[kb], 0, 0, 0);
-            }
-        }
-    };
-    // the output product of a tile from a value slot
-    auto outputs = [&](auto slot_c, const bf16x8 (&pb)[4]) {
-        constexpr int slot = decltype(slot_c)::value;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) o_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb[t], o_sum, 0, 0, 0);
-#pragma unroll
-        for (int f = 0; f < FB; ++f)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const u32x4 a = *reinterpret_cast<const u32x4*>(v_get[slot] + f * 32 * VROW + t * 16);
-                o[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), pb[t], o[f], 0, 0, 0);
-            }
+        for (int j = 0; j < 4; ++j) k_get[j] ^= SLOT;
+        v_get = v_lane + v_slot * SLOT;
     };
     const float slack = kSlack / scale2;
-    // Iteration of tile i, whose parity relative to the first tile is PAR.  The keys of tile i + 1 lie in key slot
-    // PAR ^ 1, the values of tile i - 1 in value slot PAR ^ 1; `cur` holds the scores of tile i, `nxt` takes those of
-    // tile i + 1; `pb_prev` holds the probabilities of tile i - 1, `pb_new` takes those of tile i.
-    auto iterate = [&](auto par_c, int tile, f32x16 (&cur)[2], f32x16 (&nxt)[2], const bf16x8 (&pb_prev)[4],
-                       bf16x8 (&pb_new)[4]) {
-        constexpr int par = decltype(par_c)::value;
-        // what the iteration before has loaded goes into the slots that it has read for the last time (the barrier
-        // at its end lies between); the loads of this iteration have all of it to arrive
-        trim_k(tile + 2);
-        stash_k(std::integral_constant<int, par>{});     // read from the next iteration on
-        trim_v(tile);
-        stash_v(std::integral_constant<int, par>{});
+    float limit = -INFINITY, shift = 0.0f;           // a row's maximum beyond which there is rescaling; what the exponents are shifted by
+    auto vector_step = [&](int tile, auto&& load) {
         const int key0 = tile * KT + ksi * 64;
-        if (!(wave_any && key0 + 63 <= w_p_min && key0 >= w_lo_max)) {   // the diagonal, a window's edge, or nothing at all
+        // the diagonal, a window's edge, or nothing at all (a wavefront without rows has nothing to mask: nobody reads its results)
+        const int upto = p_row - key0 - lh * 8, from = lo_row - key0 - lh * 8;
+        if (wave_any && key0 + 63 > w_p_min) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int key = key0 + kb * 32 + (e / 4) * 8 + lh * 4 + e % 4;
-                    if (!(key <= p_row && key >= lo_row)) cur[kb][e] = -INFINITY;
-                }
+                for (int e = 0; e < 16; ++e)
+                    if (kb * 32 + (e / 8) * 16 + e % 8 > upto) acc[kb][e] = -INFINITY;
         }
-        // The straight line, group by group: a matrix instruction, the LDS read of the operand that the matrix
-        // instruction three groups on will take, and a share of the vector work; a scheduling fence after every group
-        // keeps them in this order.  The matrix instructions: 2 NQ for the scores of tile i + 1, four that sum the rows
-        // of tile i - 1, 4 FB for its output.  The vector work: the rows' maxima of tile i in the first four groups (with
-        // the loads of the tiles to come, whose addresses are a few instructions), the new maximum and what follows
-        // from it in the fifth, then the 32 exponentials of a lane dealt over the groups that are left.
-        constexpr int N_QK = 2 * NQ, N_MATRIX = N_QK + 4 + 4 * FB, AHEAD = 3, MAX_GROUPS = 4;
-        constexpr int EXP_GROUPS = N_MATRIX - MAX_GROUPS - 1;
-        u32x4 operand[AHEAD + 1];
-        // (consecutive matrix instructions go to different accumulators: one that adds to the result of the one before
-        // it would wait for it)
-        auto read_operand = [&](auto g_c) {
-            constexpr int g = decltype(g_c)::value;
-            if constexpr (g < N_QK) {
-                operand[g % (AHEAD + 1)] =
-                    *reinterpret_cast<const u32x4*>(k_get[par ^ 1] + (g % 2) * 32 * KROW + (g / 2) * 16);
-            } else if constexpr (g < N_MATRIX && (g - N_QK) % (1 + FB) != 0) {
-                constexpr int t = (g - N_QK) / (1 + FB), f = (g - N_QK) % (1 + FB) - 1;
-                operand[g % (AHEAD + 1)] = *reinterpret_cast<const u32x4*>(v_get[par ^ 1] + f * 32 * VROW + t * 16);
-            }
-        };
-        float mx = -INFINITY, mx1 = -INFINITY, alpha = 1.0f, shift = 0.0f;
-        bool rescale = false;
-        auto group = [&](auto g_c) {
-            constexpr int g = decltype(g_c)::value;
-            read_operand(std::integral_constant<int, g + AHEAD>{});
-            const bf16x8 from_lds = __builtin_bit_cast(bf16x8, operand[g % (AHEAD + 1)]);
-            if constexpr (g < N_QK) {
-                nxt[g % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(from_lds, q[g / 2], g / 2 == 0 ? zero16 : nxt[g % 2],
-                                                                     0, 0, 0);
-            } else if constexpr ((g - N_QK) % (1 + FB) == 0) {
-                o_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb_prev[(g - N_QK) / (1 + FB)], o_sum, 0, 0, 0);
-            } else {
-                constexpr int t = (g - N_QK) / (1 + FB), f = (g - N_QK) % (1 + FB) - 1;
-                o[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(from_lds, pb_prev[t], o[f], 0, 0, 0);
-            }
-            if constexpr (g < MAX_GROUPS) {
-                // a quarter of the 32 scores of a lane: four of each of its two blocks
+        if (wave_any && key0 < w_lo_max) {
 #pragma unroll
-                for (int e = 4 * g; e < 4 * g + 4; e += 2) {
-                    mx = max3(mx, cur[0][e], cur[0][e + 1]);
-                    mx1 = max3(mx1, cur[1][e], cur[1][e + 1]);
-                }
-                if constexpr (g == 0) fetch_k();          // tile i + 3, whose page number the iteration before looked up
-                if constexpr (g == 1) fetch_v();          // tile i + 1
-                if constexpr (g == 2) lookup_k(tile + 4);
-                if constexpr (g == 3) lookup_v(tile + 2);
-            } else if constexpr (g == MAX_GROUPS) {
-                mx = fmaxf(mx, mx1);
-                mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-                // (without a branch, which would cut the straight line in two)
-                rescale = __any(mx > m_run + slack);      // (-inf + slack is -inf: the first key a row sees counts)
-                const float m_new = rescale ? fmaxf(m_run, mx) : m_run;
-                const float m_use = m_new == -INFINITY ? 0.f : m_new;
-                alpha = __builtin_amdgcn_exp2f((m_run - m_use) * scale2);
-                m_run = m_new;
-                shift = -m_use * scale2;
-            } else {
-                // the second product's steps of 16 keys: step t takes elements 8 (t % 2) .. + 7 of block t / 2 from a lane
-                constexpr int eg = g - MAX_GROUPS - 1;
-                constexpr int first = eg * 32 / EXP_GROUPS, last = (eg + 1) * 32 / EXP_GROUPS;
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int i = first; i < last; ++i) {
-                    const int t = i / 8, e = i % 8;
-                    pb_new[t][e] = static_cast<__bf16>(__builtin_amdgcn_exp2f(fmaf(cur[t / 2][(t % 2) * 8 + e], scale2, shift)));
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        static_for<AHEAD>(read_operand);
-        __builtin_amdgcn_sched_barrier(0);
-        static_for<N_MATRIX>(group);
-        // (the probabilities are first used in the next iteration; this keeps the compiler from moving their
-        // computation out of the straight line, behind the branch below)
+                for (int e = 0; e < 16; ++e)
+                    if (kb * 32 + (e / 8) * 16 + e % 8 < from) acc[kb][e] = -INFINITY;
+        }
+        float mx = -INFINITY, mx1 = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(pb_new[t]));
-        if (rescale) {               // what is accumulated, the product of tile i - 1 included, in units of the new maximum
-            o_sum[0] *= alpha;
+        for (int e = 0; e < 16; e += 4) {
+            // (as one piece: between two of them the compiler puts a pause)
+            asm("v_max3_f32 %0, %0, %2, %3\n\tv_max3_f32 %1, %1, %6, %7\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %1, %1, %8, %9"
+                : "+&v"(mx), "+&v"(mx1)
+                : "v"(acc[0][e]), "v"(acc[0][e + 1]), "v"(acc[0][e + 2]), "v"(acc[0][e + 3]), "v"(acc[1][e]), "v"(acc[1][e + 1]),
+                  "v"(acc[1][e + 2]), "v"(acc[1][e + 3]));
+        }
+        mx = max3(mx, mx, mx1);
+        const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = max3(__uint_as_float(halves[0]), __uint_as_float(halves[0]), __uint_as_float(halves[1]));
+        if (__any(mx > limit)) {                     // (-inf is no more than -inf: the first key a row sees counts)
+            const float m_new = fmaxf(m_run, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
+            const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * scale2);
+            m_run = m_new;
+            limit = m_new + slack;
+            shift = -m_use * scale2;
+#pragma unroll
+            for (int c = 0; c < SUMS; ++c) o_sum[c][0] *= alpha;
 #pragma unroll
             for (int f = 0; f < FB; ++f)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[f][e] *= alpha;
         }
-        __syncthreads();
+        // the second product's steps of 16 keys: step t takes elements 8 (t % 2) .. + 7 of block t / 2 from a lane
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+            for (int i = (t * N_LOADS + 3) / 4; i < ((t + 1) * N_LOADS + 3) / 4; ++i) {
+                load(i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                pb[t][e] = static_cast<__bf16>(__builtin_amdgcn_exp2f(fmaf(acc[t / 2][(t % 2) * 8 + e], scale2, shift)));
+        }
+        // (they are used in the next step: this keeps their computation in this one)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(pb[t]));
+        __builtin_amdgcn_sched_barrier(0);
     };
 
-    f32x16 acc_a[2], acc_b[2];
-    bf16x8 pb_a[4], pb_b[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pb_b[t][e] = static_cast<__bf16>(0.0f);
-    lookup_k(t_begin);
-    fetch_k();
-    lookup_k(t_begin + 1);
-    trim_k(t_begin);
-    stash_k(std::integral_constant<int, 0>{});
-    fetch_k();
-    lookup_k(t_begin + 2);
+        for (int e = 0; e < 8; ++e) pb[t][e] = static_cast<__bf16>(0.0f);
+    pages = lookup(t_begin);
 #pragma unroll
-    for (int u = 0; u < CH; ++u) v_regs[u] = u32x4{0u, 0u, 0u, 0u};
-    stash_v(std::integral_constant<int, 1>{});       // the first iteration multiplies this slot by probabilities of zero
-    lookup_v(t_begin);
-    fetch_v();
-    lookup_v(t_begin + 1);
-    trim_k(t_begin + 1);
-    stash_k(std::integral_constant<int, 1>{});
-    fetch_k();                                       // tile 2, for the first iteration to put into slot 0
-    lookup_k(t_begin + 3);
+    for (int i = 0; i < N_LOADS; ++i) load_k(pages, i, 0);
+#pragma unroll
+    for (int i = 0; i < N_LOADS; ++i) load_v(pages, i, 0);
+    pages = lookup(t_begin + 1);
+    next_pages = lookup(t_begin + 2);
+    // (the first step multiplies this slot of values by probabilities of zero)
+#pragma unroll
+    for (int i = 0; i < N_LOADS; ++i) *reinterpret_cast<u32x4*>(smem + 4 * SLOT + (wave * N_LOADS + i) * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    arrived<0>();                                    // (and the queries: nothing else makes the compiler wait for loads in the loop)
     __syncthreads();
-    scores(std::integral_constant<int, 0>{}, acc_a);
-    __syncthreads();                 // every wavefront has read the first tile's keys before their slot is written again
-    for (int tile = t_begin; tile < t_end; tile += 2) {
-        iterate(std::integral_constant<int, 0>{}, tile, acc_a, acc_b, pb_b, pb_a);
-        if (tile + 1 < t_end) iterate(std::integral_constant<int, 1>{}, tile + 1, acc_b, acc_a, pb_a, pb_b);
+    auto keys_of_next = [&](int i) { load_k(pages, i, k_slot ^ 1); };
+    auto values_of_next = [&](int i) { load_v(pages, i, after(v_slot)); };
+    if (second) {
+#pragma unroll
+        for (int i = 0; i < N_LOADS; ++i) keys_of_next(i);
+        __syncthreads();
+#pragma unroll 1
+        for (int tile = t_begin; tile < t_end; ++tile) {
+            matrix_step(values_of_next);
+            loads_arrived(tile);
+            __syncthreads();
+            k_slot ^= 1;
+            v_slot = after(v_slot);
+            pages = next_pages;
+            next_pages = lookup(tile + 3);
+            vector_step(tile, keys_of_next);
+            __syncthreads();
+        }
+    } else {
+#pragma unroll 1
+        for (int tile = t_begin; tile < t_end; ++tile) {
+            matrix_step(keys_of_next);
+            __syncthreads();
+            vector_step(tile, values_of_next);
+            loads_arrived(tile);
+            k_slot ^= 1;
+            v_slot = after(v_slot);
+            pages = next_pages;
+            next_pages = lookup(tile + 3);
+            __syncthreads();
+        }
+        if (TURNS) __syncthreads();                  // (as many barriers as the others)
     }
+    arrived<0>();                                    // (behind the last tile there were loads that nobody reads)
     // the output product of the last tile
-    if ((t_end - t_begin) & 1) outputs(std::integral_constant<int, 0>{}, pb_a);
-    else outputs(std::integral_constant<int, 1>{}, pb_b);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        o_sum[t % SUMS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb[t], o_sum[t % SUMS], 0, 0, 0);
+#pragma unroll
+        for (int f = 0; f < FB; ++f)
+            o[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(smem + v_get + t * GROUP + f * 1024)), pb[t], o[f], 0, 0, 0);
+    }
     if constexpr (KS > 1) __syncthreads();           // the combination below writes over the tiles
+    if constexpr (SUMS == 2) o_sum[0][0] += o_sum[1][0];
     // the row's sum: feature 0 of the block of ones, which lane lr of half 0 holds
-    float l = __shfl(o_sum[0], lr, kWave);
+    float l = __shfl(o_sum[0][0], lr, kWave);
     [[maybe_unused]] float m_part = m_run;           // the maximum that o and l are in units of
     if constexpr (KS > 1) {
         // The wavefronts of one block of rows hold partial results over their keys: those with ks > 0 leave
@@ -1647,7 +1663,7 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
                           int page_shift, float scale, int window, int skip_single, float* part_o, float* part_ml,
                           int n_splits, hipStream_t s) {
     const long groups = (static_cast<long>(n_tokens) * (nq / nkv)) / (32 * RB) + n_seqs;   // upper bound
-    dim3 grid(static_cast<unsigned>(groups), nkv, n_splits);
+    dim3 grid(static_cast<unsigned>(groups * nkv), 1, n_splits);
 #define EGPT_ROWS32_ARGS                                                                                           \
     static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache),               \
         static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,    \
@@ -1704,6 +1720,7 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
             case 124: EGPT_ROWS32(64, 2, 4); break;
             case 141: EGPT_ROWS32(64, 4, 1); break;
             case 142: EGPT_ROWS32(64, 4, 2); break;
+            case 181: EGPT_ROWS32(64, 8, 1); break;
             case 41: EGPT_TILED(64, 4, 1); break;
             case 42: EGPT_TILED(64, 4, 2); break;
             case 44: EGPT_TILED(64, 4, 4); break;
@@ -1716,6 +1733,8 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
             case 121: EGPT_ROWS32(128, 2, 1); break;
             case 122: EGPT_ROWS32(128, 2, 2); break;
             case 141: EGPT_ROWS32(128, 4, 1); break;
+            case 142: EGPT_ROWS32(128, 4, 2); break;
+            case 181: EGPT_ROWS32(128, 8, 1); break;
             case 41: EGPT_TILED(128, 4, 1); break;
             case 42: EGPT_TILED(128, 4, 2); break;
             case 22: EGPT_TILED(128, 2, 2); break;

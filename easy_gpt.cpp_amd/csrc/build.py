@@ -19,7 +19,7 @@ import time
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ["elementwise.hip", "gemm.hip", "gemm_skinny.hip", "gemm_gate_up.hip", "gemm_rows.hip", "attention.hip", "attention_mfma.hip", "attention_any.hip",
            "attention_window.hip", "head_prep.hip", "sampling.hip", "stream_ops.hip", "linear_recurrence.hip", "constant_decay.hip", "moe.hip", "activations.hip"]
-HEADERS = ["api.h", "common.h"]
+HEADERS = ["api.h", "common.h", "lds_loads.h"]
 LIB_NAME = "libeasygpt_hip.so"
 ARCH = "gfx950"
 # packed-fp32 instructions are kept out of the generated code on purpose

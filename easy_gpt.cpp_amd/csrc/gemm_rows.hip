@@ -35,6 +35,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "lds_loads.h"
 
 namespace egpt {
 
@@ -43,33 +44,10 @@ typedef __attribute__((ext_vector_type(4))) float r_f32x4;
 typedef __attribute__((ext_vector_type(4))) __bf16 r_bf16x4;
 typedef __attribute__((ext_vector_type(2))) unsigned r_u32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned r_u32x4;
-typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kLdsOfCu = 160 * 1024;
 constexpr int kStrip = 8;                      // tiles of rows that are walked together, column by column
 constexpr int kRowsStep = 64;                  // values of k per step: 128 bytes a row
-
-// At most N of this wavefront's memory operations are still on their way (they end in the order in which they were made).
-// The loads into LDS are written in assembly and have no result in registers; __syncthreads() alone does not wait for them.
-template <int N>
-__device__ __forceinline__ void arrived() { __builtin_amdgcn_s_waitcnt((N & 15) | 0x0f70 | (N >> 4) << 14); }
-
-typedef __attribute__((ext_vector_type(4))) int r_i32x4;
-
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"        // (m0 is a reserved register; nothing else here uses it)
-// 16 bytes a lane from `resource` at byte `offset` + `at` to LDS: `lds` (the same for the whole wavefront) + 16 x lane.
-__device__ __forceinline__ void load_to_lds(r_i32x4 resource, int offset, int at, char* lds) {
-    const unsigned to = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_void*)lds));
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(offset), "s"(resource), "s"(at)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-__device__ __forceinline__ r_i32x4 buffer_of(const void* p, size_t bytes) {
-    const uint64_t at = reinterpret_cast<uint64_t>(p);
-    return r_i32x4{__builtin_amdgcn_readfirstlane(static_cast<int>(at)), __builtin_amdgcn_readfirstlane(static_cast<int>(at >> 32) & 0xffff),
-                   __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000};
-}
 
 // gate_activation of four values.  A wavefront issues a vector instruction in four cycles and holds 64 gates a lane, so what an
 // activation takes is seen in the kernel: expf and the division with their cases spelled out are some 45 instructions a value

@@ -1066,39 +1066,42 @@ class HipKernels(KernelBackend):
         row_tiles = -(-t * (nq // nkv) // 16) * nkv
         # Measured (us for one layer's prompt on a GPU that is warm; row tiles of 16 rows; shape = row tiles x key
         # splits of a workgroup, 1xx the kernel of 32-row blocks, whose tiles of 64 keys must be whole pages):
-        #   head size 64, 14 heads on 2:   448 tiles 24: 9.4, 44: 10.4 |  896 tiles 24: 16.9, 44: 14.7, 142: 16.4
-        #     1,344 tiles 44: 20.0, 142: 21.3 | 1,792 tiles 44: 29.7, 142: 26.2 | 3,584 tiles 42: 76, 142: 53
-        #     7,168 tiles (8,192 tokens) 42: 292, 142: 175 | 28,560 tiles (32,640 tokens) 42: 3,840, 142: 2,400
-        #   head size 128, 12 heads on 2:  768 tiles 22: 31.0, 42: 26.1, 141: 27.8 | 1,536 tiles 42: 47.1, 141: 47.3
-        #     3,072 tiles 42: 158, 141: 87;  28 heads on 4: 896 tiles 22: 28.8, 42: 16.3, 141: 19.3 | 1,792 tiles
-        #     42: 40.7, 141: 30.0 | 7,168 tiles 42: 341, 141: 190;  40 heads on 8: 1,280 tiles 42: 23.2, 141: 19.6
+        #   head size 64, 14 heads on 2:   448 tiles 24: 8.9, 44: 10.2, 142: 11.2 |  896 tiles 24: 17.7, 44: 15.4, 142: 16.0
+        #     1,138 tiles 44: 19.3, 142: 19.1 | 12 prompts of 100, 1,050 tiles 44: 14.4, 142: 9.4 | 1,792 tiles 44: 30.9, 142: 25.1
+        #     3,584 tiles 44: 86, 142: 47, 181: 72 | 7,168 tiles (8,192 tokens) 44: 293, 142: 156, 181: 146
+        #   head size 128, 12 heads on 2:  192 tiles 42: 10.8, 142: 12.7 | 300 tiles 42: 15.3, 142: 14.8 | 768 tiles 42: 26.3, 142: 21.0 | 4
+        #     prompts of 200, 600 tiles 42: 10.9, 142: 13.3 | 1,536 tiles 42: 47.4, 142: 32.8;  28 heads on 4: 448 tiles 42: 10.9, 142: 12.8 |
+        #     700 tiles 15.3 both | 1,344 tiles 42: 28.3, 142: 19.2 | 3,584 tiles 42: 102, 142: 46, 181: 53 | 5,376 tiles 42: 199, 142: 87,
+        #     181: 82 | 7,168 tiles 42: 331, 142: 139, 181: 122
+        # A workgroup of 256 rows (181) reads a tile's keys half as often, but a single prompt needs more than 20 of them for every 16
+        # CUs before their different lengths even out; prompts of the same length need only one for a CU: 8 of 301, 2,107 tiles, head size 64
+        # 142: 16.7, 181: 12.9; 28 heads of 128 on 4, 6 of 300, 3,150 tiles 142: 27.9, 181: 19.4.
         blocks_of_32 = page_size <= 64
         if hd == 64:
-            shape = 24 if row_tiles <= 512 else 44 if row_tiles <= 1536 or not blocks_of_32 else 142
-            if shape == 44 and row_tiles > 2048:
-                shape = 42
+            shape = 24 if row_tiles <= 512 else 44 if row_tiles <= (1000 if blocks_of_32 else 2048) else 142 if blocks_of_32 else 42
         else:
-            shape = 22 if row_tiles <= 192 else 42 if row_tiles <= 1024 or not blocks_of_32 else 141
+            shape = 22 if row_tiles <= 192 else 142 if blocks_of_32 and (row_tiles > 1024 or longest >= 400) else 42
+        if shape == 142 and (row_tiles >= 5376 or (2048 < row_tiles <= 4096 and t >= 4 * longest)):
+            shape = 181
         # Portions behind a prefix walk many keys per row and are few blocks of rows: the kernel of 32-row blocks
         # with 128 rows to a workgroup, and the tiles of keys of a block of rows dealt over as many workgroups
-        # as give every CU one.  Measured (us, a layer; shape x workgroups that share the keys): head size 64,
-        # 14 heads on 2, 512 tokens behind 4,096 / 8,192 / 32,768 keys 24x1: 35 / 70 / 257, 124x1: 32 / 59 / 196,
-        # 142x1: 45 / 84 / 300, 142x4: 27 / 38 / 98; 256 tokens behind 32,768 124x1: 195, 124x4: 66, 142x8: 57; 64
-        # tokens 124x1: 201, 142x16: 40; behind 2,048 keys nothing is gained (24x1: 24, 142x4: 23) and a prompt
-        # without a prefix loses (2,048 tokens 142x1: 28, 142x2: 47); three portions of 512 behind 30,000 keys
-        # 142x1: 283, 124x1: 397.  Head size 128, 12 heads on 2, 512 tokens behind 2,048 / 32,768 keys 42x1: 59 /
-        # 643, 141x1: 59 / 665, 141x4: 30 / 185; 28 heads on 4: 141x1: 61 / 671, 141x2: 48 / 378; 40 heads on 8
-        # (160 workgroups): 141x1: 103 / 679.
+        # as give every CU one, in two only from 40 tiles on.  Measured (us, a layer; shape x workgroups that share the keys): head size 64,
+        # 14 heads on 2, 512 tokens behind 2,048 / 8,192 / 32,000 keys 24x1: 23 / 68 / 236, 142x1: 28 / 77 / 289, 142x4: 22 / 36 / 86;
+        # 128 tokens behind 4,096 24x1: 35, 142x8: 16; 64 tokens behind 16,000 24x1: 124, 142x16: 22; 1,024 tokens behind 4,096 142x1: 49,
+        # 142x2: 41.  Head size 128, 12 heads on 2, 512 tokens behind 2,048 / 8,192 / 32,000 keys 42x1: 54 / 170 / 616, 142x1: 36 / 100 / 344, 142x4:
+        # 28 / 43 / 114; 28 heads on 4 142x1: 36 / 100 / 345, 142x2: 40 / 77 / 230.
         key_splits = 1
         # (behind a prefix: the portions' longest context is a few thousand tokens and at least twice the step's own.  Not the
         # longest of all: one portion of 512 tokens of a new prompt beside 40 decoded tokens behind 128 to 2,048, 12 heads of
         # 128 on 2: 51.8 us a layer in four key ranges, 48.0 in one; 8 behind 1,400 and 28 heads on 4 46.6 and 31.1)
         if (blocks_of_32 and longest >= 2 * t
                 and longest >= (cls.prefix_keys if hd == 64 else cls.prefix_keys // 2)):
-            shape = 142 if hd == 64 else 141
+            shape = 142
             workgroups = -(-row_tiles // 8)
-            tiles = -(-longest // (64 * (shape % 10)))
+            tiles = -(-longest // 128)
             key_splits = max(1, min(256 // workgroups, tiles // 4, 16))
+            if key_splits == 2 and tiles < 40:
+                key_splits = 1
         return shape, key_splits
 
     @classmethod

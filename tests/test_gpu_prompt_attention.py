@@ -1,0 +1,39 @@
+"""Prompt attention in blocks of 32 rows: the workgroup shapes that prompts take, and what lies in pages beyond a context."""
+import pytest
+import torch
+
+from test_gpu_kernels import DEV, build_paged, k, run_paged  # noqa: F401  (k: the fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hd,shape", [(64, 181), (128, 142), (128, 181)])
+@pytest.mark.parametrize("window,ps,splits", [(0, 16, 1), (0, 64, 3), (100, 32, 1), (300, 16, 2)])
+def test_workgroups_of_eight_wavefronts(k, hd, shape, window, ps, splits):  # noqa: F811
+    # lengths at and around the tiles (64 or 128 keys) and the blocks of rows (128 or 256), wavefronts without rows, single tokens,
+    # prefixes; the error is that of bfloat16 probabilities and results, as for every other shape
+    seqs = [(300, 700), (1, 1), (64, 64), (65, 129), (2, 513), (1, 257), (127, 128), (17, 1000), (43, 43)]
+    assert run_paged(k, seqs, 6, 2, hd, ps, torch.bfloat16, window=window, tiled_shape=shape, key_splits=splits) <= 1.2e-2
+    assert run_paged(k, seqs, 7, 1, hd, ps, torch.bfloat16, window=window, tiled_shape=shape, key_splits=splits, ramp=0.9, seed=3) <= 1.2e-2
+
+
+@pytest.mark.parametrize("hd,shape", [(64, 142), (64, 181), (128, 142), (128, 181), (64, 121), (128, 141)])
+@pytest.mark.parametrize("window,ps", [(0, 16), (0, 64), (70, 32)])
+def test_nothing_behind_the_context_counts(k, hd, shape, window, ps):  # noqa: F811
+    # slots of a request's last page that hold no token, and pages of nobody, hold no numbers: the same bits
+    seqs = [(130, 130), (9, 200), (1, 17), (61, 333)]
+    nq, nkv, t = 6, 2, 201
+    kc, vc, table, _, _ = build_paged(seqs, nkv, hd, ps, torch.bfloat16, seed=5)
+    qkv = torch.randn(t, (nq + 2 * nkv) * hd, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(DEV)
+    q_len = torch.tensor([q for q, _ in seqs], dtype=torch.int32)
+    q_start = (torch.cumsum(q_len, 0, dtype=torch.int32) - q_len).to(DEV)
+    q_len, kv_len = q_len.to(DEV), torch.tensor([kv for _, kv in seqs], dtype=torch.int32, device=DEV)
+    outs = []
+    for keys, vals in ((kc, vc), (torch.where(kc.abs() > 9e3, float("nan"), kc), torch.where(vc.abs() > 9e3, float("nan"), vc))):
+        out = torch.empty(t, nq * hd, dtype=torch.bfloat16, device=DEV)
+        k._run("egpt_paged_attention_tiled", qkv.data_ptr(), out.data_ptr(), keys.data_ptr(), vals.data_ptr(), table.data_ptr(), table.shape[1],
+               q_start.data_ptr(), q_len.data_ptr(), kv_len.data_ptr(), len(seqs), t, nq, nkv, hd, ps, hd ** -0.5, window, shape, 1, None, None,
+               0, 0, 0, k._stream())
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.isfinite(outs[0].float()).all() and torch.equal(outs[0], outs[1])
