@@ -76,8 +76,7 @@ __device__ __forceinline__ void softmax_chunk(f32x4 (&acc)[NKT], float& m_run, f
 #pragma unroll
     for (int kt = 1; kt < NKT; ++kt)
         mx = fmaxf(mx, fmaxf(fmaxf(acc[kt][0], acc[kt][1]), fmaxf(acc[kt][2], acc[kt][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    mx = fold_rows(mx, MaxOf());
     const float m_new = fmaxf(m_run, mx);
     // a row without any visible key so far keeps maximum -inf; a finite stand-in makes every exp below 0
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -282,8 +281,7 @@ __global__ __launch_bounds__(64 * RT) void attention_any_tiled_kernel(
         if constexpr (SEGMENTS) {
             settle_matrix_results();
             float l = l_run;
-            l += __shfl_xor(l, 16, kWave);
-            l += __shfl_xor(l, 32, kWave);
+            l = fold_rows(l, AddOf());
             float M_new, wa, wb;
             fold_weights(M, m_run, scale2, M_new, wa, wb);
             L = fold_value(L, l, wa, wb);
@@ -407,8 +405,7 @@ __global__ __launch_bounds__(64 * RT) void attention_any_tiled_kernel(
     } else {
         settle_matrix_results();
         l = l_run;
-        l += __shfl_xor(l, 16, kWave);
-        l += __shfl_xor(l, 32, kWave);
+        l = fold_rows(l, AddOf());
     }
     if (valid) {
         T* op = out + (static_cast<size_t>(tok) * nq + head) * hd + lg * 4;
@@ -571,8 +568,7 @@ __global__ __launch_bounds__(256) void attention_any_decode_kernel(
     }
     settle_matrix_results();
     float l = l_run;
-    l += __shfl_xor(l, 16, kWave);
-    l += __shfl_xor(l, 32, kWave);
+    l = fold_rows(l, AddOf());
     if (valid) {
         const size_t prow = (static_cast<size_t>(seg) * n_tokens + tok) * nq + head;
         float* pp = part_o + prow * hd + lg * 4;

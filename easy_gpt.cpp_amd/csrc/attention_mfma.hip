@@ -185,8 +185,7 @@ __global__ __launch_bounds__(64) void attention_mfma_kernel(
                         }
                     }
                 }
-                mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+                mx = fold_rows(mx, MaxOf());
                 const float m_new = fmaxf(m_run[t], mx);
                 // a row without any visible key so far keeps maximum -inf; subtracting a finite stand-in makes
                 // every exp below 0 without a special case (exp2(-inf) = 0)
@@ -227,8 +226,7 @@ __global__ __launch_bounds__(64) void attention_mfma_kernel(
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         float l = l_run[t];
-        l += __shfl_xor(l, 16, kWave);
-        l += __shfl_xor(l, 32, kWave);
+        l = fold_rows(l, AddOf());
         if (!valid[t]) continue;
         const size_t row = static_cast<size_t>(tok[t]) * nq + head[t];
         if (n_splits == 1) {
@@ -428,8 +426,7 @@ __global__ __launch_bounds__(64 * RT * KS) void attention_tiled_kernel(
             float mx = fmaxf(fmaxf(acc[0][0], acc[0][1]), fmaxf(acc[0][2], acc[0][3]));
 #pragma unroll
             for (int kt = 1; kt < 4; ++kt) mx = fmaxf(mx, fmaxf(fmaxf(acc[kt][0], acc[kt][1]), fmaxf(acc[kt][2], acc[kt][3])));
-            mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            mx = fold_rows(mx, MaxOf());
             const float m_new = fmaxf(m_run, mx);
             const float m_use = m_new == -INFINITY ? 0.f : m_new;
             if (__any(m_new != m_run)) {             // some row's maximum moved: rescale what is accumulated
@@ -1385,8 +1382,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
                     mx = fmaxf(mx, s[kt][v]);
                 }
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            mx = fold_rows(mx, MaxOf());
             const float m_new = fmaxf(m_run, mx);
             const bool none = m_new == -INFINITY;
             const float alpha = none ? 1.f : __expf(m_run - m_new);
@@ -1413,8 +1409,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
         kb0 += PF;
     } while (kb0 < w_end);
     float l = l_run;
-    l += __shfl_xor(l, 16, kWave);
-    l += __shfl_xor(l, 32, kWave);
+    l = fold_rows(l, AddOf());
 
     // every wavefront leaves its state in LDS; then all threads combine
     float* mine = wave_state + (wave * 16 + lj) * kRow;

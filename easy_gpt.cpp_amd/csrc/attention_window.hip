@@ -647,8 +647,7 @@ __global__ __launch_bounds__(64 * RT, (DT * RW <= 8 ? 2 : 1)) void window_attent
                         mx = fmaxf(mx, sc);
                     }
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            mx = fold_rows(mx, MaxOf());
             const float m_new = fmaxf(m_run[w], mx);
             const float m_use = m_new == -INFINITY ? 0.f : m_new;      // a row that has seen nothing yet: every exp below is 0
             if (__any(m_new != m_run[w])) {                             // (a factor of exactly 1 otherwise)
@@ -702,8 +701,7 @@ __global__ __launch_bounds__(64 * RT, (DT * RW <= 8 ? 2 : 1)) void window_attent
 #pragma unroll
     for (int w = 0; w < RW; ++w) {
         l_sum[w] = l_run[w];
-        l_sum[w] += __shfl_xor(l_sum[w], 16, kWave);
-        l_sum[w] += __shfl_xor(l_sum[w], 32, kWave);
+        l_sum[w] = fold_rows(l_sum[w], AddOf());
     }
     if (a.n_splits > 1) {
 #pragma unroll
@@ -751,8 +749,7 @@ __global__ __launch_bounds__(64 * RT, (DT * RW <= 8 ? 2 : 1)) void window_attent
                     ss = fmaf(x, x, ss);
                 }
             }
-            ss += __shfl_xor(ss, 16, kWave);
-            ss += __shfl_xor(ss, 32, kWave);
+            ss = fold_rows(ss, AddOf());
             const float f = a.out_scale * inv_rms(ss, 1.0f / static_cast<float>(dv), a.out_eps);
             if (!valid[w]) continue;
             T* op = static_cast<T*>(a.out) + (static_cast<size_t>(tok[w]) * nq + head[w]) * dv + lg * 4;

@@ -152,16 +152,52 @@ struct RowFactor {
     }
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
+// Reductions over a wavefront's lanes in registers: rotations and exchanges of rows of 16 lanes (DPP, v_permlane*_swap) are vector
+// instructions, where a shuffle goes through LDS and its result is waited for.  (Decode steps of the 0.5B sizes, us: one user 769.6
+// with shuffles and 763.6 so, 64 users 1,358.9 and 1,336.0.)  The pairs that are added up, and so the bits, are those of shuffles with
+// lanes 32, 16, 8, 4, 2, 1 apart (or 1, 2, 4, 8): behind a step the values repeat at its distance, so that a rotation by the next one
+// reaches the partner's value.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-    return v;
+struct AddOf {
+    __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct MaxOf {
+    __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+template <class Op>
+__device__ __forceinline__ float fold_32_apart(float v, Op op) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+template <class Op>
+__device__ __forceinline__ float fold_16_apart(float v, Op op) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <class Op>
+__device__ __forceinline__ float fold_wave(float v, Op op) {
+    v = fold_16_apart(fold_32_apart(v, op), op);
+    v = op(v, dpp_move<0x128>(v));                        // row_ror:8, 4, 2, 1
+    v = op(v, dpp_move<0x124>(v));
+    v = op(v, dpp_move<0x122>(v));
+    return op(v, dpp_move<0x121>(v));
+}
+// over the 16 lanes of a row, with lanes 1, 2, 4, 8 apart
+template <class Op>
+__device__ __forceinline__ float fold_row(float v, Op op) {
+    v = op(v, dpp_move<0xb1>(v));                         // quad_perm 1 0 3 2, 2 3 0 1, row_half_mirror, row_mirror
+    v = op(v, dpp_move<0x4e>(v));
+    v = op(v, dpp_move<0x141>(v));
+    return op(v, dpp_move<0x140>(v));
+}
+// over the four lanes with the same place in their rows, with lanes 16, 32 apart
+template <class Op>
+__device__ __forceinline__ float fold_rows(float v, Op op) { return fold_32_apart(fold_16_apart(v, op), op); }
+__device__ __forceinline__ float wave_sum(float v) { return fold_wave(v, AddOf()); }
+__device__ __forceinline__ float wave_max(float v) { return fold_wave(v, MaxOf()); }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.  `scratch` holds >= 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {

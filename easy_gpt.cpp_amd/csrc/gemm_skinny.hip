@@ -185,20 +185,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs a) {
                     ls[i] = has ? p[1] : 0.f;
                 }
                 float mx = fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3]));
-                mx = fmaxf(mx, __shfl_xor(mx, 1, kWave));
-                mx = fmaxf(mx, __shfl_xor(mx, 2, kWave));
-                mx = fmaxf(mx, __shfl_xor(mx, 4, kWave));
-                mx = fmaxf(mx, __shfl_xor(mx, 8, kWave));
+                mx = fold_row(mx, MaxOf());
                 float wg[4], denom = 0.f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     wg[i] = ms[i] == -INFINITY ? 0.f : __expf(ms[i] - mx);
                     denom += wg[i] * ls[i];
                 }
-                denom += __shfl_xor(denom, 1, kWave);
-                denom += __shfl_xor(denom, 2, kWave);
-                denom += __shfl_xor(denom, 4, kWave);
-                denom += __shfl_xor(denom, 8, kWave);
+                denom = fold_row(denom, AddOf());
                 const float inv = 1.0f / denom;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) head_wgt[pair * kMaxAttnSplits + sub + 16 * i] = wg[i] * inv;
@@ -374,10 +368,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs a) {
             float ssq = chunk(s, step_begin + s, r, (rem % 16) * 8);
             if constexpr (PRO == kNorm) {
                 // the 16 threads of a (step, row) sit side by side in one wavefront
-                ssq += __shfl_xor(ssq, 1, kWave);
-                ssq += __shfl_xor(ssq, 2, kWave);
-                ssq += __shfl_xor(ssq, 4, kWave);
-                ssq += __shfl_xor(ssq, 8, kWave);
+                ssq = fold_row(ssq, AddOf());
                 if (rem % 16 == 0) ss_part[s][r] = ssq;
             }
         }
@@ -446,10 +437,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs a) {
         if constexpr (PRO == kNorm) {
             if (blockIdx.x == 0) {
                 float ss = ss_acc;
-                ss += __shfl_xor(ss, 1, kWave);
-                ss += __shfl_xor(ss, 2, kWave);
-                ss += __shfl_xor(ss, 4, kWave);
-                ss += __shfl_xor(ss, 8, kWave);
+                ss = fold_row(ss, AddOf());
                 const int r = tid / 16;
                 if (tid % 16 == 0 && r < m) a.ss_out[split * m + r] = ss;
             }

@@ -37,3 +37,12 @@ def test_nothing_behind_the_context_counts(k, hd, shape, window, ps):  # noqa: F
         torch.cuda.synchronize()
         outs.append(out)
     assert torch.isfinite(outs[0].float()).all() and torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("n", [4, 5, 64, 65, 130])
+@pytest.mark.parametrize("hd,dtype,shape,line", [(64, torch.bfloat16, 24, 1.2e-2), (128, torch.bfloat16, 142, 1.2e-2), (48, torch.float32, None, 2e-6)])
+def test_a_block_of_rows_finds_its_request_among_many(k, n, hd, dtype, shape, line):  # noqa: F811
+    # n requests, the portions at the ends and in the middle: few are searched one after the other, many 64 at a time
+    seqs = [(1, 1 + 7 * i % 40) for i in range(n)]
+    seqs[0], seqs[n // 2], seqs[n - 1] = (70, 70), (9, 30), (133, 140)
+    assert run_paged(k, seqs, 6, 2, hd, 16, dtype, tiled_shape=shape) <= line
