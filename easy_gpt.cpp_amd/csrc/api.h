@@ -48,6 +48,11 @@ int egpt_gemm_skinny(const void* x, const void* w, const void* bias, float* out_
 // egpt_swiglu).  shape: the tile (0 to 6).  k % 64 == 0, n % 4 == 0, operands on 16 bytes.
 int egpt_gemm_rows(const void* x, const void* w, void* out, int m, int n, int k, int n_splits, int kind, int act, int shape,
                    void* stream);
+// The same product for queries, keys and values, w [(nq + 2 nkv) * hd][k], with what egpt_qkv_rope_store does behind it (the whole head
+// rotated, angles from cos_sin [m][hd / 2][2], bias or null): queries go to out [m][(nq + 2 nkv) * hd], whose other columns are left as
+// they are, keys and values to their slots.  hd: 32, 64, 128 or 256.
+int egpt_gemm_rows_rotated(const void* x, const void* w, const void* bias, const float* cos_sin, const int32_t* slots, void* out, void* k_cache,
+                           void* v_cache, int m, int k, int nq, int nkv, int hd, int page_size, int shape, void* stream);
 // float32 product on the matrix cores (float32 operands as three bfloat16 numbers each, float32 accumulation, see gemm.hip):
 // out [n_splits][m][n] are partial sums over n_splits ranges of k (bias only with one).  k % 4 == 0.  A row's values do not
 // depend on m or on the other rows.

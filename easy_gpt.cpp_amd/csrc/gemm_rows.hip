@@ -79,7 +79,19 @@ __device__ __forceinline__ r_f32x4 gate4(r_f32x4 z) {
     return v;
 }
 
-enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsGated = 2, kRowsRelu2 = 3 };
+enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsGated = 2, kRowsRelu2 = 3, kRowsRotated = 4 };
+
+// kRowsRotated: w makes queries, keys and values, whole heads of 2 `half` columns each, and what a tile ends with is what
+// qkv_rope_store_rows_kernel does with such a product, operation for operation: bias, the rotation of queries and keys, keys and values
+// into their pages.  `n` counts pairs (i, i + half) of a head's columns; a wavefront holds both of a pair as it holds gate and up.
+struct RotatedOut {
+    const bf16_t* bias;            // [2 n] or null
+    const float* cos_sin;          // [rows of x][half][2]
+    const int32_t* slots;          // [rows of x] page * page_size + offset
+    bf16_t* k_cache;
+    bf16_t* v_cache;
+    int nq, nkv, half, page_size;
+};
 
 // Products of rows grouped by expert (moe.hip makes the table of tiles): tile i has rows tiles[3 i + 2 ..] of one expert, the
 // numbers of tiles[1 + 3 i ..] being the expert, the tile's first grouped row and its rows; w is [experts][rows of w][k].
@@ -92,7 +104,7 @@ struct Groups {
 template <int BM, int BN, int WM, int WN, int XB, int WB, int OUT, bool GROUPED>
 __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) void gemm_rows_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k, int splits,
-    int steps_per_split, int act, Groups groups) {
+    int steps_per_split, int act, Groups groups, RotatedOut rot) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int NW = WM * WN;
     constexpr int TM = BM / WM / 16, TN = BN / WN / 16;        // 16 x 16 tiles of a wavefront
@@ -108,7 +120,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
     // Workgroups are handed to the eight dies in turn: a die gets a contiguous range of items, rows of x fastest, so that
     // its L2 holds the few rows of w and x that its tiles share.  A workgroup takes items blockIdx.x, blockIdx.x +
     // gridDim.x ... (a grid of several items to a workgroup is a multiple of eight).
-    constexpr int BC = OUT == kRowsGated ? BN / 2 : BN;         // columns of the result in a tile
+    constexpr int BC = OUT == kRowsGated || OUT == kRowsRotated ? BN / 2 : BN;         // columns of the result (or pairs) in a tile
     const int mt = GROUPED ? groups.tiles[0] : (m + BM - 1) / BM, nt = (n + BC - 1) / BC;
     const int tiles = mt * nt, items = tiles * splits;
     const int strips = (mt + kStrip - 1) / kStrip, per_strip = (mt + strips - 1) / strips;
@@ -150,7 +162,9 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
         it.begin = it.split * steps_per_split;
         it.end = min(total, it.begin + steps_per_split);
         it.x = gather ? buffer_of(x, groups.x_rows * row_bytes) : buffer_of(x + static_cast<size_t>(it.m0) * k, it.rows * row_bytes);
-        it.w = buffer_of(from + static_cast<size_t>(it.n0) * k, (OUT == kRowsGated ? 2 * n - it.n0 : min(n - it.n0, BN)) * row_bytes);
+        const int w0 = OUT == kRowsRotated ? it.n0 / rot.half * 2 * rot.half + it.n0 % rot.half : it.n0;      // (a tile is whole heads or a part of one)
+        it.w = buffer_of(from + static_cast<size_t>(w0) * k,
+                         (OUT == kRowsGated || OUT == kRowsRotated ? 2 * n - w0 : min(n - it.n0, BN)) * row_bytes);
         return it;
     };
     int index = blockIdx.x;
@@ -174,6 +188,12 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
             // a wavefront's columns: the first half of them gates, the second half the up columns of the same numbers
             constexpr int C = BN / WN;
             g = r / C * (C / 2) + r % (C / 2) + (r % C >= C / 2 ? n : 0);
+        }
+        if (OUT == kRowsRotated) {
+            // and so are the first and the second columns of pairs
+            constexpr int C = BN / WN;
+            const int pair = r / C * (C / 2) + r % (C / 2);
+            g = pair / rot.half * 2 * rot.half + pair % rot.half + (r % C >= C / 2 ? rot.half : 0);
         }
         wo[i] = g * static_cast<int>(row_bytes) + piece * 16;
     }
@@ -283,7 +303,71 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
             }
         }
     };
+    [[maybe_unused]] auto store_rotated = [&]() {
+        const int width = 2 * n;
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j) {
+            const int pair = now.n0 + wn * (BC / WN) + j * 16 + lg * 4;               // the first of this lane's four
+            if (pair >= n) continue;
+            const int head = pair / rot.half, at = pair % rot.half, col = head * 2 * rot.half + at;
+            const bool is_v = head >= rot.nq + rot.nkv;
+            r_f32x4 ba{0.f, 0.f, 0.f, 0.f}, bb = ba;
+            if (rot.bias) {
+                ba = __builtin_convertvector(*reinterpret_cast<const r_bf16x4*>(rot.bias + col), r_f32x4);
+                bb = __builtin_convertvector(*reinterpret_cast<const r_bf16x4*>(rot.bias + col + rot.half), r_f32x4);
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int r = wm * (BM / WM) + i * 16 + li;
+                if (r >= now.rows) continue;
+                const size_t t = static_cast<size_t>(now.m0) + r;
+                r_f32x4 a = acc[i][j], b = acc[i][j + TN / 2];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    a[e] = scale_then_bias(a[e], 1.f, ba[e]);
+                    b[e] = scale_then_bias(b[e], 1.f, bb[e]);
+                }
+                if (!is_v) {
+                    const r_f32x4* cs = reinterpret_cast<const r_f32x4*>(rot.cos_sin + (t * rot.half + at) * 2);
+                    const r_f32x4 c0 = cs[0], c1 = cs[1];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float ra, rb;
+                        rotate_pair(a[e], b[e], e < 2 ? c0[2 * e] : c1[2 * e - 4], e < 2 ? c0[2 * e + 1] : c1[2 * e - 3], ra, rb);
+                        a[e] = ra;
+                        b[e] = rb;
+                    }
+                }
+                const r_bf16x4 ya = __builtin_convertvector(a, r_bf16x4), yb = __builtin_convertvector(b, r_bf16x4);
+                if (head < rot.nq) {
+                    bf16_t* to = static_cast<bf16_t*>(out) + t * width + col;
+                    *reinterpret_cast<r_bf16x4*>(to) = ya;
+                    *reinterpret_cast<r_bf16x4*>(to + rot.half) = yb;
+                    continue;
+                }
+                const int slot = rot.slots[t];
+                if (slot < 0) continue;
+                const size_t page = slot / rot.page_size, off = slot % rot.page_size, kh = is_v ? head - rot.nq - rot.nkv : head - rot.nq;
+                if (!is_v) {             // keys: [page][kv head][offset][feature]
+                    bf16_t* to = rot.k_cache + ((page * rot.nkv + kh) * rot.page_size + off) * (2 * rot.half) + at;
+                    *reinterpret_cast<r_bf16x4*>(to) = ya;
+                    *reinterpret_cast<r_bf16x4*>(to + rot.half) = yb;
+                } else {                 // values: [page][kv head][feature][offset]
+                    bf16_t* to = rot.v_cache + ((page * rot.nkv + kh) * (2 * rot.half) + at) * rot.page_size + off;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        *reinterpret_cast<__bf16*>(to + static_cast<size_t>(e) * rot.page_size) = ya[e];
+                        *reinterpret_cast<__bf16*>(to + static_cast<size_t>(e + rot.half) * rot.page_size) = yb[e];
+                    }
+                }
+            }
+        }
+    };
     auto store = [&]() {
+        if constexpr (OUT == kRowsRotated) {
+            store_rotated();
+            return;
+        }
         if (OUT == kRowsGated && act != kGateSilu) store_as(std::integral_constant<int, kGateGeluTanh>());
         else store_as(std::integral_constant<int, kGateSilu>());
     };
@@ -342,7 +426,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
         store();
         if (next.rows == 0) break;
         clear();
-        stored = true;
+        stored = OUT != kRowsRotated;                     // (which makes as many stores as its rows ask for)
         index += gridDim.x;
         now = next;
         next = item_of(index + gridDim.x);
@@ -365,9 +449,24 @@ int launch_rows(const void* x, const void* w, void* out, int m, int n, int k, in
     const auto* xp = static_cast<const bf16_t*>(x);
     const auto* wp = static_cast<const bf16_t*>(w);
     const Groups none{nullptr, nullptr, 0};
-    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsGated, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
-    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsF32, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
-    else gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsBf16, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none);
+    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsGated, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none, {});
+    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsF32, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none, {});
+    else gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsBf16, false><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, m, n, k, splits, per, act, none, {});
+    EGPT_CHECK_LAUNCH();
+    return EGPT_OK;
+}
+
+template <int BM, int BN, int WM, int WN, int XB, int WB>
+int launch_rotated(const void* x, const void* w, void* out, int m, int pairs, int k, const RotatedOut& rot, hipStream_t s) {
+    constexpr int BC = BN / 2;
+    if (BC % rot.half != 0 && rot.half % BC != 0) return EGPT_UNSUPPORTED_SIZE;
+    const long items = static_cast<long>((m + BM - 1) / BM) * ((pairs + BC - 1) / BC);
+    if (items > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
+    constexpr int kHeld = kLdsOfCu / ((XB * BM + WB * BN) * 128);
+    const int steps = k / kRowsStep;
+    const long held = steps >= WB ? 256L * kHeld : items;
+    gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsRotated, false><<<static_cast<unsigned>(items < held ? items : held), WM * WN * 64, 0, s>>>(
+        static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), out, m, pairs, k, 1, steps, 0, Groups{nullptr, nullptr, 0}, rot);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
@@ -380,9 +479,9 @@ int launch_groups(const void* x, const void* w, void* out, const Groups& g, long
     const auto* xp = static_cast<const bf16_t*>(x);
     const auto* wp = static_cast<const bf16_t*>(w);
     const int per = k / kRowsStep;
-    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsGated, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
-    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsF32, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
-    else gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsRelu2, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g);
+    if (kind == kRowsGated) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsGated, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g, {});
+    else if (kind == kRowsF32) gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsF32, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g, {});
+    else gemm_rows_kernel<BM, BN, WM, WN, XB, WB, kRowsRelu2, true><<<grid, WM * WN * 64, 0, s>>>(xp, wp, out, 0, n, k, 1, per, act, g, {});
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
@@ -411,6 +510,34 @@ extern "C" int egpt_gemm_rows(const void* x, const void* w, void* out, int m, in
         case 4: return launch_rows<64, 64, 2, 2, 2, 3>(x, w, out, m, n, k, splits, per, kind, act, s);
         case 5: return launch_rows<64, 64, 2, 2, 5, 5>(x, w, out, m, n, k, splits, per, kind, act, s);
         case 6: return launch_rows<64, 128, 2, 2, 6, 6>(x, w, out, m, n, k, splits, per, kind, act, s);
+        default: return EGPT_BAD_ARGUMENT;
+    }
+}
+
+extern "C" int egpt_gemm_rows_rotated(const void* x, const void* w, const void* bias, const float* cos_sin, const int32_t* slots, void* out,
+                                      void* k_cache, void* v_cache, int m, int k, int nq, int nkv, int hd, int page_size, int shape,
+                                      void* stream) {
+    if (!x || !w || !cos_sin || !slots || !out || !k_cache || !v_cache || m < 0 || k <= 0 || nq <= 0 || nkv <= 0 || hd <= 0 || page_size <= 0) return EGPT_BAD_ARGUMENT;
+    const long long width = (static_cast<long long>(nq) + 2LL * nkv) * hd;
+    // (heads of 32 to 256 columns: a tile is whole heads or a power of two of a head's pairs)
+    if (k % kRowsStep != 0 || hd < 32 || hd > 256 || (hd & (hd - 1)) != 0 || width > 0x1fffff) return EGPT_UNSUPPORTED_SIZE;
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(bias) |
+         reinterpret_cast<uintptr_t>(cos_sin) | reinterpret_cast<uintptr_t>(k_cache)) % 16)
+        return EGPT_UNSUPPORTED_SIZE;
+    // a lane's byte offsets from its tile's first row are 32-bit numbers
+    if (static_cast<long long>(k) * 2 * 512 > 0x7fffffffLL || width * k * 2 > 0x7fffffffLL) return EGPT_UNSUPPORTED_SIZE;
+    if (m == 0) return EGPT_OK;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const RotatedOut rot{static_cast<const bf16_t*>(bias), cos_sin, slots, static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), nq, nkv, hd / 2, page_size};
+    const int pairs = static_cast<int>(width / 2);
+    switch (shape) {
+        case 0: return launch_rotated<256, 256, 2, 4, 2, 3>(x, w, out, m, pairs, k, rot, s);
+        case 1: return launch_rotated<192, 256, 2, 4, 2, 3>(x, w, out, m, pairs, k, rot, s);
+        case 2: return launch_rotated<128, 256, 2, 4, 2, 3>(x, w, out, m, pairs, k, rot, s);
+        case 3: return launch_rotated<128, 128, 2, 2, 2, 3>(x, w, out, m, pairs, k, rot, s);
+        case 4: return launch_rotated<64, 64, 2, 2, 2, 3>(x, w, out, m, pairs, k, rot, s);
+        case 5: return launch_rotated<64, 64, 2, 2, 5, 5>(x, w, out, m, pairs, k, rot, s);
+        case 6: return launch_rotated<64, 128, 2, 2, 6, 6>(x, w, out, m, pairs, k, rot, s);
         default: return EGPT_BAD_ARGUMENT;
     }
 }

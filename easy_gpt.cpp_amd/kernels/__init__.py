@@ -215,6 +215,11 @@ class KernelBackend:
         the rows are many (`qkv_rope_store` with a whole rotation)."""
         return self.product(x, w, unrounded=True)
 
+    def product_rotated(self, x, w, bias, cos_sin, slots, k_cache, v_cache, nq, nkv, hd, page_size):
+        """act [T, (nq + 2 nkv) * hd] whose queries are those that `qkv_rope_store` makes of product_parts(x, w) (the whole head rotated;
+        the other columns hold nothing), keys and values stored at their slots, in one go; or None."""
+        return None
+
     def product_normed(self, h, delta, norm_weight, w, weight_offset=0.0):
         """((h + delta) * (weight_offset + norm_weight)) w^T without the rows' 1/rms factor: (float32 partial sums [S, T, N], row sums
         of squares [S2, T], h + delta as a new tensor), or None."""

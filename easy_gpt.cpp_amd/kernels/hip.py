@@ -103,6 +103,7 @@ class HipKernels(KernelBackend):
             "egpt_gemm_f32_gated": [vp, vp, vp, i, i, i, i, i, i, vp],
             "egpt_gemm_skinny": [vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp],
             "egpt_gemm_rows": [vp, vp, vp, i, i, i, i, i, i, i, vp],
+            "egpt_gemm_rows_rotated": [vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, vp],
             "egpt_paged_attention": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp],
             "egpt_paged_attention_mfma": [vp, vp, vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, i, i, vp],
             "egpt_attention_any_tiled": [vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp],
@@ -878,6 +879,46 @@ class HipKernels(KernelBackend):
         shape, s = self._rows_plan(m, n, k, self.rope_parts, 1)
         out = torch.empty((s, m, n), dtype=_F32, device=x.device)
         self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, 1, 0, shape, self._stream())
+        return out
+
+    @classmethod
+    @functools.lru_cache(maxsize=4096)
+    def _rotated_shape(cls, m: int, n: int, k: int) -> int | None:
+        """The tile of the product that ends with bias, rotation and the store into the cache, or None where a product that splits the k
+        range, or the library's, and a kernel for those are faster.  us, weights from memory, replayed from a graph, against those two:
+        1,152 x 896 at 70 / 320 / 1,024 / 2,048 / 4,096 / 8,191 rows 7.5 / 8.1 / 9.7 / 12.8 / 18.9 / 30.1 against 8.6 / 10.3 / 15.1 / 18.9 / 25.5 / 42.5,
+        2,048 x 1,536 at 70 / 128 / 576 / 1,024 / 2,048 / 8,191 10.2 / 10.2 / 13.3 / 13.8 / 23.2 / 55.9 against 9.7 / 10.8 / 17.9 / 21.4 / 28.1 / 76.0, 2,560 x
+        2,048 at 70 / 128 / 200 / 576 / 2,048 / 4,096 12.1 / 12.2 / 12.3 / 17.2 / 36.0 / 48.9 against 10.8 / 12.0 / 13.8 / 19.4 / 36.8 / 58.7: few rows
+        want their k range split, the larger the matrix the more of them.  A large matrix has no second round of tiles to fill the first one's
+        gaps, so three of four CUs should have one: 4,608 x 3,584 at 200 (144 tiles) / 400 (252) / 1,024 (144) / 1,536 (216) / 2,048 (198)
+        26.8 / 28.2 / 61.9 / 60.6 / 71.3 against 22.8 / 34.2 / 53.6 / 66.8 / 81.5, 7,168 x 5,120 at 512 (224) / 640 (140) / 900 (224) / 2,048 (224) 57.5 / 87.1 /
+        81.7 / 128 against 62.4 / 69.8 / 89.3 / 147."""
+        shape = cls._rows_plan(m, n, k, 1, 1)[0]
+        if n * k < 1 << 23:
+            return shape if m >= 40 + n * k // 45000 else None
+        bm, bn = cls._rows_shapes[shape][:2]
+        tiles = -(-m // bm) * -(-n // bn)
+        return shape if tiles >= 0.72 * 256 * -(-tiles // 256) else None
+
+    def product_rotated(self, x, w, bias, cos_sin, slots, k_cache, v_cache, nq, nkv, hd, page_size):
+        m, k = x.shape
+        n = w.shape[0]
+        if (m <= 64 or hd not in (32, 64, 128, 256) or not self._rows_fit(x, w, k) or k_cache.data_ptr() % 16 or cos_sin.data_ptr() % 16
+                or (bias is not None and bias.data_ptr() % 16)):
+            return None
+        shape = self._rotated_shape(m, n, k)
+        if shape is None:
+            return None
+        self._need(x, "x")
+        self._need(w, "w", x.dtype, ((nq + 2 * nkv) * hd, k))
+        if bias is not None:
+            self._need(bias, "bias", x.dtype, (n,))
+        self._need(cos_sin, "cos_sin", _F32, (m, hd // 2, 2))
+        self._need(slots, "slots", _I32, (m,))
+        self._caches(k_cache, v_cache, x.dtype, nkv, page_size, hd)
+        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+        self._run("egpt_gemm_rows_rotated", x.data_ptr(), w.data_ptr(), self._ptr(bias), cos_sin.data_ptr(), slots.data_ptr(), out.data_ptr(),
+                  k_cache.data_ptr(), v_cache.data_ptr(), m, k, nq, nkv, hd, page_size, shape, self._stream())
         return out
 
     def rope_table(self, positions, inv_freq):

@@ -116,26 +116,31 @@ class GQAttention(Mixer):
                 dtype, device, t = self.w_qkv.dtype, h_new.device, h_new.shape[0]
             else:
                 x = x.materialize()
-        if prod is None:
-            # act [T, W], or float32 partial sums [S, T, W]: several also of many rows, where all of a head turns, but not for the
-            # attention of decoded tokens, which reads them once for every range of keys
-            if rot is not None and rot[1] == self.head_dim and not (ctx.max_q_len == 1 and ctx.rows_independent):
-                prod = k.product_parts(x, self.w_qkv)
-            else:
-                prod = k.product(x, self.w_qkv, unrounded=True)
-            dtype, device, t = x.dtype, x.device, x.shape[0]
         slots = cache.slots if cache.writes else None
         common = dict(
             k_cache=cache.k, v_cache=cache.v, nq=self.n_heads, nkv=self.n_kv_heads,
             hd=self.head_dim, page_size=cache.page_size,
         )
+        rotated = None
+        if prod is None:
+            # act [T, W], or float32 partial sums [S, T, W]: several also of many rows, where all of a head turns, but not for the
+            # attention of decoded tokens, which reads them once for every range of keys.  Many rows may be rotated and stored by the
+            # product itself.
+            if rot is not None and rot[1] == self.head_dim and not (ctx.max_q_len == 1 and ctx.rows_independent):
+                if slots is not None:
+                    rotated = k.product_rotated(x, self.w_qkv, self.b_qkv, self.position.table(ctx), slots, **common)
+                if rotated is None:
+                    prod = k.product_parts(x, self.w_qkv)
+            else:
+                prod = k.product(x, self.w_qkv, unrounded=True)
+            dtype, device, t = x.dtype, x.device, x.shape[0]
         attn = torch.empty((t, self.q_size), dtype=dtype, device=device)
         want_parts = self.b_o is None and t <= k.fused_rows
         # ---- single decoded tokens: bias, rotation, the store of the new key and value and the attention over
         # the cache in one kernel, straight from the product's partial sums
         parts = False
         cos_sin = self.position.table(ctx) if rot is not None else None
-        fused = (prod.dim() == 3 and rot is not None and slots is not None and ctx.max_q_len == 1
+        fused = (rotated is None and prod.dim() == 3 and rot is not None and slots is not None and ctx.max_q_len == 1
                  and ctx.rows_independent)
         ranges = None if want_parts else self._ranges(k, ctx, dtype, cache.page_size, fused and rot[1] == self.head_dim)
         if fused:
@@ -144,7 +149,9 @@ class GQAttention(Mixer):
                 ctx.positions, rot[0], rot[1], slots, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.kv_len,
                 self.n_heads, self.n_kv_heads, self.head_dim, cache.page_size, self.scale, self.window or 0,
                 ctx.max_kv_len, combine=not want_parts, cos_sin=cos_sin, ranges=ranges)
-        if parts is False:
+        if rotated is not None:
+            parts = self._attention(k, rotated, ctx, cache, attn, want_parts, ranges)
+        elif parts is False:
             if cos_sin is not None:
                 scale_args = dict(scale_args, cos_sin=cos_sin)
             parts = self._epilogue_and_attention(k, prod, t, width, dtype, device, rot, slots, common, scale_args, ctx,
@@ -203,7 +210,10 @@ class GQAttention(Mixer):
             self.position.apply(q_view, k_view, ctx.positions)
             if slots is not None:
                 k.qkv_rope_store(qkv, None, ctx.positions, None, 0, slots, out=qkv, **common)
-        # ---- attention over the cache.  If the kernel splits the keys, the output projection combines the parts.
+        return self._attention(k, qkv, ctx, cache, attn, want_parts, ranges)
+
+    def _attention(self, k, qkv, ctx, cache, attn, want_parts, ranges):
+        """Attention over the cache.  If the kernel splits the keys, the output projection combines the parts."""
         args = dict(
             nq=self.n_heads, nkv=self.n_kv_heads, hd=self.head_dim, page_size=cache.page_size,
             scale=self.scale, window=self.window or 0, max_q_len=ctx.max_q_len, max_kv_len=ctx.max_kv_len,
