@@ -1140,7 +1140,7 @@ class HipKernels(KernelBackend):
             shape = 142
             workgroups = -(-row_tiles // 8)
             tiles = -(-longest // 128)
-            key_splits = max(1, min(256 // workgroups, tiles // 4, 16))
+            key_splits = max(1, min(256 // workgroups, tiles // (4 if hd == 64 else 3), 16))
             if key_splits == 2 and tiles < 40:
                 key_splits = 1
         return shape, key_splits
