@@ -210,16 +210,10 @@ __global__ __launch_bounds__(64 * RT) void attention_any_tiled_kernel(
     const int kh = blockIdx.y;
     const int group_size = nq / nkv;
 
-    int b = 0, grp = blockIdx.x;
-    for (; b < n_seqs; ++b) {
-        const int groups = (q_len[b] * group_size + ROWS - 1) / ROWS;
-        if (grp < groups) {
-            grp = groups - 1 - grp;          // the last rows first: they have the most keys to walk
-            break;
-        }
-        grp -= groups;
-    }
-    if (b >= n_seqs) return;
+    int b, grp;
+    auto groups_of = [&](int n) { return (n * group_size + ROWS - 1) / ROWS; };
+    if (!find_block(q_len, n_seqs, blockIdx.x, groups_of, b, grp)) return;
+    grp = groups_of(q_len[b]) - 1 - grp;     // the last rows first: they have the most keys to walk
     const int n = q_len[b], kv = kv_len[b], qs = q_start[b];
     const int rows = n * group_size;
     const int width = (nq + 2 * nkv) * hd;

@@ -42,16 +42,10 @@ __global__ __launch_bounds__(64) void attention_mfma_kernel(
 
     // which request, and which group of 16*QT rows of it; within a request the last rows come first: they
     // have the most keys to walk, and the launch is over when the longest wavefront is
-    int b = 0, grp = blockIdx.x;
-    for (; b < n_seqs; ++b) {
-        const int groups = (q_len[b] * group_size + 16 * QT - 1) / (16 * QT);
-        if (grp < groups) {
-            grp = groups - 1 - grp;
-            break;
-        }
-        grp -= groups;
-    }
-    if (b >= n_seqs) return;
+    int b, grp;
+    auto groups_of = [&](int n) { return (n * group_size + 16 * QT - 1) / (16 * QT); };
+    if (!find_block(q_len, n_seqs, blockIdx.x, groups_of, b, grp)) return;
+    grp = groups_of(q_len[b]) - 1 - grp;
     const int n = q_len[b], kv = kv_len[b], qs = q_start[b];
     const int rows = n * group_size;
     const int row_base = grp * 16 * QT;
@@ -286,17 +280,11 @@ __global__ __launch_bounds__(64 * RT * KS) void attention_tiled_kernel(
     const int kh = blockIdx.y;
     const int group_size = nq / nkv;
 
-    int b = 0, grp = blockIdx.x;
-    for (; b < n_seqs; ++b) {
-        // (skip_single: requests of one token are the decode kernel's, which spreads their keys over wavefronts)
-        const int groups = (skip_single && q_len[b] == 1) ? 0 : (q_len[b] * group_size + ROWS - 1) / ROWS;
-        if (grp < groups) {
-            grp = groups - 1 - grp;          // the last rows first: they have the most keys to walk
-            break;
-        }
-        grp -= groups;
-    }
-    if (b >= n_seqs) return;
+    int b, grp;
+    // (skip_single: requests of one token are the decode kernel's, which spreads their keys over wavefronts)
+    auto groups_of = [&](int n) { return (skip_single && n == 1) ? 0 : (n * group_size + ROWS - 1) / ROWS; };
+    if (!find_block(q_len, n_seqs, blockIdx.x, groups_of, b, grp)) return;
+    grp = groups_of(q_len[b]) - 1 - grp;     // the last rows first: they have the most keys to walk
     const int n = q_len[b], kv = kv_len[b], qs = q_start[b];
     const int rows = n * group_size;
     const int width = (nq + 2 * nkv) * HD;
@@ -590,17 +578,11 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     const int kh = blockIdx.x % nkv;
     const int group_size = nq / nkv;
 
-    int b = 0, grp = blockIdx.x / nkv;
-    for (; b < n_seqs; ++b) {
-        // (skip_single: requests of one token are the decode kernel's, which spreads their keys over wavefronts)
-        const int groups = (skip_single && q_len[b] == 1) ? 0 : (q_len[b] * group_size + ROWS - 1) / ROWS;
-        if (grp < groups) {
-            grp = groups - 1 - grp;          // the last rows first: they have the most keys to walk
-            break;
-        }
-        grp -= groups;
-    }
-    if (b >= n_seqs) return;
+    int b, grp;
+    // (skip_single: requests of one token are the decode kernel's, which spreads their keys over wavefronts)
+    auto groups_of = [&](int n) { return (skip_single && n == 1) ? 0 : (n * group_size + ROWS - 1) / ROWS; };
+    if (!find_block(q_len, n_seqs, blockIdx.x / nkv, groups_of, b, grp)) return;
+    grp = groups_of(q_len[b]) - 1 - grp;     // the last rows first: they have the most keys to walk
     const int n = q_len[b], kv = kv_len[b], qs = q_start[b];
     const int rows = n * group_size;
     const int width = (nq + 2 * nkv) * HD;

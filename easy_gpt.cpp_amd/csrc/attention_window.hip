@@ -328,13 +328,8 @@ __global__ __launch_bounds__(64 * RT, (DT * RW <= 8 ? 2 : 1)) void window_attent
     const int kh = blockIdx.y;
     const int group_size = nq / nkv;
 
-    int b = 0, grp = blockIdx.x;
-    for (; b < a.n_seqs; ++b) {
-        const int groups = (a.q_len[b] * group_size + ROWS - 1) / ROWS;
-        if (grp < groups) break;
-        grp -= groups;
-    }
-    if (b >= a.n_seqs) return;
+    int b, grp;
+    if (!find_block(a.q_len, a.n_seqs, blockIdx.x, [&](int n) { return (n * group_size + ROWS - 1) / ROWS; }, b, grp)) return;
     const int n = a.q_len[b], kv = a.kv_len[b], qs = a.q_start[b];
     const int rows = n * group_size;
     const int32_t* table = a.block_table + static_cast<size_t>(b) * a.table_width;

@@ -199,6 +199,41 @@ __device__ __forceinline__ float fold_rows(float v, Op op) { return fold_32_apar
 __device__ __forceinline__ float wave_sum(float v) { return fold_wave(v, AddOf()); }
 __device__ __forceinline__ float wave_max(float v) { return fold_wave(v, MaxOf()); }
 
+// Which request's rows a workgroup has: the requests' blocks of rows lie one after the other, request s has blocks_of(q_len[s]) of
+// them.  False: block `index` is nobody's.  64 requests at a time, by a sum over the lanes; one after the other they are a chain of
+// loads (40 decoded tokens in front of the one portion of a step of the 1.5B sizes: 4,031 us a step, 3,933 so), which is only as good for a few.
+template <class F>
+__device__ __forceinline__ bool find_block(const int32_t* __restrict__ q_len, int n_seqs, int index, F blocks_of, int& seq, int& block) {
+    if (n_seqs <= 4) {
+        for (seq = 0, block = index; seq < n_seqs; ++seq) {
+            const int n = blocks_of(q_len[seq]);
+            if (block < n) return true;
+            block -= n;
+        }
+        return false;
+    }
+    const int lane = threadIdx.x % kWave;
+    for (int s0 = 0; s0 < n_seqs; s0 += kWave) {
+        const int n = s0 + lane < n_seqs ? blocks_of(q_len[s0 + lane]) : 0;
+        int upto = n;
+        upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, true);          // row_shr:1, 2, 4, 8: the sum within a row
+        upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, true);
+        upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, true);
+        upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, true);
+        upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);         // row_bcast:15 and 31: the rows before it
+        upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xc, 0xf, false);
+        const unsigned long long behind = __ballot(upto > index);
+        if (behind != 0) {
+            const int at = __builtin_ctzll(behind);
+            seq = s0 + at;
+            block = index - (__builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(n, at));
+            return true;
+        }
+        index -= __builtin_amdgcn_readlane(upto, kWave - 1);
+    }
+    return false;
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result.  `scratch` holds >= 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;

@@ -79,13 +79,7 @@ __device__ __forceinline__ float gate_of(const DecayArgs<T>& a, size_t t, int co
 // which request and which of its chunks a workgroup has; false: none
 template <typename T>
 __device__ __forceinline__ bool find_chunk(const DecayArgs<T>& a, int index, int chunk, int& b, int& c) {
-    b = 0, c = index;
-    for (; b < a.n_seqs; ++b) {
-        const int n = (a.q_len[b] + chunk - 1) / chunk;
-        if (c < n) return true;
-        c -= n;
-    }
-    return false;
+    return find_block(a.q_len, a.n_seqs, index, [&](int n) { return (n + chunk - 1) / chunk; }, b, c);
 }
 
 // Rotated heads of a chunk's tokens into LDS [chunk][row], columns dk .. padded and rows behind the chunk's tokens zero.
