@@ -551,9 +551,14 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_each(std::make_integer_sequence<int, N>{}, f);
 }
 
+// LDS of a workgroup: keys, slots 0 and 1, then values, slots 0 to 2; at the end the parts of KS wavefronts (FB * 16 + 2 floats a lane)
+template <int HD, int RB, int KS>
+constexpr int kRows32Lds = 5 * 64 * KS * HD * 2 > (KS - 1) * RB * 64 * (HD / 2 + 2) * 4 ? 5 * 64 * KS * HD * 2 : (KS - 1) * RB * 64 * (HD / 2 + 2) * 4;
+
+// Workgroup `index` of a launch (and range `part` of the keys).
 template <int HD, int RB, int KS, bool SPLIT>
-__global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
-    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+__device__ __forceinline__ void rows32_block(
+    char* smem, int index, int part, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
     int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int skip_single,
@@ -565,23 +570,20 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     constexpr int GROUP = 16 * HD * 2;           // bytes of 16 keys (or of their values)
     constexpr int SLOT = KT * HD * 2;            // bytes of a tile of keys (or of values)
     constexpr int PER_LANE = FB * 16 + 2;        // floats a lane leaves for the combination
-    constexpr int COMBINE = (KS - 1) * RB * 64 * PER_LANE * 4;
     constexpr int LOADS = HD / 32, N_LOADS = 4 * LOADS / RB;     // loads of a group; of a tile's keys (and values) by a wavefront
     constexpr int OWN = N_LOADS > LOADS ? N_LOADS / LOADS : 1;   // groups that they are of
     static_assert(N_LOADS * RB == 4 * LOADS && (N_LOADS % LOADS == 0 || LOADS % N_LOADS == 0), "a tile is whole loads");
-    // keys, slots 0 and 1, then values, slots 0 to 2
-    __shared__ __attribute__((aligned(128))) char smem[(5 * SLOT > COMBINE) ? 5 * SLOT : COMBINE];
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int rb = wave % RB, ksi = wave / RB;
     const int lr = lane % 32, lh = lane / 32;
     // (the kv heads of a block of rows after each other, so that all heads' last rows, which have the most keys, begin first)
-    const int kh = blockIdx.x % nkv;
+    const int kh = index % nkv;
     const int group_size = nq / nkv;
 
     int b, grp;
     // (skip_single: requests of one token are the decode kernel's, which spreads their keys over wavefronts)
     auto groups_of = [&](int n) { return (skip_single && n == 1) ? 0 : (n * group_size + ROWS - 1) / ROWS; };
-    if (!find_block(q_len, n_seqs, blockIdx.x / nkv, groups_of, b, grp)) return;
+    if (!find_block(q_len, n_seqs, index / nkv, groups_of, b, grp)) return;
     grp = groups_of(q_len[b]) - 1 - grp;     // the last rows first: they have the most keys to walk
     const int n = q_len[b], kv = kv_len[b], qs = q_start[b];
     const int rows = n * group_size;
@@ -593,15 +595,15 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     const int blk_p_hi = kv - n + blk_last / group_size;
     const int blk_first_pos = kv - n + blk_first / group_size;
     const int blk_lo = window > 0 ? max(0, blk_first_pos - window + 1) : 0;
-    // n_splits > 1: the tiles of keys are dealt over as many workgroups (blockIdx.z), each of which leaves its rows'
+    // n_splits > 1: the tiles of keys are dealt over as many workgroups (`part`), each of which leaves its rows'
     // unnormalised result with its maximum and sum in part_o / part_ml for the kernel that combines them
     // (SPLIT is a parameter of the template so that the kernel without it is compiled as if this were not here; a
     // workgroup takes four tiles at least: fewer are not worth sharing)
     const int t_first = blk_lo / KT, t_last = blk_p_hi / KT + 1;
     const int t_per = SPLIT ? max((t_last - t_first + n_splits - 1) / n_splits, 4) : t_last - t_first;
-    const int t_begin = SPLIT ? t_first + static_cast<int>(blockIdx.z) * t_per : t_first;
+    const int t_begin = SPLIT ? t_first + part * t_per : t_first;
     const int t_end = SPLIT ? min(t_last, t_begin + t_per) : t_last;
-    [[maybe_unused]] const size_t part_row0 = SPLIT ? static_cast<size_t>(blockIdx.z) * n_tokens * nq : 0;
+    [[maybe_unused]] const size_t part_row0 = SPLIT ? static_cast<size_t>(part) * n_tokens * nq : 0;
 
     // this wavefront's block of 32 rows, this lane's row
     const int row_base = blk_first + rb * 32;
@@ -998,6 +1000,18 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     }
 }
 
+template <int HD, int RB, int KS, bool SPLIT>
+__global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
+    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
+    const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
+    int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int skip_single,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens) {
+    __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, RB, KS>];
+    rows32_block<HD, RB, KS, SPLIT>(smem, blockIdx.x, blockIdx.z, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len,
+                                    n_seqs, nq, nkv, page_size, page_shift, scale, window, skip_single, part_o, part_ml, n_splits, n_tokens);
+}
+
 // Deals the keys of a step's decoded tokens out over `slots` workgroups (per kv head): a request's blocks of 32 keys go to as few
 // of them as leave none with more than `per` blocks, `per` being the least for which they all suffice (kLeastPer at least).  One
 // launch a step, for all layers.  With the same number of key ranges for every request the longest one sets a layer's
@@ -1098,8 +1112,10 @@ struct FusedQkv {
 //
 // RANGED: the keys are dealt out by `decode_ranges_kernel`, every request getting as many workgroups as its context is long;
 // grid (slots, kv heads), and a part is kept by its slot.
-template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false>
-__global__ __launch_bounds__(512) void attention_decode_kernel(
+// Workgroup (bx, by, bz) of a launch.
+template <int HD, int PF, bool FUSED, bool MIXED, bool RANGED>
+__device__ __forceinline__ void decode_block(
+    float* wave_state, int bx, int by, int bz,
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ q_start,
@@ -1111,17 +1127,17 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
     // by request (n_tokens is the number of requests then) and the rest is another kernel's.  (A parameter of the
     // template, so that the kernel of the decode step is compiled as if this were not here.)
     if constexpr (MIXED && !RANGED) {
-        if (q_len[blockIdx.x] != 1) return;
+        if (q_len[bx] != 1) return;
     }
-    const int32_t* range = ranges + (RANGED ? blockIdx.x * kRangeInts : 0);
+    const int32_t* range = ranges + (RANGED ? bx * kRangeInts : 0);
     if constexpr (RANGED) {
         if (range[0] < 0) return;
     }
-    extern __shared__ float wave_state[];          // [n_waves][16][HD + 2]: O, then maximum, then sum
+    // wave_state: [n_waves][16][HD + 2]: O, then maximum, then sum
     const int lane = threadIdx.x % kWave, n_waves = blockDim.x / kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // known to be the same for the wavefront
     const int lj = lane % 16, lg = lane / 16;
-    const int b = RANGED ? range[0] : blockIdx.x, kh = blockIdx.y, split = blockIdx.z;
+    const int b = RANGED ? range[0] : bx, kh = by, split = bz;
     const int group_size = nq / nkv;
     const int kv = RANGED ? range[3] : kv_len[b], tok = RANGED ? range[4] : q_start[b];
     const int p = kv - 1;
@@ -1433,7 +1449,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
         if (n_splits == 1) {
             out[(row0 + r) * HD + d] = from_float<bf16_t>(num / den);
         } else {
-            const size_t prow = RANGED ? static_cast<size_t>(blockIdx.x) * nq + kh * group_size + r
+            const size_t prow = RANGED ? static_cast<size_t>(bx) * nq + kh * group_size + r
                                        : static_cast<size_t>(split) * n_tokens * nq +
                                              (MIXED ? static_cast<size_t>(b) * nq + kh * group_size : row0) + r;
             part_o[prow * HD + d] = num;
@@ -1442,6 +1458,43 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
                 part_ml[prow * 2 + 1] = den;
             }
         }
+    }
+}
+
+template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false>
+__global__ __launch_bounds__(512) void attention_decode_kernel(
+    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
+    float* __restrict__ part_ml, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ q_start,
+    const int32_t* __restrict__ kv_len, int n_tokens, int nq, int nkv, int page_size, float scale, int window,
+    int n_splits, FusedQkv f, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ranges) {
+    extern __shared__ float wave_state[];
+    decode_block<HD, PF, FUSED, MIXED, RANGED>(wave_state, blockIdx.x, blockIdx.y, blockIdx.z, qkv, out, part_o, part_ml, k_cache, v_cache, block_table,
+                                               table_width, q_start, kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, f, q_len, ranges);
+}
+
+// Portions of prompts in blocks of 128 rows and, behind them in the same launch, the requests of one token dealt out by `ranges`
+// (range_slots workgroups for each kv head).  The portions' longest block of rows and the decoded tokens' longest range take about as long as
+// each other and neither fills the chip: 512 tokens of a new prompt beside 40 decoded ones behind 128 to 2,048, 12 heads of 128 on 2, are
+// 48 workgroups of 20 us and 256 of 13, a layer 32.1 us one launch after the other and 21.9 so.  A CU holds one workgroup of either kind.
+template <int HD>
+__global__ __launch_bounds__(512) void attention_mixed_kernel(
+    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
+    const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
+    int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int row_blocks,
+    const int32_t* __restrict__ ranges, int range_slots, float* __restrict__ range_o, float* __restrict__ range_ml) {
+    __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, 4, 2>];
+    static_assert(kRows32Lds<HD, 4, 2> >= 8 * 16 * (HD + 2) * 4, "room for what eight wavefronts of decoded tokens leave");
+    const int index = blockIdx.x;
+    if (index < row_blocks) {
+        rows32_block<HD, 4, 2, false>(smem, index, 0, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,
+                                      page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0);
+    } else {
+        const int i = index - row_blocks;
+        decode_block<HD, 2, false, true, true>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, qkv, out, range_o, range_ml, k_cache,
+                                               v_cache, block_table, table_width, q_start, kv_len, n_seqs, nq, nkv, page_size, scale, window, 1,
+                                               FusedQkv{}, q_len, ranges);
     }
 }
 
@@ -1669,6 +1722,25 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
                                                              HD, n_splits);
 }
 
+template <int HD>
+static int launch_mixed(const void* qkv, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table, int table_width,
+                        const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv,
+                        int page_size, int page_shift, float scale, int window, const int32_t* ranges, int slots, float* range_o,
+                        float* range_ml, hipStream_t s) {
+    const long blocks = ((static_cast<long>(n_tokens) * (nq / nkv)) / 128 + n_seqs) * nkv;          // upper bound
+    const long grid = blocks + static_cast<long>(slots) * nkv;
+    if (grid > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
+    attention_mixed_kernel<HD><<<static_cast<unsigned>(grid), 512, 0, s>>>(
+        static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
+        block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, static_cast<int>(blocks), ranges,
+        slots, range_o, range_ml);
+    EGPT_CHECK_LAUNCH();
+    attention_reduce_kernel<<<n_seqs * nq, 64, 0, s>>>(range_o, range_ml, static_cast<bf16_t*>(out), n_seqs * nq, HD, 1, q_start, q_len, nq,
+                                                       ranges + slots * kRangeInts);
+    EGPT_CHECK_LAUNCH();
+    return EGPT_OK;
+}
+
 static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache, const void* v_cache,
                                           const int32_t* block_table, int table_width, const int32_t* q_start,
                                           const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens,
@@ -1695,6 +1767,12 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
     int page_shift = 0;
     while ((1 << page_shift) < page_size) ++page_shift;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (ranges && shape == 142 && key_splits == 1) {
+        if (slots < n_seqs || slots > kRangeSlots) return EGPT_BAD_ARGUMENT;
+        return (hd == 64 ? launch_mixed<64> : launch_mixed<128>)(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
+                                                                 n_tokens, nq, nkv, page_size, page_shift, scale, window, ranges, slots, range_o,
+                                                                 range_ml, s);
+    }
 #define EGPT_TILED(HD_, RT_, KS_)                                                                                  \
     launch_tiled<HD_, RT_, KS_>(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len,      \
                                 n_seqs, n_tokens, nq, nkv, page_size, page_shift, scale, window, skip_single, s)

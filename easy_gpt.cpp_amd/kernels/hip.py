@@ -1046,6 +1046,13 @@ class HipKernels(KernelBackend):
                 part_o = part_ml = None
                 n_splits = n_waves = lean = 0
                 if ranges is not None and singles and nq // nkv <= 16:
+                    # the portions' blocks of rows and the decoded tokens' ranges in one launch, which has the portions in blocks of 128
+                    # rows (us a layer, against the shape that the portions take alone and a second launch: 12 heads of 128 on 2, 40 of 128 to
+                    # 2,048 beside 512 21.9 against 32.1, 16 of 100 to 1,500 beside 64 15.1 and 17.9, 30 of 1,500 to 3,000 beside 256 behind 1,000
+                    # 31.3 and 50.0; 28 on 4, 3 of 1,200 beside 1,000 26.6 and 51.5; 14 heads of 64 on 2, 40 of 128 to 3,000 beside 512
+                    # 18.9 and 22.2, 20 of 2,500 to 4,000 beside 64 19.0 and 19.4, 20 of 100 to 8,000 beside 1,000 21.8 and 30.5)
+                    if key_splits == 1 and page_size <= 64:
+                        shape = 142
                     slots = self._need_ranges(ranges, b, nkv)
                     range_o = torch.empty((slots, nq, hd), dtype=_F32, device=qkv.device)
                     range_ml = torch.empty((slots, nq, 2), dtype=_F32, device=qkv.device)

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+import test_gpu_decode_ranges as decode_ranges
 from test_gpu_kernels import DEV, build_paged, k, run_paged  # noqa: F401  (k: the fixture)
 
 pytestmark = pytest.mark.gpu
@@ -46,3 +47,9 @@ def test_a_block_of_rows_finds_its_request_among_many(k, n, hd, dtype, shape, li
     seqs = [(1, 1 + 7 * i % 40) for i in range(n)]
     seqs[0], seqs[n // 2], seqs[n - 1] = (70, 70), (9, 30), (133, 140)
     assert run_paged(k, seqs, 6, 2, hd, 16, dtype, tiled_shape=shape) <= line
+
+
+@pytest.mark.parametrize("hd,nq,nkv", [(64, 14, 2), (128, 12, 2)])
+@pytest.mark.parametrize("portions", [[(300, 900), (129, 129)], [(1000, 1000)]])
+def test_portions_of_several_blocks_beside_decoded_tokens_in_one_launch(k, hd, nq, nkv, portions):  # noqa: F811
+    decode_ranges.test_a_mixed_step_dealt_out(k, hd, nq, nkv, portions)
