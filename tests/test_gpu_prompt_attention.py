@@ -53,3 +53,23 @@ def test_a_block_of_rows_finds_its_request_among_many(k, n, hd, dtype, shape, li
 @pytest.mark.parametrize("portions", [[(300, 900), (129, 129)], [(1000, 1000)]])
 def test_portions_of_several_blocks_beside_decoded_tokens_in_one_launch(k, hd, nq, nkv, portions):  # noqa: F811
     decode_ranges.test_a_mixed_step_dealt_out(k, hd, nq, nkv, portions)
+
+
+@pytest.mark.parametrize("hd,dtype,line", [(16, torch.float32, 2e-6), (64, torch.float32, 2e-6), (96, torch.bfloat16, 1.2e-2), (256, torch.float32, 2e-6)])
+@pytest.mark.parametrize("window", [0, 9])
+def test_decoded_tokens_of_one_segment(k, hd, dtype, line, window):  # noqa: F811
+    # contexts of at most 64 tokens are one segment, whose result is written as it is; the same rows beside a longer context are folded
+    # and have the same bits in float32
+    short = [(1, 1), (1, 16), (1, 17), (1, 33), (1, 63), (1, 64)]
+    assert run_paged(k, short, 6, 2, hd, 16, dtype, window=window) <= line
+    nq, nkv, b = 6, 2, len(short)
+    outs = []
+    kc, vc, table, _, _ = build_paged(short, nkv, hd, 16, dtype, seed=9)
+    qkv = torch.randn(b, (nq + 2 * nkv) * hd, generator=torch.Generator().manual_seed(1)).to(dtype).to(DEV)
+    one, start, kv = torch.ones(b, dtype=torch.int32, device=DEV), torch.arange(b, dtype=torch.int32, device=DEV), torch.tensor([n for _, n in short], dtype=torch.int32, device=DEV)
+    wide = torch.nn.functional.pad(table, (0, 4), value=-1)
+    for longest in (64, 128):                                # the launch's bound alone makes one segment or two
+        out = torch.empty(b, nq * hd, dtype=dtype, device=DEV)
+        k.paged_attention(qkv, out, kc, vc, wide.contiguous(), start, one, kv, nq, nkv, hd, 16, hd ** -0.5, window, 1, longest)
+        outs.append(out)
+    assert torch.equal(*outs)
