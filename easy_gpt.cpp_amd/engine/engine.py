@@ -394,7 +394,7 @@ class Engine:
         position + 1 and whose block table is its request's.  That shape depends on the number of tokens alone,
         so it is captured and replayed like a decode step, where the same step run kernel by kernel would spend
         twice its device time on the host.  Keys and values of all rows are stored before attention reads them
-        (`rows_independent` is False).  Logits are computed for every row, the wanted ones are returned.  Not for
+        (`rows_independent` is False).  Logits are computed for the wanted rows, their number rounded up to a power of two.  Not for
         models with per-request state, whose parts walk a portion token after token."""
         rcs = self._check(entries)
         counts = [len(e.tokens) for e in entries]
@@ -402,20 +402,16 @@ class Engine:
         with self.cache.reserved(rcs, counts):
             widths = self._table_widths(rcs)
             kv_bound = -(-max(rc.num_tokens + n for rc, n in zip(rcs, counts)) // 512) * 512
-            key = (t, tuple(widths), kv_bound)
-            plan = self._plan(self._row_plans, key, lambda: _DecodePlan(self, t, widths, kv_bound, rows_independent=False))
+            n_want = sum(len(e.want) for e in entries)
+            r_pad = 1
+            while r_pad < min(n_want, t):
+                r_pad *= 2
+            r_pad = min(r_pad, t) if n_want <= t else n_want            # (a row may be wanted more than once)
+            key = (t, tuple(widths), kv_bound, r_pad)
+            plan = self._plan(self._row_plans, key, lambda: _DecodePlan(self, t, widths, kv_bound, rows_independent=False, wanted=r_pad))
             plan.fill_rows(rcs, entries, counts)
             logits = self._run(plan)
-        want, base = [], 0
-        for e, n in zip(entries, counts):
-            want.extend(base + int(w) for w in e.want)
-            base += n
-        if not want:
-            return None
-        if want == list(range(t)):
-            return logits
-        return logits.index_select(0, torch.tensor(want, dtype=torch.int64, device=self.device))
-
+        return logits[:n_want] if n_want else None
 
     # ------------------------------------------------------------------ any mix, from a graph for its padded size
     def _step_padded(self, entries) -> torch.Tensor | None:
@@ -603,17 +599,21 @@ class _PaddedPlan:
 class _DecodePlan:
     """Static device buffers, a host mirror and the captured graph of one decode batch shape."""
 
-    def __init__(self, engine: Engine, batch: int, widths: list[int], kv_bound: int, rows_independent: bool = True, spread: int = 0):
+    def __init__(self, engine: Engine, batch: int, widths: list[int], kv_bound: int, rows_independent: bool = True, spread: int = 0,
+                 wanted: int | None = None):
         self.batch, self.widths = batch, list(widths)
         dev = engine.device
         n_groups = len(widths)
         b = batch
-        n_small = (7 + n_groups) * b
-        self.host_small = torch.empty(n_small, dtype=torch.int32, pin_memory=True)
-        self.dev_small = torch.empty(n_small, dtype=torch.int32, device=dev)
-        n_tab = sum(b * w for w in widths)
-        self.host_tab = torch.full((max(n_tab, 1),), -1, dtype=torch.int32).pin_memory()
-        self.dev_tab = torch.full((max(n_tab, 1),), -1, dtype=torch.int32, device=dev)
+        # the rows' numbers, the wanted rows (a step of decoded tokens wants all of them: its row numbers) and the block tables lie behind
+        # each other, so that a step is one copy to the device
+        n_small, n_tab = (7 + n_groups) * b, max(sum(b * w for w in widths), 1)
+        n_want = wanted or 0
+        self.host = torch.full((n_small + n_want + n_tab,), -1, dtype=torch.int32).pin_memory()
+        self.dev = torch.full((n_small + n_want + n_tab,), -1, dtype=torch.int32, device=dev)
+        self.host_small, self.dev_small = self.host[:n_small], self.dev[:n_small]
+        self.host_tab, self.dev_tab = self.host[n_small + n_want :], self.dev[n_small + n_want :]
+        self.np_want = self.host[n_small : n_small + n_want].numpy()
         self.np_small = self.host_small.numpy()
         v = lambda i: self.dev_small[i * b : (i + 1) * b]
         groups, off = [], 0
@@ -623,7 +623,7 @@ class _DecodePlan:
         ps = engine.page_size
         self.ctx = StepContext(
             num_tokens=b, num_seqs=b, token_ids=v(0), positions=v(1), q_start=v(2), q_len=v(3), kv_len=v(4),
-            want_rows=v(6), max_q_len=1, max_kv_len=min([kv_bound] + [w * ps for w in widths]),
+            want_rows=v(6) if wanted is None else self.dev[n_small : n_small + n_want], max_q_len=1, max_kv_len=min([kv_bound] + [w * ps for w in widths]),
             q_start_host=list(range(b)), q_len_host=[1] * b, kv_len_host=[0] * b,
             state_slots=v(5), state_slots_host=[0] * b, groups=groups, page_size=ps, kv_storage=engine.kv,
             state_storage=engine.states, cache_location=engine.model.cache_location,
@@ -672,9 +672,10 @@ class _DecodePlan:
                         tables_changed = True
                 off += rows * w
             self.row_state[2 * b : 2 * rows : 2] = -2
-        self.dev_small.copy_(self.host_small, non_blocking=True)
         if tables_changed:
-            self.dev_tab.copy_(self.host_tab, non_blocking=True)
+            self.dev.copy_(self.host, non_blocking=True)
+        else:
+            self.dev_small.copy_(self.host_small, non_blocking=True)
         if self.copied is None:
             self.copied = torch.cuda.Event()
         self.copied.record()
@@ -689,9 +690,13 @@ class _DecodePlan:
         n_groups = len(self.widths)
         small = self.np_small.reshape(7 + n_groups, t)
         pos = 0
+        want: list[int] = []
         for e, n in zip(entries, counts):
             small[0, pos : pos + n] = e.tokens
+            want.extend(pos + int(w) for w in e.want)
             pos += n
+        self.np_want[: len(want)] = want
+        self.np_want[len(want) :] = 0
         per_request = np.empty((4, b), dtype=np.int32)               # q_start, q_len, kv_len, state slots
         slots = np.empty(max(n_groups * t, 1), dtype=np.int32)
         tables = np.empty(max(sum(b * w for w in self.widths), 1), dtype=np.int32)
@@ -714,8 +719,7 @@ class _DecodePlan:
             off_out += t * w
         self.ctx.kv_len_host = (small[4]).tolist()
         self.ctx.state_slots_host = small[5].tolist()
-        self.dev_small.copy_(self.host_small, non_blocking=True)
-        self.dev_tab.copy_(self.host_tab, non_blocking=True)
+        self.dev.copy_(self.host, non_blocking=True)
         if self.copied is None:
             self.copied = torch.cuda.Event()
         self.copied.record()
