@@ -80,9 +80,15 @@ int egpt_paged_attention_mfma(const void* qkv, void* out, float* part_o, float* 
                               const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs,
                               int n_tokens, int nq, int nkv, int hd, int page_size, float scale, int window,
                               int n_splits, int rows_per_wave, int combine, void* stream);
+// Prompt portions of heads of 64 or 128 (keys and values alike), bfloat16, queries [n_tokens][nq][hd], with dist_bias [nq][dist_far + 1]
+// (float32, or null) added to the scaled scores by distance, the last entry beyond dist_far; pages of 16, 32 or 64 tokens.
+// row_blocks: blocks of 32 rows to a workgroup, 4 or 8.  EGPT_UNSUPPORTED_SIZE where a kv head's rows of the table leave LDS no room.
+int egpt_heads_attention(const void* q, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table, int table_width,
+                         const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv, int hd,
+                         int page_size, float scale, int window, const float* dist_bias, int dist_far, int row_blocks, void* stream);
 // Prompt portions: the wavefronts of a workgroup share key/value tiles through LDS (n_splits == 1 semantics);
 // page sizes that are powers of two; shape = 10 * row tiles + key splits per workgroup (41, 42, 44, 22, 24), or
-// 100 + 10 * blocks of 32 rows + key splits (121, 122, 124, 141, 142; page sizes up to 64).
+// 100 + 10 * blocks of 32 rows + key splits (121, 122, 124, 141, 142, 181; page sizes up to 64).
 // key_splits > 1 (shapes from 100 on): the tiles of keys that a block of rows walks are dealt over as many workgroups,
 // whose results part_o [key_splits][n_tokens][nq][hd] and part_ml [key_splits][n_tokens][nq][2] (float32) hold until a
 // second kernel has combined them.

@@ -555,14 +555,26 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int HD, int RB, int KS>
 constexpr int kRows32Lds = 5 * 64 * KS * HD * 2 > (KS - 1) * RB * 64 * (HD / 2 + 2) * 4 ? 5 * 64 * KS * HD * 2 : (KS - 1) * RB * 64 * (HD / 2 + 2) * 4;
 
-// Workgroup `index` of a launch (and range `part` of the keys).
-template <int HD, int RB, int KS, bool SPLIT>
+// What a score gets for the distance between its row and its key, by the query head: table [nq][far + 1], float32, added to the scaled
+// score; beyond `far` the last entry counts.  In LDS (behind the tiles) a head's entries lie turned round and divided by the scale, so that
+// keys that follow each other find theirs one behind the other, with kBiasFront and kBiasBack copies of the last and the first at the
+// ends, which rows and keys of a tile that is partly beyond `far` or the diagonal run into.
+struct DistanceBias {
+    const float* table;
+    int far;
+    float* lds;
+};
+constexpr int kBiasFront = 96, kBiasBack = 64;
+__host__ __device__ constexpr int bias_row(int far) { return (kBiasFront + far + 1 + kBiasBack + 1) | 1; }     // (odd: the heads' banks differ)
+
+// Workgroup `index` of a launch (and range `part` of the keys); a token's queries lie `width` values behind those of the one before.
+template <int HD, int RB, int KS, bool SPLIT, bool BIAS = false>
 __device__ __forceinline__ void rows32_block(
     char* smem, int index, int part, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
     int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int skip_single,
-    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens) {
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens, int width, DistanceBias bias = {}) {
     constexpr int NQ = HD / 16;                  // steps of 16 features of the score product
     constexpr int FB = HD / 32;                  // blocks of 32 output features
     constexpr int ROWS = 32 * RB;
@@ -587,7 +599,6 @@ __device__ __forceinline__ void rows32_block(
     grp = groups_of(q_len[b]) - 1 - grp;     // the last rows first: they have the most keys to walk
     const int n = q_len[b], kv = kv_len[b], qs = q_start[b];
     const int rows = n * group_size;
-    const int width = (nq + 2 * nkv) * HD;
     const int32_t* table = block_table + static_cast<size_t>(b) * table_width;
 
     // the workgroup's rows and the keys they need
@@ -803,8 +814,21 @@ __device__ __forceinline__ void rows32_block(
     };
     const float slack = kSlack / scale2;
     float limit = -INFINITY, shift = 0.0f;           // a row's maximum beyond which there is rescaling; what the exponents are shifted by
+    const float* const bias_of_row = BIAS ? bias.lds + (valid ? r % group_size : 0) * bias_row(bias.far) + kBiasFront : nullptr;
     auto vector_step = [&](int tile, auto&& load) {
         const int key0 = tile * KT + ksi * 64;
+        float beyond = 0.f;                          // what all of a tile's scores get that is `far` or more behind every row
+        if constexpr (BIAS) {
+            if (w_p_min - (key0 + 63) >= bias.far) {
+                beyond = bias_of_row[0];
+            } else {
+                const float* from = bias_of_row + min(max(bias.far - p_row + key0, -kBiasFront), bias.far + 1) + lh * 8;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[kb][e] += from[kb * 32 + (e / 8) * 16 + e % 8];
+            }
+        }
         // the diagonal, a window's edge, or nothing at all (a wavefront without rows has nothing to mask: nobody reads its results)
         const int upto = p_row - key0 - lh * 8, from = lo_row - key0 - lh * 8;
         if (wave_any && key0 + 63 > w_p_min) {
@@ -833,6 +857,7 @@ __device__ __forceinline__ void rows32_block(
         mx = max3(mx, mx, mx1);
         const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
         mx = max3(__uint_as_float(halves[0]), __uint_as_float(halves[0]), __uint_as_float(halves[1]));
+        if constexpr (BIAS) mx += beyond;
         if (__any(mx > limit)) {                     // (-inf is no more than -inf: the first key a row sees counts)
             const float m_new = fmaxf(m_run, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * scale2);
@@ -846,6 +871,7 @@ __device__ __forceinline__ void rows32_block(
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[f][e] *= alpha;
         }
+        const float moved = BIAS ? fmaf(beyond, scale2, shift) : shift;
         // the second product's steps of 16 keys: step t takes elements 8 (t % 2) .. + 7 of block t / 2 from a lane
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -856,7 +882,7 @@ __device__ __forceinline__ void rows32_block(
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                pb[t][e] = static_cast<__bf16>(__builtin_amdgcn_exp2f(fmaf(acc[t / 2][(t % 2) * 8 + e], scale2, shift)));
+                pb[t][e] = static_cast<__bf16>(__builtin_amdgcn_exp2f(fmaf(acc[t / 2][(t % 2) * 8 + e], scale2, moved)));
         }
         // (they are used in the next step: this keeps their computation in this one)
 #pragma unroll
@@ -871,6 +897,12 @@ __device__ __forceinline__ void rows32_block(
     pages = lookup(t_begin);
 #pragma unroll
     for (int i = 0; i < N_LOADS; ++i) load_k(pages, i, 0);
+    if constexpr (BIAS) {
+        const int row = bias_row(bias.far);
+        for (int idx = threadIdx.x; idx < group_size * row; idx += 64 * RB * KS)
+            bias.lds[idx] = bias.table[static_cast<size_t>(kh * group_size + idx / row) * (bias.far + 1) +
+                                       min(max(bias.far - (idx % row - kBiasFront), 0), bias.far)] / scale;
+    }
 #pragma unroll
     for (int i = 0; i < N_LOADS; ++i) load_v(pages, i, 0);
     pages = lookup(t_begin + 1);
@@ -1009,7 +1041,21 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens) {
     __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, RB, KS>];
     rows32_block<HD, RB, KS, SPLIT>(smem, blockIdx.x, blockIdx.z, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len,
-                                    n_seqs, nq, nkv, page_size, page_shift, scale, window, skip_single, part_o, part_ml, n_splits, n_tokens);
+                                    n_seqs, nq, nkv, page_size, page_shift, scale, window, skip_single, part_o, part_ml, n_splits, n_tokens,
+                                    (nq + 2 * nkv) * HD);
+}
+
+// The same for queries that lie by themselves, [tokens][nq][HD], with a bias by distance or without one.
+template <int HD, int RB, int KS, bool BIAS>
+__global__ __launch_bounds__(64 * RB * KS) void attention_heads32_kernel(
+    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
+    const int32_t* __restrict__ kv_len, int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window,
+    const float* __restrict__ table, int far) {
+    extern __shared__ __attribute__((aligned(128))) char heads_lds[];
+    const DistanceBias bias{table, far, reinterpret_cast<float*>(heads_lds + kRows32Lds<HD, RB, KS>)};
+    rows32_block<HD, RB, KS, false, BIAS>(heads_lds, blockIdx.x, 0, q, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
+                                          nq, nkv, page_size, page_shift, scale, window, 0, nullptr, nullptr, 1, 0, nq * HD, bias);
 }
 
 // Deals the keys of a step's decoded tokens out over `slots` workgroups (per kv head): a request's blocks of 32 keys go to as few
@@ -1489,7 +1535,7 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
     const int index = blockIdx.x;
     if (index < row_blocks) {
         rows32_block<HD, 4, 2, false>(smem, index, 0, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,
-                                      page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0);
+                                      page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0, (nq + 2 * nkv) * HD);
     } else {
         const int i = index - row_blocks;
         decode_block<HD, 2, false, true, true>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, qkv, out, range_o, range_ml, k_cache,
@@ -1818,6 +1864,51 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
                                q_start, kv_len, n_seqs, nq, nkv, hd, page_size, scale, window, single_splits, single_waves, 1,
                                single_lean != 0, nullptr, q_len, ranges, slots, s);
     return EGPT_OK;
+}
+
+constexpr int kLdsMost = 160 * 1024;
+template <int HD, int RB, int KS, bool BIAS>
+static int launch_heads32(const void* q, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table, int table_width,
+                          const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv,
+                          int page_size, int page_shift, float scale, int window, const float* table, int far, hipStream_t s) {
+    const long blocks = ((static_cast<long>(n_tokens) * (nq / nkv)) / (32 * RB) + n_seqs) * nkv;          // upper bound
+    const long lds = kRows32Lds<HD, RB, KS> + (BIAS ? static_cast<long>(nq / nkv) * bias_row(far) * 4 : 0);
+    if (lds > kLdsMost || blocks > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
+    static bool raised = false;                      // (more than 64 KB: asked for once per instance)
+    if (!raised) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_heads32_kernel<HD, RB, KS, BIAS>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                kLdsMost) != hipSuccess)
+            return EGPT_UNSUPPORTED_SIZE;
+        raised = true;
+    }
+    attention_heads32_kernel<HD, RB, KS, BIAS><<<static_cast<unsigned>(blocks), 64 * RB * KS, static_cast<size_t>(lds), s>>>(
+        static_cast<const bf16_t*>(q), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
+        block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, table, far);
+    EGPT_CHECK_LAUNCH();
+    return EGPT_OK;
+}
+
+extern "C" int egpt_heads_attention(const void* q, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table,
+                                    int table_width, const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs,
+                                    int n_tokens, int nq, int nkv, int hd, int page_size, float scale, int window, const float* dist_bias,
+                                    int dist_far, int row_blocks, void* stream) {
+    if (!q || !out || !k_cache || !v_cache || !block_table || !q_start || !q_len || !kv_len) return EGPT_BAD_ARGUMENT;
+    if (n_seqs <= 0 || n_tokens < 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || table_width <= 0 || window < 0 || !(scale > 0.f) || dist_far < 0 ||
+        (row_blocks != 4 && row_blocks != 8))
+        return EGPT_BAD_ARGUMENT;
+    if ((hd != 64 && hd != 128) || page_size < 16 || page_size > 64 || (page_size & (page_size - 1)) != 0 || dist_far > 16384) return EGPT_UNSUPPORTED_SIZE;
+    if (n_tokens == 0) return EGPT_OK;
+    int page_shift = 0;
+    while ((1 << page_shift) < page_size) ++page_shift;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define EGPT_HEADS32(HD_, RB_, KS_)                                                                                                    \
+    (dist_bias ? launch_heads32<HD_, RB_, KS_, true> : launch_heads32<HD_, RB_, KS_, false>)(                                          \
+        q, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, n_tokens, nq, nkv, page_size, page_shift,  \
+        scale, window, dist_bias, dist_far, s)
+    if (hd == 64) return row_blocks == 4 ? EGPT_HEADS32(64, 4, 2) : EGPT_HEADS32(64, 8, 1);
+    // (with a bias two slots of 128 keys and three of their values leave no room for its table)
+    return row_blocks == 4 && !dist_bias ? EGPT_HEADS32(128, 4, 2) : EGPT_HEADS32(128, 8, 1);
+#undef EGPT_HEADS32
 }
 
 extern "C" int egpt_paged_attention_tiled(const void* qkv, void* out, const void* k_cache, const void* v_cache,
