@@ -59,7 +59,9 @@ def test_portions_of_several_blocks_beside_decoded_tokens_in_one_launch(k, hd, n
 @pytest.mark.parametrize("window", [0, 9])
 def test_decoded_tokens_of_one_segment(k, hd, dtype, line, window):  # noqa: F811
     # contexts of at most 64 tokens are one segment, whose result is written as it is; the same rows beside a longer context are folded
-    # and have the same bits in float32
+    # and have the same bits in float32.  (A score is hd products of size one, added up four at a time and divided by sqrt(hd): off by hd / 4
+    # roundings of sums of sqrt(hd) at most, which with few keys to a row goes into the result: 3.8e-6 at 256.)
+    line = max(line, hd / 4 * 2.0 ** -24)
     short = [(1, 1), (1, 16), (1, 17), (1, 33), (1, 63), (1, 64)]
     assert run_paged(k, short, 6, 2, hd, 16, dtype, window=window) <= line
     nq, nkv, b = 6, 2, len(short)
