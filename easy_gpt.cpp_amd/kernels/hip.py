@@ -1501,10 +1501,9 @@ class HipKernels(KernelBackend):
             raise ValueError(f"key size {dk} / value size {dv} is not supported (at most {self.max_window_attention_dim})")
         # (a block of positions bounds the keys that a row sees as a window of that many does)
         reach = min(window, block) if window and block else (window or block)
-        if (q.dtype == _BF16 and dk == dv and dk in (64, 128) and page_size in (16, 32, 64) and keep_first == 0 and sink is None and not block
-                and slopes is None and softcap is None and head_gate is None and maps == 1 and scale > 0 and dist_far <= 1024
-                and all(v.data_ptr() % 16 == 0 for v in (q, k_cache, v_cache))):
-            row_blocks = self._heads_blocks(t, b, nq, nkv, dk, window, max_q_len, max_kv_len)
+        if max_q_len >= self.heads_portion and self._heads_fit(q, k_cache, v_cache, nq // nkv, dk, dv, page_size, scale, keep_first, sink, dist_bias,
+                                                               dist_far, block, slopes, softcap, head_gate, maps):
+            row_blocks = self._heads_blocks(t, nq, nkv, dk, window, max_kv_len)
             if row_blocks:
                 self._run("egpt_heads_attention", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), width,
                           q_start.data_ptr(), q_len.data_ptr(), kv_len.data_ptr(), b, t, nq, nkv, dk, page_size, float(scale), int(window),
@@ -1532,8 +1531,19 @@ class HipKernels(KernelBackend):
                   self._stream())
 
 
+    heads_portion = 96           # tokens of a step's longest portion from which the kernel below is asked for
+
     @staticmethod
-    def _heads_blocks(t, b, nq, nkv, hd, window, max_q_len, max_kv_len) -> int:
+    def _heads_fit(q, k_cache, v_cache, group, dk, dv, page_size, scale, keep_first, sink, dist_bias, dist_far, block, slopes, softcap, head_gate,
+                   maps) -> bool:
+        """Whether egpt_heads_attention takes the call: its tiles take 80 KB of LDS at most, a kv head's bias, divided by the scale, the rest."""
+        return (q.dtype == _BF16 and dk == dv and dk in (64, 128) and page_size in (16, 32, 64) and keep_first == 0 and sink is None and not block
+                and slopes is None and softcap is None and head_gate is None and maps == 1 and scale >= 1e-6 and dist_far <= 16384
+                and (dist_bias is None or 80 * 1024 + group * (dist_far + 163) * 4 <= 160 * 1024)
+                and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0)
+
+    @staticmethod
+    def _heads_blocks(t, nq, nkv, hd, window, max_kv_len) -> int:
         """Blocks of 32 rows to a workgroup of the prompt kernel for heads of 64 and 128 (attention_rows32_kernel's loop on queries that lie by
         themselves, with a bias by distance or without), or 0 for the window kernel.  us a layer against that: 14 heads of 64 on 2 with a
         bias, prompts of 128 / 512 / 2,048 / 5,000 tokens 11.0 / 16.2 / 30.5 / 86 against 13.5 / 26.0 / 101 / 305, three of 333 to 1,357 27.1 against 74.5, 6 of
@@ -1542,7 +1552,7 @@ class HipKernels(KernelBackend):
         1,000 / 2,000 20.6 / 31.5 against 33.1 / 39.3 (head size 128 36.7 / 64 against 48.3 / 65), 128 tokens beside 4 behind 1,000 20.4 against 17.9, 66 beside one
         behind 3,042 42 against 23.  A narrow window leaves little to walk (100: 17.8 against 16.7).  256 rows to a workgroup as
         `_portion_shape` has them."""
-        if max_q_len < 96 or 0 < window < 192 or max_kv_len > ((4 if hd == 64 else 3) * t if t >= 256 else 512 if hd == 64 else 300):
+        if 0 < window < 192 or max_kv_len > ((4 if hd == 64 else 3) * t if t >= 256 else 512 if hd == 64 else 300):
             return 0
         row_tiles = -(-t * (nq // nkv) // 16) * nkv
         return 8 if row_tiles >= 5376 or (2048 < row_tiles <= 4096 and t >= 4 * max_kv_len) else 4

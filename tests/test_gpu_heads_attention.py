@@ -85,4 +85,15 @@ def test_wrapper_takes_it_only_where_it_covers_the_call(monkeypatch):
     k.window_attention(*args, 0, 0, None, 200, 200, slopes=torch.zeros(nq, device=DEV))
     k.window_attention(*args, 0, 0, None, 200, 200, block=64)
     k.window_attention(*args, 200, 4, None, 200, 200)                                             # kept first tokens
-    assert names == ["egpt_window_attention_tiled"] * 6
+    k.window_attention(*args, 0, 0, None, 200, 200, dist_bias=torch.zeros(nq, 20001, device=DEV))  # a table that LDS does not hold
+    assert names == ["egpt_window_attention_tiled"] * 7
+    # the largest that it does, of a kv head's many heads
+    names.clear()
+    nq, nkv = 32, 1
+    kc, vc, table, _, _ = build_paged([(200, 200)], nkv, hd, ps, torch.bfloat16, seed=1)
+    q = torch.randn(200, nq * hd, device=DEV).bfloat16()
+    args = (q, torch.empty_like(q), kc, vc, table, one(0), one(200), one(200), nq, nkv, hd, hd, ps, 0.125)
+    most = (80 * 1024 // 4) // nq - 163
+    for far in (most, most + 1):
+        k.window_attention(*args, 0, 0, None, 200, 200, dist_bias=torch.zeros(nq, far + 1, device=DEV))
+    assert names == ["egpt_heads_attention", "egpt_window_attention_tiled"]
