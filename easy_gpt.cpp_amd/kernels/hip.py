@@ -1159,17 +1159,18 @@ class HipKernels(KernelBackend):
             return None
         return cls._portion_shape(tokens, nq, nkv, hd, page_size, portion_kv)
 
-    # A mixed step's requests of one token go to the decode kernel when the step's longest context is beyond this: the
-    # second launch (and a third that combines key ranges) costs some 8 us, a workgroup of the tiled kernel that walks
-    # 4,000 keys alone some 30.  Measured, us for one layer's attention of the 0.5B sizes, tiled kernel alone against
-    # the two: one portion of 512 tokens beside 8 decoded tokens behind 600 keys each 11.0 against 18.3, behind 1,300
-    # 16.2 against 18.6, behind 4,000 33.2 against 20.5, behind 16,000 122 against 32; four portions beside 24 decoded
+    # A mixed step's requests of one token are taken apart from the portions when the step's longest context is beyond this.
+    # Without a table of ranges that is a launch of the decode kernel (and a third that combines key ranges), some 8 us, where
+    # a workgroup of the tiled kernel that walks 4,000 keys alone takes some 30.  us for one layer's attention of the 0.5B sizes,
+    # tiled kernel alone against the two: one portion of 512 tokens beside 8 decoded tokens behind 600 keys each 11.0 against 18.3,
+    # behind 1,300 16.2 against 18.6, behind 4,000 33.2 against 20.5, behind 16,000 122 against 32; four portions beside 24 decoded
     # tokens behind 1,300 keys 36.7 against 38.1, behind 4,000 61.6 against 43.5, behind 16,000 152 against 66
     singles_apart_beyond = 2048
-    # Dealt out by the contexts' lengths (`decode_ranges`) they go there, at head size 128, beyond this.  The tiled kernel alone against it, one
-    # portion of 512 tokens of a new prompt beside decoded ones: 12 heads of 128 on 2, 40 behind 128 to 2,048 48.3 and 36.7 (in equal
-    # ranges 42.3); 28 heads of 128 on 4, 8 behind 1,400 31.3 and 29.9, behind 700 23.4 and 28.6; 14 heads of 64 on 2, 40 behind 128 to
-    # 2,048 24.0 and 29.7, 8 behind 4,000 35.6 and 21.2 (in equal ranges 21.0)
+    # Dealt out by the contexts' lengths (`decode_ranges`) they share the portions' launch, at head size 128 beyond this.  The kernel of
+    # the portions alone against it, a new prompt's 512 tokens beside decoded ones: 12 heads of 128 on 2, 40 behind 128 to 2,048 51.5
+    # and 21.9, behind 128 to 1,000 20.6 and 20.0, 8 behind 1,400 35.6 and 19.2, 300 tokens beside 8 behind 300 12.9 and 17.7; 28 on 4,
+    # 40 behind 128 to 2,048 71.8 and 34.2, to 1,000 25.1 and 24.9.  14 heads of 64 on 2, 40 behind 128 to 3,000 36.2 and 18.9, to 2,000
+    # 18.9 and 15.9, to 1,000 11.7 and 14.8, 8 behind 1,500 15.1 and 14.8: there what is gained below 2,048 the table's 5 us a step use up
     singles_dealt_beyond = 1024
     prefix_keys = 4096           # a step's longest context from which its portions are taken to lie behind a prefix
     attention_segment = 64       # keys per segment of the decode kernel for any head size (kSegment in attention_any.hip)
