@@ -568,7 +568,10 @@ constexpr int kBiasFront = 96, kBiasBack = 64;
 __host__ __device__ constexpr int bias_row(int far) { return (kBiasFront + far + 1 + kBiasBack + 1) | 1; }     // (odd: the heads' banks differ)
 
 // Workgroup `index` of a launch (and range `part` of the keys); a token's queries lie `width` values behind those of the one before.
-template <int HD, int RB, int KS, bool SPLIT, bool BIAS = false>
+// WIDE: scores of any finite size.  score x scale - maximum x scale as one multiply-add has the rounding of its last operand in it, the
+// same factor for a whole row, which divides out as long as it is a number: 2^64 at 2^30.  Beyond (a bias that stands for a mask) the maximum
+// is taken off first.
+template <int HD, int RB, int KS, bool SPLIT, bool BIAS = false, bool WIDE = BIAS>
 __device__ __forceinline__ void rows32_block(
     char* smem, int index, int part, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
@@ -816,6 +819,7 @@ __device__ __forceinline__ void rows32_block(
     // the others: 2-norm of the error against 64 bits at 1,024 tokens of head size 128 0.00197 and 0.00201.  Where a row has some
     // thousand keys that is lost among them; shorter contexts, and those with a bias, are rescaled whenever a maximum grows.)
     const float slack = BIAS || blk_p_hi < 1536 ? 0.f : kSlack / scale2;
+    [[maybe_unused]] bool beyond_shift = false;      // WIDE: a row of the wavefront has such a maximum
     float limit = -INFINITY, shift = 0.0f;           // a row's maximum beyond which there is rescaling; what the exponents are shifted by
     const float* const bias_of_row = BIAS ? bias.lds + (valid ? r % group_size : 0) * bias_row(bias.far) + kBiasFront : nullptr;
     auto vector_step = [&](int tile, auto&& load) {
@@ -867,6 +871,7 @@ __device__ __forceinline__ void rows32_block(
             m_run = m_new;
             limit = m_new + slack;
             shift = -m_use * scale2;
+            if constexpr (WIDE) beyond_shift = __any(!(fabsf(shift) < 0x1p30f));
 #pragma unroll
             for (int c = 0; c < SUMS; ++c) o_sum[c][0] *= alpha;
 #pragma unroll
@@ -874,7 +879,17 @@ __device__ __forceinline__ void rows32_block(
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[f][e] *= alpha;
         }
-        const float moved = BIAS ? fmaf(beyond, scale2, shift) : shift;
+        float moved = BIAS ? fmaf(beyond, scale2, shift) : shift;
+        if constexpr (WIDE) {
+            if (beyond_shift) {
+                const float m_use = m_run == -INFINITY ? 0.f : m_run;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[kb][e] = acc[kb][e] + beyond - m_use;
+                moved = 0.f;
+            }
+        }
         // the second product's steps of 16 keys: step t takes elements 8 (t % 2) .. + 7 of block t / 2 from a lane
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -903,8 +918,12 @@ __device__ __forceinline__ void rows32_block(
     if constexpr (BIAS) {
         const int row = bias_row(bias.far);
         for (int idx = threadIdx.x; idx < group_size * row; idx += 64 * RB * KS)
-            bias.lds[idx] = bias.table[static_cast<size_t>(kh * group_size + idx / row) * (bias.far + 1) +
-                                       min(max(bias.far - (idx % row - kBiasFront), 0), bias.far)] / scale;
+        {
+            const float of = bias.table[static_cast<size_t>(kh * group_size + idx / row) * (bias.far + 1) +
+                                        min(max(bias.far - (idx % row - kBiasFront), 0), bias.far)];
+            // (a finite entry stays finite: a row all of whose keys have the lowest number sees them all alike)
+            bias.lds[idx] = __builtin_isfinite(of) ? fminf(fmaxf(of / scale, -3.402823466e38f), 3.402823466e38f) : of;
+        }
     }
 #pragma unroll
     for (int i = 0; i < N_LOADS; ++i) load_v(pages, i, 0);
@@ -1057,7 +1076,7 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_heads32_kernel(
     const float* __restrict__ table, int far) {
     extern __shared__ __attribute__((aligned(128))) char heads_lds[];
     const DistanceBias bias{table, far, reinterpret_cast<float*>(heads_lds + kRows32Lds<HD, RB, KS>)};
-    rows32_block<HD, RB, KS, false, BIAS>(heads_lds, blockIdx.x, 0, q, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
+    rows32_block<HD, RB, KS, false, BIAS, true>(heads_lds, blockIdx.x, 0, q, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
                                           nq, nkv, page_size, page_shift, scale, window, 0, nullptr, nullptr, 1, 0, nq * HD, bias);
 }
 

@@ -56,6 +56,39 @@ def test_heads_with_a_bias_by_distance(hd, row_blocks, nq, nkv, ps, far, window)
             assert float((got[s : s + n] - want).abs().max()) <= (1.2e-2 if size == 1.0 or far is None else 2.4e-2), (i, size)
 
 
+@pytest.mark.parametrize("hd,row_blocks", [(64, 4), (64, 8), (128, 8)])
+@pytest.mark.parametrize("mask", [-1e10, -1e30, torch.finfo(torch.float32).min, -math.inf])
+def test_a_bias_that_stands_for_a_mask(hd, row_blocks, mask):
+    # beyond `far` (which the first tiles of long rows see alone), and, where it is a finite number that swallows any score, at the
+    # nearest distances too: the first rows see masked keys alone then, all alike
+    k = kernels.backend()
+    nq, nkv, ps, far = 4, 2, 16, 100
+    seqs = [(300, 700), (260, 260), (65, 129)]
+    kc, vc, table, keys, vals = build_paged(seqs, nkv, hd, ps, torch.bfloat16, seed=7)
+    g = torch.Generator().manual_seed(hd)
+    t = sum(n for n, _ in seqs)
+    q = torch.randn(t, nq, hd, generator=g).to(torch.bfloat16)
+    bias = torch.randn(nq, far + 1, generator=g)
+    bias[:3, far] = mask
+    bias[1, 50:] = mask
+    if -math.inf < mask < -1e20:
+        bias[2, :5] = mask
+        bias[3] = mask
+    q_len = torch.tensor([n for n, _ in seqs], dtype=torch.int32)
+    q_start = torch.cumsum(q_len, 0, dtype=torch.int32) - q_len
+    out = torch.full((t, nq * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    bd, qd, qs, ql = bias.to(DEV), q.to(DEV), q_start.to(DEV), q_len.to(DEV)
+    kl = torch.tensor([n for _, n in seqs], dtype=torch.int32, device=DEV)
+    k._run("egpt_heads_attention", qd.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], qs.data_ptr(),
+           ql.data_ptr(), kl.data_ptr(), len(seqs), t, nq, nkv, hd, ps, hd ** -0.5, 0, bd.data_ptr(), far, row_blocks, k._stream())
+    torch.cuda.synchronize()
+    got = out.double().cpu().view(t, nq, hd)
+    for i, (n, _) in enumerate(seqs):
+        s = int(q_start[i])
+        want = _reference(q[s : s + n].double(), keys[i].double(), vals[i].double(), nq, nkv, hd ** -0.5, 0, bias.double())
+        assert float((got[s : s + n] - want).abs().max()) <= 1.2e-2, i
+
+
 def test_tables_that_leave_no_room_are_refused():
     k = kernels.backend()
     p = torch.zeros(1 << 20, device=DEV, dtype=torch.uint8).data_ptr()
