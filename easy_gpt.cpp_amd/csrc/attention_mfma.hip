@@ -567,6 +567,15 @@ struct DistanceBias {
 constexpr int kBiasFront = 96, kBiasBack = 64;
 __host__ __device__ constexpr int bias_row(int far) { return (kBiasFront + far + 1 + kBiasBack + 1) | 1; }     // (odd: the heads' banks differ)
 
+// Rows are rescaled late, by a maximum that has grown by 2^8, in steps of more row tiles of 16 than this and where the keys are dealt out,
+// behind so many keys.  Against a row's own maximum the largest probability is one, which bfloat16 has exactly; against an older
+// one it is rounded like the others, and the result is further from 64 bits: 2-norm of its error at scores of deviation two, late
+// and exact, head size 64, 2,048 / 5,000 tokens 0.00185 and 0.00181 / 0.00195 and 0.00182; 512 tokens behind 1,600 keys 0.00216 and 0.00184 (the
+// kernel of 16-row tiles 0.00180).  The large steps gain 2 to 6 % by it (us a layer: 14 heads of 64 on 2, 8,191 tokens 168 and 175; 28 of 128
+// on 4, 5,000 tokens 195 and 205) and are nearer to 64 bits so than with every row late from the first key on (0.00199, 0.00205); the others,
+// which have kernels with exact maxima to compare with, keep them.
+constexpr int kLateFrom = 1536, kLateTiles64 = 1536, kLateTiles128 = 1024;
+
 // Workgroup `index` of a launch (and range `part` of the keys); a token's queries lie `width` values behind those of the one before.
 // WIDE: scores of any finite size.  score x scale - maximum x scale as one multiply-add has the rounding of its last operand in it, the
 // same factor for a whole row, which divides out as long as it is a number: 2^64 at 2^30.  Beyond (a bias that stands for a mask) the maximum
@@ -577,7 +586,7 @@ __device__ __forceinline__ void rows32_block(
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
     int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int skip_single,
-    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens, int width, DistanceBias bias = {}) {
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens, int width, int late, DistanceBias bias = {}) {
     constexpr int NQ = HD / 16;                  // steps of 16 features of the score product
     constexpr int FB = HD / 32;                  // blocks of 32 output features
     constexpr int ROWS = 32 * RB;
@@ -681,8 +690,8 @@ __device__ __forceinline__ void rows32_block(
     // instructions (the probabilities of tile i).  The two wavefronts of a SIMD take them in turn: wavefronts 4 to 7 are one
     // step behind, so that one of the two is at its matrix instructions while the other is at its vector instructions, and a
     // barrier behind every step keeps them so.
-    // Behind long contexts the accumulated output is rescaled only when a row's maximum has grown by more than 2^kSlack since the last
-    // time: until then the exponentials are taken against the old maximum, so they may reach 2^kSlack instead of 1, which
+    // With `late`, behind long contexts the accumulated output is rescaled only when a row's maximum has grown by more than 2^kSlack since
+    // the last time: until then the exponentials are taken against the old maximum, so they may reach 2^kSlack instead of 1, which
     // float32 sums and bfloat16 probabilities (the same relative precision at any magnitude) do not mind.
     // Keys and values go from memory straight to LDS, 16 keys (never more than a page's) to a load's base address and a
     // constant of the lane beside it, so that they cost no vector instructions and no registers.  A wavefront that issues a load waits
@@ -816,9 +825,8 @@ __device__ __forceinline__ void rows32_block(
         v_get = v_lane + v_slot * SLOT;
     };
     // (Against the row's own maximum the largest probability is one, which bfloat16 has exactly; against an older one it is rounded like
-    // the others: 2-norm of the error against 64 bits at 1,024 tokens of head size 128 0.00197 and 0.00201.  Where a row has some
-    // thousand keys that is lost among them; shorter contexts, and those with a bias, are rescaled whenever a maximum grows.)
-    const float slack = BIAS || blk_p_hi < 1536 ? 0.f : kSlack / scale2;
+    // the others, at any context: see kLateFrom.)
+    const float slack = late && blk_p_hi >= kLateFrom ? kSlack / scale2 : 0.f;
     [[maybe_unused]] bool beyond_shift = false;      // WIDE: a row of the wavefront has such a maximum
     float limit = -INFINITY, shift = 0.0f;           // a row's maximum beyond which there is rescaling; what the exponents are shifted by
     const float* const bias_of_row = BIAS ? bias.lds + (valid ? r % group_size : 0) * bias_row(bias.far) + kBiasFront : nullptr;
@@ -1060,11 +1068,11 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_rows32_kernel(
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
     int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int skip_single,
-    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens) {
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int n_tokens, int late) {
     __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, RB, KS>];
     rows32_block<HD, RB, KS, SPLIT>(smem, blockIdx.x, blockIdx.z, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len,
                                     n_seqs, nq, nkv, page_size, page_shift, scale, window, skip_single, part_o, part_ml, n_splits, n_tokens,
-                                    (nq + 2 * nkv) * HD);
+                                    (nq + 2 * nkv) * HD, late);
 }
 
 // The same for queries that lie by themselves, [tokens][nq][HD], with a bias by distance or without one.
@@ -1077,7 +1085,7 @@ __global__ __launch_bounds__(64 * RB * KS) void attention_heads32_kernel(
     extern __shared__ __attribute__((aligned(128))) char heads_lds[];
     const DistanceBias bias{table, far, reinterpret_cast<float*>(heads_lds + kRows32Lds<HD, RB, KS>)};
     rows32_block<HD, RB, KS, false, BIAS, true>(heads_lds, blockIdx.x, 0, q, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
-                                          nq, nkv, page_size, page_shift, scale, window, 0, nullptr, nullptr, 1, 0, nq * HD, bias);
+                                          nq, nkv, page_size, page_shift, scale, window, 0, nullptr, nullptr, 1, 0, nq * HD, 0, bias);
 }
 
 // Deals the keys of a step's decoded tokens out over `slots` workgroups (per kv head): a request's blocks of 32 keys go to as few
@@ -1550,14 +1558,14 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
-    int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int row_blocks,
+    int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int late, int row_blocks,
     const int32_t* __restrict__ ranges, int range_slots, float* __restrict__ range_o, float* __restrict__ range_ml) {
     __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, 4, 2>];
     static_assert(kRows32Lds<HD, 4, 2> >= 8 * 16 * (HD + 2) * 4, "room for what eight wavefronts of decoded tokens leave");
     const int index = blockIdx.x;
     if (index < row_blocks) {
         rows32_block<HD, 4, 2, false>(smem, index, 0, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,
-                                      page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0, (nq + 2 * nkv) * HD);
+                                      page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0, (nq + 2 * nkv) * HD, late);
     } else {
         const int i = index - row_blocks;
         decode_block<HD, 2, false, true, true>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, qkv, out, range_o, range_ml, k_cache,
@@ -1773,13 +1781,13 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
                           const int32_t* block_table, int table_width, const int32_t* q_start, const int32_t* q_len,
                           const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv, int page_size,
                           int page_shift, float scale, int window, int skip_single, float* part_o, float* part_ml,
-                          int n_splits, hipStream_t s) {
+                          int n_splits, int late, hipStream_t s) {
     const long groups = (static_cast<long>(n_tokens) * (nq / nkv)) / (32 * RB) + n_seqs;   // upper bound
     dim3 grid(static_cast<unsigned>(groups * nkv), 1, n_splits);
 #define EGPT_ROWS32_ARGS                                                                                           \
     static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache),               \
         static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,    \
-        page_size, page_shift, scale, window, skip_single, part_o, part_ml, n_splits, n_tokens
+        page_size, page_shift, scale, window, skip_single, part_o, part_ml, n_splits, n_tokens, late
     if (n_splits > 1) attention_rows32_kernel<HD, RB, KS, true><<<grid, 64 * RB * KS, 0, s>>>(EGPT_ROWS32_ARGS);
     else attention_rows32_kernel<HD, RB, KS, false><<<grid, 64 * RB * KS, 0, s>>>(EGPT_ROWS32_ARGS);
 #undef EGPT_ROWS32_ARGS
@@ -1793,14 +1801,14 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
 template <int HD>
 static int launch_mixed(const void* qkv, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table, int table_width,
                         const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv,
-                        int page_size, int page_shift, float scale, int window, const int32_t* ranges, int slots, float* range_o,
+                        int page_size, int page_shift, float scale, int window, int late, const int32_t* ranges, int slots, float* range_o,
                         float* range_ml, hipStream_t s) {
     const long blocks = ((static_cast<long>(n_tokens) * (nq / nkv)) / 128 + n_seqs) * nkv;          // upper bound
     const long grid = blocks + static_cast<long>(slots) * nkv;
     if (grid > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
     attention_mixed_kernel<HD><<<static_cast<unsigned>(grid), 512, 0, s>>>(
         static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
-        block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, static_cast<int>(blocks), ranges,
+        block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, late, static_cast<int>(blocks), ranges,
         slots, range_o, range_ml);
     EGPT_CHECK_LAUNCH();
     attention_reduce_kernel<<<n_seqs * nq, 64, 0, s>>>(range_o, range_ml, static_cast<bf16_t*>(out), n_seqs * nq, HD, 1, q_start, q_len, nq,
@@ -1835,10 +1843,11 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
     int page_shift = 0;
     while ((1 << page_shift) < page_size) ++page_shift;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const int late = key_splits > 1 || (static_cast<long>(n_tokens) * (nq / nkv) + 15) / 16 * nkv > (hd == 64 ? kLateTiles64 : kLateTiles128);
     if (ranges && shape == 142 && key_splits == 1) {
         if (slots < n_seqs || slots > kRangeSlots) return EGPT_BAD_ARGUMENT;
         return (hd == 64 ? launch_mixed<64> : launch_mixed<128>)(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
-                                                                 n_tokens, nq, nkv, page_size, page_shift, scale, window, ranges, slots, range_o,
+                                                                 n_tokens, nq, nkv, page_size, page_shift, scale, window, late, ranges, slots, range_o,
                                                                  range_ml, s);
     }
 #define EGPT_TILED(HD_, RT_, KS_)                                                                                  \
@@ -1847,7 +1856,7 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
 #define EGPT_ROWS32(HD_, RB_, KS_)                                                                                 \
     launch_rows32<HD_, RB_, KS_>(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len,     \
                                  n_seqs, n_tokens, nq, nkv, page_size, page_shift, scale, window, skip_single,     \
-                                 part_o, part_ml, key_splits, s)
+                                 part_o, part_ml, key_splits, late, s)
     // shape = 10 * row tiles + key splits of a workgroup; 100 + 10 * blocks of 32 rows + key splits: the kernel of
     // 32-row blocks
     if (hd == 64) {

@@ -1,0 +1,82 @@
+"""How far prompt attention is from 64 bits: no further in the kernel of 32-row blocks than in the kernels that take the same calls otherwise."""
+import pytest
+import torch
+
+from easy_gpt.cpp_amd import kernels
+from easy_gpt.cpp_amd.kernels.hip import HipKernels
+from test_gpu_decode_ranges import attention64
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+PS = 16
+
+
+class Step:
+    """Requests of (tokens, tokens before them), bfloat16, scores of deviation `size`."""
+
+    def __init__(self, seqs, nq, nkv, hd, size):
+        g = torch.Generator(device=DEV).manual_seed(len(seqs) + hd)
+        self.seqs, self.nq, self.nkv, self.hd = seqs, nq, nkv, hd
+        t, kv = sum(n for n, _ in seqs), [n + p for n, p in seqs]
+        pages = [-(-n // PS) for n in kv]
+        self.qkv = torch.randn(t, nq + 2 * nkv, hd, device=DEV, generator=g)
+        self.qkv[:, :nq] *= size
+        self.qkv = self.qkv.to(torch.bfloat16)
+        self.kc = torch.randn(sum(pages), nkv, PS, hd, device=DEV, generator=g).to(torch.bfloat16)
+        self.vc = torch.randn(sum(pages), nkv, hd, PS, device=DEV, generator=g).to(torch.bfloat16)
+        numbers = torch.randperm(sum(pages), device=DEV, generator=g, dtype=torch.int32).split(pages)
+        self.table = torch.nn.utils.rnn.pad_sequence(numbers, batch_first=True, padding_value=0).contiguous()
+        ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+        starts = [sum(n for n, _ in seqs[:i]) for i in range(len(seqs))]
+        self.q_start, self.q_len, self.kv_len = ints(starts), ints([n for n, _ in seqs]), ints(kv)
+        self.max_q, self.max_kv, self.t = max(n for n, _ in seqs), max(kv), t
+        self.portion_kv = max(n + p for n, p in seqs if n > 1)
+        self.portions = [(i, at, n, n + p) for i, (at, (n, p)) in enumerate(zip(starts, seqs)) if n > 1]
+        self.want = [attention64(self.qkv[at : at + n, :nq].double(), self.kc, self.vc, self.table[i], m, 0, hd ** -0.5) for i, at, n, m in self.portions]
+
+    def error(self, out):
+        off = [(out[at : at + n].double() - w).norm() ** 2 for (_, at, n, _), w in zip(self.portions, self.want)]
+        return float((sum(off) / sum(w.norm() ** 2 for w in self.want)).sqrt())
+
+    def paged(self, k, dealt=False):
+        nq, nkv, hd = self.nq, self.nkv, self.hd
+        out = torch.empty(self.t, nq * hd, dtype=torch.bfloat16, device=DEV)
+        ranges = k.decode_ranges(self.kv_len, self.q_start, self.q_len, nkv, 0) if dealt else None
+        k.paged_attention_mixed(self.qkv.view(self.t, -1), out, self.kc, self.vc, self.table, self.q_start, self.q_len, self.kv_len, nq, nkv, hd, PS,
+                                hd ** -0.5, 0, self.max_q, self.max_kv, ranges=ranges, portion_kv=self.portion_kv)
+        return self.error(out)
+
+    def heads(self, k, **hints):
+        nq, nkv, hd = self.nq, self.nkv, self.hd
+        out = torch.empty(self.t, nq * hd, dtype=torch.bfloat16, device=DEV)
+        q = self.qkv[:, :nq].contiguous().view(self.t, -1)
+        k.window_attention(q, out, self.kc, self.vc, self.table, self.q_start, self.q_len, self.kv_len, nq, nkv, hd, hd, PS, hd ** -0.5, 0, 0, None,
+                           self.max_q, self.max_kv, **hints)
+        return self.error(out)
+
+
+# The same products and roundings in both, over keys that are split between wavefronts alike or finer: what is left is the order of float32 sums
+# and which keys meet in a tile, a few thousandths of the error over some 10^6 values; 12 to 20 % is what maxima of before cost here.
+NO_FURTHER = 1.01
+
+
+@pytest.mark.parametrize("size", [1.0, 2.0, 3.0])
+@pytest.mark.parametrize("nq,nkv,hd,before,seqs,dealt", [
+    (12, 2, 128, 42, [(512, 1100)], False), (12, 2, 128, 42, [(300, 1500)], False),
+    (12, 2, 128, 42, [(1, 100 + 200 * i) for i in range(20)] + [(1000, 900)], True), (28, 4, 128, 42, [(1, 2000)] * 8 + [(400, 1300)], True)])
+def test_portions(size, nq, nkv, hd, before, seqs, dealt, monkeypatch):
+    k = kernels.backend()
+    step = Step(seqs, nq, nkv, hd, size)
+    now = step.paged(k, dealt)
+    monkeypatch.setattr(HipKernels, "_portion_shape", classmethod(lambda cls, *a: (before, 1)))
+    assert now <= NO_FURTHER * step.paged(k)
+
+
+@pytest.mark.parametrize("size", [1.0, 2.0, 3.0])
+@pytest.mark.parametrize("nq,nkv,hd", [(14, 2, 64), (16, 4, 128)])
+def test_heads_by_themselves(size, nq, nkv, hd, monkeypatch):
+    k = kernels.backend()
+    step = Step([(3500, 0)], nq, nkv, hd, size)
+    now = step.heads(k)
+    monkeypatch.setattr(HipKernels, "_heads_blocks", staticmethod(lambda *a: 0))
+    assert now <= NO_FURTHER * step.heads(k)
