@@ -1116,7 +1116,9 @@ class HipKernels(KernelBackend):
         # Measured (us for one layer's prompt on a GPU that is warm; row tiles of 16 rows; shape = row tiles x key
         # splits of a workgroup, 1xx the kernel of 32-row blocks, whose tiles of 64 keys must be whole pages):
         #   head size 64, 14 heads on 2:   448 tiles 24: 8.9, 44: 10.2, 142: 11.2 |  896 tiles 24: 17.7, 44: 15.4, 142: 16.0
-        #     1,138 tiles 44: 19.3, 142: 19.1 | 12 prompts of 100, 1,050 tiles 44: 14.4, 142: 9.4 | 1,792 tiles 44: 30.9, 142: 25.1
+        #     1,226 tiles 44: 19.9, 142: 21.1 | 1,400 tiles 44: 22.0, 142: 23.8 | 12 prompts of 100, 1,050 tiles 44: 14.4, 142: 9.4 | 1,792
+        #     tiles 44: 30.9, 142: 25.1; two prompts of 700 16.6 and 15.2, but the result's error is 0.5 to 1 % larger (keys in two parts with
+        #     maxima of their own in place of four): only prompts that are one tile of 128 keys, where the parts are the same, go there earlier
         #     3,584 tiles 44: 86, 142: 47, 181: 72 | 7,168 tiles (8,192 tokens) 44: 293, 142: 156, 181: 146
         #   head size 128, 12 heads on 2:  192 tiles 42: 10.8, 142: 12.7 | 300 tiles 42: 15.3, 142: 14.8 | 768 tiles 42: 26.3, 142: 21.0 | 4
         #     prompts of 200, 600 tiles 42: 10.9, 142: 13.3 | 1,536 tiles 42: 47.4, 142: 32.8;  28 heads on 4: 448 tiles 42: 10.9, 142: 12.8 |
@@ -1127,7 +1129,7 @@ class HipKernels(KernelBackend):
         # 142: 16.7, 181: 12.9; 28 heads of 128 on 4, 6 of 300, 3,150 tiles 142: 27.9, 181: 19.4.
         blocks_of_32 = page_size <= 64
         if hd == 64:
-            shape = 24 if row_tiles <= 512 else 44 if row_tiles <= (1000 if blocks_of_32 else 2048) else 142 if blocks_of_32 else 42
+            shape = 24 if row_tiles <= 512 else 44 if row_tiles <= (2048 if not blocks_of_32 else 1536 if longest > 128 else 1000) else 142 if blocks_of_32 else 42
         else:
             shape = 22 if row_tiles <= 192 else 142 if blocks_of_32 and (row_tiles > 1024 or longest >= 400) else 42
         if shape == 142 and (row_tiles >= 5376 or (2048 < row_tiles <= 4096 and t >= 4 * longest)):
