@@ -1549,22 +1549,23 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
                                                table_width, q_start, kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, f, q_len, ranges);
 }
 
-// Portions of prompts in blocks of 128 rows and, behind them in the same launch, the requests of one token dealt out by `ranges`
+// Portions of prompts in blocks of 32 RB rows and, behind them in the same launch, the requests of one token dealt out by `ranges`
 // (range_slots workgroups for each kv head).  The portions' longest block of rows and the decoded tokens' longest range take about as long as
 // each other and neither fills the chip: 512 tokens of a new prompt beside 40 decoded ones behind 128 to 2,048, 12 heads of 128 on 2, are
 // 48 workgroups of 20 us and 256 of 13, a layer 32.1 us one launch after the other and 21.9 so.  A CU holds one workgroup of either kind.
-template <int HD>
+template <int HD, int RB, int KS>
 __global__ __launch_bounds__(512) void attention_mixed_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
     int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int late, int row_blocks,
     const int32_t* __restrict__ ranges, int range_slots, float* __restrict__ range_o, float* __restrict__ range_ml) {
-    __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, 4, 2>];
-    static_assert(kRows32Lds<HD, 4, 2> >= 8 * 16 * (HD + 2) * 4, "room for what eight wavefronts of decoded tokens leave");
+    static_assert(RB * KS == 8, "eight wavefronts, as the decoded tokens have");
+    __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, RB, KS>];
+    static_assert(kRows32Lds<HD, RB, KS> >= 8 * 16 * (HD + 2) * 4, "room for what eight wavefronts of decoded tokens leave");
     const int index = blockIdx.x;
     if (index < row_blocks) {
-        rows32_block<HD, 4, 2, false>(smem, index, 0, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,
+        rows32_block<HD, RB, KS, false>(smem, index, 0, qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv,
                                       page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0, (nq + 2 * nkv) * HD, late);
     } else {
         const int i = index - row_blocks;
@@ -1798,15 +1799,15 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
                                                              HD, n_splits);
 }
 
-template <int HD>
+template <int HD, int RB, int KS>
 static int launch_mixed(const void* qkv, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table, int table_width,
                         const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv,
                         int page_size, int page_shift, float scale, int window, int late, const int32_t* ranges, int slots, float* range_o,
                         float* range_ml, hipStream_t s) {
-    const long blocks = ((static_cast<long>(n_tokens) * (nq / nkv)) / 128 + n_seqs) * nkv;          // upper bound
+    const long blocks = ((static_cast<long>(n_tokens) * (nq / nkv)) / (32 * RB) + n_seqs) * nkv;          // upper bound
     const long grid = blocks + static_cast<long>(slots) * nkv;
     if (grid > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
-    attention_mixed_kernel<HD><<<static_cast<unsigned>(grid), 512, 0, s>>>(
+    attention_mixed_kernel<HD, RB, KS><<<static_cast<unsigned>(grid), 512, 0, s>>>(
         static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
         block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, late, static_cast<int>(blocks), ranges,
         slots, range_o, range_ml);
@@ -1844,11 +1845,11 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
     while ((1 << page_shift) < page_size) ++page_shift;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int late = key_splits > 1 || (static_cast<long>(n_tokens) * (nq / nkv) + 15) / 16 * nkv > (hd == 64 ? kLateTiles64 : kLateTiles128);
-    if (ranges && shape == 142 && key_splits == 1) {
+    if (ranges && key_splits == 1 && (shape == 142 || (shape == 124 && hd == 64))) {
         if (slots < n_seqs || slots > kRangeSlots) return EGPT_BAD_ARGUMENT;
-        return (hd == 64 ? launch_mixed<64> : launch_mixed<128>)(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs,
-                                                                 n_tokens, nq, nkv, page_size, page_shift, scale, window, late, ranges, slots, range_o,
-                                                                 range_ml, s);
+        return (shape == 124 ? launch_mixed<64, 2, 4> : hd == 64 ? launch_mixed<64, 4, 2> : launch_mixed<128, 4, 2>)(
+            qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len, n_seqs, n_tokens, nq, nkv, page_size, page_shift, scale,
+            window, late, ranges, slots, range_o, range_ml, s);
     }
 #define EGPT_TILED(HD_, RT_, KS_)                                                                                  \
     launch_tiled<HD_, RT_, KS_>(qkv, out, k_cache, v_cache, block_table, table_width, q_start, q_len, kv_len,      \

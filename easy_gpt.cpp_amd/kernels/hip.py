@@ -1049,11 +1049,13 @@ class HipKernels(KernelBackend):
                 if ranges is not None and singles and nq // nkv <= 16:
                     # the portions' blocks of rows and the decoded tokens' ranges in one launch, which has the portions in blocks of 128
                     # rows (us a layer, against the shape that the portions take alone and a second launch: 12 heads of 128 on 2, 40 of 128 to
-                    # 2,048 beside 512 21.9 against 32.1, 16 of 100 to 1,500 beside 64 15.1 and 17.9, 30 of 1,500 to 3,000 beside 256 behind 1,000
-                    # 31.3 and 50.0; 28 on 4, 3 of 1,200 beside 1,000 26.6 and 51.5; 14 heads of 64 on 2, 40 of 128 to 3,000 beside 512
-                    # 18.9 and 22.2, 20 of 2,500 to 4,000 beside 64 19.0 and 19.4, 20 of 100 to 8,000 beside 1,000 21.8 and 30.5)
+                    # 2,048 beside 512 22.8 against 32.9, 16 of 100 to 1,500 beside 64 15.8 and 18.5, 30 of 1,500 to 3,000 beside 256 behind 1,000
+                    # 33.6 and 51.3; 28 on 4, 3 of 1,200 beside 1,000 26.6 and 51.5), at head size 64 in blocks of 64, which split a row's keys
+                    # between four wavefronts, as the shapes 24 and 44 do, and are as near to 64 bits as those (142, with two, is 0.5 to 2 % further off: 14
+                    # heads on 2, 40 of 128 to 3,000 beside 512 21.2 against 22.7 (142: 20.0), behind 1,600 26.2 and 36.1 (33.4), 20 of 100 to 8,000 beside
+                    # 1,000 27.3 and 31.4 (23.6), 20 of 100 to 4,000 beside 1,700 34.1 and 36.2 (31.1))
                     if key_splits == 1 and page_size <= 64:
-                        shape = 142
+                        shape = 124 if hd == 64 and -(-t * (nq // nkv) // 16) * nkv <= 1536 else 142
                     slots = self._need_ranges(ranges, b, nkv)
                     range_o = torch.empty((slots, nq, hd), dtype=_F32, device=qkv.device)
                     range_ml = torch.empty((slots, nq, 2), dtype=_F32, device=qkv.device)

@@ -63,7 +63,8 @@ NO_FURTHER = 1.01
 @pytest.mark.parametrize("size", [1.0, 2.0, 3.0])
 @pytest.mark.parametrize("nq,nkv,hd,before,seqs,dealt", [
     (12, 2, 128, 42, [(512, 1100)], False), (12, 2, 128, 42, [(300, 1500)], False),
-    (12, 2, 128, 42, [(1, 100 + 200 * i) for i in range(20)] + [(1000, 900)], True), (28, 4, 128, 42, [(1, 2000)] * 8 + [(400, 1300)], True)])
+    (12, 2, 128, 42, [(1, 100 + 200 * i) for i in range(20)] + [(1000, 900)], True), (28, 4, 128, 42, [(1, 2000)] * 8 + [(400, 1300)], True),
+    (14, 2, 64, 24, [(1, 100 + 200 * i) for i in range(20)] + [(512, 1600)], True), (14, 2, 64, 44, [(1, 3000)] * 9 + [(1000, 1000), (200, 700)], True)])
 def test_portions(size, nq, nkv, hd, before, seqs, dealt, monkeypatch):
     k = kernels.backend()
     step = Step(seqs, nq, nkv, hd, size)

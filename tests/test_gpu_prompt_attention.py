@@ -50,7 +50,7 @@ def test_a_block_of_rows_finds_its_request_among_many(k, n, hd, dtype, shape, li
 
 
 @pytest.mark.parametrize("hd,nq,nkv", [(64, 14, 2), (128, 12, 2)])
-@pytest.mark.parametrize("portions", [[(300, 900), (129, 129)], [(1000, 1000)]])
+@pytest.mark.parametrize("portions", [[(300, 900), (129, 129)], [(1000, 1000)], [(1800, 1800)]])
 def test_portions_of_several_blocks_beside_decoded_tokens_in_one_launch(k, hd, nq, nkv, portions):  # noqa: F811
     decode_ranges.test_a_mixed_step_dealt_out(k, hd, nq, nkv, portions)
 
