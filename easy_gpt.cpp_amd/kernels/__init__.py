@@ -274,6 +274,15 @@ class KernelBackend:
         more than one token."""
         return self.paged_attention(*args, **kwargs)
 
+    def window_portion_choice(self, dtype, dk, dv, page_size, window, tokens, portion_kv):
+        """What window_attention_mixed, of heads without sink, cap, slopes, kept tokens, gate, block or second map, does otherwise for another
+        `portion_kv` in a step of so many tokens, as a value to compare."""
+        return None
+
+    def window_attention_mixed(self, *args, portion_kv=None, **kwargs):
+        """window_attention with a hint: the longest context of a request that brings more than one token."""
+        return self.window_attention(*args, **kwargs)
+
     def combine_attention(self, part_o, part_ml, out):
         """out act [T, nq*hd] from the parts of a split attention."""
         raise NotImplementedError

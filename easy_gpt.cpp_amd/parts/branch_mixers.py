@@ -118,6 +118,11 @@ class DistanceBiasAttention(_Branch):
         self.k_weight = self._to(get(p + n["k_norm"]), "compute", dtype, device)
         self.dist_bias = distance_bias_table(get(p + n["rel"]), self.bias_far).to(device)
 
+    def step_choices(self, page_size, tokens, requests, max_kv_len, spread, portion_kv):
+        if spread is not None:
+            return None
+        return kernels.backend().window_portion_choice(self.w_in.dtype, self.key_dim, self.value_dim, page_size, 0, tokens, min(portion_kv, max_kv_len))
+
     def branch(self, x, ctx, cache, state=None):
         k = kernels.backend()
         t = x.shape[0]
@@ -127,9 +132,9 @@ class DistanceBiasAttention(_Branch):
                            cache.slots if cache.writes else None, cache.k, cache.v, self.n_heads, self.n_kv_heads,
                            self.key_dim, self.value_dim, cache.page_size)
         attn = torch.empty((t, self.out_width), dtype=x.dtype, device=x.device)
-        k.window_attention(q, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len, self.n_heads,
-                           self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size, self.scale, 0, 0, None,
-                           ctx.max_q_len, ctx.max_kv_len, dist_bias=self.dist_bias)
+        k.window_attention_mixed(q, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len, self.n_heads,
+                                 self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size, self.scale, 0, 0, None,
+                                 ctx.max_q_len, ctx.max_kv_len, portion_kv=getattr(ctx, "portion_kv", None), dist_bias=self.dist_bias)
         gated = torch.empty_like(attn)
         k.sigmoid_gate(attn, 0, proj, self.q_width + self.k_width + self.v_width, gated)
         return k.product(gated, self.w_o, unrounded=True), self.b_o

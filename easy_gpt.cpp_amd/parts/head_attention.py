@@ -212,6 +212,12 @@ class NormedAttention(_TwoPhases):
         p = self.project(x, ctx)
         return kernels.backend().product(self._heads_out(p, ctx, cache), self.w_o, unrounded=True), None
 
+    def step_choices(self, page_size, tokens, requests, max_kv_len, spread, portion_kv):
+        if spread is not None or self.sink is not None or self.softcap is not None or self.gate_per_head or self.difference is not None or self.keep_first:
+            return None
+        return kernels.backend().window_portion_choice(self.w_qkv.dtype, self.key_dim, self.value_dim, page_size, self.window or 0, tokens,
+                                                       min(portion_kv, max_kv_len))
+
     def _heads_out(self, p, ctx, cache):
         if cache.writes and self.shares_cache:
             raise RuntimeError("a layer that reads another's keys and values must not write its cache")
@@ -249,9 +255,10 @@ class NormedAttention(_TwoPhases):
                           cache.slots if cache.writes else None, cache.k, cache.v, self.n_heads, self.stored_heads,
                           self.key_dim, self.value_dim, cache.page_size, **p.factor, **rotation)
         attn = torch.empty((t, self.out_width), dtype=p.dtype, device=p.device)
-        k.window_attention(q, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len,
-                           self.n_heads, self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size, self.scale,
-                           self.window or 0, self.keep_first, self.sink, ctx.max_q_len, ctx.max_kv_len, **scores)
+        k.window_attention_mixed(q, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len,
+                                 self.n_heads, self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size, self.scale,
+                                 self.window or 0, self.keep_first, self.sink, ctx.max_q_len, ctx.max_kv_len,
+                                 portion_kv=getattr(ctx, "portion_kv", None), **scores)
         if not self.gated:
             return attn
         gated = torch.empty_like(attn)

@@ -74,6 +74,11 @@ class BlockLocalAttention(Mixer):
         if self.slope_span is not None:
             self.slopes = head_slopes(self.n_heads, self.slope_span).to(device)
 
+    def step_choices(self, page_size, tokens, requests, max_kv_len, spread, portion_kv):
+        if spread is not None or self.block or self.slopes is not None:
+            return None
+        return kernels.backend().window_portion_choice(self.w_in.dtype, self.key_dim, self.value_dim, page_size, 0, tokens, min(portion_kv, max_kv_len))
+
     def forward(self, x, ctx, cache, state=None):
         if cache.writes == self.shares_cache:
             raise RuntimeError("a layer that shares another's cache must not write it, and a layer of its own must")
@@ -88,9 +93,9 @@ class BlockLocalAttention(Mixer):
             k.whole_norm_store(proj, None, q, self.q_weight, self.k_weight, self.eps, ctx.positions, 0.0, 0, cache.slots,
                                cache.k, cache.v, self.n_heads, self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size)
         attn = torch.empty((t, self.out_width), dtype=x.dtype, device=x.device)
-        k.window_attention(q, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len, self.n_heads,
-                           self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size, self.scale, 0, 0, None,
-                           ctx.max_q_len, ctx.max_kv_len, block=self.block, slopes=self.slopes)
+        k.window_attention_mixed(q, attn, cache.k, cache.v, cache.block_table, ctx.q_start, ctx.q_len, ctx.kv_len, self.n_heads,
+                                 self.n_kv_heads, self.key_dim, self.value_dim, cache.page_size, self.scale, 0, 0, None,
+                                 ctx.max_q_len, ctx.max_kv_len, portion_kv=getattr(ctx, "portion_kv", None), block=self.block, slopes=self.slopes)
         return k.product(attn, self.w_o, unrounded=True)
 
 

@@ -75,9 +75,10 @@ def test_portions(size, nq, nkv, hd, before, seqs, dealt, monkeypatch):
 
 @pytest.mark.parametrize("size", [1.0, 2.0, 3.0])
 @pytest.mark.parametrize("nq,nkv,hd", [(14, 2, 64), (16, 4, 128)])
-def test_heads_by_themselves(size, nq, nkv, hd, monkeypatch):
+@pytest.mark.parametrize("seqs", [[(3500, 0)], [(512, 700)], [(1000, 1500)], [(800, 200)], [(1, 1500)] * 20 + [(512, 0)], [(1, 800)] * 5 + [(400, 700)]])
+def test_heads_by_themselves(size, nq, nkv, hd, seqs, monkeypatch):
     k = kernels.backend()
-    step = Step([(3500, 0)], nq, nkv, hd, size)
-    now = step.heads(k)
+    step = Step(seqs, nq, nkv, hd, size)
+    now = step.heads(k, portion_kv=step.portion_kv)
     monkeypatch.setattr(HipKernels, "_heads_blocks", staticmethod(lambda *a: 0))
     assert now <= NO_FURTHER * step.heads(k)

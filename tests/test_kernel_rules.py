@@ -215,7 +215,7 @@ def attention_of(dtype, heads, kv_heads, head_dim, window=None):
 
 
 class RulesOnly(EmulatedKernels):
-    deals_out, portion_choice = K.deals_out, K.portion_choice
+    deals_out, portion_choice, window_portion_choice = K.deals_out, K.portion_choice, K.window_portion_choice
 
 
 @pytest.fixture()
@@ -253,3 +253,24 @@ def test_steps_with_the_same_kernels_are_kept_by_the_same_hints(rules_only):
                     own *= 2
                 assert longest <= bound <= most
                 assert part.step_choices(16, tokens, 8, most, None, bound) == part.step_choices(16, tokens, 8, most, None, min(own, most))
+
+
+def test_heads_by_themselves_are_kept_by_what_lies_in_front_of_portions(rules_only):
+    from easy_gpt.cpp_amd.parts import PartSpec, make_part
+
+    assert K._heads_portion(96, 96) and K._heads_portion(800, 300) and not K._heads_portion(95, 95) and not K._heads_portion(800, 801)
+
+    def part(dtype, dim=64, **kw):
+        p = make_part("mixer", PartSpec("normed_attention", dict(n_heads=4, n_kv_heads=2, key_dim=dim, value_dim=dim, scale=0.1, eps=1e-6, **kw), "a."), hidden_size=32)
+        p.load(lambda name: torch.zeros(next(s for s in p.param_specs() if s.name == name).shape), dtype, "cpu")
+        return p
+
+    bound = lambda p, tokens, longest, most: _same_portion(lambda n: p.step_choices(16, tokens, 8, most, None, n), tokens, longest, most)  # noqa: E731
+    plain = part(torch.bfloat16)
+    # two kinds of steps of one size: new prompts, and portions behind a prefix, however long; one where nothing goes by it
+    assert bound(plain, 512, 300, 4096) == 512 and {bound(plain, 512, n, 4096) for n in (513, 1024, 4096)} == {4096}
+    assert bound(plain, 64, 64, 4096) == bound(plain, 64, 3000, 4096) == 4096
+    for other in (part(torch.float32), part(torch.bfloat16, 96), part(torch.bfloat16, sink=True), part(torch.bfloat16, softcap=30.0),
+                  part(torch.bfloat16, window=100), part(torch.bfloat16, window=500, keep_first=4), part(torch.bfloat16, gated="heads")):
+        assert {bound(other, 512, n, 4096) for n in (300, 513, 4096)} == {4096}
+    assert plain.step_choices(16, 40, 40, 4096, 1, None) is None
