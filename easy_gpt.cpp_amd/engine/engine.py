@@ -394,24 +394,28 @@ class Engine:
         position + 1 and whose block table is its request's.  That shape depends on the number of tokens alone,
         so it is captured and replayed like a decode step, where the same step run kernel by kernel would spend
         twice its device time on the host.  Keys and values of all rows are stored before attention reads them
-        (`rows_independent` is False).  Logits are computed for the wanted rows, their number rounded up to a power of two.  Not for
-        models with per-request state, whose parts walk a portion token after token."""
+        (`rows_independent` is False).  Logits are computed for as many rows as there are tokens, the wanted ones first, whose numbers come
+        with the step: a graph for each number of wanted rows would be 0 to 1 % shorter (20 rows, 4 wanted, of the 0.5B sizes 1,171 and 1,180 us,
+        60 and 1 1,230 and 1,238), and a capture more for every pair of tokens and wanted rows that a server meets.  Not for models with
+        per-request state, whose parts walk a portion token after token."""
         rcs = self._check(entries)
         counts = [len(e.tokens) for e in entries]
         t = sum(counts)
         with self.cache.reserved(rcs, counts):
             widths = self._table_widths(rcs)
             kv_bound = -(-max(rc.num_tokens + n for rc, n in zip(rcs, counts)) // 512) * 512
-            n_want = sum(len(e.want) for e in entries)
-            r_pad = 1
-            while r_pad < min(n_want, t):
-                r_pad *= 2
-            r_pad = min(r_pad, t) if n_want <= t else n_want            # (a row may be wanted more than once)
-            key = (t, tuple(widths), kv_bound, r_pad)
-            plan = self._plan(self._row_plans, key, lambda: _DecodePlan(self, t, widths, kv_bound, rows_independent=False, wanted=r_pad))
-            plan.fill_rows(rcs, entries, counts)
+            want, base = [], 0
+            for e, n in zip(entries, counts):
+                want.extend(base + int(w) for w in e.want)
+                base += n
+            key = (t, tuple(widths), kv_bound)
+            plan = self._plan(self._row_plans, key, lambda: _DecodePlan(self, t, widths, kv_bound, rows_independent=False))
+            more = len(want) > t                           # (a row may be wanted more than once: all rows then, gathered behind the graph)
+            plan.fill_rows(rcs, entries, counts, range(t) if more else want)
             logits = self._run(plan)
-        return logits[:n_want] if n_want else None
+        if more:
+            return logits.index_select(0, torch.tensor(want, dtype=torch.int64, device=self.device))
+        return logits[: len(want)] if want else None
 
     # ------------------------------------------------------------------ any mix, from a graph for its padded size
     def _step_padded(self, entries) -> torch.Tensor | None:
@@ -599,21 +603,17 @@ class _PaddedPlan:
 class _DecodePlan:
     """Static device buffers, a host mirror and the captured graph of one decode batch shape."""
 
-    def __init__(self, engine: Engine, batch: int, widths: list[int], kv_bound: int, rows_independent: bool = True, spread: int = 0,
-                 wanted: int | None = None):
+    def __init__(self, engine: Engine, batch: int, widths: list[int], kv_bound: int, rows_independent: bool = True, spread: int = 0):
         self.batch, self.widths = batch, list(widths)
         dev = engine.device
         n_groups = len(widths)
         b = batch
-        # the rows' numbers, the wanted rows (a step of decoded tokens wants all of them: its row numbers) and the block tables lie behind
-        # each other, so that a step is one copy to the device
+        # the rows' numbers and the block tables lie behind each other, so that a step is one copy to the device
         n_small, n_tab = (7 + n_groups) * b, max(sum(b * w for w in widths), 1)
-        n_want = wanted or 0
-        self.host = torch.full((n_small + n_want + n_tab,), -1, dtype=torch.int32).pin_memory()
-        self.dev = torch.full((n_small + n_want + n_tab,), -1, dtype=torch.int32, device=dev)
+        self.host = torch.full((n_small + n_tab,), -1, dtype=torch.int32).pin_memory()
+        self.dev = torch.full((n_small + n_tab,), -1, dtype=torch.int32, device=dev)
         self.host_small, self.dev_small = self.host[:n_small], self.dev[:n_small]
-        self.host_tab, self.dev_tab = self.host[n_small + n_want :], self.dev[n_small + n_want :]
-        self.np_want = self.host[n_small : n_small + n_want].numpy()
+        self.host_tab, self.dev_tab = self.host[n_small:], self.dev[n_small:]
         self.np_small = self.host_small.numpy()
         v = lambda i: self.dev_small[i * b : (i + 1) * b]
         groups, off = [], 0
@@ -623,7 +623,7 @@ class _DecodePlan:
         ps = engine.page_size
         self.ctx = StepContext(
             num_tokens=b, num_seqs=b, token_ids=v(0), positions=v(1), q_start=v(2), q_len=v(3), kv_len=v(4),
-            want_rows=v(6) if wanted is None else self.dev[n_small : n_small + n_want], max_q_len=1, max_kv_len=min([kv_bound] + [w * ps for w in widths]),
+            want_rows=v(6), max_q_len=1, max_kv_len=min([kv_bound] + [w * ps for w in widths]),
             q_start_host=list(range(b)), q_len_host=[1] * b, kv_len_host=[0] * b,
             state_slots=v(5), state_slots_host=[0] * b, groups=groups, page_size=ps, kv_storage=engine.kv,
             state_storage=engine.states, cache_location=engine.model.cache_location,
@@ -680,23 +680,19 @@ class _DecodePlan:
             self.copied = torch.cuda.Event()
         self.copied.record()
 
-    def fill_rows(self, rcs, entries, counts) -> None:
+    def fill_rows(self, rcs, entries, counts, want) -> None:
         """The metadata of a step whose tokens are laid out as rows of one token each: the cache manager's library
         writes the step as it is (positions and slots per token, a table per request), and the per-request parts
-        are repeated for every token of the request."""
+        are repeated for every token of the request.  want: the rows whose logits are wanted, at most as many as there are tokens."""
         if self.copied is not None:
             self.copied.synchronize()
         t, b = self.batch, len(rcs)
         n_groups = len(self.widths)
         small = self.np_small.reshape(7 + n_groups, t)
         pos = 0
-        want: list[int] = []
         for e, n in zip(entries, counts):
             small[0, pos : pos + n] = e.tokens
-            want.extend(pos + int(w) for w in e.want)
             pos += n
-        self.np_want[: len(want)] = want
-        self.np_want[len(want) :] = 0
         per_request = np.empty((4, b), dtype=np.int32)               # q_start, q_len, kv_len, state slots
         slots = np.empty(max(n_groups * t, 1), dtype=np.int32)
         tables = np.empty(max(sum(b * w for w in self.widths), 1), dtype=np.int32)
@@ -705,11 +701,10 @@ class _DecodePlan:
             (small[1].ctypes.data, per_request[0].ctypes.data, per_request[1].ctypes.data, per_request[2].ctypes.data,
              per_request[3].ctypes.data, slots.ctypes.data if n_groups else None, tables.ctypes.data if n_groups else None),
         )
-        rows = np.arange(t, dtype=np.int32)
         reps = np.asarray(counts)
-        small[2], small[3], small[4] = rows, 1, small[1] + 1
+        small[2], small[3], small[4] = np.arange(t, dtype=np.int32), 1, small[1] + 1
         small[5] = np.repeat(per_request[3], reps)
-        small[6] = rows
+        small[6, : len(want)], small[6, len(want) :] = want, 0
         tab = self.host_tab.numpy()
         off_in = off_out = 0
         for g, w in enumerate(self.widths):
