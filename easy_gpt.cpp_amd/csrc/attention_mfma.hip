@@ -621,9 +621,10 @@ __device__ __forceinline__ void rows32_block(
     // n_splits > 1: the tiles of keys are dealt over as many workgroups (`part`), each of which leaves its rows'
     // unnormalised result with its maximum and sum in part_o / part_ml for the kernel that combines them
     // (SPLIT is a parameter of the template so that the kernel without it is compiled as if this were not here; a
-    // workgroup takes four tiles at least: fewer are not worth sharing)
+    // workgroup takes four tiles at least, three at head size 128, where a tile takes twice as long: fewer are not worth sharing)
+    constexpr int kLeastTiles = HD == 128 ? 3 : 4;
     const int t_first = blk_lo / KT, t_last = blk_p_hi / KT + 1;
-    const int t_per = SPLIT ? max((t_last - t_first + n_splits - 1) / n_splits, 4) : t_last - t_first;
+    const int t_per = SPLIT ? max((t_last - t_first + n_splits - 1) / n_splits, kLeastTiles) : t_last - t_first;
     const int t_begin = SPLIT ? t_first + part * t_per : t_first;
     const int t_end = SPLIT ? min(t_last, t_begin + t_per) : t_last;
     [[maybe_unused]] const size_t part_row0 = SPLIT ? static_cast<size_t>(part) * n_tokens * nq : 0;

@@ -40,6 +40,29 @@ def test_nothing_behind_the_context_counts(k, hd, shape, window, ps):  # noqa: F
     assert torch.isfinite(outs[0].float()).all() and torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("hd,least", [(64, 4), (128, 3)])
+def test_key_ranges_of_the_fewest_tiles_that_the_rule_asks_for(k, hd, least):  # noqa: F811
+    # portions behind a prefix whose tiles of 128 keys are dealt out in ranges of `least`: every workgroup has keys, and one range more
+    # than that leaves the others as they were, with nothing for itself
+    nq, nkv, ps, n, ranges = 6, 2, 16, 64, 8
+    kv = ranges * least * 128
+    assert k._portion_shape(n, nq, nkv, hd, ps, 32 * 128) == (142, 32 // least)
+    kc, vc, table, _, _ = build_paged([(n, kv)], nkv, hd, ps, torch.bfloat16, seed=2)
+    qkv = torch.randn(n, (nq + 2 * nkv) * hd, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(DEV)
+    one = lambda v: torch.tensor([v], dtype=torch.int32, device=DEV)  # noqa: E731
+    start, length, context = one(0), one(n), one(kv)
+    outs = []
+    for splits in (ranges, ranges + 1):
+        out = torch.empty(n, nq * hd, dtype=torch.bfloat16, device=DEV)
+        part_o, part_ml = torch.empty(splits, n, nq, hd, device=DEV), torch.full((splits, n, nq, 2), 7.0, device=DEV)
+        k._run("egpt_paged_attention_tiled", qkv.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], start.data_ptr(),
+               length.data_ptr(), context.data_ptr(), 1, n, nq, nkv, hd, ps, hd ** -0.5, 0, 142, splits, part_o.data_ptr(), part_ml.data_ptr(), 0, 0, 0, k._stream())
+        torch.cuda.synchronize()
+        assert torch.isfinite(part_ml[:ranges, -1]).all() and torch.all(part_ml[ranges:, :, :, 0] == float("-inf"))
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("n", [4, 5, 64, 65, 130])
 @pytest.mark.parametrize("hd,dtype,shape,line", [(64, torch.bfloat16, 24, 1.2e-2), (128, torch.bfloat16, 142, 1.2e-2), (48, torch.float32, None, 2e-6)])
 def test_a_block_of_rows_finds_its_request_among_many(k, n, hd, dtype, shape, line):  # noqa: F811
