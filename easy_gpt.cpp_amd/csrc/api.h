@@ -88,7 +88,8 @@ int egpt_heads_attention(const void* q, void* out, const void* k_cache, const vo
                          int page_size, float scale, int window, const float* dist_bias, int dist_far, int row_blocks, void* stream);
 // Prompt portions: the wavefronts of a workgroup share key/value tiles through LDS (n_splits == 1 semantics);
 // page sizes that are powers of two; shape = 10 * row tiles + key splits per workgroup (41, 42, 44, 22, 24), or
-// 100 + 10 * blocks of 32 rows + key splits (121, 122, 124, 141, 142, 181; page sizes up to 64).
+// 100 + 10 * blocks of 32 rows + key splits (121, 122, 124, 141, 142, 181; page sizes up to 64); 1,000 more: rows are rescaled late behind
+// long contexts, as they are with key_splits > 1 (faster, and further from 64 bits).
 // key_splits > 1 (shapes from 100 on): the tiles of keys that a block of rows walks are dealt over as many workgroups,
 // whose results part_o [key_splits][n_tokens][nq][hd] and part_ml [key_splits][n_tokens][nq][2] (float32) hold until a
 // second kernel has combined them.

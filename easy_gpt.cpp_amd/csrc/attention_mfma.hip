@@ -567,14 +567,14 @@ struct DistanceBias {
 constexpr int kBiasFront = 96, kBiasBack = 64;
 __host__ __device__ constexpr int bias_row(int far) { return (kBiasFront + far + 1 + kBiasBack + 1) | 1; }     // (odd: the heads' banks differ)
 
-// Rows are rescaled late, by a maximum that has grown by 2^8, in steps of more row tiles of 16 than this and where the keys are dealt out,
-// behind so many keys.  Against a row's own maximum the largest probability is one, which bfloat16 has exactly; against an older
+// Rows are rescaled late, when their maximum has grown by 2^8, where the caller says so and where the keys are dealt out, behind so many
+// keys.  Against a row's own maximum the largest probability is one, which bfloat16 has exactly; against an older
 // one it is rounded like the others, and the result is further from 64 bits: 2-norm of its error at scores of deviation two, late
 // and exact, head size 64, 2,048 / 5,000 tokens 0.00185 and 0.00181 / 0.00195 and 0.00182; 512 tokens behind 1,600 keys 0.00216 and 0.00184 (the
 // kernel of 16-row tiles 0.00180).  The large steps gain 2 to 6 % by it (us a layer: 14 heads of 64 on 2, 8,191 tokens 168 and 175; 28 of 128
 // on 4, 5,000 tokens 195 and 205) and are nearer to 64 bits so than with every row late from the first key on (0.00199, 0.00205); the others,
 // which have kernels with exact maxima to compare with, keep them.
-constexpr int kLateFrom = 1536, kLateTiles64 = 1536, kLateTiles128 = 1024;
+constexpr int kLateFrom = 1536;
 
 // Workgroup `index` of a launch (and range `part` of the keys); a token's queries lie `width` values behind those of the one before.
 // WIDE: scores of any finite size.  score x scale - maximum x scale as one multiply-add has the rounding of its last operand in it, the
@@ -691,7 +691,7 @@ __device__ __forceinline__ void rows32_block(
     // instructions (the probabilities of tile i).  The two wavefronts of a SIMD take them in turn: wavefronts 4 to 7 are one
     // step behind, so that one of the two is at its matrix instructions while the other is at its vector instructions, and a
     // barrier behind every step keeps them so.
-    // With `late`, behind long contexts the accumulated output is rescaled only when a row's maximum has grown by more than 2^kSlack since
+    // With `late` (or SPLIT), behind long contexts the accumulated output is rescaled only when a row's maximum has grown by more than 2^kSlack since
     // the last time: until then the exponentials are taken against the old maximum, so they may reach 2^kSlack instead of 1, which
     // float32 sums and bfloat16 probabilities (the same relative precision at any magnitude) do not mind.
     // Keys and values go from memory straight to LDS, 16 keys (never more than a page's) to a load's base address and a
@@ -827,7 +827,7 @@ __device__ __forceinline__ void rows32_block(
     };
     // (Against the row's own maximum the largest probability is one, which bfloat16 has exactly; against an older one it is rounded like
     // the others, at any context: see kLateFrom.)
-    const float slack = late && blk_p_hi >= kLateFrom ? kSlack / scale2 : 0.f;
+    const float slack = (SPLIT || late) && blk_p_hi >= kLateFrom ? kSlack / scale2 : 0.f;
     [[maybe_unused]] bool beyond_shift = false;      // WIDE: a row of the wavefront has such a maximum
     float limit = -INFINITY, shift = 0.0f;           // a row's maximum beyond which there is rescaling; what the exponents are shifted by
     const float* const bias_of_row = BIAS ? bias.lds + (valid ? r % group_size : 0) * bias_row(bias.far) + kBiasFront : nullptr;
@@ -1832,6 +1832,9 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
         return EGPT_BAD_ARGUMENT;
     if ((hd != 64 && hd != 128) || page_size < 16 || (page_size & (page_size - 1)) != 0 || nkv > 65535)
         return EGPT_UNSUPPORTED_SIZE;
+    const int late = shape >= 1000;
+    shape -= late * 1000;
+    if (late && shape < 100) return EGPT_BAD_ARGUMENT;
     const int skip_single = single_waves != 0;
     if (skip_single) {
         if (single_waves < 0 || single_splits < 1 || (single_splits > 1 && (!part_o || !part_ml)))
@@ -1845,7 +1848,6 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
     int page_shift = 0;
     while ((1 << page_shift) < page_size) ++page_shift;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int late = key_splits > 1 || (static_cast<long>(n_tokens) * (nq / nkv) + 15) / 16 * nkv > (hd == 64 ? kLateTiles64 : kLateTiles128);
     if (ranges && key_splits == 1 && (shape == 142 || (shape == 124 && hd == 64))) {
         if (slots < n_seqs || slots > kRangeSlots) return EGPT_BAD_ARGUMENT;
         return (shape == 124 ? launch_mixed<64, 2, 4> : hd == 64 ? launch_mixed<64, 4, 2> : launch_mixed<128, 4, 2>)(

@@ -1055,7 +1055,7 @@ class HipKernels(KernelBackend):
                     # heads on 2, 40 of 128 to 3,000 beside 512 21.2 against 22.7 (142: 20.0), behind 1,600 26.2 and 36.1 (33.4), 20 of 100 to 8,000 beside
                     # 1,000 27.3 and 31.4 (23.6), 20 of 100 to 4,000 beside 1,700 34.1 and 36.2 (31.1))
                     if key_splits == 1 and page_size <= 64:
-                        shape = 124 if hd == 64 and -(-t * (nq // nkv) // 16) * nkv <= 1536 else 142
+                        shape = 124 if hd == 64 and -(-t * (nq // nkv) // 16) * nkv <= 1536 else 1142 if shape > 1000 else 142
                     slots = self._need_ranges(ranges, b, nkv)
                     range_o = torch.empty((slots, nq, hd), dtype=_F32, device=qkv.device)
                     range_ml = torch.empty((slots, nq, 2), dtype=_F32, device=qkv.device)
@@ -1136,6 +1136,10 @@ class HipKernels(KernelBackend):
             shape = 22 if row_tiles <= 192 else 142 if blocks_of_32 and (row_tiles > 1024 or longest >= 400) else 42
         if shape == 142 and (row_tiles >= 5376 or (2048 < row_tiles <= 4096 and t >= 4 * longest)):
             shape = 181
+        # (1,000 more: rows rescaled late, 2 to 6 % of the time.  Large steps and portions behind a prefix, not where the kernels of 16-row
+        # tiles or of other heads, which have exact maxima, would be taken otherwise: see kLateFrom)
+        if shape > 100 and row_tiles > (1536 if hd == 64 else 1024):
+            shape += 1000
         # Portions behind a prefix walk many keys per row and are few blocks of rows: the kernel of 32-row blocks
         # with 128 rows to a workgroup, and the tiles of keys of a block of rows dealt over as many workgroups
         # as give every CU one, in two only from 40 tiles on.  Measured (us, a layer; shape x workgroups that share the keys): head size 64,
@@ -1149,7 +1153,7 @@ class HipKernels(KernelBackend):
         # 128 on 2: 51.8 us a layer in four key ranges, 48.0 in one; 8 behind 1,400 and 28 heads on 4 46.6 and 31.1)
         if (blocks_of_32 and longest >= 2 * t
                 and longest >= (cls.prefix_keys if hd == 64 else cls.prefix_keys // 2)):
-            shape = 142
+            shape = 1142
             workgroups = -(-row_tiles // 8)
             tiles = -(-longest // 128)
             key_splits = max(1, min(256 // workgroups, tiles // (4 if hd == 64 else 3), 16))

@@ -46,7 +46,7 @@ def test_key_ranges_of_the_fewest_tiles_that_the_rule_asks_for(k, hd, least):  #
     # than that leaves the others as they were, with nothing for itself
     nq, nkv, ps, n, ranges = 6, 2, 16, 64, 8
     kv = ranges * least * 128
-    assert k._portion_shape(n, nq, nkv, hd, ps, 32 * 128) == (142, 32 // least)
+    assert k._portion_shape(n, nq, nkv, hd, ps, 32 * 128) == (1142, 32 // least)
     kc, vc, table, _, _ = build_paged([(n, kv)], nkv, hd, ps, torch.bfloat16, seed=2)
     qkv = torch.randn(n, (nq + 2 * nkv) * hd, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(DEV)
     one = lambda v: torch.tensor([v], dtype=torch.int32, device=DEV)  # noqa: E731
@@ -98,3 +98,11 @@ def test_decoded_tokens_of_one_segment(k, hd, dtype, line, window):  # noqa: F81
         k.paged_attention(qkv, out, kc, vc, wide.contiguous(), start, one, kv, nq, nkv, hd, 16, hd ** -0.5, window, 1, longest)
         outs.append(out)
     assert torch.equal(*outs)
+
+
+def test_rows_are_rescaled_late_in_blocks_of_32_only(k):  # noqa: F811
+    p = torch.zeros(1 << 16, device=DEV, dtype=torch.uint8).data_ptr()
+    for shape in (1044, 1024, 1000, 2142):
+        with pytest.raises(RuntimeError):
+            k._run("egpt_paged_attention_tiled", p, p, p, p, p, 1, p, p, p, 1, 1, 2, 1, 64, 16, 0.1, 0, shape, 1, None, None, 0, 0, 0, k._stream())
+    assert run_paged(k, [(64, 2000), (200, 1700)], 6, 2, 64, 16, torch.bfloat16, tiled_shape=1142, ramp=0.9, seed=3) <= 1.2e-2

@@ -28,10 +28,12 @@ def test_decode_attention_shapes_are_launchable():
 def test_shapes_of_new_prompts():
     # (tokens, nq, nkv, head size, page size, longest context) and the workgroup shape, at and around the lines
     for sizes, shape in [((580, 14, 2, 64, 16, 580), 24), ((590, 14, 2, 64, 16, 590), 44), ((1300, 14, 2, 64, 16, 1300), 44), ((1400, 14, 2, 64, 16, 700), 44),
-                         ((1755, 14, 2, 64, 16, 1755), 44), ((1756, 14, 2, 64, 16, 1756), 142), ((1200, 14, 2, 64, 16, 100), 142),
+                         ((1755, 14, 2, 64, 16, 1755), 44), ((1756, 14, 2, 64, 16, 1756), 1142), ((1200, 14, 2, 64, 16, 100), 142),
                          ((1100, 14, 2, 64, 16, 100), 44), ((1800, 14, 2, 64, 128, 1800), 44), ((2400, 14, 2, 64, 128, 2400), 42),
                          ((200, 12, 2, 128, 16, 200), 22), ((300, 12, 2, 128, 16, 300), 42), ((400, 12, 2, 128, 16, 400), 142),
-                         ((1000, 28, 4, 128, 128, 1000), 42), ((6500, 14, 2, 64, 16, 6500), 181)]:
+                         ((1000, 28, 4, 128, 128, 1000), 42), ((6500, 14, 2, 64, 16, 6500), 1181),
+                         ((800, 28, 4, 128, 16, 800), 1142), ((500, 28, 4, 128, 16, 500), 142), ((512, 28, 4, 128, 16, 4096), 1142),
+                         ((512, 28, 4, 128, 16, 1000), 142)]:
         assert K._portion_shape(*sizes) == (shape, 1), sizes
 
 
