@@ -1126,15 +1126,12 @@ class HipKernels(KernelBackend):
         #     prompts of 200, 600 tiles 42: 10.9, 142: 13.3 | 1,536 tiles 42: 47.4, 142: 32.8;  28 heads on 4: 448 tiles 42: 10.9, 142: 12.8 |
         #     700 tiles 15.3 both | 1,344 tiles 42: 28.3, 142: 19.2 | 3,584 tiles 42: 102, 142: 46, 181: 53 | 5,376 tiles 42: 199, 142: 87,
         #     181: 82 | 7,168 tiles 42: 331, 142: 139, 181: 122
-        # A workgroup of 256 rows (181) reads a tile's keys half as often, but a single prompt needs more than 20 of them for every 16
-        # CUs before their different lengths even out; prompts of the same length need only one for a CU: 8 of 301, 2,107 tiles, head size 64
-        # 142: 16.7, 181: 12.9; 28 heads of 128 on 4, 6 of 300, 3,150 tiles 142: 27.9, 181: 19.4.
         blocks_of_32 = page_size <= 64
         if hd == 64:
             shape = 24 if row_tiles <= 512 else 44 if row_tiles <= (2048 if not blocks_of_32 else 1536 if longest > 128 else 1000) else 142 if blocks_of_32 else 42
         else:
             shape = 22 if row_tiles <= 192 else 142 if blocks_of_32 and (row_tiles > 1024 or longest >= 400) else 42
-        if shape == 142 and (row_tiles >= 5376 or (2048 < row_tiles <= 4096 and t >= 4 * longest)):
+        if shape == 142 and cls._blocks_of_256(hd, row_tiles, t, longest):
             shape = 181
         # (1,000 more: rows rescaled late, 2 to 6 % of the time.  Large steps and portions behind a prefix, not where the kernels of 16-row
         # tiles or of other heads, which have exact maxima, would be taken otherwise: see kLateFrom)
@@ -1160,6 +1157,19 @@ class HipKernels(KernelBackend):
             if key_splits == 2 and tiles < 40:
                 key_splits = 1
         return shape, key_splits
+
+    @staticmethod
+    def _blocks_of_256(hd, row_tiles, t, longest) -> bool:
+        """Whether a workgroup of the kernel of 32-row blocks takes 256 rows (181) and not 128 (142).  It reads a tile's keys half as often, but a
+        single prompt needs more than 20 of them for every 16 CUs before their different lengths even out; prompts of the same length need only one
+        for a CU.  us of 181 for one of 142, as many prompts of one length as named: 14 heads of 64 on 2, 2,100 tiles 1: 1.55, 4: 1.19, 5: 1.07, 6: 1.00, 8:
+        0.81, 12: 0.75; 2,400 4: 1.06, 5: 0.90; 2,800 1: 1.59, 3: 1.15, 4: 0.97, 6: 0.82; 4,000 1: 1.37, 3: 1.00, 4: 0.92, 8: 0.76; 5,300 1: 1.04, 4: 1.05, 12: 0.89;
+        5,800 1: 1.03, 2: 0.92, 4: 1.07, 8: 0.93; 7,000 1: 0.94, 3: 1.02.  12 of 128 on 2, 2,100 1: 1.53, 3: 1.20, 4: 0.99, 6: 0.95, 12: 0.76; 4,000 1: 1.27, 3: 0.95, 6:
+        0.85; 28 on 4, 2,100 1: 1.41, 2: 1.02, 3: 0.91, 4: 0.80, 12: 0.63; 4,000 1: 1.11, 3: 0.85, 4: 0.76; 5,800 1: 0.89, 4: 0.93.  (Between 4,096 and 5,376 three prompts
+        and more would gain 4 to 17 %, one would lose as much.)"""
+        if row_tiles >= 5376:
+            return True
+        return 2048 < row_tiles <= 4096 and t >= (6 if hd == 64 and row_tiles <= 2400 else 4) * longest
 
     @classmethod
     def portion_choice(cls, dtype, nq, nkv, hd, page_size, tokens, portion_kv):
@@ -1582,7 +1592,7 @@ class HipKernels(KernelBackend):
         if 0 < window < 192 or max_kv_len > ((4 if hd == 64 else 3) * t if t >= 256 else 512 if hd == 64 else 300):
             return 0
         row_tiles = -(-t * (nq // nkv) // 16) * nkv
-        return 8 if row_tiles >= 5376 or (2048 < row_tiles <= 4096 and t >= 4 * max_kv_len) else 4
+        return 8 if HipKernels._blocks_of_256(hd, row_tiles, t, max_kv_len) else 4
 
     # ------------------------------------------------------------------ stream operations beyond the RMS norm
     def embed_scaled(self, token_ids, table, factor, out):

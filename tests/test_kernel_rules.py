@@ -33,7 +33,8 @@ def test_shapes_of_new_prompts():
                          ((200, 12, 2, 128, 16, 200), 22), ((300, 12, 2, 128, 16, 300), 42), ((400, 12, 2, 128, 16, 400), 142),
                          ((1000, 28, 4, 128, 128, 1000), 42), ((6500, 14, 2, 64, 16, 6500), 1181),
                          ((800, 28, 4, 128, 16, 800), 1142), ((500, 28, 4, 128, 16, 500), 142), ((512, 28, 4, 128, 16, 4096), 1142),
-                         ((512, 28, 4, 128, 16, 1000), 142)]:
+                         ((512, 28, 4, 128, 16, 1000), 142), ((2400, 14, 2, 64, 16, 600), 1142), ((2400, 14, 2, 64, 16, 400), 1181),
+                         ((2800, 14, 2, 64, 16, 700), 1181), ((2800, 12, 2, 128, 16, 700), 1181), ((2800, 12, 2, 128, 16, 701), 1142)]:
         assert K._portion_shape(*sizes) == (shape, 1), sizes
 
 
