@@ -18,6 +18,30 @@ def test_workgroups_of_eight_wavefronts(k, hd, shape, window, ps, splits):  # no
     assert run_paged(k, seqs, 7, 1, hd, ps, torch.bfloat16, window=window, tiled_shape=shape, key_splits=splits, ramp=0.9, seed=3) <= 1.2e-2
 
 
+@pytest.mark.parametrize("hd,shape", [(64, 1142), (64, 1181), (128, 1142), (128, 1181), (64, 181), (128, 142), (128, 181)])
+@pytest.mark.parametrize("ramp", [0.26, 0.9, -0.26, 4.0])
+def test_scores_that_grow_along_long_contexts(k, hd, shape, ramp):  # noqa: F811
+    # behind 1,536 keys the shapes from 1,000 on rescale a row only when its maximum has grown by 2^8: scores that rise by about 3 (in powers of
+    # two) from one 64 keys to the next stay below that for several tiles in a row, a rise of 10 is over it in every tile, 45 by far; falling
+    # scores never rescale after the first tile.  Blocks of rows on both sides of the 1,536, one head to a group and sixteen, a window
+    seqs = [(300, 2500), (64, 64), (33, 1700), (200, 1600)]
+    r = ramp * (hd / 64) ** 0.5
+    assert run_paged(k, seqs, 6, 2, hd, 16, torch.bfloat16, tiled_shape=shape, seed=9, ramp=r) <= 1.2e-2
+    assert run_paged(k, seqs, 3, 3, hd, 64, torch.bfloat16, window=700, tiled_shape=shape, seed=11, ramp=r) <= 1.2e-2
+    assert run_paged(k, [(90, 2400), (1, 77)], 16, 1, hd, 32, torch.bfloat16, tiled_shape=shape, seed=12, ramp=r) <= 1.2e-2
+
+
+@pytest.mark.parametrize("hd,shape", [(128, 142), (128, 1142), (64, 1142)])
+@pytest.mark.parametrize("key_splits", [2, 3, 7])
+def test_key_ranges_of_portions_behind_prefixes(k, hd, shape, key_splits):  # noqa: F811
+    # prefixes of different lengths (one with fewer tiles of keys than workgroups that share them), a new prompt, a window; the keys' ramp
+    # makes every far key count, so a range that is left out or taken twice shows
+    seqs = [(70, 1300), (33, 33), (5, 2100), (130, 130), (40, 700)]
+    assert run_paged(k, seqs, 6, 2, hd, 16, torch.bfloat16, tiled_shape=shape, key_splits=key_splits, seed=31, ramp=8.0 / 2100) <= 1.2e-2
+    assert run_paged(k, seqs, 7, 1, hd, 64, torch.bfloat16, window=500, tiled_shape=shape, key_splits=key_splits, seed=32) <= 1.2e-2
+    assert run_paged(k, [(96, 9000), (1, 5000), (40, 12001), (3, 3)], 6, 2, hd, 16, torch.bfloat16, tiled_shape=shape, key_splits=key_splits, seed=5) <= 1.2e-2
+
+
 @pytest.mark.parametrize("hd,shape", [(64, 142), (64, 181), (128, 142), (128, 181), (64, 121), (128, 141)])
 @pytest.mark.parametrize("window,ps", [(0, 16), (0, 64), (70, 32)])
 def test_nothing_behind_the_context_counts(k, hd, shape, window, ps):  # noqa: F811

@@ -76,7 +76,7 @@ def test_rotated_products_that_are_refused():
 
 @pytest.mark.parametrize("m", [65, 200, 700])
 def test_wrapper_agrees_with_the_two_kernels(m):
-    # the same sums but for the order of a split k range: within a unit of bfloat16
+    # product, then bias, rotation and store: the same sums but for the order of a split k range
     k = kernels.backend()
     nq, nkv, hd, ps, kk = 14, 2, 64, 16, 896
     x, w, b, positions, inv, slots, pages, want = _case(m, kk, nq, nkv, hd, ps, True, seed=m)
@@ -85,7 +85,19 @@ def test_wrapper_agrees_with_the_two_kernels(m):
     cs = k.rope_table(pd, fd)
     out = k.product_rotated(xd, wd, bd, cs, sd, *new, nq, nkv, hd, ps)
     assert out is not None
-    _check(out.view(m, -1, hd)[:, :nq], want[:, :nq])
+    old = [torch.zeros_like(c) for c in new]
+    both = torch.empty_like(out)
+    k.qkv_rope_store(k.product_parts(xd, wd), bd, pd, fd, hd, sd, *old, nq, nkv, hd, ps, out=both, cos_sin=cs)
+    torch.cuda.synchronize()
+    stored = slots >= 0
+    page, off = (slots[stored] // ps).long(), (slots[stored] % ps).long()
+    for q, kc, vc in ((out, *new), (both, *old)):
+        _check(q.view(m, -1, hd)[:, :nq], want[:, :nq])
+        _check(kc.cpu()[page, :, off], want[stored, nq : nq + nkv])
+        _check(vc.cpu()[page, :, :, off], want[stored, nq + nkv :])
+    # float32 sums in another order are off by 1e-5 (values of size one), which takes one in a hundred to the other side of a rounding
+    for a, b in ((out.view(m, -1, hd)[:, :nq], both.view(m, -1, hd)[:, :nq]), *zip(new, old)):
+        assert float((a != b).float().mean()) <= 0.01 and torch.all((a.double() - b.double()).abs() <= 2.0 ** -7 * 1.01 * b.double().abs() + 4e-5)
     # operands that it does not take
     assert k.product_rotated(xd[:64], wd, bd, cs[:64].contiguous(), sd[:64], *new, nq, nkv, hd, ps) is None
     assert k.product_rotated(xd.float(), wd.float(), bd.float(), cs, sd, *new, nq, nkv, hd, ps) is None
