@@ -82,7 +82,7 @@ int egpt_paged_attention_mfma(const void* qkv, void* out, float* part_o, float* 
                               int n_splits, int rows_per_wave, int combine, void* stream);
 // Prompt portions of heads of 64 or 128 (keys and values alike), bfloat16, queries [n_tokens][nq][hd], with dist_bias [nq][dist_far + 1]
 // (float32, or null) added to the scaled scores by distance, the last entry beyond dist_far; pages of 16, 32 or 64 tokens.
-// row_blocks: blocks of 32 rows to a workgroup, 4 or 8.  EGPT_UNSUPPORTED_SIZE where a kv head's rows of the table leave LDS no room.
+// row_blocks: blocks of 32 rows to a workgroup, 4 or 8 (8 in any case at head size 128 with dist_bias).  EGPT_UNSUPPORTED_SIZE where a kv head's rows of the table leave LDS no room.
 int egpt_heads_attention(const void* q, void* out, const void* k_cache, const void* v_cache, const int32_t* block_table, int table_width,
                          const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int n_seqs, int n_tokens, int nq, int nkv, int hd,
                          int page_size, float scale, int window, const float* dist_bias, int dist_far, int row_blocks, void* stream);

@@ -520,12 +520,12 @@ __global__ __launch_bounds__(64 * RT * KS) void attention_tiled_kernel(
 // of rows; KS wavefronts per block split each tile of 64 * KS keys and are combined through LDS at the end.  The tiles
 // of 64 keys must be whole pages (page sizes 16, 32, 64).
 //
-// What bounds it: the vector instructions of the softmax.  A block of 32 rows and 64 keys is 100 of them (an exponential takes a
-// wavefront's issue slot for about 8.5 cycles, the others for 4.4: some 800 cycles with the matrix instructions of the SIMD's other
+// What bounds it: the vector instructions of the softmax.  A block of 32 rows and 64 keys is 143 of them by the counters (an exponential
+// takes a wavefront's issue slot for about 8.5 cycles, the others for 4.4: some 800 cycles with the matrix instructions of the SIMD's other
 // wavefront between them), against 640 cycles of the matrix cores at head size 64 and 1,152 at 128.  With two wavefronts to a SIMD
 // that take matrix and vector instructions in turns a step of both takes 1,000 to 1,300 cycles.  What it was before: one straight line of
-// code that alternated matrix and vector instructions, keys and values through registers into LDS (84 more vector instructions
-// a block, bank conflicts, every load waited for in front of the iteration's barrier), four wavefronts a CU at head size 128, and a
+// code that alternated matrix and vector instructions, keys and values through registers into LDS (184 vector instructions a
+// block by the counters, bank conflicts, every load waited for in front of the iteration's barrier), four wavefronts a CU at head size 128, and a
 // block without rows masked in every tile, by which a prompt whose last rows fill their workgroup badly took half as long again.  us a
 // layer: 14 heads of 64 on 2, 2,048 / 6,000 / 8,191 tokens 25.9 / 117 / 171 -> 25.1 / 96 / 146; 12 heads of 128 on 2, 1,024 / 2,048 / 5,000
 // 25.9 / 47.2 / 136 -> 21.0 / 32.8 / 88.6; 28 on 4, 1,024 / 2,048 / 5,000 29.5 / 72.9 / 289 -> 22.6 / 46.0 / 178.

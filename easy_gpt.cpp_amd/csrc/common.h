@@ -153,8 +153,8 @@ struct RowFactor {
 };
 
 // Reductions over a wavefront's lanes in registers: rotations and exchanges of rows of 16 lanes (DPP, v_permlane*_swap) are vector
-// instructions, where a shuffle goes through LDS and its result is waited for.  (Decode steps of the 0.5B sizes, us: one user 769.6
-// with shuffles and 763.6 so, 64 users 1,358.9 and 1,336.0.)  The pairs that are added up, and so the bits, are those of shuffles with
+// instructions, where a shuffle goes through LDS and its result is waited for.  (Decode steps of the 0.5B sizes, us: 64 users 1,359
+// with shuffles and 1,336 so; one user's within what two runs differ by.)  The pairs that are added up, and so the bits, are those of shuffles with
 // lanes 32, 16, 8, 4, 2, 1 apart (or 1, 2, 4, 8): behind a step the values repeat at its distance, so that a rotation by the next one
 // reaches the partner's value.
 template <int CTRL>

@@ -1524,7 +1524,7 @@ class HipKernels(KernelBackend):
         longest = max_kv_len if portion_kv is None else min(portion_kv, max_kv_len)
         if self._heads_portion(max_q_len, longest) and self._heads_fit(q, k_cache, v_cache, nq // nkv, dk, dv, page_size, scale, keep_first, sink, dist_bias,
                                                                dist_far, block, slopes, softcap, head_gate, maps):
-            row_blocks = self._heads_blocks(t, nq, nkv, dk, window, max_kv_len)
+            row_blocks = self._heads_blocks(t, nq, nkv, dk, window, max_kv_len, dist_bias is not None)
             if row_blocks:
                 self._run("egpt_heads_attention", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), width,
                           q_start.data_ptr(), q_len.data_ptr(), kv_len.data_ptr(), b, t, nq, nkv, dk, page_size, float(scale), int(window),
@@ -1573,24 +1573,29 @@ class HipKernels(KernelBackend):
     @staticmethod
     def _heads_fit(q, k_cache, v_cache, group, dk, dv, page_size, scale, keep_first, sink, dist_bias, dist_far, block, slopes, softcap, head_gate,
                    maps) -> bool:
-        """Whether egpt_heads_attention takes the call: its tiles take 80 KB of LDS at most, a kv head's bias, divided by the scale, the rest."""
+        """Whether egpt_heads_attention takes the call: with a bias its tiles take 80 KB of LDS at most, a kv head's entries, divided by the
+        scale, what is left of 160."""
         return (q.dtype == _BF16 and dk == dv and dk in (64, 128) and page_size in (16, 32, 64) and keep_first == 0 and sink is None and not block
                 and slopes is None and softcap is None and head_gate is None and maps == 1 and scale >= 1e-6 and dist_far <= 16384
                 and (dist_bias is None or 80 * 1024 + group * (dist_far + 163) * 4 <= 160 * 1024)
                 and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0)
 
     @staticmethod
-    def _heads_blocks(t, nq, nkv, hd, window, max_kv_len) -> int:
+    def _heads_blocks(t, nq, nkv, hd, window, max_kv_len, biased) -> int:
         """Blocks of 32 rows to a workgroup of the prompt kernel for heads of 64 and 128 (attention_rows32_kernel's loop on queries that lie by
         themselves, with a bias by distance or without), or 0 for the window kernel.  us a layer against that: 14 heads of 64 on 2 with a
         bias, prompts of 128 / 512 / 2,048 / 5,000 tokens 11.0 / 16.2 / 30.5 / 86 against 13.5 / 26.0 / 101 / 305, three of 333 to 1,357 27.1 against 74.5, 6 of
         40 tokens 11.2 against 9.9; 16 heads of 128 on 4 15.8 / 29.0 / 63 / 160 against 16.9 / 37.8 / 144 / 572; without a bias, 2,048 tokens 35.5 against
         112.  It walks a request's keys with one workgroup, where the window kernel deals them out: 512 tokens beside 8 decoded ones behind
         1,000 / 2,000 20.6 / 31.5 against 33.1 / 39.3 (head size 128 36.7 / 64 against 48.3 / 65), 128 tokens beside 4 behind 1,000 20.4 against 17.9, 66 beside one
-        behind 3,042 42 against 23.  A narrow window leaves little to walk (100: 17.8 against 16.7).  256 rows to a workgroup as
-        `_portion_shape` has them."""
+        behind 3,042 42 against 23; 40 and 64 decoded ones, each a workgroup that walks all its keys, beside 512 or 1,024 tokens behind 500 to
+        3,000, head size 64 with a bias 17.6 to 49.4 against 30.5 to 138, head size 128 without 19.3 to 102 against 43.1 to 166 (60 behind 300 beside 300
+        28.5 against 27.0).  A narrow window leaves little to walk (100: 17.8 against 16.7).  256 rows to a workgroup as `_portion_shape` has them, and
+        with a bias at head size 128 always: two slots of 128 keys and three of their values leave its table no room."""
         if 0 < window < 192 or max_kv_len > ((4 if hd == 64 else 3) * t if t >= 256 else 512 if hd == 64 else 300):
             return 0
+        if biased and hd == 128:
+            return 8
         row_tiles = -(-t * (nq // nkv) // 16) * nkv
         return 8 if HipKernels._blocks_of_256(hd, row_tiles, t, max_kv_len) else 4
 
