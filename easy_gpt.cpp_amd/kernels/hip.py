@@ -1187,8 +1187,8 @@ class HipKernels(KernelBackend):
     # Dealt out by the contexts' lengths (`decode_ranges`) they share the portions' launch, at head size 128 beyond this.  The kernel of
     # the portions alone against it, a new prompt's 512 tokens beside decoded ones: 12 heads of 128 on 2, 40 behind 128 to 2,048 51.5
     # and 21.9, behind 128 to 1,000 20.6 and 20.0, 8 behind 1,400 35.6 and 19.2, 300 tokens beside 8 behind 300 12.9 and 17.7; 28 on 4,
-    # 40 behind 128 to 2,048 71.8 and 34.2, to 1,000 25.1 and 24.9.  14 heads of 64 on 2, 40 behind 128 to 3,000 36.2 and 18.9, to 2,000
-    # 18.9 and 15.9, to 1,000 11.7 and 14.8, 8 behind 1,500 15.1 and 14.8: there what is gained below 2,048 the table's 5 us a step use up
+    # 40 behind 128 to 2,048 71.8 and 34.2, to 1,000 25.1 and 24.9.  14 heads of 64 on 2, 40 behind 128 to 3,000 26.2 and 19.9, to 2,000
+    # 18.9 and 16.2, to 1,000 11.8 and 14.1, 8 behind 1,500 15.1 and 13.9: there what is gained below 2,048 the table's 5 us a step use up
     singles_dealt_beyond = 1024
     prefix_keys = 4096           # a step's longest context from which its portions are taken to lie behind a prefix
     attention_segment = 64       # keys per segment of the decode kernel for any head size (kSegment in attention_any.hip)
