@@ -1206,7 +1206,7 @@ __device__ __forceinline__ void decode_block(
     if constexpr (MIXED && !RANGED) {
         if (q_len[bx] != 1) return;
     }
-    const int32_t* range = ranges + (RANGED ? bx * kRangeInts : 0);
+    const int32_t* range = RANGED ? ranges + bx * kRangeInts : nullptr;
     if constexpr (RANGED) {
         if (range[0] < 0) return;
     }
@@ -1540,11 +1540,13 @@ __device__ __forceinline__ void decode_block(
 
 template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false>
 __global__ __launch_bounds__(512) void attention_decode_kernel(
-    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
-    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ kv_len, int n_tokens, int nq, int nkv, int page_size, float scale, int window,
-    int n_splits, FusedQkv f, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ranges) {
+    // (what the first loads are addressed by: 14 words that arrive with the wavefronts)
+    const int32_t* __restrict__ lengths, const int32_t* __restrict__ q_start, const int32_t* __restrict__ block_table,
+    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, int table_width, int page_size, int nkv, int n_splits,
+    int nq, int window, float scale, int n_tokens, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
+    float* __restrict__ part_ml, const int32_t* __restrict__ q_len, FusedQkv f) {
+    const int32_t* kv_len = RANGED ? nullptr : lengths;
+    const int32_t* ranges = RANGED ? lengths : nullptr;
     extern __shared__ float wave_state[];
     decode_block<HD, PF, FUSED, MIXED, RANGED>(wave_state, blockIdx.x, blockIdx.y, blockIdx.z, qkv, out, part_o, part_ml, k_cache, v_cache, block_table,
                                                table_width, q_start, kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, f, q_len, ranges);
@@ -1581,10 +1583,10 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
 // round of loads; the partial outputs are then read eight splits at a time.
 __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml,
-                                                              bf16_t* __restrict__ out, int n_rows, int hd, int n_splits,
-                                                              const int32_t* __restrict__ q_start = nullptr,
-                                                              const int32_t* __restrict__ q_len = nullptr, int nq = 1,
-                                                              const int32_t* __restrict__ dealt = nullptr) {
+                                                              const int32_t* __restrict__ q_start,
+                                                              const int32_t* __restrict__ q_len,
+                                                              const int32_t* __restrict__ dealt, int n_rows, int hd, int n_splits, int nq,
+                                                              bf16_t* __restrict__ out) {
     const int row = blockIdx.x, lane = threadIdx.x;
     // q_start given: the parts are kept by request, of which only those of one token have any, and the result goes
     // to that token's row
@@ -1666,8 +1668,8 @@ static int launch_mfma(const void* qkv, void* out, float* part_o, float* part_ml
         q_len, kv_len, n_seqs, n_tokens, nq, nkv, page_size, scale, window, n_splits);
     EGPT_CHECK_LAUNCH();
     if (n_splits > 1 && combine) {
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), n_tokens * nq,
-                                                             HD, n_splits);
+        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, nullptr, nullptr, nullptr, n_tokens * nq, HD, n_splits, 1,
+                                                             static_cast<bf16_t*>(out));
         EGPT_CHECK_LAUNCH();
     }
     return EGPT_OK;
@@ -1703,40 +1705,25 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
             raised = true;
         }
     }
-    FusedQkv fq = fused ? *fused : FusedQkv{};
-    if (ranges && fused)
-        attention_decode_kernel<HD, 2, true, false, true><<<grid, n_waves * kWave, lds, s>>>(
-            nullptr, static_cast<bf16_t*>(out), part_o, part_ml, static_cast<const bf16_t*>(k_cache),
-            static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start, kv_len, n_tokens, nq, nkv,
-            page_size, scale, window, 1, fq, nullptr, ranges);
-    else if (ranges)
-        attention_decode_kernel<HD, 2, false, true, true><<<grid, n_waves * kWave, lds, s>>>(
-            static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), part_o, part_ml,
-            static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start,
-            kv_len, n_tokens, nq, nkv, page_size, scale, window, 1, fq, q_len, ranges);
-    else if (fused)
-        attention_decode_kernel<HD, PF, true><<<grid, n_waves * kWave, lds, s>>>(
-            nullptr, static_cast<bf16_t*>(out), part_o, part_ml, static_cast<const bf16_t*>(k_cache),
-            static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start, kv_len, n_tokens, nq, nkv,
-            page_size, scale, window, n_splits, fq, nullptr, nullptr);
-    else if (q_len)
-        attention_decode_kernel<HD, PF, false, true><<<grid, n_waves * kWave, lds, s>>>(
-            static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), part_o, part_ml,
-            static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start,
-            kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, fq, q_len, nullptr);
-    else
-        attention_decode_kernel<HD, PF, false><<<grid, n_waves * kWave, lds, s>>>(
-            static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), part_o, part_ml,
-            static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), block_table, table_width, q_start,
-            kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, fq, nullptr, nullptr);
+    const FusedQkv fq = fused ? *fused : FusedQkv{};
+    auto launch = [&](auto kernel, const int32_t* lengths, const void* q, const int32_t* counts, int splits) {
+        kernel<<<grid, n_waves * kWave, lds, s>>>(lengths, q_start, block_table, static_cast<const bf16_t*>(k_cache),
+                                                  static_cast<const bf16_t*>(v_cache), table_width, page_size, nkv, splits, nq, window, scale,
+                                                  n_tokens, static_cast<const bf16_t*>(q), static_cast<bf16_t*>(out), part_o, part_ml, counts, fq);
+    };
+    if (ranges && fused) launch(attention_decode_kernel<HD, 2, true, false, true>, ranges, nullptr, nullptr, 1);
+    else if (ranges) launch(attention_decode_kernel<HD, 2, false, true, true>, ranges, qkv, q_len, 1);
+    else if (fused) launch(attention_decode_kernel<HD, PF, true>, kv_len, nullptr, nullptr, n_splits);
+    else if (q_len) launch(attention_decode_kernel<HD, PF, false, true>, kv_len, qkv, q_len, n_splits);
+    else launch(attention_decode_kernel<HD, PF, false>, kv_len, qkv, nullptr, n_splits);
     EGPT_CHECK_LAUNCH();
     if (ranges) {
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), n_tokens * nq,
-                                                             HD, 1, q_start, q_len, nq, ranges + slots * kRangeInts);
+        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, q_start, q_len, ranges + slots * kRangeInts, n_tokens * nq, HD, 1, nq,
+                                                             static_cast<bf16_t*>(out));
         EGPT_CHECK_LAUNCH();
     } else if (n_splits > 1 && combine) {
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), n_tokens * nq,
-                                                             HD, n_splits, q_len ? q_start : nullptr, q_len, nq);
+        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, q_len ? q_start : nullptr, q_len, nullptr, n_tokens * nq, HD,
+                                                             n_splits, nq, static_cast<bf16_t*>(out));
         EGPT_CHECK_LAUNCH();
     }
     return EGPT_OK;
@@ -1796,8 +1783,8 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
     // (the rows of requests that were left out have no parts: what is combined for them is written over by the
     // kernel that takes them, which runs behind this one)
     if (n_splits > 1)
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), n_tokens * nq,
-                                                             HD, n_splits);
+        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, nullptr, nullptr, nullptr, n_tokens * nq, HD, n_splits, 1,
+                                                             static_cast<bf16_t*>(out));
 }
 
 template <int HD, int RB, int KS>
@@ -1813,8 +1800,8 @@ static int launch_mixed(const void* qkv, void* out, const void* k_cache, const v
         block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, late, static_cast<int>(blocks), ranges,
         slots, range_o, range_ml);
     EGPT_CHECK_LAUNCH();
-    attention_reduce_kernel<<<n_seqs * nq, 64, 0, s>>>(range_o, range_ml, static_cast<bf16_t*>(out), n_seqs * nq, HD, 1, q_start, q_len, nq,
-                                                       ranges + slots * kRangeInts);
+    attention_reduce_kernel<<<n_seqs * nq, 64, 0, s>>>(range_o, range_ml, q_start, q_len, ranges + slots * kRangeInts, n_seqs * nq, HD, 1, nq,
+                                                       static_cast<bf16_t*>(out));
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
@@ -2096,9 +2083,8 @@ extern "C" int egpt_attention_combine(const float* part_o, const float* part_ml,
     if (!part_o || !part_ml || !out || n_rows < 0 || hd <= 0 || n_splits < 1) return EGPT_BAD_ARGUMENT;
     if (n_splits > 64 || hd > 256) return EGPT_UNSUPPORTED_SIZE;
     if (n_rows == 0) return EGPT_OK;
-    attention_reduce_kernel<<<n_rows, 64, 0, static_cast<hipStream_t>(stream)>>>(part_o, part_ml,
-                                                                               static_cast<bf16_t*>(out), n_rows, hd,
-                                                                               n_splits);
+    attention_reduce_kernel<<<n_rows, 64, 0, static_cast<hipStream_t>(stream)>>>(part_o, part_ml, nullptr, nullptr, nullptr, n_rows, hd,
+                                                                               n_splits, 1, static_cast<bf16_t*>(out));
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }

@@ -22,9 +22,12 @@ SOURCES = ["elementwise.hip", "gemm.hip", "gemm_skinny.hip", "gemm_gate_up.hip",
 HEADERS = ["api.h", "common.h", "lds_loads.h"]
 LIB_NAME = "libeasygpt_hip.so"
 ARCH = "gfx950"
-# packed-fp32 instructions are kept out of the generated code on purpose
+# packed-fp32 instructions are kept out of the generated code on purpose.  The first 14 words of a kernel's arguments (all that
+# fits) arrive in registers with its wavefronts instead of by a load that every kernel would begin with: a kernel is a link of a chain, and
+# that load is a trip to memory before the first one that it asks for (64 rows decoded at the 0.5B sizes 1,322 -> 1,292 us a step, a
+# prompt of 2,048 tokens there 3,290 -> 3,248).  So the arguments that a kernel's first addresses come from stand first, and structs last.
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
-         "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-Wno-pass-failed"]
+         "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=14", "-Wno-unused-command-line-argument", "-Wno-pass-failed"]
 
 
 HOST_SOURCES = ["host/cache_core.cpp", "host/draws.cpp"]

@@ -5,6 +5,16 @@
 
 namespace egpt {
 
+template <typename T>
+__host__ __device__ static ProductView<T> make_view(const void* p, int n_splits, size_t split_stride) {
+    ProductView<T> v;
+    v.whole = n_splits == 0 ? static_cast<const T*>(p) : nullptr;
+    v.partial = n_splits > 0 ? static_cast<const float*>(p) : nullptr;
+    v.n_splits = n_splits;
+    v.split_stride = split_stride;
+    return v;
+}
+
 // ----------------------------------------------------------------------------- embedding
 // x[t, :] = E[id_t, :]   (/root/reference/src/models/embedding.cpp:54-76); output: the residual stream, float32 or
 // fixed point.
@@ -24,11 +34,21 @@ __global__ void embed_kernel(const int32_t* __restrict__ ids, const T* __restric
 // distance from (1, say), added in float32
 // (/root/reference/src/models/norm.cpp:47-59, /root/reference/src/cuda/ops/self_attn_detail.cuh:385-418).
 // The residual addition h += delta happens here too, in float32.
+
+// Threads of a row's workgroup.  Few rows with many partial sums each: more threads, so that each has fewer dependent loads to wait
+// for; and enough threads for a row to stay in registers (four values a thread, eight for the widest rows).  (The kernel computes
+// it again: blockDim would be a load.)
+__host__ __device__ static constexpr int norm_threads(int n_splits, int hidden) {
+    return (n_splits > 1 || hidden > 2048) ? 1024 : (hidden > 1024 ? 512 : 256);
+}
+
 template <typename T, typename R, int KEEP>
-__global__ void add_rmsnorm_kernel(R* __restrict__ h, ProductView<T> delta,
-                                   const int32_t* __restrict__ rows, const T* __restrict__ weight, float w_off, float eps,
-                                   T* __restrict__ out, int hidden) {
+__global__ void add_rmsnorm_kernel(R* __restrict__ h, const void* __restrict__ added, int n_splits, int hidden, size_t split_stride,
+                                   const int32_t* __restrict__ rows, const T* __restrict__ weight, T* __restrict__ out, float w_off,
+                                   float eps) {
+    const ProductView<T> delta = make_view<T>(added, n_splits, split_stride);
     __shared__ float scratch[16];
+    const int threads = norm_threads(n_splits, hidden);
     const int r = blockIdx.x;
     const size_t src = rows ? static_cast<size_t>(rows[r]) : static_cast<size_t>(r);
     R* hrow = h + src * hidden;
@@ -40,11 +60,11 @@ __global__ void add_rmsnorm_kernel(R* __restrict__ h, ProductView<T> delta,
     // stores.  (A loop over the row instead waits for memory once per round: 10 us for a row of 3,584 values with 512
     // threads, 7.4 us for one of 5,120 with 1,024 against 6.2 from registers; eight where four are enough cost 0.3 to
     // 0.7 us.)
-    if (hidden <= KEEP * static_cast<int>(blockDim.x)) {
+    if (hidden <= KEEP * threads) {
         float v[KEEP], w[KEEP];
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            const int j = threadIdx.x + i * blockDim.x;
+            const int j = threadIdx.x + i * threads;
             v[i] = 0.f;
             w[i] = 0.f;
             if (j < hidden) {
@@ -55,14 +75,14 @@ __global__ void add_rmsnorm_kernel(R* __restrict__ h, ProductView<T> delta,
         if (has_delta) {
 #pragma unroll
             for (int i = 0; i < KEEP; ++i) {
-                const int j = threadIdx.x + i * blockDim.x;
+                const int j = threadIdx.x + i * threads;
                 if (j < hidden) v[i] += delta.at(dbase + j);
             }
         }
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            const int j = threadIdx.x + i * blockDim.x;
+            const int j = threadIdx.x + i * threads;
             if (write_back && j < hidden) residual_store(hrow + j, v[i]);
             ss += v[i] * v[i];
         }
@@ -71,13 +91,13 @@ __global__ void add_rmsnorm_kernel(R* __restrict__ h, ProductView<T> delta,
         T* orow = out + static_cast<size_t>(r) * hidden;
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
-            const int j = threadIdx.x + i * blockDim.x;
+            const int j = threadIdx.x + i * threads;
             if (j < hidden) orow[j] = from_float<T>(v[i] * inv * w[i]);
         }
         return;
     }
     float ss = 0.f;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+    for (int j = threadIdx.x; j < hidden; j += threads) {
         float v = residual_load(hrow + j);
         if (has_delta) v += delta.at(dbase + j);
         if (write_back) residual_store(hrow + j, v);
@@ -86,7 +106,7 @@ __global__ void add_rmsnorm_kernel(R* __restrict__ h, ProductView<T> delta,
     ss = block_sum(ss, scratch);
     const float inv = 1.0f / sqrtf(ss / static_cast<float>(hidden) + eps);
     T* orow = out + static_cast<size_t>(r) * hidden;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+    for (int j = threadIdx.x; j < hidden; j += threads) {
         float v = residual_load(hrow + j);       // already updated when written back
         if (has_delta && !write_back) v += delta.at(dbase + j);
         orow[j] = from_float<T>(v * inv * (w_off + to_float(weight[j])));
@@ -199,7 +219,9 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict
 // out = up * gate / (1 + exp(-gate))   (/root/reference/src/cuda/ops/mlp.cu:152-162); [gate | up] per row.  act names the
 // gate's activation (gate_activation in common.h).
 template <typename T>
-__global__ void swiglu_kernel(ProductView<T> gate_up, T* __restrict__ out, int n_tokens, int inter, int act) {
+__global__ void swiglu_kernel(const void* __restrict__ product, int n_splits, int n_tokens, int inter, int act, size_t split_stride,
+                              T* __restrict__ out) {
+    const ProductView<T> gate_up = make_view<T>(product, n_splits, split_stride);
     const size_t total = static_cast<size_t>(n_tokens) * inter;
     for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < total;
          i += static_cast<size_t>(gridDim.x) * blockDim.x) {
@@ -214,8 +236,10 @@ __global__ void swiglu_kernel(ProductView<T> gate_up, T* __restrict__ out, int n
 // the product leaves the factor to its consumer): scale = 1/sqrt(sum_s row_ss[s][t] / hidden + eps) multiplies gate and
 // up before the activation.  One row of workgroups per token.
 template <typename T>
-__global__ void swiglu_scaled_kernel(ProductView<float> gate_up, const float* __restrict__ row_ss, int ss_splits,
-                                     float inv_hidden, float eps, T* __restrict__ out, int n_tokens, int inter, int act) {
+__global__ void swiglu_scaled_kernel(const float* __restrict__ product, const float* __restrict__ row_ss, int n_splits, int ss_splits,
+                                     int n_tokens, int inter, size_t split_stride, T* __restrict__ out, float inv_hidden, float eps,
+                                     int act) {
+    const ProductView<float> gate_up = make_view<float>(product, n_splits, split_stride);
     const size_t t = blockIdx.y;
     float ss = 0.f;
     for (int s = 0; s < ss_splits; ++s) ss += row_ss[static_cast<size_t>(s) * n_tokens + t];
@@ -259,12 +283,13 @@ __global__ __launch_bounds__(256) void swiglu_vec8_kernel(const GT* __restrict__
 constexpr int kHeadsPerBlock = 2;   // heads of one token that a workgroup of the QKV epilogue handles
 
 template <typename T>
-__global__ void qkv_rope_store_kernel(ProductView<T> qkv_in, const float* __restrict__ row_ss, int ss_splits,
-                                      float inv_hidden, float eps, T* __restrict__ qkv_out, const T* __restrict__ bias,
-                                      const int32_t* __restrict__ positions, const float* __restrict__ inv_freq,
-                                      const float* __restrict__ cos_sin, int rotary_dim,
+__global__ void qkv_rope_store_kernel(const void* __restrict__ product, int n_splits, int nq, int nkv, int hd, size_t split_stride,
+                                      const int32_t* __restrict__ positions, const float* __restrict__ row_ss,
+                                      const T* __restrict__ bias, int ss_splits, float inv_hidden, float eps, T* __restrict__ qkv_out,
+                                      const float* __restrict__ inv_freq, const float* __restrict__ cos_sin, int rotary_dim,
                                       const int32_t* __restrict__ slots, T* __restrict__ k_cache,
-                                      T* __restrict__ v_cache, int nq, int nkv, int hd, int page_size) {
+                                      T* __restrict__ v_cache, int page_size) {
+    const ProductView<T> qkv_in = make_view<T>(product, n_splits, split_stride);
     const int t = blockIdx.x;
     const int n_heads = nq + 2 * nkv;
     const int item_begin = blockIdx.y * kHeadsPerBlock * hd;
@@ -476,16 +501,6 @@ extern "C" int egpt_embed(const int32_t* ids, const void* table, void* out, int 
     return EGPT_OK;
 }
 
-template <typename T>
-static ProductView<T> make_view(const void* p, int n_splits, size_t split_stride) {
-    ProductView<T> v;
-    v.whole = n_splits == 0 ? static_cast<const T*>(p) : nullptr;
-    v.partial = n_splits > 0 ? static_cast<const float*>(p) : nullptr;
-    v.n_splits = n_splits;
-    v.split_stride = split_stride;
-    return v;
-}
-
 extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta_splits, int delta_rows,
                                 const int32_t* rows, const void* weight, float weight_offset, float eps, void* out,
                                 int n_rows, int hidden, int dtype, void* stream) {
@@ -493,9 +508,7 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
     if (delta && delta_rows <= 0) return EGPT_BAD_ARGUMENT;
     if (n_rows == 0) return EGPT_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // few rows with many partial sums each: more threads, so that each has fewer dependent loads to wait for; and
-    // enough threads for a row to stay in registers (four values a thread, eight for the widest rows)
-    const int threads = (delta_splits > 1 || hidden > 2048) ? 1024 : (hidden > 1024 ? 512 : 256);
+    const int threads = norm_threads(delta_splits, hidden);
     const size_t stride = static_cast<size_t>(delta_rows) * hidden;
     // (loads and stores of 16 bytes: operands that begin elsewhere take the kernel of single values)
     const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(weight) |
@@ -517,8 +530,8 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
     if (dtype != 0 && dtype != 1) return EGPT_BAD_ARGUMENT;
 #define EGPT_NORM_KEEP(T_, R_, KEEP_)                                                                      \
     add_rmsnorm_kernel<T_, R_, KEEP_><<<n_rows, threads, 0, s>>>(                                          \
-        static_cast<R_*>(h), make_view<T_>(delta, delta_splits, stride), rows, static_cast<const T_*>(weight), \
-        weight_offset, eps, static_cast<T_*>(out), hidden)
+        static_cast<R_*>(h), delta, delta_splits, hidden, stride, rows, static_cast<const T_*>(weight),        \
+        static_cast<T_*>(out), weight_offset, eps)
 #define EGPT_NORM(T_, R_)                                        \
     do {                                                         \
         /* (a wide row behind partial sums is faster in the loop: 7.7 against 8.7 us at 64 rows of 5,120) */ \
@@ -549,13 +562,13 @@ extern "C" int egpt_swiglu(const void* gate_up, int n_splits, const float* row_s
             return EGPT_BAD_ARGUMENT;
         const dim3 grid(static_cast<unsigned>((inter + 255) / 256 > 64 ? 64 : (inter + 255) / 256),
                         static_cast<unsigned>(n_tokens));
-        const ProductView<float> view = make_view<float>(gate_up, n_splits, stride);
+        const float* partial = static_cast<const float*>(gate_up);
         if (dtype == 0)
-            swiglu_scaled_kernel<float><<<grid, 256, 0, s>>>(view, row_ss, ss_splits, 1.0f / hidden, eps,
-                                                             static_cast<float*>(out), n_tokens, inter, act);
+            swiglu_scaled_kernel<float><<<grid, 256, 0, s>>>(partial, row_ss, n_splits, ss_splits, n_tokens, inter, stride,
+                                                             static_cast<float*>(out), 1.0f / hidden, eps, act);
         else
-            swiglu_scaled_kernel<bf16_t><<<grid, 256, 0, s>>>(view, row_ss, ss_splits, 1.0f / hidden, eps,
-                                                              static_cast<bf16_t*>(out), n_tokens, inter, act);
+            swiglu_scaled_kernel<bf16_t><<<grid, 256, 0, s>>>(partial, row_ss, n_splits, ss_splits, n_tokens, inter, stride,
+                                                              static_cast<bf16_t*>(out), 1.0f / hidden, eps, act);
         EGPT_CHECK_LAUNCH();
         return EGPT_OK;
     }
@@ -572,11 +585,9 @@ extern "C" int egpt_swiglu(const void* gate_up, int n_splits, const float* row_s
         return EGPT_OK;
     }
     if (dtype == 0)
-        swiglu_kernel<float><<<blocks, 256, 0, s>>>(make_view<float>(gate_up, n_splits, stride),
-                                                    static_cast<float*>(out), n_tokens, inter, act);
+        swiglu_kernel<float><<<blocks, 256, 0, s>>>(gate_up, n_splits, n_tokens, inter, act, stride, static_cast<float*>(out));
     else if (dtype == 1)
-        swiglu_kernel<bf16_t><<<blocks, 256, 0, s>>>(make_view<bf16_t>(gate_up, n_splits, stride),
-                                                     static_cast<bf16_t*>(out), n_tokens, inter, act);
+        swiglu_kernel<bf16_t><<<blocks, 256, 0, s>>>(gate_up, n_splits, n_tokens, inter, act, stride, static_cast<bf16_t*>(out));
     else
         return EGPT_BAD_ARGUMENT;
     EGPT_CHECK_LAUNCH();
@@ -610,16 +621,14 @@ extern "C" int egpt_qkv_rope_store(const void* qkv_in, int n_splits, const float
     const int block = kHeadsPerBlock * hd >= 256 ? 256 : (kHeadsPerBlock * hd >= 128 ? 128 : 64);
     if (dtype == 0)
         qkv_rope_store_kernel<float><<<grid, block, 0, s>>>(
-            make_view<float>(qkv_in, n_splits, stride), row_ss, ss_splits, inv_hidden, eps,
-            static_cast<float*>(qkv_out), static_cast<const float*>(bias),
-            positions, inv_freq, cos_sin, rotary_dim, slots, static_cast<float*>(k_cache), static_cast<float*>(v_cache), nq,
-            nkv, hd, page_size);
+            qkv_in, n_splits, nq, nkv, hd, stride, positions, row_ss, static_cast<const float*>(bias), ss_splits, inv_hidden, eps,
+            static_cast<float*>(qkv_out), inv_freq, cos_sin, rotary_dim, slots, static_cast<float*>(k_cache), static_cast<float*>(v_cache),
+            page_size);
     else if (dtype == 1)
         qkv_rope_store_kernel<bf16_t><<<grid, block, 0, s>>>(
-            make_view<bf16_t>(qkv_in, n_splits, stride), row_ss, ss_splits, inv_hidden, eps,
-            static_cast<bf16_t*>(qkv_out), static_cast<const bf16_t*>(bias), positions, inv_freq, cos_sin, rotary_dim, slots,
-            static_cast<bf16_t*>(k_cache),
-            static_cast<bf16_t*>(v_cache), nq, nkv, hd, page_size);
+            qkv_in, n_splits, nq, nkv, hd, stride, positions, row_ss, static_cast<const bf16_t*>(bias), ss_splits, inv_hidden, eps,
+            static_cast<bf16_t*>(qkv_out), inv_freq, cos_sin, rotary_dim, slots, static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache),
+            page_size);
     else
         return EGPT_BAD_ARGUMENT;
     EGPT_CHECK_LAUNCH();

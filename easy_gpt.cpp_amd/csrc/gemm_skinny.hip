@@ -121,11 +121,43 @@ __device__ __forceinline__ float sum_splits(const float* p, int n_splits, size_t
     return v;
 }
 
+// What every instance reads first stands in front of the struct (14 words that arrive with the wavefronts): w, the operand that x
+// comes from with its number of parts, and the sizes.
+template <int PRO>
+__device__ __forceinline__ void take_first(SkinnyArgs& a, const bf16_t* w, const void* from, const void* with, int m, int n, int k,
+                                           int steps_per_split, int parts, int more, int last) {
+    a.w = w;
+    a.m = m; a.n = n; a.k = k;
+    a.steps_per_split = steps_per_split;
+    if constexpr (PRO == kPlain) a.x = static_cast<const bf16_t*>(from);
+    if constexpr (PRO == kNorm) {
+        a.h_in_fixed = parts ? static_cast<const fixed_t*>(from) : nullptr;
+        a.h_in = static_cast<const float*>(from);
+        a.norm_w = static_cast<const bf16_t*>(with);
+    }
+    if constexpr (PRO == kSwiglu || PRO == kRelu2) {
+        a.gu = static_cast<const float*>(from);
+        a.gu_splits = parts;
+        a.ss_in = static_cast<const float*>(with);
+        a.ss_splits = more;
+    }
+    if constexpr (PRO == kAttn) {
+        a.part_o = static_cast<const float*>(from);
+        a.part_ml = static_cast<const float*>(with);
+        a.a_splits = parts;
+        a.nq = more;
+        a.hd = last;
+    }
+}
+
 // INF: how many splits' loads of the prologue's input are in flight together (kNorm, kAttn)
 // NW: wavefronts per workgroup (each 16 rows of w); they share the staged x, so a wide workgroup reads the
 // prologue's inputs fewer times
 template <int MT, int PRO, int INF, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs a) {
+__global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __restrict__ w, const void* __restrict__ from,
+                                                              const void* __restrict__ with, int m, int n, int k, int steps_per_split,
+                                                              int parts, int more, int last, SkinnyArgs a) {
+    take_first<PRO>(a, w, from, with, m, n, k, steps_per_split, parts, more, last);
     constexpr int kThreads = 64 * NW;
     __shared__ __attribute__((aligned(16))) bf16_t xs[2][MT * 16][kLdsRow];
     __shared__ float ss_part[2][16];                                     // kNorm: sums of squares of a short range
@@ -133,7 +165,6 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs a) {
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int li = lane % 16, lg = lane / 16;
     const int split = blockIdx.y;
-    const int m = a.m, n = a.n, k = a.k;
     const int n0 = (blockIdx.x * NW + wave) * kRowsPerWave;
     const int total_steps = (k + kStep - 1) / kStep;
     const int step_begin = split * a.steps_per_split;
@@ -578,14 +609,29 @@ static dim3 skinny_grid(int n, int n_splits, int waves) {
     return dim3((n + kRowsPerWave * waves - 1) / (kRowsPerWave * waves), n_splits);
 }
 
+template <int MT, int PRO, int INF, int NW>
+static void launch_skinny(const SkinnyArgs& a, int n_splits, hipStream_t s) {
+    const void *from = a.x, *with = nullptr;
+    int parts = 0, more = 0, last = 0;
+    if (PRO == kNorm) {
+        from = a.h_in_fixed ? static_cast<const void*>(a.h_in_fixed) : a.h_in;
+        with = a.norm_w;
+        parts = a.h_in_fixed ? 1 : 0;
+    } else if (PRO == kSwiglu || PRO == kRelu2) {
+        from = a.gu; with = a.ss_in; parts = a.gu_splits; more = a.ss_splits;
+    } else if (PRO == kAttn) {
+        from = a.part_o; with = a.part_ml; parts = a.a_splits; more = a.nq; last = a.hd;
+    }
+    gemm_skinny_kernel<MT, PRO, INF, NW><<<skinny_grid(a.n, n_splits, NW), 64 * NW, 0, s>>>(a.w, from, with, a.m, a.n, a.k, a.steps_per_split,
+                                                                                            parts, more, last, a);
+}
+
 // launches the instance for `waves` wavefronts per workgroup (4, 8 or 16)
 #define EGPT_SKINNY(MT_, PRO_, INF_)                                                                         \
     do {                                                                                                     \
-        const dim3 grid = skinny_grid(a.n, n_splits, waves);                                                 \
-        hipStream_t s_ = static_cast<hipStream_t>(stream);                                                   \
-        if (waves == 4) gemm_skinny_kernel<MT_, PRO_, INF_, 4><<<grid, 256, 0, s_>>>(a);                     \
-        else if (waves == 8) gemm_skinny_kernel<MT_, PRO_, INF_, 8><<<grid, 512, 0, s_>>>(a);                \
-        else gemm_skinny_kernel<MT_, PRO_, INF_, 16><<<grid, 1024, 0, s_>>>(a);                              \
+        if (waves == 4) launch_skinny<MT_, PRO_, INF_, 4>(a, n_splits, static_cast<hipStream_t>(stream));    \
+        else if (waves == 8) launch_skinny<MT_, PRO_, INF_, 8>(a, n_splits, static_cast<hipStream_t>(stream)); \
+        else launch_skinny<MT_, PRO_, INF_, 16>(a, n_splits, static_cast<hipStream_t>(stream));              \
     } while (0)
 
 }  // namespace egpt
