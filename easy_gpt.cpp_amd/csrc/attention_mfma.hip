@@ -1189,15 +1189,39 @@ struct FusedQkv {
 //
 // RANGED: the keys are dealt out by `decode_ranges_kernel`, every request getting as many workgroups as its context is long;
 // grid (slots, kv heads), and a part is kept by its slot.
-// Workgroup (bx, by, bz) of a launch.
-template <int HD, int PF, bool FUSED, bool MIXED, bool RANGED>
+
+// What a workgroup reads that is no address: sizes, and what stands for divisions by them.
+struct DecodeSizes {
+    int table_width, page_size, nkv, n_splits;
+    unsigned page_magic, split_magic, wave_magic;                // magic_of(page_size / 16), (n_splits), (n_waves)
+    int group, window, n_tokens;                                 // group: query heads of a kv head
+    float scale;
+    int n_waves;                                                 // of a workgroup (blockDim would be a load by itself)
+};
+
+// floor(x / d) for x and d < 2^27, as a product: no more than one too many, which is put right (a division is 30 instructions, and
+// a kernel like this one is as long as its chain of them).
+static unsigned magic_of(int d) { return static_cast<unsigned>((1ULL << 32) / (2 * static_cast<unsigned>(d)) + 1); }
+__device__ __forceinline__ int divided(int x, int d, unsigned magic) {
+    const int q = static_cast<int>(__umulhi(2 * static_cast<unsigned>(x), magic));
+    return q - (q * d > x ? 1 : 0);
+}
+
+// The order of the loads is what this kernel's time is: everything that depends on no other load goes out at once (the
+// context's length, the product's partial sums with what is computed from them), then the page numbers, then the first round of keys
+// and values, and only then are the queries made.  Loads are bounded by their buffer's size instead of branches, so that none of
+// them ends a batch: a page that is not there is a buffer of no bytes, which reads as zeros; a partial sum past the last one adds
+// zero.  (Written with conditions around the loads, the compiler moved the queries' arithmetic in front of the keys' loads and waited
+// five times one after the other.)  Instructions count as much: a kernel begins with an empty instruction cache, a jump over code that is
+// not needed is a trip for the next line, and 300 instructions take 1 us.  So there are no divisions, code for rare sizes lies behind the
+// common path, and a round's keys share one maximum.  A layer, 14 heads of 64 on 2 behind 2,048 tokens: one request 8.1 -> 6.1 us, eight
+// 8.3 -> 6.4; of the 6 the loads' issue is 1.5, the trip to the keys 1.2, their products and softmax 1, the wavefronts' combination 0.6.
+template <int HD, int PF, bool FUSED, bool MIXED, bool RANGED, int INF>
 __device__ __forceinline__ void decode_block(
-    float* wave_state, int bx, int by, int bz,
-    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
-    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ kv_len, int n_tokens, int nq, int nkv, int page_size, float scale, int window,
-    int n_splits, FusedQkv f, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ranges) {
+    float* wave_state, int bx, int by, int bz, const int32_t* __restrict__ lengths, const int32_t* __restrict__ block_table,
+    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, const DecodeSizes& d, const bf16_t* __restrict__ qkv,
+    bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, const int32_t* __restrict__ q_start,
+    const int32_t* __restrict__ q_len, const FusedQkv& f) {
     constexpr int KD = HD / 32, DT = HD / 16;
     constexpr int kRow = HD + 2;
     // MIXED: a step that also holds portions of prompts; this kernel takes its requests of one token, parts are kept
@@ -1206,223 +1230,228 @@ __device__ __forceinline__ void decode_block(
     if constexpr (MIXED && !RANGED) {
         if (q_len[bx] != 1) return;
     }
-    const int32_t* range = RANGED ? ranges + bx * kRangeInts : nullptr;
+    const int32_t* range = RANGED ? lengths + bx * kRangeInts : nullptr;
+    const int b = RANGED ? range[0] : bx, kh = by;
     if constexpr (RANGED) {
-        if (range[0] < 0) return;
+        if (b < 0) return;
     }
     // wave_state: [n_waves][16][HD + 2]: O, then maximum, then sum
-    const int lane = threadIdx.x % kWave, n_waves = blockDim.x / kWave;
+    const int lane = threadIdx.x % kWave, n_waves = d.n_waves, n_threads = n_waves * kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // known to be the same for the wavefront
     const int lj = lane % 16, lg = lane / 16;
-    const int b = RANGED ? range[0] : bx, kh = by, split = bz;
-    const int group_size = nq / nkv;
-    const int kv = RANGED ? range[3] : kv_len[b], tok = RANGED ? range[4] : q_start[b];
-    const int p = kv - 1;
-    const int lo = window > 0 ? max(0, p - window + 1) : 0;
-    const bool valid = lj < group_size;
-    const int head = kh * group_size + (valid ? lj : 0);
-    if constexpr (RANGED) n_splits = range[5];
+    const int group_size = d.group, nkv = d.nkv, nq = group_size * nkv, page_size = d.page_size;
+    const int kv = RANGED ? range[3] : lengths[b];
+    __builtin_amdgcn_sched_barrier(0);                // (asked for before anything else)
+    const int tok = RANGED ? range[4] : FUSED ? b : q_start[b];
+    const int n_splits = RANGED ? range[5] : d.n_splits;
     const int width = (nq + 2 * nkv) * HD;
-    const int32_t* table = block_table + static_cast<size_t>(b) * table_width;
-
-    const int kb_begin = lo / 32, kb_end = p / 32 + 1;
-    const int per_split = (kb_end - kb_begin + n_splits - 1) / n_splits;
-    const int s_begin = RANGED ? range[1] : kb_begin + split * per_split, s_end = RANGED ? range[2] : min(kb_end, s_begin + per_split);
-    const int per_wave = (max(s_end - s_begin, 0) + n_waves - 1) / n_waves;
-    const int w_begin = s_begin + wave * per_wave, w_end = min(s_end, w_begin + per_wave);
-    // FUSED: does this workgroup's key range end with the new token?
-    const bool writer = FUSED && (RANGED ? s_end == kb_end : split == (kb_end - 1 - kb_begin) / per_split);
+    const int32_t* table = block_table + static_cast<size_t>(b) * d.table_width;
+    // (all arguments that did not come with the wavefront, and the length, in one trip)
+    if constexpr (FUSED)
+        asm volatile("" ::"s"(f.prod), "s"(f.in_splits), "s"(f.row_ss), "s"(f.ss_splits), "s"(f.bias), "s"(f.cos_sin), "s"(f.slots), "s"(group_size),
+                     "s"(d.window), "s"(d.n_tokens), "s"(n_waves), "s"(kv));
     bf16_t* q_lds = reinterpret_cast<bf16_t*>(wave_state + n_waves * 16 * kRow);   // FUSED: [16][HD], then k, v [HD]
     bf16_t* k_lds = q_lds + 16 * HD;
     bf16_t* v_lds = k_lds + HD;
 
-    // One round of loads: PF blocks of 32 keys and their values for this wavefront, first all page numbers
-    // (one wait for all of them), then all key and value loads.  The first round is issued before anything
-    // else, so that the queries (a round trip of their own, two in the fused variant) arrive meanwhile.
-    uint4 kk[PF][2][KD];
-    uint2 vv[PF][2][DT];
-    auto load_round = [&](int kb0) {
-        int pages[PF][2];
-        bool live[PF][2];
-#pragma unroll
-        for (int i = 0; i < PF; ++i)
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                const int key0 = (kb0 + i) * 32 + kt * 16;
-                live[i][kt] = kb0 + i < w_end && key0 <= p && key0 + 15 >= lo;
-                pages[i][kt] = table[live[i][kt] ? key0 / page_size : 0];
-            }
-#pragma unroll
-        for (int i = 0; i < PF; ++i)
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                const int key0 = (kb0 + i) * 32 + kt * 16;
-                const bool ok = live[i][kt] && pages[i][kt] >= 0;
-                const long page = ok ? pages[i][kt] : 0;
-                const int off = ok ? key0 % page_size : 0;
-                const bf16_t* kp = k_cache + ((page * nkv + kh) * page_size + off + lj) * HD + lg * 8;
-                const bf16_t* vp = v_cache + ((page * nkv + kh) * HD + lj) * static_cast<long>(page_size) + off + lg * 4;
-#pragma unroll
-                for (int kd = 0; kd < KD; ++kd)
-                    kk[i][kt][kd] = ok ? *reinterpret_cast<const uint4*>(kp + kd * 32) : uint4{0u, 0u, 0u, 0u};
-#pragma unroll
-                for (int d = 0; d < DT; ++d)
-                    vv[i][kt][d] = ok ? *reinterpret_cast<const uint2*>(vp + static_cast<long>(d) * 16 * page_size)
-                                      : uint2{0u, 0u};
-            }
-    };
-    // The queries.  Their loads are issued here, ahead of the first round of keys and values, and used behind
-    // it: loads are waited for in the order of their issue, so what the fused variant computes from its loads
-    // (which come from L2) is done while the keys and values (from HBM) are still on their way.
-    bf16x8 q[KD];
-    constexpr int half = HD / 2, INF = 8;
+    // ---- FUSED: what the queries, and the new token's key and value, are made of.  An item is two neighbouring pairs
+    // (i, i + half), (i + 1, i + 1 + half) of a head; heads past the queries are the key and the value.
+    constexpr int half = HD / 2, kItems = half / 2;
     struct Item {
-        float ta[INF], tb[INF], b0, b1, cs, sn;
+        u32x2 ta[INF], tb[INF];
+        uint32_t ba, bb;                         // bias
+        u32x4 turn;                              // cos, sin of both pairs
+    };
+    auto item_col = [&](unsigned it) {
+        const int h = it / kItems, i = it % kItems * 2, past = h - group_size;
+        const int query = kh * group_size + h, other = nq + kh + past * nkv;
+        return (past < 0 ? query : other) * HD + i;
+    };
+    const int stride = d.n_tokens * width;                       // values of a partial sum
+    const buffer_t prod_buf = values_of(f.prod + static_cast<size_t>(tok) * width, ((f.in_splits - 1) * stride + width) * 4);
+    const buffer_t bias_buf = values_of(f.bias, f.bias ? width * 2 : 0);
+    const buffer_t turn_buf = values_of(f.cos_sin + static_cast<size_t>(tok) * HD, HD * 4);
+    auto parts_load = [&](int col, int j0, u32x2 (&ta)[INF], u32x2 (&tb)[INF]) {
+#pragma unroll
+        for (int j = 0; j < INF; ++j) {
+            const int at = (j0 + j) * stride * 4 + col * 4;              // (behind the last sum: past the buffer's end)
+            ta[j] = read8(prod_buf, at);
+            tb[j] = read8(prod_buf, at + half * 4);
+        }
+    };
+    auto item_load = [&](unsigned it, Item& r) {
+        const int col = item_col(it);
+        parts_load(col, 0, r.ta, r.tb);
+        r.ba = read4(bias_buf, col * 2);
+        r.bb = read4(bias_buf, col * 2 + half * 2);
+        r.turn = read16(turn_buf, it % kItems * 16);
     };
     [[maybe_unused]] Item first;
-    [[maybe_unused]] float sst[16];
-    [[maybe_unused]] int slot_page = 0, slot_off = 0;
-    const int n_items = FUSED ? (group_size + (writer ? 2 : 0)) * half : 0;      // pairs (i, i + half) of a head
-    const size_t stride = static_cast<size_t>(n_tokens) * width;
-    auto item_col = [&](int it) {
-        const int h = it / half, i = it % half;
-        return (h < group_size ? kh * group_size + h : h == group_size ? nq + kh : nq + nkv + kh) * HD + i;
-    };
-    auto item_load = [&](int it, Item& r) {
-        const int h = it / half, i = it % half, col = item_col(it);
-        const float* src = f.prod + static_cast<size_t>(tok) * width + col;
-#pragma unroll
-        for (int j = 0; j < INF; ++j) {
-            const float* pj = src + min(j, f.in_splits - 1) * stride;
-            r.ta[j] = pj[0];
-            r.tb[j] = pj[half];
-        }
-        r.b0 = f.bias ? to_float(f.bias[col]) : 0.f;
-        r.b1 = f.bias ? to_float(f.bias[col + half]) : 0.f;
-        r.cs = 1.f;
-        r.sn = 0.f;
-        if (h <= group_size) {                   // queries and the key are rotated, the value is not
-            r.cs = f.cos_sin[(static_cast<size_t>(tok) * half + i) * 2];
-            r.sn = f.cos_sin[(static_cast<size_t>(tok) * half + i) * 2 + 1];
-        }
-    };
-    auto item_finish = [&](int it, const Item& r, float row_scale) {
-        const int h = it / half, i = it % half, col = item_col(it);
-        float x0 = 0.f, x1 = 0.f;
-#pragma unroll
-        for (int j = 0; j < INF; ++j) {
-            if (j < f.in_splits) {
-                x0 += r.ta[j];
-                x1 += r.tb[j];
-            }
-        }
-        const float* src = f.prod + static_cast<size_t>(tok) * width + col;
-        // more partial sums than one batch of loads (7B and 14B sizes): a batch is one trip to memory, not a trip each (8 requests of
-        // 500 to 1,400 tokens, 28 heads of 128 on 4, 14 partial sums: 16.8 us with a trip each, 12.8 so)
-        for (int j0 = INF; j0 < f.in_splits; j0 += INF) {
-            float ta[INF], tb[INF];
-#pragma unroll
-            for (int j = 0; j < INF; ++j) {
-                const float* pj = src + min(j0 + j, f.in_splits - 1) * stride;
-                ta[j] = pj[0];
-                tb[j] = pj[half];
-            }
-#pragma unroll
-            for (int j = 0; j < INF; ++j) {
-                if (j0 + j < f.in_splits) {
-                    x0 += ta[j];
-                    x1 += tb[j];
-                }
-            }
-        }
-        x0 = scale_then_bias(x0, row_scale, r.b0);
-        x1 = scale_then_bias(x1, row_scale, r.b1);
-        if (h <= group_size) {
-            float r0, r1;
-            rotate_pair(x0, x1, r.cs, r.sn, r0, r1);
-            x0 = r0;
-            x1 = r1;
-        }
-        const bf16_t y0 = from_float<bf16_t>(x0), y1 = from_float<bf16_t>(x1);
-        const long page = slot_page, off = slot_off;
-        if (h < group_size) {
-            q_lds[h * HD + i] = y0;
-            q_lds[h * HD + i + half] = y1;
-        } else if (h == group_size) {            // keys: [page][kv head][offset][feature]
-            k_lds[i] = y0;
-            k_lds[i + half] = y1;
-            bf16_t* dst = f.k_cache_w + ((page * nkv + kh) * page_size + off) * HD;
-            dst[i] = y0;
-            dst[i + half] = y1;
-        } else {                                 // values: [page][kv head][feature][offset]
-            v_lds[i] = y0;
-            v_lds[i + half] = y1;
-            f.v_cache_w[((page * nkv + kh) * HD + i) * page_size + off] = y0;
-            f.v_cache_w[((page * nkv + kh) * HD + i + half) * page_size + off] = y1;
-        }
-    };
-    if constexpr (!FUSED) {
-        const bf16_t* qp = qkv + static_cast<size_t>(tok) * width + head * HD + lg * 8;
-#pragma unroll
-        for (int kd = 0; kd < KD; ++kd) {
-            const uint4 v = valid ? *reinterpret_cast<const uint4*>(qp + kd * 32) : uint4{0u, 0u, 0u, 0u};
-            q[kd] = __builtin_bit_cast(bf16x8, v);
-        }
-    } else {
-        if (f.row_ss) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) sst[i] = f.row_ss[min(i, f.ss_splits - 1) * n_tokens + tok];
-        }
-        const int slot = f.slots[tok];
-        slot_page = slot / page_size;
-        slot_off = slot % page_size;
-        if (static_cast<int>(threadIdx.x) < n_items) item_load(threadIdx.x, first);
+    [[maybe_unused]] uint32_t ss_lane = 0;
+    [[maybe_unused]] uint32_t slot = 0;
+    if constexpr (FUSED) {
+        // lane s has the sum of squares of split s
+        ss_lane = read4(values_of(f.row_ss, f.row_ss ? f.ss_splits * d.n_tokens * 4 : 0), lane < f.ss_splits ? (lane * d.n_tokens + tok) * 4 : kNowhere);
+        // (a wavefront without items goes on: a CU's loads go out one after the other.  The key's and the value's items, which only the
+        // last range has, are loaded by every range)
+        if (wave * kWave < (group_size + 2) * kItems) item_load(min(static_cast<int>(threadIdx.x), (group_size + 2) * kItems - 1), first);
+        int here = tok * 4;
+        asm volatile("" : "+v"(here));           // (a lane's value: as the wavefront's it would be waited for at once)
+        slot = read4(values_of(f.slots, d.n_tokens * 4), here);
     }
-    auto make_q = [&]() {
-        if constexpr (FUSED) {
-            float row_scale = 1.f;
-            if (f.row_ss) {
-                float ss = 0.f;
+    bf16x8 q[KD];
+    const bool valid = lj < group_size;
+    if constexpr (!FUSED) {
+        const bf16_t* qp = qkv + static_cast<size_t>(tok) * width + (kh * group_size + (valid ? lj : 0)) * HD + lg * 8;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) ss += i < f.ss_splits ? sst[i] : 0.f;
-                for (int s0 = 16; s0 < f.ss_splits; s0 += 16) {
-                    float part[16];
+        for (int kd = 0; kd < KD; ++kd) q[kd] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + kd * 32));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the keys of this wavefront
+    const int p = kv - 1;
+    const int lo = d.window > 0 ? max(0, p - d.window + 1) : 0;
+    const int kb_begin = lo >> 5, kb_end = (max(p, 0) >> 5) + 1;
+    const int per_split = RANGED ? 0 : divided(kb_end - kb_begin + n_splits - 1, n_splits, d.split_magic);
+    const int s_begin = RANGED ? range[1] : kb_begin + bz * per_split, s_end = RANGED ? range[2] : min(kb_end, s_begin + per_split);
+    const int per_wave = divided(max(s_end - s_begin, 0) + n_waves - 1, n_waves, d.wave_magic);
+    const int w_begin = s_begin + wave * per_wave, w_end = min(s_end, w_begin + per_wave);
+    // FUSED: does this workgroup's key range end with the new token?
+    const bool writer = FUSED && (RANGED ? s_end == kb_end : s_begin < kb_end && s_begin + per_split >= kb_end);
+
+    // One round of loads: PF blocks of 32 keys and their values for this wavefront, first all page numbers
+    // (one wait for all of them), then all key and value loads.
+    uint4 kk[PF][2][KD];
+    uint2 vv[PF][2][DT];
+    const unsigned head_bytes = page_size * (HD * 2), page_bytes = head_bytes * nkv;
+    const char* k_head = reinterpret_cast<const char*>(k_cache) + static_cast<size_t>(kh) * head_bytes;
+    const char* v_head = reinterpret_cast<const char*>(v_cache) + static_cast<size_t>(kh) * head_bytes;
+    const int k_at = lj * (HD * 2) + lg * 16;
+    int v_at[DT];
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) part[i] = f.row_ss[min(s0 + i, f.ss_splits - 1) * n_tokens + tok];
+    for (int dt = 0; dt < DT; ++dt) v_at[dt] = (dt * 16 + lj) * page_size * 2 + lg * 8;
+    auto load_round = [&](int kb0) {
+        int pages[PF][2], offs[PF][2];
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) ss += s0 + i < f.ss_splits ? part[i] : 0.f;
-                }
-                row_scale = inv_rms(ss, f.inv_hidden, f.eps);
+        for (int i = 0; i < PF; ++i)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const int key0 = (kb0 + i) * 32 + kt * 16;
+                const bool live = kb0 + i < w_end && key0 <= p && key0 + 15 >= lo;
+                const int at = divided(key0 >> 4, page_size >> 4, d.page_magic);
+                offs[i][kt] = live ? key0 - at * page_size : -1;
+                pages[i][kt] = table[live ? at : 0];
             }
-            if (static_cast<int>(threadIdx.x) < n_items) item_finish(threadIdx.x, first, row_scale);
-            for (int it = threadIdx.x + blockDim.x; it < n_items; it += blockDim.x) {
-                Item r;
-                item_load(it, r);
-                item_finish(it, r, row_scale);
-            }
-            __syncthreads();
+        // (all of them asked for before one is waited for)
+        if constexpr (PF == 1) asm volatile("" : "+s"(pages[0][0]), "+s"(pages[0][1]));
+        if constexpr (PF >= 2) asm volatile("" : "+s"(pages[0][0]), "+s"(pages[0][1]), "+s"(pages[1][0]), "+s"(pages[1][1]));
+        if constexpr (PF == 4) asm volatile("" : "+s"(pages[2][0]), "+s"(pages[2][1]), "+s"(pages[3][0]), "+s"(pages[3][1]));
 #pragma unroll
-            for (int kd = 0; kd < KD; ++kd) {
-                const uint4 v = valid ? *reinterpret_cast<const uint4*>(q_lds + lj * HD + kd * 32 + lg * 8)
-                                      : uint4{0u, 0u, 0u, 0u};
-                q[kd] = __builtin_bit_cast(bf16x8, v);
+        for (int i = 0; i < PF; ++i)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const bool ok = offs[i][kt] >= 0 && pages[i][kt] >= 0;
+                const unsigned off = ok ? offs[i][kt] : 0;
+                const size_t at = static_cast<size_t>(static_cast<unsigned>(ok ? pages[i][kt] : 0)) * page_bytes;
+                const buffer_t kr = values_of(k_head + at + off * (HD * 2), ok ? 16 * HD * 2 : 0);
+                const buffer_t vr = values_of(v_head + at + off * 2, ok ? static_cast<size_t>(head_bytes - off * 2) : 0);
+#pragma unroll
+                for (int kd = 0; kd < KD; ++kd) kk[i][kt][kd] = __builtin_bit_cast(uint4, read16(kr, k_at + kd * 64));
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) vv[i][kt][dt] = __builtin_bit_cast(uint2, read8(vr, v_at[dt]));
             }
-        }
     };
+    load_round(w_begin);
+    __builtin_amdgcn_sched_barrier(0);
+
+    if constexpr (FUSED) {
+        float row_scale = 1.f;
+        if (f.row_ss) {
+            float ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ss += __uint_as_float(__builtin_amdgcn_readlane(ss_lane, i));
+            if (__builtin_expect(f.ss_splits > 8, 0)) {
+                for (int s0 = 8; s0 < min(f.ss_splits, kWave); s0 += 8)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) ss += __uint_as_float(__builtin_amdgcn_readlane(ss_lane, s0 + i));
+                for (int s0 = kWave; s0 < f.ss_splits; ++s0) ss += f.row_ss[s0 * d.n_tokens + tok];
+            }
+            row_scale = inv_rms(ss, f.inv_hidden, f.eps);
+        }
+        auto item_finish = [&](unsigned it, const Item& r) {
+            const int h = it / kItems, i = it % kItems * 2;
+            float x0[2] = {0.f, 0.f}, x1[2] = {0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < INF; ++j)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    x0[e] += __uint_as_float(r.ta[j][e]);
+                    x1[e] += __uint_as_float(r.tb[j][e]);
+                }
+            // more partial sums than one batch of loads: a batch is one trip to memory, not a trip each
+            for (int j0 = INF; __builtin_expect(j0 < f.in_splits, 0); j0 += INF) {
+                u32x2 ta[INF], tb[INF];
+                parts_load(item_col(it), j0, ta, tb);
+#pragma unroll
+                for (int j = 0; j < INF; ++j)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        x0[e] += __uint_as_float(ta[j][e]);
+                        x1[e] += __uint_as_float(tb[j][e]);
+                    }
+            }
+            const uint32_t b0[2] = {r.ba << 16, r.ba & 0xffff0000u}, b1[2] = {r.bb << 16, r.bb & 0xffff0000u};
+            bf16_t y0[2], y1[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                x0[e] = scale_then_bias(x0[e], row_scale, __uint_as_float(b0[e]));
+                x1[e] = scale_then_bias(x1[e], row_scale, __uint_as_float(b1[e]));
+                float r0, r1;                    // queries and the key are rotated, the value is not
+                rotate_pair(x0[e], x1[e], __uint_as_float(r.turn[2 * e]), __uint_as_float(r.turn[2 * e + 1]), r0, r1);
+                x0[e] = h <= group_size ? r0 : x0[e];
+                x1[e] = h <= group_size ? r1 : x1[e];
+                y0[e] = from_float<bf16_t>(x0[e]);
+                y1[e] = from_float<bf16_t>(x1[e]);
+            }
+            bf16_t* to = q_lds + (h < group_size ? h : 16 + h - group_size) * HD;      // (the key and the value lie behind 16 queries)
+            *reinterpret_cast<uint32_t*>(to + i) = y0[0].bits | static_cast<uint32_t>(y0[1].bits) << 16;
+            *reinterpret_cast<uint32_t*>(to + i + half) = y1[0].bits | static_cast<uint32_t>(y1[1].bits) << 16;
+            if (__builtin_expect(h < group_size, 1)) return;
+            const uint32_t page = slot / static_cast<uint32_t>(page_size), off = slot - page * page_size;
+            if (h == group_size) {               // keys: [page][kv head][offset][feature]
+                bf16_t* dst = f.k_cache_w + ((static_cast<size_t>(page) * nkv + kh) * page_size + off) * HD + i;
+                dst[0] = y0[0];
+                dst[1] = y0[1];
+                dst[half] = y1[0];
+                dst[half + 1] = y1[1];
+            } else {                             // values: [page][kv head][feature][offset]
+                bf16_t* dst = f.v_cache_w + ((static_cast<size_t>(page) * nkv + kh) * HD + i) * page_size + off;
+                dst[0] = y0[0];
+                dst[page_size] = y0[1];
+                dst[half * page_size] = y1[0];
+                dst[(half + 1) * page_size] = y1[1];
+            }
+        };
+        const int n_items = (group_size + (writer ? 2 : 0)) * kItems;
+        if (static_cast<int>(threadIdx.x) < n_items) item_finish(threadIdx.x, first);
+        for (int it = threadIdx.x + n_threads; __builtin_expect(it < n_items, 0); it += n_threads) {
+            Item r;
+            item_load(it, r);
+            item_finish(it, r);
+        }
+        __syncthreads();
+        // (a row past the last head holds anything: it is a column of the products that nobody reads)
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd)
+            q[kd] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(q_lds + lj * HD + kd * 32 + lg * 8));
+    }
 
     f32x4 o[DT];
 #pragma unroll
-    for (int d = 0; d < DT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
-
-    // Every wavefront goes through the body at least once (one with no keys loads nothing and multiplies
-    // nothing): the fused variant's queries are made there, behind the first round's loads, with a barrier.
-    int kb0 = w_begin;
-    do {
-        load_round(kb0);
-        if (kb0 == w_begin) {
-            make_q();
-        }
+    for (int kb0 = w_begin; kb0 < w_end; kb0 += PF) {
+        if (kb0 > w_begin) load_round(kb0);
         if constexpr (FUSED) {
             // the new token's key and value come from LDS, not from the cache line that was just written
             if (writer && kb0 <= kb_end - 1 && kb_end - 1 < min(w_end, kb0 + PF)) {
@@ -1433,29 +1462,33 @@ __device__ __forceinline__ void decode_block(
 #pragma unroll
                     for (int kt = 0; kt < 2; ++kt) {
                         const int key0 = (kb0 + i) * 32 + kt * 16;
+                        if (key0 > p || key0 + 15 < p) continue;
                         if (key0 + lj == p) {
 #pragma unroll
                             for (int kd = 0; kd < KD; ++kd)
                                 kk[i][kt][kd] = *reinterpret_cast<const uint4*>(k_lds + kd * 32 + lg * 8);
                         }
                         const int e = p - (key0 + lg * 4);          // which of this lane's four keys, if any
-                        if (e >= 0 && e < 4) {
+                        // what is kept of the lane's two words, and where the new value goes
+                        const uint32_t kx = e == 0 ? 0xffff0000u : e == 1 ? 0x0000ffffu : 0xffffffffu;
+                        const uint32_t ky = e == 2 ? 0xffff0000u : e == 3 ? 0x0000ffffu : 0xffffffffu;
 #pragma unroll
-                            for (int d = 0; d < DT; ++d) {
-                                const uint32_t nv = v_lds[d * 16 + lj].bits;
-                                uint32_t& word = (e < 2) ? vv[i][kt][d].x : vv[i][kt][d].y;
-                                word = (e & 1) ? ((word & 0x0000ffffu) | (nv << 16)) : ((word & 0xffff0000u) | nv);
-                            }
+                        for (int dt = 0; dt < DT; ++dt) {
+                            const uint32_t nv = v_lds[dt * 16 + lj].bits, both = nv | nv << 16;
+                            vv[i][kt][dt].x = (vv[i][kt][dt].x & kx) | (both & ~kx);
+                            vv[i][kt][dt].y = (vv[i][kt][dt].y & ky) | (both & ~ky);
                         }
                     }
                 }
             }
         }
+        // the scores of all the round's keys, then one maximum, one factor for what was there before and their products (a block
+        // past the wavefront's last has no visible key and zeros for values)
+        const int last = min(p, w_end * 32 - 1);
+        float s[PF][2][4];
+        float mx = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < PF; ++i) {
-            if (kb0 + i >= w_end) break;
-            float s[2][4];
-            float mx = -INFINITY;
+        for (int i = 0; i < PF; ++i)
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
                 f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1466,71 +1499,82 @@ __device__ __forceinline__ void decode_block(
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int key = (kb0 + i) * 32 + kt * 16 + lg * 4 + v;
-                    const bool vis = valid && key <= p && key >= lo;
-                    s[kt][v] = vis ? acc[v] * scale : -INFINITY;
-                    mx = fmaxf(mx, s[kt][v]);
+                    const bool vis = valid && key <= last && key >= lo;
+                    s[i][kt][v] = vis ? acc[v] * d.scale : -INFINITY;
+                    mx = fmaxf(mx, s[i][kt][v]);
                 }
             }
-            mx = fold_rows(mx, MaxOf());
-            const float m_new = fmaxf(m_run, mx);
-            const bool none = m_new == -INFINITY;
-            const float alpha = none ? 1.f : __expf(m_run - m_new);
-            float sum = 0.f;
+        mx = fold_rows(mx, MaxOf());
+        const float m_new = fmaxf(m_run, mx);
+        const bool none = m_new == -INFINITY;
+        const float from = none ? 0.f : m_new;             // (no key yet: exp(-infinity - 0) is zero)
+        const float alpha = none ? 1.f : __expf(m_run - m_new);
+        float sum = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) { o[dt][0] *= alpha; o[dt][1] *= alpha; o[dt][2] *= alpha; o[dt][3] *= alpha; }
+#pragma unroll
+        for (int i = 0; i < PF; ++i) {
             bf16x8 pb;
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const float pv = none ? 0.f : __expf(s[kt][v] - m_new);
+                    const float pv = __expf(s[i][kt][v] - from);
                     sum += pv;
                     pb[kt * 4 + v] = static_cast<__bf16>(pv);
                 }
-            l_run = l_run * alpha + sum;
-            m_run = m_new;
 #pragma unroll
-            for (int d = 0; d < DT; ++d) {
-                const uint4 av = uint4{vv[i][0][d].x, vv[i][0][d].y, vv[i][1][d].x, vv[i][1][d].y};
-                f32x4 acc = o[d];
-                acc[0] *= alpha; acc[1] *= alpha; acc[2] *= alpha; acc[3] *= alpha;
-                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb, acc, 0, 0, 0);
+            for (int dt = 0; dt < DT; ++dt) {
+                const uint4 av = uint4{vv[i][0][dt].x, vv[i][0][dt].y, vv[i][1][dt].x, vv[i][1][dt].y};
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), pb, o[dt], 0, 0, 0);
             }
         }
-        kb0 += PF;
-    } while (kb0 < w_end);
+        l_run = l_run * alpha + sum;
+        m_run = m_new;
+    }
     float l = l_run;
     l = fold_rows(l, AddOf());
 
     // every wavefront leaves its state in LDS; then all threads combine
     float* mine = wave_state + (wave * 16 + lj) * kRow;
 #pragma unroll
-    for (int d = 0; d < DT; ++d)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) mine[d * 16 + lg * 4 + v] = o[d][v];
+        for (int v = 0; v < 4; ++v) mine[dt * 16 + lg * 4 + v] = o[dt][v];
     if (lg == 0) {
         mine[HD] = m_run;
         mine[HD + 1] = l;
     }
     __syncthreads();
     const size_t row0 = static_cast<size_t>(tok) * nq + kh * group_size;
-    for (int idx = threadIdx.x; idx < group_size * HD; idx += blockDim.x) {
-        const int r = idx / HD, d = idx % HD;
-        float mx = -INFINITY;
-        for (int w = 0; w < n_waves; ++w) mx = fmaxf(mx, wave_state[(w * 16 + r) * kRow + HD]);
+    for (int idx = threadIdx.x; idx < group_size * HD; idx += n_threads) {
+        const int r = idx / HD, c = idx % HD;
+        // the states of all wavefronts are read together (past the last one the last again, which weighs nothing)
+        float ms[8], ls[8], os[8], mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            const float* st = wave_state + (min(w, n_waves - 1) * 16 + r) * kRow;
+            const float m = st[HD];
+            ms[w] = w < n_waves ? m : -INFINITY;
+            ls[w] = st[HD + 1];
+            os[w] = st[c];
+            mx = fmaxf(mx, ms[w]);
+        }
         float num = 0.f, den = 0.f;
-        for (int w = 0; w < n_waves; ++w) {
-            const float* st = wave_state + (w * 16 + r) * kRow;
-            const float wgt = st[HD] == -INFINITY ? 0.f : __expf(st[HD] - mx);
-            num += wgt * st[d];
-            den += wgt * st[HD + 1];
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            const float wgt = ms[w] == -INFINITY ? 0.f : __expf(ms[w] - mx);
+            num += wgt * os[w];
+            den += wgt * ls[w];
         }
         if (n_splits == 1) {
-            out[(row0 + r) * HD + d] = from_float<bf16_t>(num / den);
+            out[(row0 + r) * HD + c] = from_float<bf16_t>(num / den);
         } else {
             const size_t prow = RANGED ? static_cast<size_t>(bx) * nq + kh * group_size + r
-                                       : static_cast<size_t>(split) * n_tokens * nq +
+                                       : static_cast<size_t>(bz) * d.n_tokens * nq +
                                              (MIXED ? static_cast<size_t>(b) * nq + kh * group_size : row0) + r;
-            part_o[prow * HD + d] = num;
-            if (d == 0) {
+            part_o[prow * HD + c] = num;
+            if (c == 0) {
                 part_ml[prow * 2] = mx;
                 part_ml[prow * 2 + 1] = den;
             }
@@ -1538,18 +1582,20 @@ __device__ __forceinline__ void decode_block(
     }
 }
 
-template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false>
+// INF: partial sums of the product that are read in one batch (FUSED)
+template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false, int INF = 8>
 __global__ __launch_bounds__(512) void attention_decode_kernel(
-    // (what the first loads are addressed by: 14 words that arrive with the wavefronts)
-    const int32_t* __restrict__ lengths, const int32_t* __restrict__ q_start, const int32_t* __restrict__ block_table,
-    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, int table_width, int page_size, int nkv, int n_splits,
-    int nq, int window, float scale, int n_tokens, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, const int32_t* __restrict__ q_len, FusedQkv f) {
-    const int32_t* kv_len = RANGED ? nullptr : lengths;
-    const int32_t* ranges = RANGED ? lengths : nullptr;
+    // (what the first loads are addressed by: 14 words that arrive with the wavefronts; `lengths` is the table of ranges where
+    // there is one)
+    const int32_t* __restrict__ lengths, const int32_t* __restrict__ block_table, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, int table_width, int page_size, int nkv, int n_splits, unsigned page_magic, unsigned split_magic,
+    unsigned wave_magic, int group, int window, int n_tokens, float scale, int n_waves, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out,
+    float* __restrict__ part_o, float* __restrict__ part_ml, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
+    FusedQkv f) {
     extern __shared__ float wave_state[];
-    decode_block<HD, PF, FUSED, MIXED, RANGED>(wave_state, blockIdx.x, blockIdx.y, blockIdx.z, qkv, out, part_o, part_ml, k_cache, v_cache, block_table,
-                                               table_width, q_start, kv_len, n_tokens, nq, nkv, page_size, scale, window, n_splits, f, q_len, ranges);
+    const DecodeSizes d{table_width, page_size, nkv, n_splits, page_magic, split_magic, wave_magic, group, window, n_tokens, scale, n_waves};
+    decode_block<HD, PF, FUSED, MIXED, RANGED, INF>(wave_state, blockIdx.x, blockIdx.y, blockIdx.z, lengths, block_table, k_cache, v_cache, d, qkv, out,
+                                                    part_o, part_ml, q_start, q_len, f);
 }
 
 // Portions of prompts in blocks of 32 RB rows and, behind them in the same launch, the requests of one token dealt out by `ranges`
@@ -1561,7 +1607,7 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_width,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ kv_len,
-    int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int late, int row_blocks,
+    int n_seqs, int nq, int nkv, int page_size, int page_shift, float scale, int window, int late, int row_blocks, unsigned page_magic,
     const int32_t* __restrict__ ranges, int range_slots, float* __restrict__ range_o, float* __restrict__ range_ml) {
     static_assert(RB * KS == 8, "eight wavefronts, as the decoded tokens have");
     __shared__ __attribute__((aligned(128))) char smem[kRows32Lds<HD, RB, KS>];
@@ -1572,9 +1618,9 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
                                       page_size, page_shift, scale, window, 1, nullptr, nullptr, 1, 0, (nq + 2 * nkv) * HD, late);
     } else {
         const int i = index - row_blocks;
-        decode_block<HD, 2, false, true, true>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, qkv, out, range_o, range_ml, k_cache,
-                                               v_cache, block_table, table_width, q_start, kv_len, n_seqs, nq, nkv, page_size, scale, window, 1,
-                                               FusedQkv{}, q_len, ranges);
+        const DecodeSizes d{table_width, page_size, nkv, 1, page_magic, 0, (1u << 28) + 1, nq / nkv, window, n_seqs, scale, 8};
+        decode_block<HD, 2, false, true, true, 8>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, ranges, block_table, k_cache, v_cache,
+                                                  d, qkv, out, range_o, range_ml, q_start, q_len, FusedQkv{});
     }
 }
 
@@ -1677,6 +1723,14 @@ static int launch_mfma(const void* qkv, void* out, float* part_o, float* part_ml
 
 constexpr int kDecodeLdsMost = 96 * 1024;       // bytes of LDS a workgroup of the decode kernel may ask for
 
+template <auto Kernel>
+static bool raise_lds() {
+    static bool raised = false;
+    if (!raised)
+        raised = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kDecodeLdsMost) == hipSuccess;
+    return raised;
+}
+
 // PF: key blocks per round of loads of a wavefront.  More of them in flight is fewer round trips but more
 // registers; when there are so many workgroups that they must share CUs, fewer registers are worth more.
 template <int HD, int PF>
@@ -1690,32 +1744,26 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
     size_t lds = static_cast<size_t>(n_waves) * 16 * (HD + 2) * sizeof(float);
     if (fused) lds += 18 * HD * sizeof(bf16_t);          // 16 query heads, the new key and value
     if (lds > kDecodeLdsMost) return EGPT_UNSUPPORTED_SIZE;
-    if (lds > 64 * 1024) {
-        // (eight wavefronts at head size 128: more than a kernel may take without being asked; once per instance)
-        static bool raised_fused = false, raised_plain = false, raised_mixed = false, raised_ranged_fused = false, raised_ranged = false;
-        bool& raised = ranges ? (fused ? raised_ranged_fused : raised_ranged) : fused ? raised_fused : q_len ? raised_mixed : raised_plain;
-        if (!raised) {
-            const void* fn = ranges && fused ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, 2, true, false, true>)
-                             : ranges        ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, 2, false, true, true>)
-                             : fused   ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, true>)
-                             : q_len ? reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, false, true>)
-                                     : reinterpret_cast<const void*>(&attention_decode_kernel<HD, PF, false>);
-            if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kDecodeLdsMost) != hipSuccess)
-                return EGPT_UNSUPPORTED_SIZE;
-            raised = true;
-        }
-    }
     const FusedQkv fq = fused ? *fused : FusedQkv{};
-    auto launch = [&](auto kernel, const int32_t* lengths, const void* q, const int32_t* counts, int splits) {
-        kernel<<<grid, n_waves * kWave, lds, s>>>(lengths, q_start, block_table, static_cast<const bf16_t*>(k_cache),
-                                                  static_cast<const bf16_t*>(v_cache), table_width, page_size, nkv, splits, nq, window, scale,
-                                                  n_tokens, static_cast<const bf16_t*>(q), static_cast<bf16_t*>(out), part_o, part_ml, counts, fq);
+    auto launch = [&](auto kernel, bool (*raise)(), const int32_t* lengths, const void* q, const int32_t* counts, int splits) {
+        // (eight wavefronts at head size 128: more than a kernel may take without being asked; once per instance)
+        if (lds > 64 * 1024 && !raise()) return EGPT_UNSUPPORTED_SIZE;
+        kernel<<<grid, n_waves * kWave, lds, s>>>(lengths, block_table, static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
+                                                  table_width, page_size, nkv, splits, magic_of(page_size / 16), magic_of(splits), magic_of(n_waves), nq / nkv,
+                                                  window, n_tokens, scale, n_waves, static_cast<const bf16_t*>(q), static_cast<bf16_t*>(out), part_o, part_ml, q_start, counts, fq);
+        return EGPT_OK;
     };
-    if (ranges && fused) launch(attention_decode_kernel<HD, 2, true, false, true>, ranges, nullptr, nullptr, 1);
-    else if (ranges) launch(attention_decode_kernel<HD, 2, false, true, true>, ranges, qkv, q_len, 1);
-    else if (fused) launch(attention_decode_kernel<HD, PF, true>, kv_len, nullptr, nullptr, n_splits);
-    else if (q_len) launch(attention_decode_kernel<HD, PF, false, true>, kv_len, qkv, q_len, n_splits);
-    else launch(attention_decode_kernel<HD, PF, false>, kv_len, qkv, nullptr, n_splits);
+    int e;
+#define EGPT_DECODE(...) attention_decode_kernel<HD, __VA_ARGS__>, raise_lds<attention_decode_kernel<HD, __VA_ARGS__>>
+    if (ranges && fused) e = fused->in_splits > 8 ? launch(EGPT_DECODE(2, true, false, true, 16), ranges, nullptr, nullptr, 1)
+                                                  : launch(EGPT_DECODE(2, true, false, true, 8), ranges, nullptr, nullptr, 1);
+    else if (ranges) e = launch(EGPT_DECODE(2, false, true, true), ranges, qkv, q_len, 1);
+    else if (fused) e = fused->in_splits > 8 ? launch(EGPT_DECODE(PF, true, false, false, 16), kv_len, nullptr, nullptr, n_splits)
+                                             : launch(EGPT_DECODE(PF, true, false, false, 8), kv_len, nullptr, nullptr, n_splits);
+    else if (q_len) e = launch(EGPT_DECODE(PF, false, true), kv_len, qkv, q_len, n_splits);
+    else e = launch(EGPT_DECODE(PF, false), kv_len, qkv, nullptr, n_splits);
+#undef EGPT_DECODE
+    if (e != EGPT_OK) return e;
     EGPT_CHECK_LAUNCH();
     if (ranges) {
         attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, q_start, q_len, ranges + slots * kRangeInts, n_tokens * nq, HD, 1, nq,
@@ -1797,8 +1845,8 @@ static int launch_mixed(const void* qkv, void* out, const void* k_cache, const v
     if (grid > 0x7fffffffL) return EGPT_UNSUPPORTED_SIZE;
     attention_mixed_kernel<HD, RB, KS><<<static_cast<unsigned>(grid), 512, 0, s>>>(
         static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
-        block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, late, static_cast<int>(blocks), ranges,
-        slots, range_o, range_ml);
+        block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, late, static_cast<int>(blocks),
+        magic_of(page_size / 16), ranges, slots, range_o, range_ml);
     EGPT_CHECK_LAUNCH();
     attention_reduce_kernel<<<n_seqs * nq, 64, 0, s>>>(range_o, range_ml, q_start, q_len, ranges + slots * kRangeInts, n_seqs * nq, HD, 1, nq,
                                                        static_cast<bf16_t*>(out));
@@ -2000,6 +2048,8 @@ static int attention_decode_fused(const float* qkv_prod, int in_splits, const fl
     if ((hd != 64 && hd != 128) || page_size % 16 != 0 || nq / nkv > 16 || nkv > 65535 || n_splits > 64 ||
         n_waves < 1 || n_waves > 8)
         return EGPT_UNSUPPORTED_SIZE;
+    // (a row's partial sums are read through a buffer whose places are 32 bits, up to 32 more of them than there are; two biases at once)
+    if ((in_splits + 32LL) * n_seqs * (nq + 2 * nkv) * hd * 4 > INT32_MAX || (reinterpret_cast<uintptr_t>(bias) & 3) != 0) return EGPT_UNSUPPORTED_SIZE;
     FusedQkv f = {};
     f.prod = qkv_prod; f.in_splits = in_splits;
     f.row_ss = row_ss; f.ss_splits = row_ss ? ss_splits : 0;

@@ -29,4 +29,18 @@ __device__ __forceinline__ r_i32x4 buffer_of(const void* p, size_t bytes) {
                    __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000};
 }
 
+// Loads bounded by a buffer's bytes: what lies past them reads as zero, without a branch around the load.  `p` and `bytes` are the
+// same for the whole wavefront, at most kNowhere.
+constexpr int kNowhere = static_cast<int>(0x80000000u);
+typedef __amdgpu_buffer_rsrc_t buffer_t;
+typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+__device__ __forceinline__ buffer_t values_of(const void* p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
+}
+__device__ __forceinline__ uint32_t read2(buffer_t b, int offset) { return __builtin_amdgcn_raw_buffer_load_b16(b, offset, 0, 0); }
+__device__ __forceinline__ uint32_t read4(buffer_t b, int offset) { return __builtin_amdgcn_raw_buffer_load_b32(b, offset, 0, 0); }
+__device__ __forceinline__ u32x2 read8(buffer_t b, int offset) { return __builtin_amdgcn_raw_buffer_load_b64(b, offset, 0, 0); }
+__device__ __forceinline__ u32x4 read16(buffer_t b, int offset) { return __builtin_amdgcn_raw_buffer_load_b128(b, offset, 0, 0); }
+
 }  // namespace egpt
