@@ -34,7 +34,7 @@ __device__ __forceinline__ void store_piece(bf16_t* p, const float* v) {
     uint32_t w[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        w[i] = static_cast<uint32_t>(f32_to_bf16_bits(v[2 * i])) | (static_cast<uint32_t>(f32_to_bf16_bits(v[2 * i + 1])) << 16);
+        w[i] = bf16_pair(v[2 * i], v[2 * i + 1]);
     *reinterpret_cast<uint4*>(p) = uint4{w[0], w[1], w[2], w[3]};
 }
 

@@ -229,8 +229,8 @@ __global__ __launch_bounds__(64) void attention_mfma_kernel(
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
                 uint2 packed;
-                packed.x = f32_to_bf16_bits(o[t][d][0] * inv) | (static_cast<uint32_t>(f32_to_bf16_bits(o[t][d][1] * inv)) << 16);
-                packed.y = f32_to_bf16_bits(o[t][d][2] * inv) | (static_cast<uint32_t>(f32_to_bf16_bits(o[t][d][3] * inv)) << 16);
+                packed.x = bf16_pair(o[t][d][0] * inv, o[t][d][1] * inv);
+                packed.y = bf16_pair(o[t][d][2] * inv, o[t][d][3] * inv);
                 *reinterpret_cast<uint2*>(op + d * 16) = packed;
             }
         } else {
@@ -505,8 +505,8 @@ __global__ __launch_bounds__(64 * RT * KS) void attention_tiled_kernel(
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             uint2 packed;
-            packed.x = f32_to_bf16_bits(o[d][0] * inv) | (static_cast<uint32_t>(f32_to_bf16_bits(o[d][1] * inv)) << 16);
-            packed.y = f32_to_bf16_bits(o[d][2] * inv) | (static_cast<uint32_t>(f32_to_bf16_bits(o[d][3] * inv)) << 16);
+            packed.x = bf16_pair(o[d][0] * inv, o[d][1] * inv);
+            packed.y = bf16_pair(o[d][2] * inv, o[d][3] * inv);
             *reinterpret_cast<uint2*>(op + d * 16) = packed;
         }
     }
@@ -1056,8 +1056,8 @@ __device__ __forceinline__ void rows32_block(
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 uint2 packed;
-                packed.x = f32_to_bf16_bits(o[f][g * 4] * inv) | (static_cast<uint32_t>(f32_to_bf16_bits(o[f][g * 4 + 1] * inv)) << 16);
-                packed.y = f32_to_bf16_bits(o[f][g * 4 + 2] * inv) | (static_cast<uint32_t>(f32_to_bf16_bits(o[f][g * 4 + 3] * inv)) << 16);
+                packed.x = bf16_pair(o[f][g * 4] * inv, o[f][g * 4 + 1] * inv);
+                packed.y = bf16_pair(o[f][g * 4 + 2] * inv, o[f][g * 4 + 3] * inv);
                 *reinterpret_cast<uint2*>(op + f * 32 + g * 8) = packed;
             }
     }

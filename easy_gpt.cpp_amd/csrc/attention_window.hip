@@ -246,8 +246,8 @@ template <typename T>
 __device__ __forceinline__ void store_four(T* dst, float a, float b, float c, float d) {
     if constexpr (sizeof(T) == 2) {
         uint2 packed;
-        packed.x = f32_to_bf16_bits(a) | (static_cast<uint32_t>(f32_to_bf16_bits(b)) << 16);
-        packed.y = f32_to_bf16_bits(c) | (static_cast<uint32_t>(f32_to_bf16_bits(d)) << 16);
+        packed.x = bf16_pair(a, b);
+        packed.y = bf16_pair(c, d);
         *reinterpret_cast<uint2*>(dst) = packed;
     } else {
         *reinterpret_cast<float4*>(dst) = float4{a, b, c, d};

@@ -16,11 +16,13 @@ __device__ __forceinline__ float to_float(float v) { return v; }
 __device__ __forceinline__ float to_float(bf16_t v) { return __uint_as_float(static_cast<uint32_t>(v.bits) << 16); }
 
 // round to nearest even; NaN stays NaN
-__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x0040u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
+// (v_cvt_pk_bf16_f32: one instruction for two values in the place of some fourteen; the same bits as rounding half to even on the
+// integer, NaN made quiet, for every one of the 2^32 float32 values)
+__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
+__device__ __forceinline__ uint32_t bf16_pair(float low, float high) {
+    typedef __attribute__((ext_vector_type(2))) float two;
+    typedef __attribute__((ext_vector_type(2))) __bf16 two_bf16;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((two{low, high}), two_bf16));
 }
 
 template <typename T>

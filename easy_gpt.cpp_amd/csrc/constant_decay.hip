@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64 * RT) void chunk_outputs_kernel(DecayArgs<T> a) 
                     uint32_t w[4];
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        w[i] = f32_to_bf16_bits(y[d + 2 * i]) | (static_cast<uint32_t>(f32_to_bf16_bits(y[d + 2 * i + 1])) << 16);
+                        w[i] = bf16_pair(y[d + 2 * i], y[d + 2 * i + 1]);
                     *reinterpret_cast<uint4*>(dst + lj * DT + d) = uint4{w[0], w[1], w[2], w[3]};
                 }
                 continue;

@@ -207,10 +207,10 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict
 #pragma unroll
         for (int i = 0; i < 8; ++i) w[i] += w_off;
         uint4 o;
-        o.x = f32_to_bf16_bits(v[0] * inv * w[0]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[1] * inv * w[1])) << 16);
-        o.y = f32_to_bf16_bits(v[2] * inv * w[2]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[3] * inv * w[3])) << 16);
-        o.z = f32_to_bf16_bits(v[4] * inv * w[4]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[5] * inv * w[5])) << 16);
-        o.w = f32_to_bf16_bits(v[6] * inv * w[6]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[7] * inv * w[7])) << 16);
+        o.x = bf16_pair(v[0] * inv * w[0], v[1] * inv * w[1]);
+        o.y = bf16_pair(v[2] * inv * w[2], v[3] * inv * w[3]);
+        o.z = bf16_pair(v[4] * inv * w[4], v[5] * inv * w[5]);
+        o.w = bf16_pair(v[6] * inv * w[6], v[7] * inv * w[7]);
         *reinterpret_cast<uint4*>(orow + j) = o;
     }
 }
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(256) void swiglu_vec8_kernel(const GT* __restrict__
         for (int i = 0; i < 4; ++i) {
             const float r0 = u[2 * i] * gate_activation(g[2 * i], act);
             const float r1 = u[2 * i + 1] * gate_activation(g[2 * i + 1], act);
-            ow[i] = f32_to_bf16_bits(r0) | (static_cast<uint32_t>(f32_to_bf16_bits(r1)) << 16);
+            ow[i] = bf16_pair(r0, r1);
         }
         *reinterpret_cast<uint4*>(out + t * inter + j) = uint4{ow[0], ow[1], ow[2], ow[3]};
     }
@@ -375,8 +375,8 @@ __device__ __forceinline__ void load4_as_float(const bf16_t* p, float* v) {
 __device__ __forceinline__ void store4(float* p, const float* v) { *reinterpret_cast<float4*>(p) = float4{v[0], v[1], v[2], v[3]}; }
 __device__ __forceinline__ void store4(bf16_t* p, const float* v) {
     uint2 bits;
-    bits.x = f32_to_bf16_bits(v[0]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[1])) << 16);
-    bits.y = f32_to_bf16_bits(v[2]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[3])) << 16);
+    bits.x = bf16_pair(v[0], v[1]);
+    bits.y = bf16_pair(v[2], v[3]);
     *reinterpret_cast<uint2*>(p) = bits;
 }
 

@@ -75,10 +75,10 @@ __device__ __forceinline__ uint4 load16(const bf16_t* p, bool ok) {
 
 __device__ __forceinline__ uint4 pack8(const float* v) {
     uint4 r;
-    r.x = f32_to_bf16_bits(v[0]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[1])) << 16);
-    r.y = f32_to_bf16_bits(v[2]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[3])) << 16);
-    r.z = f32_to_bf16_bits(v[4]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[5])) << 16);
-    r.w = f32_to_bf16_bits(v[6]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[7])) << 16);
+    r.x = bf16_pair(v[0], v[1]);
+    r.y = bf16_pair(v[2], v[3]);
+    r.z = bf16_pair(v[4], v[5]);
+    r.w = bf16_pair(v[6], v[7]);
     return r;
 }
 

@@ -373,8 +373,8 @@ __global__ __launch_bounds__(1024) void connect_streams_kernel(const float* x, s
         for (int e = 0; e < VEC; ++e) v[e] = row_s[j + e] * inv * to_float(norm_w[j + e]);
         if constexpr (VEC == 4 && sizeof(T) == 2) {
             uint2 packed;
-            packed.x = f32_to_bf16_bits(v[0]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[1])) << 16);
-            packed.y = f32_to_bf16_bits(v[2]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[3])) << 16);
+            packed.x = bf16_pair(v[0], v[1]);
+            packed.y = bf16_pair(v[2], v[3]);
             *reinterpret_cast<uint2*>(orow + j) = packed;
         } else {
 #pragma unroll
