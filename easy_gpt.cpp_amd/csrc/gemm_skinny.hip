@@ -24,6 +24,7 @@
 //   ATTN    x = sum_s wgt_s * o_s: the combination of the partial attention results over key splits.
 #include "api.h"
 #include "common.h"
+#include "lds_loads.h"
 
 namespace egpt {
 
@@ -45,6 +46,7 @@ struct SkinnyArgs {
     bf16_t* out_bf16;
     fixed_t* acc_fixed;        // [m][n] residual stream in fixed point that the product is added into, or null
     int m, n, k, steps_per_split;
+    int whole_out;             // out_f32 takes four neighbouring values at once
     // kPlain
     const bf16_t* x;
     // kNorm
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
     __shared__ __attribute__((aligned(16))) bf16_t xs[2][MT * 16][kLdsRow];
     __shared__ float ss_part[2][16];                                     // kNorm: sums of squares of a short range
     __shared__ float head_wgt[PRO == kAttn ? 16 * kMaxLocalHeads * kMaxAttnSplits : 1];
-    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int li = lane % 16, lg = lane / 16;
     const int split = blockIdx.y;
     const int n0 = (blockIdx.x * NW + wave) * kRowsPerWave;
@@ -170,10 +172,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
     const int step_begin = split * a.steps_per_split;
     const int step_end = min(total_steps, step_begin + a.steps_per_split);
     const int n_steps = step_end - step_begin;
-    const int w_row = min(n0 + li, n - 1);
     // lane group lg takes the lg-th 16 bytes of each 64 of a row: the four groups of a load instruction read 64
-    // contiguous bytes of each of its 16 rows (a memory request is 64 bytes wide; x is read from LDS the same way)
-    const bf16_t* wp = a.w + static_cast<size_t>(w_row) * k + lg * 8;
+    // contiguous bytes of each of its 16 rows (a memory request is 64 bytes wide; x is read from LDS the same way).  What lies past k is
+    // read as zero through the buffer's bound, not behind a branch: eight branches around eight loads are 0.2 us of a kernel of 3.
+    const int row0 = min(n0, n - 1);
+    const buffer_t w_rows = values_of(a.w + static_cast<size_t>(row0) * k, static_cast<size_t>(min(n - row0, kRowsPerWave)) * k * 2);
+    const int w_at = min(li, n - 1 - row0) * k * 2 + lg * 16;
 
     f32x4 acc[MT];
 #pragma unroll
@@ -183,11 +187,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
     auto load_w = [&](uint4* av, int step) {
         const int k0 = step * kStep + lg * 8;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) av[q] = load16(wp + static_cast<size_t>(step) * kStep + q * 32, k0 + q * 32 < k);
+        for (int q = 0; q < 4; ++q)
+            av[q] = __builtin_bit_cast(uint4, read16(w_rows, k0 + q * 32 < k ? w_at + (step * kStep + q * 32) * 2 : kNowhere));
     };
-    // the stream of w starts before anything else
-    if (n_steps > 0) load_w(a_cur, step_begin);
-    if (n_steps > 1) load_w(a_next, step_begin + 1);
+    // the stream of w starts before anything else (a range of one step loads the next one, which is another range's or past k, in vain)
+    load_w(a_cur, step_begin);
+    load_w(a_next, step_begin + 1);
+    // and the arguments that are used last are asked for now
+    asm volatile("" ::"s"(a.out_f32), "s"(a.out_bf16), "s"(a.acc_fixed), "s"(a.bias), "s"(a.whole_out));
+    if constexpr (PRO == kNorm) asm volatile("" ::"s"(a.ss_out), "s"(a.norm_off), "s"(a.delta), "s"(a.delta_splits));
+    if constexpr (PRO == kSwiglu || PRO == kRelu2) asm volatile("" ::"s"(a.inv_hidden), "s"(a.eps), "s"(a.act));
 
     // ---- kAttn with many key splits: the weights of the splits once per workgroup, through LDS
     int head_begin = 0;
@@ -389,12 +398,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
         }
     };
 
-    if (n_steps <= 2) {
+    if (__builtin_expect(n_steps <= 2, 1)) {
         // A short range (the usual case when the k range is split): both steps are staged at once, the
         // chunks of the valid rows dealt out over all threads, so that the prologue is one round of loads.
         const int per_step = m * 16;
         for (int it = tid; it < n_steps * per_step; it += kThreads) {
-            const int s = it / per_step, rem = it % per_step;
+            const int s = it >= per_step ? 1 : 0, rem = it - (s ? per_step : 0);
             const int r = rem / 16;
             float ssq = chunk(s, step_begin + s, r, (rem % 16) * 8);
             if constexpr (PRO == kNorm) {
@@ -490,6 +499,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
                 const int r = idx / (NW * 16), c = idx % (NW * 16);
                 if (col0 + c < n) fixed_add(a.acc_fixed + static_cast<size_t>(r) * n + col0 + c, turned[r][c]);
             }
+        }
+        return;
+    }
+    if (__builtin_expect(a.whole_out, 1)) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const int mm = t * 16 + li, nn = n0 + lg * 4;
+            if (mm < m && nn < n) *reinterpret_cast<f32x4*>(a.out_f32 + (static_cast<size_t>(split) * m + mm) * n + nn) = acc[t];
         }
         return;
     }
@@ -622,8 +639,10 @@ static void launch_skinny(const SkinnyArgs& a, int n_splits, hipStream_t s) {
     } else if (PRO == kAttn) {
         from = a.part_o; with = a.part_ml; parts = a.a_splits; more = a.nq; last = a.hd;
     }
+    SkinnyArgs args = a;
+    args.whole_out = a.out_f32 && !a.bias && a.n % 4 == 0 && reinterpret_cast<uintptr_t>(a.out_f32) % 16 == 0;
     gemm_skinny_kernel<MT, PRO, INF, NW><<<skinny_grid(a.n, n_splits, NW), 64 * NW, 0, s>>>(a.w, from, with, a.m, a.n, a.k, a.steps_per_split,
-                                                                                            parts, more, last, a);
+                                                                                            parts, more, last, args);
 }
 
 // launches the instance for `waves` wavefronts per workgroup (4, 8 or 16)
