@@ -1624,9 +1624,12 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
     }
 }
 
-// out[row, :] = sum_s exp(m_s - M) o_s / sum_s exp(m_s - M) l_s over the splits; one wavefront per row.
-// Lane s first takes split s's (maximum, sum) so that the weights of up to 64 splits are known after one
-// round of loads; the partial outputs are then read eight splits at a time.
+// out[row, :] = sum_s exp(m_s - M) o_s / sum_s exp(m_s - M) l_s over the splits; one wavefront per row, R features of it a lane (R * 64
+// of them or fewer).  Lane s takes split s's (maximum, sum) so that the weights of up to 64 splits are known after one round of loads;
+// the first eight splits' partial outputs are asked for together with them (a part of a split without visible keys may hold anything:
+// it is read and then dropped), the others eight at a time.  A layer of 64 decoded tokens, 14 heads of 64, two splits: 4.6 us with four
+// features a lane whatever the head size and shuffles through LDS, 3.4 so.
+template <int R>
 __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml,
                                                               const int32_t* __restrict__ q_start,
@@ -1651,53 +1654,51 @@ __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __res
         first_part = dealt[2 * seq] * nq + row % nq;
         between = nq;
     }
-    // the first eight splits' parts are asked for together with their weights' inputs, not behind them (a part of a
-    // split without visible keys may hold anything: it is read and then dropped)
-    float first[8][4];
+    const float* from = part_o + static_cast<size_t>(first_part) * hd;
+    const size_t step = static_cast<size_t>(between) * hd;
+    int at[R];                                           // (a lane past the head's last feature reads that one again)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const size_t pr = static_cast<size_t>(min(i, n_splits - 1)) * between + first_part;
+    for (int r = 0; r < R; ++r) at[r] = min(lane + r * kWave, hd - 1);
+    float v[8][R];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int d = lane + r * kWave;
-            first[i][r] = d < hd ? part_o[pr * hd + d] : 0.f;
-        }
-    }
-    float m = -INFINITY, l = 0.f;
-    if (lane < n_splits) {
-        const size_t pr = static_cast<size_t>(lane) * between + first_part;
-        m = part_ml[pr * 2];
-        l = part_ml[pr * 2 + 1];
-    }
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[i][r] = from[min(i, n_splits - 1) * step + at[r]];
+    const size_t mine = (static_cast<size_t>(min(lane, n_splits - 1)) * between + first_part) * 2;
+    const float m_read = part_ml[mine], l = part_ml[mine + 1];
+    const float m = lane < n_splits ? m_read : -INFINITY;
     const float m_max = wave_max(m);
     const float wgt = m == -INFINITY ? 0.f : __expf(m - m_max);    // a split without visible keys weighs nothing
-    const float inv = 1.0f / wave_sum(wgt * l);
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < n_splits; s0 += 8) {
-        float v[8][4], w8[8];
+    const float inv = 1.0f / wave_sum(m == -INFINITY ? 0.f : wgt * l);
+    float acc[R] = {};
+    auto add = [&](int s0) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int s = s0 + i;
-            w8[i] = __shfl(wgt, s < n_splits ? s : 0, kWave);
-            if (s >= n_splits) w8[i] = 0.f;
-            const size_t pr = static_cast<size_t>(s < n_splits ? s : 0) * between + first_part;
+            const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wgt), s0 + i));
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int d = lane + r * kWave;
-                if (s0 == 0) v[i][r] = w8[i] != 0.f ? first[i][r] : 0.f;
-                else v[i][r] = (d < hd && w8[i] != 0.f) ? part_o[pr * hd + d] : 0.f;
-            }
+            for (int r = 0; r < R; ++r) acc[r] += w * (w != 0.f ? v[i][r] : 0.f);
         }
+    };
+    add(0);
+    for (int s0 = 8; s0 < n_splits; s0 += 8) {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] += w8[i] * v[i][r];
+            for (int r = 0; r < R; ++r) v[i][r] = from[min(s0 + i, n_splits - 1) * step + at[r]];
+        add(s0);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int d = lane + r * kWave;
-        if (d < hd) out[static_cast<size_t>(out_row) * hd + d] = from_float<bf16_t>(acc[r] * inv);
-    }
+    for (int r = 0; r < R; ++r)
+        if (lane + r * kWave < hd) out[static_cast<size_t>(out_row) * hd + lane + r * kWave] = from_float<bf16_t>(acc[r] * inv);
+}
+static void launch_reduce(const float* part_o, const float* part_ml, const int32_t* q_start, const int32_t* q_len, const int32_t* dealt, int n_rows,
+                          int hd, int n_splits, int nq, void* out, hipStream_t s) {
+    auto launch = [&](auto kernel) {
+        kernel<<<n_rows, 64, 0, s>>>(part_o, part_ml, q_start, q_len, dealt, n_rows, hd, n_splits, nq, static_cast<bf16_t*>(out));
+    };
+    if (hd <= 64) launch(attention_reduce_kernel<1>);
+    else if (hd <= 128) launch(attention_reduce_kernel<2>);
+    else launch(attention_reduce_kernel<4>);
 }
 
 template <int HD, int QT>
@@ -1714,8 +1715,7 @@ static int launch_mfma(const void* qkv, void* out, float* part_o, float* part_ml
         q_len, kv_len, n_seqs, n_tokens, nq, nkv, page_size, scale, window, n_splits);
     EGPT_CHECK_LAUNCH();
     if (n_splits > 1 && combine) {
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, nullptr, nullptr, nullptr, n_tokens * nq, HD, n_splits, 1,
-                                                             static_cast<bf16_t*>(out));
+        launch_reduce(part_o, part_ml, nullptr, nullptr, nullptr, n_tokens * nq, HD, n_splits, 1, out, s);
         EGPT_CHECK_LAUNCH();
     }
     return EGPT_OK;
@@ -1766,12 +1766,10 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
     if (e != EGPT_OK) return e;
     EGPT_CHECK_LAUNCH();
     if (ranges) {
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, q_start, q_len, ranges + slots * kRangeInts, n_tokens * nq, HD, 1, nq,
-                                                             static_cast<bf16_t*>(out));
+        launch_reduce(part_o, part_ml, q_start, q_len, ranges + slots * kRangeInts, n_tokens * nq, HD, 1, nq, out, s);
         EGPT_CHECK_LAUNCH();
     } else if (n_splits > 1 && combine) {
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, q_len ? q_start : nullptr, q_len, nullptr, n_tokens * nq, HD,
-                                                             n_splits, nq, static_cast<bf16_t*>(out));
+        launch_reduce(part_o, part_ml, q_len ? q_start : nullptr, q_len, nullptr, n_tokens * nq, HD, n_splits, nq, out, s);
         EGPT_CHECK_LAUNCH();
     }
     return EGPT_OK;
@@ -1831,8 +1829,7 @@ static void launch_rows32(const void* qkv, void* out, const void* k_cache, const
     // (the rows of requests that were left out have no parts: what is combined for them is written over by the
     // kernel that takes them, which runs behind this one)
     if (n_splits > 1)
-        attention_reduce_kernel<<<n_tokens * nq, 64, 0, s>>>(part_o, part_ml, nullptr, nullptr, nullptr, n_tokens * nq, HD, n_splits, 1,
-                                                             static_cast<bf16_t*>(out));
+        launch_reduce(part_o, part_ml, nullptr, nullptr, nullptr, n_tokens * nq, HD, n_splits, 1, out, s);
 }
 
 template <int HD, int RB, int KS>
@@ -1848,8 +1845,7 @@ static int launch_mixed(const void* qkv, void* out, const void* k_cache, const v
         block_table, table_width, q_start, q_len, kv_len, n_seqs, nq, nkv, page_size, page_shift, scale, window, late, static_cast<int>(blocks),
         magic_of(page_size / 16), ranges, slots, range_o, range_ml);
     EGPT_CHECK_LAUNCH();
-    attention_reduce_kernel<<<n_seqs * nq, 64, 0, s>>>(range_o, range_ml, q_start, q_len, ranges + slots * kRangeInts, n_seqs * nq, HD, 1, nq,
-                                                       static_cast<bf16_t*>(out));
+    launch_reduce(range_o, range_ml, q_start, q_len, ranges + slots * kRangeInts, n_seqs * nq, HD, 1, nq, out, s);
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
@@ -2133,8 +2129,7 @@ extern "C" int egpt_attention_combine(const float* part_o, const float* part_ml,
     if (!part_o || !part_ml || !out || n_rows < 0 || hd <= 0 || n_splits < 1) return EGPT_BAD_ARGUMENT;
     if (n_splits > 64 || hd > 256) return EGPT_UNSUPPORTED_SIZE;
     if (n_rows == 0) return EGPT_OK;
-    attention_reduce_kernel<<<n_rows, 64, 0, static_cast<hipStream_t>(stream)>>>(part_o, part_ml, nullptr, nullptr, nullptr, n_rows, hd,
-                                                                               n_splits, 1, static_cast<bf16_t*>(out));
+    launch_reduce(part_o, part_ml, nullptr, nullptr, nullptr, n_rows, hd, n_splits, 1, out, static_cast<hipStream_t>(stream));
     EGPT_CHECK_LAUNCH();
     return EGPT_OK;
 }
