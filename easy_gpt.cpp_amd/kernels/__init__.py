@@ -210,6 +210,16 @@ class KernelBackend:
         a residual stream in fixed point that the backend can add the product into, that stream."""
         raise NotImplementedError
 
+    writes_sums_in_place = False     # whether expert_mixture takes `out`
+
+    def product_room(self, x, w):
+        """`product` unrounded as float32 [1 + splits, m, n]: the sums behind a first one that the caller writes."""
+        import torch
+
+        s = self.product(x, w, unrounded=True)
+        s = s if s.dim() == 3 else s.float()[None]
+        return torch.cat([torch.empty_like(s[:1]), s], dim=0)
+
     def product_parts(self, x, w):
         """product(x, w, unrounded=True) for a consumer that adds up a few partial sums at no more than their bytes' cost also where
         the rows are many (`qkv_rope_store` with a whole rotation)."""

@@ -800,7 +800,14 @@ class HipKernels(KernelBackend):
         self._run("egpt_attention_combine", part_o.data_ptr(), part_ml.data_ptr(), out.data_ptr(), t * nq, hd,
                   int(a_splits), self._stream())
 
-    def product(self, x, w, unrounded=False, residual=None):
+    writes_sums_in_place = True
+
+    def product_room(self, x, w):
+        """`product` unrounded, with room for one more float32 sum of the same size in front: [1 + splits, m, n], the first for the caller
+        to write."""
+        return self.product(x, w, unrounded=True, room=1)
+
+    def product(self, x, w, unrounded=False, residual=None, room=0):
         """x w^T for a consumer that takes partial sums: returns act [m, n], or float32 [splits, m, n] whose sum
         over splits is the product (few rows in bfloat16: the k range is split over workgroups).  unrounded=True
         asks for float32 also from the many-row library product (as [1, m, n]): for consumers that go on computing
@@ -809,6 +816,8 @@ class HipKernels(KernelBackend):
         in fixed point [m, n], a product of few rows is added into it instead and the stream is returned."""
         m, k = x.shape
         n = w.shape[0]
+        if room and not (x.dtype == _BF16 and m > 64 and k % 8 == 0):
+            return super().product_room(x, w)
         if 16 < m <= 64 and self._rows_fit(x, w, k):
             # A few dozen rows: the kernel for many, whose workgroups keep more of the weights on their way than the weight-streaming one and
             # split the k range, which the library does not.  us, weights from memory, at 17 / 32 / 64 rows, with the norm that reads the
@@ -845,17 +854,18 @@ class HipKernels(KernelBackend):
             form = 1 if unrounded or self._sums_kept(m, n, k) else 0
             shape, s = self._rows_plan(m, n, k, 1 if unrounded else 10, form)
             kind = 1 if form or s > 1 else 0
-            out = torch.empty((s, m, n) if kind else (m, n), dtype=_F32 if kind else _BF16, device=x.device)
-            self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, s, kind, 0, shape, self._stream())
+            out = torch.empty((room + s, m, n) if kind else (m, n), dtype=_F32 if kind else _BF16, device=x.device)
+            self._run("egpt_gemm_rows", x.data_ptr(), w.data_ptr(), out[room if kind else 0].data_ptr() if room else out.data_ptr(), m, n, k, s, kind, 0,
+                      shape, self._stream())
             return out
         if unrounded and x.dtype == _BF16 and m > 0 and k % 8 == 0:
             # many rows: the library's product (the reference uses cuBLAS for every linear layer), written out in
             # float32; it goes on as a single "partial sum" [1, m, n]
             self._need(x, "x")
             self._need(w, "w", x.dtype, (n, k))
-            out = torch.empty((1, m, n), dtype=_F32, device=x.device)
+            out = torch.empty((room + 1, m, n), dtype=_F32, device=x.device)
             with _FirstChoice():
-                torch.mm(x, w.t(), out_dtype=_F32, out=out[0])
+                torch.mm(x, w.t(), out_dtype=_F32, out=out[room])
             return out
         if x.dtype == _F32 and m > 0 and k % 4 == 0:
             self._need(x, "x")
@@ -2011,7 +2021,7 @@ class HipKernels(KernelBackend):
         return 16 if per_expert <= 24 else (32 if per_expert <= 96 else 64)
 
     def expert_mixture(self, x, router, router_bias, w_gate_up, w_down, top, gated=True, score_all=False, correction=None,
-                       weight_scale=1.0, identities=0, groups=1, keep_groups=1, normalized=True, residual=None):
+                       weight_scale=1.0, identities=0, groups=1, keep_groups=1, normalized=True, residual=None, out=None):
         """float32 [T, H]: for every token the `top` experts with the largest float32 router logits (x router^T + bias),
         weighted by the softmax over those logits; an expert is down(silu(gate x) * (up x)).  w_gate_up [E, 2 ff, H]
         (an expert's gate rows, then its up rows), w_down [E, H, ff].  gated False: an expert is down(relu(up x)^2) and
@@ -2062,7 +2072,10 @@ class HipKernels(KernelBackend):
         counts = torch.empty((experts,), dtype=_I32, device=dev)
         act = torch.empty((n_rows, ff), dtype=x.dtype, device=dev)
         y = torch.empty((n_rows, hidden), dtype=_F32, device=dev)
-        out = None if residual is not None else torch.empty((t, hidden), dtype=_F32, device=dev)
+        if out is not None:
+            self._need(out, "out", _F32, (t, hidden))
+        elif residual is None:
+            out = torch.empty((t, hidden), dtype=_F32, device=dev)
         st = self._stream()
         self._run("egpt_moe_route", x.data_ptr(), router.data_ptr(), self._ptr(router_bias), chosen.data_ptr(),
                   weight.data_ptr(), t, hidden, outputs, top, int(bool(score_all)), self._ptr(correction), float(weight_scale),

@@ -109,9 +109,14 @@ class ExpertMixture(FeedForward):
             options.update(identities=self.identities, groups=self.groups, keep_groups=self.keep_groups, normalized=self.normalized)
         if residual is not None:
             options.update(residual=residual)
+        room = self.shared.with_room(x, ctx) if hasattr(self.shared, "with_room") else None
+        if room is not None:                          # the experts' sum goes in front of the shared branch's
+            options.update(out=room[0])
         out = kernels.backend().expert_mixture(x, self.w_router, self.b_router, self.w_gate_up, self.w_down, self.top, **options)
         if residual is not None:
             return None
+        if room is not None:
+            return room
         out = out[None]
         if self.shared is None:
             return out

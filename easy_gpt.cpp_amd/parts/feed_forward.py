@@ -92,6 +92,19 @@ class SwiGLU(FeedForward):
         return down(act)
 
 
+    def with_room(self, x, ctx=None):
+        """What `forward` returns for many tokens as float32 [1 + splits, T, H], the first sum for the caller to write: another branch's
+        output stands beside this one's without a copy of either.  None where the backend has no use for it."""
+        k = kernels.backend()
+        if not self.unrounded or not k.writes_sums_in_place or x.shape[0] <= 64:
+            return None
+        act = k.gate_up_rows(x, self.w_gate_up, activation=self.activation)
+        if act is None:
+            act = torch.empty((x.shape[0], self.intermediate_size), dtype=x.dtype, device=x.device)
+            k.swiglu(k.product(x, self.w_gate_up), act, activation=self.activation)
+        return k.product_room(act, self.w_down)
+
+
 class ActivatedFeedForward(FeedForward):
     """A feed-forward without a gate product: y = W_down act(W_up x), no biases.
 
