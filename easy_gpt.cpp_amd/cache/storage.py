@@ -49,5 +49,5 @@ class StateStorage:
         }
 
     def reset(self, slot: int) -> None:
-        for t in self.data.values():
-            t[slot].zero_()
+        if self.data:                        # (one launch for all layers' records, not one each)
+            torch._foreach_zero_([t[slot] for t in self.data.values()])

@@ -123,7 +123,6 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
     constexpr int BC = OUT == kRowsGated || OUT == kRowsRotated ? BN / 2 : BN;         // columns of the result (or pairs) in a tile
     const int mt = GROUPED ? groups.tiles[0] : (m + BM - 1) / BM, nt = (n + BC - 1) / BC;
     const int tiles = mt * nt, items = tiles * splits;
-    const int strips = (mt + kStrip - 1) / kStrip, per_strip = (mt + strips - 1) / strips;
     if (GROUPED && static_cast<int>(blockIdx.x) >= items) return;      // (the grid is sized for the most tiles that the rows can make)
     const int total = k / kRowsStep;
     const size_t row_bytes = static_cast<size_t>(k) * 2;
@@ -152,11 +151,18 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN / (WM * WN) > 8192 ? 1 : 2) v
             it.split = 0;
             from += static_cast<size_t>(entry[0]) * (OUT == kRowsGated ? 2 * n : n) * k;
         } else {
-            it.split = item / tiles;
-            const int tile = item - it.split * tiles, strip = tile / (per_strip * nt), top = strip * per_strip;
-            const int high = min(per_strip, mt - top), at = tile - top * nt, column = at / high;
-            it.m0 = (top + at - column * high) * BM;
-            it.n0 = column * BC;
+            it.split = splits == 1 ? 0 : item / tiles;
+            const int tile = item - it.split * tiles;
+            if (mt == 1) {                                 // (a division is 25 instructions, in front of everything)
+                it.m0 = 0;
+                it.n0 = tile * BC;
+            } else {
+                const int strips = (mt + kStrip - 1) / kStrip, per_strip = (mt + strips - 1) / strips;
+                const int strip = tile / (per_strip * nt), top = strip * per_strip;
+                const int high = min(per_strip, mt - top), at = tile - top * nt, column = at / high;
+                it.m0 = (top + at - column * high) * BM;
+                it.n0 = column * BC;
+            }
             it.rows = min(m - it.m0, BM);
         }
         it.begin = it.split * steps_per_split;
