@@ -1199,14 +1199,6 @@ struct DecodeSizes {
     int n_waves;                                                 // of a workgroup (blockDim would be a load by itself)
 };
 
-// floor(x / d) for x and d < 2^27, as a product: no more than one too many, which is put right (a division is 30 instructions, and
-// a kernel like this one is as long as its chain of them).
-static unsigned magic_of(int d) { return static_cast<unsigned>((1ULL << 32) / (2 * static_cast<unsigned>(d)) + 1); }
-__device__ __forceinline__ int divided(int x, int d, unsigned magic) {
-    const int q = static_cast<int>(__umulhi(2 * static_cast<unsigned>(x), magic));
-    return q - (q * d > x ? 1 : 0);
-}
-
 // The order of the loads is what this kernel's time is: everything that depends on no other load goes out at once (the
 // context's length, the product's partial sums with what is computed from them), then the page numbers, then the first round of keys
 // and values, and only then are the queries made.  Loads are bounded by their buffer's size instead of branches, so that none of

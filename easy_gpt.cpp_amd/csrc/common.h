@@ -140,6 +140,50 @@ __device__ __forceinline__ void read_values(const ProductView<T>& p, const size_
     }
 }
 
+// Four neighbouring values: kernels whose time is their instructions read and write a row by quads, with one index and one test for
+// four values.  A quad begins on a multiple of four values of an operand that itself begins on 16 bytes (`quads`, on the host).
+__device__ __forceinline__ void read_quad(const float* p, float (&v)[4]) {
+    const float4 a = *reinterpret_cast<const float4*>(p);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+__device__ __forceinline__ void read_quad(const bf16_t* p, float (&v)[4]) {
+    const uint2 a = *reinterpret_cast<const uint2*>(p);
+    v[0] = __uint_as_float(a.x << 16); v[1] = __uint_as_float(a.x & 0xffff0000u);
+    v[2] = __uint_as_float(a.y << 16); v[3] = __uint_as_float(a.y & 0xffff0000u);
+}
+__device__ __forceinline__ void write_quad(float* p, const float (&v)[4]) { *reinterpret_cast<float4*>(p) = float4{v[0], v[1], v[2], v[3]}; }
+__device__ __forceinline__ void write_quad(bf16_t* p, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
+}
+// of a product, partial sums added in the order of at(), the loads of three of them on their way together
+template <typename T>
+__device__ __forceinline__ void read_quad(const ProductView<T>& p, size_t at, float (&v)[4]) {
+    if (p.n_splits == 0) return read_quad(p.whole + at, v);
+    read_quad(p.partial + at, v);
+    for (int s0 = 1; s0 < p.n_splits; s0 += 3) {
+        float t[3][4];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) read_quad(p.partial + min(s0 + u, p.n_splits - 1) * p.split_stride + at, t[u]);
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = s0 + u < p.n_splits ? v[e] + t[u][e] : v[e];
+    }
+}
+// Whether all of these begin on 16 bytes (null does).
+template <typename... P>
+static inline bool quads(const P*... p) { return ((reinterpret_cast<uintptr_t>(p) | ...) & 15) == 0; }
+// Threads for a row of so many quads, a quad each.
+static inline int quad_threads(int values) { return (values / 4 + kWave - 1) / kWave * kWave; }
+
+// floor(x / d) for x and d < 2^27, as a product: no more than one too many, which is put right (a division is 30 instructions, and
+// a kernel like this one is as long as its chain of them).
+static unsigned magic_of(int d) { return static_cast<unsigned>((1ULL << 32) / (2 * static_cast<unsigned>(d)) + 1); }
+__device__ __forceinline__ int divided(int x, int d, unsigned magic) {
+    const int q = static_cast<int>(__umulhi(2 * static_cast<unsigned>(x), magic));
+    return q - (q * d > x ? 1 : 0);
+}
+
 // A product whose x operand was (h * norm weight) still lacks each row's factor 1 / sqrt(sum_s ss[s][row] / hidden + eps):
 // the sums of squares arrive beside it (null: the product is complete).
 struct RowFactor {
@@ -247,6 +291,22 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     float total = 0.f;
     for (int w = 0; w < n_waves; ++w) total += scratch[w];
     return total;
+}
+// The same of N values at once by `waves` wavefronts, 16 at most, with scratch of its own that nothing else uses: one wait.
+template <int N>
+__device__ __forceinline__ void block_totals(float (&v)[N], float (*scratch)[16], int waves) {
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        v[i] = wave_sum(v[i]);
+        if (lane == 0) scratch[i][wave] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float part = scratch[i][lane % 16];
+        v[i] = fold_row(lane % 16 < waves ? part : 0.f, AddOf());
+    }
 }
 __device__ __forceinline__ float block_max(float v, float* scratch) {
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;

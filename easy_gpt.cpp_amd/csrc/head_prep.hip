@@ -6,6 +6,8 @@
 //
 // A product arrives as one tensor of the activation type or as float32 partial sums (ProductView in common.h).
 // Keys lie in pages [page][kv head][offset][key size], values in pages [page][kv head][value size][offset].
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -303,6 +305,22 @@ __global__ __launch_bounds__(256) void sigmoid_gate_kernel(const T* __restrict__
 }
 
 
+// The same where x lies [T][N] and quads fit, a row of workgroups per token: 2,535 tokens of 896 7.2 -> 4.8 us (a value found its token by
+// a division of 64 bits).
+template <typename T>
+__global__ __launch_bounds__(256) void sigmoid_gate_quads_kernel(const T* __restrict__ x, T* __restrict__ out, int n, int gate_width, int gate_off,
+                                                                 ProductView<T> g, RowFactor factor) {
+    const int t = blockIdx.x, j = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (j >= n) return;
+    float v[4], gate[4];
+    read_quad(x + static_cast<size_t>(t) * n + j, v);
+    read_quad(g, static_cast<size_t>(t) * gate_width + gate_off + j, gate);
+    const float f = factor.of(t);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * (1.0f / (1.0f + expf(-(gate[e] * f))));
+    write_quad(out + static_cast<size_t>(t) * n + j, v);
+}
+
 // One workgroup per token of a product row [nq heads of dk | nkv heads of dk | nkv heads of dv | anything else]: the
 // bias [nq * dk + nkv * dk + nkv * dv] is added, the queries are RMS-normed over all heads at once (one statistic
 // over nq * dk values, a weight per value), and so are the keys (over nkv * dk); the queries are then multiplied by
@@ -395,6 +413,63 @@ __global__ __launch_bounds__(256) void whole_norm_store_kernel(
     }
 }
 
+// The same with a quad of the row in each thread's registers: the three parts, the row and the heads multiples of four values, up to 4,096
+// of them.  2,535 rows of 896 + 128 + 128 19.0 -> 10.6 us: single values found their head and page by two divisions each.
+constexpr int kQuadsMost = 4096;
+template <typename T>
+__global__ __launch_bounds__(kQuadsMost / 4) void whole_norm_store_quads_kernel(
+    const T* __restrict__ bias, T* __restrict__ q_out, const T* __restrict__ q_weight, const T* __restrict__ k_weight,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, T* __restrict__ k_cache, T* __restrict__ v_cache, int row_width,
+    int qw, int kw, int vw, int nkv, int dk, int dv, int page_size, int every, float coef, float eps, ProductView<T> proj) {
+    __shared__ float sums[2][16];
+    const int t = blockIdx.x, j = threadIdx.x * 4, all = qw + kw + vw;
+    const bool here = j < all, is_q = j < qw, is_k = j >= qw && j < qw + kw;
+    float v[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {1.f, 1.f, 1.f, 1.f};
+    int slot = 0;
+    if (here) {
+        read_quad(proj, static_cast<size_t>(t) * row_width + j, v);
+        if (bias) {
+            read_quad(bias + j, w);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += w[e];
+        }
+        const T* of = is_q ? q_weight : is_k ? k_weight : nullptr;
+        if (of) read_quad(of + (is_q ? j : j - qw), w);
+        if (slots) slot = slots[t];
+    }
+    float ss[2] = {0.f, 0.f};
+    const float squares = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
+    ss[0] = is_q ? squares : 0.f;
+    ss[1] = is_k ? squares : 0.f;
+    block_totals(ss, sums, (all / 4 + kWave - 1) / kWave);
+    if (!here) return;
+    float factor = 1.f;
+    if (is_q) {
+        if (q_weight) factor = inv_rms(ss[0], 1.0f / static_cast<float>(qw), eps);
+        if (every > 0) factor *= 1.0f + coef * logf(static_cast<float>((positions[t] + 1) / every + 1));
+    } else if (is_k && k_weight) {
+        factor = inv_rms(ss[1], 1.0f / static_cast<float>(kw), eps);
+    }
+    const bool weighed = is_q ? q_weight != nullptr : is_k && k_weight != nullptr;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] *= factor;
+        if (weighed) v[e] *= w[e];
+    }
+    if (is_q) return write_quad(q_out + static_cast<size_t>(t) * qw + j, v);
+    if (slots == nullptr) return;
+    const long page = slot / page_size, off = slot % page_size;
+    if (is_k) {
+        const int jj = j - qw, head = jj / dk;
+        write_quad(k_cache + ((page * nkv + head) * page_size + off) * dk + jj - head * dk, v);
+    } else {
+        const int jj = j - qw - kw, head = jj / dv;
+        T* to = v_cache + ((page * nkv + head) * dv + jj - head * dv) * page_size + off;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[static_cast<long>(e) * page_size] = from_float<T>(v[e]);
+    }
+}
+
 // out[t][h * dv + d] = x[t][h * dv + d] / rms(x[t][h * dv ..]) * weight[d] * act(g[t][gate_off + h * dv + d]): the
 // RMS norm of every head's output with a weight that the heads share (null: none), and a gate from columns of a product row (no
 // gate: the normed heads as they are).  x is float32 (one tensor, or partial sums that are added here) or, with xa
@@ -452,6 +527,39 @@ __global__ __launch_bounds__(kWave) void head_norm_gate_kernel(ProductView<float
         }
         out[(static_cast<size_t>(t) * heads + h) * dv + d] = from_float<T>(y);
     }
+}
+
+// The same for heads of 64, 128 or 256 values: 16, 32 or 64 lanes a head, a quad each, a workgroup of four wavefronts for the next heads
+// of all tokens.  2,535 rows of seven heads of 128 13.1 -> 10.5 us: one wavefront a workgroup is bound by how fast they are handed out.
+template <typename T, int LANES>
+__global__ __launch_bounds__(256) void head_norm_gate_quads_kernel(const T* __restrict__ weight, T* __restrict__ out, int n_items, int heads,
+                                                                   unsigned heads_magic, int x_width, int gate_width, int gate_off, int gate_act,
+                                                                   float eps, ProductView<float> x, ProductView<T> xa, ProductView<T> g) {
+    constexpr int dv = LANES * 4;
+    const int item = blockIdx.x * (256 / LANES) + threadIdx.x / LANES, d = threadIdx.x % LANES * 4;
+    if (item >= n_items) return;                          // (whole heads: the lanes of one go together)
+    const int t = divided(item, heads, heads_magic), h = item - t * heads;
+    const size_t xr = static_cast<size_t>(t) * x_width + h * dv + d;
+    float v[4], gate[4], w[4];
+    if (xa.present()) read_quad(xa, xr, v);
+    else read_quad(x, xr, v);
+    const bool gated = g.present();
+    if (gated) read_quad(g, static_cast<size_t>(t) * gate_width + gate_off + h * dv + d, gate);
+    if (weight) read_quad(weight + d, w);
+    float ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
+    ss = fold_row(ss, AddOf());
+    if (LANES >= 32) ss = fold_16_apart(ss, AddOf());
+    if (LANES == 64) ss = fold_32_apart(ss, AddOf());
+    const float inv = inv_rms(ss, 1.0f / static_cast<float>(dv), eps);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = v[e] * inv * (weight ? w[e] : 1.0f);
+        if (gated) {
+            const float sig = 1.0f / (1.0f + expf(-gate[e]));
+            v[e] *= gate_act == 0 ? gate[e] * sig : (gate_act == 1 ? sig : gate[e]);
+        }
+    }
+    write_quad(out + static_cast<size_t>(item) * dv + d, v);
 }
 
 // The same for heads of many values: a workgroup of four wavefronts per (token, head), the statistics through LDS.
@@ -636,6 +744,17 @@ extern "C" int egpt_sigmoid_gate(const void* x, int heads, const void* gate, int
     const size_t total = static_cast<size_t>(n_tokens) * n;
     const size_t stride = static_cast<size_t>(n_tokens) * gate_width;
     const unsigned blocks = static_cast<unsigned>((total + 255) / 256);
+    if (heads == 0 && n % 4 == 0 && gate_width % 4 == 0 && gate_off % 4 == 0 && n <= 65535 * 1024 && quads(x, gate, out)) {
+        const dim3 grid(n_tokens, (n / 4 + 255) / 256);
+        if (dtype == 0)
+            sigmoid_gate_quads_kernel<float><<<grid, 256, 0, s>>>(static_cast<const float*>(x), static_cast<float*>(out), n, gate_width, gate_off,
+                                                                  view_of<float>(gate, gate_splits, stride), factor);
+        else
+            sigmoid_gate_quads_kernel<bf16_t><<<grid, 256, 0, s>>>(static_cast<const bf16_t*>(x), static_cast<bf16_t*>(out), n, gate_width, gate_off,
+                                                                   view_of<bf16_t>(gate, gate_splits, stride), factor);
+        EGPT_CHECK_LAUNCH();
+        return EGPT_OK;
+    }
     if (dtype == 0)
         sigmoid_gate_kernel<float><<<blocks, 256, 0, s>>>(static_cast<const float*>(x), heads,
                                                           view_of<float>(gate, gate_splits, stride), factor, gate_width, gate_off,
@@ -662,6 +781,20 @@ extern "C" int egpt_whole_norm_store(const void* proj, int n_splits, int row_wid
     if (n_tokens == 0) return EGPT_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t stride = static_cast<size_t>(n_tokens) * row_width;
+    const long all = static_cast<long>(nq + nkv) * dk + static_cast<long>(nkv) * dv;
+    if (dk % 4 == 0 && dv % 4 == 0 && row_width % 4 == 0 && all <= kQuadsMost && quads(proj, bias, q_out, q_weight, k_weight, k_cache)) {
+        auto launch = [&](auto kernel, auto* to) {
+            using T = std::remove_pointer_t<decltype(to)>;
+            kernel<<<n_tokens, quad_threads(static_cast<int>(all)), 0, s>>>(
+                static_cast<const T*>(bias), to, static_cast<const T*>(q_weight), static_cast<const T*>(k_weight), positions, slots,
+                static_cast<T*>(k_cache), static_cast<T*>(v_cache), row_width, nq * dk, nkv * dk, nkv * dv, nkv, dk, dv, page_size, every, coef, eps,
+                view_of<T>(proj, n_splits, stride));
+        };
+        if (dtype == 0) launch(whole_norm_store_quads_kernel<float>, static_cast<float*>(q_out));
+        else launch(whole_norm_store_quads_kernel<bf16_t>, static_cast<bf16_t*>(q_out));
+        EGPT_CHECK_LAUNCH();
+        return EGPT_OK;
+    }
     if (dtype == 0)
         whole_norm_store_kernel<float><<<n_tokens, 256, 0, s>>>(
             view_of<float>(proj, n_splits, stride), row_width, static_cast<const float*>(bias), static_cast<float*>(q_out),
@@ -695,6 +828,27 @@ extern "C" int egpt_head_norm_gate(const void* x, int x_splits, int x_is_act, in
     xv.partial = x_splits > 0 ? static_cast<const float*>(x) : nullptr;
     xv.n_splits = x_splits;
     xv.split_stride = static_cast<size_t>(n_tokens) * x_width;
+    const long items = static_cast<long>(n_tokens) * heads;
+    if ((dv == 64 || dv == 128 || dv == 256) && x_width % 4 == 0 && (!gate || (gate_width % 4 == 0 && gate_off % 4 == 0)) && items < (1 << 27) &&
+        quads(x, weight, gate, out)) {
+        auto launch = [&](auto kernel, auto* to, int lanes) {
+            using T = std::remove_pointer_t<decltype(to)>;
+            const int per = 256 / lanes;
+            kernel<<<static_cast<unsigned>((items + per - 1) / per), 256, 0, s>>>(
+                static_cast<const T*>(weight), to, static_cast<int>(items), heads, magic_of(heads), x_width, gate_width, gate_off, gate_act, eps, xv,
+                view_of<T>(x_is_act ? x : nullptr, 0, 0), view_of<T>(gate, gate_splits, stride));
+        };
+        auto pick = [&](auto* to) {
+            using T = std::remove_pointer_t<decltype(to)>;
+            if (dv == 64) launch(head_norm_gate_quads_kernel<T, 16>, to, 16);
+            else if (dv == 128) launch(head_norm_gate_quads_kernel<T, 32>, to, 32);
+            else launch(head_norm_gate_quads_kernel<T, 64>, to, 64);
+        };
+        if (dtype == 0) pick(static_cast<float*>(out));
+        else pick(static_cast<bf16_t*>(out));
+        EGPT_CHECK_LAUNCH();
+        return EGPT_OK;
+    }
     if (dv > 256) {                                       // heads of many values: four wavefronts a head
         if (dtype == 0)
             head_norm_gate_wide_kernel<float><<<grid, 256, 0, s>>>(xv, view_of<float>(x_is_act ? x : nullptr, 0, 0), x_width,

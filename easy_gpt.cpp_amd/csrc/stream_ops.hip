@@ -3,6 +3,8 @@
 // stream, the mean of two RMS-normed branch outputs, parallel residual streams that a sublayer reads as a weighted sum and
 // rewrites as a mixture, and the tanh cap on logits.  Statistics and sums are float32;
 // values are rounded once, when they are written in the activation type.
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -104,6 +106,50 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(float* __restrict__ 
     }
 }
 
+// The same with a quad of the row in each thread's registers (hidden % 4 == 0, up to 4,096): 2,535 rows of 896 behind two float32 arrays
+// 10.9 -> 8.0 us; single values through LDS took three times the instructions, and those are what it costs.
+constexpr int kQuadsMost = 4096;
+template <typename T>
+__global__ __launch_bounds__(kQuadsMost / 4) void add_layernorm_quads_kernel(float* __restrict__ h, const T* __restrict__ weight,
+                                                                             const T* __restrict__ bias, const int32_t* __restrict__ rows,
+                                                                             T* __restrict__ out, int hidden, float eps,
+                                                                             ProductView<T> delta) {
+    __shared__ float sums[1][16], devs[1][16];
+    const int waves = (hidden / 4 + kWave - 1) / kWave, j = threadIdx.x * 4;
+    const int r = blockIdx.x;
+    const size_t src = rows ? rows[r] : r, at = src * hidden + j;
+    const bool here = j < hidden;
+    float v[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
+    if (here) {
+        read_quad(h + at, v);
+        read_quad(weight + j, w);
+        if (bias) read_quad(bias + j, b);
+        if (delta.present()) {
+            float d[4];
+            read_quad(delta, at, d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += d[e];
+            if (!rows) write_quad(h + at, v);
+        }
+    }
+    float total[1] = {(v[0] + v[1]) + (v[2] + v[3])};
+    block_totals(total, sums, waves);
+    const float mean = total[0] / static_cast<float>(hidden);
+    float dev[1] = {0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] -= mean;
+        dev[0] = fmaf(v[e], v[e], dev[0]);
+    }
+    if (!here) dev[0] = 0.f;
+    block_totals(dev, devs, waves);
+    const float inv = 1.0f / sqrtf(dev[0] / static_cast<float>(hidden) + eps);
+    if (!here) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = scaled_then_added(v[e] * inv, w[e], b[e], bias != nullptr);
+    write_quad(out + static_cast<size_t>(r) * hidden + j, v);
+}
+
 // out[t, :] = factor_a * a[t, :] / rms(a[t, :]) * wa + factor_b * b[t, :] / rms(b[t, :]) * wb, float32: what two branches
 // that are normed before they are joined leave for the residual stream.  Without weights (wa null) the branches are not
 // normed: out = factor_a * a + factor_b * b.
@@ -159,6 +205,56 @@ __global__ __launch_bounds__(256) void normed_pair_mean_kernel(ProductView<T> a,
                                                  : factor_a * (a_s[j] * inv_a * to_float(u[i])) + factor_b * (b_s[j] * inv_b * to_float(w[i]));
         }
     }
+}
+
+// The same with a quad of either row in each thread's registers (hidden % 4 == 0, up to 4,096): 2,535 rows of 896 11.5 -> 8.0 us.
+template <typename T>
+__global__ __launch_bounds__(kQuadsMost / 4) void normed_pair_mean_quads_kernel(const T* __restrict__ bias_a, const T* __restrict__ bias_b,
+                                                                                const T* __restrict__ wa, const T* __restrict__ wb,
+                                                                                float* __restrict__ out, int hidden, float eps, float factor_a,
+                                                                                float factor_b, ProductView<T> a, ProductView<T> b) {
+    __shared__ float sums[2][16];
+    const int j = threadIdx.x * 4;
+    const size_t at = static_cast<size_t>(blockIdx.x) * hidden + j;
+    const bool here = j < hidden;
+    float x[4] = {0.f, 0.f, 0.f, 0.f}, y[4] = {0.f, 0.f, 0.f, 0.f}, u[4], w[4];
+    if (here) {
+        read_quad(a, at, x);
+        read_quad(b, at, y);
+        if (bias_a) {
+            read_quad(bias_a + j, u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] += u[e];
+        }
+        if (bias_b) {
+            read_quad(bias_b + j, w);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] += w[e];
+        }
+    }
+    float z[4];
+    if (wa == nullptr) {
+        if (!here) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[e] = factor_a * x[e] + factor_b * y[e];
+    } else {
+        float ss[2] = {0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            ss[0] = fmaf(x[e], x[e], ss[0]);
+            ss[1] = fmaf(y[e], y[e], ss[1]);
+        }
+        block_totals(ss, sums, (hidden / 4 + kWave - 1) / kWave);
+        if (!here) return;
+        const float inv_a = inv_rms(ss[0], 1.0f / static_cast<float>(hidden), eps), inv_b = inv_rms(ss[1], 1.0f / static_cast<float>(hidden), eps);
+        read_quad(wa + j, u);
+        read_quad(wb + j, w);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            z[e] = factor_a == factor_b ? factor_a * (x[e] * inv_a * u[e] + y[e] * inv_b * w[e])
+                                        : factor_a * (x[e] * inv_a * u[e]) + factor_b * (y[e] * inv_b * w[e]);
+    }
+    write_quad(out + at, z);
 }
 
 // x[t, :] = factor * E[id_t, :] + P[position_t, :]: a token's vector plus a learned vector of its position, added in float32
@@ -419,6 +515,17 @@ extern "C" int egpt_add_layernorm(float* h, const void* delta, int delta_splits,
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t stride = static_cast<size_t>(delta_rows) * hidden;
     const size_t lds = static_cast<size_t>(hidden) * sizeof(float);
+    if (hidden % 4 == 0 && hidden <= kQuadsMost && quads(h, delta, weight, bias, out)) {
+        auto launch = [&](auto kernel, auto* typed) {
+            using T = std::remove_const_t<std::remove_pointer_t<decltype(typed)>>;
+            kernel<<<n_rows, quad_threads(hidden), 0, s>>>(h, typed, static_cast<const T*>(bias), rows, static_cast<T*>(out), hidden, eps,
+                                                           stream_view<T>(delta, delta_splits, stride));
+        };
+        if (dtype == 0) launch(add_layernorm_quads_kernel<float>, static_cast<const float*>(weight));
+        else launch(add_layernorm_quads_kernel<bf16_t>, static_cast<const bf16_t*>(weight));
+        EGPT_CHECK_LAUNCH();
+        return EGPT_OK;
+    }
     if (dtype == 0)
         add_layernorm_kernel<float><<<n_rows, 256, lds, s>>>(h, stream_view<float>(delta, delta_splits, stride), rows,
                                                              static_cast<const float*>(weight), static_cast<const float*>(bias),
@@ -441,6 +548,18 @@ extern "C" int egpt_normed_pair_mean(const void* a, int a_splits, const void* b,
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t stride = static_cast<size_t>(n_rows) * hidden;
     const size_t lds = 2 * static_cast<size_t>(hidden) * sizeof(float);
+    if (hidden % 4 == 0 && hidden <= kQuadsMost && quads(a, b, bias_a, bias_b, wa, wb, out)) {
+        auto launch = [&](auto kernel, auto* typed) {
+            using T = std::remove_const_t<std::remove_pointer_t<decltype(typed)>>;
+            kernel<<<n_rows, quad_threads(hidden), 0, s>>>(static_cast<const T*>(bias_a), static_cast<const T*>(bias_b), typed, static_cast<const T*>(wb),
+                                                           out, hidden, eps, factor, factor_b, stream_view<T>(a, a_splits, stride),
+                                                           stream_view<T>(b, b_splits, stride));
+        };
+        if (dtype == 0) launch(normed_pair_mean_quads_kernel<float>, static_cast<const float*>(wa));
+        else launch(normed_pair_mean_quads_kernel<bf16_t>, static_cast<const bf16_t*>(wa));
+        EGPT_CHECK_LAUNCH();
+        return EGPT_OK;
+    }
     if (dtype == 0)
         normed_pair_mean_kernel<float><<<n_rows, 256, lds, s>>>(
             stream_view<float>(a, a_splits, stride), stream_view<float>(b, b_splits, stride), static_cast<const float*>(bias_a),

@@ -1,6 +1,6 @@
 """The small kernels of a decode step at the edges of their sizes: the norm of few rows, the gate's activation behind partial sums, and the
 combination of attention's parts, against plain torch in 64 bits.  What they return is rounded to bfloat16 once, so a value is off by at
-most 2^-8 of itself (half a unit in the last of eight bits, and as much again where float32 sums fall on the other side of a tie)."""
+most 2^-8 of itself (half a unit in the last of its eight bits); what is added to that is the float32 sums' own error."""
 import pytest
 import torch
 
