@@ -236,7 +236,8 @@ __device__ __forceinline__ void store_stream(fixed_t* p, const float (&v)[4]) {
 enum Added { kNothing = 0, kWhole = 1, kParts = 2 };
 constexpr int kFewMost = 4096;              // features: four for each of 1,024 threads
 
-template <typename R, int ADDED>
+// BATCH: partial sums whose loads are on their way together
+template <typename R, int ADDED, int BATCH = 1>
 __global__ __launch_bounds__(kFewMost / 4) void add_rmsnorm_few_kernel(R* __restrict__ h, const void* __restrict__ added,
                                                                        const bf16_t* __restrict__ weight, bf16_t* __restrict__ out,
                                                                        int hidden, int n_splits, int split_stride,
@@ -248,12 +249,12 @@ __global__ __launch_bounds__(kFewMost / 4) void add_rmsnorm_few_kernel(R* __rest
     const int j = threadIdx.x * 4;
     const bool here = j < hidden;
     float v[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {0.f, 0.f, 0.f, 0.f};
-    u32x4 t[8];
+    u32x4 t[BATCH];
     const buffer_t parts = values_of(static_cast<const float*>(added) + (ADDED == kParts ? src * hidden : 0),
                                      ADDED == kParts ? ((n_splits - 1) * split_stride + hidden) * 4 : 0);
     if constexpr (ADDED == kParts) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) t[i] = read16(parts, here ? (i * split_stride + j) * 4 : kNowhere);
+        for (int i = 0; i < BATCH; ++i) t[i] = read16(parts, here ? (i * split_stride + j) * 4 : kNowhere);
     }
     uint2 whole = uint2{0u, 0u};
     if (here) {
@@ -266,14 +267,14 @@ __global__ __launch_bounds__(kFewMost / 4) void add_rmsnorm_few_kernel(R* __rest
     if constexpr (ADDED == kParts) {
         float d[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < BATCH; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) d[e] += __uint_as_float(t[i][e]);
-        for (int s0 = 8; s0 < n_splits; s0 += 8) {
+        for (int s0 = BATCH; s0 < n_splits; s0 += BATCH) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) t[i] = read16(parts, here ? ((s0 + i) * split_stride + j) * 4 : kNowhere);
+            for (int i = 0; i < BATCH; ++i) t[i] = read16(parts, here ? ((s0 + i) * split_stride + j) * 4 : kNowhere);
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int i = 0; i < BATCH; ++i)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) d[e] += __uint_as_float(t[i][e]);
         }
@@ -308,7 +309,9 @@ static void launch_norm_few(void* h, const void* delta, int n_splits, int stride
     };
     if (!delta) launch(add_rmsnorm_few_kernel<R, kNothing>);
     else if (n_splits == 0) launch(add_rmsnorm_few_kernel<R, kWhole>);
-    else launch(add_rmsnorm_few_kernel<R, kParts>);
+    else if (n_splits == 1) launch(add_rmsnorm_few_kernel<R, kParts, 1>);
+    else if (n_splits == 2) launch(add_rmsnorm_few_kernel<R, kParts, 2>);
+    else launch(add_rmsnorm_few_kernel<R, kParts, 8>);
 }
 
 // ----------------------------------------------------------------------------- SwiGLU
@@ -653,7 +656,14 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
     // (loads and stores of 16 bytes: operands that begin elsewhere take the kernel of single values)
     const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(weight) |
                            reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    if (dtype == 1 && hidden % 8 == 0 && aligned && !fixed && (delta_splits <= 1 ? n_rows >= 32 : n_rows > 64)) {
+    if (dtype != 0 && dtype != 1) return EGPT_BAD_ARGUMENT;
+    // Many rows go by quads as well up to 2,048 values: 2,048 rows of 896 behind two partial sums 8.1 -> 6.6 us, behind a rounded product 6.9 ->
+    // 6.0, 552 rows of 1,536 7.0 -> 5.6 and 5.7 -> 5.5.  Wider ones are the same either way (prompts of the 7B sizes 24.06 and 24.08 ms) and keep
+    // eight values a thread, which holds more of them.
+    const bool many = delta_splits <= 1 ? n_rows >= 32 : n_rows > 64;
+    const bool by_quads = dtype == 1 && hidden % 4 == 0 && hidden <= (many && !fixed && hidden % 8 == 0 ? 2048 : kFewMost) && aligned &&
+                          (delta_splits + 8) * static_cast<long long>(stride) * 4 <= INT32_MAX;
+    if (dtype == 1 && hidden % 8 == 0 && aligned && !fixed && many && !by_quads) {
         const int threads = hidden >= 2048 ? 256 : 128;
         float* hf = static_cast<float*>(h);
         if (delta_splits == 0)
@@ -667,8 +677,7 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
         EGPT_CHECK_LAUNCH();
         return EGPT_OK;
     }
-    if (dtype != 0 && dtype != 1) return EGPT_BAD_ARGUMENT;
-    if (dtype == 1 && hidden % 4 == 0 && hidden <= kFewMost && aligned && (delta_splits + 8) * static_cast<long long>(stride) * 4 <= INT32_MAX) {
+    if (by_quads) {
         if (fixed) launch_norm_few<fixed_t>(h, delta, delta_splits, static_cast<int>(stride), rows, weight, weight_offset, eps, out, n_rows, hidden, s);
         else launch_norm_few<float>(h, delta, delta_splits, static_cast<int>(stride), rows, weight, weight_offset, eps, out, n_rows, hidden, s);
         EGPT_CHECK_LAUNCH();
