@@ -1206,8 +1206,9 @@ struct DecodeSizes {
 // zero.  (Written with conditions around the loads, the compiler moved the queries' arithmetic in front of the keys' loads and waited
 // five times one after the other.)  Instructions count as much: a kernel begins with an empty instruction cache, a jump over code that is
 // not needed is a trip for the next line, and 300 instructions take 1 us.  So there are no divisions, code for rare sizes lies behind the
-// common path, and a round's keys share one maximum.  A layer, 14 heads of 64 on 2 behind 2,048 tokens: one request 8.1 -> 6.1 us, eight
-// 8.3 -> 6.4; of the 6 the loads' issue is 1.5, the trip to the keys 1.2, their products and softmax 1, the wavefronts' combination 0.6.
+// common path, and a round's keys share one maximum.  14 heads of 64 on 2 behind 2,048 tokens: a step of 24 layers for one request 732 ->
+// 693 us, for eight 806 -> 768; by the kernel trace 8.8 -> 7.8 us a layer for one (the fastest 7.0 -> 6.2), of which by timestamps inside the
+// loads' issue is 1.5, the trip to the keys 1.2, their products and softmax 1, the wavefronts' combination 0.6.
 template <int HD, int PF, bool FUSED, bool MIXED, bool RANGED, int INF>
 __device__ __forceinline__ void decode_block(
     float* wave_state, int bx, int by, int bz, const int32_t* __restrict__ lengths, const int32_t* __restrict__ block_table,
@@ -1619,8 +1620,9 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
 // out[row, :] = sum_s exp(m_s - M) o_s / sum_s exp(m_s - M) l_s over the splits; one wavefront per row, R features of it a lane (R * 64
 // of them or fewer).  Lane s takes split s's (maximum, sum) so that the weights of up to 64 splits are known after one round of loads;
 // the first eight splits' partial outputs are asked for together with them (a part of a split without visible keys may hold anything:
-// it is read and then dropped), the others eight at a time.  A layer of 64 decoded tokens, 14 heads of 64, two splits: 4.6 us with four
-// features a lane whatever the head size and shuffles through LDS, 3.4 so.
+// it is read and then dropped), the others eight at a time.  A layer of 64 decoded tokens, 14 heads of 64, two splits, against four
+// features a lane whatever the head size and shuffles through LDS: the fastest 3.7 -> 2.0 us, the median, which is the trips to memory
+// behind attention's writes, 4.7 and 5.0.
 template <int R>
 __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml,

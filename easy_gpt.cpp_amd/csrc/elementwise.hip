@@ -218,8 +218,8 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict
 
 // The same for few rows of bfloat16, a workgroup to a row, four neighbouring features a thread: what bounds it is the trip to what the
 // kernels before wrote and the instructions around it, so every load goes out at once (partial sums past the last one are past the
-// buffer's end and add zero) and nothing stands behind a branch.  us, in a decode step, with single values: 64 rows of 896 behind
-// 13 partial sums 4.1 -> 3.3; 8 rows of 3,584 in fixed point 5.0 -> 4.0.
+// buffer's end and add zero) and nothing stands behind a branch.  With single values, then so, in decode steps: 64 rows of 896
+// behind partial sums 4.4 -> 3.7 us on average (the fastest 3.4 -> 1.9); a step with 29 norms of 8 rows of 3,584 in fixed point 3,516 -> 3,484.
 __device__ __forceinline__ void load_stream(const float* p, float (&v)[4]) {
     const float4 a = *reinterpret_cast<const float4*>(p);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
@@ -348,50 +348,6 @@ __global__ void swiglu_scaled_kernel(const float* __restrict__ product, const fl
         const float u = scale_then_bias(gate_up.at(t * 2 * inter + inter + j), scale, 0.f);
         out[t * inter + j] = from_float<T>(u * gate_activation(g, act));
     }
-}
-
-// Either in bfloat16 with four features per thread and a row of workgroups per token (inter % 4 == 0): one trip for up to four partial
-// sums and for the rows' factors, and no division to find a place.  8 rows of 18,944 from three partial sums 5.1 -> 3.9 us in a step.
-template <bool SCALED>
-__global__ __launch_bounds__(256) void swiglu_few_kernel(const float* __restrict__ product, bf16_t* __restrict__ out, int n_splits, int n_tokens,
-                                                         int inter, int split_stride, int act, const float* __restrict__ row_ss, int ss_splits,
-                                                         float inv_hidden, float eps) {
-    const int j = (blockIdx.x * 256 + threadIdx.x) * 4, t = blockIdx.y;
-    if (j >= inter) return;
-    const buffer_t parts = values_of(product + static_cast<size_t>(t) * 2 * inter, ((n_splits - 1) * split_stride + 2 * inter) * 4);
-    float g[4] = {0.f, 0.f, 0.f, 0.f}, u[4] = {0.f, 0.f, 0.f, 0.f};
-    auto add = [&](int s0) {
-        u32x4 tg[4], tu[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int at = s0 + i < n_splits ? ((s0 + i) * split_stride + j) * 4 : kNowhere;
-            tg[i] = read16(parts, at);
-            tu[i] = read16(parts, s0 + i < n_splits ? at + inter * 4 : kNowhere);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                g[e] += __uint_as_float(tg[i][e]);
-                u[e] += __uint_as_float(tu[i][e]);
-            }
-    };
-    add(0);
-    for (int s0 = 4; s0 < n_splits; s0 += 4) add(s0);
-    if constexpr (SCALED) {
-        float ss = 0.f;
-        for (int i = 0; i < ss_splits; ++i) ss += row_ss[i * n_tokens + t];
-        const float scale = inv_rms(ss, inv_hidden, eps);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            g[e] = scale_then_bias(g[e], scale, 0.f);
-            u[e] = scale_then_bias(u[e], scale, 0.f);
-        }
-    }
-    float y[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = u[e] * gate_activation(g[e], act);
-    *reinterpret_cast<uint2*>(out + static_cast<size_t>(t) * inter + j) = uint2{bf16_pair(y[0], y[1]), bf16_pair(y[2], y[3])};
 }
 
 // bfloat16, eight features per thread (inter % 8 == 0, one tensor, no partial sums)
@@ -711,19 +667,6 @@ extern "C" int egpt_swiglu(const void* gate_up, int n_splits, const float* row_s
     const size_t total = static_cast<size_t>(n_tokens) * inter;
     const int blocks = static_cast<int>(total / 256 + 1 > 8192 ? 8192 : total / 256 + 1);
     const size_t stride = total * 2;
-    if (dtype == 1 && (row_ss ? n_splits >= 1 && ss_splits >= 1 && hidden > 0 : n_splits >= 2) && inter % 4 == 0 && n_tokens <= 65535 &&
-        n_splits * static_cast<long long>(stride) * 4 <= INT32_MAX &&
-        ((reinterpret_cast<uintptr_t>(gate_up) & 15) | (reinterpret_cast<uintptr_t>(out) & 7)) == 0) {
-        const dim3 grid(static_cast<unsigned>((inter / 4 + 255) / 256), static_cast<unsigned>(n_tokens));
-        auto launch = [&](auto kernel) {
-            kernel<<<grid, 256, 0, s>>>(static_cast<const float*>(gate_up), static_cast<bf16_t*>(out), n_splits, n_tokens, inter,
-                                        static_cast<int>(stride), act, row_ss, ss_splits, row_ss ? 1.0f / hidden : 0.f, eps);
-        };
-        if (row_ss) launch(swiglu_few_kernel<true>);
-        else launch(swiglu_few_kernel<false>);
-        EGPT_CHECK_LAUNCH();
-        return EGPT_OK;
-    }
     if (row_ss) {
         // float32 partial sums with a pending row factor
         if (n_splits < 1 || ss_splits < 1 || hidden <= 0 || n_tokens > 65535 || (dtype != 0 && dtype != 1))
