@@ -1542,15 +1542,16 @@ __device__ __forceinline__ void decode_block(
     const size_t row0 = static_cast<size_t>(tok) * nq + kh * group_size;
     for (int idx = threadIdx.x; idx < group_size * HD; idx += n_threads) {
         const int r = idx / HD, c = idx % HD;
-        // the states of all wavefronts are read together (past the last one the last again, which weighs nothing)
+        // the states of all wavefronts are read together (past the last one the last again, of which nothing counts: a weight of zero
+        // would leave its infinities)
         float ms[8], ls[8], os[8], mx = -INFINITY;
 #pragma unroll
         for (int w = 0; w < 8; ++w) {
             const float* st = wave_state + (min(w, n_waves - 1) * 16 + r) * kRow;
-            const float m = st[HD];
+            const float m = st[HD], l = st[HD + 1], x = st[c];
             ms[w] = w < n_waves ? m : -INFINITY;
-            ls[w] = st[HD + 1];
-            os[w] = st[c];
+            ls[w] = w < n_waves ? l : 0.f;
+            os[w] = w < n_waves ? x : 0.f;
             mx = fmaxf(mx, ms[w]);
         }
         float num = 0.f, den = 0.f;

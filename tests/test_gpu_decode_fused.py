@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import plain_qwen2 as plain
-from test_gpu_kernels import DEV, build_paged, rnd
+from test_gpu_kernels import DEV, build_paged, paged_reference, rnd
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,29 @@ def test_places_of_pages_and_partial_sums(k, nq, nkv, hd, ps, parts, squares, ba
                                     kv_len.to(DEV), nq, nkv, hd, ps, 1.0 / math.sqrt(hd), window, int(kv_len.max())) is None
     assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
     assert torch.equal(out1, out2)
+
+
+@pytest.mark.parametrize("hd,lean", [(64, 0), (64, 1), (128, 0), (128, 1)])
+@pytest.mark.parametrize("waves", [1, 2, 3, 4, 7, 8])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_infinite_values_stay_infinite(k, hd, lean, waves, splits):
+    # a value that is infinite makes its feature infinite, and that one alone, whichever wavefront has its key and however many there are
+    nq, nkv, ps = 6, 2, 16
+    kv = 32 * waves * splits                     # a block of keys for each wavefront
+    kc, vc, table, keys, vals = build_paged([(1, kv)], nkv, hd, ps, torch.bfloat16, seed=41)
+    qkv = rnd(1, (nq + 2 * nkv) * hd, dtype=torch.bfloat16, seed=42)
+    start, context = (torch.tensor([v], dtype=torch.int32, device=DEV) for v in (0, kv))
+    for at, feature, sign in ((kv - 2, 5, 1.0), (3, hd - 1, -1.0), (kv // 2, 17, 1.0)):
+        vv = vc.clone()
+        vv[table[0, at // ps].long(), :, feature, at % ps] = sign * float("inf")
+        out, part_o, part_ml = torch.empty(1, nq * hd, dtype=torch.bfloat16, device=DEV), rnd(splits, nq, hd), rnd(splits, nq, 2)
+        k._run("egpt_paged_attention_decode", qkv.data_ptr(), out.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(), kc.data_ptr(), vv.data_ptr(),
+               table.data_ptr(), table.shape[1], start.data_ptr(), context.data_ptr(), 1, nq, nkv, hd, ps, hd ** -0.5, 0, splits, waves, 1, lean,
+               k._stream())
+        with_inf = vals[0].double()
+        with_inf[at, :, feature] = sign * float("inf")
+        want = paged_reference(qkv.double().cpu().view(1, nq + 2 * nkv, hd)[:, :nq], keys[0].double(), with_inf, nq, nkv, hd ** -0.5, 0)[0]
+        got = out.double().cpu().view(nq, hd)
+        assert torch.isinf(want[:, feature]).all() and torch.equal(got[:, feature], want[:, feature])
+        rest = torch.arange(hd) != feature
+        assert float((got[:, rest] - want[:, rest]).abs().max()) <= 1.2e-2
