@@ -1209,7 +1209,10 @@ struct DecodeSizes {
 // common path, and a round's keys share one maximum.  14 heads of 64 on 2 behind 2,048 tokens: a step of 24 layers for one request 732 ->
 // 693 us, for eight 806 -> 768; by the kernel trace 8.8 -> 7.8 us a layer for one (the fastest 7.0 -> 6.2), of which by timestamps inside the
 // loads' issue is 1.5, the trip to the keys 1.2, their products and softmax 1, the wavefronts' combination 0.6.
-template <int HD, int PF, bool FUSED, bool MIXED, bool RANGED, int INF>
+//
+// WIDE: operands that 32 bits of place or loads of two values don't reach (partial sums of 2 GB and more, biases that begin between two of
+// 4 bytes, pages of a head's gigabytes): plain loads behind conditions.
+template <int HD, int PF, bool FUSED, bool MIXED, bool RANGED, int INF, bool WIDE>
 __device__ __forceinline__ void decode_block(
     float* wave_state, int bx, int by, int bz, const int32_t* __restrict__ lengths, const int32_t* __restrict__ block_table,
     const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, const DecodeSizes& d, const bf16_t* __restrict__ qkv,
@@ -1260,13 +1263,21 @@ __device__ __forceinline__ void decode_block(
         const int query = kh * group_size + h, other = nq + kh + past * nkv;
         return (past < 0 ? query : other) * HD + i;
     };
-    const int stride = d.n_tokens * width;                       // values of a partial sum
-    const buffer_t prod_buf = values_of(f.prod + static_cast<size_t>(tok) * width, ((f.in_splits - 1) * stride + width) * 4);
+    using place_t = std::conditional_t<WIDE, size_t, int>;
+    const place_t stride = static_cast<place_t>(d.n_tokens) * width;      // values of a partial sum
+    const buffer_t prod_buf = values_of(f.prod + static_cast<size_t>(tok) * width, WIDE ? 0 : ((f.in_splits - 1) * stride + width) * 4);
     const buffer_t bias_buf = values_of(f.bias, f.bias ? width * 2 : 0);
     const buffer_t turn_buf = values_of(f.cos_sin + static_cast<size_t>(tok) * HD, HD * 4);
     auto parts_load = [&](int col, int j0, u32x2 (&ta)[INF], u32x2 (&tb)[INF]) {
 #pragma unroll
         for (int j = 0; j < INF; ++j) {
+            if constexpr (WIDE) {
+                const float* src = f.prod + static_cast<size_t>(tok) * width + min(j0 + j, f.in_splits - 1) * stride + col;
+                const bool there = j0 + j < f.in_splits;
+                ta[j] = u32x2{there ? __float_as_uint(src[0]) : 0u, there ? __float_as_uint(src[1]) : 0u};
+                tb[j] = u32x2{there ? __float_as_uint(src[half]) : 0u, there ? __float_as_uint(src[half + 1]) : 0u};
+                continue;
+            }
             const int at = (j0 + j) * stride * 4 + col * 4;              // (behind the last sum: past the buffer's end)
             ta[j] = read8(prod_buf, at);
             tb[j] = read8(prod_buf, at + half * 4);
@@ -1275,8 +1286,13 @@ __device__ __forceinline__ void decode_block(
     auto item_load = [&](unsigned it, Item& r) {
         const int col = item_col(it);
         parts_load(col, 0, r.ta, r.tb);
-        r.ba = read4(bias_buf, col * 2);
-        r.bb = read4(bias_buf, col * 2 + half * 2);
+        if constexpr (WIDE) {
+            r.ba = read2(bias_buf, col * 2) | read2(bias_buf, col * 2 + 2) << 16;
+            r.bb = read2(bias_buf, col * 2 + half * 2) | read2(bias_buf, col * 2 + half * 2 + 2) << 16;
+        } else {
+            r.ba = read4(bias_buf, col * 2);
+            r.bb = read4(bias_buf, col * 2 + half * 2);
+        }
         r.turn = read16(turn_buf, it % kItems * 16);
     };
     [[maybe_unused]] Item first;
@@ -1344,6 +1360,17 @@ __device__ __forceinline__ void decode_block(
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
                 const bool ok = offs[i][kt] >= 0 && pages[i][kt] >= 0;
+                if constexpr (WIDE) {
+                    const size_t row = (static_cast<size_t>(ok ? pages[i][kt] : 0) * nkv + kh) * page_size, o = ok ? offs[i][kt] : 0;
+                    const bf16_t* kp = k_cache + (row + o + lj) * HD + lg * 8;
+                    const bf16_t* vp = v_cache + row * HD + static_cast<size_t>(lj) * page_size + o + lg * 4;
+#pragma unroll
+                    for (int kd = 0; kd < KD; ++kd) kk[i][kt][kd] = ok ? *reinterpret_cast<const uint4*>(kp + kd * 32) : uint4{0u, 0u, 0u, 0u};
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt)
+                        vv[i][kt][dt] = ok ? *reinterpret_cast<const uint2*>(vp + static_cast<size_t>(dt * 16) * page_size) : uint2{0u, 0u};
+                    continue;
+                }
                 const unsigned off = ok ? offs[i][kt] : 0;
                 const size_t at = static_cast<size_t>(static_cast<unsigned>(ok ? pages[i][kt] : 0)) * page_bytes;
                 const buffer_t kr = values_of(k_head + at + off * (HD * 2), ok ? 16 * HD * 2 : 0);
@@ -1421,8 +1448,8 @@ __device__ __forceinline__ void decode_block(
                 bf16_t* dst = f.v_cache_w + ((static_cast<size_t>(page) * nkv + kh) * HD + i) * page_size + off;
                 dst[0] = y0[0];
                 dst[page_size] = y0[1];
-                dst[half * page_size] = y1[0];
-                dst[(half + 1) * page_size] = y1[1];
+                dst[half * static_cast<size_t>(page_size)] = y1[0];
+                dst[(half + 1) * static_cast<size_t>(page_size)] = y1[1];
             }
         };
         const int n_items = (group_size + (writer ? 2 : 0)) * kItems;
@@ -1577,7 +1604,7 @@ __device__ __forceinline__ void decode_block(
 }
 
 // INF: partial sums of the product that are read in one batch (FUSED)
-template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false, int INF = 8>
+template <int HD, int PF, bool FUSED, bool MIXED = false, bool RANGED = false, int INF = 8, bool WIDE = false>
 __global__ __launch_bounds__(512) void attention_decode_kernel(
     // (what the first loads are addressed by: 14 words that arrive with the wavefronts; `lengths` is the table of ranges where
     // there is one)
@@ -1588,7 +1615,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(
     FusedQkv f) {
     extern __shared__ float wave_state[];
     const DecodeSizes d{table_width, page_size, nkv, n_splits, page_magic, split_magic, wave_magic, group, window, n_tokens, scale, n_waves};
-    decode_block<HD, PF, FUSED, MIXED, RANGED, INF>(wave_state, blockIdx.x, blockIdx.y, blockIdx.z, lengths, block_table, k_cache, v_cache, d, qkv, out,
+    decode_block<HD, PF, FUSED, MIXED, RANGED, INF, WIDE>(wave_state, blockIdx.x, blockIdx.y, blockIdx.z, lengths, block_table, k_cache, v_cache, d, qkv, out,
                                                     part_o, part_ml, q_start, q_len, f);
 }
 
@@ -1613,7 +1640,7 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
     } else {
         const int i = index - row_blocks;
         const DecodeSizes d{table_width, page_size, nkv, 1, page_magic, 0, (1u << 28) + 1, nq / nkv, window, n_seqs, scale, 8};
-        decode_block<HD, 2, false, true, true, 8>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, ranges, block_table, k_cache, v_cache,
+        decode_block<HD, 2, false, true, true, 8, false>(reinterpret_cast<float*>(smem), i % range_slots, i / range_slots, 0, ranges, block_table, k_cache, v_cache,
                                                   d, qkv, out, range_o, range_ml, q_start, q_len, FusedQkv{});
     }
 }
@@ -1740,6 +1767,9 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
     if (fused) lds += 18 * HD * sizeof(bf16_t);          // 16 query heads, the new key and value
     if (lds > kDecodeLdsMost) return EGPT_UNSUPPORTED_SIZE;
     const FusedQkv fq = fused ? *fused : FusedQkv{};
+    // (up to 16 partial sums behind the last one are asked for by their place, which has to be past the buffer's end and not around it)
+    const bool wide = 2.0 * page_size * HD * nkv > 4294967295.0 || 2.0 * page_size * HD > 2147483647.0 ||
+                      (fused && ((fq.in_splits + 32.0) * n_tokens * (nq + 2 * nkv) * HD * 4 > 2147483647.0 || (reinterpret_cast<uintptr_t>(fq.bias) & 3) != 0));
     auto launch = [&](auto kernel, bool (*raise)(), const int32_t* lengths, const void* q, const int32_t* counts, int splits) {
         // (eight wavefronts at head size 128: more than a kernel may take without being asked; once per instance)
         if (lds > 64 * 1024 && !raise()) return EGPT_UNSUPPORTED_SIZE;
@@ -1750,7 +1780,13 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
     };
     int e;
 #define EGPT_DECODE(...) attention_decode_kernel<HD, __VA_ARGS__>, raise_lds<attention_decode_kernel<HD, __VA_ARGS__>>
-    if (ranges && fused) e = fused->in_splits > 8 ? launch(EGPT_DECODE(2, true, false, true, 16), ranges, nullptr, nullptr, 1)
+    if (wide) {
+        if (ranges && fused) e = launch(EGPT_DECODE(2, true, false, true, 8, true), ranges, nullptr, nullptr, 1);
+        else if (ranges) e = launch(EGPT_DECODE(2, false, true, true, 8, true), ranges, qkv, q_len, 1);
+        else if (fused) e = launch(EGPT_DECODE(2, true, false, false, 8, true), kv_len, nullptr, nullptr, n_splits);
+        else if (q_len) e = launch(EGPT_DECODE(2, false, true, false, 8, true), kv_len, qkv, q_len, n_splits);
+        else e = launch(EGPT_DECODE(2, false, false, false, 8, true), kv_len, qkv, nullptr, n_splits);
+    } else if (ranges && fused) e = fused->in_splits > 8 ? launch(EGPT_DECODE(2, true, false, true, 16), ranges, nullptr, nullptr, 1)
                                                   : launch(EGPT_DECODE(2, true, false, true, 8), ranges, nullptr, nullptr, 1);
     else if (ranges) e = launch(EGPT_DECODE(2, false, true, true), ranges, qkv, q_len, 1);
     else if (fused) e = fused->in_splits > 8 ? launch(EGPT_DECODE(PF, true, false, false, 16), kv_len, nullptr, nullptr, n_splits)
@@ -2039,8 +2075,6 @@ static int attention_decode_fused(const float* qkv_prod, int in_splits, const fl
     if ((hd != 64 && hd != 128) || page_size % 16 != 0 || nq / nkv > 16 || nkv > 65535 || n_splits > 64 ||
         n_waves < 1 || n_waves > 8)
         return EGPT_UNSUPPORTED_SIZE;
-    // (a row's partial sums are read through a buffer whose places are 32 bits, up to 32 more of them than there are; two biases at once)
-    if ((in_splits + 32LL) * n_seqs * (nq + 2 * nkv) * hd * 4 > INT32_MAX || (reinterpret_cast<uintptr_t>(bias) & 3) != 0) return EGPT_UNSUPPORTED_SIZE;
     FusedQkv f = {};
     f.prod = qkv_prod; f.in_splits = in_splits;
     f.row_ss = row_ss; f.ss_splits = row_ss ? ss_splits : 0;

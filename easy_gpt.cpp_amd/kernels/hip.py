@@ -1308,8 +1308,6 @@ class HipKernels(KernelBackend):
         b, table_width = block_table.shape
         if t != b or width != (nq + 2 * nkv) * hd:
             return False
-        if (in_splits + 32) * t * width * 4 >= 1 << 31 or (bias is not None and bias.data_ptr() % 4):
-            return False                 # (the kernel's places in the partial sums are 32 bits; two biases are one load)
         self._need(prod, "prod", _F32)
         self._need(out, "out", _BF16, (t, nq * hd))
         self._caches(k_cache, v_cache, _BF16, nkv, page_size, hd)

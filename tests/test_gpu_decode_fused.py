@@ -73,3 +73,70 @@ def test_infinite_values_stay_infinite(k, hd, lean, waves, splits):
         assert torch.isinf(want[:, feature]).all() and torch.equal(got[:, feature], want[:, feature])
         rest = torch.arange(hd) != feature
         assert float((got[:, rest] - want[:, rest]).abs().max()) <= 1.2e-2
+
+
+def both_ways(k, prod, row_ss, bias, kv_len, caches, table, slots, nq, nkv, hd, ps, window=0):
+    """(fused, the two kernels it stands for): output and caches of decoded tokens."""
+    t, width = len(kv_len), (nq + 2 * nkv) * hd
+    inv_freq = torch.as_tensor(plain.rope_inv_freq(hd, 1e4), dtype=torch.float32).to(DEV)
+    kv, start, one = kv_len.to(DEV), torch.arange(t, dtype=torch.int32, device=DEV), torch.ones(t, dtype=torch.int32, device=DEV)
+    got = []
+    for fused in (True, False):
+        kc, vc = (c.clone() for c in caches)
+        out = torch.zeros(t, nq * hd, dtype=torch.bfloat16, device=DEV)
+        if fused:
+            assert k.attention_decode_fused(prod, row_ss, 96, 1e-5, bias, kv - 1, inv_freq, hd, slots, out, kc, vc, table, start, kv, nq, nkv, hd, ps,
+                                            hd ** -0.5, window, int(kv_len.max())) is None
+        else:
+            qkv = torch.empty(t, width, dtype=torch.bfloat16, device=DEV)
+            k.qkv_rope_store(prod, bias, kv - 1, inv_freq, hd, slots, kc, vc, nq, nkv, hd, ps, out=qkv, row_ss=row_ss, hidden=96, eps=1e-5)
+            k.paged_attention(qkv, out, kc, vc, table, start, one, kv, nq, nkv, hd, ps, hd ** -0.5, window, 1, int(kv_len.max()))
+        got.append((out, kc, vc))
+    return got
+
+
+def near(one, other):
+    """bfloat16 results of the same sums in another order of blocks (a value may round to its neighbour)."""
+    a, b = one.double(), other.double()
+    return bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2e-3).all())
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(14, 2, 64), (16, 1, 128)])
+@pytest.mark.parametrize("parts,squares,batch", [(1, 1, 1), (9, 9, 5), (33, 70, 70)])
+def test_a_bias_that_begins_between_two_of_four_bytes(k, nq, nkv, hd, parts, squares, batch):
+    kv_len = torch.tensor([1 + (577 * i + 900) % 1500 for i in range(batch)], dtype=torch.int32)
+    kc, vc, table, _, _ = build_paged([(1, int(n)) for n in kv_len], nkv, hd, 16, torch.bfloat16, seed=51)
+    slots = torch.stack([table[b, (int(n) - 1) // 16].cpu() * 16 + (int(n) - 1) % 16 for b, n in enumerate(kv_len)]).to(torch.int32).to(DEV)
+    width = (nq + 2 * nkv) * hd
+    prod, row_ss = rnd(parts, batch, width, seed=52), rnd(squares, batch, seed=53).abs() * 30 + 1
+    bias = rnd(width + 1, dtype=torch.bfloat16, seed=54)[1:]
+    assert bias.data_ptr() % 4 == 2
+    (out, k1, v1), (want, k2, v2) = both_ways(k, prod, row_ss, bias, kv_len, (kc, vc), table, slots, nq, nkv, hd, 16)
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and near(out, want)
+
+
+def test_partial_sums_of_more_than_two_gigabytes(k):
+    nq, nkv, hd, t, parts = 28, 4, 128, 300, 400
+    kv_len = torch.tensor([1 + 7 * i % 90 for i in range(t)], dtype=torch.int32)
+    kc, vc, table, _, _ = build_paged([(1, int(n)) for n in kv_len], nkv, hd, 16, torch.bfloat16, seed=61)
+    slots = torch.stack([table[b, (int(n) - 1) // 16].cpu() * 16 + (int(n) - 1) % 16 for b, n in enumerate(kv_len)]).to(torch.int32).to(DEV)
+    width = (nq + 2 * nkv) * hd
+    assert parts * t * width * 4 > 1 << 31
+    prod = torch.randn(parts, t, width, device=DEV, generator=torch.Generator(device=DEV).manual_seed(62)) * 0.05
+    (out, k1, v1), (want, k2, v2) = both_ways(k, prod, None, rnd(width, dtype=torch.bfloat16, seed=63), kv_len, (kc, vc), table, slots, nq, nkv, hd, 16)
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and near(out, want)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_a_page_of_more_than_two_gigabytes_a_head(k, hd):
+    # one page for a request's whole context: a feature's values lie gigabytes behind the head's first
+    nq, nkv, ps = 4, 1, (1 << 31) // (2 * hd) + 16
+    kv_len = torch.tensor([77], dtype=torch.int32)
+    big = [torch.empty(1, nkv, *shape, dtype=torch.bfloat16, device=DEV) for shape in ((ps, hd), (hd, ps))]
+    small = [torch.randn(1, nkv, *shape, device=DEV, generator=torch.Generator(device=DEV).manual_seed(71)).to(torch.bfloat16) for shape in ((80, hd), (hd, 80))]
+    big[0][:, :, :80], big[1][..., :80] = small
+    width, table, slots = (nq + 2 * nkv) * hd, torch.zeros(1, 1, dtype=torch.int32, device=DEV), torch.tensor([76], dtype=torch.int32, device=DEV)
+    prod = rnd(3, 1, width, seed=72)
+    both = [both_ways(k, prod, None, None, kv_len, caches, table, slots, nq, nkv, hd, caches[0].shape[2]) for caches in (big, small)]
+    for (out, kc, vc), (want, k2, v2) in zip(both[0], both[1]):
+        assert torch.equal(kc[:, :, :80], k2) and torch.equal(vc[..., :80], v2) and near(out, want)
