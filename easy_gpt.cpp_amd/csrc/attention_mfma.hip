@@ -1575,11 +1575,18 @@ __device__ __forceinline__ void decode_block(
 #pragma unroll
         for (int w = 0; w < 8; ++w) {
             const float* st = wave_state + (min(w, n_waves - 1) * 16 + r) * kRow;
-            const float m = st[HD], l = st[HD + 1], x = st[c];
+            const float m = st[HD];
             ms[w] = w < n_waves ? m : -INFINITY;
-            ls[w] = w < n_waves ? l : 0.f;
-            os[w] = w < n_waves ? x : 0.f;
+            ls[w] = st[HD + 1];
+            os[w] = st[c];
             mx = fmaxf(mx, ms[w]);
+        }
+        if (__builtin_expect(n_waves < 8, 0)) {
+#pragma unroll
+            for (int w = 1; w < 8; ++w) {
+                ls[w] = w < n_waves ? ls[w] : 0.f;
+                os[w] = w < n_waves ? os[w] : 0.f;
+            }
         }
         float num = 0.f, den = 0.f;
 #pragma unroll
