@@ -2052,7 +2052,7 @@ extern "C" int egpt_paged_attention_decode(const void* qkv, void* out, float* pa
     if (n_seqs <= 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || table_width <= 0 || window < 0 || n_splits < 1 ||
         (n_splits > 1 && (!part_o || !part_ml)))
         return EGPT_BAD_ARGUMENT;
-    if ((hd != 64 && hd != 128) || page_size % 16 != 0 || nq / nkv > 16 || nkv > 65535 || n_splits > 64 ||
+    if ((hd != 64 && hd != 128) || page_size < 16 || page_size % 16 != 0 || nq / nkv > 16 || nkv > 65535 || n_splits > 64 ||
         n_waves < 1 || n_waves > 8)
         return EGPT_UNSUPPORTED_SIZE;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2079,7 +2079,7 @@ static int attention_decode_fused(const float* qkv_prod, int in_splits, const fl
     if (n_seqs <= 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || table_width <= 0 || window < 0 || n_splits < 1 ||
         (n_splits > 1 && (!part_o || !part_ml)))
         return EGPT_BAD_ARGUMENT;
-    if ((hd != 64 && hd != 128) || page_size % 16 != 0 || nq / nkv > 16 || nkv > 65535 || n_splits > 64 ||
+    if ((hd != 64 && hd != 128) || page_size < 16 || page_size % 16 != 0 || nq / nkv > 16 || nkv > 65535 || n_splits > 64 ||
         n_waves < 1 || n_waves > 8)
         return EGPT_UNSUPPORTED_SIZE;
     FusedQkv f = {};
@@ -2136,7 +2136,7 @@ extern "C" int egpt_paged_attention_mfma(const void* qkv, void* out, float* part
     if (n_seqs <= 0 || n_tokens < 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || table_width <= 0 || window < 0 ||
         n_splits < 1 || (n_splits > 1 && (!part_o || !part_ml)))
         return EGPT_BAD_ARGUMENT;
-    if ((hd != 64 && hd != 128) || page_size % 16 != 0 || nkv > 65535 || n_splits > 64 ||
+    if ((hd != 64 && hd != 128) || page_size < 16 || page_size % 16 != 0 || nkv > 65535 || n_splits > 64 ||
         (rows_per_wave != 16 && rows_per_wave != 32))
         return EGPT_UNSUPPORTED_SIZE;
     if (n_tokens == 0) return EGPT_OK;
