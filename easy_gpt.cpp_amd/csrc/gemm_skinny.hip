@@ -173,8 +173,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
     const int step_end = min(total_steps, step_begin + a.steps_per_split);
     const int n_steps = step_end - step_begin;
     // lane group lg takes the lg-th 16 bytes of each 64 of a row: the four groups of a load instruction read 64
-    // contiguous bytes of each of its 16 rows (a memory request is 64 bytes wide; x is read from LDS the same way).  What lies past k is
-    // read as zero through the buffer's bound, not behind a branch: with eight branches around eight loads
+    // contiguous bytes of each of its 16 rows (a memory request is 64 bytes wide; x is read from LDS the same way).  What lies past the
+    // range is read as zero through the buffer's bound, not behind a branch: with eight branches around eight loads
     // a step of 97 products for eight rows took 768 us, 760 so.
     const int row0 = min(n0, n - 1);
     const buffer_t w_rows = values_of(a.w + static_cast<size_t>(row0) * k, static_cast<size_t>(min(n - row0, kRowsPerWave)) * k * 2);
@@ -185,13 +185,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(const bf16_t* __re
     for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     uint4 a_cur[4], a_next[4];
+    const int k_end = min(k, step_end * kStep);
     auto load_w = [&](uint4* av, int step) {
         const int k0 = step * kStep + lg * 8;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            av[q] = __builtin_bit_cast(uint4, read16(w_rows, k0 + q * 32 < k ? w_at + (step * kStep + q * 32) * 2 : kNowhere));
+            av[q] = __builtin_bit_cast(uint4, read16(w_rows, k0 + q * 32 < k_end ? w_at + (step * kStep + q * 32) * 2 : kNowhere));
     };
-    // the stream of w starts before anything else (a range of one step loads the next one, which is another range's or past k, in vain)
+    // the stream of w starts before anything else (the second step of a range of one is past its end and costs no memory: fetched all the
+    // same it made a step of the 0.5B sizes, whose QKV and output products have such ranges, 668 us for one user, 659 so, and 737 and 734 for eight)
     load_w(a_cur, step_begin);
     load_w(a_next, step_begin + 1);
     // and the arguments that are used last are asked for now
