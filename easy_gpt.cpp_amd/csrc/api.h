@@ -123,7 +123,7 @@ int egpt_attention_decode_ranged(const float* qkv_prod, int in_splits, const flo
                                  int hd, int page_size, float scale, int window, const int32_t* ranges, int range_slots,
                                  void* stream);
 // One decoded token per request: workgroups of n_waves wavefronts per (request, kv head, key split); lean != 0: the
-// variant with half the loads in flight per round and fewer registers.
+// variant with half the loads in flight per round and fewer registers, 2: with rounds of one block of 32 keys.
 int egpt_paged_attention_decode(const void* qkv, void* out, float* part_o, float* part_ml, const void* k_cache,
                                 const void* v_cache, const int32_t* block_table, int table_width,
                                 const int32_t* q_start, const int32_t* kv_len, int n_seqs, int nq, int nkv, int hd,

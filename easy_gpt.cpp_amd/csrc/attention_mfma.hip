@@ -1503,7 +1503,8 @@ __device__ __forceinline__ void decode_block(
             }
         }
         // the scores of all the round's keys, then one maximum, one factor for what was there before and their products (a block
-        // past the wavefront's last has no visible key and zeros for values)
+        // past the wavefront's last counts for nothing and is jumped over: computed all the same, behind 100 tokens, where that is every
+        // wavefront's second one, it made the kernel 3 to 8 % slower)
         const int last = min(p, w_end * 32 - 1);
         float s[PF][2][4];
         float mx = -INFINITY;
@@ -1511,6 +1512,11 @@ __device__ __forceinline__ void decode_block(
         for (int i = 0; i < PF; ++i)
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
+                if (i > 0 && kb0 + i >= w_end) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s[i][kt][v] = -INFINITY;
+                    continue;
+                }
                 f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int kd = 0; kd < KD; ++kd)
@@ -1534,6 +1540,7 @@ __device__ __forceinline__ void decode_block(
         for (int dt = 0; dt < DT; ++dt) { o[dt][0] *= alpha; o[dt][1] *= alpha; o[dt][2] *= alpha; o[dt][3] *= alpha; }
 #pragma unroll
         for (int i = 0; i < PF; ++i) {
+            if (i > 0 && kb0 + i >= w_end) continue;
             bf16x8 pb;
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
@@ -1567,47 +1574,52 @@ __device__ __forceinline__ void decode_block(
     }
     __syncthreads();
     const size_t row0 = static_cast<size_t>(tok) * nq + kh * group_size;
-    for (int idx = threadIdx.x; idx < group_size * HD; idx += n_threads) {
-        const int r = idx / HD, c = idx % HD;
-        // the states of all wavefronts are read together (past the last one the last again, of which nothing counts: a weight of zero
-        // would leave its infinities)
-        float ms[8], ls[8], os[8], mx = -INFINITY;
+    // (the states of all wavefronts are read together, of four or eight; past the last one the last again, of which nothing counts: a weight of
+    // zero would leave its infinities)
+    auto combine = [&](auto most) {
+        constexpr int N = decltype(most)::value;
+        for (int idx = threadIdx.x; idx < group_size * HD; idx += n_threads) {
+            const int r = idx / HD, c = idx % HD;
+            float ms[N], ls[N], os[N], mx = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            const float* st = wave_state + (min(w, n_waves - 1) * 16 + r) * kRow;
-            const float m = st[HD];
-            ms[w] = w < n_waves ? m : -INFINITY;
-            ls[w] = st[HD + 1];
-            os[w] = st[c];
-            mx = fmaxf(mx, ms[w]);
-        }
-        if (__builtin_expect(n_waves < 8, 0)) {
+            for (int w = 0; w < N; ++w) {
+                const float* st = wave_state + (min(w, n_waves - 1) * 16 + r) * kRow;
+                const float m = st[HD];
+                ms[w] = w < n_waves ? m : -INFINITY;
+                ls[w] = st[HD + 1];
+                os[w] = st[c];
+                mx = fmaxf(mx, ms[w]);
+            }
+            if (__builtin_expect(n_waves < N, 0)) {
 #pragma unroll
-            for (int w = 1; w < 8; ++w) {
-                ls[w] = w < n_waves ? ls[w] : 0.f;
-                os[w] = w < n_waves ? os[w] : 0.f;
+                for (int w = 1; w < N; ++w) {
+                    ls[w] = w < n_waves ? ls[w] : 0.f;
+                    os[w] = w < n_waves ? os[w] : 0.f;
+                }
+            }
+            float num = 0.f, den = 0.f;
+#pragma unroll
+            for (int w = 0; w < N; ++w) {
+                const float wgt = ms[w] == -INFINITY ? 0.f : __expf(ms[w] - mx);
+                num += wgt * os[w];
+                den += wgt * ls[w];
+            }
+            if (n_splits == 1) {
+                out[(row0 + r) * HD + c] = from_float<bf16_t>(num / den);
+            } else {
+                const size_t prow = RANGED ? static_cast<size_t>(bx) * nq + kh * group_size + r
+                                           : static_cast<size_t>(bz) * d.n_tokens * nq +
+                                                 (MIXED ? static_cast<size_t>(b) * nq + kh * group_size : row0) + r;
+                part_o[prow * HD + c] = num;
+                if (c == 0) {
+                    part_ml[prow * 2] = mx;
+                    part_ml[prow * 2 + 1] = den;
+                }
             }
         }
-        float num = 0.f, den = 0.f;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            const float wgt = ms[w] == -INFINITY ? 0.f : __expf(ms[w] - mx);
-            num += wgt * os[w];
-            den += wgt * ls[w];
-        }
-        if (n_splits == 1) {
-            out[(row0 + r) * HD + c] = from_float<bf16_t>(num / den);
-        } else {
-            const size_t prow = RANGED ? static_cast<size_t>(bx) * nq + kh * group_size + r
-                                       : static_cast<size_t>(bz) * d.n_tokens * nq +
-                                             (MIXED ? static_cast<size_t>(b) * nq + kh * group_size : row0) + r;
-            part_o[prow * HD + c] = num;
-            if (c == 0) {
-                part_ml[prow * 2] = mx;
-                part_ml[prow * 2 + 1] = den;
-            }
-        }
-    }
+    };
+    if (__builtin_expect(n_waves > 4, 1)) combine(std::integral_constant<int, 8>());
+    else combine(std::integral_constant<int, 4>());
 }
 
 // INF: partial sums of the product that are read in one batch (FUSED)
@@ -1816,15 +1828,15 @@ static int launch_decode(const void* qkv, void* out, float* part_o, float* part_
 static int dispatch_decode(const void* qkv, void* out, float* part_o, float* part_ml, const void* k_cache,
                            const void* v_cache, const int32_t* block_table, int table_width, const int32_t* q_start,
                            const int32_t* kv_len, int n_seqs, int nq, int nkv, int hd, int page_size, float scale,
-                           int window, int n_splits, int n_waves, int combine, bool lean, const FusedQkv* fused,
+                           int window, int n_splits, int n_waves, int combine, int lean, const FusedQkv* fused,
                            const int32_t* q_len, const int32_t* ranges, int slots, hipStream_t s) {
-    // lean: the variant with half the loads in flight and fewer registers (the caller's choice, see the wrapper)
+    // lean: the variant with half the loads in flight and fewer registers, 2: with a block of keys a round (the caller's choice, see the wrapper)
 #define EGPT_LAUNCH_DECODE(HD_, PF_)                                                                                \
     launch_decode<HD_, PF_>(qkv, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len, \
                             n_seqs, n_seqs, nq, nkv, page_size, scale, window, n_splits, n_waves, combine, fused,   \
                             q_len, ranges, slots, s)
     if (ranges && (slots < n_seqs || slots > kRangeSlots || !part_o || !part_ml)) return EGPT_BAD_ARGUMENT;
-    if (hd == 64) return lean ? EGPT_LAUNCH_DECODE(64, 2) : EGPT_LAUNCH_DECODE(64, 4);
+    if (hd == 64) return lean == 2 ? EGPT_LAUNCH_DECODE(64, 1) : lean ? EGPT_LAUNCH_DECODE(64, 2) : EGPT_LAUNCH_DECODE(64, 4);
     return lean ? EGPT_LAUNCH_DECODE(128, 1) : EGPT_LAUNCH_DECODE(128, 2);
 #undef EGPT_LAUNCH_DECODE
 }
@@ -1966,7 +1978,7 @@ static int paged_attention_tiled(const void* qkv, void* out, const void* k_cache
     if (skip_single)
         return dispatch_decode(qkv, out, ranges ? range_o : part_o, ranges ? range_ml : part_ml, k_cache, v_cache, block_table, table_width,
                                q_start, kv_len, n_seqs, nq, nkv, hd, page_size, scale, window, single_splits, single_waves, 1,
-                               single_lean != 0, nullptr, q_len, ranges, slots, s);
+                               single_lean, nullptr, q_len, ranges, slots, s);
     return EGPT_OK;
 }
 
@@ -2057,7 +2069,7 @@ extern "C" int egpt_paged_attention_decode(const void* qkv, void* out, float* pa
         return EGPT_UNSUPPORTED_SIZE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     return dispatch_decode(qkv, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean != 0, nullptr, nullptr, nullptr, 0, s);
+                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean, nullptr, nullptr, nullptr, 0, s);
 }
 
 // The same with the QKV epilogue folded in: the queries, and the new token's key and value, are computed from
@@ -2092,7 +2104,7 @@ static int attention_decode_fused(const float* qkv_prod, int in_splits, const fl
     f.k_cache_w = static_cast<bf16_t*>(k_cache); f.v_cache_w = static_cast<bf16_t*>(v_cache);
     hipStream_t s = static_cast<hipStream_t>(stream);
     return dispatch_decode(nullptr, out, part_o, part_ml, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean != 0, &f, nullptr, ranges, range_slots, s);
+                           n_seqs, nq, nkv, hd, page_size, scale, window, n_splits, n_waves, combine, lean, &f, nullptr, ranges, range_slots, s);
 }
 
 extern "C" int egpt_attention_decode_fused(const float* qkv_prod, int in_splits, const float* row_ss, int ss_splits,

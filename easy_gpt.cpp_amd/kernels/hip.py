@@ -1036,6 +1036,7 @@ class HipKernels(KernelBackend):
             if max_q_len == 1 and t == b and nq // nkv <= 16:
                 # only decoded tokens: workgroups of several wavefronts per (request, kv head, key split)
                 n_splits, n_waves, lean = self._decode_shape(b, nkv, hd, max_kv_len, combine)
+                lean = self._decode_form(n_splits, n_waves, lean, hd, max_kv_len)
                 part_o = part_ml = None
                 if n_splits > 1:
                     part_o = torch.empty((n_splits, t, nq, hd), dtype=_F32, device=qkv.device)
@@ -1080,6 +1081,7 @@ class HipKernels(KernelBackend):
                     return None
                 if singles and b > 1 and nq // nkv <= 16 and max_kv_len > self.singles_apart_beyond:
                     n_splits, n_waves, lean = self._decode_shape(b, nkv, hd, max_kv_len, True)
+                    lean = self._decode_form(n_splits, n_waves, lean, hd, max_kv_len)
                 parts_rows = max(n_splits * b if n_splits > 1 else 0, key_splits * t if key_splits > 1 else 0)
                 if parts_rows:
                     part_o = torch.empty((parts_rows, nq, hd), dtype=_F32, device=qkv.device)
@@ -1290,8 +1292,18 @@ class HipKernels(KernelBackend):
         # (with more pairs than half the CUs also behind 8,192 tokens, 34 blocks per wavefront: 4.04 against 4.13 at batch 128)
         per_wave = -(-key_blocks // (n_splits * n_waves))
         # (and with 65 to 128 pairs behind 32,000 tokens: 5.77 against 5.85 at batch 64)
-        lean = (per_wave <= 17 or pairs > 64) if hd == 64 else pairs * n_splits > 384
+        # (head size 128: also where no wavefront has a second block for the full variant's round.  31 batches and sizes of 1 to 200 requests,
+        # times of the full variant: behind 100 tokens 0.80, behind 250 0.79, behind 2,048 0.82 to 1, as it was so)
+        lean = (per_wave <= 17 or pairs > 64) if hd == 64 else (pairs * n_splits > 384 or per_wave == 1)
         return n_splits, n_waves, 1 if lean else 0
+
+    @staticmethod
+    def _decode_form(n_splits, n_waves, lean, hd, max_kv_len):
+        """The kernel's `lean`: at head size 64 a third variant, with rounds of one key block, where no wavefront has a second one: the same bits
+        with half the loads and products, and what a round of two spends on a block that isn't there is a tenth of such a kernel's time
+        (29 batches and sizes of 1 to 200 requests, times of the variant with two, with the epilogue folded in and without: behind 60 tokens 0.85 and
+        0.89, behind 250 0.83 and 0.83)."""
+        return 2 if lean and hd == 64 and n_splits * n_waves >= -(-max_kv_len // 32) else lean
 
     def attention_decode_fused(self, prod, row_ss, hidden, eps, bias, positions, inv_freq, rotary_dim, slots, out,
                                k_cache, v_cache, block_table, q_start, kv_len, nq, nkv, hd, page_size, scale, window,
@@ -1337,6 +1349,7 @@ class HipKernels(KernelBackend):
                       int(window), ranges.data_ptr(), n_slots, self._stream())
             return None
         n_splits, n_waves, lean = self._decode_shape(b, nkv, hd, max_kv_len, combine)
+        lean = self._decode_form(n_splits, n_waves, lean, hd, max_kv_len)
         part_o = part_ml = None
         if n_splits > 1:
             part_o = torch.empty((n_splits, t, nq, hd), dtype=_F32, device=prod.device)

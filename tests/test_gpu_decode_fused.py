@@ -49,7 +49,7 @@ def test_places_of_pages_and_partial_sums(k, nq, nkv, hd, ps, parts, squares, ba
     assert torch.equal(out1, out2)
 
 
-@pytest.mark.parametrize("hd,lean", [(64, 0), (64, 1), (128, 0), (128, 1)])
+@pytest.mark.parametrize("hd,lean", [(64, 0), (64, 1), (64, 2), (128, 0), (128, 1)])
 @pytest.mark.parametrize("waves", [1, 2, 3, 4, 7, 8])
 @pytest.mark.parametrize("splits", [1, 2])
 def test_infinite_values_stay_infinite(k, hd, lean, waves, splits):
@@ -140,3 +140,26 @@ def test_a_page_of_more_than_two_gigabytes_a_head(k, hd):
     both = [both_ways(k, prod, None, None, kv_len, caches, table, slots, nq, nkv, hd, caches[0].shape[2]) for caches in (big, small)]
     for (out, kc, vc), (want, k2, v2) in zip(both[0], both[1]):
         assert torch.equal(kc[:, :, :80], k2) and torch.equal(vc[..., :80], v2) and near(out, want)
+
+
+@pytest.mark.parametrize("hd,leans", [(64, (0, 1, 2)), (128, (0, 1))])
+@pytest.mark.parametrize("kv", [1, 31, 33, 100, 255, 256, 257, 700])
+@pytest.mark.parametrize("waves,splits", [(8, 1), (4, 1), (3, 2), (8, 3)])
+def test_variants_of_the_kernel_agree(k, hd, leans, kv, waves, splits):
+    # rounds of one, two and four blocks of keys, also where a wavefront has fewer: the same bits where it has one block at most, and the same
+    # keys in any case (the reference)
+    nq, nkv, ps = 6, 2, 48
+    kc, vc, table, keys, vals = build_paged([(1, kv)], nkv, hd, ps, torch.bfloat16, seed=81)
+    qkv = rnd(1, (nq + 2 * nkv) * hd, dtype=torch.bfloat16, seed=82) * 2
+    start, context = (torch.tensor([v], dtype=torch.int32, device=DEV) for v in (0, kv))
+    want = paged_reference(qkv.double().cpu().view(1, nq + 2 * nkv, hd)[:, :nq], keys[0].double(), vals[0].double(), nq, nkv, hd ** -0.5, 0)[0]
+    outs = []
+    for lean in leans:
+        out, part_o, part_ml = torch.empty(1, nq * hd, dtype=torch.bfloat16, device=DEV), rnd(splits, nq, hd), rnd(splits, nq, 2)
+        k._run("egpt_paged_attention_decode", qkv.data_ptr(), out.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+               table.data_ptr(), table.shape[1], start.data_ptr(), context.data_ptr(), 1, nq, nkv, hd, ps, hd ** -0.5, 0, splits, waves, 1, lean,
+               k._stream())
+        outs.append(out)
+        assert float((out.double().cpu().view(nq, hd) - want).abs().max()) <= 1.2e-2
+    if -(-kv // 32) <= waves * splits:
+        assert all(torch.equal(outs[0], o) for o in outs)

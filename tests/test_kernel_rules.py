@@ -25,6 +25,14 @@ def test_decode_attention_shapes_are_launchable():
         assert lds <= 96 * 1024, what
 
 
+def test_decode_attention_takes_rounds_of_one_block_where_no_wavefront_has_two():
+    for b, nkv, hd, ctx in itertools.product(BATCHES, [1, 2, 3, 4, 8, 16, 40], [64, 128], CONTEXTS + [129, 250, 256, 600]):
+        n_splits, n_waves, lean = K._decode_shape(b, nkv, hd, ctx, True)
+        one = -(-(-(-ctx // 32)) // (n_splits * n_waves)) == 1
+        assert not one or lean == 1, (b, nkv, hd, ctx)
+        assert K._decode_form(n_splits, n_waves, lean, hd, ctx) == (2 if one and hd == 64 else lean), (b, nkv, hd, ctx)
+
+
 def test_shapes_of_new_prompts():
     # (tokens, nq, nkv, head size, page size, longest context) and the workgroup shape, at and around the lines
     for sizes, shape in [((580, 14, 2, 64, 16, 580), 24), ((590, 14, 2, 64, 16, 590), 44), ((1300, 14, 2, 64, 16, 1300), 44), ((1400, 14, 2, 64, 16, 700), 44),
