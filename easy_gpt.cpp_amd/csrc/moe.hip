@@ -250,7 +250,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* __restri
     __syncthreads();
     const int share = (n_rows + n_waves - 1) / n_waves, begin = wave * share, end = min(n_rows, begin + share);
     constexpr int kKeep = 16;
-    const bool kept = share <= kKeep * kWave;
+    const bool kept = share > kWave && share <= kKeep * kWave;       // (one choice a lane needs no loads together)
     int own[kKeep];                              // (an expert past the last one: nothing to count)
     if (kept) {
 #pragma unroll
