@@ -155,20 +155,29 @@ __device__ __forceinline__ void write_quad(float* p, const float (&v)[4]) { *rei
 __device__ __forceinline__ void write_quad(bf16_t* p, const float (&v)[4]) {
     *reinterpret_cast<uint2*>(p) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
 }
-// of a product, partial sums added in the order of at(), the loads of three of them on their way together
+// of a product, partial sums added in the order of at(), the loads of up to three of them on their way together (and none in vain: one
+// sum after the first is read once, not three times)
+template <int N>
+__device__ __forceinline__ void add_quads(const float* p, size_t stride, float (&v)[4]) {
+    float t[N][4];
+#pragma unroll
+    for (int u = 0; u < N; ++u) read_quad(p + u * stride, t[u]);
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += t[u][e];
+}
 template <typename T>
 __device__ __forceinline__ void read_quad(const ProductView<T>& p, size_t at, float (&v)[4]) {
     if (p.n_splits == 0) return read_quad(p.whole + at, v);
-    read_quad(p.partial + at, v);
-    for (int s0 = 1; s0 < p.n_splits; s0 += 3) {
-        float t[3][4];
-#pragma unroll
-        for (int u = 0; u < 3; ++u) read_quad(p.partial + min(s0 + u, p.n_splits - 1) * p.split_stride + at, t[u]);
-#pragma unroll
-        for (int u = 0; u < 3; ++u)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = s0 + u < p.n_splits ? v[e] + t[u][e] : v[e];
-    }
+    const float* from = p.partial + at;
+    read_quad(from, v);
+    if (p.n_splits == 1) return;
+    from += p.split_stride;
+    int left = p.n_splits - 1;
+    for (; left >= 3; left -= 3, from += 3 * p.split_stride) add_quads<3>(from, p.split_stride, v);
+    if (left == 2) add_quads<2>(from, p.split_stride, v);
+    if (left == 1) add_quads<1>(from, p.split_stride, v);
 }
 // Whether all of these begin on 16 bytes (null does).
 template <typename... P>
