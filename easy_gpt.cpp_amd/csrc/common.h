@@ -155,20 +155,35 @@ __device__ __forceinline__ void write_quad(float* p, const float (&v)[4]) { *rei
 __device__ __forceinline__ void write_quad(bf16_t* p, const float (&v)[4]) {
     *reinterpret_cast<uint2*>(p) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
 }
+// (and pairs and single values by the same names)
+__device__ __forceinline__ void read_quad(const float* p, float (&v)[2]) {
+    const float2 a = *reinterpret_cast<const float2*>(p);
+    v[0] = a.x; v[1] = a.y;
+}
+__device__ __forceinline__ void read_quad(const bf16_t* p, float (&v)[2]) {
+    const uint32_t a = *reinterpret_cast<const uint32_t*>(p);
+    v[0] = __uint_as_float(a << 16); v[1] = __uint_as_float(a & 0xffff0000u);
+}
+template <typename T>
+__device__ __forceinline__ void read_quad(const T* p, float (&v)[1]) { v[0] = to_float(p[0]); }
+__device__ __forceinline__ void write_quad(float* p, const float (&v)[2]) { *reinterpret_cast<float2*>(p) = float2{v[0], v[1]}; }
+__device__ __forceinline__ void write_quad(bf16_t* p, const float (&v)[2]) { *reinterpret_cast<uint32_t*>(p) = bf16_pair(v[0], v[1]); }
+template <typename T>
+__device__ __forceinline__ void write_quad(T* p, const float (&v)[1]) { p[0] = from_float<T>(v[0]); }
 // of a product, partial sums added in the order of at(), the loads of up to three of them on their way together (and none in vain: one
 // sum after the first is read once, not three times)
-template <int N>
-__device__ __forceinline__ void add_quads(const float* p, size_t stride, float (&v)[4]) {
-    float t[N][4];
+template <int N, int E>
+__device__ __forceinline__ void add_quads(const float* p, size_t stride, float (&v)[E]) {
+    float t[N][E];
 #pragma unroll
     for (int u = 0; u < N; ++u) read_quad(p + u * stride, t[u]);
 #pragma unroll
     for (int u = 0; u < N; ++u)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += t[u][e];
+        for (int e = 0; e < E; ++e) v[e] += t[u][e];
 }
-template <typename T>
-__device__ __forceinline__ void read_quad(const ProductView<T>& p, size_t at, float (&v)[4]) {
+template <typename T, int E>
+__device__ __forceinline__ void read_quad(const ProductView<T>& p, size_t at, float (&v)[E]) {
     if (p.n_splits == 0) return read_quad(p.whole + at, v);
     const float* from = p.partial + at;
     read_quad(from, v);

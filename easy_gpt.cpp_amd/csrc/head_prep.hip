@@ -13,6 +13,16 @@
 
 namespace egpt {
 
+template <typename T>
+__host__ __device__ static ProductView<T> view_of(const void* p, int n_splits, size_t split_stride) {
+    ProductView<T> v;
+    v.whole = n_splits == 0 ? static_cast<const T*>(p) : nullptr;
+    v.partial = n_splits > 0 ? static_cast<const float*>(p) : nullptr;
+    v.n_splits = n_splits;
+    v.split_stride = split_stride;
+    return v;
+}
+
 constexpr int kMaxHeadWidth = 1024;                   // the widest head (or latent) these kernels take
 constexpr int kOwn = kMaxHeadWidth / kWave;           // values of it that a lane keeps
 
@@ -416,6 +426,9 @@ __global__ __launch_bounds__(256) void whole_norm_store_kernel(
 // The same with a quad of the row in each thread's registers: the three parts, the row and the heads multiples of four values, up to 4,096
 // of them.  2,535 rows of 896 + 128 + 128 19.0 -> 10.6 us: single values found their head and page by two divisions each.
 constexpr int kQuadsMost = 4096;
+constexpr long kGatedFew = 250000;      // values below which a gated norm of heads takes a wavefront a head (the lines between measured sizes: 7 and 16 heads
+                                         // of 128 at 290,000, 14 of 64 at 215,000; us by wavefronts and by quads, bfloat16, one float32 array: 100 rows of
+                                         // 16 heads of 128 2.4 and 2.6, 360 rows 3.5 and 3.1)
 template <typename T>
 __global__ __launch_bounds__(kQuadsMost / 4) void whole_norm_store_quads_kernel(
     const T* __restrict__ bias, T* __restrict__ q_out, const T* __restrict__ q_weight, const T* __restrict__ k_weight,
@@ -529,30 +542,53 @@ __global__ __launch_bounds__(kWave) void head_norm_gate_kernel(ProductView<float
     }
 }
 
-// The same for heads of 64, 128 or 256 values: 16, 32 or 64 lanes a head, a quad each, a workgroup of four wavefronts for the next heads
-// of all tokens.  2,535 rows of seven heads of 128 13.1 -> 10.5 us: one wavefront a workgroup is bound by how fast they are handed out.
-template <typename T, int LANES>
-__global__ __launch_bounds__(256) void head_norm_gate_quads_kernel(const T* __restrict__ weight, T* __restrict__ out, int n_items, int heads,
-                                                                   unsigned heads_magic, int x_width, int gate_width, int gate_off, int gate_act,
-                                                                   float eps, ProductView<float> x, ProductView<T> xa, ProductView<T> g) {
-    constexpr int dv = LANES * 4;
-    const int item = blockIdx.x * (256 / LANES) + threadIdx.x / LANES, d = threadIdx.x % LANES * 4;
+// The same for heads of 64, 128 or 256 values, V neighbouring ones a lane.  Many rows: quads, 16, 32 or 64 lanes a head, a workgroup of four
+// wavefronts for the next heads of all tokens.  2,535 rows of seven heads of 128 13.1 -> 10.5 us: one wavefront a workgroup is bound by how fast
+// they are handed out.  Few rows: a wavefront a head, which is as long as its instructions, four sigmoids a lane among them; the squares
+// are added in the quads' order, so the rows of both are the same bits.  Eight rows of 14 heads of 64, float32, in a chain of them: 2.5 us by
+// quads, 2.1 so.  What the operands are addressed by stands in the 14 words that arrive with the wavefronts (as structs they
+// were a trip of their own).
+template <typename T, int LANES, int V>
+__global__ __launch_bounds__(V == 4 ? 256 : 64) void head_norm_gate_quads_kernel(
+    const void* __restrict__ x, const void* __restrict__ gates, int x_splits, int gate_splits, int n_items, int heads, unsigned heads_magic,
+    int x_width, int gate_width, int gate_off, int x_is_act, int gate_act, const T* __restrict__ weight, T* __restrict__ out, size_t x_stride,
+    size_t gate_stride, float eps) {
+    constexpr int dv = LANES * V;
+    const int item = blockIdx.x * ((V == 4 ? 256 : 64) / LANES) + threadIdx.x / LANES, d = threadIdx.x % LANES * V;
     if (item >= n_items) return;                          // (whole heads: the lanes of one go together)
     const int t = divided(item, heads, heads_magic), h = item - t * heads;
     const size_t xr = static_cast<size_t>(t) * x_width + h * dv + d;
-    float v[4], gate[4], w[4];
-    if (xa.present()) read_quad(xa, xr, v);
-    else read_quad(x, xr, v);
-    const bool gated = g.present();
-    if (gated) read_quad(g, static_cast<size_t>(t) * gate_width + gate_off + h * dv + d, gate);
+    float v[V], gate[V], w[V];
+    if (x_is_act) read_quad(static_cast<const T*>(x) + xr, v);
+    else read_quad(view_of<float>(x, x_splits, x_stride), xr, v);
+    const bool gated = gates != nullptr;
+    if (gated) read_quad(view_of<T>(gates, gate_splits, gate_stride), static_cast<size_t>(t) * gate_width + gate_off + h * dv + d, gate);
     if (weight) read_quad(weight + d, w);
-    float ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
-    ss = fold_row(ss, AddOf());
-    if (LANES >= 32) ss = fold_16_apart(ss, AddOf());
-    if (LANES == 64) ss = fold_32_apart(ss, AddOf());
+    // the quad's values, in every lane that has some of them, then the quads 1, 2, 4, .. apart
+    float ss;
+    if constexpr (V == 4) {
+        ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
+        ss = fold_row(ss, AddOf());
+        if (LANES >= 32) ss = fold_16_apart(ss, AddOf());
+        if (LANES == 64) ss = fold_32_apart(ss, AddOf());
+    } else {
+        float q[4];
+        if constexpr (V == 2) {                           // quad_perm 0 0 2 2 and 1 1 3 3
+            q[0] = dpp_move<0xa0>(v[0]); q[1] = dpp_move<0xa0>(v[1]);
+            q[2] = dpp_move<0xf5>(v[0]); q[3] = dpp_move<0xf5>(v[1]);
+        } else {
+            q[0] = dpp_move<0x00>(v[0]); q[1] = dpp_move<0x55>(v[0]);
+            q[2] = dpp_move<0xaa>(v[0]); q[3] = dpp_move<0xff>(v[0]);
+        }
+        ss = fmaf(q[3], q[3], fmaf(q[2], q[2], fmaf(q[1], q[1], q[0] * q[0])));
+        if (V == 2) ss += dpp_move<0x4e>(ss);             // (as in fold_row)
+        ss += dpp_move<0x141>(ss);
+        ss += dpp_move<0x140>(ss);
+        ss = fold_rows(ss, AddOf());
+    }
     const float inv = inv_rms(ss, 1.0f / static_cast<float>(dv), eps);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < V; ++e) {
         v[e] = v[e] * inv * (weight ? w[e] : 1.0f);
         if (gated) {
             const float sig = 1.0f / (1.0f + expf(-gate[e]));
@@ -601,16 +637,6 @@ __global__ __launch_bounds__(256) void head_norm_gate_wide_kernel(ProductView<fl
         if (d < dv) put(d, v[i]);
     }
     for (int d = threadIdx.x + kKeep * 256; d < dv; d += 256) put(d, act_typed ? xa.at(xr + d) : x.at(xr + d));
-}
-
-template <typename T>
-static ProductView<T> view_of(const void* p, int n_splits, size_t split_stride) {
-    ProductView<T> v;
-    v.whole = n_splits == 0 ? static_cast<const T*>(p) : nullptr;
-    v.partial = n_splits > 0 ? static_cast<const float*>(p) : nullptr;
-    v.n_splits = n_splits;
-    v.split_stride = split_stride;
-    return v;
 }
 
 }  // namespace egpt
@@ -831,18 +857,21 @@ extern "C" int egpt_head_norm_gate(const void* x, int x_splits, int x_is_act, in
     const long items = static_cast<long>(n_tokens) * heads;
     if ((dv == 64 || dv == 128 || dv == 256) && x_width % 4 == 0 && (!gate || (gate_width % 4 == 0 && gate_off % 4 == 0)) && items < (1 << 27) &&
         quads(x, weight, gate, out)) {
-        auto launch = [&](auto kernel, auto* to, int lanes) {
+        auto launch = [&](auto kernel, auto* to, int threads, int lanes) {
             using T = std::remove_pointer_t<decltype(to)>;
-            const int per = 256 / lanes;
-            kernel<<<static_cast<unsigned>((items + per - 1) / per), 256, 0, s>>>(
-                static_cast<const T*>(weight), to, static_cast<int>(items), heads, magic_of(heads), x_width, gate_width, gate_off, gate_act, eps, xv,
-                view_of<T>(x_is_act ? x : nullptr, 0, 0), view_of<T>(gate, gate_splits, stride));
+            const int per = threads / lanes;
+            kernel<<<static_cast<unsigned>((items + per - 1) / per), threads, 0, s>>>(
+                x, gate, x_splits, gate_splits, static_cast<int>(items), heads, magic_of(heads), x_width, gate_width, gate_off, x_is_act, gate_act,
+                static_cast<const T*>(weight), to, xv.split_stride, stride, eps);
         };
+        const bool few = items * dv < kGatedFew;
         auto pick = [&](auto* to) {
             using T = std::remove_pointer_t<decltype(to)>;
-            if (dv == 64) launch(head_norm_gate_quads_kernel<T, 16>, to, 16);
-            else if (dv == 128) launch(head_norm_gate_quads_kernel<T, 32>, to, 32);
-            else launch(head_norm_gate_quads_kernel<T, 64>, to, 64);
+            if (dv == 64 && few) launch(head_norm_gate_quads_kernel<T, 64, 1>, to, 64, 64);
+            else if (dv == 64) launch(head_norm_gate_quads_kernel<T, 16, 4>, to, 256, 16);
+            else if (dv == 128 && few) launch(head_norm_gate_quads_kernel<T, 64, 2>, to, 64, 64);
+            else if (dv == 128) launch(head_norm_gate_quads_kernel<T, 32, 4>, to, 256, 32);
+            else launch(head_norm_gate_quads_kernel<T, 64, 4>, to, 256, 64);
         };
         if (dtype == 0) pick(static_cast<float*>(out));
         else pick(static_cast<bf16_t*>(out));

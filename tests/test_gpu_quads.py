@@ -109,6 +109,27 @@ def test_gates_of_heads(k, dtype, heads, dv, splits, gate, weighed):
             assert torch.equal(out, other)                    # (no statistic: the same operations)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,dv", [(14, 64), (7, 128), (1, 64), (8, 256)])
+@pytest.mark.parametrize("splits", [0, 1, 2, 3, 4, 5, 7, 8])
+def test_a_row_of_gated_heads_is_the_same_among_few_and_among_many(k, dtype, heads, dv, splits):
+    # 250,000 values are the line between a wavefront for a head and quads; the partial sums' loads go by threes and what is left of them
+    n = heads * dv
+    t = 250000 // n + 3
+    x, w, g = draw(max(splits, 1), t, n, seed=20), draw(dv, seed=21, dtype=dtype), draw(max(splits, 1), t, n + 4, seed=22)
+    many = torch.empty(t, n, dtype=dtype, device=DEV)
+    k.head_norm_gate(x[0] if splits == 0 else x, w, 1e-5, g, 4, many, heads, dv)
+    total, gate = x.double().sum(0).view(t, heads, dv), g.double().sum(0)[:, 4:]
+    want = (total * torch.rsqrt((total * total).mean(-1, keepdim=True) + 1e-5) * w.double()).view(t, n) * gate * torch.sigmoid(gate)
+    step = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0       # (one rounding, and 32-bit sums of values of a size of `splits`)
+    assert ((many.double() - want).abs() <= step * want.abs() + 1e-5 * (want.abs() + 1)).all()
+    for first, count in ((0, 1), (t - 37, 37), (5, 250000 // n - 4)):
+        some = torch.empty(count, n, dtype=dtype, device=DEV)
+        rows = slice(first, first + count)
+        k.head_norm_gate(x[0, rows].contiguous() if splits == 0 else x[:, rows].contiguous(), w, 1e-5, g[:, rows].contiguous(), 4, some, heads, dv)
+        assert torch.equal(some, many[rows])
+
+
 @pytest.mark.parametrize("hidden,experts,top,tokens", [(64, 4, 2, 65), (192, 16, 4, 1300), (192, 16, 4, 4200), (896, 16, 4, 90)])
 def test_experts_of_many_tokens_into_a_given_sum(k, hidden, experts, top, tokens):
     # a choice's place in its expert's rows is nobody's business: the sums are the same bits whichever way the choices are grouped
