@@ -1667,9 +1667,10 @@ __global__ __launch_bounds__(512) void attention_mixed_kernel(
 // out[row, :] = sum_s exp(m_s - M) o_s / sum_s exp(m_s - M) l_s over the splits; one wavefront per row, R features of it a lane (R * 64
 // of them or fewer).  Lane s takes split s's (maximum, sum) so that the weights of up to 64 splits are known after one round of loads;
 // the first eight splits' partial outputs are asked for together with them (a part of a split without visible keys may hold anything:
-// it is read and then dropped), the others eight at a time.  A layer of 64 decoded tokens, 14 heads of 64, two splits, against four
-// features a lane whatever the head size and shuffles through LDS: the fastest 3.7 -> 2.0 us, the median, which is the trips to memory
-// behind attention's writes, 4.7 and 5.0.
+// it is read and then dropped), the others eight at a time.  Against four features a lane whatever the head size and shuffles through LDS, the same
+// step with this kernel alone exchanged, us: 14 heads of 64 on 2, 24 layers, 64 users behind 130 to 2,048 tokens 1,161 -> 1,141, 32 behind 2,048
+// 1,024 -> 1,004; 12 of 128 on 2, 28 layers, 32 behind 1,500 to 2,000 1,837 -> 1,800, 40 beside a portion of 512 3,490 -> 3,467.  (A kernel trace has
+// the same 4.9 us for both, the trips to memory behind attention's writes; the fastest 2.6 -> 1.5.)
 template <int R>
 __global__ __launch_bounds__(64) void attention_reduce_kernel(const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml,
