@@ -76,33 +76,36 @@ class SwiGLU(FeedForward):
                 return down(act)
             x = x.materialize()
             residual = pending.residual()
-        t = x.shape[0]
-        act = k.gate_up_swiglu(x, self.w_gate_up, activation=self.activation)        # a few dozen tokens: product and activation in one kernel
-        if act is None:
-            act = k.gate_up_rows(x, self.w_gate_up, activation=self.activation)      # and more of them
-        if act is not None:
-            return down(act)
-        gate_up = k.product(x, self.w_gate_up)           # act [T, 2I] or float32 partial sums [S, T, 2I]
-        if gate_up.dim() == 3:
+        act, gate_up = self._gated(x)
+        if act is None and gate_up.dim() == 3:
             out = k.product_swiglu(gate_up, None, self.hidden_size, 0.0, self.w_down, residual=residual, activation=self.activation)
             if out is not None:
                 return None if out is residual else out
-        act = torch.empty((t, self.intermediate_size), dtype=x.dtype, device=x.device)
-        k.swiglu(gate_up, act, activation=self.activation)
-        return down(act)
+        return down(self._activated(gate_up, x) if act is None else act)
 
+    def _gated(self, x):
+        """(act [T, I], None), or (None, gate_up) where product and activation are not one kernel: act [T, 2I] or float32 partial sums
+        [S, T, 2I]."""
+        k = kernels.backend()
+        act = k.gate_up_swiglu(x, self.w_gate_up, activation=self.activation)        # a few dozen tokens
+        if act is None:
+            act = k.gate_up_rows(x, self.w_gate_up, activation=self.activation)      # and more of them
+        return (act, None) if act is not None else (None, k.product(x, self.w_gate_up))
+
+    def _activated(self, gate_up, x):
+        act = torch.empty((x.shape[0], self.intermediate_size), dtype=x.dtype, device=x.device)
+        kernels.backend().swiglu(gate_up, act, activation=self.activation)
+        return act
 
     def with_room(self, x, ctx=None):
         """What `forward` returns for many tokens as float32 [1 + splits, T, H], the first sum for the caller to write: another branch's
-        output stands beside this one's without a copy of either.  None where the backend has no use for it."""
+        output stands beside this one's without a copy of either.  None where the backend has no use for it, and for a class of its own
+        `forward`, which this one knows nothing of."""
         k = kernels.backend()
-        if not self.unrounded or not k.writes_sums_in_place or x.shape[0] <= 64:
+        if not self.unrounded or not k.writes_sums_in_place or x.shape[0] <= 64 or type(self).forward is not SwiGLU.forward:
             return None
-        act = k.gate_up_rows(x, self.w_gate_up, activation=self.activation)
-        if act is None:
-            act = torch.empty((x.shape[0], self.intermediate_size), dtype=x.dtype, device=x.device)
-            k.swiglu(k.product(x, self.w_gate_up), act, activation=self.activation)
-        return k.product_room(act, self.w_down)
+        act, gate_up = self._gated(x)
+        return k.product_room(self._activated(gate_up, x) if act is None else act, self.w_down)
 
 
 class ActivatedFeedForward(FeedForward):

@@ -142,3 +142,28 @@ def test_experts_of_many_tokens_into_a_given_sum(k, hidden, experts, top, tokens
     assert torch.equal(into[1], want) and (into[0] == 7).all() and (into[2] == 7).all()
     few = torch.cat([k.expert_mixture(x[i : i + 64].contiguous(), router, None, up, down, top) for i in range(0, tokens, 64)])
     assert ((want - few).abs() <= 1e-2 * few.abs().amax()).all()
+
+
+@pytest.mark.parametrize("dtype,m,n,kk", [
+    (torch.bfloat16, 65, 128, 256), (torch.bfloat16, 300, 896, 768), (torch.bfloat16, 2048, 896, 896),         # the framework's own kernel
+    (torch.bfloat16, 130, 896, 4864), (torch.bfloat16, 2535, 896, 768), (torch.bfloat16, 300, 72, 72),         # the library's
+    (torch.bfloat16, 64, 128, 256), (torch.bfloat16, 7, 896, 896), (torch.bfloat16, 100, 64, 36),      # few rows, k no multiple of eight: copied
+    (torch.float32, 100, 96, 64), (torch.float32, 700, 896, 768), (torch.float32, 3, 64, 60)])
+def test_product_with_room_in_front(k, dtype, m, n, kk):
+    x, w = draw(m, kk, seed=30, dtype=dtype), draw(n, kk, seed=31, dtype=dtype) * 0.1
+    want = k.product(x, w, unrounded=True)
+    want = want if want.dim() == 3 else want.float()[None]
+    got = k.product_room(x, w)
+    assert got.dtype == torch.float32 and got.is_contiguous() and got.shape == (1 + want.shape[0], m, n)
+    got[0].fill_(float("nan"))                                # (the caller's: nothing of the sums lies there)
+    assert torch.equal(got[1:], want)
+    assert ((got[1:].double().sum(0) - x.double() @ w.double().T).abs() <= 2e-2 * (kk ** 0.5)).all()
+
+
+def test_whose_products_with_room_are(k, monkeypatch):
+    # the sizes above
+    run, own = k._run, []
+    monkeypatch.setattr(k, "_run", lambda name, *a: (own.append(a[3:6]) if name == "egpt_gemm_rows" else None, run(name, *a))[1])
+    for m, n, kk in ((65, 128, 256), (300, 896, 768), (2048, 896, 896), (130, 896, 4864), (2535, 896, 768), (300, 72, 72)):
+        k.product_room(draw(m, kk, seed=1, dtype=torch.bfloat16), draw(n, kk, seed=2, dtype=torch.bfloat16))
+    assert own == [(65, 128, 256), (300, 896, 768), (2048, 896, 896)]
