@@ -163,3 +163,38 @@ def test_variants_of_the_kernel_agree(k, hd, leans, kv, waves, splits):
         assert float((out.double().cpu().view(nq, hd) - want).abs().max()) <= 1.2e-2
     if -(-kv // 32) <= waves * splits:
         assert all(torch.equal(outs[0], o) for o in outs)
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(14, 2, 64), (16, 1, 128), (6, 6, 128)])
+@pytest.mark.parametrize("ps", [48, 80, 256])
+@pytest.mark.parametrize("batch,ctx,window", [(1, 2049, 0), (9, 497, 131), (2, 3000, 700)])
+@pytest.mark.parametrize("folded", [True, False])
+def test_pages_of_any_sixteens_against_64_bits(k, nq, nkv, hd, ps, batch, ctx, window, folded):
+    # queries from so short that hundreds of keys count to so long that a single one has most of a row's weight: what is read from the wrong place,
+    # left out or seen twice shows as an error of the size of the values, which are N(0, 1).  Otherwise an output is a mean of values, off by
+    # the rounding of probabilities (2^-9 of each) and of the result (2^-9 of up to 4)
+    kv_len = torch.tensor([max(1, ctx - 37 * i % ctx) for i in range(batch)], dtype=torch.int32)
+    kc, vc, table, keys, vals = build_paged([(1, int(n)) for n in kv_len], nkv, hd, ps, torch.bfloat16, seed=91)
+    slots = torch.stack([table[b, (int(n) - 1) // ps].cpu() * ps + (int(n) - 1) % ps for b, n in enumerate(kv_len)]).to(torch.int32).to(DEV)
+    width = (nq + 2 * nkv) * hd
+    prod = rnd(2, batch, width, seed=92)
+    prod[:, :, : nq * hd] *= torch.linspace(1.0, 8.0, nq, device=DEV).repeat_interleave(hd)
+    inv_freq = torch.as_tensor(plain.rope_inv_freq(hd, 1e4), dtype=torch.float32).to(DEV)
+    kv, start, one = kv_len.to(DEV), torch.arange(batch, dtype=torch.int32, device=DEV), torch.ones(batch, dtype=torch.int32, device=DEV)
+    k1, v1 = kc.clone(), vc.clone()
+    qkv, out = torch.empty(batch, width, dtype=torch.bfloat16, device=DEV), torch.empty(batch, nq * hd, dtype=torch.bfloat16, device=DEV)
+    k.qkv_rope_store(prod, None, kv - 1, inv_freq, hd, slots, k1, v1, nq, nkv, hd, ps, out=qkv)
+    if folded:
+        assert k.attention_decode_fused(prod, None, 0, 0.0, None, kv - 1, inv_freq, hd, slots, out, kc, vc, table, start, kv, nq, nkv, hd, ps,
+                                        hd ** -0.5, window, int(kv_len.max())) is None
+    else:
+        k.paged_attention(qkv, out, k1, v1, table, start, one, kv, nq, nkv, hd, ps, hd ** -0.5, window, 1, int(kv_len.max()))
+    row = qkv.double().cpu().view(batch, nq + 2 * nkv, hd)
+    for b in range(batch):
+        lo = max(0, int(kv_len[b]) - window) if window else 0
+        kk, vv = keys[b].double(), vals[b].double()
+        kk[-1], vv[-1] = row[b, nq : nq + nkv], row[b, nq + nkv :]
+        q = row[b, :nq].view(nkv, nq // nkv, hd)
+        scores = torch.matmul(q, kk[lo:].permute(1, 2, 0).contiguous()) * hd ** -0.5
+        want = torch.matmul(torch.softmax(scores, -1), vv[lo:].permute(1, 0, 2).contiguous()).view(nq, hd)
+        assert float((out[b].double().cpu().view(nq, hd) - want).abs().max()) <= 3e-2, b
