@@ -81,3 +81,33 @@ def test_keys_of_two_wavefronts_are_combined_with_the_same_rounding(k, hd, shape
     own, other = parts.sum(1)
     expected = np.where(other_first, combined(own, other, 3, weight, True), combined(own, other, 3, weight, False))
     assert (got[0] == expected).all()
+
+
+@pytest.mark.parametrize("pairs", [False, True])
+def test_rounding_to_bfloat16_is_half_to_even(k, pairs):  # noqa: F811
+    # Every upper half of a float32 with the lower halves at which rounding turns, subnormals, the largest numbers, infinities and NaN among them,
+    # as values of heads, which the QKV epilogue rounds and does nothing else to: one by one (no rotation), or in pairs (the kernel for many
+    # tokens).  (x 1 + 0 stands in front of the rounding: a zero's sign is not asked for.)
+    low = np.array([0, 1, 0x7FFF, 0x8000, 0x8001, 0xFFFF], np.uint32)
+    bits = ((np.arange(1 << 16, dtype=np.uint32) << 16)[:, None] | low).reshape(96, 4096)
+    t, heads, hd = 96, 32, 128
+    prod = torch.from_numpy(np.tile(bits, (1, 3)).view(np.float32)).to(DEV)[None].contiguous()
+    assert (prod.view(torch.int32)[0, :, :4096].cpu().numpy().view(np.uint32) == bits).all()
+    positions = torch.arange(t, dtype=torch.int32, device=DEV)
+    slots = positions + 0
+    kc, vc = torch.zeros(6, heads, 16, hd, dtype=torch.bfloat16, device=DEV), torch.zeros(6, heads, hd, 16, dtype=torch.bfloat16, device=DEV)
+    out = torch.zeros(t, 3 * heads * hd, dtype=torch.bfloat16, device=DEV)
+    if pairs:
+        inv_freq = torch.ones(hd // 2, device=DEV)
+        k.qkv_rope_store(prod, None, positions, inv_freq, hd, slots, kc, vc, heads, heads, hd, 16, out=out, cos_sin=k.rope_table(positions, inv_freq))
+    else:
+        k.qkv_rope_store(prod, None, positions, None, 0, slots, kc, vc, heads, heads, hd, 16, out=out)
+    want = bf16(bits.view(np.float32))
+    want = np.where(want == 0x8000, 0, want)
+    nan = (want & 0x7FFF) > 0x7F80
+    stored = vc.permute(0, 3, 1, 2).reshape(t, heads * hd)
+    for got in [out[:, 2 * heads * hd :], stored] + ([] if pairs else [out[:, : heads * hd]]):
+        got = got.contiguous().cpu().view(torch.int16).numpy().view(np.uint16)
+        got = np.where(got == 0x8000, 0, got)
+        assert (((got & 0x7FFF) > 0x7F80) == nan).all()
+        assert (got[~nan] == want[~nan]).all()
