@@ -17,7 +17,7 @@ __device__ __forceinline__ float to_float(bf16_t v) { return __uint_as_float(sta
 
 // round to nearest even; NaN stays NaN
 // (v_cvt_pk_bf16_f32: one instruction for two values in the place of some fourteen; the same bits as rounding half to even on the
-// integer, NaN made quiet, for every one of the 2^32 float32 values)
+// integer, NaN made quiet: tests/test_gpu_rounding.py has every upper half with lower halves around the tie, subnormals among them)
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
 __device__ __forceinline__ uint32_t bf16_pair(float low, float high) {
     typedef __attribute__((ext_vector_type(2))) float two;

@@ -216,9 +216,10 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec8_kernel(float* __restrict
     }
 }
 
-// The same for few rows of bfloat16, a workgroup to a row, four neighbouring features a thread: what bounds it is the trip to what the
-// kernels before wrote and the instructions around it, so every load goes out at once (partial sums past the last one are past the
-// buffer's end and add zero) and nothing stands behind a branch.  With single values, then so, in decode steps: 64 rows of 896
+// The same for rows of bfloat16 up to 4,096 values (of many rows up to 2,048), a workgroup to a row, four neighbouring features a thread:
+// what bounds it is the trip to what the kernels before wrote and the instructions around it.  So the loads of the row, its weight and up to
+// eight partial sums go out together, the partial sums bounded by a buffer (what lies past the last one adds zero), the others behind one
+// test for the row's end; partial sums past the eighth are further rounds of eight.  With single values, then so, in decode steps: 64 rows of 896
 // behind partial sums 4.4 -> 3.7 us on average (the fastest 3.4 -> 1.9); a step with 29 norms of 8 rows of 3,584 in fixed point 3,516 -> 3,484.
 __device__ __forceinline__ void load_stream(const float* p, float (&v)[4]) {
     const float4 a = *reinterpret_cast<const float4*>(p);
@@ -234,11 +235,11 @@ __device__ __forceinline__ void store_stream(fixed_t* p, const float (&v)[4]) {
     *reinterpret_cast<longlong2*>(p + 2) = longlong2{to_fixed(v[2]), to_fixed(v[3])};
 }
 enum Added { kNothing = 0, kWhole = 1, kParts = 2 };
-constexpr int kFewMost = 4096;              // features: four for each of 1,024 threads
+constexpr int kQuadsMost = 4096;              // features: four for each of 1,024 threads
 
 // BATCH: partial sums whose loads are on their way together
 template <typename R, int ADDED, int BATCH = 1>
-__global__ __launch_bounds__(kFewMost / 4) void add_rmsnorm_few_kernel(R* __restrict__ h, const void* __restrict__ added,
+__global__ __launch_bounds__(kQuadsMost / 4) void add_rmsnorm_quads_kernel(R* __restrict__ h, const void* __restrict__ added,
                                                                        const bf16_t* __restrict__ weight, bf16_t* __restrict__ out,
                                                                        int hidden, int n_splits, int split_stride,
                                                                        const int32_t* __restrict__ rows, float w_off, float eps) {
@@ -300,18 +301,18 @@ __global__ __launch_bounds__(kFewMost / 4) void add_rmsnorm_few_kernel(R* __rest
     }
 }
 template <typename R>
-static void launch_norm_few(void* h, const void* delta, int n_splits, int stride, const int32_t* rows, const void* weight, float w_off, float eps,
+static void launch_norm_quads(void* h, const void* delta, int n_splits, int stride, const int32_t* rows, const void* weight, float w_off, float eps,
                             void* out, int n_rows, int hidden, hipStream_t s) {
     const int threads = (hidden / 4 + kWave - 1) / kWave * kWave;
     auto launch = [&](auto kernel) {
         kernel<<<n_rows, threads, 0, s>>>(static_cast<R*>(h), delta, static_cast<const bf16_t*>(weight), static_cast<bf16_t*>(out), hidden, n_splits,
                                           stride, rows, w_off, eps);
     };
-    if (!delta) launch(add_rmsnorm_few_kernel<R, kNothing>);
-    else if (n_splits == 0) launch(add_rmsnorm_few_kernel<R, kWhole>);
-    else if (n_splits == 1) launch(add_rmsnorm_few_kernel<R, kParts, 1>);
-    else if (n_splits == 2) launch(add_rmsnorm_few_kernel<R, kParts, 2>);
-    else launch(add_rmsnorm_few_kernel<R, kParts, 8>);
+    if (!delta) launch(add_rmsnorm_quads_kernel<R, kNothing>);
+    else if (n_splits == 0) launch(add_rmsnorm_quads_kernel<R, kWhole>);
+    else if (n_splits == 1) launch(add_rmsnorm_quads_kernel<R, kParts, 1>);
+    else if (n_splits == 2) launch(add_rmsnorm_quads_kernel<R, kParts, 2>);
+    else launch(add_rmsnorm_quads_kernel<R, kParts, 8>);
 }
 
 // ----------------------------------------------------------------------------- SwiGLU
@@ -615,9 +616,9 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
     if (dtype != 0 && dtype != 1) return EGPT_BAD_ARGUMENT;
     // Many rows go by quads as well up to 2,048 values: 2,048 rows of 896 behind two partial sums 8.1 -> 6.6 us, behind a rounded product 6.9 ->
     // 6.0, 552 rows of 1,536 7.0 -> 5.6 and 5.7 -> 5.5.  Wider ones are the same either way (prompts of the 7B sizes 24.06 and 24.08 ms) and keep
-    // eight values a thread, which holds more of them.
+    // eight values a thread, which holds more of them; so do partial sums that 32 bits of place don't reach, whatever the width.
     const bool many = delta_splits <= 1 ? n_rows >= 32 : n_rows > 64;
-    const bool by_quads = dtype == 1 && hidden % 4 == 0 && hidden <= (many && !fixed && hidden % 8 == 0 ? 2048 : kFewMost) && aligned &&
+    const bool by_quads = dtype == 1 && hidden % 4 == 0 && hidden <= (many && !fixed && hidden % 8 == 0 ? 2048 : kQuadsMost) && aligned &&
                           (delta_splits + 8) * static_cast<long long>(stride) * 4 <= INT32_MAX;
     if (dtype == 1 && hidden % 8 == 0 && aligned && !fixed && many && !by_quads) {
         const int threads = hidden >= 2048 ? 256 : 128;
@@ -634,8 +635,8 @@ extern "C" int egpt_add_rmsnorm(void* h, int fixed, const void* delta, int delta
         return EGPT_OK;
     }
     if (by_quads) {
-        if (fixed) launch_norm_few<fixed_t>(h, delta, delta_splits, static_cast<int>(stride), rows, weight, weight_offset, eps, out, n_rows, hidden, s);
-        else launch_norm_few<float>(h, delta, delta_splits, static_cast<int>(stride), rows, weight, weight_offset, eps, out, n_rows, hidden, s);
+        if (fixed) launch_norm_quads<fixed_t>(h, delta, delta_splits, static_cast<int>(stride), rows, weight, weight_offset, eps, out, n_rows, hidden, s);
+        else launch_norm_quads<float>(h, delta, delta_splits, static_cast<int>(stride), rows, weight, weight_offset, eps, out, n_rows, hidden, s);
         EGPT_CHECK_LAUNCH();
         return EGPT_OK;
     }
