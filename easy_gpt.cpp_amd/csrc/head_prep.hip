@@ -426,6 +426,7 @@ __global__ __launch_bounds__(256) void whole_norm_store_kernel(
 // The same with a quad of the row in each thread's registers: the three parts, the row and the heads multiples of four values, up to 4,096
 // of them.  2,535 rows of 896 + 128 + 128 19.0 -> 10.6 us: single values found their head and page by two divisions each.
 constexpr int kQuadsMost = 4096;
+constexpr size_t kGateFew = 131072;     // values up to which a gate behind more than eight partial sums goes by single ones
 constexpr long kGatedFew = 250000;      // values below which a gated norm of heads takes a wavefront a head (the lines between measured sizes: 7 and 16 heads
                                          // of 128 at 290,000, 14 of 64 at 215,000; us by wavefronts and by quads, bfloat16, one float32 array: 100 rows of
                                          // 16 heads of 128 2.4 and 2.6, 360 rows 3.5 and 3.1)
@@ -770,7 +771,11 @@ extern "C" int egpt_sigmoid_gate(const void* x, int heads, const void* gate, int
     const size_t total = static_cast<size_t>(n_tokens) * n;
     const size_t stride = static_cast<size_t>(n_tokens) * gate_width;
     const unsigned blocks = static_cast<unsigned>((total + 255) / 256);
-    if (heads == 0 && n % 4 == 0 && gate_width % 4 == 0 && gate_off % 4 == 0 && n <= 65535 * 1024 && quads(x, gate, out)) {
+    // Few values behind many partial sums take single ones, whose loads of sixteen sums are on their way together where a quad's go by threes: us
+    // by single values and by quads, 8 rows of 896 in float32, 7 sums 2.11 and 2.01, 8 2.12 and 2.17, 11 2.17 and 2.27, 16 2.32 and 2.44; 64 rows of
+    // 2,048, 16 sums 2.57 and 2.62; 128 rows of them 3.19 and 2.83.  The same bits.
+    const bool deep = gate_splits > 8 && total <= kGateFew;
+    if (heads == 0 && !deep && n % 4 == 0 && gate_width % 4 == 0 && gate_off % 4 == 0 && n <= 65535 * 1024 && quads(x, gate, out)) {
         const dim3 grid(n_tokens, (n / 4 + 255) / 256);
         if (dtype == 0)
             sigmoid_gate_quads_kernel<float><<<grid, 256, 0, s>>>(static_cast<const float*>(x), static_cast<float*>(out), n, gate_width, gate_off,

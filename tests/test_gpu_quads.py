@@ -130,6 +130,25 @@ def test_a_row_of_gated_heads_is_the_same_among_few_and_among_many(k, dtype, hea
         assert torch.equal(some, many[rows])
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("splits", [8, 9, 16, 17])
+def test_a_gated_row_is_the_same_among_few_and_among_many(k, dtype, splits):
+    # more than eight partial sums of up to 131,072 values go by single values
+    n = 2048
+    t = 131072 // n + 1
+    x, g = draw(t, n, seed=30, dtype=dtype), draw(splits, t, n + 4, seed=31)
+    many = torch.empty_like(x)
+    k.sigmoid_gate(x, 0, g, 4, many)
+    want = x.double() * torch.sigmoid(g.double().sum(0)[:, 4:])
+    # one rounding, and sixteen additions of sums below 16, each off by 2^-24 of itself: 1.6e-5 in the gate, a quarter of it in the sigmoid, of x < 5
+    step = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    assert ((many.double() - want).abs() <= step * want.abs() + 2e-5 * (want.abs() + 1)).all()
+    for first, count in ((0, 1), (1, t - 1)):
+        some = torch.empty_like(x[:count])
+        k.sigmoid_gate(x[first : first + count].contiguous(), 0, g[:, first : first + count].contiguous(), 4, some)
+        assert torch.equal(some, many[first : first + count])
+
+
 @pytest.mark.parametrize("hidden,experts,top,tokens", [(64, 4, 2, 65), (192, 16, 4, 1300), (192, 16, 4, 4200), (896, 16, 4, 90)])
 def test_experts_of_many_tokens_into_a_given_sum(k, hidden, experts, top, tokens):
     # a choice's place in its expert's rows is nobody's business: the sums are the same bits whichever way the choices are grouped
